@@ -60,32 +60,37 @@ sage_k_colsum_kernel(const __half *k, uint32_t capacity, uint32_t kv_len, uint32
     }
 }
 
-// One workgroup of 256 threads per head: column d = tid % D, part lanes tid / D take parts pl, pl + 256 / D, ... (eight
-// loads in flight at a time), then the lanes in order.
+// Adds the parts of a head in a fixed order: a workgroup of 1024 threads owns MEAN_FIN_COLS columns of one head, so that a
+// launch has D / MEAN_FIN_COLS workgroups per head and every thread adds at most a few parts, all of its loads in flight at
+// once. Thread (column d = tid % COLS, part lane tid / COLS) takes the parts pl, pl + lanes, ...; the lanes are added through
+// LDS in a tree. Latency-bound: with one workgroup of 256 threads per head, 32 dependent batches of loads deep, SmolLM3 at 32K
+// (4 heads x 512 parts x 128 columns, 1 MB) took 8.0 us of the build's 28.1; the build is 22.7 us now.
+constexpr int MEAN_FIN_COLS = 16, MEAN_FIN_NT = 1024, MEAN_FIN_LANES = MEAN_FIN_NT / MEAN_FIN_COLS;
+constexpr int MEAN_FIN_LOADS = MEAN_MAX_PARTS / MEAN_FIN_LANES;  // parts per thread at most
+
 template <int D>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(MEAN_FIN_NT)
 sage_k_mean_finish_kernel(const float *partial, uint32_t n_parts, uint32_t kv_len, float *mean) {
-    __shared__ float sm[256];
-    const uint32_t h = blockIdx.x, tid = threadIdx.x;
-    const uint32_t d = tid % D, pl = tid / D, npl = 256 / D;
+    __shared__ float sm[MEAN_FIN_NT];
+    const uint32_t h = blockIdx.y, tid = threadIdx.x;
+    const uint32_t d = blockIdx.x * MEAN_FIN_COLS + tid % MEAN_FIN_COLS, pl = tid / MEAN_FIN_COLS;
     const float *hp = partial + (size_t)h * n_parts * D + d;
+    float v[MEAN_FIN_LOADS];
+#pragma unroll
+    for (int u = 0; u < MEAN_FIN_LOADS; ++u) {
+        const uint32_t p = pl + u * MEAN_FIN_LANES;
+        v[u] = p < n_parts ? hp[(size_t)p * D] : 0.0f;
+    }
     float t = 0.0f;
-    for (uint32_t p0 = pl; p0 < n_parts; p0 += npl * 8) {
-        float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const uint32_t p = p0 + u * npl;
-            v[u] = p < n_parts ? hp[(size_t)p * D] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) t += v[u];
-    }
+    for (int u = 0; u < MEAN_FIN_LOADS; ++u) t += v[u];
     sm[tid] = t;
-    __syncthreads();
-    if (pl == 0) {
-        for (uint32_t j = 1; j < npl; ++j) t += sm[j * D + d];
-        mean[(size_t)h * D + d] = kv_len ? t / (float)kv_len : 0.0f;
+#pragma unroll
+    for (uint32_t half = MEAN_FIN_NT / 2; half >= MEAN_FIN_COLS; half >>= 1) {
+        __syncthreads();
+        if (tid < half) sm[tid] = t = t + sm[tid + half];
     }
+    if (tid < MEAN_FIN_COLS) mean[(size_t)h * D + d] = kv_len ? t / (float)kv_len : 0.0f;
 }
 
 __device__ __forceinline__ int quant_i8(float x, float scale) {
@@ -330,9 +335,9 @@ fa_status fa_launch_sage_k_mean(fa_ctx *ctx, const void *k, uint32_t n_kv_heads,
     }
     FaLaunchScope scope(ctx, "sage_k_mean_finish_kernel", true);
     if (head_dim == 128)
-        scope.launch(sage_k_mean_finish_kernel<128>, dim3(n_kv_heads), dim3(256), 0, partial, n_parts, kv_len, mean_out);
+        scope.launch(sage_k_mean_finish_kernel<128>, dim3(128 / MEAN_FIN_COLS, n_kv_heads), dim3(MEAN_FIN_NT), 0, partial, n_parts, kv_len, mean_out);
     else
-        scope.launch(sage_k_mean_finish_kernel<64>, dim3(n_kv_heads), dim3(256), 0, partial, n_parts, kv_len, mean_out);
+        scope.launch(sage_k_mean_finish_kernel<64>, dim3(64 / MEAN_FIN_COLS, n_kv_heads), dim3(MEAN_FIN_NT), 0, partial, n_parts, kv_len, mean_out);
     return scope.finish();
 }
 
