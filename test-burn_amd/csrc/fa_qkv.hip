@@ -23,6 +23,7 @@
 // the MatMul op (src/metals/matmul.rs:190-239 -> GemvV2, write stage src/metals/gemv/stages.rs:200-224): the o_proj
 // consumer of the attention output.
 #include "fa_internal.h"
+#include "fa_norm.h"
 #include "fa_qkv_rope.h"
 #include <atomic>
 #include <type_traits>
@@ -58,12 +59,6 @@ struct QkvDev {
 template <typename T>
 __device__ __forceinline__ T pick3(int mat, T x0, T x1, T x2) {
     return mat == 0 ? x0 : mat == 1 ? x1 : x2;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
 }
 
 // WB: bits per weight - 16 (f16), 8 (Q8_0) or 4 (Q4_0)
@@ -216,6 +211,20 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
     __half *const out0 = a.out[0], *const out1 = a.out[1], *const out2 = a.out[2];
     const float eps = a.eps, alpha = a.alpha, beta = a.beta;
     asm volatile("" ::"s"(residual), "s"(bias0), "s"(bias1), "s"(bias2), "s"(out0), "s"(out1), "s"(out2), "s"(eps), "s"(alpha), "s"(beta));
+    // The thread that will store (row, column) of the first tile asks for its bias and residual here, behind the weights: asked
+    // for where they are added, after the last sum, they put another trip to memory between the products and the store. (Every
+    // lane loads, from an address that is valid whatever its slot: no branch around a load.)
+    const uint32_t w_row = ((uint32_t)tid >> 4) & 15u, w_col = (uint32_t)tid & 15u;
+    _Float16 pre_bias, pre_res;
+    {
+        int mat;
+        uint32_t lrow;
+        locate(min(row_begin + w_row, row_end - 1u), mat, lrow);
+        const __half *pb = bias0 ? pick3(mat, bias0, bias1, bias2) + lrow : x_in;
+        const uint32_t N = pick3(mat, rows0, rows1, rows1);
+        const __half *pr = residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * N + lrow : x_in;
+        pre_bias = *reinterpret_cast<const _Float16 *>(pb), pre_res = *reinterpret_cast<const _Float16 *>(pr);
+    }
 
     // Input rows of this pass into LDS, normalised: x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16.
     // Four rows or more: a wave takes whole rows (row r by wave r % 8) and needs no workgroup barrier for the sum of
@@ -233,7 +242,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
                 for (int i = 0; i < 8; ++i) ss += (float)v[i] * (float)v[i];
             }
             if (gamma) {
-                const float inv_rms = rsqrtf(wave_sum(ss) / (float)K + eps);
+                const float inv_rms = rsqrtf(fa_norm::wave_sum(ss) / (float)K + eps);
                 for (uint32_t k8 = lane; k8 < K / 8; k8 += 64) {  // each lane rewrites what it wrote
                     h8_t v = *reinterpret_cast<const h8_t *>(dst + k8 * 16);
                     const h8_t g = *reinterpret_cast<const h8_t *>(gamma + k8 * 8);
@@ -257,7 +266,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
             for (int i = 0; i < 8; ++i) ss += (float)v[i] * (float)v[i];
         }
         if (gamma) {
-            ss = wave_sum(ss);
+            ss = fa_norm::wave_sum(ss);
             if (lane == 0) red[wave] = ss;
             __syncthreads();
             float tot = 0.0f;
@@ -265,7 +274,9 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
             for (int w = 0; w < QKV_NW; ++w) tot += red[w];
             const float inv_rms = rsqrtf(tot / (float)K + eps);
             for (uint32_t k8 = tid, j = 0; k8 < K / 8; k8 += QKV_NT, ++j) {  // each thread rewrites what it wrote
-                h8_t v = *reinterpret_cast<const h8_t *>(dst + k8 * 16);
+                h8_t v;
+                if (r == 0 && j < (uint32_t)XPRE) v = j == 0 ? x0[0] : x0[1];
+                else v = *reinterpret_cast<const h8_t *>(dst + k8 * 16);
                 h8_t g;
                 if (j < (uint32_t)XPRE) g = j == 0 ? g0[0] : g0[1];
                 else g = *reinterpret_cast<const h8_t *>(gamma + k8 * 8);
@@ -273,7 +284,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
                 for (int i = 0; i < 8; ++i) v[i] = (_Float16)(((float)v[i] * inv_rms) * (float)g[i]);
                 *reinterpret_cast<h8_t *>(dst + k8 * 16) = v;
             }
-            __syncthreads();  // `red` is reused by the next row
+            if (r + 1 < cols) __syncthreads();  // `red` is reused by the next row
         }
     }
     if (Q8) {
@@ -287,7 +298,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 
     // Sums the 8 waves' partial results of tile t in wave order, adds the bias, rounds once, stores token-major.
     auto finish_tile = [&](uint32_t t, const f4v_t &mine) __attribute__((always_inline)) {
-        __syncthreads();  // `red` may still be read for the previous tile
+        if (t) __syncthreads();  // `red` may still be read for the previous tile
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[((size_t)wave * 16 + c * 4 + i) * 17 + n] = mine[i];
         __syncthreads();
@@ -305,8 +316,8 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
                 __half *out = pick3(mat, out0, out1, out2);
                 const uint32_t N = pick3(mat, rows0, rows1, rows1);
                 s *= alpha;
-                if (bias) s += __half2float(bias[lrow]);
-                if (residual) s += __half2float(residual[(size_t)(m0 + col) * N + lrow]) * beta;
+                if (bias) s += t ? __half2float(bias[lrow]) : (float)pre_bias;
+                if (residual) s += (t ? __half2float(residual[(size_t)(m0 + col) * N + lrow]) : (float)pre_res) * beta;
                 out[(size_t)(m0 + col) * N + lrow] = __float2half(s);
             }
         }
@@ -516,30 +527,12 @@ __global__ void __launch_bounds__(QKV_NT, 1) fused_qkv_rows32_kernel(Rows32Dev a
             for (int w = 0; w < QKV_NW; ++w) tot += ss_lds[w * 32 + 16 * h + n];
             inv_rms[h] = rsqrtf(tot / (float)K + eps);
         }
-        // (x * inv_rms) * gamma, each product rounded to f32, the result to f16: two instructions per element that take the
-        // f16 halves as they lie in the registers (the plain form converts both factors and the result separately, five per
-        // element, and with all 32 rows to scale in every workgroup that was a quarter of the launch)
-        typedef uint32_t u4v_t __attribute__((ext_vector_type(4)));
-        const float neg_zero = -0.0f;  // (a sum with -0 keeps the sign of a zero product)
+        // (the plain form of the scaling, five instructions per element, was a quarter of the launch: every workgroup scales all 32 rows)
 #pragma unroll
         for (int j = 0; j < XJ; ++j) {
-            const u4v_t g2 = *reinterpret_cast<const u4v_t *>(g_lds + kb_of(j) * 32u + c * 8);
+            const h8_t g = *reinterpret_cast<const h8_t *>(g_lds + kb_of(j) * 32u + c * 8);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const u4v_t x2 = __builtin_bit_cast(u4v_t, xs[j][h]);
-                u4v_t y2;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float t0, t1;
-                    uint32_t y;
-                    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(x2[e]), "v"(inv_rms[h]), "v"(neg_zero));
-                    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(x2[e]), "v"(inv_rms[h]), "v"(neg_zero));
-                    asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,1,0]" : "=v"(y) : "v"(t0), "v"(g2[e]), "v"(neg_zero));
-                    asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "+v"(y) : "v"(t1), "v"(g2[e]), "v"(neg_zero));
-                    y2[e] = y;
-                }
-                xs[j][h] = __builtin_bit_cast(h8_t, y2);
-            }
+            for (int h = 0; h < 2; ++h) xs[j][h] = fa_norm::scale8(xs[j][h], inv_rms[h], g);
         }
     }
 #pragma unroll
@@ -738,6 +731,11 @@ fa_status fa_launch_fused_qkv_rows32_rope(fa_ctx *ctx, const FusedQkvLaunch &l, 
 }
 
 fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_stream_only) {
+    if (l.m == 1 && !(ctx->gemm_min_m == 1 && !weight_stream_only)) {
+        bool taken = false;
+        FA_TRY(fa_launch_gemv_row(ctx, l, &taken));
+        if (taken) return FA_OK;
+    }
     QkvDev a;
     for (int i = 0; i < 3; ++i) a.w[i] = l.w[i], a.bias[i] = l.bias[i], a.out[i] = l.out[i];
     a.rows[0] = l.n_dim, a.rows[1] = l.n_kv, a.rows[2] = l.n_kv;
