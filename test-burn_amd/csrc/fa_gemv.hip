@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
 #pragma unroll
         for (int p = 0; p < XP; ++p) {
             xv[u][p] = *reinterpret_cast<const h8_t *>(reinterpret_cast<const unsigned char *>(x) + off + p * 16);
-            gv[u][p] = *reinterpret_cast<const h8_t *>(reinterpret_cast<const unsigned char *>(gamma ? gamma : x) + off + p * 16);
+            gv[u][p] = fa_norm::load_global<h8_t>(reinterpret_cast<const unsigned char *>(gamma ? gamma : x) + off + p * 16);
         }
     }
     // every weight of the workgroup; a group past the last re-reads the last (its sums are not stored)
@@ -123,13 +123,13 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
     for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int t = 0; t < T; ++t)
-            wv[t][u] = __builtin_nontemporal_load(reinterpret_cast<const u4_t *>(base[t] + (rsub * row_stride + kb[u] * kbs[t] + part * 16)));
+            wv[t][u] = fa_norm::load_global_once<u4_t>(base[t] + (rsub * row_stride + kb[u] * kbs[t] + part * 16));
     if constexpr (WB != 16) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                sc[t][u] = *reinterpret_cast<const _Float16 *>(reinterpret_cast<const unsigned char *>(sbase[t]) + (rsub * nkb + kb[u]) * 2);
+                sc[t][u] = fa_norm::load_global<_Float16>(reinterpret_cast<const unsigned char *>(sbase[t]) + (rsub * nkb + kb[u]) * 2);
     }
     // what the thread that stores row tid of the workgroup adds to its sum
     const uint32_t rows0 = a.rows0, rows1 = a.rows1;
@@ -147,8 +147,8 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
         lrow -= rows0, bp = b1, op = o1;
         if (lrow >= rows1) lrow -= rows1, bp = b2, op = o2;
     }
-    const _Float16 bias = *reinterpret_cast<const _Float16 *>(b0 ? bp + lrow : x);
-    const _Float16 res = *reinterpret_cast<const _Float16 *>(residual ? residual + lrow : x);
+    const _Float16 bias = fa_norm::load_global<_Float16>(b0 ? bp + lrow : x);
+    const _Float16 res = fa_norm::load_global<_Float16>(residual ? residual + lrow : x);
 
     if (gamma) {
         float ss = 0.0f;
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
         __syncthreads();
         float tot = 0.0f;
         for (uint32_t i = 0; i < n_waves; ++i) tot += ss_lds[i];
-        const float inv_rms = rsqrtf(tot * (1.0f / RL) * inv_k + eps);
+        const float inv_rms = fa_norm::inv_rms(tot, inv_k * (1.0f / RL), eps);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
         s *= alpha;
         if (b0) s += (float)bias;
         if (residual) s += beta * (float)res;
-        op[lrow] = __float2half(s);
+        fa_norm::store_global(op + lrow, (_Float16)s);
     }
 }
 

@@ -11,6 +11,32 @@ typedef _Float16 norm_h8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t norm_u4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int norm_u2_t __attribute__((ext_vector_type(2)));
 
+// A load from device memory through an address that is chosen per lane. (The compiler does not see that such a pointer - a select
+// between arguments - is to global memory and would use flat loads, which also count as LDS accesses: every wait for one is a
+// wait for both.)
+template <typename T>
+__device__ __forceinline__ T load_global(const void *p) {
+    return *(const __attribute__((address_space(1))) T *)(uintptr_t)p;
+}
+template <typename T>
+__device__ __forceinline__ T load_global_once(const void *p) {  // read once per launch: not kept in the caches
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) T *)(uintptr_t)p);
+}
+
+template <typename T>
+__device__ __forceinline__ void store_global(void *p, T v) {
+    *(__attribute__((address_space(1))) T *)(uintptr_t)p = v;
+}
+
+// 1 / sqrt(mean + eps) from a row's sum of squares: one hardware reciprocal square root (within an ulp; the library's rsqrtf
+// adds a rescaling of denormal arguments, which epsilon keeps away from here). The empty slots: an instruction that uses a
+// transcendental's result must not follow at once; the compiler sees to that by itself, but not in front of scale8's assembly.
+__device__ __forceinline__ float inv_rms(float sum_sq, float inv_k, float eps) {
+    float r = __builtin_amdgcn_rsqf(fmaf(sum_sq, inv_k, eps));
+    asm volatile("s_nop 1" : "+v"(r));
+    return r;
+}
+
 // v + the values of lanes l ^ 16, l ^ 32, l ^ 48, in every lane
 __device__ __forceinline__ float sum_rows_of_16(float v) {
     norm_u2_t t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);

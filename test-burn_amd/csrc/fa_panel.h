@@ -1,0 +1,74 @@
+// FusedQkv and MatMul of a chunk of input rows that fits a workgroup's LDS 32 rows at a time ("panel"): one launch, RMSNorm and
+// KvPrepFused included. Reference: the same ops as fa_qkv.hip and fa_gemm.hip - src/metals/gemv/qkv_step.rs:14-120,
+// src/metals/matmul.rs:190-239, src/metals/rmsnorm/rmsnorm.metal:17-96, write stage src/metals/gemv/stages.rs:200-224,
+// src/metals/kv_prep/kv_prep_fused.metal:45-122.
+//
+// A chunk of a few dozen rows (a default prefill chunk of 32, a server's batch of sequences) is still a weight stream, but every
+// compute unit needs all of its input rows, normalised. What that costs is how they are asked for: a request in the layout of
+// the matrix instruction's operand (16 rows x 64 bytes, one row per lane of a 16-lane group) moves 37 KB/us into a compute unit
+// from L2, a request along a row 108 to 130 KB/us. So rows are fetched along themselves, whole rows per wave (row r by wave
+// r % 8), normalised in the registers they arrive in (no exchange between waves), written to LDS and read back as operands:
+//   * a workgroup (8 waves) owns up to 32 weight rows - two 16-row tiles - and walks over its passes of 32 input rows (16 where
+//     rows are longer than 2048 features). All its weights are requested once, straight into the operand layout, behind the
+//     first pass's input rows; a pass's rows are requested while the one before is multiplied;
+//   * wave w multiplies the feature blocks 16 j + 2 w and 16 j + 2 w + 1 of every 512 features (adjacent: the two requests touch
+//     the same lines);
+//   * the eight waves' partial tiles meet in LDS and are added in wave order; then alpha, bias, beta * residual and one
+//     rounding, or the KvPrepFused work on the rounded values (a workgroup then takes whole rotation pairs);
+//   * few weight rows and many input rows: the passes are spread over workgroups (grid y), each keeping its 32 weight rows.
+// Block-quantised weights become f16(weight * scale) as in the GEMM (src/metals/mma/tile_loader.metal:100-120); below 12 input
+// rows (SUMS) they follow the weight stream: a matrix instruction covers one 32-feature block, its f32 sums times the scale.
+#pragma once
+
+#include <type_traits>
+
+#include "fa_internal.h"
+#include "fa_norm.h"
+#include "fa_qkv_rope.h"
+
+namespace fa_panel {
+
+constexpr int NTHREADS = 512, NW = NTHREADS / 64;
+
+struct PanelDev {
+    const unsigned char *w[3];
+    const __half *scales[3], *bias[3];
+    __half *out[3];
+    uint32_t rows0, rows1, rows2, total_rows;
+    const __half *x, *gamma, *residual;
+    uint32_t k_dim, m, rows_per_wg, canonical, n_pass;
+    float eps, inv_k, alpha, beta;
+    RopeDev r;
+    uint32_t rcp_half_nkb, scale_pairs;  // floor(2^32 / ceil(blocks / 2)) + 1; a row holds an even number of scales
+    uint32_t block_shift;  // log2 of the page size, 32 = not a power of two
+};
+
+// A row in LDS: its 512-feature pieces, and 16 bytes so that 16 consecutive rows fall into 16 different bank groups.
+template <int PK>
+constexpr int row_bytes() { return PK * 1024 + 16; }
+template <int NT, int NC>
+constexpr int reduce_bytes() { return NW * NT * NC * 16 * 17 * 4; }
+template <int PK>
+constexpr bool G_IN_LDS = PK > 4;  // the longest rows: the norm's weights in LDS instead of registers
+template <int PK>
+constexpr int LDS_SHARE = (PK <= 2 ? 80 * 1024 : 160 * 1024) - 6 * 1024;  // two workgroups per compute unit, or one; less the scales
+// Two workgroups per compute unit: rows of up to 1024 features, except where the registers do not allow it.
+constexpr bool two_per_cu(uint32_t nt, uint32_t nc, uint32_t pk, bool rope) { return pk <= 2 && !(rope && nt == 2 && nc == 2); }
+// The waves' sums get LDS of their own where it is there (a barrier less per pass), else they go over the rows.
+template <int NT, int NC, int PK>
+constexpr bool REDUCE_APART = NC * 16 * row_bytes<PK>() + reduce_bytes<NT, NC>() + (G_IN_LDS<PK> ? PK * 1024 : 0) <= LDS_SHARE<PK>;
+template <int NT, int NC, int PK>
+constexpr int lds_rows_bytes() {
+    const int rows = NC * 16 * row_bytes<PK>(), red = reduce_bytes<NT, NC>();
+    return REDUCE_APART<NT, NC, PK> ? rows + red : rows > red ? rows : red;
+}
+template <int NT, int PK>
+constexpr int scale_bytes() { return NT * 16 * PK * 16 * 2; }  // block-quantised weights: [block][slot] f16
+template <int WB, int NT, int NC, int PK>
+constexpr int lds_bytes() { return lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0) + (WB != 16 ? scale_bytes<NT, PK>() : 0); }
+
+// launchers per weight width (one translation unit each): nt = 16-row tiles of weight rows, nc = 16-row groups of input rows per pass, pk = 512-feature pieces
+template <int WB>
+fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a);
+
+}  // namespace fa_panel

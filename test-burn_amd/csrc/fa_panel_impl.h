@@ -1,0 +1,409 @@
+// The panel kernel (see fa_panel.h) and its launcher for one weight width.
+#pragma once
+#include <atomic>
+
+#include "fa_panel.h"
+
+namespace fa_panel {
+
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef float f4v_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u2v_t __attribute__((ext_vector_type(2)));
+typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
+
+template <typename T>
+__device__ __forceinline__ T pick3(int mat, T x0, T x1, T x2) {
+    return mat == 0 ? x0 : mat == 1 ? x1 : x2;
+}
+
+__device__ __forceinline__ float dot8_self(h8_t a, float acc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_fdot2(h2_t{a[2 * i], a[2 * i + 1]}, h2_t{a[2 * i], a[2 * i + 1]}, acc, false);
+    return acc;
+}
+
+// Weight width -> what a lane holds of 8 consecutive weights, and those as f16 (times the block's scale, rounded to f16).
+template <int WB>
+struct Weights;
+template <>
+struct Weights<16> {
+    typedef h8_t raw_t;
+    static __device__ __forceinline__ h8_t f16(raw_t w, _Float16) { return w; }
+    static __device__ __forceinline__ h8_t plain(raw_t w) { return w; }
+    static __device__ __forceinline__ raw_t part(raw_t w, int) { return w; }
+};
+// s + 128 is a byte u, the f16 with bits 0x6400 | u is 1024 + u, minus 1152: exact
+__device__ __forceinline__ h8_t bytes_f16(uint32_t a, uint32_t b, _Float16 off) {
+    const h2_t bias = {off, off};
+    h8_t r;
+    const uint32_t w[2] = {a, b};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const h2_t lo = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x05010400u)) - bias;
+        const h2_t hi = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x07030602u)) - bias;
+        r[4 * i] = lo[0], r[4 * i + 1] = lo[1], r[4 * i + 2] = hi[0], r[4 * i + 3] = hi[1];
+    }
+    return r;
+}
+template <>
+struct Weights<8> {
+    typedef u2v_t raw_t;
+    static __device__ __forceinline__ raw_t part(u4v_t w, int i) { return raw_t{w[2 * i], w[2 * i + 1]}; }  // 8 weights of 16
+    static __device__ __forceinline__ h8_t plain(raw_t w) { return bytes_f16(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u, (_Float16)1152.0f); }
+    static __device__ __forceinline__ h8_t f16(raw_t w, _Float16 s) { return plain(w) * h8_t{s, s, s, s, s, s, s, s}; }
+};
+template <>
+struct Weights<4> {  // element 2i in the low nibble of byte i, value = nibble - 8
+    typedef uint32_t raw_t;
+    static __device__ __forceinline__ raw_t part(u4v_t w, int i) { return w[i]; }  // 8 weights of 32
+    static __device__ __forceinline__ h8_t plain(raw_t w) {
+        const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+        return bytes_f16(__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u), (_Float16)1032.0f);
+    }
+    static __device__ __forceinline__ h8_t f16(raw_t w, _Float16 s) { return plain(w) * h8_t{s, s, s, s, s, s, s, s}; }
+};
+
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
+__global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    static_assert(std::is_trivially_copyable<PanelDev>::value, "read as raw bytes from the argument block, where it is the first member");
+    const PanelDev &a = *(const PanelDev *)__builtin_amdgcn_kernarg_segment_ptr();
+    (void)a_by_value;
+    typedef Weights<WB> W;
+    typedef typename W::raw_t raw_t;
+    constexpr int XROW = row_bytes<PK>(), NR = 2 * NC, NB = 2 * PK;
+    const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
+    const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
+    const __half *const x_in = a.x, *const gamma = a.gamma;
+    const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
+    const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
+    const uint32_t normal = a.r.normal, head_dim = a.r.head_dim, rcp_half_nkb = a.rcp_half_nkb, scale_pairs = a.scale_pairs;
+    // (the launch's arguments in two trips through the scalar cache: what the first requests need, and the rest behind them)
+    asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(rows0), "s"(rows1), "s"(total_rows), "s"(x_in), "s"(gamma), "s"(K), "s"(m_rows),
+                 "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass));
+    if constexpr (WB != 16) asm volatile("" ::"s"(sp0), "s"(sp1), "s"(sp2), "s"(rcp_half_nkb), "s"(scale_pairs));
+    if constexpr (ROPE) asm volatile("" ::"s"(normal), "s"(head_dim));
+    const bool canonical = canonical_u != 0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, c = lane >> 4;
+    const uint32_t nkb = K / 32, n_pieces = K / 8;
+    const uint32_t row_begin = blockIdx.x * rows_per_wg;
+    const uint32_t row_end = min(total_rows, row_begin + rows_per_wg);
+    if (row_begin >= row_end) return;
+    // ROPE (rows_per_wg is even, the matrices hold whole heads): the pairing and the head size
+    uint32_t neox = 0, half_shift = 0, pair_begin = 0, pair_end = 0;
+    if constexpr (ROPE) {
+        neox = normal ? 0u : 1u, half_shift = head_dim == 128 ? 6u : 5u;
+        pair_begin = row_begin >> 1, pair_end = row_end >> 1;
+    }
+    // Weight row of slot (tile t, row n of the tile) across the three matrices laid end to end; a slot past the workgroup's
+    // last row gives the workgroup's first row with valid = false. NeoX pairs: tile 0 holds rows of first halves of heads, tile
+    // 1 their mates half a head on.
+    auto slot_row = [&](uint32_t t, uint32_t n_, bool &valid) __attribute__((always_inline)) -> uint32_t {
+        if (ROPE && neox) {
+            const uint32_t p = pair_begin + n_, pv = p < pair_end ? p : pair_begin;
+            valid = p < pair_end;
+            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + (t << half_shift);
+        }
+        const uint32_t gr = row_begin + 16u * t + n_;
+        valid = gr < row_end;
+        return valid ? gr : row_begin;
+    };
+    auto locate = [&](uint32_t row, int &mat) __attribute__((always_inline)) -> uint32_t {
+        const bool in1 = row >= rows0, in2 = row >= rows0 + rows1;
+        mat = (in1 ? 1 : 0) + (in2 ? 1 : 0);
+        return row - (in2 ? rows0 + rows1 : in1 ? rows0 : 0u);
+    };
+
+    // ---- input rows of a pass: rows wave, wave + 8, ... of it (a row past the chunk's last re-reads the last: its column is not
+    // stored), piece j of a row = features 512 j + 8 lane ..
+    h8_t xr[NR][PK];
+    auto request_rows = [&](uint32_t pass) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const __half *row = x_in + (size_t)min(pass * (NC * 16u) + (uint32_t)wave + 8u * i, m_rows - 1u) * K;
+#pragma unroll
+            for (int j = 0; j < PK; ++j) xr[i][j] = *reinterpret_cast<const h8_t *>(row + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
+        }
+    };
+    uint32_t pass = blockIdx.y;
+    request_rows(pass);
+    h8_t gv[PK];
+#pragma unroll
+    for (int j = 0; j < PK; ++j) gv[j] = *reinterpret_cast<const h8_t *>((gamma ? gamma : x_in) + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
+    // (the longest rows leave no registers for the norm's weights through the passes: they wait in LDS, behind the rows; every
+    // wave writes them all, so no wave waits for another's)
+    h8_t *const g_lds = reinterpret_cast<h8_t *>(smem + lds_rows_bytes<NT, NC, PK>());
+    if constexpr (G_IN_LDS<PK>) {
+#pragma unroll
+        for (int j = 0; j < PK; ++j) g_lds[j * 64 + lane] = gv[j];
+    }
+    // ---- block scales (block-quantised weights): [block][slot] f16 in LDS, fetched along the rows of the scale matrix, two at a
+    // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request)
+    _Float16 *const sc_lds = reinterpret_cast<_Float16 *>(smem + lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0));
+    constexpr int SLOTS = NT * 16, SC_LOADS = WB == 16 ? 1 : (SLOTS * PK * 8 + NTHREADS - 1) / NTHREADS;  // pairs per thread
+    uint32_t sc_raw[SC_LOADS];
+    const uint32_t half_nkb = (nkb + 1) / 2;
+    auto scale_at = [&](int i, uint32_t &slot, uint32_t &kb2) __attribute__((always_inline)) -> bool {
+        const uint32_t idx = (uint32_t)tid + (uint32_t)i * NTHREADS;
+        slot = __umulhi(idx, rcp_half_nkb), kb2 = idx - slot * half_nkb;  // (quotients of numbers below 2^16)
+        if (half_nkb == 1) slot = idx, kb2 = 0;
+        return slot < (uint32_t)SLOTS;
+    };
+    if constexpr (WB != 16) {
+#pragma unroll
+        for (int i = 0; i < SC_LOADS; ++i) {
+            uint32_t slot, kb2;
+            int mat;
+            bool valid;
+            if (!scale_at(i, slot, kb2)) slot = 0, kb2 = 0;
+            const uint32_t lrow = locate(slot_row(slot >> 4, slot & 15u, valid), mat);
+            const __half *sp = pick3(mat, sp0, sp1, sp2) + (size_t)lrow * nkb + 2 * kb2;
+            if (scale_pairs) {
+                sc_raw[i] = fa_norm::load_global<uint32_t>(sp);
+            } else {
+                const uint32_t lo = fa_norm::load_global<unsigned short>(sp);
+                sc_raw[i] = lo | ((uint32_t)fa_norm::load_global<unsigned short>(sp + (2 * kb2 + 1 < nkb ? 1 : 0)) << 16);
+            }
+        }
+    }
+    // ---- all weights of the workgroup. F16 (and SUMS): block kb of slot (t, n), features 8c .. 8c + 7. Block-quantised: 16 bytes
+    // per lane, half a block of one of two (Q8_0) or a block of four (Q4_0); the features that lane c holds for step s of such a
+    // request follow from that, for the weights and for the input rows alike.
+    constexpr bool WIDE = WB != 16 && !SUMS;
+    constexpr int GB = !WIDE ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
+    typedef typename std::conditional<WIDE, u4v_t, raw_t>::type req_t;
+    auto kb_of = [&](int i) __attribute__((always_inline)) -> uint32_t {
+        return GB == 1 ? 16u * (uint32_t)(i >> 1) + 2u * (uint32_t)wave + (uint32_t)(i & 1) : GB == 2 ? 16u * (uint32_t)i + 2u * (uint32_t)wave : 32u * (uint32_t)i + 4u * (uint32_t)wave;
+    };
+    const uint32_t lane_blk = GB == 1 ? 0u : GB == 2 ? (uint32_t)c >> 1 : (uint32_t)c;  // the lane's block of a request
+    req_t wv[NT][NQ];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        bool valid;
+        int mat;
+        const uint32_t lrow = locate(slot_row((uint32_t)t, (uint32_t)n, valid), mat);
+        const uint32_t N = pick3(mat, rows0, rows1, rows1);
+        // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
+        const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
+        const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
+        const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) wv[t][i] = fa_norm::load_global_once<req_t>(p0 + (size_t)min(kb_of(i) + lane_blk, nkb - 1u) * kb_stride);
+    }
+    const float eps = a.eps, inv_k = a.inv_k, alpha = a.alpha, beta = a.beta;
+    const __half *const residual = a.residual;
+    const __half *const bias0 = a.bias[0], *const bias1 = a.bias[1], *const bias2 = a.bias[2];
+    __half *const out0 = a.out[0], *const out1 = a.out[1], *const out2 = a.out[2];
+    asm volatile("" ::"s"(residual), "s"(bias0), "s"(bias1), "s"(bias2), "s"(out0), "s"(out1), "s"(out2), "s"(eps), "s"(inv_k), "s"(alpha), "s"(beta));
+    RopeDev r{};
+    uint32_t block_shift = 32;  // log2 of the page size, 32 = not a power of two
+    if constexpr (ROPE) {
+        r = a.r, block_shift = a.block_shift;
+        asm volatile("" ::"s"(r.cos_t), "s"(r.sin_t), "s"(r.block_table), "s"(r.n_kv_heads), "s"(r.position_offset), "s"(r.max_seq_len),
+                     "s"(r.block_size), "s"(r.capacity), "s"(r.table_rows), "s"(r.apply), "s"(block_shift));
+    }
+    // ---- what the thread that stores slot (t, w_row) of input row w_col needs beside the sums; lanes of a store run along the
+    // weight rows. Asked for ahead, from addresses that are valid whatever the slot.
+    const uint32_t w_row = (uint32_t)tid & 15u, w_col = (uint32_t)tid >> 4;
+    uint32_t s_row[NT];
+    int s_mat[NT];
+    bool s_ok[NT];
+    _Float16 s_bias[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        s_row[t] = locate(slot_row((uint32_t)t, w_row, s_ok[t]), s_mat[t]);
+        s_bias[t] = fa_norm::load_global<_Float16>(bias0 ? pick3(s_mat[t], bias0, bias1, bias2) + s_row[t] : x_in);
+    }
+    constexpr bool APART = REDUCE_APART<NT, NC, PK>;
+    float *red = reinterpret_cast<float *>(smem + (APART ? NC * 16 * XROW : 0));  // [NW][NT][NC][16][17]; not APART: over the rows once they have been read
+
+    while (true) {
+        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = pass + gridDim.y;
+        if (gamma) {  // x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16; a wave holds whole rows
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                float ss = 0.0f;
+#pragma unroll
+                for (int j = 0; j < PK; ++j) {
+                    const float q = dot8_self(xr[i][j], 0.0f);
+                    ss += (uint32_t)(j * 64 + lane) < n_pieces ? q : 0.0f;
+                }
+                const float inv_rms = fa_norm::inv_rms(fa_norm::wave_sum(ss), inv_k, eps);
+#pragma unroll
+                for (int j = 0; j < PK; ++j) xr[i][j] = fa_norm::scale8(xr[i][j], inv_rms, G_IN_LDS<PK> ? g_lds[j * 64 + lane] : gv[j]);
+            }
+        }
+        f4v_t d[NT][NC];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < NC; ++h) d[t][h] = f4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+        _Float16 s_res[NT], rc[NT], rs[NT];
+        uint32_t r_pos = 0, r_blk = 0;
+        if (!APART && pass != blockIdx.y) __syncthreads();  // the sums have been read
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < PK; ++j) {
+                h8_t v = xr[i][j];
+                if (j >= PK - 2 && (uint32_t)(j * 64 + lane) >= n_pieces) v = h8_t{0, 0, 0, 0, 0, 0, 0, 0};
+                *reinterpret_cast<h8_t *>(smem + (wave + 8 * i) * XROW + (j * 64 + lane) * 16) = v;
+            }
+        if constexpr (WB != 16) {
+            if (pass == blockIdx.y) {
+#pragma unroll
+                for (int i = 0; i < SC_LOADS; ++i) {
+                    uint32_t slot, kb2;
+                    if (!scale_at(i, slot, kb2)) continue;
+                    unsigned short *dst = reinterpret_cast<unsigned short *>(sc_lds) + 2 * kb2 * SLOTS + slot;
+                    dst[0] = (unsigned short)sc_raw[i], dst[SLOTS] = (unsigned short)(sc_raw[i] >> 16);
+                }
+            }
+        }
+        __syncthreads();
+        // what this pass's write stage takes, then the next pass's rows
+        if constexpr (ROPE) {
+            r_pos = r.position_offset + m0 + min(w_col, cols - 1u);
+            const uint32_t tp = min(r_pos, r.table_rows - 1u);  // stay inside the tables
+            const uint32_t hmask = (1u << half_shift) - 1u;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const uint32_t hd = s_row[t] & (2u * hmask + 1u), tc = neox ? (hd & hmask) : (hd >> 1);
+                rc[t] = fa_norm::load_global<_Float16>(r.cos_t + ((size_t)tp << half_shift) + tc);
+                rs[t] = fa_norm::load_global<_Float16>(r.sin_t + ((size_t)tp << half_shift) + tc);
+            }
+            if (r.block_table) r_blk = (uint32_t)r.block_table[block_shift < 32 ? r_pos >> block_shift : r_pos / r.block_size];
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                s_res[t] = fa_norm::load_global<_Float16>(
+                    residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * pick3(s_mat[t], rows0, rows1, rows1) + s_row[t] : x_in);
+        }
+        if (next < n_pass) request_rows(next);
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const uint32_t kb = kb_of(i) + lane_blk;
+            const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
+            const _Float16 *const scp = sc_lds + min(kb, nkb - 1u) * SLOTS + (SUMS ? c * 4 : n);  // (past the last block: a finite scale for zeros)
+            req_t raw[NT];
+            _Float16 sc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                raw[t] = wv[t][i];
+                // (opaque: made f16 here in every pass, not ahead of the passes, where it would wait for the weights)
+                if constexpr (WB != 16) asm volatile("" : "+v"(raw[t]));
+                if constexpr (WIDE) sc[t] = scp[t * 16];
+            }
+#pragma unroll
+            for (int st = 0; st < GB; ++st) {
+                h8_t xb[NC];
+#pragma unroll
+                for (int h = 0; h < NC; ++h) xb[h] = *reinterpret_cast<const h8_t *>(xp + st * 16 + h * 16 * XROW);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    if constexpr (SUMS) {
+                        typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+                        const h4_t s4 = *reinterpret_cast<const h4_t *>(scp + t * 16);
+                        const f4v_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int h = 0; h < NC; ++h) {
+                            const f4v_t blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(W::plain(raw[t]), xb[h], z, 0, 0, 0);
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) d[t][h][q] += blk[q] * (float)s4[q];
+                        }
+                    } else {
+                        const h8_t w = WB == 16 ? W::f16(W::part(raw[t], 0), (_Float16)1.0f) : W::f16(W::part(raw[t], st), sc[t]);
+#pragma unroll
+                        for (int h = 0; h < NC; ++h) d[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[h], d[t][h], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        if (!APART) __syncthreads();  // everyone has read the rows
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < NC; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) red[(((wave * NT + t) * NC + h) * 16 + c * 4 + i) * 17 + n] = d[t][h][i];
+        __syncthreads();
+        if (w_col < NC * 16u) {
+            const int h = (int)(w_col >> 4), cn = (int)(w_col & 15u);
+            _Float16 y2[NT];
+            float s2[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                float s = 0.0f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) s += red[(((w * NT + t) * NC + h) * 16 + w_row) * 17 + cn];
+                s *= alpha;
+                asm volatile("" : "+v"(s_bias[t]));  // (converted here, not ahead of the passes)
+                if (bias0) s += (float)s_bias[t];
+                s2[t] = s, y2[t] = (_Float16)s;
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                if constexpr (ROPE) {
+                    const uint32_t D = 2u << half_shift, half = 1u << half_shift;
+                    // the mate: the same slot of the other tile (NeoX), or the neighbouring slot = the neighbouring lane
+                    const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], 1, 64);
+                    const _Float16 ym = neox ? y2[NT == 2 ? t ^ 1 : 0] : y_adj;
+                    if (!s_ok[t] || w_col >= cols) continue;
+                    const uint32_t hd = s_row[t] & (D - 1u), head = s_row[t] >> (half_shift + 1);
+                    const bool first = neox ? hd < half : (hd & 1u) == 0;
+                    _Float16 y = y2[t];
+                    if (s_mat[t] != 2 && r.apply) y = (_Float16)rope_one((float)y, (float)ym, (float)rc[t], (float)rs[t], first);
+                    _Float16 *dst;
+                    if (s_mat[t] == 0) {
+                        dst = reinterpret_cast<_Float16 *>(out0) + ((size_t)head * m_rows + (m0 + w_col)) * D + hd;
+                    } else {
+                        if (r_pos >= r.capacity) continue;  // never outside the cache
+                        const size_t crow = r.block_table ? (((size_t)r_blk * r.n_kv_heads + head) * r.block_size + (block_shift < 32 ? r_pos & (r.block_size - 1) : r_pos % r.block_size)) * D
+                                                          : ((size_t)head * r.max_seq_len + r_pos) * D;
+                        dst = reinterpret_cast<_Float16 *>(s_mat[t] == 1 ? out1 : out2) + crow + hd;
+                    }
+                    fa_norm::store_global(dst, y);
+                } else {
+                    if (!s_ok[t] || w_col >= cols) continue;
+                    float s = s2[t];
+                    if (residual) s += (float)s_res[t] * beta;
+                    const uint32_t N = pick3(s_mat[t], rows0, rows1, rows1);
+                    fa_norm::store_global(pick3(s_mat[t], out0, out1, out2) + (size_t)(m0 + w_col) * N + s_row[t], (_Float16)s);
+                }
+            }
+        }
+        if (next >= n_pass) break;
+        pass = next;
+    }
+}
+
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
+fa_status launch_one(FaLaunchScope &scope, dim3 grid, const PanelDev &a) {
+    constexpr int lds = lds_bytes<WB, NT, NC, PK>();
+    static std::atomic<uint64_t> allowed{0};  // devices this kernel's LDS size has been asked for on (the calls are idempotent)
+    const uint64_t bit = 1ull << (scope.ctx->device & 63);
+    if (!(allowed.load(std::memory_order_acquire) & bit)) {
+        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        allowed.fetch_or(bit, std::memory_order_release);
+    }
+    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS>, grid, dim3(NTHREADS), lds, a);
+    return FA_OK;
+}
+template <int WB, int NT, int NC, bool SUMS>
+fa_status launch_pk(FaLaunchScope &scope, bool rope, uint32_t pk, dim3 grid, const PanelDev &a) {
+    if (pk <= 2) return rope ? launch_one<WB, NT, NC, 2, true, SUMS>(scope, grid, a) : launch_one<WB, NT, NC, 2, false, SUMS>(scope, grid, a);
+    if (NC == 2 || pk <= 4) return rope ? launch_one<WB, NT, NC, 4, true, SUMS>(scope, grid, a) : launch_one<WB, NT, NC, 4, false, SUMS>(scope, grid, a);
+    return rope ? launch_one<WB, NT, 1, 6, true, SUMS>(scope, grid, a) : launch_one<WB, NT, 1, 6, false, SUMS>(scope, grid, a);  // (16 rows per pass: registers)
+}
+template <int WB>
+fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a) {
+    if constexpr (WB != 16) {
+        if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true>(scope, rope, pk, grid, a);
+    }
+    if (nt == 1) return nc == 1 ? launch_pk<WB, 1, 1, false>(scope, rope, pk, grid, a) : launch_pk<WB, 1, 2, false>(scope, rope, pk, grid, a);
+    return nc == 1 ? launch_pk<WB, 2, 1, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 2, false>(scope, rope, pk, grid, a);
+}
+
+}  // namespace fa_panel

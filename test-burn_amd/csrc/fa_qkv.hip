@@ -24,6 +24,7 @@
 // consumer of the attention output.
 #include "fa_internal.h"
 #include "fa_norm.h"
+#include "fa_panel.h"
 #include "fa_qkv_rope.h"
 #include <atomic>
 #include <type_traits>
@@ -388,346 +389,90 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
     }
 }
 
-// The same weight stream for 12 to 32 input rows (the reference's default prefill chunk is 32 rows): one launch where the
-// GEMM route takes three (norm, split GEMM, finish) for a launch that is still all weight stream. Differences from the
-// kernel above:
-//   * the input rows do not fit a compute unit's LDS (32 x 3072 f16 = 196 KB), and no wave needs them all: wave w
-//     multiplies its own feature blocks only (an eighth of them), so it keeps just those features of all 32 rows in registers, in
-//     the layout of the matrix instruction's second operand (XJ blocks x 2 row halves x 16 bytes per lane);
-//   * RMSNorm: every wave sums the squares of its slice per row, the eight partial sums meet in LDS, and the wave scales
-//     its slice (the norm's weights are staged in LDS once); the same roundings as above;
-//   * one workgroup per compute unit takes up to 32 weight rows as two 16-row tiles against the two 16-row halves of the
-//     input: four accumulators, and every weight of the workgroup is requested before the first is used - a fixed
-//     number of requests per wave, so that the compiler's waits are exact.
-// XJ = feature blocks per wave = k_dim / 256 (8 or 12: k_dim 2048, 3072; 16 spills); F16 weights.
-// ROPE: the write stage is KvPrepFused (kv_prep_fused.metal:45-122) on the f16 values FusedQkv would store - rotation of Q
-// and K, Q to q_rot [H, m, D], K and V to their cache rows. A workgroup then takes whole rotation pairs: adjacent weight
-// rows (2i, 2i + 1), or - NeoX pairing - tile 0 = the rows of up to 16 pairs in the first half of a head and tile 1 = their
-// mates half a head on, so that the thread that stores an element finds its mate in the workgroup's own partial sums.
-struct Rows32Dev {
-    QkvDev q;
-    RopeDev r;
-};
-template <int XJ, bool ROPE>
-__global__ void __launch_bounds__(QKV_NT, 1) fused_qkv_rows32_kernel(Rows32Dev a_by_value) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    static_assert(std::is_trivially_copyable<Rows32Dev>::value, "read as raw bytes from the argument block, where it is the first member");
-    const Rows32Dev &args = *(const Rows32Dev *)__builtin_amdgcn_kernarg_segment_ptr();
-    const QkvDev &a = args.q;
-    (void)a_by_value;
-    const unsigned char *const w0 = reinterpret_cast<const unsigned char *>(a.w[0]), *const w1 = reinterpret_cast<const unsigned char *>(a.w[1]),
-                        *const w2 = reinterpret_cast<const unsigned char *>(a.w[2]);
-    const uint32_t rows0 = a.rows[0], rows1 = a.rows[1], rows2 = a.rows[2];
-    const __half *const x_in = a.x, *const gamma = a.gamma;
-    const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical;
-    asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(rows0), "s"(rows1), "s"(rows2), "s"(x_in), "s"(gamma), "s"(K), "s"(m_rows),
-                 "s"(rows_per_wg), "s"(canonical_u));
-    const bool canonical = canonical_u != 0;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, c = lane >> 4;
-    const uint32_t total_rows = rows0 + rows1 + rows2;
-    const uint32_t row_begin = blockIdx.x * rows_per_wg;
-    const uint32_t row_end = min(total_rows, row_begin + rows_per_wg);
-    if (row_begin >= row_end) return;
-    const uint32_t m0 = blockIdx.y * 32u, cols = min(32u, m_rows - m0);
-    // ROPE (rows_per_wg is even, the matrices hold whole heads): the pairing and the head size
-    uint32_t neox = 0, half_shift = 0, pair_begin = 0, pair_end = 0;
-    if constexpr (ROPE) {
-        const uint32_t normal = args.r.normal, head_dim = args.r.head_dim;
-        asm volatile("" ::"s"(normal), "s"(head_dim));
-        neox = normal ? 0u : 1u, half_shift = head_dim == 128 ? 6u : 5u;
-        pair_begin = row_begin >> 1, pair_end = row_end >> 1;
-    }
-    // Weight row of slot (tile t, row n of the tile) across the three matrices laid end to end; a slot past the workgroup's
-    // last row gives the workgroup's first row with valid = false.
-    auto slot_row = [&](uint32_t t, uint32_t n_, bool &valid) __attribute__((always_inline)) -> uint32_t {
-        if (ROPE && neox) {
-            const uint32_t p = pair_begin + n_, pv = p < pair_end ? p : pair_begin;
-            valid = p < pair_end;
-            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + (t << half_shift);
-        }
-        const uint32_t gr = row_begin + 16u * t + n_;
-        valid = gr < row_end;
-        return valid ? gr : row_begin;
-    };
-    _Float16 *g_lds = reinterpret_cast<_Float16 *>(smem);                   // [K] the norm's weights
-    float *ss_lds = reinterpret_cast<float *>(smem + (size_t)K * 2);        // [QKV_NW][32] sums of squares of the waves' slices
-    float *red = ss_lds + QKV_NW * 32;                                      // [QKV_NW][2 tiles][2 halves][16][17]
-
-    // The norm's weights (one 16-byte piece per thread and pass) and this wave's slice of the input rows, before any weight
-    // is requested: a compute unit's requests return in order.
-    constexpr int GPRE = 2;  // pieces per thread: k_dim up to 8192
-    h8_t g0[GPRE];
-#pragma unroll
-    for (int j = 0; j < GPRE; ++j) {
-        const uint32_t k8 = min((uint32_t)tid + j * QKV_NT, K / 8 - 1);
-        g0[j] = *reinterpret_cast<const h8_t *>((gamma ? gamma : x_in) + k8 * 8);
-    }
-    // Wave w takes the feature blocks 2w, 2w + 1, 2w + 16, 2w + 17, ...: adjacent pairs, so that the two requests for a
-    // pair touch the same 16 cache lines one after the other (a request of the operand's shape covers 64 bytes of each of
-    // 16 rows - half a line; with blocks w, w + 8, ... the other halves belonged to the next wave and every line came from
-    // L2 twice).
-    auto kb_of = [&](int j) __attribute__((always_inline)) -> uint32_t { return 2u * (uint32_t)wave + 16u * (uint32_t)(j >> 1) + (uint32_t)(j & 1); };
-    h8_t xs[XJ][2];
-#pragma unroll
-    for (int j = 0; j < XJ; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t row = min(m0 + 16u * h + (uint32_t)n, m_rows - 1);  // (rows past the last are zeroed below)
-            xs[j][h] = *reinterpret_cast<const h8_t *>(x_in + (size_t)row * K + kb_of(j) * 32u + c * 8);
-        }
-    // Every weight of the workgroup: tile t is the weight rows row_begin + 16 t .., lane (n, c) takes features 8c .. 8c + 7
-    // of block kb for row n of the tile (a row past the workgroup's last reads the first row's block: never written).
-    h8_t wv[2][XJ];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        bool slot_valid;
-        uint32_t lrow = slot_row((uint32_t)t, (uint32_t)n, slot_valid);
-        int mat = 0;
-        if (lrow >= rows0) {
-            lrow -= rows0, mat = 1;
-            if (lrow >= rows1) lrow -= rows1, mat = 2;
-        }
-        const unsigned char *base = pick3(mat, w0, w1, w2);
-        const uint32_t N = pick3(mat, rows0, rows1, rows1);
-        // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
-        const unsigned char *p0 = base + (canonical ? (size_t)lrow * 32 + c * 8 : (size_t)lrow * K + c * 8) * 2;
-        const size_t kb_stride = (canonical ? (size_t)N * 32 : 32) * 2;
-#pragma unroll
-        for (int j = 0; j < XJ; ++j)
-            wv[t][j] = __builtin_nontemporal_load(reinterpret_cast<const h8_t *>(p0 + (size_t)kb_of(j) * kb_stride));
-    }
-    const float eps = a.eps;
-    if (gamma) {
-#pragma unroll
-        for (int j = 0; j < GPRE; ++j) {
-            const uint32_t k8 = (uint32_t)tid + j * QKV_NT;
-            if (k8 < K / 8) *reinterpret_cast<h8_t *>(g_lds + k8 * 8) = g0[j];
-        }
-        // sums of squares of the slice, per input row: over the blocks, then over the four lanes that share a row
-        float ss[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int j = 0; j < XJ; ++j)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) ss[h] += (float)xs[j][h][i] * (float)xs[j][h][i];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            ss[h] += __shfl_xor(ss[h], 16, 64);
-            ss[h] += __shfl_xor(ss[h], 32, 64);
-            if (c == 0) ss_lds[wave * 32 + 16 * h + n] = ss[h];
-        }
-        __syncthreads();
-        float inv_rms[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float tot = 0.0f;
-#pragma unroll
-            for (int w = 0; w < QKV_NW; ++w) tot += ss_lds[w * 32 + 16 * h + n];
-            inv_rms[h] = rsqrtf(tot / (float)K + eps);
-        }
-        // (the plain form of the scaling, five instructions per element, was a quarter of the launch: every workgroup scales all 32 rows)
-#pragma unroll
-        for (int j = 0; j < XJ; ++j) {
-            const h8_t g = *reinterpret_cast<const h8_t *>(g_lds + kb_of(j) * 32u + c * 8);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) xs[j][h] = fa_norm::scale8(xs[j][h], inv_rms[h], g);
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-        if (16u * h + (uint32_t)n >= cols) {
-#pragma unroll
-            for (int j = 0; j < XJ; ++j) xs[j][h] = h8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        }
-    // what the write stage takes, while the weights are on their way
-    const __half *const residual = a.residual;
-    const __half *const bias0 = a.bias[0], *const bias1 = a.bias[1], *const bias2 = a.bias[2];
-    __half *const out0 = a.out[0], *const out1 = a.out[1], *const out2 = a.out[2];
-    const float alpha = a.alpha, beta = a.beta;
-    asm volatile("" ::"s"(residual), "s"(bias0), "s"(bias1), "s"(bias2), "s"(out0), "s"(out1), "s"(out2), "s"(alpha), "s"(beta));
-    // ROPE: thread (row = tid % 16, col = tid / 16) stores the elements of slot row of both tiles for input row col, rows
-    // fastest (the lanes of a store cover consecutive elements of a head). Its two table entries and, in a paged cache, its
-    // block are requested here, behind the weights, from addresses that are valid whatever the slot.
-    const uint32_t w_row = (uint32_t)tid & 15u, w_col = (uint32_t)tid >> 4;
-    _Float16 rc[2] = {(_Float16)0.0f, (_Float16)0.0f}, rs[2] = {(_Float16)0.0f, (_Float16)0.0f};
-    uint32_t r_pos = 0, r_blk = 0;
-    uint32_t n_kv_heads = 0, max_seq_len = 0, block_size = 1, capacity = 0, apply = 0;
-    bool paged = false;
-    if constexpr (ROPE) {
-        const __half *const cos_t = args.r.cos_t, *const sin_t = args.r.sin_t;
-        const int32_t *const block_table = args.r.block_table;
-        const uint32_t position_offset = args.r.position_offset, table_rows = args.r.table_rows;
-        block_size = args.r.block_size, n_kv_heads = args.r.n_kv_heads, max_seq_len = args.r.max_seq_len, capacity = args.r.capacity;
-        apply = args.r.apply;
-        asm volatile("" ::"s"(cos_t), "s"(sin_t), "s"(block_table), "s"(position_offset), "s"(table_rows), "s"(block_size), "s"(n_kv_heads),
-                     "s"(max_seq_len), "s"(capacity), "s"(apply));
-        paged = block_table != nullptr;
-        r_pos = position_offset + m0 + min(w_col, cols - 1u);
-        const uint32_t tp = min(r_pos, table_rows - 1u);  // stay inside the tables
-        const uint32_t hmask = (1u << half_shift) - 1u;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            bool v_;
-            const uint32_t hd = slot_row((uint32_t)t, w_row, v_) & (2u * hmask + 1u);
-            const uint32_t tc = neox ? (hd & hmask) : (hd >> 1);
-            rc[t] = *reinterpret_cast<const _Float16 *>(cos_t + ((size_t)tp << half_shift) + tc);
-            rs[t] = *reinterpret_cast<const _Float16 *>(sin_t + ((size_t)tp << half_shift) + tc);
-        }
-        if (block_table) r_blk = (uint32_t)block_table[r_pos / block_size];
-    }
-
-    f4v_t d[2][2] = {{{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}, {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}};
-#pragma unroll
-    for (int j = 0; j < XJ; ++j)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) d[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t][j], xs[j][h], d[t][h], 0, 0, 0);
-    // The eight waves' partial tiles are summed in wave order, the write stage applied, rows rounded once.
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) red[((((size_t)wave * 2 + t) * 2 + h) * 16 + c * 4 + i) * 17 + n] = d[t][h][i];
-    __syncthreads();
-    if constexpr (ROPE) {
-        const uint32_t D = 2u << half_shift, half = 1u << half_shift;
-        const int h = (int)(w_col >> 4), cn = (int)(w_col & 15u);
-        auto tile_sum = [&](uint32_t t, uint32_t row) __attribute__((always_inline)) -> float {
-            float s = 0.0f;
-#pragma unroll
-            for (int w = 0; w < QKV_NW; ++w) s += red[((((size_t)w * 2 + t) * 2 + h) * 16 + row) * 17 + cn];
-            return s;
-        };
-        // the f16 values FusedQkv stores, of the thread's slot in both tiles (of the workgroup's first row where the slot is
-        // past its last: every lane takes part in the exchange below)
-        _Float16 y2[2];
-        uint32_t lrow2[2];
-        int mat2[2];
-        bool valid2[2];
-#pragma unroll
-        for (uint32_t t = 0; t < 2; ++t) {
-            uint32_t lrow = slot_row(t, w_row, valid2[t]);
-            int mat = 0;
-            if (lrow >= rows0) {
-                lrow -= rows0, mat = 1;
-                if (lrow >= rows1) lrow -= rows1, mat = 2;
-            }
-            const __half *bias = pick3(mat, bias0, bias1, bias2);
-            float s = tile_sum(t, w_row) * alpha;
-            if (bias) s += __half2float(bias[lrow]);
-            y2[t] = (_Float16)s, lrow2[t] = lrow, mat2[t] = mat;
-        }
-#pragma unroll
-        for (uint32_t t = 0; t < 2; ++t) {
-            // the mate: the same slot of the other tile (NeoX), or the neighbouring slot = the neighbouring lane
-            const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], 1, 64);
-            const _Float16 ym = neox ? y2[t ^ 1u] : y_adj;
-            if (!valid2[t] || w_col >= cols) continue;
-            const uint32_t lrow = lrow2[t];
-            const int mat = mat2[t];
-            const uint32_t hd = lrow & (D - 1u), head = lrow >> (half_shift + 1);
-            const bool first = neox ? hd < half : (hd & 1u) == 0;
-            _Float16 y = y2[t];
-            if (mat != 2 && apply) y = (_Float16)rope_one((float)y, (float)ym, (float)rc[t], (float)rs[t], first);
-            _Float16 *dst;
-            if (mat == 0) {
-                dst = reinterpret_cast<_Float16 *>(out0) + ((size_t)head * m_rows + (m0 + w_col)) * D + hd;
-            } else {
-                if (r_pos >= capacity) continue;  // never outside the cache
-                const size_t crow = paged ? (((size_t)r_blk * n_kv_heads + head) * block_size + r_pos % block_size) * D
-                                          : ((size_t)head * max_seq_len + r_pos) * D;
-                dst = reinterpret_cast<_Float16 *>(mat == 1 ? out1 : out2) + crow + hd;
-            }
-            *dst = y;
-        }
-        return;
-    }
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-        // (tile, input row, weight row of the tile), weight rows fastest: the lanes of a store cover consecutive outputs
-        const int t = pass, row = tid & 15, col = tid >> 4, h = col >> 4, cn = col & 15;
-        const uint32_t gr = row_begin + 16u * t + (uint32_t)row;
-        if (gr < row_end && (uint32_t)col < cols) {
-            float s = 0.0f;
-#pragma unroll
-            for (int w = 0; w < QKV_NW; ++w) s += red[((((size_t)w * 2 + t) * 2 + h) * 16 + row) * 17 + cn];
-            uint32_t lrow = gr;
-            int mat = 0;
-            if (lrow >= rows0) {
-                lrow -= rows0, mat = 1;
-                if (lrow >= rows1) lrow -= rows1, mat = 2;
-            }
-            const __half *bias = pick3(mat, bias0, bias1, bias2);
-            __half *out = pick3(mat, out0, out1, out2);
-            const uint32_t N = pick3(mat, rows0, rows1, rows1);
-            s *= alpha;
-            if (bias) s += __half2float(bias[lrow]);
-            if (residual) s += __half2float(residual[(size_t)(m0 + col) * N + lrow]) * beta;
-            out[(size_t)(m0 + col) * N + lrow] = __float2half(s);
-        }
-    }
-}
-
 }  // namespace
 
-// Whether a FusedQkv / MatMul launch goes to the one-launch kernel for 12 to 32 input rows: F16 weights, k_dim 2048 or 3072
-// (at 4096 a wave's slice and its weights no longer fit the registers), at most 32 weight rows per compute unit; an explicit
-// GEMM threshold (fa_set_gemm_min_m) wins.
+// How a FusedQkv / MatMul launch runs on the panel kernel (fa_panel.h): 16-row tiles of weight rows per workgroup, 16-row groups
+// of input rows per pass, weight rows per workgroup, workgroups along the passes.
+struct PanelPlan {
+    uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y;
+};
+static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope, bool neox_rope) {
+    PanelPlan p;
+    const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
+    p.pk = ceil_div_u32(l.k_dim, 512), p.nc = l.m <= 16 || p.pk > 4 ? 1u : 2u, p.n_pass = ceil_div_u32(l.m, 16 * p.nc);
+    // Weight rows per workgroup: what a pass costs is mostly its input rows, whatever the weight rows, so as few passes as
+    // possible one after the other; of equal choices the fewest weight rows.
+    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
+    uint32_t best = 0xffffffffu;
+    const uint32_t least = ceil_div_u32(total_rows, n_cus) < 32 ? (ceil_div_u32(total_rows, n_cus) + 1) & ~1u : 32u;
+    for (uint32_t rpw : {least, 16u, 32u}) {
+        const uint32_t gx = ceil_div_u32(total_rows, rpw), nt = neox_rope || rpw > 16 ? 2u : 1u;
+        const uint32_t slots = n_cus * (fa_panel::two_per_cu(nt, p.nc, p.pk, rope) ? 2u : 1u);
+        uint32_t gy = slots / gx;
+        gy = gy < 1 ? 1u : gy > p.n_pass ? p.n_pass : gy;
+        const uint32_t cost = ceil_div_u32(gx * gy, slots) * ceil_div_u32(p.n_pass, gy) * (4 + nt);
+        if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy;
+    }
+    return p;
+}
+
+// Whether a FusedQkv / MatMul launch goes to the panel kernel: rows of up to 3072 features, from two input rows (four layers of the
+// Llama-3.2-3B block with 2 / 4 / 8 / 11 rows: 113 / 113 / 115 / 117 us against 120 / 128 / 137 / 155 with the kernel for up to 16
+// rows) to as many as it is measured to beat the GEMM with; an explicit GEMM threshold (fa_set_gemm_min_m) wins.
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
-    constexpr uint32_t ROWS32_MIN_M_DEFAULT = 12;
+    constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
-    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    const uint32_t xj = l.k_dim / 256, rpw = ceil_div_u32(total_rows, n_cus);
-    const uint32_t min_m = ctx->qkv_rows32_min_m ? ctx->qkv_rows32_min_m : ROWS32_MIN_M_DEFAULT;
-    return l.scales[0] == nullptr && l.weight_bits == 16 && l.k_dim % 256 == 0 && (xj == 8 || xj == 12) && rpw <= 32 && l.m >= min_m &&
-           l.m <= 32 && !(ctx->gemm_min_m && l.m >= ctx->gemm_min_m) && aligned16(l.x) && aligned16(l.w[0]) && aligned16(l.w[1]) &&
-           aligned16(l.w[2]) && aligned16(l.gamma);
+    const uint32_t min_m = ctx->qkv_rows32_min_m ? ctx->qkv_rows32_min_m : PANEL_MIN_M_DEFAULT;
+    const uint32_t max_m = l.k_dim <= 1024 ? 512u : l.k_dim <= 2048 ? 128u : 64u;
+    if (min_m > 32 || l.m < min_m || l.m > max_m || l.k_dim > 3072 || l.k_dim % 32 != 0) return false;
+    if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
+    return aligned16(l.x) && aligned16(l.w[0]) && aligned16(l.w[1]) && aligned16(l.w[2]) && aligned16(l.gamma);
 }
 
-static size_t rows32_lds_bytes(uint32_t k_dim) {
-    return (size_t)k_dim * 2 + (size_t)QKV_NW * 32 * sizeof(float) + (size_t)QKV_NW * 2 * 2 * 16 * 17 * sizeof(float);
-}
-
-// FusedQkv + KvPrepFused of a chunk of 12 to 32 rows as one launch.
-fa_status fa_launch_fused_qkv_rows32_rope(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch &r) {
-    if (!fa_qkv_rows32_takes(ctx, l)) return fa_fail(FA_ERR_INVALID_OPERATION, "fa_launch_fused_qkv_rows32_rope: not a launch of the 32-row weight stream");
-    if (!(r.head_dim == 64 || r.head_dim == 128))
-        return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "FusedQkv with the KvPrepFused write stage supports head_dim 64 or 128, got %u", r.head_dim);
-    if (l.n_dim != r.n_heads * r.head_dim || l.n_kv != r.n_kv_heads * r.head_dim)
-        return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: n_dim %u / n_kv %u are not n_heads %u / n_kv_heads %u x head_dim %u", l.n_dim,
-                       l.n_kv, r.n_heads, r.n_kv_heads, r.head_dim);
-    if (l.residual) return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "the KvPrepFused write stage takes no residual");
-    if (r.table_rows == 0) return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: empty RoPE tables");
-    Rows32Dev args;
-    memset(&args, 0, sizeof(args));
-    QkvDev &a = args.q;
-    for (int i = 0; i < 3; ++i) a.w[i] = l.w[i], a.bias[i] = l.bias[i];
-    a.out[0] = r.q_rot, a.out[1] = r.k_cache, a.out[2] = r.v_cache;
-    a.rows[0] = l.n_dim, a.rows[1] = l.n_kv, a.rows[2] = l.n_kv;
-    a.x = l.x, a.gamma = l.gamma, a.k_dim = l.k_dim, a.m = l.m, a.eps = l.eps, a.canonical = l.canonical ? 1u : 0u;
-    a.alpha = l.alpha, a.beta = l.beta;
-    RopeDev &d = args.r;
-    d.cos_t = r.cos_t, d.sin_t = r.sin_t, d.block_table = r.block_table;
-    d.on = 1, d.head_dim = r.head_dim, d.n_kv_heads = r.n_kv_heads, d.position_offset = r.position_offset;
-    d.max_seq_len = r.max_seq_len, d.block_size = r.block_size ? r.block_size : 1, d.capacity = r.capacity;
-    d.table_rows = r.table_rows, d.normal = r.rope_normal ? 1u : 0u, d.apply = r.apply_rope ? 1u : 0u;
-    // whole pairs per workgroup: an even number of weight rows, at most 32 (the matrices hold whole heads, so the total is even)
-    const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
-    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    const uint32_t rpw = 2 * ceil_div_u32(total_rows / 2, n_cus);
-    if (rpw > 32) return fa_fail(FA_ERR_INVALID_OPERATION, "fa_launch_fused_qkv_rows32_rope: %u weight rows per workgroup", rpw);
-    a.rows_per_wg = rpw, a.cols_per_pass = 32, a.x_stride = 0;
-    const uint32_t xj = l.k_dim / 256;
-    const dim3 grid(ceil_div_u32(total_rows, rpw), 1);
-    FaLaunchScope scope(ctx, "fused_qkv_rows32_rope_kernel", true);
-    if (xj == 8) scope.launch(fused_qkv_rows32_kernel<8, true>, grid, dim3(QKV_NT), rows32_lds_bytes(l.k_dim), args);
-    else scope.launch(fused_qkv_rows32_kernel<12, true>, grid, dim3(QKV_NT), rows32_lds_bytes(l.k_dim), args);
+static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch *rope) {
+    fa_panel::PanelDev a;
+    memset(&a, 0, sizeof(a));
+    for (int i = 0; i < 3; ++i)
+        a.w[i] = reinterpret_cast<const unsigned char *>(l.w[i]), a.scales[i] = l.scales[i], a.bias[i] = l.bias[i], a.out[i] = l.out[i];
+    a.rows0 = l.n_dim, a.rows1 = l.n_kv, a.rows2 = l.n_kv, a.total_rows = l.n_dim + 2 * l.n_kv;
+    a.x = l.x, a.gamma = l.gamma, a.residual = l.residual, a.k_dim = l.k_dim, a.m = l.m, a.canonical = l.canonical ? 1u : 0u;
+    a.eps = l.eps, a.inv_k = 1.0f / (float)l.k_dim, a.alpha = l.alpha, a.beta = l.beta;
+    if (rope) {
+        const QkvRopeLaunch &r = *rope;
+        if (!(r.head_dim == 64 || r.head_dim == 128))
+            return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "FusedQkv with the KvPrepFused write stage supports head_dim 64 or 128, got %u", r.head_dim);
+        if (l.n_dim != r.n_heads * r.head_dim || l.n_kv != r.n_kv_heads * r.head_dim)
+            return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: n_dim %u / n_kv %u are not n_heads %u / n_kv_heads %u x head_dim %u", l.n_dim,
+                           l.n_kv, r.n_heads, r.n_kv_heads, r.head_dim);
+        if (l.residual) return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "the KvPrepFused write stage takes no residual");
+        if (r.table_rows == 0) return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: empty RoPE tables");
+        a.out[0] = r.q_rot, a.out[1] = r.k_cache, a.out[2] = r.v_cache;
+        RopeDev &d = a.r;
+        d.cos_t = r.cos_t, d.sin_t = r.sin_t, d.block_table = r.block_table;
+        d.on = 1, d.head_dim = r.head_dim, d.n_kv_heads = r.n_kv_heads, d.position_offset = r.position_offset;
+        d.max_seq_len = r.max_seq_len, d.block_size = r.block_size ? r.block_size : 1, d.capacity = r.capacity;
+        d.table_rows = r.table_rows, d.normal = r.rope_normal ? 1u : 0u, d.apply = r.apply_rope ? 1u : 0u;
+        a.block_shift = (d.block_size & (d.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(d.block_size) : 32u;
+    }
+    const PanelPlan p = panel_plan(ctx, l, rope != nullptr, rope && !rope->rope_normal);
+    a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass;
+    const uint32_t nkb = l.k_dim / 32, half_nkb = (nkb + 1) / 2;
+    a.rcp_half_nkb = half_nkb > 1 ? (uint32_t)((1ull << 32) / half_nkb) + 1u : 0u, a.scale_pairs = nkb % 2 == 0 ? 1u : 0u;
+    for (int i = 0; i < 3; ++i)
+        if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) a.scale_pairs = 0;
+    FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
+    const bool sums = l.m < FA_GEMM_MIN_M_DEFAULT;  // (of interest to block-quantised weights only: the arithmetic, see fa_panel.h)
+    const dim3 grid(p.grid_x, p.grid_y);
+    if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
+    else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
+    else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
     return scope.finish();
+}
+
+// FusedQkv + KvPrepFused of a chunk that the panel kernel takes, as one launch.
+fa_status fa_launch_fused_qkv_rows32_rope(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch &r) {
+    if (!fa_qkv_rows32_takes(ctx, l)) return fa_fail(FA_ERR_INVALID_OPERATION, "fa_launch_fused_qkv_rows32_rope: not a launch of the panel kernel");
+    return launch_panel(ctx, l, &r);
 }
 
 fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_stream_only) {
@@ -755,23 +500,9 @@ fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_
                          aligned16(l.w[2]) && aligned16(l.gamma);
     const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    // A chunk of up to 32 input rows (the reference's default prefill chunk) is still a weight stream: one launch of the
-    // kernel that keeps each wave's slice of the input rows in registers, where the GEMM route takes three launches.
-    {
-        const uint32_t xj = l.k_dim / 256, rpw = ceil_div_u32(total_rows, n_cus);
-        const bool ok = fa_qkv_rows32_takes(ctx, l);
-        if (ok) {
-            a.rows_per_wg = rpw, a.cols_per_pass = 32, a.x_stride = 0;
-            Rows32Dev args;
-            memset(&args, 0, sizeof(args));
-            args.q = a;
-            const dim3 grid(ceil_div_u32(total_rows, rpw), 1);
-            FaLaunchScope scope(ctx, l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
-            if (xj == 8) scope.launch(fused_qkv_rows32_kernel<8, false>, grid, dim3(QKV_NT), rows32_lds_bytes(l.k_dim), args);
-            else scope.launch(fused_qkv_rows32_kernel<12, false>, grid, dim3(QKV_NT), rows32_lds_bytes(l.k_dim), args);
-            return scope.finish();
-        }
-    }
+    // A chunk of a few dozen input rows (the reference's default prefill chunk is 32) is still a weight stream: one launch where
+    // the GEMM route takes three.
+    if (fa_qkv_rows32_takes(ctx, l)) return launch_panel(ctx, l, nullptr);
     if (!weight_stream_only && gemm_ok && l.m >= (ctx->gemm_min_m ? ctx->gemm_min_m : GEMM_MIN_M_DEFAULT)) return fa_launch_fused_qkv_gemm(ctx, l);
     // Workgroups: a multiple of the CU count, enough of them that a workgroup's rows fit one 16-row tile where the
     // matrix allows (5120 rows, 256 CUs: 512 workgroups of 10 rows, two resident per CU - every CU requests the same

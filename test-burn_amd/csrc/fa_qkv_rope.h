@@ -32,6 +32,6 @@ __device__ __forceinline__ float rope_one(float x, float mate, float c, float s,
 
 // The GEMM of fa_launch_fused_qkv_gemm with that write stage (l.out[] is ignored). head_dim must be 64 or 128.
 fa_status fa_launch_fused_qkv_gemm_rope(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch &r);
-// The one-launch weight stream for 12 to 32 input rows (fa_qkv_rows32_takes) with that write stage: a workgroup takes whole
-// rotation pairs. head_dim must be 64 or 128.
+// The one-launch kernel for short chunks (fa_qkv_rows32_takes, fa_panel.h) with that write stage: a workgroup takes whole rotation
+// pairs. head_dim must be 64 or 128.
 fa_status fa_launch_fused_qkv_rows32_rope(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch &r);

@@ -1,0 +1,74 @@
+"""GPU parity of the one-launch kernel for chunks of input rows (FusedQkv and MatMul, fa_panel.h) where its split of the work
+ends: row lengths around its 512-feature pieces, an odd number of feature blocks, weight rows that do not fill a tile or straddle
+the matrices, one and several passes, passes spread over workgroups, the block-quantised arithmetic on either side of 12 rows.
+Against the oracle with the bars of test_gpu_qkv.py."""
+import numpy as np
+import pytest
+
+import foundry_attn as fa
+import orc
+from gpu_util import announce, ctx
+from test_gpu_qkv import _close, _data
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,layout", [
+    (32, 8, 8, 2, 1),          # one block
+    (96, 40, 24, 11, 0),       # an odd number of blocks; the last row count of the weight stream's arithmetic
+    (1024, 200, 40, 12, 1),    # the longest rows of the two-piece form, the first row count of the GEMM's arithmetic
+    (1056, 72, 8, 16, 1),      # 33 blocks: just past it, 16 rows exactly
+    (896, 264, 72, 33, 0),     # two passes, the second of one row
+    (896, 64, 32, 100, 1),     # passes spread over workgroups
+    (2048, 40, 16, 17, 0),
+    (2080, 40, 16, 47, 1),     # 65 blocks: 16 rows per pass
+    (3072, 24, 8, 5, 0),       # the longest rows it takes
+    (3072, 4136, 1024, 20, 1), # as many weight rows per compute unit as two tiles hold, two passes
+])
+def test_chunk_in_one_launch(K, N, NK, m, layout, weights):
+    announce("panel", K, N, NK, m, layout, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + N + m)
+    x, g, ws, bs = _data(rng, K, N, NK, m)
+    res = rng.uniform(-1, 1, (m, N)).astype(np.float16)
+    dx, dg, db, dres, dout = f.array(x), f.array(g), [f.array(b) for b in bs], f.array(res), f.zeros((m, N))
+    outs = [f.zeros((m, n)) for n in (N, NK, NK)]
+    scales, dev_s = None, []
+    if weights == "f16":
+        dev_w = [f.array(orc.to_canonical(w) if layout else w.reshape(-1)) for w in ws]
+        arg = [w.arg() for w in dev_w]
+        full = ws
+    else:
+        quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
+        dev_s = [f.array(s) for _, s in quant]
+        scales = [s.arg() for s in dev_s]
+        flat = [orc.to_canonical(q) if layout else q.reshape(-1) for q, _ in quant]
+        dev_w = [f.array(q if weights == "q8" else orc.pack_q4_0(q)) for q in flat]
+        arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev_w, (N, NK, NK))]
+        full = [orc.dequantize_blocks(q, s) for q, s in quant]
+    if weights != "f16" and m < 12:
+        want = orc.fused_qkv_q8(x, [q for q, _ in quant], [s for _, s in quant], gamma=g, biases=bs)
+        want_mm = orc.matmul_gemv_q8(x, quant[0][0], quant[0][1], bs[0], res, 0, 32, 0.5, 0.75)
+    else:
+        want = orc.fused_qkv(x, *full, gamma=g, biases=bs, layout=0)
+        want_mm = orc.matmul_gemv(x, full[0], bs[0], res, 0, 32, 0.5, 0.75)
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, gamma=dg.arg(), biases=[b.arg() for b in db],
+                    layout=layout, scales=scales)
+        f.matmul(dx.arg(), arg[0], dout.arg(), m, N, K, bias=db[0].arg(), c=dres.arg(), transpose_b=not layout, alpha=0.5,
+                 beta=0.75, b_scales=scales[0] if scales else None)
+        f.synchronize()
+        assert f.profile_query("fused_qkv_rows32_kernel")[0] == 1 and f.profile_query("matmul_rows32_kernel")[0] == 1
+    finally:
+        f.profile_enable(False)
+    for o, w, name in zip(outs, want, "qkv"):
+        got = o.download()
+        assert np.all(np.isfinite(got)), name
+        assert _close(got, w, K), (name, float(np.max(np.abs(got.astype(np.float64) - w.astype(np.float64)))))
+    got, w = dout.download().astype(np.float64), want_mm.astype(np.float64)
+    assert np.all(np.abs(got - w) <= 2 * np.maximum(np.abs(w), 2.0 ** -10) * 2.0 ** -10 + 1e-4), float(np.max(np.abs(got - w)))
+    for b in [dx, dg, dres, dout] + db + outs + dev_w + dev_s:
+        b.free()
