@@ -538,17 +538,17 @@ fa_status fa_matmul(fa_ctx *ctx, const fa_tensor_arg *a, const fa_tensor_arg *b,
 /* Tuning override for fa_fused_qkv and fa_matmul: the number of input rows m from which the tiled
  * GEMM runs instead of passes of 16 rows over the weight stream (the reference makes the same choice between GemvV2
  * and its GEMM by m, src/metals/matmul.rs:190-239). 0 = the library's default. With a gamma the GEMM writes the
- * normalised input (m * k_dim f16) into the context's workspace, which also holds the f32 partial tiles of short chunks
+ * normalised input (m * k_dim f16) into the context's workspace, which also holds f32 partial tiles where k_dim is no multiple of 64
  * (k_splits * m * (n_dim + 2 n_kv) floats): inside a capture the workspace cannot grow - call the op once eagerly with
  * the same shape, or fa_ctx_reserve_workspace, before fa_start_capture.
  * Environment: FOUNDRY_ATTN_GEMM_MIN_M (read at fa_ctx_create). */
 fa_status fa_set_gemm_min_m(fa_ctx *ctx, uint32_t min_m);
 
-/* Which GEMM kernel fa_fused_qkv / fa_matmul use (same tiling, step order and split points: bit-equal results): 1 = operand tiles staged through registers (any
- * shape, every weight policy); 2 = tiles loaded from memory straight into LDS in steps of 64 features, two workgroups
- * per compute unit; 3 = the same in steps of 32 features, four workgroups per compute unit; 0 (default) = 2 or 3 by
- * the number of output tiles. 2 and 3 need F16 weights, k_dim a multiple of 64 and operands below 2 GiB, and fall back
- * to 1 otherwise. No counterpart in the reference (a tuning switch like fa_set_prefill_variant).
+/* Which GEMM kernel fa_fused_qkv / fa_matmul use (F16 results are bit-equal): 1 = operand tiles of 128 x 128 staged
+ * through registers (any shape, every weight policy); 2 = tiles of 128 x 128 loaded from memory straight into LDS; 3 =
+ * the same with tiles of 64 x 64; 0 (default) = the tile by the number of output tiles that the launch has. 2 and 3 need
+ * k_dim a multiple of 64, weight rows that are multiples of 8, 16-byte aligned outputs and operands below 2 GiB, and fall
+ * back to 1 otherwise. No counterpart in the reference (a tuning switch like fa_set_prefill_variant).
  * Environment: FOUNDRY_ATTN_GEMM_VARIANT. */
 fa_status fa_set_gemm_variant(fa_ctx *ctx, uint32_t variant);
 

@@ -1,0 +1,114 @@
+// What the GEMM kernels of FusedQkv / MatMul share (fa_gemm.hip, fa_tile_*.hip): the launch's description, the RoPE write stage, the
+// conversion of block-quantised weights, and how the tile kernels are launched.
+#pragma once
+#include "fa_internal.h"
+#include "fa_qkv_rope.h"
+
+namespace fa_gemm {
+
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef float f4v_t __attribute__((ext_vector_type(4)));
+typedef float f16v_t __attribute__((ext_vector_type(16)));
+
+struct GemmDev {
+    const void *w[3];       // f16, or int8 (Q8_0) / nibbles (Q4_0) in the same element order
+    const __half *scales[3];  // Q8_0: f16 [rows, k_dim / 32] per matrix
+    const __half *bias[3];
+    __half *out[3];
+    uint32_t rows[3];       // weight rows per matrix
+    uint32_t tiles[3];      // 128-row tiles per matrix
+    const __half *x;        // [m, k_dim] (already normalised when the op has a gamma)
+    const __half *residual; // nullable, [m, rows[0]]
+    uint32_t k_dim, m, m_tiles, n_tiles, canonical, vec_store;
+    float alpha, beta;
+    // split-K: the feature steps are divided over k_splits workgroups per output tile, which store f32 partial tiles
+    // [split][m][n_total]; gemm_finish_kernel adds them up in split order and applies the write stage
+    uint32_t k_splits, steps_per_split, n_total;
+    float *partial;
+    // the weights of all matrices as one range of bytes, and where in it each begins (for tiles that hold rows of two matrices)
+    const void *w_low;
+    uint32_t w_span, w_at[3];
+    RopeDev rope;
+};
+
+// Write stage of one piece: y = the projections of token gm, columns gn .. gn + 7 of matrix mat (0 Q, 1 K, 2 V),
+// already rounded to f16 as FusedQkv stores them; mate = the piece half a head away (NeoX pairing; unused otherwise).
+// Q goes to q_rot[h][gm][hd], K (rotated) and V (as is) to cache row position_offset + gm of KV head h.
+__device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint32_t gm, uint32_t gn, h8_t y, const h8_t mate) {
+    const RopeDev &r = a.rope;
+    const uint32_t D = r.head_dim, half = D >> 1, h = gn / D, hd = gn - h * D;
+    const uint32_t pos = r.position_offset + gm;
+    __half *dst;
+    if (mat == 0) {
+        dst = a.out[0] + ((size_t)h * a.m + gm) * D + hd;
+    } else {
+        if (pos >= r.capacity) return;  // never outside the cache
+        size_t row;
+        if (!r.block_table) {
+            row = ((size_t)h * r.max_seq_len + pos) * D;
+        } else {
+            const size_t blk = (size_t)r.block_table[pos / r.block_size];
+            row = ((blk * r.n_kv_heads + h) * r.block_size + pos % r.block_size) * D;
+        }
+        dst = (mat == 1 ? a.out[1] : a.out[2]) + row + hd;
+    }
+    if (mat != 2 && r.apply) {
+        const uint32_t tp = pos < r.table_rows ? pos : r.table_rows - 1;  // stay inside the tables
+        if (r.normal) {  // pairs (hd + 2i, hd + 2i + 1), table columns hd / 2 + i
+            typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
+            const h4v_t c4 = *reinterpret_cast<const h4v_t *>(r.cos_t + (size_t)tp * half + (hd >> 1));
+            const h4v_t s4 = *reinterpret_cast<const h4v_t *>(r.sin_t + (size_t)tp * half + (hd >> 1));
+            h8_t o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[2 * i] = (_Float16)rope_one((float)y[2 * i], (float)y[2 * i + 1], (float)c4[i], (float)s4[i], true);
+                o[2 * i + 1] = (_Float16)rope_one((float)y[2 * i + 1], (float)y[2 * i], (float)c4[i], (float)s4[i], false);
+            }
+            y = o;
+        } else {  // pairs (hd, hd + D / 2), table column hd mod D / 2
+            const bool first = hd < half;
+            const uint32_t pc = first ? hd : hd - half;
+            const h8_t c8 = *reinterpret_cast<const h8_t *>(r.cos_t + (size_t)tp * half + pc);
+            const h8_t s8 = *reinterpret_cast<const h8_t *>(r.sin_t + (size_t)tp * half + pc);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = (_Float16)rope_one((float)y[e], (float)mate[e], (float)c8[e], (float)s8[e], first);
+        }
+    }
+    *reinterpret_cast<h8_t *>(dst) = y;
+}
+
+typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
+typedef _Float16 h2v_t __attribute__((ext_vector_type(2)));
+
+// 16 int8 weights -> two pieces of 8 f16, exactly: s + 128 is a byte u, the f16 with bits 0x6400 | u is 1024 + u, and
+// 1024 + u - 1152 = s (two byte permutes and one packed subtraction per four weights).
+__device__ __forceinline__ void q8_to_f16(const u4v_t raw, h8_t &p0, h8_t &p1) {
+    const h2v_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+#pragma unroll
+    for (int hw = 0; hw < 4; ++hw) {
+        const uint32_t u = raw[hw] ^ 0x80808080u;
+        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
+        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
+        h8_t &dst = hw < 2 ? p0 : p1;
+        const int o = (hw & 1) * 4;
+        dst[o + 0] = lo[0], dst[o + 1] = lo[1], dst[o + 2] = hi[0], dst[o + 3] = hi[1];
+    }
+}
+
+// 8 Q4_0 weights (one word: element 2i in the low nibble of byte i, value = nibble - 8) -> one piece of 8 f16, exactly:
+// the nibbles become two words of four bytes 0..15 in element order, then 0x6400 | u is 1024 + u and 1024 + u - 1032.
+__device__ __forceinline__ h8_t q4_to_f16(uint32_t w) {
+    const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+    const uint32_t b[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
+    const h2v_t bias = {(_Float16)1032.0f, (_Float16)1032.0f};
+    h8_t r;
+#pragma unroll
+    for (int hw = 0; hw < 2; ++hw) {
+        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x05010400u)) - bias;
+        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x07030602u)) - bias;
+        r[4 * hw + 0] = lo[0], r[4 * hw + 1] = lo[1], r[4 * hw + 2] = hi[0], r[4 * hw + 3] = hi[1];
+    }
+    return r;
+}
+
+}  // namespace fa_gemm

@@ -3,14 +3,12 @@
 // (MatMul; its large-m form is a GEMM, src/metals/mma) - with the write stage of src/metals/gemv/stages.rs:200-224.
 //
 // With more than a few input rows the step is no longer a weight stream: out[m, n] = x[m, :] . W[n, :] is
-// 2 * m * n * k flops on m * k + n * k operands, so it runs as a GEMM:
+// 2 * m * n * k flops on m * k + n * k operands, so it runs as a GEMM. Almost every launch goes to the tile kernels of fa_tile.h
+// (choose_tile below); this file holds the normalisation in front of them and the kernel that takes every other shape:
 //   * a workgroup (4 waves) owns a 128 (weight rows) x 128 (input rows) output tile; a wave owns 64 x 64 of it as
 //     2 x 2 v_mfma_f32_32x32x16_f16 tiles (64 accumulator registers);
-//   * both operands move through LDS in steps of 64 (or 32) features, two stages, one barrier per step. Three
-//     kernels differ in how the tiles get there: through registers (qkv_gemm_kernel: any shape, and block-quantised
-//     weights, which become f16 on the way), or from memory straight into LDS (qkv_gemm_dma_kernel, 64 features per
-//     step, two workgroups per CU; qkv_gemm_dma32_kernel, 32 features, four per CU) - see the notes at each;
-//   * LDS layouts are chosen per kernel so that writes (served 8 lanes at a time) and operand reads (16 lanes at a
+//   * both operands move through registers and LDS in steps of 64 features, two stages, one barrier per step;
+//   * LDS layouts are chosen so that writes (served 8 lanes at a time) and operand reads (16 lanes at a
 //     time) are free of bank conflicts; the blocked ("canonical") weight layout is one contiguous 8 KiB per (tile, 32
 //     features);
 //   * the rows of W_q, W_k, W_v are tiled per matrix (a tile never straddles two); the workgroups of one XCD take
@@ -21,8 +19,10 @@
 // RMSNorm: a small kernel in front writes the normalised input, rounded to f16 as qkv_project.metal:66-67 does, into
 // the context's workspace; the GEMM reads that. Launches with few output tiles divide a tile's feature steps over
 // several workgroups (split-K: f32 partial tiles in the workspace, added in split order by gemm_finish_kernel).
-#include "fa_internal.h"
-#include "fa_qkv_rope.h"
+#include "fa_gemm.h"
+#include "fa_norm.h"
+#include "fa_tile.h"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -44,77 +44,41 @@ constexpr int GM_T_STRIDE = GM_TN * 4 + 16;             // epilogue tile: bytes 
 constexpr int GM_LDS_BYTES = 2 * GM_STAGE_BYTES > GM_TM * GM_T_STRIDE ? 2 * GM_STAGE_BYTES : GM_TM * GM_T_STRIDE;
 constexpr int GM_LOADS = GM_TN * GM_PIECES / GM_NT;     // 16-byte pieces per thread, operand and step (4)
 
-typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-typedef float f4v_t __attribute__((ext_vector_type(4)));
-typedef float f16v_t __attribute__((ext_vector_type(16)));
+using namespace fa_gemm;
 
-struct GemmDev {
-    const void *w[3];       // f16, or int8 (Q8_0) / nibbles (Q4_0) in the same element order
-    const __half *scales[3];  // Q8_0: f16 [rows, k_dim / 32] per matrix
-    const __half *bias[3];
-    __half *out[3];
-    uint32_t rows[3];       // weight rows per matrix
-    uint32_t tiles[3];      // 128-row tiles per matrix
-    const __half *x;        // [m, k_dim] (already normalised when the op has a gamma)
-    const __half *residual; // nullable, [m, rows[0]]
-    uint32_t k_dim, m, m_tiles, n_tiles, canonical, vec_store;
-    float alpha, beta;
-    // split-K: the feature steps are divided over k_splits workgroups per output tile, which store f32 partial tiles
-    // [split][m][n_total]; gemm_finish_kernel adds them up in split order and applies the write stage
-    uint32_t k_splits, steps_per_split, n_total;
-    float *partial;
-    RopeDev rope;
-};
-
-// Write stage of one piece: y = the projections of token gm, columns gn .. gn + 7 of matrix mat (0 Q, 1 K, 2 V),
-// already rounded to f16 as FusedQkv stores them; mate = the piece half a head away (NeoX pairing; unused otherwise).
-// Q goes to q_rot[h][gm][hd], K (rotated) and V (as is) to cache row position_offset + gm of KV head h.
-__device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint32_t gm, uint32_t gn, h8_t y, const h8_t mate) {
-    const RopeDev &r = a.rope;
-    const uint32_t D = r.head_dim, half = D >> 1, h = gn / D, hd = gn - h * D;
-    const uint32_t pos = r.position_offset + gm;
-    __half *dst;
-    if (mat == 0) {
-        dst = a.out[0] + ((size_t)h * a.m + gm) * D + hd;
-    } else {
-        if (pos >= r.capacity) return;  // never outside the cache
-        size_t row;
-        if (!r.block_table) {
-            row = ((size_t)h * r.max_seq_len + pos) * D;
-        } else {
-            const size_t blk = (size_t)r.block_table[pos / r.block_size];
-            row = ((blk * r.n_kv_heads + h) * r.block_size + pos % r.block_size) * D;
-        }
-        dst = (mat == 1 ? a.out[1] : a.out[2]) + row + hd;
-    }
-    if (mat != 2 && r.apply) {
-        const uint32_t tp = pos < r.table_rows ? pos : r.table_rows - 1;  // stay inside the tables
-        if (r.normal) {  // pairs (hd + 2i, hd + 2i + 1), table columns hd / 2 + i
-            typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
-            const h4v_t c4 = *reinterpret_cast<const h4v_t *>(r.cos_t + (size_t)tp * half + (hd >> 1));
-            const h4v_t s4 = *reinterpret_cast<const h4v_t *>(r.sin_t + (size_t)tp * half + (hd >> 1));
-            h8_t o;
+// inv_rms of each input row, then (x * inv_rms) * gamma in f32, rounded to f16 (rmsnorm.metal:17-96). A wave takes a row: all of it
+// is requested at once, kept in registers (P pieces of 16 bytes per lane) and read once, and no wave waits for another.
+constexpr int NORM_ROWS = 4;  // rows (waves) per workgroup
+template <int P>
+__global__ void __launch_bounds__(NORM_ROWS * 64) rmsnorm_rows_kernel(const __half *x, const __half *gamma, __half *y, uint32_t m, uint32_t K,
+                                                                      float inv_k, float eps) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row = blockIdx.x * NORM_ROWS + wave;
+    if (row >= m) return;
+    const __half *xr = x + (size_t)row * K;
+    __half *yr = y + (size_t)row * K;
+    h8_t v[P], g[P];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                o[2 * i] = (_Float16)rope_one((float)y[2 * i], (float)y[2 * i + 1], (float)c4[i], (float)s4[i], true);
-                o[2 * i + 1] = (_Float16)rope_one((float)y[2 * i + 1], (float)y[2 * i], (float)c4[i], (float)s4[i], false);
-            }
-            y = o;
-        } else {  // pairs (hd, hd + D / 2), table column hd mod D / 2
-            const bool first = hd < half;
-            const uint32_t pc = first ? hd : hd - half;
-            const h8_t c8 = *reinterpret_cast<const h8_t *>(r.cos_t + (size_t)tp * half + pc);
-            const h8_t s8 = *reinterpret_cast<const h8_t *>(r.sin_t + (size_t)tp * half + pc);
+    for (int i = 0; i < P; ++i) v[i] = *reinterpret_cast<const h8_t *>(xr + min((uint32_t)(lane + 64 * i) * 8, K - 8));
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = (_Float16)rope_one((float)y[e], (float)mate[e], (float)c8[e], (float)s8[e], first);
-        }
+    for (int i = 0; i < P; ++i) g[i] = *reinterpret_cast<const h8_t *>(gamma + min((uint32_t)(lane + 64 * i) * 8, K - 8));
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const h8_t z = {0, 0, 0, 0, 0, 0, 0, 0}, u = (uint32_t)(lane + 64 * i) * 8 < K ? v[i] : z;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += (float)u[e] * (float)u[e];
     }
-    *reinterpret_cast<h8_t *>(dst) = y;
+    const float inv_rms = fa_norm::inv_rms(fa_norm::wave_sum(ss), inv_k, eps);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const h8_t o = fa_norm::scale8(v[i], inv_rms, g[i]);
+        if ((uint32_t)(lane + 64 * i) * 8 < K) *reinterpret_cast<h8_t *>(yr + (uint32_t)(lane + 64 * i) * 8) = o;
+    }
 }
-
-// inv_rms of each input row, then (x * inv_rms) * gamma in f32, rounded to f16 (rmsnorm.metal:17-96).
-__global__ void __launch_bounds__(256) rmsnorm_rows_kernel(const __half *x, const __half *gamma, __half *y, uint32_t K,
-                                                           float eps) {
+// The same for rows of more than 4096 features: a workgroup per row, which is read twice.
+__global__ void __launch_bounds__(256) rmsnorm_long_rows_kernel(const __half *x, const __half *gamma, __half *y, uint32_t K, float inv_k,
+                                                                float eps) {
     __shared__ float red[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const __half *xr = x + (size_t)blockIdx.x * K;
@@ -125,157 +89,106 @@ __global__ void __launch_bounds__(256) rmsnorm_rows_kernel(const __half *x, cons
 #pragma unroll
         for (int i = 0; i < 8; ++i) ss += (float)v[i] * (float)v[i];
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    ss = fa_norm::wave_sum(ss);
     if (lane == 0) red[wave] = ss;
     __syncthreads();
-    const float tot = ((red[0] + red[1]) + red[2]) + red[3];
-    const float inv_rms = rsqrtf(tot / (float)K + eps);
-    for (uint32_t k8 = tid; k8 < K / 8; k8 += 256) {
-        h8_t v = *reinterpret_cast<const h8_t *>(xr + k8 * 8);
-        const h8_t g = *reinterpret_cast<const h8_t *>(gamma + k8 * 8);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = (_Float16)(((float)v[i] * inv_rms) * (float)g[i]);
-        *reinterpret_cast<h8_t *>(yr + k8 * 8) = v;
-    }
+    const float inv_rms = fa_norm::inv_rms(((red[0] + red[1]) + red[2]) + red[3], inv_k, eps);
+    for (uint32_t k8 = tid; k8 < K / 8; k8 += 256)
+        *reinterpret_cast<h8_t *>(yr + k8 * 8) =
+            fa_norm::scale8(*reinterpret_cast<const h8_t *>(xr + k8 * 8), inv_rms, *reinterpret_cast<const h8_t *>(gamma + k8 * 8));
 }
 
 // The end of an output tile, shared by the GEMM kernels: accumulators -> LDS (f32, [input row][weight row]) -> either
-// the write stage and token-major f16 stores, or (split-K) the f32 partial tile. HALVES: the tile goes through LDS in
-// two halves of 64 input rows (tile j of every wave), for kernels that keep their LDS footprint at half a tile.
-template <bool HALVES>
+// the write stage and token-major f16 stores, or (split-K) the f32 partial tile.
 __device__ __forceinline__ void gemm_epilogue(const GemmDev &a, unsigned char *smem, const f16v_t (&acc)[2][2], int tid,
                                               int lane, int wn, int wm, int mat, uint32_t N, uint32_t n0, uint32_t m0,
                                               uint32_t split) {
-    constexpr int NH = HALVES ? 2 : 1;
-    constexpr uint32_t T_ROWS = HALVES ? GM_TM / 2 : GM_TM;
     const __half *bias = mat == 0 ? a.bias[0] : mat == 1 ? a.bias[1] : a.bias[2];
     __half *out = mat == 0 ? a.out[0] : mat == 1 ? a.out[1] : a.out[2];
     const uint32_t col0 = (mat >= 1 ? a.rows[0] : 0u) + (mat == 2 ? a.rows[1] : 0u) + n0;
+    // Accumulators -> LDS as f32 [input row][weight row]. Register r of lane l of a 32 x 32 tile is weight row
+    // 8 (r / 4) + 4 (l / 32) + r % 4 and input row l % 32: four consecutive weight rows per 16-byte write.
 #pragma unroll
-    for (int half = 0; half < NH; ++half) {
-        if (half) __syncthreads();  // the first half has been read out
-        // Accumulators -> LDS as f32 [input row][weight row]. Register r of lane l of a 32 x 32 tile is weight row
-        // 8 (r / 4) + 4 (l / 32) + r % 4 and input row l % 32: four consecutive weight rows per 16-byte write.
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (HALVES && j != half) continue;
-                const uint32_t t0 = HALVES ? wm * 32 : wm * 64 + j * 32;  // LDS row of the tile's first input row
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const uint32_t nrow = wn * 64 + i * 32 + g * 8 + (lane >> 5) * 4;
-                    const uint32_t trow = t0 + (lane & 31);
-                    const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
-                    *reinterpret_cast<f4v_t *>(smem + trow * GM_T_STRIDE + nrow * 4) = q;
-                }
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t nrow = wn * 64 + i * 32 + g * 8 + (lane >> 5) * 4;
+                const uint32_t trow = wm * 64 + j * 32 + (lane & 31);
+                const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+                *reinterpret_cast<f4v_t *>(smem + trow * GM_T_STRIDE + nrow * 4) = q;
             }
-        __syncthreads();
-        auto tile_row = [&](uint32_t t) { return HALVES ? (t >> 5) * 64 + half * 32 + (t & 31) : t; };
-
-        if (a.k_splits > 1) {  // partial sums only; the write stage runs in gemm_finish_kernel
-            for (uint32_t q = tid; q < T_ROWS * GM_TN / 4; q += GM_NT) {
-                const uint32_t t = q / (GM_TN / 4), n4 = q % (GM_TN / 4);
-                const uint32_t gm = m0 + tile_row(t), gn = n0 + n4 * 4;
-                if (gm >= a.m || gn >= N) continue;
-                const f4v_t s = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n4 * 16);
-                float *dst = a.partial + ((size_t)split * a.m + gm) * a.n_total + col0 + n4 * 4;
-                if (a.vec_store) {
-                    *reinterpret_cast<f4v_t *>(dst) = s;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (gn + e < N) dst[e] = s[e];
-                }
-            }
-            continue;
         }
-        for (uint32_t q = tid; q < T_ROWS * GM_TN / 8; q += GM_NT) {
-            const uint32_t t = q / (GM_TN / 8), n8 = q % (GM_TN / 8);
-            const uint32_t gm = m0 + tile_row(t), gn = n0 + n8 * 8;
+    __syncthreads();
+
+    if (a.k_splits > 1) {  // partial sums only; the write stage runs in gemm_finish_kernel
+        for (uint32_t q = tid; q < (uint32_t)GM_TM * GM_TN / 4; q += GM_NT) {
+            const uint32_t t = q / (GM_TN / 4), n4 = q % (GM_TN / 4);
+            const uint32_t gm = m0 + t, gn = n0 + n4 * 4;
             if (gm >= a.m || gn >= N) continue;
-            const f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n8 * 32);
-            const f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n8 * 32 + 16);
-            const size_t o = (size_t)gm * N + gn;
-            if (a.vec_store) {  // N % 8 == 0 and 16-byte aligned tensors: whole pieces
-                const h8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-                const h8_t bv = bias ? *reinterpret_cast<const h8_t *>(bias + gn) : z;
-                const h8_t rv = a.residual ? *reinterpret_cast<const h8_t *>(a.residual + o) : z;
-                h8_t y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    float v = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
-                    if (bias) v += (float)bv[e];
-                    if (a.residual) v += a.beta * (float)rv[e];
-                    y[e] = (_Float16)v;
-                }
-                if (a.rope.on) {
-                    // the mate piece of a NeoX pair lies half a head away in the same LDS row (a tile holds whole heads)
-                    h8_t mate = z;
-                    if (!a.rope.normal && a.rope.apply && mat != 2) {
-                        const uint32_t hp = a.rope.head_dim >> 4;  // pieces in half a head
-                        const uint32_t m8 = ((n8 * 8) & (a.rope.head_dim - 1)) < (a.rope.head_dim >> 1) ? n8 + hp : n8 - hp;
-                        const f4v_t t0 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + m8 * 32);
-                        const f4v_t t1 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + m8 * 32 + 16);
-                        const h8_t bm = bias ? *reinterpret_cast<const h8_t *>(bias + n0 + m8 * 8) : z;
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            float v = (e < 4 ? t0[e & 3] : t1[e & 3]) * a.alpha;
-                            if (bias) v += (float)bm[e];
-                            mate[e] = (_Float16)v;
-                        }
-                    }
-                    rope_store_piece(a, mat, gm, gn, y, mate);
-                } else {
-                    *reinterpret_cast<h8_t *>(out + o) = y;
-                }
+            const f4v_t s = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n4 * 16);
+            float *dst = a.partial + ((size_t)split * a.m + gm) * a.n_total + col0 + n4 * 4;
+            if (a.vec_store) {
+                *reinterpret_cast<f4v_t *>(dst) = s;
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    if (gn + e >= N) break;
-                    float v = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
-                    if (bias) v += __half2float(bias[gn + e]);
-                    if (a.residual) v += a.beta * __half2float(a.residual[o + e]);
-                    out[o + e] = __float2half(v);
+                for (int e = 0; e < 4; ++e)
+                    if (gn + e < N) dst[e] = s[e];
+            }
+        }
+        return;
+    }
+    for (uint32_t q = tid; q < (uint32_t)GM_TM * GM_TN / 8; q += GM_NT) {
+        const uint32_t t = q / (GM_TN / 8), n8 = q % (GM_TN / 8);
+        const uint32_t gm = m0 + t, gn = n0 + n8 * 8;
+        if (gm >= a.m || gn >= N) continue;
+        const f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n8 * 32);
+        const f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + n8 * 32 + 16);
+        const size_t o = (size_t)gm * N + gn;
+        if (a.vec_store) {  // N % 8 == 0 and 16-byte aligned tensors: whole pieces
+            const h8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+            const h8_t bv = bias ? *reinterpret_cast<const h8_t *>(bias + gn) : z;
+            const h8_t rv = a.residual ? *reinterpret_cast<const h8_t *>(a.residual + o) : z;
+            h8_t y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float v = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
+                if (bias) v += (float)bv[e];
+                if (a.residual) v += a.beta * (float)rv[e];
+                y[e] = (_Float16)v;
+            }
+            if (a.rope.on) {
+                // the mate piece of a NeoX pair lies half a head away in the same LDS row (a tile holds whole heads)
+                h8_t mate = z;
+                if (!a.rope.normal && a.rope.apply && mat != 2) {
+                    const uint32_t hp = a.rope.head_dim >> 4;  // pieces in half a head
+                    const uint32_t m8 = ((n8 * 8) & (a.rope.head_dim - 1)) < (a.rope.head_dim >> 1) ? n8 + hp : n8 - hp;
+                    const f4v_t t0 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + m8 * 32);
+                    const f4v_t t1 = *reinterpret_cast<const f4v_t *>(smem + t * GM_T_STRIDE + m8 * 32 + 16);
+                    const h8_t bm = bias ? *reinterpret_cast<const h8_t *>(bias + n0 + m8 * 8) : z;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        float v = (e < 4 ? t0[e & 3] : t1[e & 3]) * a.alpha;
+                        if (bias) v += (float)bm[e];
+                        mate[e] = (_Float16)v;
+                    }
                 }
+                rope_store_piece(a, mat, gm, gn, y, mate);
+            } else {
+                *reinterpret_cast<h8_t *>(out + o) = y;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (gn + e >= N) break;
+                float v = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
+                if (bias) v += __half2float(bias[gn + e]);
+                if (a.residual) v += a.beta * __half2float(a.residual[o + e]);
+                out[o + e] = __float2half(v);
             }
         }
     }
-}
-
-typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
-typedef _Float16 h2v_t __attribute__((ext_vector_type(2)));
-
-// 16 int8 weights -> two pieces of 8 f16, exactly: s + 128 is a byte u, the f16 with bits 0x6400 | u is 1024 + u, and
-// 1024 + u - 1152 = s (two byte permutes and one packed subtraction per four weights).
-__device__ __forceinline__ void q8_to_f16(const u4v_t raw, h8_t &p0, h8_t &p1) {
-    const h2v_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-#pragma unroll
-    for (int hw = 0; hw < 4; ++hw) {
-        const uint32_t u = raw[hw] ^ 0x80808080u;
-        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
-        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
-        h8_t &dst = hw < 2 ? p0 : p1;
-        const int o = (hw & 1) * 4;
-        dst[o + 0] = lo[0], dst[o + 1] = lo[1], dst[o + 2] = hi[0], dst[o + 3] = hi[1];
-    }
-}
-
-// 8 Q4_0 weights (one word: element 2i in the low nibble of byte i, value = nibble - 8) -> one piece of 8 f16, exactly:
-// the nibbles become two words of four bytes 0..15 in element order, then 0x6400 | u is 1024 + u and 1024 + u - 1032.
-__device__ __forceinline__ h8_t q4_to_f16(uint32_t w) {
-    const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
-    const uint32_t b[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
-    const h2v_t bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-    h8_t r;
-#pragma unroll
-    for (int hw = 0; hw < 2; ++hw) {
-        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x05010400u)) - bias;
-        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x07030602u)) - bias;
-        r[4 * hw + 0] = lo[0], r[4 * hw + 1] = lo[1], r[4 * hw + 2] = hi[0], r[4 * hw + 3] = hi[1];
-    }
-    return r;
 }
 
 // Block-quantised weights become f16 on their way into LDS as the reference's GEMM tile loader makes them
@@ -467,295 +380,7 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
         __syncthreads();
     }
 
-    gemm_epilogue<false>(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
-}
-
-// ---------------------------------------------------------------------------------------------------------------
-// The same GEMM with the operand tiles going from memory straight into LDS (buffer_load ... lds), F16 weights, k_dim a
-// multiple of 64: no staging registers, no LDS write instructions, no wait for the loads before a write - the next
-// step's tiles are requested before this step's matrix work and waited for after it. The 64 lanes of such a load fill
-// 1 KiB of consecutive LDS bytes in lane order, so padding is impossible; instead each 1 KiB holds a whole number of
-// rows and a lane fetches, within its row, the 16-byte piece that belongs into its slot:
-//   input and row-major weights: 1 KiB = 8 rows x 8 pieces, slot = piece ^ ((row / 2) % 8)
-//   canonical weights:           1 KiB = 16 rows x 4 pieces of a 32-feature block, slot = piece ^ ((row / 4) % 4)
-// so that the 16 lanes that read one piece column of 16 consecutive rows fall into 16 different 16-byte bank groups
-// of the 256 bytes an LDS read serves per cycle (with row % 8 and (row / 2) % 4, distinct within 8 lanes only, a third
-// of the LDS cycles were bank conflicts), while the lanes of a request still cover whole 64- or 128-byte runs of memory. Rows past the end of a matrix (or of
-// the input) are out of the buffer descriptor's range and arrive as zeros.
-typedef unsigned int rsrc_words __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ rsrc_words gemm_rsrc(const void *base, uint32_t bytes) {
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    rsrc_words r;
-    r.x = (uint32_t)b, r.y = (uint32_t)(b >> 32) & 0xffffu, r.z = bytes, r.w = 0x00020000u;
-    return r;
-}
-// Four 1 KiB requests into consecutive KiB of LDS. Written as assembly: the compiler cannot tell which LDS bytes such
-// a load writes and would serialise every later LDS read behind it; completion is tracked by vmcnt, waited for by hand.
-__device__ __forceinline__ void lds_dma_4x(rsrc_words rs, uint32_t lds_addr, int v0, int v1, int v2, int v3, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %1, %6 offen lds\n\t"
-                 "s_add_i32 m0, %0, 0x400\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %3, %1, %6 offen lds\n\t"
-                 "s_add_i32 m0, %0, 0x800\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %4, %1, %6 offen lds\n\t"
-                 "s_add_i32 m0, %0, 0xc00\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %5, %1, %6 offen lds"
-                 :
-                 : "s"(lds_addr), "s"(rs), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(soff)
-                 : "memory", "scc");
-}
-// ... with one lane offset and sources 1 KiB apart as well (canonical weights): the immediate offset moves both sides
-__device__ __forceinline__ void lds_dma_4x_contiguous(rsrc_words rs, uint32_t lds_addr, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen lds\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen offset:1024 lds\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen offset:2048 lds\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen offset:3072 lds"
-                 :
-                 : "s"(lds_addr), "s"(rs), "v"(voff)
-                 : "memory");
-}
-
-constexpr int GD_OPERAND_BYTES = GM_TN * GM_BK * 2;  // 16 KiB, no padding
-constexpr int GD_STAGE_BYTES = 2 * GD_OPERAND_BYTES;
-
-template <bool CANON>
-__global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_dma_kernel(GemmDev a) {
-    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    typedef __attribute__((address_space(3))) void *lds_ptr;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)smem;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t K = a.k_dim;
-
-    const uint32_t total = a.n_tiles * a.m_tiles * a.k_splits;
-    uint32_t v = blockIdx.x;
-    if (total % 8 == 0) v = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
-    const uint32_t split = v % a.k_splits;
-    v /= a.k_splits;
-    uint32_t nt = v / a.m_tiles;
-    const uint32_t mt = v - nt * a.m_tiles;
-    int mat = 0;
-    if (nt >= a.tiles[0]) {
-        nt -= a.tiles[0], mat = 1;
-        if (nt >= a.tiles[1]) nt -= a.tiles[1], mat = 2;
-    }
-    const uint32_t N = mat == 0 ? a.rows[0] : a.rows[1];
-    const unsigned char *W = reinterpret_cast<const unsigned char *>(mat == 0 ? a.w[0] : mat == 1 ? a.w[1] : a.w[2]);
-    const uint32_t n0 = nt * GM_TN, m0 = mt * GM_TM;
-
-    // Requests of this wave: KiB 4 wave .. 4 wave + 3 of each operand tile.
-    // Input (and row-major weights): KiB c = rows 8c .. 8c + 7; lane l = (row l / 8, slot l % 8), piece = slot ^ (row / 2) % 8.
-    const uint32_t xr_lane = lane >> 3;
-    int xv[4], wv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t row = (wave * 4 + i) * 8 + xr_lane;
-        const uint32_t x_piece = (lane & 7) ^ ((row >> 1) & 7);
-        xv[i] = (int)(row * K * 2 + x_piece * 16);  // rows past the input's end are past the descriptor's range
-        wv[i] = xv[i];
-    }
-    const rsrc_words x_rs = gemm_rsrc(reinterpret_cast<const unsigned char *>(a.x) + (size_t)m0 * K * 2,
-                                      (uint32_t)min((uint64_t)(a.m - m0) * K * 2, (uint64_t)0x7fffffffu));
-    // Canonical weights: KiB c of a step = 32-feature block c / 8, rows 16 (c % 8) .. + 15; lane l = (row l / 4, slot
-    // l % 4), piece = slot ^ (row / 4) % 4; the descriptor covers one block's N rows of 64 bytes and is moved per step.
-    const uint32_t cw_row = lane >> 2, cw_piece = (lane & 3) ^ ((cw_row >> 2) & 3);
-    const int cw_voff = (int)((n0 + (wave & 1) * 64 + cw_row) * 64 + cw_piece * 16);
-    const rsrc_words w_rs = CANON ? gemm_rsrc(W, 0)
-                                  : gemm_rsrc(W + (size_t)n0 * K * 2, (uint32_t)min((uint64_t)(N - n0) * K * 2, (uint64_t)0x7fffffffu));
-    auto request = [&](uint32_t ks) {
-        const uint32_t stage = lds_base + (ks & 1) * GD_STAGE_BYTES;
-        if constexpr (CANON) {
-            const rsrc_words rs = gemm_rsrc(W + (size_t)(2 * ks + (wave >> 1)) * N * 64, N * 64);
-            lds_dma_4x_contiguous(rs, stage + wave * 4096, cw_voff);
-        } else {
-            lds_dma_4x(w_rs, stage + wave * 4096, wv[0], wv[1], wv[2], wv[3], (int)(ks * GM_BK * 2));
-        }
-        lds_dma_4x(x_rs, stage + GD_OPERAND_BYTES + wave * 4096, xv[0], xv[1], xv[2], xv[3], (int)(ks * GM_BK * 2));
-    };
-    (void)w_rs;
-
-    // Operand reads. Wave (wn, wm) owns weight rows 64 wn .. +63 and input rows 64 wm .. +63; lane l reads row l % 32
-    // (+ 32 per tile) and the 16-feature half l / 32 of each 32 features.
-    const int wn = wave & 1, wm = wave >> 1;
-    const uint32_t h = lane >> 5, r32 = lane & 31;
-    // input layout (also row-major weights): row r at KiB r / 8, 128 bytes per row, slot = piece ^ (r / 2) % 8
-    auto rowmajor_base = [&](uint32_t row) { return (row >> 3) * 1024 + (row & 7) * 128; };
-    uint32_t x_slot[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) x_slot[kk] = ((2 * kk + h) ^ ((r32 >> 1) & 7)) * 16;
-    const uint32_t b_base = rowmajor_base(wm * 64 + r32);  // + 4096 per tile of 32 rows
-    // canonical layout: row r of block b at KiB 8 b + r / 16, 64 bytes per row, slot = piece ^ (r / 4) % 4
-    uint32_t a_base, a_slot[4];
-    if constexpr (CANON) {
-        const uint32_t row = wn * 64 + r32;
-        a_base = (row >> 4) * 1024 + (row & 15) * 64;  // + 2048 per tile of 32 rows
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) a_slot[kk] = (kk >> 1) * 8192 + (((2 * (kk & 1) + h) ^ ((row >> 2) & 3)) * 16);
-    } else {
-        a_base = rowmajor_base(wn * 64 + r32);
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) a_slot[kk] = x_slot[kk];
-    }
-    constexpr uint32_t A_TILE = CANON ? 2048 : 4096;
-
-    f16v_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const uint32_t all_steps = K / GM_BK;
-    const uint32_t ks_begin = split * a.steps_per_split;
-    const uint32_t n_steps = min(all_steps, ks_begin + a.steps_per_split);
-    request(ks_begin);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    for (uint32_t ks = ks_begin; ks < n_steps; ++ks) {
-        if (ks + 1 < n_steps) request(ks + 1);  // into the stage every wave finished reading before the last barrier
-        const unsigned char *wa = smem + (ks & 1) * GD_STAGE_BYTES;
-        const unsigned char *xa = wa + GD_OPERAND_BYTES;
-#pragma unroll
-        for (int kk = 0; kk < GM_BK / 16; ++kk) {
-            h8_t fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fa[i] = *reinterpret_cast<const h8_t *>(wa + a_base + i * A_TILE + a_slot[kk]);
-                fb[i] = *reinterpret_cast<const h8_t *>(xa + b_base + i * 4096 + x_slot[kk]);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    }
-    gemm_epilogue<false>(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
-}
-
-// The LDS-direct GEMM in steps of 32 features, two stages, with the output tile leaving through LDS in two halves: a
-// workgroup then needs 33 KiB of LDS instead of 66 and four of them share a CU instead of two. Per tile this is the
-// slower kernel (twice the barriers per feature), but when the launch has more workgroups than two per CU and at most
-// four, all of them are resident at once instead of a second, partly filled round (Llama-3.2-3B Q/K/V on 2048 rows,
-// 640 tiles: 80.4 us against 95.2; 1024 rows, 320 tiles: 56.8 against 50.8; 4096 rows, 1280 tiles: 169.7 against
-// 157.8). A ring of three or four such stages (requests two or three steps ahead, three or two workgroups per CU) was
-// measured as well and is never the fastest: the latency of the requests is not what limits these kernels.
-// Both operands use the layout 1 KiB = 16 rows x 4 pieces (64 bytes of a row), slot = piece ^ ((row / 4) % 4).
-__device__ __forceinline__ void lds_dma_2x(rsrc_words rs, uint32_t lds_addr, int v0, int v1, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %1, %4 offen lds\n\t"
-                 "s_add_i32 m0, %0, 0x400\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %3, %1, %4 offen lds"
-                 :
-                 : "s"(lds_addr), "s"(rs), "v"(v0), "v"(v1), "s"(soff)
-                 : "memory", "scc");
-}
-__device__ __forceinline__ void lds_dma_2x_contiguous(rsrc_words rs, uint32_t lds_addr, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen lds\n\t"
-                 "buffer_load_dwordx4 %2, %1, 0 offen offset:1024 lds"
-                 :
-                 : "s"(lds_addr), "s"(rs), "v"(voff)
-                 : "memory");
-}
-constexpr int GR_BK = 32;
-constexpr int GR_OPERAND_BYTES = GM_TN * GR_BK * 2;  // 8 KiB
-constexpr int GR_STAGE_BYTES = 2 * GR_OPERAND_BYTES;
-constexpr int GR_T_BYTES = (GM_TM / 2) * GM_T_STRIDE;
-constexpr int GR_LDS_BYTES = 2 * GR_STAGE_BYTES > GR_T_BYTES ? 2 * GR_STAGE_BYTES : GR_T_BYTES;
-
-template <bool CANON>
-__global__ void __launch_bounds__(GM_NT, 4) qkv_gemm_dma32_kernel(GemmDev a) {
-    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    typedef __attribute__((address_space(3))) void *lds_ptr;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)smem;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t K = a.k_dim;
-
-    const uint32_t total = a.n_tiles * a.m_tiles * a.k_splits;
-    uint32_t v = blockIdx.x;
-    if (total % 8 == 0) v = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
-    const uint32_t split = v % a.k_splits;
-    v /= a.k_splits;
-    uint32_t nt = v / a.m_tiles;
-    const uint32_t mt = v - nt * a.m_tiles;
-    int mat = 0;
-    if (nt >= a.tiles[0]) {
-        nt -= a.tiles[0], mat = 1;
-        if (nt >= a.tiles[1]) nt -= a.tiles[1], mat = 2;
-    }
-    const uint32_t N = mat == 0 ? a.rows[0] : a.rows[1];
-    const unsigned char *W = reinterpret_cast<const unsigned char *>(mat == 0 ? a.w[0] : mat == 1 ? a.w[1] : a.w[2]);
-    const uint32_t n0 = nt * GM_TN, m0 = mt * GM_TM;
-
-    // Requests of this wave: KiB 2 wave and 2 wave + 1 of each operand tile = rows 32 wave .. + 31; lane l = (row l / 4,
-    // slot l % 4) of its KiB, piece = slot ^ (row / 4) % 4.
-    const uint32_t r16 = lane >> 2, piece = (lane & 3) ^ ((r16 >> 2) & 3);
-    const uint32_t row0 = wave * 32 + r16;
-    const int xv0 = (int)(row0 * K * 2 + piece * 16), xv1 = (int)((row0 + 16) * K * 2 + piece * 16);
-    const int cw_voff = (int)((n0 + row0) * 64 + piece * 16);
-    const rsrc_words x_rs = gemm_rsrc(reinterpret_cast<const unsigned char *>(a.x) + (size_t)m0 * K * 2,
-                                      (uint32_t)min((uint64_t)(a.m - m0) * K * 2, (uint64_t)0x7fffffffu));
-    const rsrc_words w_rs = CANON ? gemm_rsrc(W, 0)
-                                  : gemm_rsrc(W + (size_t)n0 * K * 2, (uint32_t)min((uint64_t)(N - n0) * K * 2, (uint64_t)0x7fffffffu));
-    auto request = [&](uint32_t ks) {
-        const uint32_t stage = lds_base + (ks & 1) * GR_STAGE_BYTES;
-        if constexpr (CANON) {  // one 32-feature block per step: N rows of 64 bytes
-            const rsrc_words rs = gemm_rsrc(W + (size_t)ks * N * 64, N * 64);
-            lds_dma_2x_contiguous(rs, stage + wave * 2048, cw_voff);
-        } else {
-            lds_dma_2x(w_rs, stage + wave * 2048, xv0, xv1, (int)(ks * GR_BK * 2));
-        }
-        lds_dma_2x(x_rs, stage + GR_OPERAND_BYTES + wave * 2048, xv0, xv1, (int)(ks * GR_BK * 2));
-    };
-    (void)w_rs;
-    (void)cw_voff;
-
-    // Operand reads: lane l reads row l % 32 (+ 32 per tile) of the wave's 64 rows, 16-feature half l / 32 of each 16.
-    const int wn = wave & 1, wm = wave >> 1;
-    const uint32_t h = lane >> 5, r32 = lane & 31;
-    auto row_base = [&](uint32_t row) { return (row >> 4) * 1024 + (row & 15) * 64; };
-    uint32_t slot[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) slot[kk] = ((2 * kk + h) ^ ((r32 >> 2) & 3)) * 16;
-    const uint32_t a_base = row_base(wn * 64 + r32), b_base = row_base(wm * 64 + r32);  // + 2048 per tile of 32 rows
-
-    f16v_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const uint32_t all_steps = K / GR_BK;
-    const uint32_t ks_begin = split * a.steps_per_split * 2;  // steps_per_split counts steps of 64 features
-    const uint32_t n_steps = min(all_steps, ks_begin + a.steps_per_split * 2);
-    request(ks_begin);
-    for (uint32_t ks = ks_begin; ks < n_steps; ++ks) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's requests for step ks have landed ...
-        __syncthreads();  // ... and everybody's; every wave is also done reading the stage of step ks - 1,
-        if (ks + 1 < n_steps) request(ks + 1);  // which step ks + 1 reuses
-        const unsigned char *wa = smem + (ks & 1) * GR_STAGE_BYTES;
-        const unsigned char *xa = wa + GR_OPERAND_BYTES;
-#pragma unroll
-        for (int kk = 0; kk < GR_BK / 16; ++kk) {
-            h8_t fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fa[i] = *reinterpret_cast<const h8_t *>(wa + a_base + i * 2048 + slot[kk]);
-                fb[i] = *reinterpret_cast<const h8_t *>(xa + b_base + i * 2048 + slot[kk]);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();  // the stages are reused by the output tile
-    gemm_epilogue<true>(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
+    gemm_epilogue(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
 }
 
 // Adds the split-K partial tiles in split order and applies the write stage: one thread per 8 output columns.
@@ -844,6 +469,55 @@ __global__ void __launch_bounds__(256) gemm_finish_kernel(GemmDev a) {
 
 }  // namespace
 
+// Whether the tile kernels (fa_tile.h) take a launch, and with which tile: whole steps of 64 features, whole 16-byte stores, operands
+// below 2 GiB (32-bit offsets). What a tile of each shape takes per step of 64 features with one workgroup on every CU, in units of the
+// 64 x 64 tile's 0.21 us (from launches of 160 to 256 tiles over 3072 features), times the rounds of workgroups that the launch has:
+// the larger tiles read less per product, the smaller ones leave fewer CUs idle.
+static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, uint32_t n_cus, fa_tile::TileShape &shape) {
+    const uint64_t max_rows = std::max(a.rows[0], a.rows[1]);
+    if (l.k_dim % 64 != 0 || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
+    for (int i = 0; i < 3; ++i)
+        if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) return false;
+    // tiles over the rows of all matrices need them within the reach of one descriptor
+    uintptr_t low = (uintptr_t)l.w[0], high = low;
+    for (int i = 0; i < 3; ++i)
+        if (a.rows[i]) low = std::min(low, (uintptr_t)l.w[i]), high = std::max(high, (uintptr_t)l.w[i] + (size_t)a.rows[i] * l.k_dim * 2);
+    const bool joined = l.weight_bits == 16 && high - low < 0xfffffff0ull && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
+    if (joined) {
+        a.w_low = (const void *)low, a.w_span = (uint32_t)(high - low);
+        for (int i = 0; i < 3; ++i) a.w_at[i] = a.rows[i] ? (uint32_t)((uintptr_t)l.w[i] - low) : 0u;
+    }
+    struct Choice {
+        fa_tile::TileShape shape;
+        uint32_t m, n;
+        float f16, quantised;
+    };
+    static const Choice choices[] = {{fa_tile::TILE_64x64, 64, 64, 1.0f, 1.0f},
+                                     {fa_tile::TILE_128x64, 128, 64, 1.75f, 1.64f},
+                                     {fa_tile::TILE_128x128, 128, 128, 2.6f, 2.7f},
+                                     {fa_tile::TILE_256x128, 256, 128, 4.65f, 4.3f},
+                                     {fa_tile::TILE_256x160, 256, 160, 6.3f, 0.0f}};
+    float best = 0.0f;
+    for (const Choice &c : choices) {
+        if (c.shape == fa_tile::TILE_256x160 && !joined) continue;
+        // (a block-quantised tile's scales lie in LDS over the whole of k_dim)
+        if (l.weight_bits != 16 && c.shape != fa_tile::TILE_64x64 && l.k_dim > 4096) continue;
+        if (ctx->gemm_variant == 2 && c.shape != fa_tile::TILE_128x128) continue;
+        if (ctx->gemm_variant == 3 && c.shape != fa_tile::TILE_64x64) continue;
+        uint32_t n_tiles = 0;
+        for (int i = 0; i < 3; ++i) n_tiles += ceil_div_u32(a.rows[i], c.n);
+        if (c.shape == fa_tile::TILE_256x160) n_tiles = ceil_div_u32(a.rows[0] + 2 * a.rows[1], c.n);
+        const uint64_t tiles = (uint64_t)n_tiles * ceil_div_u32(l.m, c.m);
+        const float cost = (float)((tiles + n_cus - 1) / n_cus) * (l.weight_bits == 16 ? c.f16 : c.quantised);
+        if (best == 0.0f || cost < best) {
+            best = cost, shape = c.shape;
+            // With a workgroup or less per CU, the block-quantised form keeps twice as many of its smaller stages on their way.
+            if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && tiles <= n_cus && l.k_dim <= 8192) shape = fa_tile::TILE_64x64_DEEP;
+        }
+    }
+    return best != 0.0f && (l.weight_bits == 16 || l.k_dim <= 16384);
+}
+
 static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch *rope) {
     if (l.k_dim % 8 != 0) return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: k_dim %u must be a multiple of 8", l.k_dim);
     GemmDev a;
@@ -886,16 +560,14 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
         return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: the GEMM path needs 16-byte aligned input and weights");
     const uint64_t n_wg = (uint64_t)a.n_tiles * a.m_tiles;
     if (n_wg > 0x7fffffffull) return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: %llu output tiles", (unsigned long long)n_wg);
-    // Few output tiles (a short prefill chunk): the feature steps of a tile are divided over enough workgroups to
-    // give every CU a share of the weight stream, at least 4 steps each (a 32-row chunk of Llama-3.2-3B: 36.9 us
-    // unsplit, 17.4 us with the 48 steps over 12 workgroups per tile; 512 rows: 42.9 -> 35.9 us with 3).
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
+    fa_tile::TileShape shape;
+    const bool tiles_whole = choose_tile(ctx, l, a, n_cus, shape);
+    // The register-staged kernel with few output tiles: the feature steps of a tile are divided over enough workgroups to give
+    // every CU a share of the weight stream, at least 4 steps each (512 rows of the Llama-3.2-3B projections: 42.9 -> 35.9 us with 3).
+    // (What the tile kernels could take is not divided either: their sums and this kernel's are the same to the bit.)
     const uint32_t all_steps = ceil_div_u32(l.k_dim, GM_BK);
-    // Two workgroups per CU as the target. With the weights still in the last-level cache from the previous call (one
-    // layer in a loop) 1.5 per CU measures faster (256 rows: 26.7 us against 31.4), but with each call's weights coming
-    // from memory, as in a model, 2 per CU wins: 512 rows 26.5 + 6.2 us (GEMM + finish) against 32.0 + 5.0.
-    const uint32_t target = 2 * n_cus;
-    uint32_t splits = (uint32_t)(target / n_wg);
+    uint32_t splits = tiles_whole ? 1u : (uint32_t)(2 * n_cus / n_wg);
     if (splits > all_steps / 4) splits = all_steps / 4;
     if (splits < 1) splits = 1;
     a.steps_per_split = ceil_div_u32(all_steps, splits);
@@ -908,7 +580,13 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
     if (a.k_splits > 1 && a.n_total % 8 != 0) a.vec_store = 0;  // (never with a RoPE write stage: whole heads of 64 or 128)
     if (l.gamma) {
         FaLaunchScope norm(ctx, "rmsnorm_rows_kernel", true);
-        norm.launch(rmsnorm_rows_kernel, dim3(l.m), dim3(256), 0, l.x, l.gamma, (__half *)ctx->workspace, l.k_dim, l.eps);
+        __half *y = (__half *)ctx->workspace;
+        const float inv_k = 1.0f / (float)l.k_dim;
+        const dim3 grid(ceil_div_u32(l.m, NORM_ROWS)), block(NORM_ROWS * 64);
+        if (l.k_dim <= 1024) norm.launch(rmsnorm_rows_kernel<2>, grid, block, 0, l.x, l.gamma, y, l.m, l.k_dim, inv_k, l.eps);
+        else if (l.k_dim <= 2048) norm.launch(rmsnorm_rows_kernel<4>, grid, block, 0, l.x, l.gamma, y, l.m, l.k_dim, inv_k, l.eps);
+        else if (l.k_dim <= 4096) norm.launch(rmsnorm_rows_kernel<8>, grid, block, 0, l.x, l.gamma, y, l.m, l.k_dim, inv_k, l.eps);
+        else norm.launch(rmsnorm_long_rows_kernel, dim3(l.m), dim3(256), 0, l.x, l.gamma, y, l.k_dim, inv_k, l.eps);
         FA_TRY(norm.finish());
         a.x = (const __half *)ctx->workspace;
     }
@@ -924,29 +602,14 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
         lds_allowed.store(true, std::memory_order_release);
     }
     FaLaunchScope scope(ctx, l.n_kv ? "fused_qkv_gemm_kernel" : "matmul_gemm_kernel", true);
+    if (tiles_whole && ctx->gemm_variant != 1) {
+        if (l.weight_bits == 16) FA_TRY(fa_tile::launch_f16(ctx, scope, shape, a, l.canonical));
+        else if (l.weight_bits == 8) FA_TRY(fa_tile::launch_q8(ctx, scope, shape, a, l.canonical));
+        else FA_TRY(fa_tile::launch_q4(ctx, scope, shape, a, l.canonical));
+        return scope.finish();
+    }
     const uint32_t grid = (uint32_t)n_wg * a.k_splits;
-    // F16 weights, whole steps of 64 features, operands below 2 GiB (32-bit buffer offsets): tiles straight into LDS
-    const uint64_t max_rows = a.rows[0] > a.rows[1] ? a.rows[0] : a.rows[1];
-    const bool dma_ok = !q8 && l.k_dim % GM_BK == 0 && (uint64_t)l.m * l.k_dim * 2 < 0x7fffffffull &&
-                        max_rows * l.k_dim * 2 < 0x7fffffffull;
-    // two LDS-direct kernels: steps of 64 features, two workgroups per CU - or steps of 32, four per CU, when that
-    // makes the whole launch resident at once
-    const uint32_t n_cus_l = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    const bool small_steps = ctx->gemm_variant == 3 || (ctx->gemm_variant == 0 && grid > 2 * n_cus_l && grid <= 4 * n_cus_l);
-    if (dma_ok && small_steps) {
-        if (l.canonical) scope.launch(qkv_gemm_dma32_kernel<true>, dim3(grid), dim3(GM_NT), GR_LDS_BYTES, a);
-        else scope.launch(qkv_gemm_dma32_kernel<false>, dim3(grid), dim3(GM_NT), GR_LDS_BYTES, a);
-    } else if (dma_ok && ctx->gemm_variant != 1) {
-        static std::atomic<bool> dma_lds_allowed_on[64];  // per device (contexts of several threads may get here together: the calls are idempotent)
-        std::atomic<bool> &dma_lds_allowed = dma_lds_allowed_on[ctx->device & 63];
-        if (!dma_lds_allowed.load(std::memory_order_acquire)) {
-            FA_HIP(hipFuncSetAttribute((const void *)qkv_gemm_dma_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS_BYTES));
-            FA_HIP(hipFuncSetAttribute((const void *)qkv_gemm_dma_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS_BYTES));
-            dma_lds_allowed.store(true, std::memory_order_release);
-        }
-        if (l.canonical) scope.launch(qkv_gemm_dma_kernel<true>, dim3(grid), dim3(GM_NT), GM_LDS_BYTES, a);
-        else scope.launch(qkv_gemm_dma_kernel<false>, dim3(grid), dim3(GM_NT), GM_LDS_BYTES, a);
-    } else if (l.weight_bits == 4) {
+    if (l.weight_bits == 4) {
         if (l.canonical) scope.launch(qkv_gemm_kernel<true, 4>, dim3(grid), dim3(GM_NT), GM_LDS_BYTES, a);
         else scope.launch(qkv_gemm_kernel<false, 4>, dim3(grid), dim3(GM_NT), GM_LDS_BYTES, a);
     } else if (q8) {

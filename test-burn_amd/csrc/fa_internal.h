@@ -61,7 +61,7 @@ struct fa_ctx {
     uint32_t *d_status = nullptr;  // device view of the same words
     fa_decode_variant decode_variant{0, 1};
     uint32_t decode_waves = 0;     // waves per decode workgroup: 0 = by launch size, 4 or 8
-    uint32_t gemm_variant = 0;     // GEMM kernel: 0 = auto, 1 = tiles through registers, 2 / 3 = straight into LDS in steps of 64 / 32 features
+    uint32_t gemm_variant = 0;     // GEMM kernel: 0 = auto, 1 = tiles through registers, 2 / 3 = straight into LDS, tiles of 128 x 128 / 64 x 64
     uint32_t gemm_min_m = 0;       // FusedQkv / MatMul: input rows from which the GEMM runs (0 = default)
     uint32_t qkv_rows32_min_m = 0;  // FusedQkv / MatMul: from this many input rows the one-launch kernel for short chunks (fa_panel.h); 0 = default, 33 = never
     bool qkv_rows32_rope = true;    // FusedQkv + KvPrepFused of such a chunk: the KvPrepFused work in that launch's write stage (false: a second launch)

@@ -418,12 +418,15 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
 
 // Whether a FusedQkv / MatMul launch goes to the panel kernel: rows of up to 3072 features, from two input rows (four layers of the
 // Llama-3.2-3B block with 2 / 4 / 8 / 11 rows: 113 / 113 / 115 / 117 us against 120 / 128 / 137 / 155 with the kernel for up to 16
-// rows) to as many as it is measured to beat the GEMM with; an explicit GEMM threshold (fa_set_gemm_min_m) wins.
+// rows) to as many as it is measured to beat the tile kernels with - later where those need the normalisation's launch in front
+// (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against 5.1), earlier
+// for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer). An explicit GEMM threshold
+// (fa_set_gemm_min_m) wins.
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const uint32_t min_m = ctx->qkv_rows32_min_m ? ctx->qkv_rows32_min_m : PANEL_MIN_M_DEFAULT;
-    const uint32_t max_m = l.k_dim <= 1024 ? 512u : l.k_dim <= 2048 ? 128u : 64u;
+    const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : 192u) : l.k_dim <= 2048 ? 128u : l.weight_bits == 16 ? 64u : 48u;
     if (min_m > 32 || l.m < min_m || l.m > max_m || l.k_dim > 3072 || l.k_dim % 32 != 0) return false;
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     return aligned16(l.x) && aligned16(l.w[0]) && aligned16(l.w[1]) && aligned16(l.w[2]) && aligned16(l.gamma);

@@ -1,0 +1,456 @@
+// The tile kernels of FusedQkv / MatMul for many input rows: out[m, n] = x[m, :] . W[n, :] as output tiles that one workgroup
+// computes over the whole of k_dim (no partial sums to write, read and add), both operands moving from memory straight into LDS.
+//
+// What bounds them, and what follows from it:
+//   * a chunk of a few hundred rows has few tiles, and its time is one workgroup's chain: with 64 x 64 tiles over 2048 features
+//     32 steps of 16 KiB at the 110 KB/us that a CU draws from L2 would be 5 us. A step is 45 instructions per wave here: the
+//     operands of step k + 1 go from LDS to registers between the products of step k, so no product waits for LDS; places in LDS
+//     are constants of the loop that is unrolled over the stages; one barrier per step. (283 rows, 3072 x 2048 weights: 9.2 us
+//     against 18.9 with the 128 x 128 split-K kernel and the launch that added its parts; 500 rows, 1152 x 896: 5.3 against 14.3.)
+//   * the LDS loads of a wave are accepted one KiB every 20 cycles or so, and a wave waits meanwhile: issued in one go after the
+//     barrier they leave the matrix cores idle. They are spread between the products (256 x 160: 98 -> 66 us at 2048 rows,
+//     5120 x 3072, where the split-K form took 74.7).
+//   * large launches read less per product with larger tiles but leave CUs idle where the tiles do not fill a round of
+//     workgroups: five shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 is there for the
+//     5120 x 2048 products of a 2048-row prompt - one tile on each of 256 CUs - and may hold rows of two matrices (JOINED).
+//   * block-quantised weights stay as they are up to the registers, where a wave turns its operands to f16 right in front of the
+//     product (f16(weight * scale), as the reference's tile loader: see fa_gemm.hip). That is 14 vector instructions per 8
+//     weights, and with one wave per SIMD they add to the chain; so that no two waves convert the same weights, the waves of a
+//     tile share the features of a step instead of the input rows (KG) where the tile is small (283 rows, 3072 x 2048 Q8_0:
+//     13.0 -> 9.7 us), and their sums meet in the write stage. The scales of the tile's rows are all in LDS from the start:
+//     a request for 4 bytes of each row would cost the memory unit as much as one for 16 (15.4 -> 13.0 us).
+// F16 sums run over the features in order, whatever the tile: all shapes, and the register-staged kernel, agree to the bit.
+#pragma once
+#include "fa_gemm.h"
+#include "fa_lds_dma.h"
+#include <atomic>
+#include <type_traits>
+
+namespace fa_tile {
+
+using namespace fa_gemm;
+typedef uint32_t u2v_t __attribute__((ext_vector_type(2)));
+
+// LDS layouts. The 64 lanes of a request fill one KiB of consecutive LDS bytes in lane order, so padding is impossible; instead a
+// KiB holds a whole number of rows, and a lane fetches, within its row, the 16-byte piece that belongs into its slot:
+//   input, row-major F16 weights   8 rows x 8 pieces,   slot = piece ^ (row / 2) % 8
+//   canonical F16, row-major Q8_0  16 rows x 4 pieces,  slot = piece ^ (row / 4) % 4
+//   canonical Q8_0                 32 rows x 2 pieces,  slot = piece ^ (row / 8) % 2
+//   Q4_0                           64 rows x 1 piece or 32 x 2, in order
+// so that the lanes of an operand read fall into different banks while the lanes of a request cover whole runs of memory. Rows
+// past the end of a matrix (or of the input) are outside the buffer descriptor, or other rows of it: what they give is not stored.
+//
+// WB bits per weight; WM x WN waves over (input rows, weight rows), each of them KG times, for a share of every 64 features; a wave
+// owns TM x TN tiles of 32 x 32; NS stages of 64 features.
+template <int WB_, bool CANON_, int WM_, int WN_, int KG_, int TM_, int TN_, int NS_, bool JOINED_ = false>
+struct Shape {
+    static constexpr int WB = WB_, WM = WM_, WN = WN_, KG = KG_, TM = TM_, TN = TN_, NS = NS_;
+    static constexpr bool CANON = CANON_, QUANT = WB_ != 16;
+    // The tiles run over the rows of all matrices as one list (F16; whole groups of 32 rows per matrix): a tile may hold rows of two.
+    static constexpr bool JOINED = JOINED_;
+    static_assert(!JOINED || WB == 16, "F16 only");
+    static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = 4 / KG;  // KN: products of 16 features per wave and stage
+    static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
+    static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
+    static constexpr int XR = X_BYTES / 1024 / NW;  // 1 KiB requests per wave and stage
+    static constexpr int W_REQ = W_BYTES / 1024, WR = W_REQ >= NW ? W_REQ / NW : 1;
+    static constexpr int REQ = XR + WR;
+    // what a lane reads of a weight row at a time: the 8 features of a product, of both halves of the wave where they are 4 bytes
+    typedef typename std::conditional<WB_ == 16, h8_t, u2v_t>::type raw_t;
+    static constexpr int READS = KN * (TM + TN);
+    static constexpr int T_STRIDE = NTR * 4 + 16, T_BYTES = WM * 32 * T_STRIDE;
+    // LDS: the stages, then (block-quantised) all scales of the tile's rows, [8 blocks][row]; the write stage over both
+    static constexpr uint32_t scale_bytes(uint32_t k_dim) { return QUANT ? (k_dim + 255) / 256 * (NTR * 16) : 0u; }
+    static constexpr uint32_t lds_bytes(uint32_t k_dim) {
+        const uint32_t s = NS * STAGE + scale_bytes(k_dim);
+        return s > (uint32_t)(KG * T_BYTES) ? s : (uint32_t)(KG * T_BYTES);
+    }
+    static_assert(X_BYTES % (1024 * NW) == 0 && (W_REQ % NW == 0 || NW % W_REQ == 0), "whole requests per wave");
+    static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63 && NTR >= 64, "LDS of a compute unit; the request counter");
+};
+
+enum TileShape { TILE_64x64_DEEP, TILE_64x64, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };  // input rows x weight rows (the first: block-quantised, more stages)
+
+template <int N>
+__device__ __forceinline__ void wait_requests() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// Workgroup barrier behind which this wave's LDS reads have arrived. (The wait is the builtin and not assembly: the compiler has to
+// know that no read is outstanding, or it waits again, behind the reads of the next step.)
+__device__ __forceinline__ void meet() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// 8 int8 weights (two words) -> f16, exactly (see q8_to_f16)
+__device__ __forceinline__ h8_t q8x8_to_f16(uint32_t a, uint32_t b) {
+    const h2v_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+    h8_t r;
+#pragma unroll
+    for (int hw = 0; hw < 2; ++hw) {
+        const uint32_t u = (hw ? b : a) ^ 0x80808080u;
+        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
+        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
+        r[4 * hw + 0] = lo[0], r[4 * hw + 1] = lo[1], r[4 * hw + 2] = hi[0], r[4 * hw + 3] = hi[1];
+    }
+    return r;
+}
+
+template <class S, int MIN_WAVES>
+__global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)smem;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave % S::WN, wm = wave / S::WN % S::WM, kg = wave / (S::WN * S::WM);
+    const uint32_t K = a.k_dim, n_steps = K / 64;
+
+    // Tile of this workgroup. Workgroup ids go round the 8 XCDs; the ids of one XCD are given consecutive tiles (weight rows
+    // outermost), so that a weight tile is fetched into one L2 only.
+    const uint32_t total = a.n_tiles * a.m_tiles, per_xcd = gridDim.x >> 3;
+    const uint32_t v = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+    if (v >= total) return;
+    uint32_t nt, mt;
+    {
+        const uint32_t G = a.m_tiles > 8 ? 4u : 1u;  // (of many input rows, the tiles at work together in an XCD are 8 x 4, not 16 x 2)
+        const uint32_t panel = v / (G * a.m_tiles), rem = v - panel * G * a.m_tiles, w = min(G, a.n_tiles - panel * G);
+        mt = rem / w, nt = panel * G + rem - mt * w;
+    }
+    int tile_mat = 0;
+    if (!S::JOINED && nt >= a.tiles[0]) {
+        nt -= a.tiles[0], tile_mat = 1;
+        if (nt >= a.tiles[1]) nt -= a.tiles[1], tile_mat = 2;
+    }
+    auto pick3 = [](int mat, auto x0, auto x1, auto x2) { return mat == 0 ? x0 : mat == 1 ? x1 : x2; };
+    const uint32_t rows0 = a.rows[0], rows1 = a.rows[1], n0 = nt * S::NTR, m0 = mt * S::MT;
+    const uint32_t N_tile = tile_mat == 0 ? rows0 : rows1;
+
+    // Matrix and weight row of tile row t. With the NeoX rotation as the write stage, 32 tile rows are 16 rows of a head and the 16
+    // that they are rotated with, half a head further on, so that a tile of any width holds both of a pair.
+    const bool pairs = a.rope.on && a.rope.apply && !a.rope.normal;
+    const uint32_t hd_shift = a.rope.head_dim == 128 ? 7u : 6u;
+    auto paired = [&](uint32_t r) -> uint32_t {
+        if (!pairs) return r;
+        const uint32_t g = r >> 5, head = g >> (hd_shift - 5), within = g & ((1u << (hd_shift - 5)) - 1u);
+        return (head << hd_shift) + within * 16 + (r & 15u) + ((r & 16u) ? 1u << (hd_shift - 1) : 0u);
+    };
+    auto matrix_of = [&](uint32_t &r) -> int {  // r: row of the list -> row of its matrix
+        int mat = tile_mat;
+        if (S::JOINED && r >= rows0) {
+            r -= rows0, mat = 1;
+            if (r >= rows1) r -= rows1, mat = 2;
+        }
+        return mat;
+    };
+    auto weight_row = [&](uint32_t t) -> uint32_t { return paired(n0 + t); };  // (not JOINED)
+
+    // Requests of this wave. Input: KiB q = rows 8q .. + 7 of 128 bytes, slot = piece ^ (row / 2) % 8.
+    int xv[S::XR], wv[S::WR];
+#pragma unroll
+    for (int i = 0; i < S::XR; ++i) {
+        const uint32_t row = (wave * S::XR + i) * 8 + (lane >> 3);
+        xv[i] = (int)(row * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
+    }
+    uint32_t w_block[S::WR];  // canonical: which of the stage's two 32-feature blocks
+#pragma unroll
+    for (int i = 0; i < S::WR; ++i) {
+        const uint32_t q = (wave * S::WR + i) % S::W_REQ;
+        w_block[i] = 0;
+        if constexpr (S::CANON) {
+            constexpr uint32_t PER_BLOCK = S::W_REQ / 2;
+            const uint32_t u = q % PER_BLOCK;
+            w_block[i] = q / PER_BLOCK;
+            if constexpr (S::WB == 16) {
+                const uint32_t row = u * 16 + (lane >> 2);
+                wv[i] = (int)(weight_row(row) * 64 + ((lane & 3) ^ ((row >> 2) & 3)) * 16);
+            } else if constexpr (S::WB == 8) {
+                const uint32_t row = u * 32 + (lane >> 1);
+                wv[i] = (int)(weight_row(row) * 32 + ((lane & 1) ^ ((row >> 3) & 1)) * 16);
+            } else {
+                wv[i] = (int)(weight_row(u * 64 + lane) * 16);
+            }
+        } else {
+            if constexpr (S::WB == 16) {
+                const uint32_t row = q * 8 + (lane >> 3);
+                wv[i] = (int)(weight_row(row) * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
+            } else if constexpr (S::WB == 8) {
+                const uint32_t row = q * 16 + (lane >> 2);
+                wv[i] = (int)(weight_row(row) * K + ((lane & 3) ^ ((row >> 2) & 3)) * 16);
+            } else {
+                const uint32_t row = q * 32 + (lane >> 1);
+                wv[i] = (int)(weight_row(row) * (K / 2) + (lane & 1) * 16);
+            }
+        }
+    }
+    const fa_lds_dma::rsrc_words x_rs = fa_lds_dma::make_rsrc_words(reinterpret_cast<const unsigned char *>(a.x) + (size_t)m0 * K * 2, (a.m - m0) * K * 2);
+    const uint32_t w_block_bytes = N_tile * 4 * S::WB;  // canonical: one 32-feature block of the matrix
+    uint32_t w_step[S::WR];                             // JOINED: bytes between the steps of a request's matrix
+    fa_lds_dma::rsrc_words w_rs;
+    if constexpr (S::JOINED) {
+        // one descriptor over all matrices, which lie within 4 GiB (the host has seen to that)
+        w_rs = fa_lds_dma::make_rsrc_words(a.w_low, a.w_span);
+#pragma unroll
+        for (int i = 0; i < S::WR; ++i) {
+            const uint32_t q = wave * S::WR + i, u = S::CANON ? q % (S::W_REQ / 2) : q;
+            const uint32_t row = S::CANON ? u * 16 + (lane >> 2) : u * 8 + (lane >> 3);  // of the tile
+            uint32_t r = min(n0 + (S::CANON ? u * 16 : u * 8), rows0 + 2 * rows1 - (S::CANON ? 16 : 8));  // (rows past the end: the last ones again)
+            const int mat = matrix_of(r);
+            const uint32_t at = pick3(mat, a.w_at[0], a.w_at[1], a.w_at[2]), wr = paired(r + (S::CANON ? lane >> 2 : lane >> 3)), rows = mat ? rows1 : rows0;
+            if constexpr (S::CANON)
+                wv[i] = (int)(at + w_block[i] * rows * 64 + wr * 64 + ((lane & 3) ^ ((row >> 2) & 3)) * 16), w_step[i] = rows * 128;
+            else
+                wv[i] = (int)(at + wr * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16), w_step[i] = 128;
+        }
+    } else {
+        w_rs = fa_lds_dma::make_rsrc_words(pick3(tile_mat, a.w[0], a.w[1], a.w[2]), N_tile * (K / 8 * S::WB));
+    }
+    // What the next step's requests start from: byte offsets that grow by the same amount per step. (Past the last step the
+    // descriptors are made empty: nothing is read, zeros arrive, and the counts that the waits go by stay the same.)
+    uint32_t asked = 0, x_soff = 0, w_soff = 0;
+    fa_lds_dma::rsrc_words x_now = x_rs, w_now = w_rs;
+    auto request = [&](int r, uint32_t stage) __attribute__((always_inline)) {
+        const uint32_t base = lds_base + stage;
+        if (r < S::WR) {
+            const uint32_t q = (wave * S::WR + r) % S::W_REQ;
+            if constexpr (S::JOINED) {
+                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], 0);
+                wv[r] += w_step[r];
+            } else {
+                const uint32_t soff = S::CANON ? w_soff + (w_block[r] ? w_block_bytes : 0u) : w_soff;
+                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
+            }
+        } else {
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, base + (wave * S::XR + r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
+        }
+        if (r == S::REQ - 1) {  // the step's last one
+            ++asked, x_soff += 128, w_soff += S::CANON ? 2 * w_block_bytes : 8 * S::WB;
+            const bool in = asked < n_steps;
+            x_now.z = in ? x_rs.z : 0u, w_now.z = in ? w_rs.z : 0u;
+        }
+    };
+
+    // Operand reads: lane l reads row l % 32 (+ 32 per tile) and the 8 features l / 32 of each 16. Places within a stage, of product
+    // q of this wave (features 16 kk .. + 15 of the stage's 64):
+    const uint32_t h = lane >> 5, r32 = lane & 31;
+    uint32_t x_at[S::KN], w_at[S::KN];
+    const uint32_t w_row = wn * S::TN * 32 + r32;  // (+ 32 per tile: the same place in the pattern)
+    constexpr uint32_t W_TILE = S::WB == 16 ? (S::CANON ? 2048 : 4096) : S::WB == 8 ? (S::CANON ? 1024 : 2048) : (S::CANON ? 512 : 1024);
+#pragma unroll
+    for (int q = 0; q < S::KN; ++q) {
+        const uint32_t kk = kg * S::KN + q, b = kk >> 1, half = kk & 1;
+        x_at[q] = wm * S::TM * 4096 + (r32 >> 3) * 1024 + (r32 & 7) * 128 + ((2 * kk + h) ^ ((r32 >> 1) & 7)) * 16;
+        if constexpr (S::WB == 16) {
+            w_at[q] = S::CANON ? b * (S::NTR * 64) + (w_row >> 4) * 1024 + (w_row & 15) * 64 + ((2 * half + h) ^ ((w_row >> 2) & 3)) * 16
+                               : (w_row >> 3) * 1024 + (w_row & 7) * 128 + ((2 * kk + h) ^ ((r32 >> 1) & 7)) * 16;
+        } else if constexpr (S::WB == 8) {
+            w_at[q] = S::CANON ? b * (S::NTR * 32) + (w_row >> 5) * 1024 + (w_row & 31) * 32 + (half ^ ((w_row >> 3) & 1)) * 16 + h * 8
+                               : (w_row >> 4) * 1024 + (w_row & 15) * 64 + (kk ^ ((w_row >> 2) & 3)) * 16 + h * 8;
+        } else {  // (the 8 bytes of both halves of the wave: 4 bytes per lane would be two lanes to a bank)
+            w_at[q] = S::CANON ? b * (S::NTR * 16) + w_row * 16 + half * 8 : (w_row >> 5) * 1024 + (w_row & 31) * 32 + kk * 8;
+        }
+        w_at[q] += S::X_BYTES;
+    }
+    // The operands of one stage as they lie in LDS (block-quantised weights become f16 in registers, in front of the product).
+    struct Operands {
+        typename S::raw_t w[S::TN][S::KN];
+        h8_t x[S::TM][S::KN];
+    };
+    auto fetch = [&](Operands &o, uint32_t stage, int e) __attribute__((always_inline)) {  // read number e of the stage
+        const int q = e / (S::TM + S::TN), t = e % (S::TM + S::TN);
+        if (t < S::TM) o.x[t][q] = *reinterpret_cast<const h8_t *>(smem + x_at[q] + stage + t * 4096);
+        else o.w[t - S::TM][q] = *reinterpret_cast<const typename S::raw_t *>(smem + w_at[q] + stage + (t - S::TM) * W_TILE);
+    };
+    u4v_t scales[S::TN] = {};  // of the wave's rows, 8 blocks = 4 stages
+    const unsigned char *scale_at = smem + S::NS * S::STAGE + w_row * 16;
+    auto fetch_scales = [&]() __attribute__((always_inline)) {
+        if constexpr (S::QUANT) {
+#pragma unroll
+            for (int i = 0; i < S::TN; ++i) scales[i] = *reinterpret_cast<const u4v_t *>(scale_at + i * 512);
+            scale_at += S::NTR * 16;
+        }
+    };
+    auto w_operand = [&](const Operands &o, int i, int q, int ks4) __attribute__((always_inline)) -> h8_t {
+        if constexpr (S::WB == 16) {
+            return o.w[i][q];
+        } else {
+            const uint32_t pair = scales[i][ks4];  // (a copy: the bit cast of a vector's element takes element 0)
+            const h2v_t s2 = __builtin_bit_cast(h2v_t, pair);
+            _Float16 s;
+            if constexpr (S::KG == 1) s = s2[q >> 1];
+            else if constexpr (S::KG == 2) s = kg ? s2[1] : s2[0];
+            else s = kg >= 2 ? s2[1] : s2[0];
+            const h8_t sc = {s, s, s, s, s, s, s, s};
+            if constexpr (S::WB == 8) return q8x8_to_f16(o.w[i][q].x, o.w[i][q].y) * sc;
+            else return q4_to_f16(h ? o.w[i][q].y : o.w[i][q].x) * sc;
+        }
+    };
+
+    f16v_t acc[S::TN][S::TM];
+#pragma unroll
+    for (int i = 0; i < S::TN; ++i)
+#pragma unroll
+        for (int j = 0; j < S::TM; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    if constexpr (S::QUANT) {  // all scales first: 16 bytes (8 blocks) of 64 rows per request
+        const __half *sp = pick3(tile_mat, a.scales[0], a.scales[1], a.scales[2]);
+        const fa_lds_dma::rsrc_words s_rs = fa_lds_dma::make_rsrc_words(sp, N_tile * (K / 32) * 2);
+        for (uint32_t q = wave; q < (K + 255) / 256 * (S::NTR / 64); q += S::NW)
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base + S::NS * S::STAGE + q * 1024, (int)(weight_row(q % (S::NTR / 64) * 64 + lane) * (K / 32) * 2),
+                                                    (int)(q / (S::NTR / 64) * 16));
+    }
+#pragma unroll
+    for (int s = 0; s < S::NS; ++s)
+#pragma unroll
+        for (int r = 0; r < S::REQ; ++r) request(r, s * S::STAGE);
+    Operands o0, o1;
+    wait_requests<S::REQ *(S::NS - 1)>();
+    meet();
+#pragma unroll
+    for (int e = 0; e < S::READS; ++e) fetch(o0, 0, e);
+    // A step multiplies the operands that are in registers while it fetches the next step's from LDS. At its barrier every wave has
+    // the operands of step ks in registers - their stage is free for step ks + NS - and step ks + 1 has landed for everybody.
+    // The requests go out between the products: the memory unit takes a KiB in about 20 cycles, and a wave that issues all of its
+    // requests in one go leaves its matrix core idle for as long.
+    auto step = [&](uint32_t cur, uint32_t next, int ks4, const Operands &now, Operands &then) __attribute__((always_inline)) {
+        wait_requests<S::REQ *(S::NS - 2)>();
+        meet();
+        constexpr int NM = S::KN * S::TN * S::TM;
+        if (ks4 == 0) fetch_scales();
+        h8_t fa[S::TN];
+#pragma unroll
+        for (int p = 0; p < NM; ++p) {
+            const int q = p / (S::TN * S::TM), i = p / S::TM % S::TN, j = p % S::TM;
+#pragma unroll
+            for (int e = p * S::READS / NM; e < (p + 1) * S::READS / NM; ++e) fetch(then, next, e);
+            if (j == 0) fa[i] = w_operand(now, i, q, ks4);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], now.x[j][q], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0x6);  // (vector and scalar arithmetic may move: addresses, the conversion of weights)
+#pragma unroll
+            for (int r = p * S::REQ / NM; r < (p + 1) * S::REQ / NM; ++r) request(r, cur);
+            __builtin_amdgcn_sched_barrier(0x6);
+        }
+    };
+    // (unrolled over the stages, so that their places are constants; operands of even and odd steps in registers of their own)
+    constexpr int UNROLL = S::QUANT ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
+    for (uint32_t left = n_steps;;) {
+        bool done = false;
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t cur = u % S::NS * S::STAGE, next = (u + 1) % S::NS * S::STAGE;
+            if (u % 2 == 0) step(cur, next, u % 4, o0, o1);
+            else step(cur, next, u % 4, o1, o0);
+            if (--left == 0) {
+                done = true;
+                break;
+            }
+        }
+        if (done) break;
+    }
+    wait_requests<0>();  // (the last ones delivered nothing, but they have to be over before the write stage reuses the LDS)
+
+    // Write stage: accumulators -> LDS as f32 [input row][weight row], 32 input rows of every wave at a time, then
+    // alpha * sum + bias + beta * residual, one rounding to f16, 16-byte stores (or the rotation and the stores of KvPrepFused).
+#pragma unroll
+    for (int j = 0; j < S::TM; ++j) {
+        __syncthreads();  // every wave is done with the stages / the previous rows have been read out
+        // register r of lane l of a 32 x 32 tile is weight row 8 (r / 4) + 4 (l / 32) + r % 4 and input row l % 32
+#pragma unroll
+        for (int i = 0; i < S::TN; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+                *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + (wm * 32 + r32) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + g * 8 + h * 4) * 4) = q;
+            }
+        __syncthreads();
+        constexpr int PIECES = S::NTR / 8;
+        for (uint32_t q = tid; q < (uint32_t)(S::WM * 32 * PIECES); q += S::NT) {
+            const uint32_t t = q / PIECES, n8 = q % PIECES;
+            const uint32_t gm = m0 + ((t >> 5) * S::TM + j) * 32 + (t & 31);
+            uint32_t r = n0 + n8 * 8;
+            const int mat = matrix_of(r);
+            const uint32_t gn = paired(r), N = S::JOINED ? (mat ? rows1 : rows0) : N_tile;
+            if (gm >= a.m || r >= N) continue;
+            const __half *bias = pick3(mat, a.bias[0], a.bias[1], a.bias[2]);
+            __half *out = pick3(mat, a.out[0], a.out[1], a.out[2]);
+            const size_t o = (size_t)gm * N + gn;
+            const h8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+            const h8_t rv = a.residual ? *reinterpret_cast<const h8_t *>(a.residual + o) : z;
+            auto value = [&](uint32_t p8, uint32_t col, bool with_residual) -> h8_t {
+                f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + t * S::T_STRIDE + p8 * 32);
+                f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + t * S::T_STRIDE + p8 * 32 + 16);
+#pragma unroll
+                for (int k = 1; k < S::KG; ++k) {
+                    s0 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + t * S::T_STRIDE + p8 * 32);
+                    s1 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + t * S::T_STRIDE + p8 * 32 + 16);
+                }
+                const h8_t bv = bias ? *reinterpret_cast<const h8_t *>(bias + col) : z;
+                h8_t y;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float s = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
+                    if (bias) s += (float)bv[e];
+                    if (with_residual) s += a.beta * (float)rv[e];
+                    y[e] = (_Float16)s;
+                }
+                return y;
+            };
+            const h8_t y = value(n8, gn, a.residual != nullptr);
+            if (a.rope.on) {
+                h8_t mate = z;
+                if (pairs && mat != 2) mate = value(n8 ^ 2, paired(r ^ 16), false);
+                rope_store_piece(a, mat, gm, gn, y, mate);
+            } else {
+                *reinterpret_cast<h8_t *>(out + o) = y;
+            }
+        }
+    }
+}
+
+template <class S, int MIN_WAVES>
+fa_status launch_shape(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
+    static std::atomic<bool> lds_allowed_on[64];  // per device (contexts of several threads may get here together: the calls are idempotent)
+    std::atomic<bool> &lds_allowed = lds_allowed_on[ctx->device & 63];
+    if (!lds_allowed.load(std::memory_order_acquire)) {
+        FA_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<S, MIN_WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        lds_allowed.store(true, std::memory_order_release);
+    }
+    a.n_tiles = 0, a.m_tiles = ceil_div_u32(a.m, S::MT);
+    for (int i = 0; i < 3; ++i) a.tiles[i] = ceil_div_u32(a.rows[i], S::NTR), a.n_tiles += a.tiles[i];
+    if (S::JOINED) a.n_tiles = ceil_div_u32(a.rows[0] + 2 * a.rows[1], S::NTR);
+    const uint32_t grid = ceil_div_u32(a.n_tiles * a.m_tiles, 8) * 8;
+    scope.launch((tile_gemm_kernel<S, MIN_WAVES>), dim3(grid), dim3(S::NT), S::lds_bytes(a.k_dim), a);
+    return FA_OK;
+}
+
+template <int WB, bool CANON>
+fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDev &a) {
+    if constexpr (WB == 16) {
+        switch (shape) {
+            case TILE_64x64_DEEP:
+            case TILE_64x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 1, 1, 4>, 2>(ctx, scope, a);
+            case TILE_128x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 2, 1, 3>, 2>(ctx, scope, a);
+            case TILE_128x128: return launch_shape<Shape<WB, CANON, 2, 4, 1, 2, 1, 4>, 2>(ctx, scope, a);
+            case TILE_256x128: return launch_shape<Shape<WB, CANON, 4, 2, 1, 2, 2, 3>, 2>(ctx, scope, a);
+            case TILE_256x160: return launch_shape<Shape<WB, CANON, 4, 1, 1, 2, 5, 3, true>, 1>(ctx, scope, a);
+        }
+    } else {
+        switch (shape) {
+            case TILE_64x64_DEEP: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 8>, 1>(ctx, scope, a);
+            case TILE_64x64: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 4>, 2>(ctx, scope, a);
+            case TILE_128x64: return launch_shape<Shape<WB, CANON, 1, 2, 4, 4, 1, 4>, 2>(ctx, scope, a);
+            case TILE_128x128: return launch_shape<Shape<WB, CANON, 1, 4, 2, 4, 1, 4>, 2>(ctx, scope, a);
+            case TILE_256x128: return launch_shape<Shape<WB, CANON, 2, 4, 1, 4, 1, 3>, 2>(ctx, scope, a);
+            case TILE_256x160: break;
+        }
+    }
+    return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "no such tile");
+}
+
+fa_status launch_f16(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDev &a, bool canonical);
+fa_status launch_q8(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDev &a, bool canonical);
+fa_status launch_q4(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDev &a, bool canonical);
+
+}  // namespace fa_tile

@@ -1,0 +1,73 @@
+"""GPU parity of the tile kernels of FusedQkv and MatMul (fa_tile.h): fewer steps than stages, steps that do not fill the unrolled
+loop, tiles cut off by the last input or weight row, every tile shape (by the number of tiles that the launch has), tiles that hold
+rows of two matrices, and both head widths of the NeoX write stage. Against the oracle with the bars of test_gpu_qkv.py; the fused
+write stage against the two ops, bit for bit."""
+import numpy as np
+import pytest
+
+import foundry_attn as fa
+import orc
+from gpu_util import announce, bits, ctx
+from test_gpu_qkv import _close, _data
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
+    (64, 3, 1, 64, 12, 1),        # one step, one ragged tile
+    (192, 1, 1, 128, 65, 0),      # three steps, a second tile of one row
+    (320, 5, 1, 64, 130, 1),      # five steps
+    (896, 2, 1, 64, 513, 0),      # fourteen steps: seven pairs, scales of three and a half units
+    (128, 16, 2, 64, 1030, 1),    # 128 x 64 tiles
+    (576, 14, 2, 64, 2047, 0),    # 128 x 128 tiles
+    (128, 40, 8, 64, 1000, 1),    # 256 x 128 tiles
+    (128, 24, 8, 128, 2040, 1),   # F16: 256 x 160 tiles, some with rows of two matrices
+    (192, 24, 8, 128, 2048, 0),
+])
+def test_tiles(K, H, Hkv, D, m, layout, weights):
+    announce("tiles", K, H, Hkv, D, m, layout, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + H + m)
+    N, NK = H * D, Hkv * D
+    x, g, ws, bs = _data(rng, K, N, NK, m)
+    res = rng.uniform(-1, 1, (m, N)).astype(np.float16)
+    scales, dev_s = None, []
+    if weights == "f16":
+        dev_w = [f.array(orc.to_canonical(w) if layout else w.reshape(-1)) for w in ws]
+        arg = [w.arg() for w in dev_w]
+        full = ws
+    else:
+        quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
+        dev_s = [f.array(s) for _, s in quant]
+        scales = [s.arg() for s in dev_s]
+        flat = [orc.to_canonical(q) if layout else q.reshape(-1) for q, _ in quant]
+        dev_w = [f.array(q if weights == "q8" else orc.pack_q4_0(q)) for q in flat]
+        arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev_w, (N, NK, NK))]
+        full = [orc.dequantize_blocks(q, s) for q, s in quant]
+    dx, dg, db, dres, dout = f.array(x), f.array(g), [f.array(b) for b in bs], f.array(res), f.zeros((m, N))
+    outs = [f.zeros((m, n)) for n in (N, NK, NK)]
+    cos, sin = fa.rope_tables(5e5, D, m + 3)
+    dcos, dsin = f.array(cos), f.array(sin)
+    rot = [[f.zeros((H, m, D)), f.zeros((Hkv, m + 3, D)), f.zeros((Hkv, m + 3, D))] for _ in range(2)]
+    kw = dict(gamma=dg.arg(), biases=[b.arg() for b in db], layout=layout, scales=scales)
+    try:
+        f.set_gemm_min_m(12)
+        f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, **kw)
+        for o, w, name in zip(outs, orc.fused_qkv(x, *full, gamma=g, biases=bs, layout=0), "qkv"):
+            assert _close(o.download(), w, K), name
+        for mode in (fa.ROPE_NEOX, fa.ROPE_NORMAL):
+            p = fa.KvPrepFusedParams.make(H, Hkv, D, m, 2, m + 3, mode)
+            f.kv_prep_fused(*[o.arg() for o in outs], *[t.arg() for t in rot[0]], dcos.arg(), dsin.arg(), p)
+            f.fused_qkv_kv_prep(dx.arg(), *arg, K, rot[1][0].arg(), dcos.arg(), dsin.arg(), p, k_cache=rot[1][1].arg(),
+                                v_cache=rot[1][2].arg(), **kw)
+            for one, two in zip(rot[0], rot[1]):
+                assert np.array_equal(bits(one.download()), bits(two.download())), mode
+        f.matmul(dx.arg(), arg[0], dout.arg(), m, N, K, bias=db[0].arg(), c=dres.arg(), transpose_b=layout == 0, alpha=0.5, beta=0.75,
+                 b_scales=scales[0] if scales else None)
+        want = orc.matmul_gemv(x, full[0], bs[0], res, 0, 32, 0.5, 0.75).astype(np.float64)
+        assert np.all(np.abs(dout.download() - want) <= 2 * np.maximum(np.abs(want), 2.0 ** -10) * 2.0 ** -10 + 1e-4)
+    finally:
+        f.set_gemm_min_m()
+    for b in dev_w + dev_s + [dx, dg, dres, dout, dcos, dsin] + db + outs + rot[0] + rot[1]:
+        b.free()
