@@ -98,6 +98,24 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     };
     uint32_t waves = ctx->decode_waves;  // 0 = by the rule above
     bool short_context = false;
+    // A paged batch whose partitions the kernel deals out by the lengths (batch_place): one round of resident workgroups, merged
+    // inside the launch, from where the rule above would give a workgroup 512 keys of 128 dims or more - below that a workgroup has
+    // one round of requests whatever its keys, and looking for its place costs 0.4 to 2 us that nothing repays (Hkv 2, D 128, 8
+    // sequences of 500 to 4000 tokens, 256 keys: 10.3 -> 12.4 us). Eight waves while there are two slots per sequence, four
+    // (twice the slots) beyond; with fewer than two the quotients leave too much idle. us per step, by the bound and by the lengths:
+    //   Hkv 2, D 128: 24 sequences of 100-4000 tokens 20.8 -> 17.8, 32 of 512-16384 60.5 -> 52.0, 64 of 16-2000 23.4 -> 19.7
+    //   Hkv 8, D 128: 4 of 100-4000 13.0 -> 10.5, 8 of 100-8000 40.7 -> 30.1, 24 of 100-4000 50.9 -> 40.4 (eight waves: 48.0)
+    //   Hkv 2, D 64:  64 of 16-4000 26.1 -> 18.8;  Hkv 4, D 128: 50 of 500-3000 52.6 -> 39.3
+    //   equal lengths have nothing to gain: Hkv 8, D 128: 8 of 2000 16.4 -> 16.8
+    uint32_t bal_slots = 0;
+    if (L.paged && L.d_len && L.batch >= 2 && L.batch <= 64 && chunk == 0 && ctx->decode_variant.merge == 2 && !L.static_scratch &&
+        bound <= (1u << 24) && auto_chunk(8, n_cus) * L.head_dim >= 512u * 128u) {
+        const uint32_t per8 = (uint32_t)(n_cus / ny);
+        const uint32_t w = waves ? waves : 2u * L.batch <= per8 ? 8u : 4u;
+        const uint32_t n = w == 4u ? 2u * per8 : per8;
+        const size_t records = (size_t)n * ny * (size_t)gt * L.head_dim / 4 * 32;
+        if (n >= 2u * L.batch && records <= ctx->poll_ws_bytes) bal_slots = n, waves = w;
+    }
     if (waves == 0) {
         const uint32_t c8 = chunk ? chunk : auto_chunk(8, n_cus);
         waves = groups * ceil_div_u32(bound, (c8 + BK - 1) / BK * BK) > n_cus ? 4u : 8u;
@@ -114,7 +132,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     chunk = (chunk + BK - 1) / BK * BK;
     // the int8 step in one launch: the open 32-row block must lie inside one partition
     if (L.sage_fused) chunk = (chunk + FA_SAGE_BLOCK - 1) / FA_SAGE_BLOCK * FA_SAGE_BLOCK;
-    const uint32_t S = ceil_div_u32(bound, chunk);
+    const uint32_t S = bal_slots ? bal_slots : ceil_div_u32(bound, chunk);
     // a contiguous cache slab is addressed with 32-bit byte offsets (tile base included)
     if (!L.paged && ((uint64_t)L.capacity + chunk + MBX * BK) * L.head_dim * 2 >= (1ull << 32))
         return fa_fail(FA_ERR_INVALID_SHAPE, "flash decode: one KV head of the contiguous cache must stay below 4 GiB");
@@ -151,9 +169,14 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         const uint32_t nt = waves * 64;
         // a workgroup reads ceil(n4 / partitions) columns of every partition (fewer than n4 + partitions records for
         // any partition count up to S), at most POLL_IPT records per thread
-        polled = S > 1 && groups * S <= slots && need <= ctx->poll_ws_bytes && (uint64_t)n4 + S <= (uint64_t)nt * POLL_IPT;
+        polled = bal_slots || (S > 1 && groups * S <= slots && need <= ctx->poll_ws_bytes && (uint64_t)n4 + S <= (uint64_t)nt * POLL_IPT);
+        a.bal_batch = bal_slots ? L.batch : 0u;
+        if (bal_slots && ctx->xcd_round_robin && bal_slots * ny % 8 == 0 && bal_slots >= 2) {
+            a.bal_per_xcd = bal_slots * ny / 8;
+            a.rcp_gx = (uint32_t)((1ull << 32) / bal_slots) + 1u;  // (exact for the few hundred workgroups of such a launch)
+        }
         a.merge_in_kernel = polled ? 2u : 0u;
-        a.xcd_local = polled && ctx->xcd_round_robin && groups % 8 == 0 ? 1u : 0u;
+        a.xcd_local = polled && !bal_slots && ctx->xcd_round_robin && groups % 8 == 0 ? 1u : 0u;
         // Fewer than 8 head groups (Qwen2.5-0.5B has 2 KV heads) and few enough partitions for an XCD to hold a group's
         // workgroups: the grid is padded to 8 head groups, group g's workgroups land on XCD g, and the workgroups of
         // the groups that do not exist leave at once. Such a launch is all latency (its partitions were sized for that
@@ -212,7 +235,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         const uint32_t streaming = (mode == MODE_FUSED || mode == MODE_FUSED_PAGED || mode == MODE_SAGE_FUSED) ? waves - 1 : waves;
         a.nb_q = (chunk / BK) / streaming, a.nb_r = (chunk / BK) % streaming;
     }
-    dim3 grid(S, ny_grid, L.batch);
+    dim3 grid(S, ny_grid, bal_slots ? 1u : L.batch);
     if (a.xcd_local) {
         // the kernel's reciprocals (see there): every workgroup index and both divisors stay below 2^16
         // (a divisor of 1 has no such reciprocal in 32 bits)

@@ -416,14 +416,13 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 // folds them with lane exchanges. A wave depends on no other wave.
 template <int D, bool LOCAL>
 __device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t c,
-                                                        uint32_t nsplits, uint32_t S, int tid) {
+                                                        uint32_t nsplits, size_t first, int tid) {  // first: the group's first partition
     constexpr int LD_POLICY = LOCAL ? 0x10 /* sc1 */ : CACHE_COHERENT, ST_POLICY = LOCAL ? 0 : CACHE_COHERENT;
     constexpr int CG = D / 4;
     const uint32_t gt = a.gt, n4 = gt * CG;
     const uint32_t sh = 32u - (uint32_t)__builtin_clz(nsplits - 1u);  // 2 <= nsplits <= 64: 1 .. 6
     const uint32_t p = (uint32_t)tid & ((1u << sh) - 1u), gi = (uint32_t)tid >> sh, gpw = (uint32_t)NT >> sh;
-    const size_t g = (size_t)b * gridDim.y + y;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.part_acc + g * S * n4 * 8);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.part_acc + first * n4 * 8);
     const unsigned long long t_begin = wall_clock64();
     bool ok = true;
     for (uint32_t base = 0; c + base * nsplits < n4; base += gpw) {  // uniform over the workgroup
@@ -484,6 +483,86 @@ __device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint
         }
     }
     return ok;
+}
+
+// Sums over the wave and running sums along its lanes of a non-negative integer (DPP moves within the rows of 16 lanes, then the
+// rows' totals carried over).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(v), 63); }
+
+// ceil(n / c) for n < 2^24, c >= 1
+__device__ __forceinline__ uint32_t ceil_quot(uint32_t n, uint32_t c, float rcp) {
+    int q = (int)((float)n * rcp), r = (int)(n - (uint32_t)q * c);
+    if (r < 0) --q, r += (int)c;
+    if (r >= (int)c) ++q, r -= (int)c;
+    return (uint32_t)q + (r > 0 ? 1u : 0u);
+}
+
+// A batch's partitions, dealt to the workgroups by the lengths the sequences have now (which only the device knows). The host
+// sizes a launch by its length bound, the longest sequence: cut that way a batch of 24 sequences of 100 to 4000 tokens has
+// 240 workgroups of which half find nothing, while the others have 800 keys each. Here every wave reads all lengths (one
+// load, lane = sequence), looks for the smallest partition with which all sequences together need at most `slots`
+// workgroups - between (all keys) / slots and (all keys) / (slots - sequences), to 1/16 - and finds its own place in the
+// running sum of the sequences' partition counts.
+struct BatchPlace {
+    uint32_t b, split, nsplits, first, len;  // first: the slot of the sequence's first partition; nsplits 0: nothing to do
+    bool dropped;                            // some sequence is longer than the launch may attend
+};
+__device__ __forceinline__ BatchPlace batch_place(const DecodeDev &a, uint32_t slot, uint32_t slots, uint32_t min_blocks) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t raw = lane < a.bal_batch ? a.d_len[(size_t)lane * a.d_len_stride] + a.kv_len_add : 0u;
+    const uint32_t blocks = (min(raw, min(a.capacity, a.kv_len_bound)) + BK - 1) / BK;
+    const uint32_t total = wave_sum(blocks);
+    // at least min_blocks, and at most 64 partitions per sequence (what the merge in registers takes)
+    const uint32_t bound_blocks = (min(a.capacity, a.kv_len_bound) + BK - 1) / BK;
+    uint32_t floor_c = min_blocks;
+    if (bound_blocks > 64u * min_blocks) {
+        uint32_t longest = blocks;
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x111, 0xf, 0xf, false));
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x112, 0xf, 0xf, false));
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x114, 0xf, 0xf, false));
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x118, 0xf, 0xf, false));
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x142, 0xa, 0xf, false));
+        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x143, 0xc, 0xf, false));
+        floor_c = max(floor_c, ((uint32_t)__builtin_amdgcn_readlane((int)longest, 63) + 63u) / 64u);
+    }
+    // (the quotients below need not be exact: `lo` is only where the search starts and `hi` is rounded up by two)
+    uint32_t lo = max(floor_c, (uint32_t)((float)total * __builtin_amdgcn_rcpf((float)slots)));
+    uint32_t hi = max(lo, (uint32_t)((float)total * __builtin_amdgcn_rcpf((float)(slots - a.bal_batch))) + 2u);
+    // Four sizes between the two at a time: their counts are independent, and two sums share a register (a count is at most
+    // slots + sequences + a few, below 2^16).
+    while (hi - lo > lo / 16u) {  // (the same in every wave of the launch; hi always fits)
+        const uint32_t step = (hi - lo + 3u) / 4u, c1 = lo + step, c2 = min(lo + 2u * step, hi), c3 = min(lo + 3u * step, hi);
+        const uint32_t q0 = ceil_quot(blocks, lo, __builtin_amdgcn_rcpf((float)lo)), q1 = ceil_quot(blocks, c1, __builtin_amdgcn_rcpf((float)c1));
+        const uint32_t q2 = ceil_quot(blocks, c2, __builtin_amdgcn_rcpf((float)c2)), q3 = ceil_quot(blocks, c3, __builtin_amdgcn_rcpf((float)c3));
+        const uint32_t s01 = wave_sum(q0 | q1 << 16), s23 = wave_sum(q2 | q3 << 16);
+        if ((s01 & 0xffffu) <= slots) hi = lo;
+        else if ((s01 >> 16) <= slots) hi = c1, lo = lo + 1u;
+        else if ((s23 & 0xffffu) <= slots) hi = c2, lo = c1 + 1u;
+        else if ((s23 >> 16) <= slots) hi = c3, lo = c2 + 1u;
+        else lo = c3 + 1u;
+        lo = min(lo, hi);
+    }
+    const uint32_t parts = ceil_quot(blocks, hi, __builtin_amdgcn_rcpf((float)hi));
+    const uint32_t end = wave_scan(parts);
+    const unsigned long long at = __ballot(end > slot);
+    BatchPlace r;
+    r.dropped = __any(raw > min(a.capacity, a.kv_len_bound));
+    r.b = at ? (uint32_t)__builtin_ctzll(at) : 0u;
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)parts, (int)r.b);
+    r.first = (uint32_t)__builtin_amdgcn_readlane((int)end, (int)r.b) - n;
+    r.len = (uint32_t)__builtin_amdgcn_readlane((int)raw, (int)r.b);
+    r.nsplits = at ? n : 0u;
+    r.split = at ? slot - r.first : 1u;  // (a workgroup without a place leaves where one of an empty partition does)
+    return r;
 }
 
 // RoPE of 8 elements (src/metals/kv_prep/kv_prep_fused.metal:66-82): products and sum are rounded separately
@@ -596,7 +675,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         asm volatile("" ::"s"(a.k), "s"(a.v), "s"(a.block_table), "s"(a.bt_stride), "s"(a.block_size), "s"(a.block_shift),
                      "s"(a.n_kv_heads), "s"(a.capacity), "s"(a.chunk), "s"(a.sub_per_kv), "s"(a.gt), "s"(a.xcd_local),
                      "s"(a.rcp_gx), "s"(a.rcp_gy), "s"(gridDim.x), "s"(gridDim.y), "s"(a.d_len), "s"(a.d_len_stride),
-                     "s"(a.kv_len_add), "s"(a.kv_len), "s"(a.kv_len_bound));
+                     "s"(a.kv_len_add), "s"(a.kv_len), "s"(a.kv_len_bound), "s"(a.bal_batch), "s"(a.bal_per_xcd));
     }
     if constexpr (EARLY_START) {
         if (tid == 0) sm_q_ready = 0;
@@ -604,7 +683,18 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     }
     uint32_t y = blockIdx.y, b = blockIdx.z;
     uint32_t split;
-    if (a.xcd_local) {
+    BatchPlace place = {};
+    if (PAGED && a.bal_batch) {
+        // Slots in an order in which an XCD (workgroup id modulo 8) has consecutive ones: most sequences then have all their
+        // partitions on one XCD and exchange them through its L2 (xcd_local below).
+        uint32_t slot = blockIdx.x;
+        if (a.bal_per_xcd) {
+            const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, pos = (lin & 7u) * a.bal_per_xcd + (lin >> 3);
+            y = __umulhi(pos, a.rcp_gx), slot = pos - y * gridDim.x;
+        }
+        place = batch_place(a, slot, gridDim.x, NW);
+        b = place.b, split = place.split;
+    } else if (a.xcd_local) {
         // All partitions of a head group on ONE XCD (workgroup id modulo 8), so that their partial states meet in that
         // XCD's L2 instead of in memory: group = id % 8 + 8 (id / 8 / S), partition = id / 8 % S. The host selects this
         // only when the number of head groups is a multiple of 8.
@@ -796,6 +886,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     // comes through the scalar cache.
     auto read_len = [&]() -> uint32_t {
         typedef const uint32_t __attribute__((address_space(4))) *const_u32p;
+        if (PAGED && a.bal_batch) return place.len;
         return a.d_len ? ((const_u32p)a.d_len)[(size_t)b * a.d_len_stride] + a.kv_len_add : a.kv_len;
     };
     // Q^T operand: lane (n, c) of step j holds segment 4j + c of head head0 + n (zero for unused columns)
@@ -1060,10 +1151,10 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     }
     if (!(FUSED && wave == 0)) n_raw = read_len();
     const uint32_t N = min(n_raw, min(a.capacity, a.kv_len_bound));
-    const uint32_t nsplits = (N + a.chunk - 1) / a.chunk;
+    const uint32_t nsplits = PAGED && a.bal_batch ? place.nsplits : (N + a.chunk - 1) / a.chunk;
     // A position at or past the launch bound / the capacity: the token is neither appended nor attended. The host
     // finds the bit at its next synchronize.
-    if (FUSED && n_raw > N && tid == 0 && blockIdx.x == 0 && y == 0 && a.status) a.status[FA_DEVSTAT_APPEND_DROPPED] = 1u;
+    if (FUSED && (PAGED && a.bal_batch ? place.dropped : n_raw > N) && tid == 0 && blockIdx.x == 0 && y == 0 && a.status) a.status[FA_DEVSTAT_APPEND_DROPPED] = 1u;
     if (split >= nsplits || pad_wg) {  // uniform over the workgroup
         FA_TR_FLUSH();
         return;
@@ -1360,7 +1451,14 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     FA_TR(8);
 
     const bool in_kernel = tl.merge_in_kernel != 0, polled = tl.merge_in_kernel == 2;
-    const size_t gbase = ((size_t)b * GY + y) * S * gt;  // first row of this (sequence, head group)
+    // the first partition of this (sequence, head group) in the exchange buffers
+    const size_t gpart = PAGED && a.bal_batch ? (size_t)y * S + place.first : ((size_t)b * GY + y) * S;
+    const size_t gbase = gpart * gt;  // and its first row
+    bool xcd_local = tl.xcd_local != 0;
+    if (PAGED && a.bal_batch) {  // all of the sequence's partitions among the slots of this XCD?
+        const uint32_t xcd_first = ((blockIdx.x + gridDim.x * blockIdx.y) & 7u) * a.bal_per_xcd;
+        xcd_local = gpart >= xcd_first && gpart + nsplits <= xcd_first + a.bal_per_xcd;  // (never for bal_per_xcd = 0)
+    }
     const uint32_t prow = split * gt;
     constexpr int CG = D / 4;
     // LPC = NW / 2 consecutive lanes share a column (head h, float4 column c4): lane j merges the states of waves 2j and
@@ -1393,9 +1491,9 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             const u4_t r0 = {__float_as_uint(not_sentinel(A[0])), __float_as_uint(not_sentinel(A[1])),
                              __float_as_uint(not_sentinel(A[2])), __float_as_uint(not_sentinel(A[3]))};
             const u2_t r1 = {__float_as_uint(not_sentinel(ms)), __float_as_uint(not_sentinel(L))};
-            const __amdgpu_buffer_rsrc_t rs = make_rsrc(tl.part_acc + ((size_t)b * GY + y) * S * (gt * CG) * 8);
+            const __amdgpu_buffer_rsrc_t rs = make_rsrc(tl.part_acc + gpart * (gt * CG) * 8);
             const uint32_t ro = (split * (gt * CG) + (uint32_t)idx) * 32u;
-            if (tl.xcd_local) {
+            if (xcd_local) {
                 __builtin_amdgcn_raw_buffer_store_b128(r0, rs, (int)ro, 0, 0);
                 __builtin_amdgcn_raw_buffer_store_b64(r1, rs, (int)ro + 16, 0, 0);
             } else {
@@ -1424,15 +1522,15 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     if (polled) {
         bool ok;
         if (nsplits <= 64) {
-            ok = tl.xcd_local ? coop_merge_in_registers<D, true>(tl, b, y, split, nsplits, S, tid)
-                             : coop_merge_in_registers<D, false>(tl, b, y, split, nsplits, S, tid);
+            ok = xcd_local ? coop_merge_in_registers<D, true>(tl, b, y, split, nsplits, gpart, tid)
+                             : coop_merge_in_registers<D, false>(tl, b, y, split, nsplits, gpart, tid);
             if (!ok && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
             FA_TR(10);
             FA_TR_FLUSH();
             return;
         }
         __syncthreads();  // the fold above read the LDS region that the merge reuses
-        if (tl.xcd_local) {
+        if (xcd_local) {
             ok = coop_merge_and_store<D, true>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));
         } else {
             ok = coop_merge_and_store<D, false>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));

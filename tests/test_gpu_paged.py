@@ -258,6 +258,68 @@ def test_paged_decode_full_batch_of_32_ragged_sequences():
         b.free()
 
 
+@pytest.mark.parametrize("H,Hkv,D,bs,lens,bound", [
+    (16, 2, 128, 16, [0, 4999], 0),                                             # one sequence has all the slots, at most 64 each
+    (16, 2, 128, 16, [1, 15, 16, 17, 31, 0, 2047, 2048, 2049, 6000] * 3, 0),    # block edges, sequences of the new token alone
+    (24, 8, 128, 32, [4000, 127, 128, 129, 2500, 3999, 1000, 64], 4096),        # 32 slots, an XCD's worth per KV head
+    (8, 8, 128, 16, [100 + 97 * i for i in range(32)], 0),                      # two slots per sequence, four waves
+    (6, 3, 128, 48, [3000, 10, 700, 1500], 0),                                  # 85 slots per head group: not dealt by XCD
+    (14, 2, 64, 16, [(i * 977) % 4100 for i in range(64)], 0),                  # 64 sequences, every lane of the wave
+    (16, 1, 128, 16, [5000, 3, 2222], 8192),                                    # 16 heads per workgroup, 256 slots
+    (16, 2, 128, 16, [200, 30, 90, 155, 64, 12], 16384),                        # a bound far above the lengths
+])
+def test_paged_batch_dealt_out_by_lengths(H, Hkv, D, bs, lens, bound):
+    """The launch whose workgroups find their (sequence, partition) from the lengths: against the oracle, and against the
+    partitions cut by the bound with the merge in a second launch. The two add the same f32 partial sums in another grouping
+    and round once to f16: two f16 units of the largest output apart at most."""
+    announce("paged batch dealt out by lengths", H, Hkv, D, bs, len(lens), max(lens), bound)
+    f = ctx()
+    rng = np.random.default_rng(H + 10 * D + len(lens))
+    B = len(lens)
+    ks = [h16(rng.normal(size=(Hkv, n + 1, D))) for n in lens]
+    vs = [h16(rng.normal(size=(Hkv, n + 1, D))) for n in lens]
+    pg = Paged(f, rng, lens, Hkv, D, bs)
+    if bound:  # (the launch's bound is cut to the block table's width)
+        pg.mb = (bound + bs - 1) // bs
+        wide = np.zeros((B, pg.mb), np.int32)
+        wide[:, :pg.bt_dev_host.shape[1]] = pg.bt_dev_host
+        pg.bt_dev_host = wide
+    pg.fill_from(ks, vs)
+    pg.upload()
+    bound = bound or max(lens) + 1
+    q, kn, vn = (h16(rng.normal(size=(B, n * D))) for n in (H, Hkv, Hkv))
+    cos, sin = fa.rope_tables(1e6, D, max(lens) + 1)
+    dq, dkn, dvn, dcos, dsin = f.array(q), f.array(kn), f.array(vn), f.array(cos), f.array(sin)
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, B, 0, 0, fa.ROPE_NEOX)
+    outs, rots, pools = [], [], []
+    for merge in (2, 2, 1):  # (twice: the exchange buffer is ready for the next launch)
+        dout, dqr = f.zeros((B, H * D)), f.zeros((B, H, D))
+        try:
+            f.set_decode_variant(0, merge)
+            f.decode_step_fused_paged(dq.arg(), dkn.arg(), dvn.arg(), dqr.arg(), pg.desc, dcos.arg(), dsin.arg(), dout.arg(), p, bound)
+            f.synchronize()
+        finally:
+            f.set_decode_variant()
+        outs.append(dout.download().reshape(B, H, D)), rots.append(dqr.download())
+        pools.append((pg.dk.download(), pg.dv.download()))
+        dout.free(), dqr.free()
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
+    for i in (0, 1):
+        assert np.array_equal(bits(rots[i]), bits(rots[2]))
+        assert all(np.array_equal(bits(x), bits(y)) for x, y in zip(pools[i], pools[2]))
+    for b, n in enumerate(lens):
+        unit = 2.0 ** (np.floor(np.log2(np.abs(outs[2][b].astype(np.float32)).max())) - 10)
+        assert max_abs(outs[0][b], outs[2][b]) <= 2 * unit, b
+        kc, vc = np.zeros((Hkv, n + 1, D), np.float16), np.zeros((Hkv, n + 1, D), np.float16)
+        kc[:, :n], vc[:, :n] = ks[b][:, :n], vs[b][:, :n]
+        qr = orc.kv_prep_fused(q[b:b + 1], kn[b:b + 1], vn[b:b + 1], kc, vc, cos, sin, orc.make_params(H, Hkv, D, 1, n, n + 1, rope_mode=0))
+        want = orc.sdpa_decode(qr[:, 0].copy(), kc, vc, H, Hkv, D, n + 1, n + 1, n_threads=8).reshape(H, D)
+        assert max_abs(outs[0][b], want) <= TOL, b
+    pg.free()
+    for x in (dq, dkn, dvn, dcos, dsin):
+        x.free()
+
+
 @pytest.mark.usefixtures("prefill_variant")
 @pytest.mark.parametrize("H,Hkv,D,bs,prefix,M", [
     (6, 2, 128, 16, 333, 100),    # context ends inside a block and inside a key tile
