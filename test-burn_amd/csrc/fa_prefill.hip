@@ -1090,6 +1090,16 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
         splits = 1;
         if (base_wgs * 2 <= n_cus) splits = n_cus / base_wgs;  // all workgroups resident at once, one per CU
         if (splits > key_tiles / 4) splits = key_tiles / 4;
+        // What splitting saves the longest item - a pair of key tiles is about 1.5 us - against what it costs: the partial states
+        // stored and the merge launch, 4 us and 0.35 us per MB. A prompt, or a chunk after a short prefix, has too few tiles to
+        // repay it. us, split by the rules above and whole: H16 / Hkv4 / D128, 500 rows: 19.6, 14.5; H16 / Hkv2 / D128, 1000 rows:
+        // 27.8, 20.3; H24 / Hkv8 / D128, 500 rows after 300: 24.4, 18.7; H14 / Hkv2 / D64, 500 rows: 13.2, 11.5, and beyond the
+        // line, 400 rows after 400: 14.4, 15.3, 500 after 1000: 16.0, 21.9.
+        if (!a.pack_heads && splits > 1) {
+            const float pairs_saved = 0.5f * (float)(key_tiles - ceil_div_u32(key_tiles, splits));
+            const float stored_mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * (float)splits * 4e-6f;
+            if (1.5f * pairs_saved < 4.0f + 0.35f * stored_mb) splits = 1;
+        }
         // (packed heads: every split is one more partial per row for the merge, so beyond 16 splits each should have 16
         // tiles. A 32-row chunk after 2K / 8K / 32K tokens measured best with 8 / 16 / 24-32 splits.)
         if (a.pack_heads && splits > 16 && key_tiles / splits < 16) splits = key_tiles / 16 > 16 ? key_tiles / 16 : 16;

@@ -286,6 +286,30 @@ def test_prefill_split_k_independent_of_split_count(split_k):
     assert max_abs(got, want) <= TOL
 
 
+@pytest.mark.parametrize("H,Hkv,D,M,prefix", [
+    (14, 2, 64, 400, 112),   # eight key tiles: whole
+    (14, 2, 64, 400, 400),   # thirteen: three splits
+    (16, 4, 128, 500, 0), (16, 4, 128, 65, 575), (16, 4, 128, 65, 1000),
+    (16, 2, 128, 1000, 0),   # many rows: what the splits would store decides
+])
+def test_prefill_automatic_split_on_both_sides_of_its_line(H, Hkv, D, M, prefix):
+    """Where the library decides whether a chunk's keys are split: the automatic choice, whole items and a forced split against
+    the oracle."""
+    announce("prefill, automatic split", H, Hkv, D, M, prefix)
+    f = ctx()
+    rng = np.random.default_rng(M + prefix)
+    N = M + prefix
+    q, k, v = h16(rng.normal(size=(H, M, D))), h16(rng.normal(size=(Hkv, N, D))), h16(rng.normal(size=(Hkv, N, D)))
+    want = orc.sdpa_prefill(q, k, v, H, Hkv, D, M, N, prefix, N, causal=True, out_layout="head_major", n_threads=8)
+    for split_k in (0, 1, 3):
+        f.set_prefill_split_k(split_k)
+        try:
+            got = gpu_prefill(q, k, v, H, D, M, N, prefix)
+        finally:
+            f.set_prefill_split_k(0)
+        assert max_abs(got, want) <= TOL, split_k
+
+
 def test_prefill_split_k_more_splits_than_tiles_and_d64():
     announce("prefill split-k edge")
     f = ctx()
