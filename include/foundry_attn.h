@@ -275,7 +275,9 @@ size_t fa_noalloc_scratch_bytes(void);
 
 /* Tuning override, the counterpart of FlashDecodeVariant + METALLIC_FA_DECODE_* (src/metals/flashattention/
  * variants.rs:36-140). keys_per_split: context partition per workgroup (rounded up to the kernel's 16-key
- * block; 0 = auto: one partition per compute unit).
+ * block; 0 = auto: one partition per compute unit; under merge = 2 the workgroups of a paged batch of 2 to 64 sequences
+ * find their sequence and partition from the lengths on the device, as one round of resident workgroups, where the length
+ * bound gives a workgroup at least 512 keys of 128 dims).
  * merge: 0 = merged by the last workgroup to finish (one launch, an arrival ticket); 1 = separate merge kernel;
  * 2 (the default of a new context) = polled: every partition's workgroup stores its partial state as records in a
  * buffer whose words hold an arrival pattern between launches, then merges a share of the output columns itself as soon
