@@ -184,8 +184,9 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const u4_t w = wv[t][u];
-            if constexpr (WB == 16) {
-                acc[t] = dot8(__builtin_bit_cast(h8_t, w), xv[u][0], acc[t]);
+            if constexpr (WB == 16) {  // (past the last block the sum is left as it is: a product with the re-read weights is NaN where one is infinite)
+                const float s = dot8(__builtin_bit_cast(h8_t, w), xv[u][0], acc[t]);
+                acc[t] = kb_ok[u] ? s : acc[t];
             } else {
                 float s;
                 if constexpr (WB == 8) {

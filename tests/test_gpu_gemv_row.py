@@ -58,3 +58,45 @@ def test_one_input_row(K, N, NK, weights, layout):
     assert np.all(np.abs(got - w) <= 2 * np.maximum(np.abs(w), 2.0 ** -10) * 2.0 ** -10 + 1e-4), float(np.max(np.abs(got - w)))
     for b in [dx, dg, dres, dout] + db + outs + dev_w + dev_s:
         b.free()
+
+
+def infinite_last_block(K, N, m, weights, layout):
+    """MatMul whose weight row 1 is infinite in its last block (F16: one weight, block-quantised: the block's scale) under an input
+    without negative values: the row's sums are infinite, every other row is the oracle's. What a kernel requests past the last block
+    must not reach the sums."""
+    f = ctx()
+    rng = np.random.default_rng(K + N + m)
+    x = rng.uniform(0.25, 1, (m, K)).astype(np.float16)
+    w = rng.uniform(-0.1, 0.1, (N, K)).astype(np.float16)
+    if weights == "f16":
+        full = w.copy()
+        w[1, K - 3] = np.inf
+        dev_w, dev_s = f.array(orc.to_canonical(w) if layout else w.reshape(-1)), None
+        arg = dev_w.arg()
+    else:
+        q, s = orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w)
+        full = orc.dequantize_blocks(q, s)
+        q[1, K - 32:] = 3
+        s[1, -1] = np.inf
+        flat = orc.to_canonical(q) if layout else q.reshape(-1)
+        dev_w, dev_s = f.array(flat if weights == "q8" else orc.pack_q4_0(flat)), f.array(s)
+        arg = dev_w.arg() if weights == "q8" else dev_w.arg((N, K), dtype=fa.DTYPE_Q4_0)
+    dx, dout = f.array(x), f.zeros((m, N))
+    f.matmul(dx.arg(), arg, dout.arg(), m, N, K, transpose_b=not layout, b_scales=dev_s.arg() if dev_s else None)
+    got = dout.download().astype(np.float64)
+    want = x.astype(np.float64) @ full.astype(np.float64).T
+    rest = np.arange(N) != 1
+    assert np.all(got[:, 1] == np.inf), got[:, 1]
+    # two f16 units of the result and the rounding of the weights that f16(weight * scale) has where it is used
+    bar = 2.0 ** -9 * np.abs(want) + 2.0 ** -11 * (x.astype(np.float64) @ np.abs(full.astype(np.float64)).T) + 1e-4
+    assert np.all(np.abs(got - want)[:, rest] <= bar[:, rest])
+    for b in [dx, dout, dev_w] + ([dev_s] if dev_s else []):
+        b.free()
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K", [160, 1056, 2080, 4064])  # blocks that do not fill the last wave's share, of one, two and four units
+def test_one_input_row_infinite_last_block(K, weights, layout):
+    announce("one input row, infinite last block", K, weights, layout)
+    infinite_last_block(K, 24, 1, weights, layout)
