@@ -64,6 +64,9 @@ struct Weights<4> {  // element 2i in the low nibble of byte i, value = nibble -
     static __device__ __forceinline__ h8_t f16(raw_t w, _Float16 s) { return plain(w) * h8_t{s, s, s, s, s, s, s, s}; }
 };
 
+// What a lane reads in the place of an F16 weight block past the row's last.
+static __device__ const h8_t zero_weights = {0, 0, 0, 0, 0, 0, 0, 0};
+
 template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
 __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -140,7 +143,8 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         for (int j = 0; j < PK; ++j) g_lds[j * 64 + lane] = gv[j];
     }
     // ---- block scales (block-quantised weights): [block][slot] f16 in LDS, fetched along the rows of the scale matrix, two at a
-    // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request)
+    // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request). Behind the last
+    // block comes one of zeros, for the requests past it: an infinite scale read again would make NaN of the input's zeros there.
     _Float16 *const sc_lds = reinterpret_cast<_Float16 *>(smem + lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0));
     constexpr int SLOTS = NT * 16, SC_LOADS = WB == 16 ? 1 : (SLOTS * PK * 8 + NTHREADS - 1) / NTHREADS;  // pairs per thread
     uint32_t sc_raw[SC_LOADS];
@@ -190,7 +194,14 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
         const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
 #pragma unroll
-        for (int i = 0; i < NQ; ++i) wv[t][i] = fa_norm::load_global_once<req_t>(p0 + (size_t)min(kb_of(i) + lane_blk, nkb - 1u) * kb_stride);
+        for (int i = 0; i < NQ; ++i) {
+            const uint32_t kb = kb_of(i) + lane_blk;
+            const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
+            // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
+            // block-quantised weights are finite, and their scale is zero there.)
+            if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
+            wv[t][i] = fa_norm::load_global_once<req_t>(p);
+        }
     }
     const float eps = a.eps, inv_k = a.inv_k, alpha = a.alpha, beta = a.beta;
     const __half *const residual = a.residual;
@@ -258,7 +269,8 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                     uint32_t slot, kb2;
                     if (!scale_at(i, slot, kb2)) continue;
                     unsigned short *dst = reinterpret_cast<unsigned short *>(sc_lds) + 2 * kb2 * SLOTS + slot;
-                    dst[0] = (unsigned short)sc_raw[i], dst[SLOTS] = (unsigned short)(sc_raw[i] >> 16);
+                    dst[0] = (unsigned short)sc_raw[i], dst[SLOTS] = 2 * kb2 + 1 < nkb ? (unsigned short)(sc_raw[i] >> 16) : (unsigned short)0;
+                    if (2 * kb2 + 2 == nkb && nkb < PK * 16u) dst[2 * SLOTS] = 0;
                 }
             }
         }
@@ -286,7 +298,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         for (int i = 0; i < NQ; ++i) {
             const uint32_t kb = kb_of(i) + lane_blk;
             const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
-            const _Float16 *const scp = sc_lds + min(kb, nkb - 1u) * SLOTS + (SUMS ? c * 4 : n);  // (past the last block: a finite scale for zeros)
+            const _Float16 *const scp = sc_lds + min(kb, nkb) * SLOTS + (SUMS ? c * 4 : n);  // (past the last block: scales of zero)
             req_t raw[NT];
             _Float16 sc[NT];
 #pragma unroll

@@ -8,6 +8,7 @@ import pytest
 import foundry_attn as fa
 import orc
 from gpu_util import announce, ctx
+from test_gpu_gemv_row import infinite_last_block
 from test_gpu_qkv import _close, _data
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +73,12 @@ def test_chunk_in_one_launch(K, N, NK, m, layout, weights):
     assert np.all(np.abs(got - w) <= 2 * np.maximum(np.abs(w), 2.0 ** -10) * 2.0 ** -10 + 1e-4), float(np.max(np.abs(got - w)))
     for b in [dx, dg, dres, dout] + db + outs + dev_w + dev_s:
         b.free()
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,m", [(32, 2), (96, 11), (96, 12), (896, 33), (1056, 5), (2016, 20), (2080, 5), (2080, 17)])
+def test_chunk_in_one_launch_infinite_last_block(K, m, weights, layout):
+    """Row lengths of every number of feature pieces whose blocks do not fill a wave's share, odd and even in number."""
+    announce("panel, infinite last block", K, m, weights, layout)
+    infinite_last_block(K, 40, m, weights, layout)
