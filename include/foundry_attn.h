@@ -276,15 +276,16 @@ size_t fa_noalloc_scratch_bytes(void);
 /* Tuning override, the counterpart of FlashDecodeVariant + METALLIC_FA_DECODE_* (src/metals/flashattention/
  * variants.rs:36-140). keys_per_split: context partition per workgroup (rounded up to the kernel's 16-key
  * block; 0 = auto: one partition per compute unit; under merge = 2 the workgroups of a paged batch of 2 to 64 sequences
- * find their sequence and partition from the lengths on the device, as one round of resident workgroups, where the length
- * bound gives a workgroup at least 512 keys of 128 dims).
+ * find their sequence and partition from the lengths on the device, no more workgroups than are resident at once, where the
+ * length bound gives a workgroup at least 512 keys of 128 dims).
  * merge: 0 = merged by the last workgroup to finish (one launch, an arrival ticket); 1 = separate merge kernel;
  * 2 (the default of a new context) = polled: every partition's workgroup stores its partial state as records in a
  * buffer whose words hold an arrival pattern between launches, then merges a share of the output columns itself as soon
  * as the other partitions' records have arrived (one launch, no ticket, the reads spread over all compute units;
  * a head group's workgroups are placed on one XCD where the launch allows, so the records meet in that XCD's L2). It
- * applies to launches whose workgroups are all resident at once (at most one 8-wave or two 4-wave workgroups per compute
- * unit; others take 1).
+ * applies to launches whose workgroups, with partitions cut by the length bound, are all resident at once (at most one 8-wave
+ * or two 4-wave workgroups per compute unit); others take 1, or 0 where the partitions are found from the lengths: no
+ * workgroup of those waits for another.
  * Form 2 ASSUMES THAT THE CONTEXT HAS THE GPU'S COMPUTE UNITS TO ITSELF while a decode launch runs: residency is counted
  * per launch against all compute units of the device. Work of another stream, context or process (or a compute-unit
  * mask) can hold part of them, and two polled launches can then each wait for workgroups the other keeps from

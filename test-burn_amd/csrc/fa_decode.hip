@@ -98,24 +98,6 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     };
     uint32_t waves = ctx->decode_waves;  // 0 = by the rule above
     bool short_context = false;
-    // A paged batch whose partitions the kernel deals out by the lengths (batch_place): one round of resident workgroups, merged
-    // inside the launch, from where the rule above would give a workgroup 512 keys of 128 dims or more - below that a workgroup has
-    // one round of requests whatever its keys, and looking for its place costs 0.4 to 2 us that nothing repays (Hkv 2, D 128, 8
-    // sequences of 500 to 4000 tokens, 256 keys: 10.3 -> 12.4 us). Eight waves while there are two slots per sequence, four
-    // (twice the slots) beyond; with fewer than two the quotients leave too much idle. us per step, by the bound and by the lengths:
-    //   Hkv 2, D 128: 24 sequences of 100-4000 tokens 20.8 -> 17.8, 32 of 512-16384 60.5 -> 52.0, 64 of 16-2000 23.4 -> 19.7
-    //   Hkv 8, D 128: 4 of 100-4000 13.0 -> 10.5, 8 of 100-8000 40.7 -> 30.1, 24 of 100-4000 50.9 -> 40.4 (eight waves: 48.0)
-    //   Hkv 2, D 64:  64 of 16-4000 26.1 -> 18.8;  Hkv 4, D 128: 50 of 500-3000 52.6 -> 39.3
-    //   equal lengths have nothing to gain: Hkv 8, D 128: 8 of 2000 16.4 -> 16.8
-    uint32_t bal_slots = 0;
-    if (L.paged && L.d_len && L.batch >= 2 && L.batch <= 64 && chunk == 0 && ctx->decode_variant.merge == 2 && !L.static_scratch &&
-        bound <= (1u << 24) && auto_chunk(8, n_cus) * L.head_dim >= 512u * 128u) {
-        const uint32_t per8 = (uint32_t)(n_cus / ny);
-        const uint32_t w = waves ? waves : 2u * L.batch <= per8 ? 8u : 4u;
-        const uint32_t n = w == 4u ? 2u * per8 : per8;
-        const size_t records = (size_t)n * ny * (size_t)gt * L.head_dim / 4 * 32;
-        if (n >= 2u * L.batch && records <= ctx->poll_ws_bytes) bal_slots = n, waves = w;
-    }
     if (waves == 0) {
         const uint32_t c8 = chunk ? chunk : auto_chunk(8, n_cus);
         waves = groups * ceil_div_u32(bound, (c8 + BK - 1) / BK * BK) > n_cus ? 4u : 8u;
@@ -132,7 +114,36 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     chunk = (chunk + BK - 1) / BK * BK;
     // the int8 step in one launch: the open 32-row block must lie inside one partition
     if (L.sage_fused) chunk = (chunk + FA_SAGE_BLOCK - 1) / FA_SAGE_BLOCK * FA_SAGE_BLOCK;
-    const uint32_t S = bal_slots ? bal_slots : ceil_div_u32(bound, chunk);
+    uint32_t S = ceil_div_u32(bound, chunk);
+    // The polled merge needs every workgroup of the launch resident at once (the merging workgroup of a head group
+    // occupies its compute unit while it waits) and its partials in the context's pattern-filled buffer.
+    const uint32_t n4 = (uint32_t)gt * L.head_dim / 4;  // records (float4 columns of all heads) per partition
+    const uint64_t slots = waves == 4 ? 2 * n_cus : n_cus;
+    // a workgroup reads ceil(n4 / partitions) columns of every partition (fewer than n4 + partitions records for
+    // any partition count up to S), at most POLL_IPT records per thread
+    const bool polled = ctx->decode_variant.merge == 2 && !L.static_scratch && S > 1 && groups * S <= slots &&
+                        (size_t)groups * S * n4 * 32 <= ctx->poll_ws_bytes && (uint64_t)n4 + S <= (uint64_t)waves * 64 * POLL_IPT;
+    // A paged batch whose partitions the kernel deals out by the lengths (batch_place): one round of resident workgroups, merged
+    // inside the launch, from where the rule above would give a workgroup 512 keys of 128 dims or more - below that a workgroup has
+    // one round of requests whatever its keys, and looking for its place costs 0.4 to 2 us that nothing repays (Hkv 2, D 128, 8
+    // sequences of 500 to 4000 tokens, 256 keys: 10.3 -> 12.4 us). Eight waves while there are two slots per sequence, four
+    // (twice the slots) beyond; with fewer than two the quotients leave too much idle. us per step, by the bound and by the lengths:
+    //   Hkv 2, D 128: 24 sequences of 100-4000 tokens 20.8 -> 17.8, 32 of 512-16384 60.5 -> 52.0, 64 of 16-2000 23.4 -> 19.7
+    //   Hkv 8, D 128: 4 of 100-4000 13.0 -> 10.5, 8 of 100-8000 40.7 -> 30.1, 24 of 100-4000 50.9 -> 40.4 (eight waves: 48.0)
+    //   Hkv 2, D 64:  64 of 16-4000 26.1 -> 18.8;  Hkv 4, D 128: 50 of 500-3000 52.6 -> 39.3
+    //   equal lengths have nothing to gain: Hkv 8, D 128: 8 of 2000 16.4 -> 16.8
+    // Its workgroups wait for each other (the polled merge) only where those of the rule above would. Where that rule has more
+    // workgroups than fit at once, and so a merge that waits for nobody, the last one of a sequence to finish merges it: 1.2 to 1.6
+    // us more than polled (32 of 512-16384: 52.2 against 53.4; 8 of 100-8000, Hkv 8: 29.9 against 31.3), and right on a GPU that
+    // other work has part of, as those batches were before.
+    uint32_t bal_slots = 0;
+    if (L.paged && L.d_len && L.batch >= 2 && L.batch <= 64 && ctx->decode_variant.keys_per_split == 0 && ctx->decode_variant.merge == 2 &&
+        !L.static_scratch && bound <= (1u << 24) && auto_chunk(8, n_cus) * L.head_dim >= 512u * 128u) {
+        const uint32_t per8 = (uint32_t)(n_cus / ny);
+        const uint32_t w = ctx->decode_waves ? ctx->decode_waves : 2u * L.batch <= per8 ? 8u : 4u;
+        const uint32_t n = w == 4u ? 2u * per8 : per8;
+        if (n >= 2u * L.batch && (size_t)n * ny * n4 * 32 <= ctx->poll_ws_bytes) bal_slots = S = n, waves = w;
+    }
     // a contiguous cache slab is addressed with 32-bit byte offsets (tile base included)
     if (!L.paged && ((uint64_t)L.capacity + chunk + MBX * BK) * L.head_dim * 2 >= (1ull << 32))
         return fa_fail(FA_ERR_INVALID_SHAPE, "flash decode: one KV head of the contiguous cache must stay below 4 GiB");
@@ -158,36 +169,28 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     a.rope_normal = L.rope_normal, a.apply_rope = L.apply_rope, a.table_rows = L.table_rows;
     a.status = ctx->d_status;
     a.sage_tail = L.sage_tail, a.sage_mean = L.sage_mean, a.q_q_out = L.q_q_out, a.q_scale_out = L.q_scale_out;
-    // The polled merge needs every workgroup of the launch resident at once (the merging workgroup of a head group
-    // occupies its compute unit while it waits) and its partials in the context's pattern-filled buffer.
-    bool polled = false;
     uint32_t ny_grid = ny;  // the grid's y dimension (see the padded form below)
-    if (ctx->decode_variant.merge == 2 && !L.static_scratch) {
-        const uint32_t n4 = (uint32_t)gt * L.head_dim / 4;  // records (float4 columns of all heads) per partition
-        const size_t need = (size_t)L.batch * ny * S * n4 * 32;
-        const uint64_t slots = waves == 4 ? 2 * n_cus : n_cus;
-        const uint32_t nt = waves * 64;
-        // a workgroup reads ceil(n4 / partitions) columns of every partition (fewer than n4 + partitions records for
-        // any partition count up to S), at most POLL_IPT records per thread
-        polled = bal_slots || (S > 1 && groups * S <= slots && need <= ctx->poll_ws_bytes && (uint64_t)n4 + S <= (uint64_t)nt * POLL_IPT);
-        a.bal_batch = bal_slots ? L.batch : 0u;
-        if (bal_slots && ctx->xcd_round_robin && bal_slots * ny % 8 == 0 && bal_slots >= 2) {
-            a.bal_per_xcd = bal_slots * ny / 8;
-            a.rcp_gx = (uint32_t)((1ull << 32) / bal_slots) + 1u;  // (exact for the few hundred workgroups of such a launch)
-        }
-        a.merge_in_kernel = polled ? 2u : 0u;
-        a.xcd_local = polled && !bal_slots && ctx->xcd_round_robin && groups % 8 == 0 ? 1u : 0u;
+    a.bal_batch = bal_slots ? L.batch : 0u;
+    if (bal_slots && ctx->xcd_round_robin && bal_slots * ny % 8 == 0) {
+        a.bal_per_xcd = bal_slots * ny / 8;
+        a.rcp_gx = (uint32_t)((1ull << 32) / bal_slots) + 1u;  // (exact for the few hundred workgroups of such a launch)
+    }
+    if (polled) {
+        a.merge_in_kernel = 2u;
+        a.xcd_local = !bal_slots && ctx->xcd_round_robin && groups % 8 == 0 ? 1u : 0u;
         // Fewer than 8 head groups (Qwen2.5-0.5B has 2 KV heads) and few enough partitions for an XCD to hold a group's
         // workgroups: the grid is padded to 8 head groups, group g's workgroups land on XCD g, and the workgroups of
         // the groups that do not exist leave at once. Such a launch is all latency (its partitions were sized for that
         // above), and the exchange through one XCD's L2 is most of a microsecond shorter than through device-coherent
         // accesses (6.15 -> 5.4 us per launch at 1K context).
-        if (polled && !a.xcd_local && ctx->xcd_round_robin && L.batch == 1 && groups < 8 && waves == 4) {  // (only the 4-wave kernels know of the padding)
-            const uint64_t per_xcd = (uint64_t)(waves == 4 ? 2u : 1u) * (n_cus / 8u);
+        if (!a.xcd_local && ctx->xcd_round_robin && L.batch == 1 && groups < 8 && waves == 4) {  // (only the 4-wave kernels know of the padding)
+            const uint64_t per_xcd = (uint64_t)2u * (n_cus / 8u);
             const size_t need_pad = (size_t)8 * S * n4 * 32;
             if (S <= per_xcd && (uint64_t)8 * S <= slots && need_pad <= ctx->poll_ws_bytes) ny_grid = 8, a.xcd_local = 1u, a.ny_real = ny;
         }
         a.poll_ticks = (unsigned long long)ctx->poll_spin_us * 100ull;
+    } else if (bal_slots) {
+        a.merge_in_kernel = 1u;
     }
     if (L.static_scratch) {
         // Nothing may be allocated on this path: no workspace growth, no event creation. The partitions' partial
@@ -197,7 +200,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         a.merge_in_kernel = 0;
     }
     if (S > 1) {
-        const size_t rows = (size_t)L.batch * ny * S * gt;
+        const size_t rows = (size_t)(bal_slots ? 1u : L.batch) * ny * S * gt;
         const size_t acc_bytes = rows * L.head_dim * sizeof(float);
         const size_t ml_bytes = rows * 2 * sizeof(float);
         if (L.static_scratch) {

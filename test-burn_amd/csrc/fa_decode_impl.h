@@ -186,8 +186,8 @@ __device__ __forceinline__ f2_t ld_f2(const float *base, __amdgpu_buffer_rsrc_t 
 // The workgroup has NTM threads and merges the heads [h_first, h_first + h_count) of the group.
 template <int D, bool COHERENT, int NTM>
 __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t nsplits,
-                                                uint32_t S, int tid, float *sm /* NTM * 6 floats, 16-byte aligned */,
-                                                int h_first, int h_count) {
+                                                size_t base /* first (partition, head) row of the group */, int tid,
+                                                float *sm /* NTM * 6 floats, 16-byte aligned */, int h_first, int h_count) {
     constexpr int CG = D / 4;     // float4 columns per head
     constexpr int RL = NTM / CG;  // row lanes
     constexpr int PPT_MAX = 17;  // partitions per thread in the largest batch (102 VGPRs in flight)
@@ -196,7 +196,6 @@ __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, 
     const int lph = RL / hpp;           // lanes per head
     const int c = tid % CG, r = tid / CG;
     const int hl = r / lph, q = r % lph;
-    const size_t base = ((size_t)b * gridDim.y + y) * S * gt;  // first (partition, head) row of this group
     const float *acc_base = a.part_acc + base * D;
     const float *ml_base = a.part_ml + base * 2;
     const __amdgpu_buffer_rsrc_t rs_acc = make_rsrc(acc_base), rs_ml = make_rsrc(ml_base);
@@ -1553,7 +1552,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     }
     __syncthreads();
     if (!sm_last) return;
-    merge_and_store<D, true, NT>(tl, b, y, nsplits, S, tid, reinterpret_cast<float *>(smem), 0, (int)gt);
+    merge_and_store<D, true, NT>(tl, b, y, nsplits, gbase, tid, reinterpret_cast<float *>(smem), 0, (int)gt);
     if (tid == 0)  // ready for the next launch
         __hip_atomic_store(&tl.counters[(size_t)b * GY + y], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1571,7 +1570,7 @@ __global__ void __launch_bounds__(NT_MERGE) flash_decode_merge_kernel(DecodeDev 
     N = min(N, min(a.capacity, a.kv_len_bound));
     const uint32_t nsplits = (N + a.chunk - 1) / a.chunk;
     if (nsplits <= 1) return;  // written directly by the partition kernel
-    merge_and_store<D, false, NT_MERGE>(a, b, y, nsplits, S, threadIdx.x, sm, (int)blockIdx.x, 1);
+    merge_and_store<D, false, NT_MERGE>(a, b, y, nsplits, ((size_t)b * gridDim.y + y) * S * a.gt, threadIdx.x, sm, (int)blockIdx.x, 1);
 }
 
 enum Mode { MODE_PLAIN = 0, MODE_PAGED = 1, MODE_SAGE = 2, MODE_FUSED = 3, MODE_FUSED_PAGED = 4, MODE_SAGE_FUSED = 5 };

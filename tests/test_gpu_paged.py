@@ -320,6 +320,49 @@ def test_paged_batch_dealt_out_by_lengths(H, Hkv, D, bs, lens, bound):
         x.free()
 
 
+def widen(pg, bound):
+    """A block table of `bound` tokens per sequence (a launch's bound is cut to the table's width)."""
+    wide = np.zeros((pg.n_seqs, (bound + pg.bs - 1) // pg.bs), np.int32)
+    wide[:, :pg.mb] = pg.bt_dev_host
+    pg.bt_dev_host, pg.mb = wide, wide.shape[1]
+
+
+@pytest.mark.parametrize("H,Hkv,D,B", [
+    (16, 2, 128, 32),   # eight-wave workgroups
+    (16, 2, 128, 60),   # four-wave workgroups
+    (24, 8, 64, 12),
+])
+def test_paged_batch_that_does_not_fit_at_once_waits_for_nobody(H, Hkv, D, B):
+    """A batch with more partitions by its bound than fit the GPU at once is merged without any workgroup waiting for another, also
+    where its partitions are dealt out by the lengths: it is right on a GPU that it shares, here with a wait bound of zero (a launch
+    whose workgroups wait would give up)."""
+    announce("paged batch, zero wait bound", H, Hkv, D, B)
+    rng = np.random.default_rng(B)
+    lens = [int(x) for x in rng.integers(1, 700, size=B)]
+    lens[1], bs, bound = 3000, 16, 16384
+    ks = [h16(rng.normal(size=(Hkv, n, D))) for n in lens]
+    vs = [h16(rng.normal(size=(Hkv, n, D))) for n in lens]
+    q = h16(rng.normal(size=(B, H, D)))
+    g = fa.Foundry(0)
+    try:
+        pg = Paged(g, rng, lens, Hkv, D, bs, extra_tokens=0)
+        widen(pg, bound)
+        pg.fill_from(ks, vs)
+        pg.upload()
+        dq, dout = g.array(q), g.zeros((B, H * D))
+        g.set_decode_poll_spin_us(0)
+        for _ in range(4):
+            dout.upload(np.zeros((B, H * D), np.float16))
+            g.flash_decode_paged(dq.arg(), pg.desc, dout.arg(), H, 0, bound)
+            g.synchronize()
+            got = dout.download().reshape(B, H, D)
+            for b, n in enumerate(lens):
+                want = orc.sdpa_decode(q[b], ks[b], vs[b], H, Hkv, D, n, n, n_threads=8).reshape(H, D)
+                assert max_abs(got[b], want) <= TOL, b
+    finally:
+        g.close()
+
+
 @pytest.mark.usefixtures("prefill_variant")
 @pytest.mark.parametrize("H,Hkv,D,bs,prefix,M", [
     (6, 2, 128, 16, 333, 100),    # context ends inside a block and inside a key tile
