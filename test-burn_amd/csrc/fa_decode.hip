@@ -125,13 +125,14 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
                         (size_t)groups * S * n4 * 32 <= ctx->poll_ws_bytes && (uint64_t)n4 + S <= (uint64_t)waves * 64 * POLL_IPT;
     // A paged batch whose partitions the kernel deals out by the lengths (batch_place): one round of resident workgroups, merged
     // inside the launch, from where the rule above would give a workgroup 512 keys of 128 dims or more - below that a workgroup has
-    // one round of requests whatever its keys, and looking for its place costs 0.4 to 2 us that nothing repays (Hkv 2, D 128, 8
-    // sequences of 500 to 4000 tokens, 256 keys: 10.3 -> 12.4 us). Eight waves while there are two slots per sequence, four
-    // (twice the slots) beyond; with fewer than two the quotients leave too much idle. us per step, by the bound and by the lengths:
-    //   Hkv 2, D 128: 24 sequences of 100-4000 tokens 20.8 -> 17.8, 32 of 512-16384 60.5 -> 52.0, 64 of 16-2000 23.4 -> 19.7
-    //   Hkv 8, D 128: 4 of 100-4000 13.0 -> 10.5, 8 of 100-8000 40.7 -> 30.1, 24 of 100-4000 50.9 -> 40.4 (eight waves: 48.0)
-    //   Hkv 2, D 64:  64 of 16-4000 26.1 -> 18.8;  Hkv 4, D 128: 50 of 500-3000 52.6 -> 39.3
-    //   equal lengths have nothing to gain: Hkv 8, D 128: 8 of 2000 16.4 -> 16.8
+    // one round of requests whatever its keys, and looking for its place is not repaid (Hkv 2, D 128, 8 sequences of 500 to 4000
+    // tokens, 256 keys: 10.3 -> 12.4 us). Eight waves while there are two slots per sequence, four (twice the slots) beyond; with
+    // fewer than two the quotients leave too much idle. us per step, by the bound and by the lengths:
+    //   Hkv 2, D 128: 24 sequences of 100-4000 tokens 20.6 -> 17.8, 32 of 512-16384 59.9 -> 53.3, 64 of 16-2000 23.3 -> 19.7
+    //   Hkv 8, D 128: 8 of 100-2080 13.9 -> 12.1, 8 of 100-8000 40.4 -> 31.4, 24 of 100-4000 50.5 -> 41.0 (eight waves: 48.0)
+    //   Hkv 2, D 64:  40 of 16-8000 29.3 -> 21.9;  Hkv 4, D 128: 50 of 500-3000 51.8 -> 39.3
+    // About equal lengths have nothing to gain and lose what reading them all takes: Hkv 2, D 128: 8 of 11000-12000 21.6 -> 21.8, 24
+    // of 3900-4000 22.0 -> 22.8; Hkv 8, D 128: 8 of 2000 15.5 -> 15.8, 8 of 4000 25.6 -> 25.9; Hkv 4, D 128: 8 of 3000-4000 15.0 -> 15.6.
     // Its workgroups wait for each other (the polled merge) only where those of the rule above would. Where that rule has more
     // workgroups than fit at once, and so a merge that waits for nobody, the last one of a sequence to finish merges it: 1.2 to 1.6
     // us more than polled (32 of 512-16384: 52.2 against 53.4; 8 of 100-8000, Hkv 8: 29.9 against 31.3), and right on a GPU that
@@ -170,10 +171,18 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     a.status = ctx->d_status;
     a.sage_tail = L.sage_tail, a.sage_mean = L.sage_mean, a.q_q_out = L.q_q_out, a.q_scale_out = L.q_scale_out;
     uint32_t ny_grid = ny;  // the grid's y dimension (see the padded form below)
-    a.bal_batch = bal_slots ? L.batch : 0u;
-    if (bal_slots && ctx->xcd_round_robin && bal_slots * ny % 8 == 0) {
-        a.bal_per_xcd = bal_slots * ny / 8;
-        a.rcp_gx = (uint32_t)((1ull << 32) / bal_slots) + 1u;  // (exact for the few hundred workgroups of such a launch)
+    if (bal_slots) {
+        auto rcp = [](uint32_t d) { return (uint32_t)((1ull << 32) / d) + 1u; };  // (exact for the few hundred workgroups of such a launch)
+        const uint32_t per_xcd = ctx->xcd_round_robin && bal_slots * ny % 8 == 0 ? bal_slots * ny / 8 : 0u;
+        // Dealt evenly: within the slots that a KV head has on one XCD, where every XCD gets a sequence.
+        uint32_t cell = bal_slots, per_cell = L.batch;
+        if (per_xcd && bal_slots % per_xcd == 0) {
+            const uint32_t cells = bal_slots / per_xcd, seqs = ceil_div_u32(L.batch, cells);
+            if (cells <= L.batch && per_xcd >= 2 * seqs) cell = per_xcd, per_cell = seqs;
+        }
+        const uint32_t even = cell / per_cell < 64u ? cell / per_cell : 64u;
+        a.bal_seqs = L.batch | even << 8 | per_cell << 16, a.bal_slots = cell | per_xcd << 16;
+        a.rcp_gx = rcp(bal_slots), a.rcp_even = rcp(even), a.rcp_cell = rcp(cell);
     }
     if (polled) {
         a.merge_in_kernel = 2u;
@@ -234,7 +243,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         mode = L.paged ? MODE_FUSED_PAGED : MODE_FUSED;
     else if (L.paged)
         mode = MODE_PAGED;
-    {   // (divisions that every wave would otherwise do before its first request)
+    if (!bal_slots) {  // (divisions that every wave would otherwise do before its first request)
         const uint32_t streaming = (mode == MODE_FUSED || mode == MODE_FUSED_PAGED || mode == MODE_SAGE_FUSED) ? waves - 1 : waves;
         a.nb_q = (chunk / BK) / streaming, a.nb_r = (chunk / BK) % streaming;
     }

@@ -186,7 +186,7 @@ __device__ __forceinline__ f2_t ld_f2(const float *base, __amdgpu_buffer_rsrc_t 
 // The workgroup has NTM threads and merges the heads [h_first, h_first + h_count) of the group.
 template <int D, bool COHERENT, int NTM>
 __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t nsplits,
-                                                size_t base /* first (partition, head) row of the group */, int tid,
+                                                size_t first /* the group's first partition */, int tid,
                                                 float *sm /* NTM * 6 floats, 16-byte aligned */, int h_first, int h_count) {
     constexpr int CG = D / 4;     // float4 columns per head
     constexpr int RL = NTM / CG;  // row lanes
@@ -196,6 +196,7 @@ __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, 
     const int lph = RL / hpp;           // lanes per head
     const int c = tid % CG, r = tid / CG;
     const int hl = r / lph, q = r % lph;
+    const size_t base = first * gt;  // first (partition, head) row of this group
     const float *acc_base = a.part_acc + base * D;
     const float *ml_base = a.part_ml + base * 2;
     const __amdgpu_buffer_rsrc_t rs_acc = make_rsrc(acc_base), rs_ml = make_rsrc(ml_base);
@@ -507,35 +508,40 @@ __device__ __forceinline__ uint32_t ceil_quot(uint32_t n, uint32_t c, float rcp)
 
 // A batch's partitions, dealt to the workgroups by the lengths the sequences have now (which only the device knows). The host
 // sizes a launch by its length bound, the longest sequence: cut that way a batch of 24 sequences of 100 to 4000 tokens has
-// 240 workgroups of which half find nothing, while the others have 800 keys each. Here every wave reads all lengths (one
+// 240 workgroups of which half find nothing, while the others have 800 keys each. Here every wave has all lengths (one
 // load, lane = sequence), looks for the smallest partition with which all sequences together need at most `slots`
 // workgroups - between (all keys) / slots and (all keys) / (slots - sequences), to 1/16 - and finds its own place in the
 // running sum of the sequences' partition counts.
+// Where the lengths are about equal, the same number of slots for every sequence gives a streaming wave no more blocks than that.
+// Then each has those, as many sequences as fit into the slots that a KV head has on one XCD (a cell), and all exchange their records
+// through that XCD's L2. One after the other, sequences of 15 and 16 partitions lie across two XCDs and exchange them through
+// memory. Hkv 2, D 128, cut by the bound / one after the other / as it is: 8 of 11000-12000 tokens 21.6 / 25.8 / 21.8 us, 24 of
+// 3900-4000 22.0 / 25.0 / 22.8; Hkv 8, D 128: 8 of 2000 15.6 / 16.1 / 15.8.
 struct BatchPlace {
     uint32_t b, split, nsplits, first, len;  // first: the slot of the sequence's first partition; nsplits 0: nothing to do
     bool dropped;                            // some sequence is longer than the launch may attend
 };
-__device__ __forceinline__ BatchPlace batch_place(const DecodeDev &a, uint32_t slot, uint32_t slots, uint32_t min_blocks) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t raw = lane < a.bal_batch ? a.d_len[(size_t)lane * a.d_len_stride] + a.kv_len_add : 0u;
-    const uint32_t blocks = (min(raw, min(a.capacity, a.kv_len_bound)) + BK - 1) / BK;
+// `raw`: the length of sequence `lane` (of the last one past the end); kw: waves that stream keys
+__device__ __forceinline__ BatchPlace batch_place(const DecodeDev &a, uint32_t raw, uint32_t slot, uint32_t slots, uint32_t min_blocks, uint32_t kw) {
+    const uint32_t batch = a.bal_seqs & 255u, n_even = a.bal_seqs >> 8 & 255u, per_cell = a.bal_seqs >> 16, n_cell = a.bal_slots & 0xffffu;
+    raw = (threadIdx.x & 63u) < batch ? raw + a.kv_len_add : 0u;
+    const uint32_t most = min(a.capacity, a.kv_len_bound), blocks = (min(raw, most) + BK - 1) / BK;
     const uint32_t total = wave_sum(blocks);
+    uint32_t longest = blocks;
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x111, 0xf, 0xf, false));
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x112, 0xf, 0xf, false));
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x114, 0xf, 0xf, false));
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x118, 0xf, 0xf, false));
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x142, 0xa, 0xf, false));
+    longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x143, 0xc, 0xf, false));
+    longest = (uint32_t)__builtin_amdgcn_readlane((int)longest, 63);
+    const uint32_t even = ceil_quot(longest, n_even, __builtin_amdgcn_rcpf((float)n_even)), even_per_wave = (even + kw - 1) / kw;
     // at least min_blocks, and at most 64 partitions per sequence (what the merge in registers takes)
-    const uint32_t bound_blocks = (min(a.capacity, a.kv_len_bound) + BK - 1) / BK;
-    uint32_t floor_c = min_blocks;
-    if (bound_blocks > 64u * min_blocks) {
-        uint32_t longest = blocks;
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x111, 0xf, 0xf, false));
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x112, 0xf, 0xf, false));
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x114, 0xf, 0xf, false));
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x118, 0xf, 0xf, false));
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x142, 0xa, 0xf, false));
-        longest = max(longest, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)longest, 0x143, 0xc, 0xf, false));
-        floor_c = max(floor_c, ((uint32_t)__builtin_amdgcn_readlane((int)longest, 63) + 63u) / 64u);
-    }
+    const uint32_t floor_c = max(min_blocks, (longest + 63u) / 64u);
     // (the quotients below need not be exact: `lo` is only where the search starts and `hi` is rounded up by two)
     uint32_t lo = max(floor_c, (uint32_t)((float)total * __builtin_amdgcn_rcpf((float)slots)));
-    uint32_t hi = max(lo, (uint32_t)((float)total * __builtin_amdgcn_rcpf((float)(slots - a.bal_batch))) + 2u);
+    uint32_t hi = lo;
+    if ((lo + kw - 1) / kw < even_per_wave) hi = max(lo, (uint32_t)((float)total * __builtin_amdgcn_rcpf((float)(slots - batch))) + 2u);
     // Four sizes between the two at a time: their counts are independent, and two sums share a register (a count is at most
     // slots + sequences + a few, below 2^16).
     while (hi - lo > lo / 16u) {  // (the same in every wave of the launch; hi always fits)
@@ -550,17 +556,29 @@ __device__ __forceinline__ BatchPlace batch_place(const DecodeDev &a, uint32_t s
         else lo = c3 + 1u;
         lo = min(lo, hi);
     }
-    const uint32_t parts = ceil_quot(blocks, hi, __builtin_amdgcn_rcpf((float)hi));
-    const uint32_t end = wave_scan(parts);
-    const unsigned long long at = __ballot(end > slot);
+    const bool evenly = (hi + kw - 1) / kw >= even_per_wave;
+    const uint32_t c = evenly ? max(even, floor_c) : hi, parts = ceil_quot(blocks, c, __builtin_amdgcn_rcpf((float)c));
     BatchPlace r;
-    r.dropped = __any(raw > min(a.capacity, a.kv_len_bound));
-    r.b = at ? (uint32_t)__builtin_ctzll(at) : 0u;
-    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)parts, (int)r.b);
-    r.first = (uint32_t)__builtin_amdgcn_readlane((int)end, (int)r.b) - n;
+    r.dropped = __any(raw > most);
+    bool mine;
+    uint32_t n;
+    if (evenly) {
+        const uint32_t cell = __umulhi(slot, a.rcp_cell), in_cell = slot - cell * n_cell, s = __umulhi(in_cell, a.rcp_even);
+        r.b = cell * per_cell + s, r.first = slot - (in_cell - s * n_even);
+        mine = s < per_cell && r.b < batch;
+        r.b = mine ? r.b : 0u;
+        n = (uint32_t)__builtin_amdgcn_readlane((int)parts, (int)r.b);
+    } else {
+        const uint32_t end = wave_scan(parts);
+        const unsigned long long at = __ballot(end > slot);
+        mine = at != 0;
+        r.b = mine ? (uint32_t)__builtin_ctzll(at) : 0u;
+        n = (uint32_t)__builtin_amdgcn_readlane((int)parts, (int)r.b);
+        r.first = (uint32_t)__builtin_amdgcn_readlane((int)end, (int)r.b) - n;
+    }
     r.len = (uint32_t)__builtin_amdgcn_readlane((int)raw, (int)r.b);
-    r.nsplits = at ? n : 0u;
-    r.split = at ? slot - r.first : 1u;  // (a workgroup without a place leaves where one of an empty partition does)
+    r.nsplits = mine ? n : 0u;
+    r.split = mine ? slot - r.first : 1u;  // (a workgroup without a place leaves where one of an empty partition does)
     return r;
 }
 
@@ -591,7 +609,9 @@ __device__ __forceinline__ U4H rope8(const U4H &x, const U4H &mate, const U4H &c
     return o;
 }
 
-template <int D, bool PAGED, bool SAGE, bool FUSED, bool BF16 = false>
+// BAL: a batch's partitions dealt out by the lengths (batch_place; a variant of its own: as a branch in the paged kernel it cost
+// every paged launch 0.15 to 0.3 us - Hkv 8, D 128, 2 sequences of 4000: 9.8 against 10.1)
+template <int D, bool PAGED, bool SAGE, bool FUSED, bool BF16 = false, bool BAL = false>
 __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(DecodeDev a_by_value) {
     // The arguments are read where the program needs them, straight from the launch's argument block (the struct is its
     // first and only member): a by-value struct is copied field by field at the kernel's entry, which puts every field
@@ -610,6 +630,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     static_assert(!(SAGE && PAGED), "the int8 variant has a contiguous cache");
     static_assert(!(SAGE && BF16), "the int8 variant keeps V in f16");
     static_assert(KSTEPS * 4 == SEGS, "a K row is KSTEPS x 4 segments");
+    static_assert(PAGED || !BAL, "only a paged batch is dealt out by lengths");
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __shared__ uint32_t sm_last;
@@ -674,7 +695,13 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         asm volatile("" ::"s"(a.k), "s"(a.v), "s"(a.block_table), "s"(a.bt_stride), "s"(a.block_size), "s"(a.block_shift),
                      "s"(a.n_kv_heads), "s"(a.capacity), "s"(a.chunk), "s"(a.sub_per_kv), "s"(a.gt), "s"(a.xcd_local),
                      "s"(a.rcp_gx), "s"(a.rcp_gy), "s"(gridDim.x), "s"(gridDim.y), "s"(a.d_len), "s"(a.d_len_stride),
-                     "s"(a.kv_len_add), "s"(a.kv_len), "s"(a.kv_len_bound), "s"(a.bal_batch), "s"(a.bal_per_xcd));
+                     "s"(a.kv_len_add), "s"(a.kv_len), "s"(a.kv_len_bound), "s"(a.bal_seqs), "s"(a.bal_slots),
+                     "s"(a.rcp_even), "s"(a.rcp_cell));
+    }
+    // (the batch's lengths, lane = sequence, ahead of the barrier)
+    uint32_t batch_len = 0;  // lane = sequence
+    if constexpr (BAL) {
+        batch_len = a.d_len[min((uint32_t)lane, (a.bal_seqs & 255u) - 1u) * a.d_len_stride];
     }
     if constexpr (EARLY_START) {
         if (tid == 0) sm_q_ready = 0;
@@ -683,15 +710,15 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     uint32_t y = blockIdx.y, b = blockIdx.z;
     uint32_t split;
     BatchPlace place = {};
-    if (PAGED && a.bal_batch) {
+    if constexpr (BAL) {
         // Slots in an order in which an XCD (workgroup id modulo 8) has consecutive ones: most sequences then have all their
         // partitions on one XCD and exchange them through its L2 (xcd_local below).
         uint32_t slot = blockIdx.x;
-        if (a.bal_per_xcd) {
-            const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, pos = (lin & 7u) * a.bal_per_xcd + (lin >> 3);
+        if (a.bal_slots >> 16) {
+            const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y, pos = (lin & 7u) * (a.bal_slots >> 16) + (lin >> 3);
             y = __umulhi(pos, a.rcp_gx), slot = pos - y * gridDim.x;
         }
-        place = batch_place(a, slot, gridDim.x, NW);
+        place = batch_place(a, batch_len, slot, gridDim.x, NW, FUSED ? NW - 1 : NW);
         b = place.b, split = place.split;
     } else if (a.xcd_local) {
         // All partitions of a head group on ONE XCD (workgroup id modulo 8), so that their partial states meet in that
@@ -885,7 +912,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     // comes through the scalar cache.
     auto read_len = [&]() -> uint32_t {
         typedef const uint32_t __attribute__((address_space(4))) *const_u32p;
-        if (PAGED && a.bal_batch) return place.len;
+        if (BAL) return place.len;
         return a.d_len ? ((const_u32p)a.d_len)[(size_t)b * a.d_len_stride] + a.kv_len_add : a.kv_len;
     };
     // Q^T operand: lane (n, c) of step j holds segment 4j + c of head head0 + n (zero for unused columns)
@@ -1150,10 +1177,10 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     }
     if (!(FUSED && wave == 0)) n_raw = read_len();
     const uint32_t N = min(n_raw, min(a.capacity, a.kv_len_bound));
-    const uint32_t nsplits = PAGED && a.bal_batch ? place.nsplits : (N + a.chunk - 1) / a.chunk;
+    const uint32_t nsplits = BAL ? place.nsplits : (N + a.chunk - 1) / a.chunk;
     // A position at or past the launch bound / the capacity: the token is neither appended nor attended. The host
     // finds the bit at its next synchronize.
-    if (FUSED && (PAGED && a.bal_batch ? place.dropped : n_raw > N) && tid == 0 && blockIdx.x == 0 && y == 0 && a.status) a.status[FA_DEVSTAT_APPEND_DROPPED] = 1u;
+    if (FUSED && (BAL ? place.dropped : n_raw > N) && tid == 0 && blockIdx.x == 0 && y == 0 && a.status) a.status[FA_DEVSTAT_APPEND_DROPPED] = 1u;
     if (split >= nsplits || pad_wg) {  // uniform over the workgroup
         FA_TR_FLUSH();
         return;
@@ -1451,12 +1478,12 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
 
     const bool in_kernel = tl.merge_in_kernel != 0, polled = tl.merge_in_kernel == 2;
     // the first partition of this (sequence, head group) in the exchange buffers
-    const size_t gpart = PAGED && a.bal_batch ? (size_t)y * S + place.first : ((size_t)b * GY + y) * S;
+    const size_t gpart = BAL ? (size_t)y * S + place.first : ((size_t)b * GY + y) * S;
     const size_t gbase = gpart * gt;  // and its first row
     bool xcd_local = tl.xcd_local != 0;
-    if (PAGED && a.bal_batch) {  // all of the sequence's partitions among the slots of this XCD?
-        const uint32_t xcd_first = ((blockIdx.x + gridDim.x * blockIdx.y) & 7u) * a.bal_per_xcd;
-        xcd_local = gpart >= xcd_first && gpart + nsplits <= xcd_first + a.bal_per_xcd;  // (never for bal_per_xcd = 0)
+    if (BAL) {  // all of the sequence's partitions among the slots of this XCD?
+        const uint32_t per_xcd = a.bal_slots >> 16, xcd_first = ((blockIdx.x + gridDim.x * blockIdx.y) & 7u) * per_xcd;
+        xcd_local = gpart >= xcd_first && gpart + nsplits <= xcd_first + per_xcd;  // (never for per_xcd = 0)
     }
     const uint32_t prow = split * gt;
     constexpr int CG = D / 4;
@@ -1552,7 +1579,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     }
     __syncthreads();
     if (!sm_last) return;
-    merge_and_store<D, true, NT>(tl, b, y, nsplits, gbase, tid, reinterpret_cast<float *>(smem), 0, (int)gt);
+    merge_and_store<D, true, NT>(tl, b, y, nsplits, BAL ? gpart : ((size_t)b * gridDim.y + y) * S, tid, reinterpret_cast<float *>(smem), 0, (int)gt);
     if (tid == 0)  // ready for the next launch
         __hip_atomic_store(&tl.counters[(size_t)b * GY + y], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1570,7 +1597,7 @@ __global__ void __launch_bounds__(NT_MERGE) flash_decode_merge_kernel(DecodeDev 
     N = min(N, min(a.capacity, a.kv_len_bound));
     const uint32_t nsplits = (N + a.chunk - 1) / a.chunk;
     if (nsplits <= 1) return;  // written directly by the partition kernel
-    merge_and_store<D, false, NT_MERGE>(a, b, y, nsplits, ((size_t)b * gridDim.y + y) * S * a.gt, threadIdx.x, sm, (int)blockIdx.x, 1);
+    merge_and_store<D, false, NT_MERGE>(a, b, y, nsplits, ((size_t)b * gridDim.y + y) * S, threadIdx.x, sm, (int)blockIdx.x, 1);
 }
 
 enum Mode { MODE_PLAIN = 0, MODE_PAGED = 1, MODE_SAGE = 2, MODE_FUSED = 3, MODE_FUSED_PAGED = 4, MODE_SAGE_FUSED = 5 };
@@ -1617,6 +1644,10 @@ fa_status launch_d(fa_ctx *ctx, const DecodeDev &a, dim3 grid, int mode) {
             FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
             FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, false, false, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
             FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
+            FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, false, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
+            FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, false, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
+            FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, true, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
+            FA_HIP(hipFuncSetAttribute((const void *)flash_decode_mfma_kernel<D, true, false, true, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, cap));
             lds_allowed = true;
         }
     }
@@ -1634,7 +1665,11 @@ fa_status launch_d(fa_ctx *ctx, const DecodeDev &a, dim3 grid, int mode) {
                     scope.launch((flash_decode_mfma_kernel<D, false, false, false>), grid, dim3(NT), lds, a);
                 break;
             case MODE_PAGED:
-                if (a.bf16)
+                if (a.bal_seqs && a.bf16)
+                    scope.launch((flash_decode_mfma_kernel<D, true, false, false, true, true>), grid, dim3(NT), lds, a);
+                else if (a.bal_seqs)
+                    scope.launch((flash_decode_mfma_kernel<D, true, false, false, false, true>), grid, dim3(NT), lds, a);
+                else if (a.bf16)
                     scope.launch((flash_decode_mfma_kernel<D, true, false, false, true>), grid, dim3(NT), lds, a);
                 else
                     scope.launch((flash_decode_mfma_kernel<D, true, false, false>), grid, dim3(NT), lds, a);
@@ -1652,7 +1687,11 @@ fa_status launch_d(fa_ctx *ctx, const DecodeDev &a, dim3 grid, int mode) {
                     scope.launch((flash_decode_mfma_kernel<D, false, false, true>), grid, dim3(NT), lds, a);
                 break;
             default:
-                if (a.bf16)
+                if (a.bal_seqs && a.bf16)
+                    scope.launch((flash_decode_mfma_kernel<D, true, false, true, true, true>), grid, dim3(NT), lds, a);
+                else if (a.bal_seqs)
+                    scope.launch((flash_decode_mfma_kernel<D, true, false, true, false, true>), grid, dim3(NT), lds, a);
+                else if (a.bf16)
                     scope.launch((flash_decode_mfma_kernel<D, true, false, true, true>), grid, dim3(NT), lds, a);
                 else
                     scope.launch((flash_decode_mfma_kernel<D, true, false, true>), grid, dim3(NT), lds, a);

@@ -211,9 +211,19 @@ struct FaDecodeDev {
     uint32_t xcd_local;  // polled merge: a head group's workgroups share an XCD and exchange partials through its L2
     uint32_t rcp_gx, rcp_gy;  // xcd_local: floor(2^32 / d) + 1 for the grid's x and y dimensions (exact quotients of numbers below 2^16 by d < 2^16)
     uint32_t ny_real;    // != 0: the grid's y dimension is padded (to a multiple of 8 head groups) and only y < ny_real exist
-    uint32_t bal_batch;  // != 0: the kernel deals the grid's x dimension out to this many sequences by their lengths
-    uint32_t bal_per_xcd; // ... and deals each XCD this many consecutive partitions (0: in the order of the workgroups)
-    uint32_t nb_q, nb_r;  // contiguous cache: a partition's 16-row blocks over the streaming waves, quotient and remainder
+    // A paged batch whose partitions the kernel deals out by the lengths: sequences (0: not such a launch), then 8 bits each how many
+    // partitions each of them has where they are dealt evenly (2 to 64) and how many sequences of those go into a cell; consecutive
+    // partitions of a cell, then from bit 16 those of an XCD (0: in the order of the workgroups). (Packed, and the reciprocals - as
+    // rcp_gx - where other launches have nb_q and nb_r: one more cache line of arguments costs every decode launch 0.03 us.)
+    uint32_t bal_seqs, bal_slots;
+    union {
+        uint32_t nb_q;      // contiguous cache: a partition's 16-row blocks over the streaming waves, quotient and remainder
+        uint32_t rcp_even;  // bal_seqs: of the partitions of a sequence
+    };
+    union {
+        uint32_t nb_r;
+        uint32_t rcp_cell;  // ... and of a cell
+    };
     unsigned long long poll_ticks;  // polled merge: how long the merging workgroup waits for partials, 100 MHz ticks
     // SAGE + FUSED (the int8 decode step in one launch): q is the raw f16 projection, k the int8 cache (written: the open
     // block's rows), k_scale is written too; the exact rows of the open block, the smoothing mean, the step's quantised query

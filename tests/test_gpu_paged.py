@@ -267,6 +267,11 @@ def test_paged_decode_full_batch_of_32_ragged_sequences():
     (14, 2, 64, 16, [(i * 977) % 4100 for i in range(64)], 0),                  # 64 sequences, every lane of the wave
     (16, 1, 128, 16, [5000, 3, 2222], 8192),                                    # 16 heads per workgroup, 256 slots
     (16, 2, 128, 16, [200, 30, 90, 155, 64, 12], 16384),                        # a bound far above the lengths
+    # about equal lengths, dealt evenly: 16 slots each on an XCD of their own half, 5 each with slots left over, a length of none
+    (16, 2, 128, 16, [8200 + 7 * i for i in range(8)], 0),
+    (16, 2, 128, 16, [2600 + 3 * i for i in range(23)] + [0], 4096),
+    (24, 8, 128, 16, [2000] * 7 + [2047], 0),
+    (6, 3, 128, 48, [3000] * 5, 9216),                                          # ... and not by XCD
 ])
 def test_paged_batch_dealt_out_by_lengths(H, Hkv, D, bs, lens, bound):
     """The launch whose workgroups find their (sequence, partition) from the lengths: against the oracle, and against the
