@@ -1090,15 +1090,21 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
         splits = 1;
         if (base_wgs * 2 <= n_cus) splits = n_cus / base_wgs;  // all workgroups resident at once, one per CU
         if (splits > key_tiles / 4) splits = key_tiles / 4;
-        // What splitting saves the longest item - a pair of key tiles is about 1.5 us - against what it costs: the partial states
-        // stored and the merge launch, 4 us and 0.35 us per MB. A prompt, or a chunk after a short prefix, has too few tiles to
-        // repay it. us, split by the rules above and whole: H16 / Hkv4 / D128, 500 rows: 19.6, 14.5; H16 / Hkv2 / D128, 1000 rows:
-        // 27.8, 20.3; H24 / Hkv8 / D128, 500 rows after 300: 24.4, 18.7; H14 / Hkv2 / D64, 500 rows: 13.2, 11.5, and beyond the
-        // line, 400 rows after 400: 14.4, 15.3, 500 after 1000: 16.0, 21.9.
+        // Split only where it repays: the longest item is spared whole pairs of key tiles (1.2 us each at D 64, 1.45 at D 128), and pays
+        // for storing its rows' partial state (up to 2.1 and 4.3 us) and for the merge launch and what it reads (0.48 and 0.58 us per
+        // MB of all partial states). A prompt, or a chunk after a short prefix, has too few tiles for that. Fitted to 332 chunks of 65
+        // to 1100 rows after 0 to 3000, 4 to 32 heads: the wrong side for six of them, by 0.1 to 0.4 us. us, whole and with the splits
+        // above:
+        //   H16 / Hkv4 / D128:  500 rows 13.4, 19.2; 400 after 600 19.7, 22.1; 100 after 500 15.3, 15.6 | 100 after 600 15.6, 15.3; 65 after 575 14.4, 13.5
+        //   H24 / Hkv8 / D128:  500 after 300 17.6, 24.3; 200 after 800 19.0, 20.2 | 100 after 700 17.4, 16.7; 128 after 800 18.8, 18.3
+        //   H14 / Hkv2 / D64:   500 rows 10.5, 12.4; 700 after 300 14.8, 17.3 | 400 after 400 13.9, 13.5; 500 after 1000 19.3, 15.6
         if (!a.pack_heads && splits > 1) {
-            const float pairs_saved = 0.5f * (float)(key_tiles - ceil_div_u32(key_tiles, splits));
+            const bool wide = L.head_dim == 128;
+            const uint32_t pairs_saved = ceil_div_u32(key_tiles, 2) - ceil_div_u32(ceil_div_u32(key_tiles, splits), 2);
+            const float item_rows = (float)(L.q_len < BM ? L.q_len : BM) / (float)BM;
             const float stored_mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * (float)splits * 4e-6f;
-            if (1.5f * pairs_saved < 4.0f + 0.35f * stored_mb) splits = 1;
+            const float spared = (wide ? 1.45f : 1.2f) * (float)pairs_saved;
+            if (spared < (wide ? 4.25f * item_rows - 0.375f + 0.575f * stored_mb : 2.125f * item_rows + 0.625f + 0.475f * stored_mb)) splits = 1;
         }
         // (packed heads: every split is one more partial per row for the merge, so beyond 16 splits each should have 16
         // tiles. A 32-row chunk after 2K / 8K / 32K tokens measured best with 8 / 16 / 24-32 splits.)

@@ -289,7 +289,9 @@ def test_prefill_split_k_independent_of_split_count(split_k):
 @pytest.mark.parametrize("H,Hkv,D,M,prefix", [
     (14, 2, 64, 400, 112),   # eight key tiles: whole
     (14, 2, 64, 400, 400),   # thirteen: three splits
+    (14, 2, 64, 700, 300),   # sixteen of many rows: whole
     (16, 4, 128, 500, 0), (16, 4, 128, 65, 575), (16, 4, 128, 65, 1000),
+    (16, 4, 128, 100, 500), (16, 4, 128, 100, 600),  # ten tiles: whole, eleven: split
     (16, 2, 128, 1000, 0),   # many rows: what the splits would store decides
 ])
 def test_prefill_automatic_split_on_both_sides_of_its_line(H, Hkv, D, M, prefix):
