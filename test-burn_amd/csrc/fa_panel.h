@@ -34,12 +34,12 @@ struct PanelDev {
     const unsigned char *w[3];
     const __half *scales[3], *bias[3];
     __half *out[3];
-    uint32_t rows0, rows1, rows2, total_rows;
+    uint32_t rows0, rows1, total_rows;  // of W_q, of W_k and W_v each, of all
     const __half *x, *gamma, *residual;
     uint32_t k_dim, m, rows_per_wg, canonical, n_pass;
     float eps, inv_k, alpha, beta;
     RopeDev r;
-    uint32_t rcp_half_nkb, scale_pairs;  // floor(2^32 / ceil(blocks / 2)) + 1; a row holds an even number of scales
+    uint32_t scale_pairs;  // a row holds an even number of scales, 4-byte aligned
     uint32_t block_shift;  // log2 of the page size, 32 = not a power of two
 };
 

@@ -81,11 +81,11 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     const __half *const x_in = a.x, *const gamma = a.gamma;
     const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
     const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
-    const uint32_t normal = a.r.normal, head_dim = a.r.head_dim, rcp_half_nkb = a.rcp_half_nkb, scale_pairs = a.scale_pairs;
+    const uint32_t normal = a.r.normal, head_dim = a.r.head_dim, scale_pairs = a.scale_pairs;
     // (the launch's arguments in two trips through the scalar cache: what the first requests need, and the rest behind them)
     asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(rows0), "s"(rows1), "s"(total_rows), "s"(x_in), "s"(gamma), "s"(K), "s"(m_rows),
                  "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass));
-    if constexpr (WB != 16) asm volatile("" ::"s"(sp0), "s"(sp1), "s"(sp2), "s"(rcp_half_nkb), "s"(scale_pairs));
+    if constexpr (WB != 16) asm volatile("" ::"s"(sp0), "s"(sp1), "s"(sp2), "s"(scale_pairs));
     if constexpr (ROPE) asm volatile("" ::"s"(normal), "s"(head_dim));
     const bool canonical = canonical_u != 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -143,16 +143,14 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         for (int j = 0; j < PK; ++j) g_lds[j * 64 + lane] = gv[j];
     }
     // ---- block scales (block-quantised weights): [block][slot] f16 in LDS, fetched along the rows of the scale matrix, two at a
-    // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request). Behind the last
-    // block comes one of zeros, for the requests past it: an infinite scale read again would make NaN of the input's zeros there.
+    // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request). Past the last block
+    // they are zero: an infinite scale would make NaN of the input's zeros there.
     _Float16 *const sc_lds = reinterpret_cast<_Float16 *>(smem + lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0));
     constexpr int SLOTS = NT * 16, SC_LOADS = WB == 16 ? 1 : (SLOTS * PK * 8 + NTHREADS - 1) / NTHREADS;  // pairs per thread
     uint32_t sc_raw[SC_LOADS];
-    const uint32_t half_nkb = (nkb + 1) / 2;
     auto scale_at = [&](int i, uint32_t &slot, uint32_t &kb2) __attribute__((always_inline)) -> bool {
         const uint32_t idx = (uint32_t)tid + (uint32_t)i * NTHREADS;
-        slot = __umulhi(idx, rcp_half_nkb), kb2 = idx - slot * half_nkb;  // (quotients of numbers below 2^16)
-        if (half_nkb == 1) slot = idx, kb2 = 0;
+        slot = idx / (PK * 8), kb2 = idx % (PK * 8);
         return slot < (uint32_t)SLOTS;
     };
     if constexpr (WB != 16) {
@@ -161,7 +159,8 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             uint32_t slot, kb2;
             int mat;
             bool valid;
-            if (!scale_at(i, slot, kb2)) slot = 0, kb2 = 0;
+            if (!scale_at(i, slot, kb2)) slot = 0;
+            kb2 = min(kb2, (nkb - 1) / 2);
             const uint32_t lrow = locate(slot_row(slot >> 4, slot & 15u, valid), mat);
             const __half *sp = pick3(mat, sp0, sp1, sp2) + (size_t)lrow * nkb + 2 * kb2;
             if (scale_pairs) {
@@ -269,8 +268,8 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                     uint32_t slot, kb2;
                     if (!scale_at(i, slot, kb2)) continue;
                     unsigned short *dst = reinterpret_cast<unsigned short *>(sc_lds) + 2 * kb2 * SLOTS + slot;
-                    dst[0] = (unsigned short)sc_raw[i], dst[SLOTS] = 2 * kb2 + 1 < nkb ? (unsigned short)(sc_raw[i] >> 16) : (unsigned short)0;
-                    if (2 * kb2 + 2 == nkb && nkb < PK * 16u) dst[2 * SLOTS] = 0;
+                    dst[0] = 2 * kb2 < nkb ? (unsigned short)sc_raw[i] : (unsigned short)0;
+                    dst[SLOTS] = 2 * kb2 + 1 < nkb ? (unsigned short)(sc_raw[i] >> 16) : (unsigned short)0;
                 }
             }
         }
@@ -298,7 +297,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         for (int i = 0; i < NQ; ++i) {
             const uint32_t kb = kb_of(i) + lane_blk;
             const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
-            const _Float16 *const scp = sc_lds + min(kb, nkb) * SLOTS + (SUMS ? c * 4 : n);  // (past the last block: scales of zero)
+            const _Float16 *const scp = sc_lds + kb * SLOTS + (SUMS ? c * 4 : n);
             req_t raw[NT];
             _Float16 sc[NT];
 #pragma unroll

@@ -437,7 +437,7 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
     memset(&a, 0, sizeof(a));
     for (int i = 0; i < 3; ++i)
         a.w[i] = reinterpret_cast<const unsigned char *>(l.w[i]), a.scales[i] = l.scales[i], a.bias[i] = l.bias[i], a.out[i] = l.out[i];
-    a.rows0 = l.n_dim, a.rows1 = l.n_kv, a.rows2 = l.n_kv, a.total_rows = l.n_dim + 2 * l.n_kv;
+    a.rows0 = l.n_dim, a.rows1 = l.n_kv, a.total_rows = l.n_dim + 2 * l.n_kv;
     a.x = l.x, a.gamma = l.gamma, a.residual = l.residual, a.k_dim = l.k_dim, a.m = l.m, a.canonical = l.canonical ? 1u : 0u;
     a.eps = l.eps, a.inv_k = 1.0f / (float)l.k_dim, a.alpha = l.alpha, a.beta = l.beta;
     if (rope) {
@@ -459,8 +459,7 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
     }
     const PanelPlan p = panel_plan(ctx, l, rope != nullptr, rope && !rope->rope_normal);
     a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass;
-    const uint32_t nkb = l.k_dim / 32, half_nkb = (nkb + 1) / 2;
-    a.rcp_half_nkb = half_nkb > 1 ? (uint32_t)((1ull << 32) / half_nkb) + 1u : 0u, a.scale_pairs = nkb % 2 == 0 ? 1u : 0u;
+    a.scale_pairs = l.k_dim / 32 % 2 == 0 ? 1u : 0u;
     for (int i = 0; i < 3; ++i)
         if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) a.scale_pairs = 0;
     FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
