@@ -342,13 +342,13 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
     const int wn = wave & 1, wm = wave >> 1;
     const uint32_t a_off = (lane >> 5) * W_STRIDE + (wn * 64 + (lane & 31)) * 16;
     const uint32_t b_off = (lane >> 5) * X_STRIDE + (wm * 64 + (lane & 31)) * 16;
-    f16v_t acc[2][2];
+    f16v_t acc[2][2], sums[2][2];  // (F16: of the last steps, and of all before, where the tile kernels add them up)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = sums[i][j][r] = 0.0f;
 
     const uint32_t all_steps = (K + GM_BK - 1) / GM_BK;
     const uint32_t ks_begin = split * a.steps_per_split;
@@ -359,6 +359,12 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
     for (uint32_t ks = ks_begin; ks < n_steps; ++ks) {
         const bool more = ks + 1 < n_steps;
         if (more) fetch(ks + 1);
+        if (WB == 16 && (ks - ks_begin) % 4 == 3) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) sums[i][j] += acc[i][j], acc[i][j] = f16v_t{};
+        }
         const unsigned char *wa = smem + (ks & 1) * GM_STAGE_BYTES;
         const unsigned char *xa = wa + GM_OPERAND_BYTES;
         {
@@ -380,6 +386,12 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
         __syncthreads();
     }
 
+    if constexpr (WB == 16) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = sums[i][j] + acc[i][j];
+    }
     gemm_epilogue(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
 }
 

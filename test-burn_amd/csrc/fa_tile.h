@@ -19,7 +19,15 @@
 //     tile share the features of a step instead of the input rows (KG) where the tile is small (283 rows, 3072 x 2048 Q8_0:
 //     13.0 -> 9.7 us), and their sums meet in the write stage. The scales of the tile's rows are all in LDS from the start:
 //     a request for 4 bytes of each row would cost the memory unit as much as one for 16 (15.4 -> 13.0 us).
-// F16 sums run over the features in order, whatever the tile: all shapes, and the register-staged kernel, agree to the bit.
+//   * a 32 x 32 x 16 matrix instruction rounds its running sum twice, so a chain's error grows with the root of its length: over 3072
+//     features 5.9 x 2^-24 of the sums' size. F16 tiles of up to 128 x 128, which took the place of parts of a few hundred features
+//     added in a second launch (2.2 x 2^-24), add their accumulators to a second set every FOLD steps, between the products, for
+//     0.5 to 1 % of the time: 2.1 to 2.2 x 2^-24 (1.9 over 896 features, 3.3 in one chain). The larger tiles have no registers for
+//     that, and the launches that they took over had one chain as well. Block-quantised weights are rounded to f16 with their scale,
+//     2^-12 of each operand, beside which a chain's error does not count (1000 x 2^-24 of the sums' size with either); a second set
+//     would cost them 3 to 5 %.
+// F16 sums run over the features in order, whatever the tile: the shapes up to 128 x 128, and the register-staged kernel, agree to
+// the bit.
 #pragma once
 #include "fa_gemm.h"
 #include "fa_lds_dma.h"
@@ -49,6 +57,7 @@ struct Shape {
     // The tiles run over the rows of all matrices as one list (F16; whole groups of 32 rows per matrix): a tile may hold rows of two.
     static constexpr bool JOINED = JOINED_;
     static_assert(!JOINED || WB == 16, "F16 only");
+    static constexpr int FOLD = WB_ == 16 && WM_ * TM_ * WN_ * TN_ <= 16 ? 4 : 0;  // steps, 0: one chain
     static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = 4 / KG;  // KN: products of 16 features per wave and stage
     static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
     static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
@@ -286,13 +295,13 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         }
     };
 
-    f16v_t acc[S::TN][S::TM];
+    f16v_t acc[S::TN][S::TM], sums[S::TN][S::TM];  // (FOLD: of the last steps, and of all before)
 #pragma unroll
     for (int i = 0; i < S::TN; ++i)
 #pragma unroll
         for (int j = 0; j < S::TM; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = sums[i][j][r] = 0.0f;
 
     if constexpr (S::QUANT) {  // all scales first: 16 bytes (8 blocks) of 64 rows per request
         const __half *sp = pick3(tile_mat, a.scales[0], a.scales[1], a.scales[2]);
@@ -314,7 +323,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     // the operands of step ks in registers - their stage is free for step ks + NS - and step ks + 1 has landed for everybody.
     // The requests go out between the products: the memory unit takes a KiB in about 20 cycles, and a wave that issues all of its
     // requests in one go leaves its matrix core idle for as long.
-    auto step = [&](uint32_t cur, uint32_t next, int ks4, const Operands &now, Operands &then) __attribute__((always_inline)) {
+    auto step = [&](uint32_t cur, uint32_t next, int ks4, bool fold, const Operands &now, Operands &then) __attribute__((always_inline)) {
         wait_requests<S::REQ *(S::NS - 2)>();
         meet();
         constexpr int NM = S::KN * S::TN * S::TM;
@@ -326,7 +335,9 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 #pragma unroll
             for (int e = p * S::READS / NM; e < (p + 1) * S::READS / NM; ++e) fetch(then, next, e);
             if (j == 0) fa[i] = w_operand(now, i, q, ks4);
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], now.x[j][q], acc[i][j], 0, 0, 0);
+            f16v_t chain = acc[i][j];
+            if (fold && q == 0) sums[i][j] += chain, chain = f16v_t{};
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], now.x[j][q], chain, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0x6);  // (vector and scalar arithmetic may move: addresses, the conversion of weights)
 #pragma unroll
             for (int r = p * S::REQ / NM; r < (p + 1) * S::REQ / NM; ++r) request(r, cur);
@@ -334,14 +345,15 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         }
     };
     // (unrolled over the stages, so that their places are constants; operands of even and odd steps in registers of their own)
-    constexpr int UNROLL = S::QUANT ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
+    constexpr int UNROLL = S::QUANT || S::FOLD ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
     for (uint32_t left = n_steps;;) {
         bool done = false;
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             const uint32_t cur = u % S::NS * S::STAGE, next = (u + 1) % S::NS * S::STAGE;
-            if (u % 2 == 0) step(cur, next, u % 4, o0, o1);
-            else step(cur, next, u % 4, o1, o0);
+            const bool fold = S::FOLD != 0 && u % 4 == 3;
+            if (u % 2 == 0) step(cur, next, u % 4, fold, o0, o1);
+            else step(cur, next, u % 4, fold, o1, o0);
             if (--left == 0) {
                 done = true;
                 break;
@@ -350,6 +362,12 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         if (done) break;
     }
     wait_requests<0>();  // (the last ones delivered nothing, but they have to be over before the write stage reuses the LDS)
+    if constexpr (S::FOLD != 0) {
+#pragma unroll
+        for (int i = 0; i < S::TN; ++i)
+#pragma unroll
+            for (int j = 0; j < S::TM; ++j) acc[i][j] = sums[i][j] + acc[i][j];
+    }
 
     // Write stage: accumulators -> LDS as f32 [input row][weight row], 32 input rows of every wave at a time, then
     // alpha * sum + bias + beta * residual, one rounding to f16, 16-byte stores (or the rotation and the stores of KvPrepFused).

@@ -71,3 +71,30 @@ def test_tiles(K, H, Hkv, D, m, layout, weights):
         f.set_gemm_min_m()
     for b in dev_w + dev_s + [dx, dg, dres, dout, dcos, dsin] + db + outs + rot[0] + rot[1]:
         b.free()
+
+
+@pytest.mark.parametrize("K,m,variant", [(3072, 300, 0), (3072, 300, 1), (3072, 300, 2), (2048, 1500, 0), (3104, 300, 0)])
+def test_f16_sums_are_added_in_parts(K, m, variant):
+    """The f32 sums of F16 weights behind the output's rounding: out = sums - f16(exact), so that what is left shows them to 2^-24.
+    A chain of n matrix products of 16 features rounds 2 n times by 0.42 x 2^-24 rms of a partial sum that is half the final one in
+    the mean square: 0.42 sqrt(n) x 2^-24 of the sums' size, 1.7 for parts of 256 features; adding N / 256 parts up rounds by
+    0.42 sqrt(N / 512), 1.0 over 3072. Together 2.0, the bar 1.5 times that; one chain over 2048 features would be 4.7, over 3072
+    5.8."""
+    announce("F16 sums", K, m, variant)
+    f = ctx()
+    rng = np.random.default_rng(K + m)
+    N = 256
+    x = rng.normal(size=(m, K)).astype(np.float16)
+    w = (rng.normal(size=(N, K)) * K ** -0.5).astype(np.float16)
+    exact = x.astype(np.float64) @ w.astype(np.float64).T
+    rounded = exact.astype(np.float16)
+    dx, dw, dres, dout = f.array(x), f.array(w.reshape(-1)), f.array(-rounded), f.zeros((m, N))
+    try:
+        f.set_gemm_variant(variant)
+        f.matmul(dx.arg(), dw.arg(), dout.arg(), m, N, K, c=dres.arg(), transpose_b=True, beta=1.0)
+        err = dout.download().astype(np.float64) - (exact - rounded.astype(np.float64))
+    finally:
+        f.set_gemm_variant()
+    assert np.sqrt(np.mean(err ** 2) / np.mean(exact ** 2)) * 2 ** 24 <= 3.0, np.sqrt(np.mean(err ** 2) / np.mean(exact ** 2)) * 2 ** 24
+    for b in (dx, dw, dres, dout):
+        b.free()
