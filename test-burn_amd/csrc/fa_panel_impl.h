@@ -245,11 +245,12 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 for (int j = 0; j < PK; ++j) xr[i][j] = fa_norm::scale8(xr[i][j], inv_rms, G_IN_LDS<PK> ? g_lds[j * 64 + lane] : gv[j]);
             }
         }
-        f4v_t d[NT][NC];
+        constexpr int CHAINS = WB == 16 && PK > 4 ? 2 : 1;
+        f4v_t d[NT][NC], d2[NT][NC];  // (the longest rows: two chains, 2.0 x 2^-24 of the sums' size as their error, 2.4 with one)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int h = 0; h < NC; ++h) d[t][h] = f4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int h = 0; h < NC; ++h) d[t][h] = d2[t][h] = f4v_t{0.0f, 0.0f, 0.0f, 0.0f};
         _Float16 s_res[NT], rc[NT], rs[NT];
         uint32_t r_pos = 0, r_blk = 0;
         if (!APART && pass != blockIdx.y) __syncthreads();  // the sums have been read
@@ -327,10 +328,19 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                     } else {
                         const h8_t w = WB == 16 ? W::f16(W::part(raw[t], 0), (_Float16)1.0f) : W::f16(W::part(raw[t], st), sc[t]);
 #pragma unroll
-                        for (int h = 0; h < NC; ++h) d[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[h], d[t][h], 0, 0, 0);
+                        for (int h = 0; h < NC; ++h) {
+                            f4v_t &sum = i % CHAINS ? d2[t][h] : d[t][h];
+                            sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[h], sum, 0, 0, 0);
+                        }
                     }
                 }
             }
+        }
+        if constexpr (CHAINS == 2) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int h = 0; h < NC; ++h) d[t][h] += d2[t][h];
         }
         if (!APART) __syncthreads();  // everyone has read the rows
 #pragma unroll
