@@ -62,8 +62,12 @@ constexpr int lds_rows_bytes() {
     const int rows = NC * 16 * row_bytes<PK>(), red = reduce_bytes<NT, NC>();
     return REDUCE_APART<NT, NC, PK> ? rows + red : rows > red ? rows : red;
 }
+// Block-quantised weights: their scales as f16 [block][slot], with 8 bytes between blocks: a wave writes the blocks of two or three
+// rows side by side, all of them to one bank without (o_proj of 1536 features x 4096 rows, 40 input rows: Q8_0 7.06 -> 6.64 us).
+template <int NT>
+constexpr int scale_stride() { return NT * 16 + 4; }
 template <int NT, int PK>
-constexpr int scale_bytes() { return NT * 16 * PK * 16 * 2; }  // block-quantised weights: [block][slot] f16
+constexpr int scale_bytes() { return scale_stride<NT>() * PK * 16 * 2; }
 template <int WB, int NT, int NC, int PK>
 constexpr int lds_bytes() { return lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0) + (WB != 16 ? scale_bytes<NT, PK>() : 0); }
 

@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request). Past the last block
     // they are zero: an infinite scale would make NaN of the input's zeros there.
     _Float16 *const sc_lds = reinterpret_cast<_Float16 *>(smem + lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0));
-    constexpr int SLOTS = NT * 16, SC_LOADS = WB == 16 ? 1 : (SLOTS * PK * 8 + NTHREADS - 1) / NTHREADS;  // pairs per thread
+    constexpr int SLOTS = NT * 16, SC_STRIDE = scale_stride<NT>(), SC_LOADS = WB == 16 ? 1 : (SLOTS * PK * 8 + NTHREADS - 1) / NTHREADS;  // pairs per thread
     uint32_t sc_raw[SC_LOADS];
     auto scale_at = [&](int i, uint32_t &slot, uint32_t &kb2) __attribute__((always_inline)) -> bool {
         const uint32_t idx = (uint32_t)tid + (uint32_t)i * NTHREADS;
@@ -159,8 +159,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             uint32_t slot, kb2;
             int mat;
             bool valid;
-            if (!scale_at(i, slot, kb2)) slot = 0;
-            kb2 = min(kb2, (nkb - 1) / 2);
+            if (!scale_at(i, slot, kb2) || 2 * kb2 >= nkb) slot = 0, kb2 = 0;
             const uint32_t lrow = locate(slot_row(slot >> 4, slot & 15u, valid), mat);
             const __half *sp = pick3(mat, sp0, sp1, sp2) + (size_t)lrow * nkb + 2 * kb2;
             if (scale_pairs) {
@@ -268,9 +267,9 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 for (int i = 0; i < SC_LOADS; ++i) {
                     uint32_t slot, kb2;
                     if (!scale_at(i, slot, kb2)) continue;
-                    unsigned short *dst = reinterpret_cast<unsigned short *>(sc_lds) + 2 * kb2 * SLOTS + slot;
+                    unsigned short *dst = reinterpret_cast<unsigned short *>(sc_lds) + 2 * kb2 * SC_STRIDE + slot;
                     dst[0] = 2 * kb2 < nkb ? (unsigned short)sc_raw[i] : (unsigned short)0;
-                    dst[SLOTS] = 2 * kb2 + 1 < nkb ? (unsigned short)(sc_raw[i] >> 16) : (unsigned short)0;
+                    dst[SC_STRIDE] = 2 * kb2 + 1 < nkb ? (unsigned short)(sc_raw[i] >> 16) : (unsigned short)0;
                 }
             }
         }
@@ -298,7 +297,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         for (int i = 0; i < NQ; ++i) {
             const uint32_t kb = kb_of(i) + lane_blk;
             const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
-            const _Float16 *const scp = sc_lds + kb * SLOTS + (SUMS ? c * 4 : n);
+            const _Float16 *const scp = sc_lds + kb * SC_STRIDE + (SUMS ? c * 4 : n);
             req_t raw[NT];
             _Float16 sc[NT];
 #pragma unroll
