@@ -515,11 +515,12 @@ fa_status fa_fused_qkv_kv_prep_paged(fa_ctx *ctx, const fa_tensor_arg *w_q, cons
  * (FA_ERR_OPERATION_NOT_SUPPORTED). bias, c: NULL or NULL buffer = absent (the reference's "zero" placeholder).
  * Any m is accepted: up to fa_set_gemm_min_m() - 1 input rows run as passes of 16 over the weight stream; from there
  * on the op is a tiled GEMM on the matrix cores, the counterpart of the reference's GEMM for large m (src/metals/mma).
- * A chunk of input rows of up to 3072 features (the reference's default prefill chunk is 32 rows; 2 to 64 rows, up to 128 where
- * rows have at most 2048 features and 512 where they have at most 1024) is one launch of a kernel of its own instead of the
- * GEMM's three, norm included, unless fa_set_gemm_min_m() was called with a threshold the chunk reaches - or, for
- * block-quantised weights, at all (environment FOUNDRY_ATTN_QKV_ROWS32_MIN_M, read at fa_ctx_create: the fewest rows it takes,
- * 33 = never).
+ * A chunk of input rows of up to 3072 features (the reference's default prefill chunk is 32 rows) is one launch of a kernel of
+ * its own instead of the GEMM's two or three, norm included: 2 to 11 rows always; from 12 on up to 64 rows (48 with block-quantised
+ * weights), 128 where rows have at most 2048 features, 192 - with a norm 416 - where they have at most 1024, unless the GEMM is
+ * clearly ahead by estimate (many weight rows). fa_set_gemm_min_m() with a threshold that the chunk reaches - or, for
+ * block-quantised weights, at all - takes it to the GEMM (environment FOUNDRY_ATTN_QKV_ROWS32_MIN_M, read at fa_ctx_create: the
+ * fewest rows the kernel takes, 33 = never).
  * Block-quantised weights follow the arithmetic of the path that runs: the weight stream multiplies each 32-block's f32
  * sum by the block scale (the GEMV policies, policy_q8.metal / policy_q4_0.metal), the GEMM works on f16(weight * scale)
  * tiles like the reference's tile loader (src/metals/mma/tile_loader.metal:100-120); the two differ by the f16 rounding

@@ -129,7 +129,7 @@ extern "C" fa_status fa_ctx_create(int device, fa_ctx **out) {
     ctx->sage_fused_step = env_u32("FOUNDRY_ATTN_SAGE_FUSED", 1);
     if (ctx->prefill_variant > 3) ctx->prefill_variant = 0;
     ctx->ledger = new FaGraphLedger();
-    fa_status s = fa_ensure_workspace(ctx, (size_t)64 << 20);
+    fa_status s = fa_ensure_workspace(ctx, FA_WORKSPACE_INITIAL);
     if (s == FA_OK) s = fa_ensure_counters(ctx, 4096);
     if (s == FA_OK) s = fa_decode_probe_xcd(ctx);
     if (s == FA_OK && env_u32("FOUNDRY_ATTN_DECODE_XCD_LOCAL", 1) == 0) ctx->xcd_round_robin = false;

@@ -481,24 +481,11 @@ __global__ void __launch_bounds__(256) gemm_finish_kernel(GemmDev a) {
 
 }  // namespace
 
-// Whether the tile kernels (fa_tile.h) take a launch, and with which tile: whole steps of 64 features, whole 16-byte stores, operands
-// below 2 GiB (32-bit offsets). What a tile of each shape takes per step of 64 features with one workgroup on every CU, in units of the
-// 64 x 64 tile's 0.21 us (from launches of 160 to 256 tiles over 3072 features), times the rounds of workgroups that the launch has:
-// the larger tiles read less per product, the smaller ones leave fewer CUs idle.
-static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, uint32_t n_cus, fa_tile::TileShape &shape) {
-    const uint64_t max_rows = std::max(a.rows[0], a.rows[1]);
-    if (l.k_dim % 64 != 0 || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
-    for (int i = 0; i < 3; ++i)
-        if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) return false;
-    // tiles over the rows of all matrices need them within the reach of one descriptor
-    uintptr_t low = (uintptr_t)l.w[0], high = low;
-    for (int i = 0; i < 3; ++i)
-        if (a.rows[i]) low = std::min(low, (uintptr_t)l.w[i]), high = std::max(high, (uintptr_t)l.w[i] + (size_t)a.rows[i] * l.k_dim * 2);
-    const bool joined = l.weight_bits == 16 && high - low < 0xfffffff0ull && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
-    if (joined) {
-        a.w_low = (const void *)low, a.w_span = (uint32_t)(high - low);
-        for (int i = 0; i < 3; ++i) a.w_at[i] = a.rows[i] ? (uint32_t)((uintptr_t)l.w[i] - low) : 0u;
-    }
+// The cheapest tile shape for a launch over rows[i] weight rows per matrix, and its cost: what a tile of each shape takes per step of
+// 64 features with one workgroup on every CU, in units of the 64 x 64 tile's 0.21 us (from launches of 160 to 256 tiles over 3072
+// features), times the rounds of workgroups that the launch has. The larger tiles read less per product, the smaller ones leave
+// fewer CUs idle. `joined`: tiles may hold rows of two matrices. `variant`: a shape asked for by name (fa_set_gemm_variant).
+static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint32_t n_cus, bool joined, uint32_t variant, fa_tile::TileShape &shape) {
     struct Choice {
         fa_tile::TileShape shape;
         uint32_t m, n;
@@ -514,11 +501,11 @@ static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, 
         if (c.shape == fa_tile::TILE_256x160 && !joined) continue;
         // (a block-quantised tile's scales lie in LDS over the whole of k_dim)
         if (l.weight_bits != 16 && c.shape != fa_tile::TILE_64x64 && l.k_dim > 4096) continue;
-        if (ctx->gemm_variant == 2 && c.shape != fa_tile::TILE_128x128) continue;
-        if (ctx->gemm_variant == 3 && c.shape != fa_tile::TILE_64x64) continue;
+        if (variant == 2 && c.shape != fa_tile::TILE_128x128) continue;
+        if (variant == 3 && c.shape != fa_tile::TILE_64x64) continue;
         uint32_t n_tiles = 0;
-        for (int i = 0; i < 3; ++i) n_tiles += ceil_div_u32(a.rows[i], c.n);
-        if (c.shape == fa_tile::TILE_256x160) n_tiles = ceil_div_u32(a.rows[0] + 2 * a.rows[1], c.n);
+        for (int i = 0; i < 3; ++i) n_tiles += ceil_div_u32(rows[i], c.n);
+        if (c.shape == fa_tile::TILE_256x160) n_tiles = ceil_div_u32(rows[0] + 2 * rows[1], c.n);
         const uint64_t tiles = (uint64_t)n_tiles * ceil_div_u32(l.m, c.m);
         const float cost = (float)((tiles + n_cus - 1) / n_cus) * (l.weight_bits == 16 ? c.f16 : c.quantised);
         if (best == 0.0f || cost < best) {
@@ -527,7 +514,85 @@ static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, 
             if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && tiles <= n_cus && l.k_dim <= 8192) shape = fa_tile::TILE_64x64_DEEP;
         }
     }
-    return best != 0.0f && (l.weight_bits == 16 || l.k_dim <= 16384);
+    return best;
+}
+
+// How the register-staged kernel divides a launch: the feature steps of a tile over enough workgroups to give every CU a share of the
+// weight stream, at least 4 steps each (512 rows of the Llama-3.2-3B projections: 42.9 -> 35.9 us with 3).
+struct Division {
+    uint32_t k_splits, steps_per_split;
+    uint64_t n_wg;  // tiles
+};
+static Division divide(const FusedQkvLaunch &l, uint32_t n_cus, bool whole) {
+    Division d;
+    d.n_wg = (uint64_t)(ceil_div_u32(l.n_dim, GM_TN) + 2 * ceil_div_u32(l.n_kv, GM_TN)) * ceil_div_u32(l.m, GM_TM);
+    const uint32_t all_steps = ceil_div_u32(l.k_dim, GM_BK);
+    uint32_t splits = whole ? 1u : (uint32_t)(2 * n_cus / d.n_wg);
+    if (splits > all_steps / 4) splits = all_steps / 4;
+    if (splits < 1) splits = 1;
+    d.steps_per_split = ceil_div_u32(all_steps, splits);
+    d.k_splits = ceil_div_u32(all_steps, d.steps_per_split);
+    return d;
+}
+
+// What a launch takes on the tile kernels and, divided, on the register-staged one, in us: fitted to launches of 16 to 400 rows over
+// 512 to 8192 features and 512 to 10240 weight rows (on the tiles within 4 to 7 % rms, divided 8 %). The norm's launch is in both.
+static float weight_mb(const FusedQkvLaunch &l) {
+    return (float)l.k_dim * (float)(l.n_dim + 2 * l.n_kv) * (l.weight_bits == 16 ? 2.0f : l.weight_bits == 8 ? 1.0625f : 0.5625f) * 1e-6f;
+}
+static float tile_us(const FusedQkvLaunch &l, float cost) {
+    const bool f16 = l.weight_bits == 16;
+    const float k = (float)l.k_dim, mb = weight_mb(l);
+    const float norm = l.gamma ? (f16 ? 2.3f + 3.0e-6f * (float)l.m * k : 2.0f + 2.6e-6f * (float)l.m * k) : 0.0f;
+    return f16 ? 1.5f + cost * (0.137f * k / 64.0f + 1.43f) + norm + 0.076f * mb : 3.4f + cost * (0.178f * k / 64.0f + 0.1f) + norm + 0.064f * mb;
+}
+static float divided_us(const FusedQkvLaunch &l, const Division &d, uint32_t n_cus) {
+    const float parts_mb = (float)d.k_splits * (float)l.m * (float)(l.n_dim + 2 * l.n_kv) * 4e-6f;
+    const float rounds = (float)((d.n_wg * d.k_splits + 2 * n_cus - 1) / (2 * n_cus));
+    return 8.0f + 0.89f * rounds * (float)d.steps_per_split + 0.35f * parts_mb + 0.094f * weight_mb(l) +
+           (l.gamma ? 2.9f + 0.76e-6f * (float)l.m * (float)l.k_dim : 0.0f);
+}
+
+// What the tile kernels ask of the features, the weight rows and the scales: whole steps of 64 features, whole 16-byte stores, pairs of
+// scales.
+static bool tiles_fit(const FusedQkvLaunch &l) {
+    for (int i = 0; i < 3; ++i)
+        if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) return false;
+    return l.k_dim % 64 == 0 && l.n_dim % 8 == 0 && l.n_kv % 8 == 0 && (l.weight_bits == 16 || l.k_dim <= 16384);
+}
+
+float fa_gemm_estimate_us(const fa_ctx *ctx, const FusedQkvLaunch &l) {
+    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u, rows[3] = {l.n_dim, l.n_kv, l.n_kv};
+    const float divided = divided_us(l, divide(l, n_cus, false), n_cus);
+    fa_tile::TileShape shape;
+    return tiles_fit(l) ? std::min(divided, tile_us(l, best_tile(l, rows, n_cus, false, 0, shape))) : divided;
+}
+
+// Whether the tile kernels (fa_tile.h) take a launch, and with which tile: whole steps of 64 features, whole 16-byte stores, operands
+// below 2 GiB (32-bit offsets).
+static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, uint32_t n_cus, fa_tile::TileShape &shape) {
+    const uint64_t max_rows = std::max(a.rows[0], a.rows[1]);
+    if (!tiles_fit(l) || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
+    // tiles over the rows of all matrices need them within the reach of one descriptor
+    uintptr_t low = (uintptr_t)l.w[0], high = low;
+    for (int i = 0; i < 3; ++i)
+        if (a.rows[i]) low = std::min(low, (uintptr_t)l.w[i]), high = std::max(high, (uintptr_t)l.w[i] + (size_t)a.rows[i] * l.k_dim * 2);
+    const bool joined = l.weight_bits == 16 && high - low < 0xfffffff0ull && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
+    if (joined) {
+        a.w_low = (const void *)low, a.w_span = (uint32_t)(high - low);
+        for (int i = 0; i < 3; ++i) a.w_at[i] = a.rows[i] ? (uint32_t)((uintptr_t)l.w[i] - low) : 0u;
+    }
+    const float cost = best_tile(l, a.rows, n_cus, joined, ctx->gemm_variant, shape);
+    if (cost == 0.0f) return false;
+    if (ctx->gemm_variant != 0) return true;
+    // Few tiles over many features are one long chain of steps each: divided where that is well ahead by both estimates (us, tiles and
+    // divided: 16 rows, 8192 features x 1024, Q8_0 25.6, 14.4; 32 rows, 5120 x 1024, Q4_0 18.0, 12.2; 64 rows, 4096 x 512, Q8_0 14.5,
+    // 11.9 | 16 rows, 4096 x 4096, Q8_0 14.8, 15.4, F16 12.8, 15.6; 100 rows, 5120 x 1536, Q8_0 21.7, 22.8), and only into partial
+    // sums that the workspace of a new context holds: a recorded graph, which cannot let it grow, takes what the tiles took.
+    const Division d = divide(l, n_cus, false);
+    const size_t norm_bytes = l.gamma ? (size_t)l.m * l.k_dim * sizeof(__half) + 256 : 0;
+    if (norm_bytes + (size_t)d.k_splits * l.m * (l.n_dim + 2 * l.n_kv) * sizeof(float) > FA_WORKSPACE_INITIAL) return true;
+    return divided_us(l, d, n_cus) >= 0.87f * tile_us(l, cost);
 }
 
 static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch *rope) {
@@ -575,15 +640,10 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     fa_tile::TileShape shape;
     const bool tiles_whole = choose_tile(ctx, l, a, n_cus, shape);
-    // The register-staged kernel with few output tiles: the feature steps of a tile are divided over enough workgroups to give
-    // every CU a share of the weight stream, at least 4 steps each (512 rows of the Llama-3.2-3B projections: 42.9 -> 35.9 us with 3).
-    // (What the tile kernels could take is not divided either: their sums and this kernel's are the same to the bit.)
-    const uint32_t all_steps = ceil_div_u32(l.k_dim, GM_BK);
-    uint32_t splits = tiles_whole ? 1u : (uint32_t)(2 * n_cus / n_wg);
-    if (splits > all_steps / 4) splits = all_steps / 4;
-    if (splits < 1) splits = 1;
-    a.steps_per_split = ceil_div_u32(all_steps, splits);
-    a.k_splits = ceil_div_u32(all_steps, a.steps_per_split);
+    // (What the tile kernels could take is not divided where the register-staged kernel is asked for by name: their sums and this
+    // kernel's are the same to the bit.)
+    const Division d = divide(l, n_cus, tiles_whole);
+    a.steps_per_split = d.steps_per_split, a.k_splits = d.k_splits;
     a.n_total = a.rows[0] + a.rows[1] + a.rows[2];
     const size_t norm_bytes = l.gamma ? (((size_t)l.m * l.k_dim * sizeof(__half) + 255) & ~(size_t)255) : 0;
     const size_t partial_bytes = a.k_splits > 1 ? (size_t)a.k_splits * l.m * a.n_total * sizeof(float) : 0;

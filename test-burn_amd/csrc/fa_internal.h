@@ -291,6 +291,7 @@ struct FusedQkvLaunch {
 // weight_stream_only: never the GEMM (whose scratch is the context's workspace), whatever the number of input rows
 fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_stream_only = false);
 fa_status fa_launch_fused_qkv_gemm(fa_ctx *ctx, const FusedQkvLaunch &l);  // fa_gemm.hip: many input rows
+float fa_gemm_estimate_us(const fa_ctx *ctx, const FusedQkvLaunch &l);     // ... and what that would take, norm included
 fa_status fa_launch_gemv_row(fa_ctx *ctx, const FusedQkvLaunch &l, bool *taken);  // fa_gemv.hip: one input row
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l);       // fa_qkv.hip: a chunk that the one-launch kernel for short chunks (fa_panel.h) takes
 
@@ -325,6 +326,7 @@ constexpr uint32_t FA_DEVSTAT_WORDS = 4u;
 // stream ends with it.
 fa_status fa_check_device_status(fa_ctx *ctx);
 
+constexpr size_t FA_WORKSPACE_INITIAL = (size_t)64 << 20;  // what a new context starts with
 fa_status fa_ensure_workspace(fa_ctx *ctx, size_t bytes);
 fa_status fa_ensure_counters(fa_ctx *ctx, uint32_t n);
 // Size of the static device array that holds the decode partials of fa_decode_step_fused_noalloc (per GPU, for the

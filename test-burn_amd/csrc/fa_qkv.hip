@@ -26,6 +26,7 @@
 #include "fa_norm.h"
 #include "fa_panel.h"
 #include "fa_qkv_rope.h"
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -394,7 +395,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 // How a FusedQkv / MatMul launch runs on the panel kernel (fa_panel.h): 16-row tiles of weight rows per workgroup, 16-row groups
 // of input rows per pass, weight rows per workgroup, workgroups along the passes.
 struct PanelPlan {
-    uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y;
+    uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y, rounds;
 };
 static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope, bool neox_rope) {
     PanelPlan p;
@@ -411,17 +412,23 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
         uint32_t gy = slots / gx;
         gy = gy < 1 ? 1u : gy > p.n_pass ? p.n_pass : gy;
         const uint32_t cost = ceil_div_u32(gx * gy, slots) * ceil_div_u32(p.n_pass, gy) * (4 + nt);
-        if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy;
+        if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy, p.rounds = ceil_div_u32(gx * gy, slots);
     }
     return p;
 }
 
 // Whether a FusedQkv / MatMul launch goes to the panel kernel: rows of up to 3072 features, from two input rows (four layers of the
 // Llama-3.2-3B block with 2 / 4 / 8 / 11 rows: 113 / 113 / 115 / 117 us against 120 / 128 / 137 / 155 with the kernel for up to 16
-// rows) to as many as it is measured to beat the tile kernels with - later where those need the normalisation's launch in front
-// (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against 5.1), earlier
-// for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer). An explicit GEMM threshold
-// (fa_set_gemm_min_m) wins.
+// rows). Up to 32 rows whose weight rows fit one round of workgroups always (a default chunk is one launch). Beyond, up to as many as
+// it is measured to beat the tile kernels with where the weight rows suit it - later where those need the normalisation's launch in
+// front (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against 5.1),
+// earlier for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer) - unless the GEMM is a tenth ahead by
+// estimate: many weight rows are many passes of the input rows here, or rounds of workgroups. A launch takes the weight stream, and
+// for each pass that a compute unit has one after the other the input rows of that pass, fetched and multiplied and, with a gamma,
+// normalised (fitted to launches of 12 to 416 rows over 512 to 3072 features and 512 to 10240 weight rows; of 1380 with both sides
+// measured, none that leaves is more than 2 % slower for it). us, here and as a GEMM: 2048 x 10240 32 rows 16.6, 12.4, 100 rows 44.5,
+// 17.6; 2048 x 2560 64 rows 8.2, 11.0, 100 rows 12.8, 11.1; 1024 x 6144 100 rows 13.2, 8.8; 3072 x 5120 32 rows 13.5, 13.5, 64 rows
+// 20.1, 14.7. An explicit GEMM threshold (fa_set_gemm_min_m) wins.
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
@@ -429,7 +436,17 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : 192u) : l.k_dim <= 2048 ? 128u : l.weight_bits == 16 ? 64u : 48u;
     if (min_m > 32 || l.m < min_m || l.m > max_m || l.k_dim > 3072 || l.k_dim % 32 != 0) return false;
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
-    return aligned16(l.x) && aligned16(l.w[0]) && aligned16(l.w[1]) && aligned16(l.w[2]) && aligned16(l.gamma);
+    if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
+    if (l.m < FA_GEMM_MIN_M_DEFAULT) return true;
+    const PanelPlan p = panel_plan(ctx, l, false, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
+    if (l.m <= 32 && p.rounds == 1) return true;
+    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
+    // passes of a compute unit (with two workgroups on it they share its way to L2)
+    const float passes = p.pk > 2 ? (float)(p.rounds * ceil_div_u32(p.n_pass, p.grid_y)) : std::max(1.0f, (float)(p.grid_x * p.n_pass) / (float)n_cus);
+    const bool f16 = l.weight_bits == 16;
+    const float k = (float)l.k_dim, mb = k * (float)(l.n_dim + 2 * l.n_kv) * (f16 ? 2.0f : l.weight_bits == 8 ? 1.0625f : 0.5625f) * 1e-6f;
+    const float per_pass = (float)p.nc * k / 1024.0f * (f16 ? (l.gamma ? 1.23f : 0.78f) : l.gamma ? 1.47f : 0.94f);
+    return fa_gemm_estimate_us(ctx, l) >= 0.9f * (2.5f + (f16 ? 0.09f : 0.115f) * mb + passes * per_pass);
 }
 
 static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRopeLaunch *rope) {

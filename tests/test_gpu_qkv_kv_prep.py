@@ -30,9 +30,9 @@ def _paths(m):
 
 @pytest.mark.parametrize("H,Hkv,D,K,m,pos,cap,mode,norm,bias,layout,layer,step", [
     (24, 8, 128, 3072, 256, 0, 512, fa.ROPE_NORMAL, True, False, 1, 0, 0),     # Llama-3.2-3B, a 256-token chunk
-    (24, 8, 128, 3072, 32, 8160, 8448, fa.ROPE_NORMAL, True, False, 1, 0, 0),  # the reference's default chunk after a prefix (split-K)
+    (24, 8, 128, 3072, 32, 8160, 8448, fa.ROPE_NORMAL, True, False, 1, 0, 0),  # the reference's default chunk after a prefix
     (14, 2, 64, 896, 200, 37, 384, fa.ROPE_NEOX, True, True, 0, 0, 0),         # Qwen2.5-0.5B: NeoX pairs, biases, 2 heads per tile, ragged tiles
-    (14, 2, 64, 896, 32, 5, 128, fa.ROPE_NEOX, True, True, 1, 0, 0),           # same through split-K: the mate piece summed a second time
+    (14, 2, 64, 896, 32, 5, 128, fa.ROPE_NEOX, True, True, 1, 0, 0),           # same, a default chunk
     (16, 4, 128, 1024, 130, 3, 256, fa.ROPE_NEOX, False, False, 1, 3, 4),      # SmolLM3 rule: layer 3 of every 4 is not rotated
     (16, 4, 128, 1024, 130, 3, 256, fa.ROPE_NEOX, False, True, 1, 2, 4),       # ... layer 2 is
     (8, 8, 64, 512, 5, 100, 128, fa.ROPE_NORMAL, True, True, 1, 0, 0),         # a few rows: weight stream, then KvPrepFused, inside the op
@@ -44,6 +44,13 @@ def _paths(m):
     (32, 8, 64, 3072, 12, 50, 64, fa.ROPE_NORMAL, True, True, 1, 0, 0),        # adjacent pairs, 64-wide heads, biases
     (16, 4, 128, 2048, 20, 3, 64, fa.ROPE_NEOX, True, False, 1, 3, 4),         # a layer that is not rotated
     (16, 4, 128, 2048, 20, 3, 64, fa.ROPE_NEOX, True, False, 1, 2, 4),         # ... and one that is
+    # few tiles over many features: partial sums, and KvPrepFused as the write stage of the kernel that adds them (NeoX: the mate's
+    # piece is added there a second time); by choice (whole steps of 64 features) and because no tile kernel takes the features
+    (4, 1, 64, 6144, 16, 5, 32, fa.ROPE_NEOX, True, True, 1, 0, 0),
+    (4, 1, 128, 5120, 33, 5, 64, fa.ROPE_NORMAL, True, True, 0, 0, 0),
+    (3, 1, 64, 3104, 40, 7, 64, fa.ROPE_NEOX, True, True, 1, 0, 0),
+    (3, 1, 128, 3104, 40, 7, 64, fa.ROPE_NORMAL, False, True, 1, 0, 0),
+    (3, 1, 128, 3104, 12, 0, 64, fa.ROPE_NEOX, True, False, 1, 3, 4),          # a layer that is not rotated
 ])
 def test_fused_op_equals_the_two_ops(H, Hkv, D, K, m, pos, cap, mode, norm, bias, layout, layer, step):
     announce("fused qkv + kv prep", H, Hkv, D, K, m, pos, cap, mode, norm, bias, layout, layer, step)
@@ -171,6 +178,33 @@ def test_fused_op_of_a_short_chunk_is_one_launch():
     kc, vc = dkc.download(), dvc.download()
     assert not kc[:, :pos].any() and not kc[:, pos + m:].any() and kc[:, pos:pos + m].any()  # only the chunk's rows are written
     assert not vc[:, :pos].any() and not vc[:, pos + m:].any() and vc[:, pos:pos + m].any()
+    for b in dev_w + [dx, dg, dcos, dsin, dqr, dkc, dvc]:
+        b.free()
+
+
+@pytest.mark.parametrize("K,norm,mode", [(3104, True, fa.ROPE_NEOX), (3104, False, fa.ROPE_NORMAL), (6144, True, fa.ROPE_NEOX)])
+def test_launches_of_a_divided_gemm(K, norm, mode):
+    """Few tiles over many features as one op: the norm, the divided GEMM, and the kernel that adds its parts and rotates them."""
+    announce("fused qkv + kv prep, launches of a divided gemm", K, norm, mode)
+    f = ctx()
+    H, Hkv, D, m, cap = 3, 1, 64, 40, 64
+    x, g, ws, _ = _data(np.random.default_rng(K), K, H * D, Hkv * D, m)
+    cos, sin = fa.rope_tables(5e5, D, cap)
+    dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+    dx, dg, dcos, dsin = f.array(x), f.array(g), f.array(cos), f.array(sin)
+    dqr, dkc, dvc = f.zeros((H, m, D)), f.zeros((Hkv, cap, D)), f.zeros((Hkv, cap, D))
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, m, 3, cap, mode)
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        f.fused_qkv_kv_prep(dx.arg(), dev_w[0].arg(), dev_w[1].arg(), dev_w[2].arg(), K, dqr.arg(), dcos.arg(), dsin.arg(), p,
+                            k_cache=dkc.arg(), v_cache=dvc.arg(), gamma=dg.arg() if norm else None)
+        f.synchronize()
+        for kernel, n in (("rmsnorm_rows_kernel", int(norm)), ("fused_qkv_gemm_kernel", 1), ("gemm_finish_kernel", 1),
+                          ("fused_qkv_rows32_rope_kernel", 0), ("kv_prep_fused_vec_kernel", 0), ("kv_prep_fused_elem_kernel", 0)):
+            assert f.profile_query(kernel)[0] == n, kernel
+    finally:
+        f.profile_enable(False)
     for b in dev_w + [dx, dg, dcos, dsin, dqr, dkc, dvc]:
         b.free()
 

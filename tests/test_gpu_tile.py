@@ -73,6 +73,62 @@ def test_tiles(K, H, Hkv, D, m, layout, weights):
         b.free()
 
 
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,panel,finish", [
+    (2048, 8192, 1024, 16, True, False),    # one round of workgroups: the panel up to 32 rows
+    (2048, 8192, 1024, 48, False, False),   # many weight rows: its passes cost more than the norm's launch and the tiles
+    (2048, 2048, 256, 64, True, False),
+    (1024, 4096, 1024, 40, True, False),    # no side a tenth ahead
+    (1024, 4096, 1024, 100, False, False),
+    (896, 896, 128, 400, True, False),
+    (896, 896, 128, 417, False, False),
+    (3072, 40, 24, 48, True, False),        # a few weight rows
+    (4096, 512, 128, 16, False, None),      # about the line between whole and divided
+    (8192, 512, 64, 12, False, True),       # few tiles over many features: divided
+    (8192, 512, 64, 130, False, True),
+    (3200, 8192, 512, 12, False, False),    # enough tiles
+    (16384, 256, 64, 20, False, True),
+])
+def test_route_of_a_chunk(K, N, NK, m, panel, finish, weights):
+    """Which launches a chunk takes is decided by what they are estimated to take; whichever it is, the outputs hold to the oracle.
+    (The longest rows without the norm: its f16 roundings differ from the oracle's in isolated elements, 60 in a million, more of
+    them in a row of 8192 than the bar allows for, whatever kernel multiplies them.)"""
+    announce("route of a chunk", K, N, NK, m, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + N + m)
+    x, g, ws, bs = _data(rng, K, N, NK, m)
+    norm = K <= 4096
+    scales, dev_s = None, []
+    if weights == "f16":
+        dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+        arg, full = [w.arg() for w in dev_w], ws
+    else:
+        quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
+        dev_s = [f.array(s) for _, s in quant]
+        scales = [s.arg() for s in dev_s]
+        flat = [orc.to_canonical(q) for q, _ in quant]
+        dev_w = [f.array(q if weights == "q8" else orc.pack_q4_0(q)) for q in flat]
+        arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev_w, (N, NK, NK))]
+        full = [orc.dequantize_blocks(q, s) for q, s in quant]
+    dx, dg, db = f.array(x), f.array(g), [f.array(b) for b in bs]
+    outs = [f.zeros((m, n)) for n in (N, NK, NK)]
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, gamma=dg.arg() if norm else None,
+                    biases=[b.arg() for b in db], layout=1, scales=scales)
+        f.synchronize()
+        assert f.profile_query("fused_qkv_rows32_kernel")[0] == int(panel) and f.profile_query("fused_qkv_gemm_kernel")[0] == int(not panel)
+        if finish is not None:
+            assert f.profile_query("gemm_finish_kernel")[0] == int(finish)
+    finally:
+        f.profile_enable(False)
+    for o, w, name in zip(outs, orc.fused_qkv(x, *full, gamma=g if norm else None, biases=bs, layout=0), "qkv"):
+        assert _close(o.download(), w, K), name
+    for b in dev_w + dev_s + [dx, dg] + db + outs:
+        b.free()
+
+
 @pytest.mark.parametrize("K,m,variant", [(3072, 300, 0), (3072, 300, 1), (3072, 300, 2), (2048, 1500, 0), (3104, 300, 0)])
 def test_f16_sums_are_added_in_parts(K, m, variant):
     """The f32 sums of F16 weights behind the output's rounding: out = sums - f16(exact), so that what is left shows them to 2^-24.
