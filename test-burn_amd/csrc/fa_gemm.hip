@@ -640,8 +640,8 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     fa_tile::TileShape shape;
     const bool tiles_whole = choose_tile(ctx, l, a, n_cus, shape);
-    // (What the tile kernels could take is not divided where the register-staged kernel is asked for by name: their sums and this
-    // kernel's are the same to the bit.)
+    // (What the tile kernels could take is not divided where the register-staged kernel is asked for by name: with F16 weights their
+    // sums and this kernel's are the same to the bit.)
     const Division d = divide(l, n_cus, tiles_whole);
     a.steps_per_split = d.steps_per_split, a.k_splits = d.k_splits;
     a.n_total = a.rows[0] + a.rows[1] + a.rows[2];

@@ -100,3 +100,26 @@ def infinite_last_block(K, N, m, weights, layout):
 def test_one_input_row_infinite_last_block(K, weights, layout):
     announce("one input row, infinite last block", K, weights, layout)
     infinite_last_block(K, 24, 1, weights, layout)
+
+
+@pytest.mark.parametrize("K", [96, 896, 4096])
+def test_one_input_row_subnormal_weights(K):
+    """F16 weights and inputs below the smallest normal number count with their values (exact in f32: products of two 11-bit numbers;
+    the bar is the f16 rounding of the result and K f32 additions)."""
+    announce("one input row, subnormal weights", K)
+    f = ctx()
+    rng = np.random.default_rng(K)
+    N = 40
+    w = (rng.integers(-1023, 1024, (N, K)) * 2.0 ** -24).astype(np.float16)  # subnormal
+    x = rng.uniform(-200, 200, (1, K)).astype(np.float16)
+    w[N // 2:] = rng.uniform(-1, 1, (N - N // 2, K)).astype(np.float16)  # (sums below the largest f16)
+    x[0, ::3] = (rng.integers(-1023, 1024, len(x[0, ::3])) * 2.0 ** -24).astype(np.float16)
+    for xv in (x, (rng.integers(-1023, 1024, (1, K)) * 2.0 ** -24).astype(np.float16)):
+        dx, dw, dout = f.array(xv), f.array(orc.to_canonical(w)), f.zeros((1, N))
+        f.matmul(dx.arg(), dw.arg(), dout.arg(), 1, N, K, transpose_b=False)
+        xd, wd = xv.astype(np.float64), w.astype(np.float64)
+        want, size = (xd @ wd.T)[0], (np.abs(xd) @ np.abs(wd).T)[0]
+        err = np.abs(dout.download()[0].astype(np.float64) - want)
+        assert np.all(err <= np.maximum(np.abs(want) * 2.0 ** -11, 2.0 ** -25) + K * 2.0 ** -24 * size)
+        for b in (dx, dw, dout):
+            b.free()

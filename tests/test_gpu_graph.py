@@ -218,9 +218,9 @@ def test_stream_timer_and_compute_units():
 
 
 def test_captured_prefill_chunks_with_the_fused_qkv_write_stage_replay():
-    """A prefill chunk of one layer as a captured graph - FusedQkv with KvPrepFused as its write stage (norm kernel, split-K
-    GEMM, finish kernel), then the chunk's attention over the cache (split-K prefill + merge) - replayed several times
-    with eager work and synchronisations between the replays; every replay must reproduce the eager result bit for bit."""
+    """A prefill chunk of one layer as a captured graph - FusedQkv with KvPrepFused as its write stage (one launch), then
+    the chunk's attention over the cache (partitions of the keys, merged inside the launch) - replayed several times with
+    eager work and synchronisations between the replays; every replay must reproduce the eager result bit for bit."""
     announce("graph replay, fused qkv + kv prep + prefill chunk")
     f = ctx()
     rng = np.random.default_rng(21)

@@ -368,6 +368,190 @@ def test_paged_batch_that_does_not_fit_at_once_waits_for_nobody(H, Hkv, D, B):
         g.close()
 
 
+class Batch:
+    """A fused decode step of a paged batch: inputs on the device, and per sequence the contiguous cache that it amounts to."""
+
+    def __init__(self, f, rng, H, Hkv, D, bs, lens, mode, bf16=False, bound=0, extra=1):
+        pack = orc.bf16_pack if bf16 else h16
+        self.f, self.H, self.Hkv, self.D, self.lens, self.mode, self.bf16 = f, H, Hkv, D, list(lens), mode, bf16
+        self.kc, self.vc = ([pack(rng.normal(size=(Hkv, n + extra, D))) for n in lens] for _ in range(2))
+        self.pg = Paged(f, rng, lens, Hkv, D, bs, extra_tokens=extra)
+        if bound:
+            widen(self.pg, bound)
+        for s in range(len(lens)):  # (rows past a sequence's length as well: they are overwritten as it grows)
+            orc.paged_scatter(self.pg.k_pool, self.pg.bt[s], Hkv, bs, D, 0, lens[s] + extra, self.kc[s])
+            orc.paged_scatter(self.pg.v_pool, self.pg.bt[s], Hkv, bs, D, 0, lens[s] + extra, self.vc[s])
+        self.pg.upload()
+        self.q, self.kn, self.vn = (pack(rng.normal(size=(len(lens), n * D))) for n in (H, Hkv, Hkv))
+        self.cos, self.sin = fa.rope_tables(1e6, D, max(lens) + extra)
+        self.dev = [f.array(x) for x in (self.q, self.kn, self.vn, self.cos, self.sin)]
+        self.dqr, self.dout = f.zeros((len(lens), H, D)), f.zeros((len(lens), H * D))
+        self.p = fa.KvPrepFusedParams.make(H, Hkv, D, len(lens), 0, 0, mode)
+        self.bound = bound or max(lens) + extra
+
+    def step(self):
+        kw = dict(dtype=fa.DTYPE_BF16) if self.bf16 else {}
+        dq, dkn, dvn, dcos, dsin = self.dev
+        self.f.decode_step_fused_paged(dq.arg(**kw), dkn.arg(**kw), dvn.arg(**kw), self.dqr.arg(**kw), self.pg.desc, dcos.arg(), dsin.arg(),
+                                       self.dout.arg(**kw), self.p, self.bound)
+
+    def value(self, x):
+        return orc.bf16_unpack(x) if self.bf16 else x
+
+    def out(self):
+        return self.value(self.dout.download()).reshape(len(self.lens), self.H, self.D)
+
+    def want(self, b, n):
+        """The oracle's step of sequence b at length n: appends to its contiguous cache, returns (q_rot, output)."""
+        def go():
+            cap = self.kc[b].shape[1]
+            qr = orc.kv_prep_fused(self.q[b:b + 1], self.kn[b:b + 1], self.vn[b:b + 1], self.kc[b], self.vc[b], self.cos, self.sin,
+                                   orc.make_params(self.H, self.Hkv, self.D, 1, n, cap, rope_mode=self.mode))
+            return qr[:, 0].copy(), self.value(orc.sdpa_decode(qr[:, 0].copy(), self.kc[b], self.vc[b], self.H, self.Hkv, self.D, cap, n + 1,
+                                                               n_threads=8)).reshape(self.H, self.D)
+        if self.bf16:
+            with orc.bf16_mode():
+                return go()
+        return go()
+
+    def caches_match(self, b):
+        n = self.kc[b].shape[1]
+        return all(np.array_equal(bits(orc.paged_gather(d.download(), self.pg.bt[b], self.Hkv, self.pg.bs, self.D, n)), bits(c))
+                   for d, c in ((self.pg.dk, self.kc[b]), (self.pg.dv, self.vc[b])))
+
+    def free(self):
+        self.pg.free()
+        for x in self.dev + [self.dqr, self.dout]:
+            x.free()
+
+
+@pytest.mark.parametrize("bf16,mode", [(False, fa.ROPE_NORMAL), (True, fa.ROPE_NEOX), (True, fa.ROPE_NORMAL)])
+@pytest.mark.parametrize("H,Hkv,D,lens", [
+    (16, 2, 128, [1, 15, 16, 17, 31, 0, 2047, 2048, 2049, 5000] * 2),  # one after the other
+    (24, 8, 128, [2000] * 7 + [2047]),                                # evenly
+    (14, 2, 64, [(i * 977) % 2100 for i in range(40)]),
+])
+def test_paged_batch_dealt_out_by_lengths_types_and_pairings(H, Hkv, D, lens, bf16, mode):
+    announce("paged batch dealt out by lengths", "bf16" if bf16 else "f16", mode, H, Hkv, D, len(lens))
+    f = ctx()
+    b = Batch(f, np.random.default_rng(H + D + mode), H, Hkv, D, 16, lens, mode, bf16)
+    try:
+        f.set_decode_variant(0, 2)
+        b.step()
+        f.synchronize()
+    finally:
+        f.set_decode_variant()
+    got, rot = b.out(), b.dqr.download()
+    for i, n in enumerate(lens):
+        qr, want = b.want(i, n)
+        assert np.array_equal(bits(rot[i]), bits(qr)) and b.caches_match(i), i
+        assert max_abs(got[i], want) <= (1.6e-2 if bf16 else TOL), i  # (bf16: the bar of test_gpu_bf16.py)
+    b.free()
+
+
+@pytest.mark.parametrize("merge", [0, 2])
+@pytest.mark.parametrize("H,Hkv,D,lens,bound,grow,steps", [
+    (16, 2, 128, [200, 90, 0, 155, 64, 12], 4096, 301, 12),      # other partitions at every replay
+    (24, 8, 128, [100 + 3 * i for i in range(8)], 2048, 157, 12),  # evenly, from a few keys each to the whole bound
+    (14, 2, 64, [127] * 20 + [900], 0, 1, 3),                    # a block edge, the last token at the bound
+])
+def test_paged_batch_in_a_graph_as_its_lengths_grow(H, Hkv, D, lens, bound, grow, steps, merge):
+    """One recorded step replayed while the lengths on the device grow: every replay against the oracle."""
+    announce("paged batch in a graph, growing lengths", H, Hkv, D, len(lens), bound, grow, merge)
+    f = ctx()
+    extra = grow * (steps - 1) + 1
+    b = Batch(f, np.random.default_rng(H + D), H, Hkv, D, 16, lens, fa.ROPE_NEOX, bound=bound, extra=extra)
+    assert max(lens) + extra <= b.bound
+    try:
+        f.set_decode_variant(0, merge)
+        b.step()  # eager: the workspace at its final size (and the rows that the first replay writes again)
+        f.synchronize()
+        f.start_capture()
+        b.step()
+        f.u32_add(b.pg.dlens, len(lens), grow)
+        graph = f.end_capture()
+    finally:
+        f.set_decode_variant()
+    for t in range(steps):
+        b.dout.upload(np.zeros(b.dout.shape, np.float16))
+        graph.launch()
+        f.synchronize()
+        got = b.out()
+        for i, n in enumerate(lens):
+            assert max_abs(got[i], b.want(i, n + t * grow)[1]) <= TOL, (t, i)
+    assert all(b.caches_match(i) for i in range(len(lens)))
+    graph.destroy()
+    b.free()
+
+
+def test_paged_batch_with_a_sequence_past_its_bound():
+    """A sequence whose position lies past the launch's bound is not appended, the others are served, and the next wait reports it:
+    the same whether the partitions are dealt out by the lengths or cut by the bound."""
+    announce("paged batch, a sequence past the bound")
+    g = fa.Foundry(0)
+    try:
+        H, Hkv, D, lens, bound = 16, 2, 128, [700, 30, 1024, 500, 1023, 999], 1024
+        outs, pools = [], []
+        for merge in (2, 1):
+            b = Batch(g, np.random.default_rng(4), H, Hkv, D, 16, lens, fa.ROPE_NEOX, bound=1040)
+            b.bound = bound
+            before = b.pg.dk.download()
+            g.set_decode_variant(0, merge)
+            b.step()
+            with pytest.raises(fa.FoundryError) as e:
+                g.synchronize()
+            assert e.value.variant == "InvalidOperation" and "neither appended nor attended" in str(e.value)
+            g.synchronize()  # nothing is left over
+            outs.append(b.out()), pools.append((b.pg.dk.download(), b.pg.dv.download()))
+            for i, n in enumerate(lens):
+                if n == bound:
+                    rows = [orc.paged_gather(x, b.pg.bt[i], Hkv, 16, D, n + 1) for x in (before, pools[-1][0])]
+                    assert np.array_equal(bits(rows[0]), bits(rows[1]))
+                else:
+                    want = b.want(i, n)[1]
+                    assert b.caches_match(i) and max_abs(outs[-1][i], want) <= TOL, i
+            b.free()
+        assert all(np.array_equal(bits(x), bits(y)) for x, y in zip(*pools))
+        assert max_abs(outs[0], outs[1]) <= TOL
+    finally:
+        g.close()
+
+
+def test_polled_paged_batch_gives_up_cleanly():
+    """The polled merge of partitions dealt out by the lengths, with a wait bound of zero: a workgroup that would have to wait gives
+    up, every kernel ends, the next wait reports it, and the context goes on - with the second launch, and polled again on request."""
+    announce("polled paged batch, zero wait bound")
+    g = fa.Foundry(0)
+    try:
+        lens = [700, 30, 1000, 500, 1023, 999, 4]
+        b = Batch(g, np.random.default_rng(5), 16, 2, 128, 16, lens, fa.ROPE_NEOX)
+        want = [b.want(i, n)[1] for i, n in enumerate(lens)]
+
+        def right():
+            got = b.out()  # waits for the stream
+            return all(max_abs(got[i], w) <= TOL for i, w in enumerate(want))
+
+        for _ in range(4):
+            g.set_decode_variant(0, 2)
+            g.set_decode_poll_spin_us(0)
+            b.step()
+            try:
+                assert right()  # nobody had to wait
+            except fa.FoundryError as e:
+                assert e.variant == "OperationFailed" and "waited longer" in str(e)
+                b.step()
+                assert right()
+            g.synchronize()
+        g.set_decode_poll_spin_us(5000)
+        g.set_decode_variant(0, 2)
+        for _ in range(3):
+            b.step()
+            assert right()
+        assert all(b.caches_match(i) for i in range(len(lens)))
+    finally:
+        g.close()
+
+
 @pytest.mark.usefixtures("prefill_variant")
 @pytest.mark.parametrize("H,Hkv,D,bs,prefix,M", [
     (6, 2, 128, 16, 333, 100),    # context ends inside a block and inside a key tile

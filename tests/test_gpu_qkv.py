@@ -59,7 +59,7 @@ def _close(got, want, K):
     (896, 896, 128, 1, True, True, 1),        # Qwen2.5-0.5B (biases)
     (2048, 2048, 256, 1, False, False, 1),    # no RMSNorm
     (3072, 3072, 1024, 5, True, False, 1),    # a few tokens
-    (896, 896, 128, 32, True, True, 1),       # a default prefill chunk: split-K GEMM, and two passes of 16 input rows
+    (896, 896, 128, 32, True, True, 1),       # a default prefill chunk, and the GEMM, and two passes of 16 input rows
     (896, 896, 128, 17, True, True, 0),
     (64, 40, 24, 3, True, True, 1),           # rows that do not fill tiles, tiles that straddle the three matrices
     (8192, 256, 64, 2, True, False, 1),       # long rows: more units than one request batch
@@ -342,7 +342,7 @@ def test_matmul_errors():
     (1024, 1024, 128, 1, True, True, 1),
     (3072, 3072, 1024, 1, True, False, 1),   # Llama-3.2-3B decode
     (896, 896, 128, 5, True, True, 1),
-    (896, 896, 128, 20, False, True, 0),     # row-major; the split-K GEMM, and two passes of input rows
+    (896, 896, 128, 20, False, True, 0),     # row-major; the chunk kernel, the GEMM, and two passes of input rows
     (64, 40, 24, 3, True, True, 1),
     (896, 896, 128, 32, True, True, 1),      # a default prefill chunk
     (3072, 3072, 1024, 200, True, False, 1), # Llama-3.2-3B, ragged input tiles
@@ -389,7 +389,7 @@ def test_fused_qkv_q8_equals_oracle(K, N, NK, m, norm, bias, layout):
     (1, 3072, 3072, True, False, True, 1.0, 1.0),   # o_proj
     (1, 256, 256, True, True, False, 0.5, 0.0),
     (7, 896, 896, True, True, True, 1.0, 0.5),
-    (40, 896, 896, False, True, True, 0.25, 0.75),   # the split-K GEMM, and passes of 16 rows
+    (40, 896, 896, False, True, True, 0.25, 0.75),   # the chunk kernel, the GEMM, and passes of 16 rows
     (256, 3072, 3072, True, False, True, 1.0, 1.0),  # o_proj of a 256-token prefill chunk
 ])
 def test_matmul_q8_equals_oracle(m, n, k, canonical, bias, resid, alpha, beta):
@@ -431,7 +431,7 @@ def test_matmul_q8_equals_oracle(m, n, k, canonical, bias, resid, alpha, beta):
     (3072, 3072, 1024, 1, True, False, 1),   # Llama-3.2-3B decode
     (896, 896, 128, 5, True, True, 0),       # row-major bytes
     (64, 40, 24, 3, True, True, 1),
-    (896, 896, 128, 20, False, True, 1),     # the split-K GEMM, and two passes of input rows
+    (896, 896, 128, 20, False, True, 1),     # the chunk kernel, the GEMM, and two passes of input rows
     (896, 896, 128, 32, True, True, 0),      # a default prefill chunk, row-major bytes
     (3072, 3072, 1024, 200, True, False, 1), # Llama-3.2-3B, ragged input tiles
     (1056, 200, 72, 130, True, True, 0),     # k_dim = 16.5 steps, weight rows that do not fill tiles
@@ -480,7 +480,7 @@ def test_fused_qkv_q4_0_equals_oracle(K, N, NK, m, norm, bias, layout):
     (1, 128, 128, False, False, False, 1.0, 0.0),
     (1, 3072, 3072, True, False, True, 1.0, 1.0),   # o_proj
     (7, 896, 896, True, True, True, 0.5, 0.5),
-    (40, 896, 896, False, True, True, 0.25, 0.75),   # the split-K GEMM
+    (40, 896, 896, False, True, True, 0.25, 0.75),   # the chunk kernel, and the GEMM
     (256, 3072, 3072, True, False, True, 1.0, 1.0),  # o_proj of a 256-token prefill chunk
 ])
 def test_matmul_q4_0_equals_oracle(m, n, k, canonical, bias, resid, alpha, beta):
@@ -507,14 +507,18 @@ def test_matmul_q4_0_equals_oracle(m, n, k, canonical, bias, resid, alpha, beta)
         z.free()
 
 
-def test_gemm_path_replays_in_a_graph_with_new_inputs():
-    """FusedQkv (split-K GEMM with the norm kernel in front and the finish kernel behind) followed by the o_proj MatMul
-    (GEMM with residual), captured once and replayed with other inputs in the same buffers: every replay equals the
-    eager result bit for bit (the partial tiles are added in split order) and the oracle to the bar above. The workspace
-    for the normalised input and the partial tiles is sized by the eager call before the capture."""
-    announce("gemm graph replay")
+@pytest.mark.parametrize("K,N,NK,m,launches", [
+    (512, 512, 128, 40, dict(fused_qkv_rows32_kernel=1, matmul_rows32_kernel=1)),  # one launch each
+    (3104, 3104, 64, 40, dict(rmsnorm_rows_kernel=1, fused_qkv_gemm_kernel=1, matmul_gemm_kernel=1, gemm_finish_kernel=2)),
+    (512, 512, 128, 430, dict(rmsnorm_rows_kernel=1, fused_qkv_gemm_kernel=1, matmul_gemm_kernel=1)),  # tiles over all features
+])
+def test_gemm_path_replays_in_a_graph_with_new_inputs(K, N, NK, m, launches):
+    """FusedQkv followed by the o_proj MatMul with residual - as one launch each, as GEMMs whose features are divided (the norm kernel
+    in front, the finish kernel behind) and as GEMMs over all features - captured once and replayed with other inputs in the same
+    buffers: every replay equals the eager result bit for bit (the partial tiles are added in split order) and the oracle to the
+    bar above. The workspace for the normalised input and the partial tiles is sized by the eager call before the capture."""
+    announce("gemm graph replay", K, N, NK, m)
     f = ctx()
-    K, N, NK, m = 512, 512, 128, 40
     rng = np.random.default_rng(99)
     _, g, ws, bs = _data(rng, K, N, NK, m)
     wo = rng.uniform(-0.1, 0.1, (K, N)).astype(np.float16)
@@ -531,8 +535,16 @@ def test_gemm_path_replays_in_a_graph_with_new_inputs():
 
     xs = [rng.uniform(-1, 1, (m, K)).astype(np.float16) for _ in range(3)]
     dx.upload(xs[0])
-    enqueue()  # eager: sizes the workspace
-    f.synchronize()
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        enqueue()  # eager: sizes the workspace
+        f.synchronize()
+        for kernel in ("fused_qkv_rows32_kernel", "matmul_rows32_kernel", "rmsnorm_rows_kernel", "fused_qkv_gemm_kernel",
+                       "matmul_gemm_kernel", "gemm_finish_kernel"):
+            assert f.profile_query(kernel)[0] == launches.get(kernel, 0), kernel
+    finally:
+        f.profile_enable(False)
     f.start_capture()
     enqueue()
     graph = f.end_capture()
@@ -560,7 +572,7 @@ def test_gemm_path_replays_in_a_graph_with_new_inputs():
 
 
 def test_gemm_workspace_must_be_reserved_before_a_capture():
-    """The GEMM form keeps the normalised input (and split-K partial tiles) in the context's workspace; inside a capture
+    """The GEMM form keeps the normalised input (and, its features divided, partial tiles) in the context's workspace; inside a capture
     the workspace cannot grow, so a call that needs more than is reserved fails with a message naming
     fa_ctx_reserve_workspace; after one eager call of the same shape (or that reservation) the capture works."""
     announce("gemm workspace under capture")

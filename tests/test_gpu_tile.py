@@ -129,6 +129,63 @@ def test_route_of_a_chunk(K, N, NK, m, panel, finish, weights):
         b.free()
 
 
+def _quantised(f, rng, K, N, m, weights):
+    x = rng.uniform(-1, 1, (m, K)).astype(np.float16)
+    q, s = (orc.quantize_q8_0 if weights == "q8" else orc.quantize_q4_0)(rng.uniform(-0.1, 0.1, (N, K)).astype(np.float16))
+    flat = orc.to_canonical(q)
+    dev_w = f.array(flat if weights == "q8" else orc.pack_q4_0(flat))
+    return x, orc.dequantize_blocks(q, s), s, dev_w, dev_w.arg() if weights == "q8" else dev_w.arg((N, K), dtype=fa.DTYPE_Q4_0)
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,m", [
+    (4096, 70), (4160, 70),    # the last row whose scales fit every tile's part of LDS, and the first past it: 64 x 64 tiles
+    (8192, 70), (8256, 70),    # ... of eight small stages up to here
+    (16384, 130),              # the longest row
+    (16448, 70),               # past it: operand tiles through registers
+])
+def test_long_quantised_rows(K, m, weights):
+    """Each kernel that takes such rows (operand tiles through registers, 128 x 128 tiles where the scales fit, 64 x 64, by choice)."""
+    announce("long quantised rows", K, m, weights)
+    f = ctx()
+    N = 200
+    x, full, s, dev_w, arg = _quantised(f, np.random.default_rng(K + m), K, N, m, weights)
+    dx, ds, dout = f.array(x), f.array(s), f.zeros((m, N))
+    got = []
+    try:
+        for variant in (0, 1, 2, 3):
+            f.set_gemm_variant(variant)
+            f.matmul(dx.arg(), arg, dout.arg(), m, N, K, transpose_b=False, b_scales=ds.arg())
+            got.append(dout.download())
+    finally:
+        f.set_gemm_variant()
+    want = orc.matmul_gemv(x, full, None, None, 0, 32, 1.0, 0.0).astype(np.float64)
+    for g in got:
+        assert np.all(np.abs(g - want) <= 2 * np.maximum(np.abs(want), 2.0 ** -10) * 2.0 ** -10 + 1e-4)
+    for b in (dx, ds, dev_w, dout):
+        b.free()
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,m", [(128, 1), (2048, 1), (64, 5), (896, 5), (896, 20), (3072, 40), (64, 500), (896, 500)])
+def test_scales_at_any_half(K, m, weights):
+    """Scales that begin at an odd f16: the kernels that read them in pairs leave them to others or read them one by one."""
+    announce("scales at any half", K, m, weights)
+    f = ctx()
+    N = 72
+    x, full, s, dev_w, arg = _quantised(f, np.random.default_rng(K + m), K, N, m, weights)
+    dx, dout = f.array(x), f.zeros((m, N))
+    moved = np.concatenate([np.full(1, 99.0, np.float16), s.reshape(-1), np.full(1, 99.0, np.float16)])
+    ds = f.array(moved)
+    f.matmul(dx.arg(), arg, dout.arg(), m, N, K, transpose_b=False, b_scales=ds.arg(s.shape, offset=2))
+    want = x.astype(np.float64) @ full.astype(np.float64).T
+    # two f16 units of the result and, from 12 rows on, the rounding of f16(weight * scale)
+    bar = 2.0 ** -9 * np.abs(want) + 2.0 ** -11 * (np.abs(x.astype(np.float64)) @ np.abs(full.astype(np.float64)).T) + 1e-4
+    assert np.all(np.abs(dout.download() - want) <= bar)
+    for b in (dx, ds, dev_w, dout):
+        b.free()
+
+
 @pytest.mark.parametrize("K,m,variant", [(3072, 300, 0), (3072, 300, 1), (3072, 300, 2), (2048, 1500, 0), (3104, 300, 0)])
 def test_f16_sums_are_added_in_parts(K, m, variant):
     """The f32 sums of F16 weights behind the output's rounding: out = sums - f16(exact), so that what is left shows them to 2^-24.
