@@ -3,6 +3,7 @@
 #pragma once
 #include "fa_internal.h"
 #include "fa_qkv_rope.h"
+#include "fa_quant.h"
 
 namespace fa_gemm {
 
@@ -16,7 +17,7 @@ struct GemmDev {
     const __half *bias[3];
     __half *out[3];
     uint32_t rows[3];       // weight rows per matrix
-    uint32_t tiles[3];      // 128-row tiles per matrix
+    uint32_t tiles[3];      // tiles per matrix, of the width that the launch takes
     const __half *x;        // [m, k_dim] (already normalised when the op has a gamma)
     const __half *residual; // nullable, [m, rows[0]]
     uint32_t k_dim, m, m_tiles, n_tiles, canonical, vec_store;
@@ -79,36 +80,5 @@ __device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint
 
 typedef unsigned int u4v_t __attribute__((ext_vector_type(4)));
 typedef _Float16 h2v_t __attribute__((ext_vector_type(2)));
-
-// 16 int8 weights -> two pieces of 8 f16, exactly: s + 128 is a byte u, the f16 with bits 0x6400 | u is 1024 + u, and
-// 1024 + u - 1152 = s (two byte permutes and one packed subtraction per four weights).
-__device__ __forceinline__ void q8_to_f16(const u4v_t raw, h8_t &p0, h8_t &p1) {
-    const h2v_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-#pragma unroll
-    for (int hw = 0; hw < 4; ++hw) {
-        const uint32_t u = raw[hw] ^ 0x80808080u;
-        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
-        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
-        h8_t &dst = hw < 2 ? p0 : p1;
-        const int o = (hw & 1) * 4;
-        dst[o + 0] = lo[0], dst[o + 1] = lo[1], dst[o + 2] = hi[0], dst[o + 3] = hi[1];
-    }
-}
-
-// 8 Q4_0 weights (one word: element 2i in the low nibble of byte i, value = nibble - 8) -> one piece of 8 f16, exactly:
-// the nibbles become two words of four bytes 0..15 in element order, then 0x6400 | u is 1024 + u and 1024 + u - 1032.
-__device__ __forceinline__ h8_t q4_to_f16(uint32_t w) {
-    const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
-    const uint32_t b[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
-    const h2v_t bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-    h8_t r;
-#pragma unroll
-    for (int hw = 0; hw < 2; ++hw) {
-        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x05010400u)) - bias;
-        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, b[hw], 0x07030602u)) - bias;
-        r[4 * hw + 0] = lo[0], r[4 * hw + 1] = lo[1], r[4 * hw + 2] = hi[0], r[4 * hw + 3] = hi[1];
-    }
-    return r;
-}
 
 }  // namespace fa_gemm

@@ -323,13 +323,11 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
             if constexpr (Q4) {
                 const h8_t sc = {wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i]};
 #pragma unroll
-                for (int q = 0; q < 4; ++q) *reinterpret_cast<h8_t *>(base + w_lds[i] + q * W_STRIDE) = q4_to_f16(wr[i][q]) * sc;
+                for (int q = 0; q < 4; ++q) *reinterpret_cast<h8_t *>(base + w_lds[i] + q * W_STRIDE) = fa_quant::q4_to_f16(wr[i][q]) * sc;
             } else if constexpr (Q8) {
                 const h8_t sc = {wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i], wsc[i]};
-                h8_t p0, p1;
-                q8_to_f16(wr[i], p0, p1);
-                *reinterpret_cast<h8_t *>(base + w_lds[i]) = p0 * sc;
-                *reinterpret_cast<h8_t *>(base + w_lds[i] + W_STRIDE) = p1 * sc;
+                *reinterpret_cast<h8_t *>(base + w_lds[i]) = fa_quant::q8_to_f16(wr[i][0], wr[i][1]) * sc;
+                *reinterpret_cast<h8_t *>(base + w_lds[i] + W_STRIDE) = fa_quant::q8_to_f16(wr[i][2], wr[i][3]) * sc;
             } else {
                 *reinterpret_cast<h8_t *>(base + w_lds[i]) = wr[i];
             }

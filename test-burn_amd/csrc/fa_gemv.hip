@@ -20,6 +20,7 @@
 // sums, one rounding at the end.
 #include "fa_internal.h"
 #include "fa_norm.h"
+#include "fa_quant.h"
 #include <type_traits>
 
 namespace {
@@ -44,20 +45,6 @@ struct GemvDev {
     uint32_t n_waves;
     float eps, inv_k, alpha, beta;
 };
-
-// Eight int8 weights (two words) as f16, exactly: s + 128 is a byte u, the f16 0x6400 | u is 1024 + u, minus 1152.
-__device__ __forceinline__ h8_t bytes_to_f16(uint32_t a, uint32_t b, uint32_t flip, _Float16 off) {
-    const h2_t bias = {off, off};
-    h8_t r;
-    const uint32_t w[2] = {a ^ flip, b ^ flip};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const h2_t lo = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x05010400u)) - bias;
-        const h2_t hi = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x07030602u)) - bias;
-        r[4 * i] = lo[0], r[4 * i + 1] = lo[1], r[4 * i + 2] = hi[0], r[4 * i + 3] = hi[1];
-    }
-    return r;
-}
 
 __device__ __forceinline__ float dot8(h8_t a, h8_t b, float acc) {
 #pragma unroll
@@ -190,16 +177,12 @@ __global__ void __launch_bounds__(64 * GV_MAX_NW, 2) gemv_row_kernel(GemvDev a_b
             } else {
                 float s;
                 if constexpr (WB == 8) {
-                    s = dot8(bytes_to_f16(w[0], w[1], 0x80808080u, (_Float16)1152.0f), xv[u][0], 0.0f);
-                    s = dot8(bytes_to_f16(w[2], w[3], 0x80808080u, (_Float16)1152.0f), xv[u][1], s);
-                } else {  // nibbles: element 2i of a word in the low half of byte i
+                    s = dot8(fa_quant::q8_to_f16<true>(w[0], w[1]), xv[u][0], 0.0f);
+                    s = dot8(fa_quant::q8_to_f16<true>(w[2], w[3]), xv[u][1], s);
+                } else {
                     s = 0.0f;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint32_t even = w[q] & 0x0f0f0f0fu, odd = (w[q] >> 4) & 0x0f0f0f0fu;
-                        s = dot8(bytes_to_f16(__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u), 0u,
-                                              (_Float16)1032.0f), xv[u][q], s);
-                    }
+                    for (int q = 0; q < 4; ++q) s = dot8(fa_quant::q4_to_f16(w[q]), xv[u][q], s);
                 }
                 acc[t] += s * (kb_ok[u] ? (float)sc[t][u] : 0.0f);
             }

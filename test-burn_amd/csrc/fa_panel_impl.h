@@ -3,6 +3,7 @@
 #include <atomic>
 
 #include "fa_panel.h"
+#include "fa_quant.h"
 
 namespace fa_panel {
 
@@ -33,34 +34,18 @@ struct Weights<16> {
     static __device__ __forceinline__ h8_t plain(raw_t w) { return w; }
     static __device__ __forceinline__ raw_t part(raw_t w, int) { return w; }
 };
-// s + 128 is a byte u, the f16 with bits 0x6400 | u is 1024 + u, minus 1152: exact
-__device__ __forceinline__ h8_t bytes_f16(uint32_t a, uint32_t b, _Float16 off) {
-    const h2_t bias = {off, off};
-    h8_t r;
-    const uint32_t w[2] = {a, b};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const h2_t lo = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x05010400u)) - bias;
-        const h2_t hi = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, w[i], 0x07030602u)) - bias;
-        r[4 * i] = lo[0], r[4 * i + 1] = lo[1], r[4 * i + 2] = hi[0], r[4 * i + 3] = hi[1];
-    }
-    return r;
-}
 template <>
 struct Weights<8> {
     typedef u2v_t raw_t;
     static __device__ __forceinline__ raw_t part(u4v_t w, int i) { return raw_t{w[2 * i], w[2 * i + 1]}; }  // 8 weights of 16
-    static __device__ __forceinline__ h8_t plain(raw_t w) { return bytes_f16(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u, (_Float16)1152.0f); }
+    static __device__ __forceinline__ h8_t plain(raw_t w) { return fa_quant::q8_to_f16<true>(w[0], w[1]); }
     static __device__ __forceinline__ h8_t f16(raw_t w, _Float16 s) { return plain(w) * h8_t{s, s, s, s, s, s, s, s}; }
 };
 template <>
-struct Weights<4> {  // element 2i in the low nibble of byte i, value = nibble - 8
+struct Weights<4> {
     typedef uint32_t raw_t;
     static __device__ __forceinline__ raw_t part(u4v_t w, int i) { return w[i]; }  // 8 weights of 32
-    static __device__ __forceinline__ h8_t plain(raw_t w) {
-        const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
-        return bytes_f16(__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u), (_Float16)1032.0f);
-    }
+    static __device__ __forceinline__ h8_t plain(raw_t w) { return fa_quant::q4_to_f16(w); }
     static __device__ __forceinline__ h8_t f16(raw_t w, _Float16 s) { return plain(w) * h8_t{s, s, s, s, s, s, s, s}; }
 };
 

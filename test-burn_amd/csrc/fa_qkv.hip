@@ -26,6 +26,7 @@
 #include "fa_norm.h"
 #include "fa_panel.h"
 #include "fa_qkv_rope.h"
+#include "fa_quant.h"
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -341,30 +342,9 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
             if constexpr (Q8) {
                 // 8 int8 weights -> f16 (exact); one MFMA covers exactly one 32-weight block, whose sums are scaled
                 // per row (lane (n, c) of the result holds rows 4c..4c+3) and then accumulated
-                // int8 -> f16 without a conversion per element: s + 128 is a byte u, the f16 with bits 0x6400 | u is
-                // 1024 + u, and 1024 + u - 1152 = s exactly (two byte permutes and one packed subtraction per four)
-                // Q4_0 (policy_q4_0.metal:70-86: value = nibble - 8): the eight nibbles first become two words of four
-                // bytes 0..15 in element order (two masks, a shift, two byte permutes), then the same route with
-                // 1024 + u - 1032
-                u2v_t raw;
-                if constexpr (Q4) {
-                    const uint32_t even = buf[i] & 0x0f0f0f0fu, odd = (buf[i] >> 4) & 0x0f0f0f0fu;
-                    raw[0] = __builtin_amdgcn_perm(odd, even, 0x05010400u);
-                    raw[1] = __builtin_amdgcn_perm(odd, even, 0x07030602u);
-                } else {
-                    raw = buf[i];
-                }
-                typedef _Float16 h2v_t __attribute__((ext_vector_type(2)));
                 h8_t wv;
-#pragma unroll
-                for (int hw = 0; hw < 2; ++hw) {
-                    const uint32_t u = Q4 ? raw[hw] : raw[hw] ^ 0x80808080u;
-                    const _Float16 off = Q4 ? (_Float16)1032.0f : (_Float16)1152.0f;
-                    const h2v_t bias = {off, off};
-                    const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
-                    const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
-                    wv[4 * hw + 0] = lo[0], wv[4 * hw + 1] = lo[1], wv[4 * hw + 2] = hi[0], wv[4 * hw + 3] = hi[1];
-                }
+                if constexpr (Q4) wv = fa_quant::q4_to_f16(buf[i]);
+                else wv = fa_quant::q8_to_f16(buf[i][0], buf[i][1]);
                 const f4v_t z = {0.0f, 0.0f, 0.0f, 0.0f};
                 const f4v_t blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xb, z, 0, 0, 0);
                 typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));

@@ -11,8 +11,9 @@
 //     barrier they leave the matrix cores idle. They are spread between the products (256 x 160: 98 -> 66 us at 2048 rows,
 //     5120 x 3072, where the split-K form took 74.7).
 //   * large launches read less per product with larger tiles but leave CUs idle where the tiles do not fill a round of
-//     workgroups: five shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 is there for the
-//     5120 x 2048 products of a 2048-row prompt - one tile on each of 256 CUs - and may hold rows of two matrices (JOINED).
+//     workgroups: five shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 (F16) fills a round where
+//     256 x 128 leaves a fifth of the chip to a second one - 8.4 to 10.5 million outputs, such as 2048 rows x 5120, and again at
+//     twice that - and may hold rows of two matrices (JOINED).
 //   * block-quantised weights stay as they are up to the registers, where a wave turns its operands to f16 right in front of the
 //     product (f16(weight * scale), as the reference's tile loader: see fa_gemm.hip). That is 14 vector instructions per 8
 //     weights, and with one wave per SIMD they add to the chain; so that no two waves convert the same weights, the waves of a
@@ -92,20 +93,6 @@ __device__ __forceinline__ void meet() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-// 8 int8 weights (two words) -> f16, exactly (see q8_to_f16)
-__device__ __forceinline__ h8_t q8x8_to_f16(uint32_t a, uint32_t b) {
-    const h2v_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    h8_t r;
-#pragma unroll
-    for (int hw = 0; hw < 2; ++hw) {
-        const uint32_t u = (hw ? b : a) ^ 0x80808080u;
-        const h2v_t lo = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010400u)) - bias;
-        const h2v_t hi = __builtin_bit_cast(h2v_t, __builtin_amdgcn_perm(0x64646464u, u, 0x07030602u)) - bias;
-        r[4 * hw + 0] = lo[0], r[4 * hw + 1] = lo[1], r[4 * hw + 2] = hi[0], r[4 * hw + 3] = hi[1];
-    }
-    return r;
-}
-
 template <class S, int MIN_WAVES>
 __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -290,8 +277,8 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             else if constexpr (S::KG == 2) s = kg ? s2[1] : s2[0];
             else s = kg >= 2 ? s2[1] : s2[0];
             const h8_t sc = {s, s, s, s, s, s, s, s};
-            if constexpr (S::WB == 8) return q8x8_to_f16(o.w[i][q].x, o.w[i][q].y) * sc;
-            else return q4_to_f16(h ? o.w[i][q].y : o.w[i][q].x) * sc;
+            if constexpr (S::WB == 8) return fa_quant::q8_to_f16(o.w[i][q].x, o.w[i][q].y) * sc;
+            else return fa_quant::q4_to_f16(h ? o.w[i][q].y : o.w[i][q].x) * sc;
         }
     };
 
