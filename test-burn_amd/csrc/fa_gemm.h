@@ -22,7 +22,7 @@ struct GemmDev {
     const __half *residual; // nullable, [m, rows[0]]
     uint32_t k_dim, m, m_tiles, n_tiles, canonical, vec_store;
     float alpha, beta;
-    // split-K: the feature steps are divided over k_splits workgroups per output tile, which store f32 partial tiles
+    // the feature steps are divided over k_splits workgroups per output tile, which store f32 partial tiles
     // [split][m][n_total]; gemm_finish_kernel adds them up in split order and applies the write stage
     uint32_t k_splits, steps_per_split, n_total;
     float *partial;

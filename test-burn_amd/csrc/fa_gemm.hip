@@ -4,7 +4,8 @@
 //
 // With more than a few input rows the step is no longer a weight stream: out[m, n] = x[m, :] . W[n, :] is
 // 2 * m * n * k flops on m * k + n * k operands, so it runs as a GEMM. Almost every launch goes to the tile kernels of fa_tile.h
-// (choose_tile below); this file holds the normalisation in front of them and the kernel that takes every other shape:
+// (choose_tile below); this file holds the normalisation in front of them and the kernel that takes every other shape, and few tiles
+// over many features:
 //   * a workgroup (4 waves) owns a 128 (weight rows) x 128 (input rows) output tile; a wave owns 64 x 64 of it as
 //     2 x 2 v_mfma_f32_32x32x16_f16 tiles (64 accumulator registers);
 //   * both operands move through registers and LDS in steps of 64 features, two stages, one barrier per step;
@@ -18,7 +19,7 @@
 //     arithmetic on those f16 values and stores to q_rot and the cache rows (rope_store_piece).
 // RMSNorm: a small kernel in front writes the normalised input, rounded to f16 as qkv_project.metal:66-67 does, into
 // the context's workspace; the GEMM reads that. Launches with few output tiles divide a tile's feature steps over
-// several workgroups (split-K: f32 partial tiles in the workspace, added in split order by gemm_finish_kernel).
+// several workgroups (f32 partial tiles in the workspace, added in split order by gemm_finish_kernel).
 #include "fa_gemm.h"
 #include "fa_norm.h"
 #include "fa_tile.h"
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(256) rmsnorm_long_rows_kernel(const __half *x,
 }
 
 // The end of an output tile, shared by the GEMM kernels: accumulators -> LDS (f32, [input row][weight row]) -> either
-// the write stage and token-major f16 stores, or (split-K) the f32 partial tile.
+// the write stage and token-major f16 stores, or (features divided) the f32 partial tile.
 __device__ __forceinline__ void gemm_epilogue(const GemmDev &a, unsigned char *smem, const f16v_t (&acc)[2][2], int tid,
                                               int lane, int wn, int wm, int mat, uint32_t N, uint32_t n0, uint32_t m0,
                                               uint32_t split) {
@@ -393,7 +394,7 @@ __global__ void __launch_bounds__(GM_NT, 2) qkv_gemm_kernel(GemmDev a) {
     gemm_epilogue(a, smem, acc, tid, lane, wn, wm, mat, N, n0, m0, split);
 }
 
-// Adds the split-K partial tiles in split order and applies the write stage: one thread per 8 output columns.
+// Adds the partial tiles in split order and applies the write stage: one thread per 8 output columns.
 __global__ void __launch_bounds__(256) gemm_finish_kernel(GemmDev a) {
     const uint32_t groups = (a.n_total + 7) / 8;
     const uint32_t id = blockIdx.x * 256 + threadIdx.x;

@@ -500,7 +500,7 @@ fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_
     const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     // A chunk of a few dozen input rows (the reference's default prefill chunk is 32) is still a weight stream: one launch where
-    // the GEMM route takes three.
+    // the GEMM route takes two or three.
     if (fa_qkv_rows32_takes(ctx, l)) return launch_panel(ctx, l, nullptr);
     if (!weight_stream_only && gemm_ok && l.m >= (ctx->gemm_min_m ? ctx->gemm_min_m : GEMM_MIN_M_DEFAULT)) return fa_launch_fused_qkv_gemm(ctx, l);
     // Workgroups: a multiple of the CU count, enough of them that a workgroup's rows fit one 16-row tile where the

@@ -209,6 +209,46 @@ def test_launches_of_a_divided_gemm(K, norm, mode):
         b.free()
 
 
+@pytest.mark.parametrize("K,N,NK,m,finish", [
+    (8192, 256, 64, 40, 1),
+    (32768, 128, 64, 800, 0),  # the normalised input and the parts would take more than a new context's workspace
+])
+def test_gemm_recorded_as_the_first_call(K, N, NK, m, finish):
+    """A GEMM that divides its features by choice does so only within the workspace that a new context has: recorded as the very first
+    call it runs, and gives the bits of an eager call."""
+    announce("gemm recorded as the first call", K, N, NK, m)
+    f = fa.Foundry(0)
+    try:
+        x, g, ws, _ = _data(np.random.default_rng(K), K, N, NK, m)
+        dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+        dx, dg = f.array(x), f.array(g)
+        outs = [f.zeros((m, n)) for n in (N, NK, NK)]
+
+        def call():
+            f.fused_qkv(dx.arg(), *[w.arg() for w in dev_w], *[o.arg() for o in outs], K, N, NK, m, gamma=dg.arg(), layout=1)
+
+        f.start_capture()
+        call()
+        graph = f.end_capture()
+        replays = []
+        for _ in range(3):
+            graph.launch()
+            f.synchronize()
+            replays.append([bits(o.download()) for o in outs])
+        f.profile_enable(True)
+        call()
+        f.synchronize()
+        assert f.profile_query("fused_qkv_gemm_kernel")[0] == 1 and f.profile_query("gemm_finish_kernel")[0] == finish
+        f.profile_enable(False)
+        eager = [o.download() for o in outs]
+        assert all(np.isfinite(o).all() and o.any() for o in eager)
+        for r in replays:
+            assert all(np.array_equal(a, bits(b)) for a, b in zip(r, eager))
+        graph.destroy()
+    finally:
+        f.close()
+
+
 def test_fused_op_errors():
     announce("fused qkv + kv prep errors")
     f = ctx()
