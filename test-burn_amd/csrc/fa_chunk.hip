@@ -34,6 +34,8 @@ namespace {
 
 using fa_lds_dma::buffer_to_lds_b128_nt;
 using fa_lds_dma::make_rsrc_words;
+using fa_lds_dma::rows16_lane_src;
+using fa_lds_dma::rows16_operand;
 using fa_lds_dma::rsrc_words;
 
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -129,7 +131,7 @@ __global__ void __launch_bounds__(NTW, 1) flash_chunk_kernel(ChunkDev a_by_value
     constexpr int DSTEPS = D / 16;  // MFMA k-steps over head_dim for S^T
     constexpr int DBLKS = D / 32;   // 32-row blocks of O^T
     constexpr int ROWB = D * 2, CHK = D / 8;
-    constexpr int RB_BYTES = CHK * 256;  // one 16-row block of K in LDS: [16-byte chunk][row]
+    constexpr int RB_BYTES = CHK * 256;  // one 16-row block of K in LDS: [64-byte column][row][64 B] (rows16_lane_src)
     constexpr int RG_BYTES = 4 * ROWB;   // one 4-row group of V in LDS: [64-byte column block][row][64 B]
     constexpr int K_DMA = CHK / 4, V_DMA = 16 * ROWB / 1024;  // instructions per wave and 16-row block
     constexpr int BLK_DMA = K_DMA + V_DMA;
@@ -196,7 +198,7 @@ __global__ void __launch_bounds__(NTW, 1) flash_chunk_kernel(ChunkDev a_by_value
     const int rounds = (part_blks + RBLKS - 1) / RBLKS;
 
     // ---- The producer waves. Memory -> LDS (fa_lds_dma.h) in the layouts of the prefill kernel: lane l of a K instruction
-    // takes chunk l / 16 of row l % 16; of a V instruction, piece l % 4 of column block (l / 16) % (ROWB / 64) of row
+    // takes a 16-byte piece of row l / 4; of a V instruction, piece l % 4 of column block (l / 16) % (ROWB / 64) of row
     // (l / (16 ROWB / 64)) * 4 + (l % 16) / 4. Producer p moves K and V of block p of every round. Rows at and past the
     // partition's end come out of the descriptor's bound check as zeros (no memory access), so every block of a round is
     // written whether it holds keys or not.
@@ -234,7 +236,7 @@ __global__ void __launch_bounds__(NTW, 1) flash_chunk_kernel(ChunkDev a_by_value
         FC_TR(13);
         constexpr int CBR = ROWB / 64;
         const int blk = wave8 - 8;
-        const int k_lane_src = (lane & 15) * ROWB + (lane >> 4) * 16;
+        const int k_lane_src = rows16_lane_src(lane, ROWB);
         const int v_lane_src = ((lane / (16 * CBR)) * 4 + ((lane & 15) >> 2)) * ROWB + ((lane >> 4) % CBR) * 64 + (lane & 3) * 16;
         rsrc_words krs = make_rsrc_words(nullptr, 0), vrs = krs;
         if (!PAGED) {
@@ -261,7 +263,7 @@ __global__ void __launch_bounds__(NTW, 1) flash_chunk_kernel(ChunkDev a_by_value
                 vr = make_rsrc_words(reinterpret_cast<const unsigned char *>(a.v) + base, valid * ROWB);
                 so = 0;
             }
-            // K: chunk quads, 64 bytes apart in a row, 1 KB apart in LDS; V: 1 KB of rows after 1 KB of rows
+            // K: 64-byte columns, 64 bytes apart in a row, 1 KB apart in LDS; V: 1 KB of rows after 1 KB of rows
             buffer_to_lds_b128_nt<K_DMA, 64, 1024>(kr, k_lds_addr + (uint32_t)slot * RB_BYTES, k_lane_src, so);
             buffer_to_lds_b128_nt<V_DMA, 1024, 1024>(vr, v_lds_addr + (uint32_t)slot * (4 * RG_BYTES), v_lane_src, so);
         };
@@ -352,19 +354,19 @@ __global__ void __launch_bounds__(NTW, 1) flash_chunk_kernel(ChunkDev a_by_value
     const uint32_t q_abs = q_row_c + a.query_offset;  // last visible key of this lane's row when causal
     // first key index that some row of this wave cannot see
     const uint32_t wave_min_limit = causal ? (min(rb * 32u, q_len - 1) + a.query_offset) : 0xffffffffu;
-    const int k_lane = (n >> 4) * RB_BYTES + hi * 256 + (n & 15) * 16;
+    const int k_lane = (n >> 4) * RB_BYTES + rows16_operand(n, hi);
     const int v_lane = hi * RG_BYTES + ((lane & 15) >> 2) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
 
     // 32 keys - the 16-row blocks tb, tb + 1 of the LDS areas, keys key0 .. - against this wave's 32 columns
     auto attend_tile = [&](int tb, uint32_t key0) __attribute__((always_inline)) {
-        const unsigned char *k_lds = k_area + tb * RB_BYTES + k_lane, *v_lds = v_area + tb * (4 * RG_BYTES) + v_lane;
+        const unsigned char *k_lds = k_area + tb * RB_BYTES, *v_lds = v_area + tb * (4 * RG_BYTES) + v_lane;
         f16_t sacc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
 #pragma unroll
         for (int s = 0; s < DSTEPS; ++s) {
             U4H8 kk;
-            kk.u = *reinterpret_cast<const uint4 *>(k_lds + s * 512);
+            kk.u = *reinterpret_cast<const uint4 *>(k_lds + (s & 1 ? k_lane ^ 32 : k_lane) + s / 2 * 1024);
             sacc = BF16 ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk.b, qreg[s].b, sacc, 0, 0, 0)
                         : __builtin_amdgcn_mfma_f32_32x32x16_f16(kk.h, qreg[s].h, sacc, 0, 0, 0);
         }

@@ -81,4 +81,14 @@ FA_LDS_DMA_DEFINE(buffer_to_lds_b128, "")
 FA_LDS_DMA_DEFINE(buffer_to_lds_b128_nt, " nt")
 #undef FA_LDS_DMA_DEFINE
 
+// Layout of 16 rows of K (or of query rows) in LDS, for the operand reads of a 32 x 32 x 16 matrix instruction (lane = row, 16
+// bytes of it): a load fills 1 KiB with a 64-byte column of the 16 rows, [row][slot of 16 bytes], and the next loads with the next
+// columns. Neighbouring lanes fetch neighbouring memory: the four lanes of a row have its 64 bytes between them, and a compute unit
+// then draws 64 bytes a cycle through its address unit (131 KB/us with all CUs at it, 149 with one), where lanes that go down
+// the rows first, 16 bytes each, get 16 (37 KB/us). Within a row the pieces are exchanged by row number, slot = piece ^ (row / 4) % 4,
+// so that the 16 rows of an operand read lie in different banks.
+__device__ __forceinline__ int rows16_lane_src(int lane, int row_stride) { return (lane >> 2) * row_stride + ((lane & 3) ^ (lane >> 4)) * 16; }
+// Place of a lane's operand piece, of row `row` and lane half hi: k-step s is at (s / 2) KiB + this, with the odd steps' places ^ 32.
+__device__ __forceinline__ int rows16_operand(int row, int hi) { return (row & 15) * 64 + ((hi ^ ((row >> 2) & 3)) * 16); }
+
 }  // namespace fa_lds_dma

@@ -25,6 +25,8 @@ namespace {
 
 using fa_lds_dma::buffer_to_lds_b128;
 using fa_lds_dma::make_rsrc_words;
+using fa_lds_dma::rows16_lane_src;
+using fa_lds_dma::rows16_operand;
 using fa_lds_dma::rsrc_words;
 
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -442,8 +444,11 @@ __device__ __forceinline__ void phase_barrier() {
 // K/V tiles go from memory straight into LDS (buffer_load ... lds: the 64 lanes of one instruction fill 1 KB of
 // consecutive LDS bytes), so no registers and no issue slots are spent on staging them. Row padding is impossible inside such a 1 KB run, so the tiles are laid out for conflict-free
 // reads with plain base + constant addressing instead:
-//   K tile  [16-row block rb][16-byte chunk c][row r of 16]        one instruction = 4 chunks x 16 rows;
-//           the S^T operand read of 16 lanes (16 rows, same chunk) is 256 consecutive bytes.
+//   K tile  [16-row block rb][64-byte column][row r of 16][64 B]    one instruction = 64 bytes of 16 rows (rows16_lane_src,
+//           fa_lds_dma.h: why, and how the S^T operand reads find their pieces).
+//           (With lanes going down 16 rows first, as the operand reads want them, a tile pair's K alone kept the address unit
+//           busy for 2048 of its 3200 cycles. 256 rows, H24 / Hkv8 / D128: 10.8 -> 9.6 us; 500 rows 13.8 -> 12.6; 2048 rows
+//           35.9 -> 34.6; 8000 rows 395 -> 388; H14 / Hkv2 / D64, 2048 rows: 23.3 -> 22.6.)
 //   V tile  [4-row group rg][64-byte column block cb][row r4][64 B] one instruction = 4 (D=128) or 8 rows;
 //           the 32 lanes of a transpose-read pass (4 rows x 64 B) are 256 consecutive bytes.
 // Wave w of a group moves rows 16w..16w+15 of every tile of its group (16 rows never straddle a page). Rows past
@@ -546,10 +551,10 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
 
     U4H8 qreg[DSTEPS];
 
-    // ---- memory -> LDS. Lane l of a K instruction takes chunk l / 16 of row l % 16; of a V instruction, piece
+    // ---- memory -> LDS. Lane l of a K instruction takes a 16-byte piece of row l / 4; of a V instruction, piece
     // l % 4 of column block (l / 16) % (ROWB / 64) of row (l / (16 ROWB / 64)) * 4 + (l % 16) / 4.
     constexpr int CBR = ROWB / 64;
-    const int k_lane_src = (lane & 15) * ROWB + (lane >> 4) * 16;
+    const int k_lane_src = rows16_lane_src(lane, ROWB);
     const int v_lane_src = ((lane / (16 * CBR)) * 4 + ((lane & 15) >> 2)) * ROWB + ((lane >> 4) % CBR) * 64 + (lane & 3) * 16;
     typedef const int32_t __attribute__((address_space(4))) *const_i32p;
     const const_i32p bt = (const_i32p)a.block_table;
@@ -578,7 +583,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             }
         }
         if (is_k) {
-            // chunk quads: 64 bytes apart in a row, 1 KB apart in LDS
+            // 64-byte columns: 64 bytes apart in a row, 1 KB apart in LDS
             buffer_to_lds_b128<K_DMA, 64, 1024>(rs, k_lds_addr + buf * K_TILE + wave * RB_BYTES, k_lane_src, so);
         } else {
             // 1 KB of rows after 1 KB of rows, in memory as in LDS
@@ -593,7 +598,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     auto q_dma = [&](uint32_t item) {
         int ql = lane;
         asm volatile("" : "+v"(ql));  // the lane's source offset is worked out here, not kept in a register across the loop
-        const int q_lane_src = (ql & 15) * (int)(a.q_stride_m * 2) + (ql >> 4) * 16;
+        const int q_lane_src = rows16_lane_src(ql, (int)(a.q_stride_m * 2));
         // the 16 rows this wave moves are half of the 32 rows of wave (wave8 / 2) of either group
         const WaveRows wr = wave_rows(item, (uint32_t)wave8 >> 1);
         const uint32_t row0 = wr.row0 + 16 * ((uint32_t)wave8 & 1);
@@ -617,19 +622,24 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     };
     const float c = a.scale_log2e;
 
-    const int k_lane = (n >> 4) * RB_BYTES + hi * 256 + (n & 15) * 16;
+    const int k_lane = (n >> 4) * RB_BYTES + rows16_operand(n, hi);
+    // this lane's places in the K tile whose operands are being read, for even and for odd k-steps (set where the tile's first
+    // operands are read: worked out again in the MFMA phase they cost a large launch at D = 64 one per cent)
+    const unsigned char *k_even = k_base, *k_odd = k_base;
+    // operand t of that tile: k-step t % DSTEPS of its 32-row half t / DSTEPS
+    auto k_operand = [&](int t) __attribute__((always_inline)) -> uint4 {
+        return *reinterpret_cast<const uint4 *>((t & 1 ? k_odd : k_even) + (t / DSTEPS) * (2 * RB_BYTES) + (t % DSTEPS / 2) * 1024);
+    };
     const int v_lane = hi * RG_BYTES + ((lane & 15) >> 2) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
     f16_t sacc[2];
     h8_t pb[2][2];
     U4H8 kpre[K_AHEAD];  // the first K operands of the next MFMA phase, read before the barrier that starts it
     auto k_prefetch = [&](int buf) {
-        const unsigned char *k_lds = k_base + buf * K_TILE + k_lane;
+        k_even = k_base + buf * K_TILE + k_lane, k_odd = k_base + buf * K_TILE + (k_lane ^ 32);
 #pragma unroll
-        for (int i = 0; i < K_AHEAD; ++i)
-            kpre[i].u = *reinterpret_cast<const uint4 *>(k_lds + (i / DSTEPS) * (2 * RB_BYTES) + (i % DSTEPS) * 512);
+        for (int i = 0; i < K_AHEAD; ++i) kpre[i].u = k_operand(i);
     };
-    auto s_tile = [&](int buf) {  // S_0 of an item, outside the phases
-        const unsigned char *k_lds = k_base + buf * K_TILE + k_lane;
+    auto s_tile = [&]() {  // S_0 of an item, outside the phases
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
@@ -638,7 +648,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             for (int s = 0; s < DSTEPS; ++s) {
                 U4H8 kk;
                 if (kb * DSTEPS + s < K_AHEAD) kk = kpre[kb * DSTEPS + s];
-                else kk.u = *reinterpret_cast<const uint4 *>(k_lds + kb * (2 * RB_BYTES) + s * 512);
+                else kk.u = k_operand(kb * DSTEPS + s);
                 sacc[kb] = BF16 ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk.b, qreg[s].b, sacc[kb], 0, 0, 0)
                                 : __builtin_amdgcn_mfma_f32_32x32x16_f16(kk.h, qreg[s].h, sacc[kb], 0, 0, 0);
             }
@@ -656,7 +666,6 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     // whenever it judges the register pressure of the function too high, and the pipe then idles through every read.
     auto mfma_phase = [&](int j) {
         constexpr int NS = 2 * DSTEPS, NG = 4, NV = NG * DBLKS;  // S MFMAs; (key block, k-step) pairs; V operands
-        const unsigned char *k_lds = k_base + ((j + 1) & 1) * K_TILE + k_lane;
         const unsigned char *v_lds = v_base + (j & 1) * V_TILE + v_lane;
         U4H8 kop[NS];
         union {
@@ -683,7 +692,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             if (i == DSTEPS) l_run += psum2[0] + psum2[1];
             if (i + K_AHEAD < NS) {  // K operand i + K_AHEAD
                 const int t = i + K_AHEAD;
-                kop[t].u = *reinterpret_cast<const uint4 *>(k_lds + (t / DSTEPS) * (2 * RB_BYTES) + (t % DSTEPS) * 512);
+                kop[t].u = k_operand(t);
             }
             const int pv = i - (NS - V_AHEAD);  // V operand pv: k-slot jj of k-step ks <-> key 32 kb + 16 ks + ... =
             if (pv >= 0 && pv < NV) {           // accumulator 8 ks + jj of block kb, for both operands
@@ -852,8 +861,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         const uint32_t next_item = item_of(round + 1);
         const bool has_next = next_item < n_items;
         // Q and K_0 (for S_0) must be there now; K_1 and V_0, requested after them (loads complete in order), have until
-        // the first MFMA phase. A CU pulls about 25 GB/s on its own, so every 16 KB not waited for here is worth half a
-        // microsecond.
+        // the first MFMA phase.
         if (ntg > 1) __builtin_amdgcn_s_waitcnt(VMCNT_KV);
         else if (ntg > 0) __builtin_amdgcn_s_waitcnt(VMCNT_V);
         else __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -862,9 +870,10 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             int lo = lane;
             asm volatile("" : "+v"(lo));  // (see write_item)
             const int rb = wave * 2 + ((lo & 31) >> 4);  // 16-row block of this lane's row; both groups hold the same 128 rows
-            const unsigned char *qp = lds + 2 * GRP_LDS + rb * RB_BYTES + (lo >> 5) * 256 + (lo & 15) * 16;
+            const int q_lane = rows16_operand(lo & 15, lo >> 5);
+            const unsigned char *qp = lds + 2 * GRP_LDS + rb * RB_BYTES;
 #pragma unroll
-            for (int s = 0; s < DSTEPS; ++s) qreg[s].u = *reinterpret_cast<const uint4 *>(qp + s * 512);
+            for (int s = 0; s < DSTEPS; ++s) qreg[s].u = *reinterpret_cast<const uint4 *>(qp + (s & 1 ? q_lane ^ 32 : q_lane) + s / 2 * 1024);
 #pragma unroll
             for (int s = 0; s < DSTEPS; ++s) {  // arrived: keep the wait out of the loop
                 u4_t t = __builtin_bit_cast(u4_t, qreg[s].u);
@@ -878,7 +887,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         const uint32_t wave_min_limit = a.causal ? (min(w_row0, a.q_len - 1) + a.query_offset) : 0xffffffffu;
         if (ntg > 0) {
             k_prefetch(0);
-            s_tile(0);
+            s_tile();
         }
         if (grp == 1) phase_barrier();  // one phase behind group 0
         for (int j = 0; j < iters; ++j) {
