@@ -257,6 +257,26 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &a);
 // whether it took the launch; `force`: also where the tiled kernel would normally be preferred (short contexts).
 fa_status fa_launch_prefill_chunk(fa_ctx *ctx, const PrefillLaunch &a, bool force, bool *taken);
 
+// Merge of the partial states of query tiles whose keys were split (fa_prefill.hip; also the kernel's argument). The rows are lists,
+// one per head, or one per KV head with its `group` heads' rows of one position after the other.
+struct PrefillMerge {
+    __half *out;
+    uint64_t out_stride_h, out_stride_m;
+    const float *part_acc, *part_ml;  // [list][tile][split][part_rows][D] unnormalised sums, [..][part_rows][2] (max, sum)
+    uint32_t n_lists, n_rows, group, rcp_group /* floor(2^32 / group) + 1, 0 for 1 */, splits;
+    uint32_t tile_rows, part_rows;    // rows of a list that a tile stands for; rows of them in the partial buffers (the rest do not exist)
+};
+fa_status fa_launch_prefill_merge(fa_ctx *ctx, const PrefillMerge &g, uint32_t head_dim, bool bf16);
+// fa_rows.hip: 32 query rows to a workgroup, for chunks and prompts of moderate size.
+struct RowsPlan {
+    uint32_t waves = 0, splits = 1;  // waves 0: the kernel cannot take the launch
+    float us = 0.0f;                 // estimate
+};
+RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &a);
+fa_status fa_launch_prefill_rows(fa_ctx *ctx, const PrefillLaunch &a, const RowsPlan &plan);
+// What the short-chunk kernel would take by estimate; 0 where it does not take the launch of its own accord.
+float fa_prefill_chunk_estimate_us(const fa_ctx *ctx, const PrefillLaunch &a);
+
 fa_status fa_launch_u32_add(fa_ctx *ctx, uint32_t *vals, uint32_t n, uint32_t delta);
 fa_status fa_launch_paged_gather(fa_ctx *ctx, const fa_paged_kv *c, uint32_t seq_index, uint32_t seq_len, void *k_out,
                                  void *v_out, uint32_t out_capacity);

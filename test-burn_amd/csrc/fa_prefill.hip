@@ -991,18 +991,18 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
 // Merge of the per-split states (flash_prefill.metal:843-888): m* = max m_s, L = sum l_s 2^(m_s - m*) over the
 // splits with l_s > 0, out = sum acc_s 2^(m_s - m*) / L (0 when L is unusable). m is kept in the exp2 domain.
 template <int D, bool BF16>
-__global__ void __launch_bounds__(256) flash_prefill_merge_kernel(PrefillDev a) {
+__global__ void __launch_bounds__(256) flash_prefill_merge_kernel(PrefillMerge a) {
     constexpr int CG = D / 4;           // float4 columns per row
     constexpr int ROWS = 256 / CG;      // rows per workgroup (8 at D = 128, 16 at D = 64)
     const uint32_t S = a.splits, PR = a.part_rows;
     const uint32_t SLABS = PR / ROWS;   // workgroups per query tile
-    const uint32_t n_qt = gridDim.x / (a.n_heads * SLABS);
+    const uint32_t n_qt = gridDim.x / (a.n_lists * SLABS);
     const uint32_t slab = blockIdx.x % SLABS, qh = blockIdx.x / SLABS;
-    const uint32_t q_tile = qh / a.n_heads, head = qh % a.n_heads;
+    const uint32_t q_tile = qh / a.n_lists, list = qh % a.n_lists;
     const int r = slab * ROWS + threadIdx.x / CG, c4 = threadIdx.x % CG;
-    const uint32_t q_row = q_tile * BM + r;
-    if (q_row >= a.q_len) return;
-    const size_t base = (((size_t)head * n_qt + q_tile) * S) * PR + r;
+    const uint32_t row = q_tile * a.tile_rows + r;
+    if (row >= a.n_rows) return;
+    const size_t base = (((size_t)list * n_qt + q_tile) * S) * PR + r;
     // All of a row's splits in ONE trip to memory when there are at most 32 of them (the usual case): the (max, sum)
     // pairs and the sums are requested together - the addresses of the sums do not depend on the pairs - and the two passes
     // of the reference (the row's maximum, then the weighted sums in split order) run on registers. The batch size is the
@@ -1046,6 +1046,7 @@ __global__ void __launch_bounds__(256) flash_prefill_merge_kernel(PrefillDev a) 
     const float inv = (isfinite(L) && fabsf(L) > 1e-6f) ? (1.0f / L) : 0.0f;
     h4_t h;
     h[0] = to_elem<BF16>(o.x * inv), h[1] = to_elem<BF16>(o.y * inv), h[2] = to_elem<BF16>(o.z * inv), h[3] = to_elem<BF16>(o.w * inv);
+    const uint32_t q_row = a.rcp_group ? __umulhi(row, a.rcp_group) : row, head = list * a.group + row - q_row * a.group;
     *reinterpret_cast<h4_t *>(a.out + (size_t)head * a.out_stride_h + (size_t)q_row * a.out_stride_m + c4 * 4) = h;
 }
 
@@ -1071,12 +1072,21 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     if (L.q_len == 0) return FA_OK;
     if (L.head_dim != 128 && L.head_dim != 64)
         return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "Prefill only supports head_dim=64 or 128, got %u", L.head_dim);
-    // A chunk of at most 64 rows after a long prefix is a memory-bound launch: fa_chunk.hip (unless a kernel or a split
-    // count has been asked for by name)
-    if (!ctx->prefill_chunk_off && ((ctx->prefill_variant == 0 && ctx->prefill_split_k == 0) || ctx->prefill_variant == 3)) {
-        bool taken = false;
-        FA_TRY(fa_launch_prefill_chunk(ctx, L, ctx->prefill_variant == 3, &taken));
-        if (taken) return FA_OK;
+    // Unless a kernel or a split count has been asked for by name: the kernel that takes 32 rows to a workgroup (fa_rows.hip), for a
+    // chunk of at most 64 rows after a long prefix the memory-bound one (fa_chunk.hip), or the tiled one, by estimate. (What the first
+    // is given it takes ahead of the others by a twentieth or more. Over 2650 shapes of 2 to 8000 rows after 0 to 36000, 4 to 32 heads,
+    // each timed with all three, it was slower than the other choice by more than 3 % for nine, by 14 % at most, and 1.6 times as fast
+    // in the mean. Beyond the keys below nothing is fitted, and the short-chunk kernel reads a KV head's keys once.)
+    const bool automatic = ctx->prefill_variant == 0 && ctx->prefill_split_k == 0;
+    const RowsPlan rows = automatic ? fa_prefill_rows_plan(ctx, L) : RowsPlan();
+    if ((automatic || ctx->prefill_variant == 3) && !ctx->prefill_chunk_off) {
+        const float chunk_us = rows.waves ? fa_prefill_chunk_estimate_us(ctx, L) : 0.0f;
+        if (chunk_us > 0.0f && rows.us < 0.95f * chunk_us && L.kv_len <= (L.head_dim == 128 ? 20000u : 65536u)) return fa_launch_prefill_rows(ctx, L, rows);
+        if (!rows.waves || chunk_us > 0.0f) {
+            bool taken = false;
+            FA_TRY(fa_launch_prefill_chunk(ctx, L, ctx->prefill_variant == 3, &taken));
+            if (taken) return FA_OK;
+        }
     }
     // Split-K (src/metals/flashattention/step.rs:849-864): few query tiles against a long context (a prefill chunk
     // after a long prefix) would leave most CUs idle, so the key tiles of each query tile are divided over several
@@ -1121,6 +1131,27 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     }
     if (splits > key_tiles) splits = key_tiles;
     if (splits < 1) splits = 1;
+    if (rows.waves) {
+        // What the tiled kernel takes: the longest item, in pairs of key tiles, or the items and the pairs of one CU's share; with splits
+        // also the partial states. 6 to 7 % from 1570 launches.
+        const bool wide = L.head_dim == 128;
+        auto pairs_of = [&](uint32_t last_row) -> float {
+            const uint64_t end = L.causal ? (uint64_t)last_row + L.query_offset + 1 : L.kv_len;
+            return (float)ceil_div_u32(ceil_div_u32(ceil_div_u32((uint32_t)(end < L.kv_len ? end : L.kv_len), BN), splits), 2);
+        };
+        const float longest = pairs_of(L.q_len - 1), first = pairs_of(L.q_len < BM ? L.q_len - 1 : BM - 1), share = (float)base_wgs / (float)n_cus;
+        float us;
+        if (splits > 1) {
+            const float mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * (float)splits * 4e-6f;
+            us = wide ? 7.49f + 1.657f * longest + 0.709f * mb : 6.80f + 1.12f * longest + 0.84f * mb;
+        } else {
+            const float one = wide ? -1.44f + 1.537f * longest : -0.73f + 1.149f * longest;
+            const float cu = wide ? share * (4.2f + 0.993f * (first + longest)) : share * (2.02f + 0.668f * (first + longest));
+            us = (wide ? 7.30f : 5.94f) + (one > cu ? one : cu);
+        }
+        // (packed heads: up to 64 rows, for which the other kernel was ahead wherever it was timed, up to 50000 keys)
+        if (a.pack_heads ? L.kv_len <= 49152u : rows.us < 0.95f * us) return fa_launch_prefill_rows(ctx, L, rows);
+    }
     a.splits = splits, a.part_acc = nullptr, a.part_ml = nullptr;
     if (splits > 1) {
         const size_t rows = (size_t)L.n_heads * ceil_div_u32(L.q_len, BM) * splits * a.part_rows;
@@ -1157,17 +1188,22 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
         FA_TRY(scope.finish());
     }
     if (splits > 1) {
-        const uint32_t merge_tiles = L.n_heads * ceil_div_u32(L.q_len, BM);  // (head, query tile) pairs
-        FaLaunchScope scope(ctx, "flash_prefill_merge_kernel", true);
-        if (L.head_dim == 128 && L.bf16)
-            scope.launch(flash_prefill_merge_kernel<128, true>, dim3(merge_tiles * (a.part_rows / 8)), dim3(256), 0, a);
-        else if (L.head_dim == 128)
-            scope.launch(flash_prefill_merge_kernel<128, false>, dim3(merge_tiles * (a.part_rows / 8)), dim3(256), 0, a);
-        else if (L.bf16)
-            scope.launch(flash_prefill_merge_kernel<64, true>, dim3(merge_tiles * (a.part_rows / 16)), dim3(256), 0, a);
-        else
-            scope.launch(flash_prefill_merge_kernel<64, false>, dim3(merge_tiles * (a.part_rows / 16)), dim3(256), 0, a);
-        FA_TRY(scope.finish());
+        PrefillMerge g;
+        g.out = L.out, g.out_stride_h = L.out_stride_h, g.out_stride_m = L.out_stride_m;
+        g.part_acc = a.part_acc, g.part_ml = a.part_ml, g.n_lists = L.n_heads, g.n_rows = L.q_len, g.group = 1, g.rcp_group = 0;
+        g.splits = splits, g.tile_rows = BM, g.part_rows = a.part_rows;
+        return fa_launch_prefill_merge(ctx, g, L.head_dim, L.bf16);
     }
     return FA_OK;
+}
+
+fa_status fa_launch_prefill_merge(fa_ctx *ctx, const PrefillMerge &g, uint32_t head_dim, bool bf16) {
+    const uint32_t tiles = g.n_lists * ceil_div_u32(g.n_rows, g.tile_rows);
+    const dim3 grid(tiles * (g.part_rows / (head_dim == 128 ? 8 : 16)));
+    FaLaunchScope scope(ctx, "flash_prefill_merge_kernel", true);
+    if (head_dim == 128 && bf16) scope.launch(flash_prefill_merge_kernel<128, true>, grid, dim3(256), 0, g);
+    else if (head_dim == 128) scope.launch(flash_prefill_merge_kernel<128, false>, grid, dim3(256), 0, g);
+    else if (bf16) scope.launch(flash_prefill_merge_kernel<64, true>, grid, dim3(256), 0, g);
+    else scope.launch(flash_prefill_merge_kernel<64, false>, grid, dim3(256), 0, g);
+    return scope.finish();
 }

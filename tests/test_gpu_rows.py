@@ -1,0 +1,137 @@
+"""GPU: the attention kernel that gives 32 query rows to a workgroup (chunks and prompts of moderate size, the automatic choice)
+against the oracle, at the edges of what it divides: rows of a KV group's heads in blocks of 32, keys in tiles of 32 over 4 or 8
+waves, keys split over workgroups, pages."""
+import numpy as np
+import pytest
+
+import foundry_attn as fa
+import orc
+from gpu_util import announce, ctx, h16, max_abs
+from test_gpu_paged import Paged
+
+pytestmark = pytest.mark.gpu
+TOL, TOL_BF16 = 2e-3, 2e-2
+BF = fa.DTYPE_BF16
+
+
+def _launches(f, call):
+    """What the call put on the stream: (this kernel, merge launches, any other attention kernel)."""
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        call()
+        f.synchronize()
+        n = {k: f.profile_query(k)[0] for k in ("flash_rows_kernel", "flash_chunk_kernel_rows", "flash_prefill_merge_kernel", "flash_")}
+    finally:
+        f.profile_enable(False)
+    rows = n["flash_rows_kernel"] + n["flash_chunk_kernel_rows"]  # (the second: at most 64 query rows)
+    return rows, n["flash_prefill_merge_kernel"], n["flash_"] - rows - n["flash_prefill_merge_kernel"]
+
+
+CASES = [
+    # H, Hkv, D, rows, prefix, splits expected
+    (14, 2, 64, 2, 0, False),        # fewest rows: 14 of a block's 32
+    (14, 2, 64, 4, 27, False),       # 28 rows of a block; 31 keys, one short of a tile
+    (14, 2, 64, 5, 27, False),       # 35 rows: three of a second block; 32 keys
+    (16, 2, 128, 4, 29, False),      # 32 rows: a whole block; 33 keys
+    (4, 4, 128, 33, 64, False),      # a head to a group: one row of a second block
+    (6, 2, 128, 17, 239, False),     # 256 keys: one tile per wave of eight
+    (6, 2, 128, 17, 240, False),     # one key more
+    (14, 2, 64, 100, 157, False),
+    (24, 8, 128, 100, 700, False),
+    (14, 2, 64, 500, 0, False),      # a prompt: every block another number of keys
+    (14, 2, 64, 650, 31, False),     # more blocks than compute units: four waves
+    (24, 8, 128, 401, 9, False),     # the same at D 128
+    (12, 4, 64, 3, 3000, True),      # few rows, many keys: split
+    (24, 8, 128, 20, 2900, True),
+    (8, 2, 64, 32, 5001, True),
+    (5, 1, 128, 7, 8161, True),      # one KV head
+]
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f16", "bf16"])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", CASES)
+def test_rows_contiguous(H, Hkv, D, M, prefix, split, bf16):
+    announce("prefill rows", H, Hkv, D, M, prefix, split, bf16)
+    f = ctx()
+    rng = np.random.default_rng(M * 7 + prefix)
+    N = prefix + M
+    cap = N + 7
+    q, k, v = (rng.normal(size=s).astype(np.float32) for s in ((H, M, D), (Hkv, cap, D), (Hkv, cap, D)))
+    k[:, N:], v[:, N:] = np.nan, np.nan  # nothing past the visible keys is used
+    conv = orc.bf16_pack if bf16 else h16
+    q, k, v = conv(q), conv(k), conv(v)
+    dt = BF if bf16 else fa.DTYPE_F16
+    dq, dk, dv, do = (f.array(x) for x in (q, k, v, np.full((M, H * D), 0x7fc0 if bf16 else 0x7e00, np.uint16)))
+    args = [b.arg(dtype=dt) for b in (dq, dk, dv, do)]
+    n = _launches(f, lambda: f.flash_attention(*args, True, prefix, H, D, N, M))
+    assert n == (1, 1 if split else 0, 0), n
+    want = lambda: orc.sdpa_prefill(q, k, v, H, Hkv, D, M, N, prefix, cap, causal=True, out_layout="token_major", n_threads=8)
+    raw = do.download()
+    if bf16:
+        with orc.bf16_mode():
+            w = orc.bf16_unpack(want())
+        got = orc.bf16_unpack(raw)
+    else:
+        w, got = want(), raw.view(np.float16)
+    assert np.all(np.isfinite(got))
+    assert max_abs(got.reshape(M, H * D), w.reshape(M, H * D)) <= (TOL_BF16 if bf16 else TOL)
+    for b in (dq, dk, dv, do):
+        b.free()
+
+
+@pytest.mark.parametrize("bs", [16, 48, 64])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", CASES[::2] + CASES[-4:-1])
+def test_rows_paged(H, Hkv, D, M, prefix, split, bs):
+    """Pages of one row group, of a number that is not a power of two, and of two tiles; the last page partly filled."""
+    announce("prefill rows, paged", H, Hkv, D, M, prefix, split, bs)
+    f = ctx()
+    rng = np.random.default_rng(M * 11 + prefix + bs)
+    N = prefix + M
+    lens = [3, N]
+    ks = [h16(rng.normal(size=(Hkv, n, D))) for n in lens]
+    vs = [h16(rng.normal(size=(Hkv, n, D))) for n in lens]
+    pg = Paged(f, rng, lens, Hkv, D, bs, extra_tokens=0)
+    pg.fill_from(ks, vs)
+    last = pg.bt[1, (N - 1) // bs]
+    if N % bs:  # rows past the sequence's end, in its own last page
+        pg.k_pool[last, :, N % bs:], pg.v_pool[last, :, N % bs:] = np.nan, np.nan
+    pg.upload()
+    q = h16(rng.normal(size=(H, M, D)))
+    dq, do = f.array(q), f.zeros((M, H * D))
+    n = _launches(f, lambda: f.flash_prefill_paged(dq.arg(), pg.desc, 1, do.arg(), True, prefix, H, N, M))
+    assert n == (1, 1 if split else 0, 0), n
+    got = do.download()
+    want = orc.sdpa_prefill(q, ks[1], vs[1], H, Hkv, D, M, N, prefix, N, causal=True, n_threads=8)
+    assert np.all(np.isfinite(got))
+    assert max_abs(got.reshape(M, H * D), want.reshape(M, H * D)) <= TOL
+    pg.free()
+    for b in (dq, do):
+        b.free()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("M,N,offset,causal", [(45, 300, 0, False), (45, 300, 3, True), (45, 60, 100, True), (9, 4000, 17, False)])
+def test_rows_masks_and_layouts(M, N, offset, causal, D):
+    """Without the causal mask; query positions in the middle of the keys and past their end; token-major queries and head-major
+    output give the bits of the head-major queries and token-major output."""
+    announce("prefill rows, masks and layouts", M, N, offset, causal, D)
+    f = ctx()
+    rng = np.random.default_rng(N + offset)
+    H, Hkv, cap = 6, 2, N + 3
+    q, k, v = h16(rng.normal(size=(H, M, D))), h16(rng.normal(size=(Hkv, cap, D))), h16(rng.normal(size=(Hkv, cap, D)))
+    dk, dv = f.array(k), f.array(v)
+    outs = []
+    for token_major in (False, True):
+        dq = f.array(np.ascontiguousarray(q.transpose(1, 0, 2)) if token_major else q)
+        do = f.zeros((H, M, D) if token_major else (M, H * D))
+        qa = dq.arg((M, H, D) if token_major else (H, M, D))
+        n = _launches(f, lambda: f.flash_attention(qa, dk.arg(), dv.arg(), do.arg(), causal, offset, H, D, N, M))
+        assert n[0] == 1 and n[2] == 0, n
+        got = do.download()
+        outs.append(got if token_major else got.reshape(M, H, D).transpose(1, 0, 2))
+        dq.free(), do.free()
+    assert np.array_equal(np.ascontiguousarray(outs[0]).view(np.uint16), outs[1].view(np.uint16))
+    want = orc.sdpa_prefill(q, k, v, H, Hkv, D, M, N, offset, cap, causal=causal, out_layout="head_major", n_threads=8)
+    assert max_abs(outs[1], want) <= TOL
+    dk.free(), dv.free()
