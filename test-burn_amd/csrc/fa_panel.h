@@ -68,8 +68,14 @@ template <int NT>
 constexpr int scale_stride() { return NT * 16 + 4; }
 template <int NT, int PK>
 constexpr int scale_bytes() { return scale_stride<NT>() * PK * 16 * 2; }
+// Q4_0 with per-block sums, more than 1024 features: weights are fetched along memory and turned into operand order in LDS.
+template <int WB, int PK, bool SUMS>
+constexpr bool TURNS = WB == 4 && SUMS && PK > 2;
+// Behind everything else, for that: room for each wave to turn weights into operand order, a KiB at a time.
 template <int WB, int NT, int NC, int PK>
-constexpr int lds_bytes() { return lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0) + (WB != 16 ? scale_bytes<NT, PK>() : 0); }
+constexpr int turn_at() { return (lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ? PK * 1024 : 0) + (WB != 16 ? scale_bytes<NT, PK>() : 0) + 15) & ~15; }
+template <int WB, int NT, int NC, int PK, bool SUMS>
+constexpr int lds_bytes() { return turn_at<WB, NT, NC, PK>() + (TURNS<WB, PK, SUMS> ? NW * 1024 : 0); }
 
 // launchers per weight width (one translation unit each): nt = 16-row tiles of weight rows, nc = 16-row groups of input rows per pass, pk = 512-feature pieces
 template <int WB>

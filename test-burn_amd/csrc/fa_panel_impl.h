@@ -155,22 +155,38 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             }
         }
     }
-    // ---- all weights of the workgroup. F16 (and SUMS): block kb of slot (t, n), features 8c .. 8c + 7. Block-quantised: 16 bytes
-    // per lane, half a block of one of two (Q8_0) or a block of four (Q4_0); the features that lane c holds for step s of such a
-    // request follow from that, for the weights and for the input rows alike.
-    constexpr bool WIDE = WB != 16 && !SUMS;
-    constexpr int GB = !WIDE ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
-    typedef typename std::conditional<WIDE, u4v_t, raw_t>::type req_t;
+    // ---- all weights of the workgroup. F16 (and SUMS, Q8_0): block kb of slot (t, n), features 8c .. 8c + 7. Block-quantised: 16
+    // bytes per lane, half a block of one of two (Q8_0) or a block of four (Q4_0); the features that lane c holds for step s of such
+    // a request follow from that, for the weights and for the input rows alike. SUMS wants a block in all lanes of a row: with Q4_0
+    // that is 4 bytes to a lane, and a compute unit's address unit takes few lanes per cycle whatever they ask for. So the lanes
+    // take 16 bytes along memory there (TURN) and the operand order is made in LDS when the weights are first used: Q4_0, 2 to 11
+    // rows, 5120 x 3072 10.1 -> 9.2 us, row-major 12.6 -> 9.3; 3072 x 3072 6.4 -> 5.7, 7.9 -> 5.8; 2560 x 2048 7.7 -> 7.4. (Rows of
+    // up to 1024 features are a request or two either way, row-major 1 to 5 % slower; F16 and the other block-quantised forms lose
+    // 3 to 15 % by it, Q8_0 per-block sums 7 to 40 % for want of registers.)
+    constexpr bool WIDE = WB != 16 && !SUMS, TURN = TURNS<WB, PK, SUMS>;
+    constexpr int GB = !WIDE && !TURN ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
+    typedef typename std::conditional<WIDE || TURN, u4v_t, raw_t>::type req_t;
     auto kb_of = [&](int i) __attribute__((always_inline)) -> uint32_t {
         return GB == 1 ? 16u * (uint32_t)(i >> 1) + 2u * (uint32_t)wave + (uint32_t)(i & 1) : GB == 2 ? 16u * (uint32_t)i + 2u * (uint32_t)wave : 32u * (uint32_t)i + 4u * (uint32_t)wave;
     };
-    const uint32_t lane_blk = GB == 1 ? 0u : GB == 2 ? (uint32_t)c >> 1 : (uint32_t)c;  // the lane's block of a request
+    // the lane's row and block of a request: of its operand, and of what it fetches (blocked weights have a block of 16 rows side by side)
+    const uint32_t lane_blk = GB == 1 ? 0u : GB == 2 ? (uint32_t)c >> 1 : (uint32_t)c;
+    const uint32_t get_row = TURN && !canonical ? (uint32_t)lane >> 2 : (uint32_t)n, get_blk = TURN && !canonical ? (uint32_t)lane & 3u : lane_blk;
+    // TURN: a KiB of LDS per wave, [block][row][16 bytes]
+    unsigned char *const turn = smem + turn_at<WB, NT, NC, PK>() + wave * 1024;
+    auto operand_order = [&](req_t &w) __attribute__((always_inline)) {
+        if constexpr (TURN) {
+            *reinterpret_cast<u4v_t *>(turn + get_blk * 256 + get_row * 16) = w;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) w[b] = *reinterpret_cast<const uint32_t *>(turn + b * 256 + n * 16 + c * 4);
+        }
+    };
     req_t wv[NT][NQ];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         bool valid;
         int mat;
-        const uint32_t lrow = locate(slot_row((uint32_t)t, (uint32_t)n, valid), mat);
+        const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
         const uint32_t N = pick3(mat, rows0, rows1, rows1);
         // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
         const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
@@ -178,7 +194,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            const uint32_t kb = kb_of(i) + lane_blk;
+            const uint32_t kb = kb_of(i) + get_blk;
             const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
             // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
             // block-quantised weights are finite, and their scale is zero there.)
@@ -280,8 +296,12 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         if (next < n_pass) request_rows(next);
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            const uint32_t kb = kb_of(i) + lane_blk;
-            const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
+            if (TURN && pass == blockIdx.y) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) operand_order(wv[t][i]);
+            }
+            const uint32_t kb = kb_of(i) + (TURN ? 0u : lane_blk);
+            const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 || TURN ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
             const _Float16 *const scp = sc_lds + kb * SC_STRIDE + (SUMS ? c * 4 : n);
             req_t raw[NT];
             _Float16 sc[NT];
@@ -296,16 +316,19 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int st = 0; st < GB; ++st) {
                 h8_t xb[NC];
 #pragma unroll
-                for (int h = 0; h < NC; ++h) xb[h] = *reinterpret_cast<const h8_t *>(xp + st * 16 + h * 16 * XROW);
+                for (int h = 0; h < NC; ++h) xb[h] = *reinterpret_cast<const h8_t *>(xp + st * (TURN ? 64 : 16) + h * 16 * XROW);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     if constexpr (SUMS) {
                         typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
-                        const h4_t s4 = *reinterpret_cast<const h4_t *>(scp + t * 16);
+                        const h4_t s4 = *reinterpret_cast<const h4_t *>(scp + st * SC_STRIDE + t * 16);
                         const f4v_t z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                         for (int h = 0; h < NC; ++h) {
-                            const f4v_t blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(W::plain(raw[t]), xb[h], z, 0, 0, 0);
+                            raw_t w;
+                            if constexpr (TURN) w = W::part(raw[t], st);
+                            else w = raw[t];
+                            const f4v_t blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(W::plain(w), xb[h], z, 0, 0, 0);
 #pragma unroll
                             for (int q = 0; q < 4; ++q) d[t][h][q] += blk[q] * (float)s4[q];
                         }
@@ -386,7 +409,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
 
 template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
 fa_status launch_one(FaLaunchScope &scope, dim3 grid, const PanelDev &a) {
-    constexpr int lds = lds_bytes<WB, NT, NC, PK>();
+    constexpr int lds = lds_bytes<WB, NT, NC, PK, SUMS>();
     static std::atomic<uint64_t> allowed{0};  // devices this kernel's LDS size has been asked for on (the calls are idempotent)
     const uint64_t bit = 1ull << (scope.ctx->device & 63);
     if (!(allowed.load(std::memory_order_acquire) & bit)) {

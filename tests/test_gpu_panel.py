@@ -82,3 +82,12 @@ def test_chunk_in_one_launch_infinite_last_block(K, m, weights, layout):
     """Row lengths of every number of feature pieces whose blocks do not fill a wave's share, odd and even in number."""
     announce("panel, infinite last block", K, m, weights, layout)
     infinite_last_block(K, 40, m, weights, layout)
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("K,N,NK,m", [(1024, 40, 24, 3), (1056, 40, 24, 2), (1088, 72, 8, 11), (1120, 200, 40, 7), (1152, 40, 24, 4), (2048, 264, 72, 11), (2080, 40, 24, 2),
+                                      (3040, 40, 16, 11), (3072, 4136, 1024, 6)])
+def test_q4_weights_turned_into_operand_order(K, N, NK, m, layout):
+    """Q4_0 with per-block sums (2 to 11 rows): the weights of four blocks go through LDS from the longest rows that do not, with one,
+    two, three and four blocks in a row's last request, one and two tiles of weight rows, both layouts."""
+    test_chunk_in_one_launch(K, N, NK, m, layout, "q4")
