@@ -52,7 +52,10 @@ struct Weights<4> {
 // What a lane reads in the place of an F16 weight block past the row's last.
 static __device__ const h8_t zero_weights = {0, 0, 0, 0, 0, 0, 0, 0};
 
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
+// FEW: at most 8 input rows, one per wave: the other half of the 16 columns is not loaded, normalised or stored. (8 rows, two per
+// wave -> one: QKV with its norm, 5120 x 3072 F16 10.1 -> 9.3 us, Q8_0 10.1 -> 9.0, Q4_0 10.0 -> 8.3; 1152 x 896 F16 4.8 -> 4.4;
+// 3072 x 3072 without a norm 6.5 -> 5.8, 6.0 -> 5.5, 6.4 -> 5.1.)
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW>
 __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     static_assert(std::is_trivially_copyable<PanelDev>::value, "read as raw bytes from the argument block, where it is the first member");
@@ -60,7 +63,13 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     (void)a_by_value;
     typedef Weights<WB> W;
     typedef typename W::raw_t raw_t;
-    constexpr int XROW = row_bytes<PK>(), NR = 2 * NC, NB = 2 * PK;
+    constexpr int XROW = row_bytes<PK>(), NR = FEW ? 1 : 2 * NC, NB = 2 * PK;
+    static_assert(!FEW || NC == 1, "one group of input rows");
+    // The order of the first requests is input rows, the norm's weights, scales, weights. Loads complete in the order in which they
+    // are issued; left to itself the compiler puts the weights ahead of the rows in most of the kernels, and what is done with
+    // the rows then waits for the whole weight stream. (m 12 .. 32, K 2048 .. 3072: o_proj 4 to 14 % less. With the longest rows and a
+    // norm of two rows per wave the norm's chain is longer than the weights' stream, and the compiler's mixture is 1 to 3 % better.)
+    constexpr bool ORDERED = FEW || !ROPE || PK <= 4;
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
@@ -107,26 +116,35 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     // ---- input rows of a pass: rows wave, wave + 8, ... of it (a row past the chunk's last re-reads the last: its column is not
     // stored), piece j of a row = features 512 j + 8 lane ..
     h8_t xr[NR][PK];
-    auto request_rows = [&](uint32_t pass) __attribute__((always_inline)) {
+    auto request_rows = [&](uint32_t pass, bool first) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
+            if (i > (first ? 1 : 0) && pass * (NC * 16u) + 8u * i >= m_rows) break;  // (uniform: no such rows in the pass; the first one is not waited for)
             const __half *row = x_in + (size_t)min(pass * (NC * 16u) + (uint32_t)wave + 8u * i, m_rows - 1u) * K;
 #pragma unroll
             for (int j = 0; j < PK; ++j) xr[i][j] = *reinterpret_cast<const h8_t *>(row + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
         }
     };
     uint32_t pass = blockIdx.y;
-    request_rows(pass);
+    request_rows(pass, true);
+    if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
     h8_t gv[PK];
+    if constexpr (!ORDERED) {
 #pragma unroll
-    for (int j = 0; j < PK; ++j) gv[j] = *reinterpret_cast<const h8_t *>((gamma ? gamma : x_in) + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
-    // (the longest rows leave no registers for the norm's weights through the passes: they wait in LDS, behind the rows; every
-    // wave writes them all, so no wave waits for another's)
+        for (int j = 0; j < PK; ++j) gv[j] = *reinterpret_cast<const h8_t *>((gamma ? gamma : x_in) + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
+    } else if (gamma) {
+#pragma unroll
+        for (int j = 0; j < PK; ++j) gv[j] = *reinterpret_cast<const h8_t *>(gamma + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
+    } else {
+#pragma unroll
+        for (int j = 0; j < PK; ++j) gv[j] = h8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    }
     h8_t *const g_lds = reinterpret_cast<h8_t *>(smem + lds_rows_bytes<NT, NC, PK>());
-    if constexpr (G_IN_LDS<PK>) {
+    if (G_IN_LDS<PK> && !ORDERED) {
 #pragma unroll
         for (int j = 0; j < PK; ++j) g_lds[j * 64 + lane] = gv[j];
     }
+    if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
     // ---- block scales (block-quantised weights): [block][slot] f16 in LDS, fetched along the rows of the scale matrix, two at a
     // time where a row holds an even number (per lane and block of the operand they were 16 lines to a request). Past the last block
     // they are zero: an infinite scale would make NaN of the input's zeros there.
@@ -155,6 +173,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             }
         }
     }
+    if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
     // ---- all weights of the workgroup. F16 (and SUMS, Q8_0): block kb of slot (t, n), features 8c .. 8c + 7. Block-quantised: 16
     // bytes per lane, half a block of one of two (Q8_0) or a block of four (Q4_0); the features that lane c holds for step s of such
     // a request follow from that, for the weights and for the input rows alike. SUMS wants a block in all lanes of a row: with Q4_0
@@ -202,6 +221,11 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             wv[t][i] = fa_norm::load_global_once<req_t>(p);
         }
     }
+    if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
+    if (G_IN_LDS<PK> && ORDERED && gamma) {
+#pragma unroll
+        for (int j = 0; j < PK; ++j) g_lds[j * 64 + lane] = gv[j];
+    }
     const float eps = a.eps, inv_k = a.inv_k, alpha = a.alpha, beta = a.beta;
     const __half *const residual = a.residual;
     const __half *const bias0 = a.bias[0], *const bias1 = a.bias[1], *const bias2 = a.bias[2];
@@ -234,6 +258,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         if (gamma) {  // x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16; a wave holds whole rows
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
+                if (i > 0 && 8u * i >= cols) break;  // (uniform: no such rows in this pass. QKV of 18 .. 24 rows: 5 to 9 % less)
                 float ss = 0.0f;
 #pragma unroll
                 for (int j = 0; j < PK; ++j) {
@@ -293,7 +318,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 s_res[t] = fa_norm::load_global<_Float16>(
                     residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * pick3(s_mat[t], rows0, rows1, rows1) + s_row[t] : x_in);
         }
-        if (next < n_pass) request_rows(next);
+        if (next < n_pass) request_rows(next, false);
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
             if (TURN && pass == blockIdx.y) {
@@ -407,31 +432,33 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     }
 }
 
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS>
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW>
 fa_status launch_one(FaLaunchScope &scope, dim3 grid, const PanelDev &a) {
     constexpr int lds = lds_bytes<WB, NT, NC, PK, SUMS>();
     static std::atomic<uint64_t> allowed{0};  // devices this kernel's LDS size has been asked for on (the calls are idempotent)
     const uint64_t bit = 1ull << (scope.ctx->device & 63);
     if (!(allowed.load(std::memory_order_acquire) & bit)) {
-        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         allowed.fetch_or(bit, std::memory_order_release);
     }
-    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS>, grid, dim3(NTHREADS), lds, a);
+    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW>, grid, dim3(NTHREADS), lds, a);
     return FA_OK;
 }
-template <int WB, int NT, int NC, bool SUMS>
+template <int WB, int NT, int NC, bool SUMS, bool FEW>
 fa_status launch_pk(FaLaunchScope &scope, bool rope, uint32_t pk, dim3 grid, const PanelDev &a) {
-    if (pk <= 2) return rope ? launch_one<WB, NT, NC, 2, true, SUMS>(scope, grid, a) : launch_one<WB, NT, NC, 2, false, SUMS>(scope, grid, a);
-    if (NC == 2 || pk <= 4) return rope ? launch_one<WB, NT, NC, 4, true, SUMS>(scope, grid, a) : launch_one<WB, NT, NC, 4, false, SUMS>(scope, grid, a);
-    return rope ? launch_one<WB, NT, 1, 6, true, SUMS>(scope, grid, a) : launch_one<WB, NT, 1, 6, false, SUMS>(scope, grid, a);  // (16 rows per pass: registers)
+    if (pk <= 2) return rope ? launch_one<WB, NT, NC, 2, true, SUMS, FEW>(scope, grid, a) : launch_one<WB, NT, NC, 2, false, SUMS, FEW>(scope, grid, a);
+    if (NC == 2 || pk <= 4) return rope ? launch_one<WB, NT, NC, 4, true, SUMS, FEW>(scope, grid, a) : launch_one<WB, NT, NC, 4, false, SUMS, FEW>(scope, grid, a);
+    return rope ? launch_one<WB, NT, 1, 6, true, SUMS, FEW>(scope, grid, a) : launch_one<WB, NT, 1, 6, false, SUMS, FEW>(scope, grid, a);  // (16 rows per pass: registers)
 }
 template <int WB>
 fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a) {
-    if constexpr (WB != 16) {
-        if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true>(scope, rope, pk, grid, a);
+    constexpr bool Q = WB != 16;  // (block-quantised weights have per-block sums wherever there are as few rows)
+    if (a.m <= 8 && (!Q || sums)) return nt == 1 ? launch_pk<WB, 1, 1, Q, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, Q, true>(scope, rope, pk, grid, a);
+    if constexpr (Q) {
+        if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true, false>(scope, rope, pk, grid, a);
     }
-    if (nt == 1) return nc == 1 ? launch_pk<WB, 1, 1, false>(scope, rope, pk, grid, a) : launch_pk<WB, 1, 2, false>(scope, rope, pk, grid, a);
-    return nc == 1 ? launch_pk<WB, 2, 1, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 2, false>(scope, rope, pk, grid, a);
+    if (nt == 1) return nc == 1 ? launch_pk<WB, 1, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 1, 2, false, false>(scope, rope, pk, grid, a);
+    return nc == 1 ? launch_pk<WB, 2, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 2, false, false>(scope, rope, pk, grid, a);
 }
 
 }  // namespace fa_panel

@@ -91,3 +91,12 @@ def test_q4_weights_turned_into_operand_order(K, N, NK, m, layout):
     """Q4_0 with per-block sums (2 to 11 rows): the weights of four blocks go through LDS from the longest rows that do not, with one,
     two, three and four blocks in a row's last request, one and two tiles of weight rows, both layouts."""
     test_chunk_in_one_launch(K, N, NK, m, layout, "q4")
+
+
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m", [(96, 40, 24, 8), (96, 40, 24, 9), (1056, 72, 8, 8), (1056, 72, 8, 24), (2080, 40, 24, 8), (2080, 40, 24, 9), (2080, 264, 72, 24),
+                                      (2048, 72, 8, 25), (2080, 40, 16, 25), (896, 64, 32, 40), (896, 64, 32, 73), (3072, 4136, 1024, 8)])
+def test_rows_absent_from_a_pass(K, N, NK, m, weights):
+    """A wave's rows of a pass are asked for and normalised only where they are there, and there is a form for a single row per wave:
+    one row group less than a pass holds and one row more, in a first, a second and a last pass, rows of two, four and six pieces."""
+    test_chunk_in_one_launch(K, N, NK, m, 1, weights)
