@@ -509,8 +509,10 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
         const float cost = (float)((tiles + n_cus - 1) / n_cus) * (l.weight_bits == 16 ? c.f16 : c.quantised);
         if (best == 0.0f || cost < best) {
             best = cost, shape = c.shape;
-            // With a workgroup or less per CU, the block-quantised form keeps twice as many of its smaller stages on their way.
-            if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && tiles <= n_cus && l.k_dim <= 8192) shape = fa_tile::TILE_64x64_DEEP;
+            // With a workgroup or less per CU, the block-quantised form has stages for each wave, or keeps twice as many of its smaller
+            // stages on their way (both measured in fa_tile.h; LDS beside the scales: up to 4096 and 8192 features).
+            if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && tiles <= n_cus && l.k_dim <= 8192)
+                shape = l.k_dim >= 1024 && l.k_dim <= 4096 ? fa_tile::TILE_64x64_OWN : fa_tile::TILE_64x64_DEEP;
         }
     }
     return best;

@@ -20,6 +20,13 @@
 //     tile share the features of a step instead of the input rows (KG) where the tile is small (283 rows, 3072 x 2048 Q8_0:
 //     13.0 -> 9.7 us), and their sums meet in the write stage. The scales of the tile's rows are all in LDS from the start:
 //     a request for 4 bytes of each row would cost the memory unit as much as one for 16 (15.4 -> 13.0 us).
+//     With a workgroup or less per CU and 1024 features or more each wave takes the whole 64 x 64 tile for every fourth step, from
+//     stages of its own (OWN): nothing is waited for but the wave's own requests, an operand is read from LDS once per tile and not
+//     once per wave that shares it, and each weight is still converted once. A step is 0.13 to 0.16 us per CU instead of 0.20 (64 to
+//     256 tiles): o_proj 200 rows, 2048 features x 1024 Q8_0 8.9 -> 8.2 us, Q4_0 9.4 -> 8.1; 3072 x 4096 13.4 -> 12.4, 13.9 -> 12.4;
+//     FusedQkv 300 rows, 2560 x 2048 14.9 -> 13.9, 14.8 -> 13.3. Below 1024 features what it adds - the first steps of four waves
+//     arrive together, four partial tiles meet in the write stage - outweighs that (896: Q8_0 6.4 -> 6.8), above 4096 the scales
+//     leave room for two stages (5120: 17.8 -> 20.0). Steps of 32 features and eight waves: 5 to 10 % slower (half lines per request).
 //   * a 32 x 32 x 16 matrix instruction rounds its running sum twice, so a chain's error grows with the root of its length: over 3072
 //     features 5.9 x 2^-24 of the sums' size. F16 tiles of up to 128 x 128, which took the place of parts of a few hundred features
 //     added in a second launch (2.2 x 2^-24), add their accumulators to a second set every FOLD steps, between the products, for
@@ -51,35 +58,40 @@ typedef uint32_t u2v_t __attribute__((ext_vector_type(2)));
 //
 // WB bits per weight; WM x WN waves over (input rows, weight rows), each of them KG times, for a share of every 64 features; a wave
 // owns TM x TN tiles of 32 x 32; NS stages of 64 features.
-template <int WB_, bool CANON_, int WM_, int WN_, int KG_, int TM_, int TN_, int NS_, bool JOINED_ = false>
+template <int WB_, bool CANON_, int WM_, int WN_, int KG_, int TM_, int TN_, int NS_, bool JOINED_ = false, bool OWN_ = false>
 struct Shape {
     static constexpr int WB = WB_, WM = WM_, WN = WN_, KG = KG_, TM = TM_, TN = TN_, NS = NS_;
     static constexpr bool CANON = CANON_, QUANT = WB_ != 16;
     // The tiles run over the rows of all matrices as one list (F16; whole groups of 32 rows per matrix): a tile may hold rows of two.
     static constexpr bool JOINED = JOINED_;
     static_assert(!JOINED || WB == 16, "F16 only");
+    // Each wave has the whole tile, stages of its own and every KG-th step: no wave waits for another before the write stage.
+    static constexpr bool OWN = OWN_;
+    static_assert(!OWN || (QUANT && WM == 1 && WN == 1 && KG == 4), "16 bytes of a row's scales are those of a step of each wave");
     static constexpr int FOLD = WB_ == 16 && WM_ * TM_ * WN_ * TN_ <= 16 ? 4 : 0;  // steps, 0: one chain
-    static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = 4 / KG;  // KN: products of 16 features per wave and stage
+    static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = OWN ? 4 : 4 / KG, LOADERS = OWN ? 1 : NW;  // KN: products of 16 features per wave and stage
     static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
     static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
-    static constexpr int XR = X_BYTES / 1024 / NW;  // 1 KiB requests per wave and stage
-    static constexpr int W_REQ = W_BYTES / 1024, WR = W_REQ >= NW ? W_REQ / NW : 1;
-    static constexpr int REQ = XR + WR;
+    static constexpr int XR = X_BYTES / 1024 / LOADERS;  // 1 KiB requests per wave and stage
+    static constexpr int W_REQ = W_BYTES / 1024, WR = W_REQ >= LOADERS ? W_REQ / LOADERS : 1;
+    static constexpr int REQ = XR + WR, ALL_STAGES = (OWN ? NW : 1) * NS * STAGE;
     // what a lane reads of a weight row at a time: the 8 features of a product, of both halves of the wave where they are 4 bytes
     typedef typename std::conditional<WB_ == 16, h8_t, u2v_t>::type raw_t;
     static constexpr int READS = KN * (TM + TN);
-    static constexpr int T_STRIDE = NTR * 4 + 16, T_BYTES = WM * 32 * T_STRIDE;
+    static constexpr int TJ = OWN ? TM : 1;  // 32-row groups of every wave that the write stage turns at a time
+    static constexpr int T_STRIDE = NTR * 4 + 16, T_BYTES = WM * TJ * 32 * T_STRIDE;
     // LDS: the stages, then (block-quantised) all scales of the tile's rows, [8 blocks][row]; the write stage over both
     static constexpr uint32_t scale_bytes(uint32_t k_dim) { return QUANT ? (k_dim + 255) / 256 * (NTR * 16) : 0u; }
     static constexpr uint32_t lds_bytes(uint32_t k_dim) {
-        const uint32_t s = NS * STAGE + scale_bytes(k_dim);
+        const uint32_t s = ALL_STAGES + scale_bytes(k_dim);
         return s > (uint32_t)(KG * T_BYTES) ? s : (uint32_t)(KG * T_BYTES);
     }
-    static_assert(X_BYTES % (1024 * NW) == 0 && (W_REQ % NW == 0 || NW % W_REQ == 0), "whole requests per wave");
+    static_assert(X_BYTES % (1024 * LOADERS) == 0 && (W_REQ % LOADERS == 0 || LOADERS % W_REQ == 0), "whole requests per wave");
     static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63 && NTR >= 64, "LDS of a compute unit; the request counter");
 };
 
-enum TileShape { TILE_64x64_DEEP, TILE_64x64, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };  // input rows x weight rows (the first: block-quantised, more stages)
+// input rows x weight rows (the first two: block-quantised, stages of each wave's own and more stages)
+enum TileShape { TILE_64x64_OWN, TILE_64x64_DEEP, TILE_64x64, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };
 
 template <int N>
 __device__ __forceinline__ void wait_requests() {
@@ -97,10 +109,12 @@ template <class S, int MIN_WAVES>
 __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     typedef __attribute__((address_space(3))) void *lds_ptr;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)smem;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int loader = S::OWN ? 0 : wave;  // which of the requests of a step are this wave's
+    const uint32_t own = S::OWN ? wave * (S::NS * S::STAGE) : 0;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr)smem + own;
     const int wn = wave % S::WN, wm = wave / S::WN % S::WM, kg = wave / (S::WN * S::WM);
-    const uint32_t K = a.k_dim, n_steps = K / 64;
+    const uint32_t K = a.k_dim, n_steps = S::OWN ? (K / 64 + 3 - wave) / 4 : K / 64;  // (this wave's)
 
     // Tile of this workgroup. Workgroup ids go round the 8 XCDs; the ids of one XCD are given consecutive tiles (weight rows
     // outermost), so that a weight tile is fetched into one L2 only.
@@ -145,13 +159,13 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     int xv[S::XR], wv[S::WR];
 #pragma unroll
     for (int i = 0; i < S::XR; ++i) {
-        const uint32_t row = (wave * S::XR + i) * 8 + (lane >> 3);
+        const uint32_t row = (loader * S::XR + i) * 8 + (lane >> 3);
         xv[i] = (int)(row * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
     }
     uint32_t w_block[S::WR];  // canonical: which of the stage's two 32-feature blocks
 #pragma unroll
     for (int i = 0; i < S::WR; ++i) {
-        const uint32_t q = (wave * S::WR + i) % S::W_REQ;
+        const uint32_t q = (loader * S::WR + i) % S::W_REQ;
         w_block[i] = 0;
         if constexpr (S::CANON) {
             constexpr uint32_t PER_BLOCK = S::W_REQ / 2;
@@ -203,12 +217,15 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     }
     // What the next step's requests start from: byte offsets that grow by the same amount per step. (Past the last step the
     // descriptors are made empty: nothing is read, zeros arrive, and the counts that the waits go by stay the same.)
-    uint32_t asked = 0, x_soff = 0, w_soff = 0;
+    constexpr uint32_t STRIDE = S::OWN ? 4 : 1;  // steps between two of this wave's
+    const uint32_t w_per_step = S::CANON ? 2 * w_block_bytes : 8 * S::WB;
+    uint32_t asked = 0, x_soff = S::OWN ? wave * 128 : 0, w_soff = S::OWN ? wave * w_per_step : 0;
     fa_lds_dma::rsrc_words x_now = x_rs, w_now = w_rs;
+    if (S::OWN && n_steps == 0) x_now.z = 0u, w_now.z = 0u;
     auto request = [&](int r, uint32_t stage) __attribute__((always_inline)) {
         const uint32_t base = lds_base + stage;
         if (r < S::WR) {
-            const uint32_t q = (wave * S::WR + r) % S::W_REQ;
+            const uint32_t q = (loader * S::WR + r) % S::W_REQ;
             if constexpr (S::JOINED) {
                 fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], 0);
                 wv[r] += w_step[r];
@@ -217,10 +234,10 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                 fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
             }
         } else {
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, base + (wave * S::XR + r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, base + (loader * S::XR + r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
         }
         if (r == S::REQ - 1) {  // the step's last one
-            ++asked, x_soff += 128, w_soff += S::CANON ? 2 * w_block_bytes : 8 * S::WB;
+            ++asked, x_soff += STRIDE * 128, w_soff += STRIDE * w_per_step;
             const bool in = asked < n_steps;
             x_now.z = in ? x_rs.z : 0u, w_now.z = in ? w_rs.z : 0u;
         }
@@ -234,7 +251,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     constexpr uint32_t W_TILE = S::WB == 16 ? (S::CANON ? 2048 : 4096) : S::WB == 8 ? (S::CANON ? 1024 : 2048) : (S::CANON ? 512 : 1024);
 #pragma unroll
     for (int q = 0; q < S::KN; ++q) {
-        const uint32_t kk = kg * S::KN + q, b = kk >> 1, half = kk & 1;
+        const uint32_t kk = (S::OWN ? 0 : kg * S::KN) + q, b = kk >> 1, half = kk & 1;
         x_at[q] = wm * S::TM * 4096 + (r32 >> 3) * 1024 + (r32 & 7) * 128 + ((2 * kk + h) ^ ((r32 >> 1) & 7)) * 16;
         if constexpr (S::WB == 16) {
             w_at[q] = S::CANON ? b * (S::NTR * 64) + (w_row >> 4) * 1024 + (w_row & 15) * 64 + ((2 * half + h) ^ ((w_row >> 2) & 3)) * 16
@@ -254,15 +271,18 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     };
     auto fetch = [&](Operands &o, uint32_t stage, int e) __attribute__((always_inline)) {  // read number e of the stage
         const int q = e / (S::TM + S::TN), t = e % (S::TM + S::TN);
-        if (t < S::TM) o.x[t][q] = *reinterpret_cast<const h8_t *>(smem + x_at[q] + stage + t * 4096);
-        else o.w[t - S::TM][q] = *reinterpret_cast<const typename S::raw_t *>(smem + w_at[q] + stage + (t - S::TM) * W_TILE);
+        if (t < S::TM) o.x[t][q] = *reinterpret_cast<const h8_t *>(smem + own + x_at[q] + stage + t * 4096);
+        else o.w[t - S::TM][q] = *reinterpret_cast<const typename S::raw_t *>(smem + own + w_at[q] + stage + (t - S::TM) * W_TILE);
     };
     u4v_t scales[S::TN] = {};  // of the wave's rows, 8 blocks = 4 stages
-    const unsigned char *scale_at = smem + S::NS * S::STAGE + w_row * 16;
+    const unsigned char *scale_at = smem + S::ALL_STAGES + w_row * 16 + (S::OWN ? wave * 4 : 0);
     auto fetch_scales = [&]() __attribute__((always_inline)) {
         if constexpr (S::QUANT) {
 #pragma unroll
-            for (int i = 0; i < S::TN; ++i) scales[i] = *reinterpret_cast<const u4v_t *>(scale_at + i * 512);
+            for (int i = 0; i < S::TN; ++i) {
+                if constexpr (S::OWN) scales[i].x = *reinterpret_cast<const uint32_t *>(scale_at + i * 512);
+                else scales[i] = *reinterpret_cast<const u4v_t *>(scale_at + i * 512);
+            }
             scale_at += S::NTR * 16;
         }
     };
@@ -270,10 +290,10 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         if constexpr (S::WB == 16) {
             return o.w[i][q];
         } else {
-            const uint32_t pair = scales[i][ks4];  // (a copy: the bit cast of a vector's element takes element 0)
+            const uint32_t pair = scales[i][S::OWN ? 0 : ks4];  // (a copy: the bit cast of a vector's element takes element 0)
             const h2v_t s2 = __builtin_bit_cast(h2v_t, pair);
             _Float16 s;
-            if constexpr (S::KG == 1) s = s2[q >> 1];
+            if constexpr (S::KN == 4) s = s2[q >> 1];
             else if constexpr (S::KG == 2) s = kg ? s2[1] : s2[0];
             else s = kg >= 2 ? s2[1] : s2[0];
             const h8_t sc = {s, s, s, s, s, s, s, s};
@@ -294,7 +314,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         const __half *sp = pick3(tile_mat, a.scales[0], a.scales[1], a.scales[2]);
         const fa_lds_dma::rsrc_words s_rs = fa_lds_dma::make_rsrc_words(sp, N_tile * (K / 32) * 2);
         for (uint32_t q = wave; q < (K + 255) / 256 * (S::NTR / 64); q += S::NW)
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base + S::NS * S::STAGE + q * 1024, (int)(weight_row(q % (S::NTR / 64) * 64 + lane) * (K / 32) * 2),
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base - own + S::ALL_STAGES + q * 1024, (int)(weight_row(q % (S::NTR / 64) * 64 + lane) * (K / 32) * 2),
                                                     (int)(q / (S::NTR / 64) * 16));
     }
 #pragma unroll
@@ -312,9 +332,10 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     // requests in one go leaves its matrix core idle for as long.
     auto step = [&](uint32_t cur, uint32_t next, int ks4, bool fold, const Operands &now, Operands &then) __attribute__((always_inline)) {
         wait_requests<S::REQ *(S::NS - 2)>();
-        meet();
+        if constexpr (S::OWN) __builtin_amdgcn_s_waitcnt(0xC07F);  // (lgkmcnt(0): the operands have left the stage that is asked for again)
+        else meet();
         constexpr int NM = S::KN * S::TN * S::TM;
-        if (ks4 == 0) fetch_scales();
+        if (S::OWN || ks4 == 0) fetch_scales();
         h8_t fa[S::TN];
 #pragma unroll
         for (int p = 0; p < NM; ++p) {
@@ -332,9 +353,10 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         }
     };
     // (unrolled over the stages, so that their places are constants; operands of even and odd steps in registers of their own)
-    constexpr int UNROLL = S::QUANT || S::FOLD ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
+    constexpr int UNROLL = (S::QUANT && !S::OWN) || S::FOLD ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
     for (uint32_t left = n_steps;;) {
         bool done = false;
+        if (S::OWN && left == 0) break;  // (a wave without a step)
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
             const uint32_t cur = u % S::NS * S::STAGE, next = (u + 1) % S::NS * S::STAGE;
@@ -359,21 +381,23 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     // Write stage: accumulators -> LDS as f32 [input row][weight row], 32 input rows of every wave at a time, then
     // alpha * sum + bias + beta * residual, one rounding to f16, 16-byte stores (or the rotation and the stores of KvPrepFused).
 #pragma unroll
-    for (int j = 0; j < S::TM; ++j) {
+    for (int j0 = 0; j0 < S::TM; j0 += S::TJ) {
         __syncthreads();  // every wave is done with the stages / the previous rows have been read out
         // register r of lane l of a 32 x 32 tile is weight row 8 (r / 4) + 4 (l / 32) + r % 4 and input row l % 32
 #pragma unroll
-        for (int i = 0; i < S::TN; ++i)
+        for (int j = j0; j < j0 + S::TJ; ++j)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
-                *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + (wm * 32 + r32) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + g * 8 + h * 4) * 4) = q;
-            }
+            for (int i = 0; i < S::TN; ++i)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+                    *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + ((wm * S::TJ + j - j0) * 32 + r32) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + g * 8 + h * 4) * 4) = q;
+                }
         __syncthreads();
         constexpr int PIECES = S::NTR / 8;
-        for (uint32_t q = tid; q < (uint32_t)(S::WM * 32 * PIECES); q += S::NT) {
+        for (uint32_t q = tid; q < (uint32_t)(S::WM * S::TJ * 32 * PIECES); q += S::NT) {
             const uint32_t t = q / PIECES, n8 = q % PIECES;
-            const uint32_t gm = m0 + ((t >> 5) * S::TM + j) * 32 + (t & 31);
+            const uint32_t gm = m0 + ((t >> 5) / S::TJ * S::TM + j0 + (t >> 5) % S::TJ) * 32 + (t & 31);
             uint32_t r = n0 + n8 * 8;
             const int mat = matrix_of(r);
             const uint32_t gn = paired(r), N = S::JOINED ? (mat ? rows1 : rows0) : N_tile;
@@ -434,6 +458,7 @@ template <int WB, bool CANON>
 fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDev &a) {
     if constexpr (WB == 16) {
         switch (shape) {
+            case TILE_64x64_OWN:
             case TILE_64x64_DEEP:
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 1, 1, 4>, 2>(ctx, scope, a);
             case TILE_128x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 2, 1, 3>, 2>(ctx, scope, a);
@@ -443,6 +468,7 @@ fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDe
         }
     } else {
         switch (shape) {
+            case TILE_64x64_OWN: return launch_shape<Shape<WB, CANON, 1, 1, 4, 2, 2, 3, false, true>, 1>(ctx, scope, a);
             case TILE_64x64_DEEP: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 8>, 1>(ctx, scope, a);
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 4>, 2>(ctx, scope, a);
             case TILE_128x64: return launch_shape<Shape<WB, CANON, 1, 2, 4, 4, 1, 4>, 2>(ctx, scope, a);

@@ -73,6 +73,27 @@ def test_tiles(K, H, Hkv, D, m, layout, weights):
         b.free()
 
 
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
+    (960, 2, 1, 64, 65, 1),       # the last length whose steps the waves of a tile share
+    (1024, 2, 1, 64, 65, 1),      # four steps for each wave, a second tile of one row
+    (1088, 1, 1, 128, 64, 0),     # a step more for one wave
+    (1152, 3, 1, 64, 130, 1),     # for two of four; scales of four and a half units
+    (1216, 5, 1, 64, 12, 0),      # for three, a ragged tile
+    (2112, 2, 2, 128, 33, 1),
+    (4096, 1, 1, 64, 70, 0),      # all of a compute unit's LDS
+    (4096, 1, 1, 128, 20, 1),
+    (4160, 1, 1, 64, 20, 1),      # past it
+])
+def test_tiles_with_steps_of_each_waves_own(K, H, Hkv, D, m, layout, weights):
+    """Block-quantised 64 x 64 tiles: every wave has every fourth step of 64 features from 1024 to 4096 of them."""
+    ctx().set_gemm_variant(3)
+    try:
+        test_tiles(K, H, Hkv, D, m, layout, weights)
+    finally:
+        ctx().set_gemm_variant()
+
+
 @pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
 @pytest.mark.parametrize("K,N,NK,m,panel,finish", [
     (2048, 8192, 1024, 16, True, False),    # one round of workgroups: the panel up to 32 rows
