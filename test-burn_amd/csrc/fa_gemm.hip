@@ -483,7 +483,11 @@ __global__ void __launch_bounds__(256) gemm_finish_kernel(GemmDev a) {
 // The cheapest tile shape for a launch over rows[i] weight rows per matrix, and its cost: what a tile of each shape takes per step of
 // 64 features with one workgroup on every CU, in units of the 64 x 64 tile's 0.21 us (from launches of 160 to 256 tiles over 3072
 // features), times the rounds of workgroups that the launch has. The larger tiles read less per product, the smaller ones leave
-// fewer CUs idle. `joined`: tiles may hold rows of two matrices. `variant`: a shape asked for by name (fa_set_gemm_variant).
+// fewer CUs idle: 64 x 96 is for 257 to 384 tiles of 64 x 64, which are one round of it (576 rows, 3072 x 2048 F16: 18.4 us as two
+// rounds or as 128 x 64, 16.0 as 64 x 96; 500 rows 3072 x 3072, with a residual, 19.5 -> 15.9, Q8_0 17.6 -> 16.4, Q4_0 17.0 -> 15.4). Three rounds
+// and more of 64 x 96, and of any small F16 tiles, take longer than their number says (1530 rows, 2048 x 3072 F16: 30.4 us in three
+// rounds of 64 x 96, 26.3 in one of 256 x 128; 1300 rows, 3072 x 3072 37.7 in four of 64 x 64, 33.7). Over 730 launches of 130 to 2200
+// rows the choice is on average within 0.1 % (F16), 0.5 % (block-quantised) of the best shape, 1.5 to 2 % without 64 x 96. `joined`: tiles may hold rows of two matrices. `variant`: a shape asked for by name (fa_set_gemm_variant).
 static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint32_t n_cus, bool joined, uint32_t variant, fa_tile::TileShape &shape) {
     struct Choice {
         fa_tile::TileShape shape;
@@ -491,6 +495,7 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
         float f16, quantised;
     };
     static const Choice choices[] = {{fa_tile::TILE_64x64, 64, 64, 1.0f, 1.0f},
+                                     {fa_tile::TILE_64x96, 64, 96, 1.4f, 1.4f},
                                      {fa_tile::TILE_128x64, 128, 64, 1.75f, 1.64f},
                                      {fa_tile::TILE_128x128, 128, 128, 2.6f, 2.7f},
                                      {fa_tile::TILE_256x128, 256, 128, 4.65f, 4.3f},
@@ -506,7 +511,9 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
         for (int i = 0; i < 3; ++i) n_tiles += ceil_div_u32(rows[i], c.n);
         if (c.shape == fa_tile::TILE_256x160) n_tiles = ceil_div_u32(rows[0] + 2 * rows[1], c.n);
         const uint64_t tiles = (uint64_t)n_tiles * ceil_div_u32(l.m, c.m);
-        const float cost = (float)((tiles + n_cus - 1) / n_cus) * (l.weight_bits == 16 ? c.f16 : c.quantised);
+        const uint64_t rounds = (tiles + n_cus - 1) / n_cus;
+        float cost = (float)rounds * (l.weight_bits == 16 ? c.f16 : c.quantised);
+        if (rounds >= 3 && (c.shape == fa_tile::TILE_64x96 || (l.weight_bits == 16 && c.m * c.n < 128 * 128))) cost *= 1.2f;
         if (best == 0.0f || cost < best) {
             best = cost, shape = c.shape;
             // With a workgroup or less per CU, the block-quantised form has stages for each wave, or keeps twice as many of its smaller

@@ -11,9 +11,10 @@
 //     barrier they leave the matrix cores idle. They are spread between the products (256 x 160: 98 -> 66 us at 2048 rows,
 //     5120 x 3072, where the split-K form took 74.7).
 //   * large launches read less per product with larger tiles but leave CUs idle where the tiles do not fill a round of
-//     workgroups: five shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 (F16) fills a round where
+//     workgroups: six shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 (F16) fills a round where
 //     256 x 128 leaves a fifth of the chip to a second one - 8.4 to 10.5 million outputs, such as 2048 rows x 5120, and again at
-//     twice that - and may hold rows of two matrices (JOINED).
+//     twice that - and may hold rows of two matrices (JOINED). 64 x 96 does so for a quarter to a half more outputs than 64 x 64 have
+//     room for. (128 x 96: no faster than 128 x 128 with a third more workgroups, 22.0 us for 700 rows of 3072 x 3072.)
 //   * block-quantised weights stay as they are up to the registers, where a wave turns its operands to f16 right in front of the
 //     product (f16(weight * scale), as the reference's tile loader: see fa_gemm.hip). That is 14 vector instructions per 8
 //     weights, and with one wave per SIMD they add to the chain; so that no two waves convert the same weights, the waves of a
@@ -72,8 +73,10 @@ struct Shape {
     static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = OWN ? 4 : 4 / KG, LOADERS = OWN ? 1 : NW;  // KN: products of 16 features per wave and stage
     static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
     static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
-    static constexpr int XR = X_BYTES / 1024 / LOADERS;  // 1 KiB requests per wave and stage
-    static constexpr int W_REQ = W_BYTES / 1024, WR = W_REQ >= LOADERS ? W_REQ / LOADERS : 1;
+    // 1 KiB requests of a stage, and per wave (where they do not divide, some are made twice)
+    static constexpr int X_REQ = X_BYTES / 1024, XR = (X_REQ + LOADERS - 1) / LOADERS;
+    static constexpr bool X_EVEN = X_REQ % LOADERS == 0;
+    static constexpr int W_REQ = W_BYTES / 1024, WR = (W_REQ + LOADERS - 1) / LOADERS;
     static constexpr int REQ = XR + WR, ALL_STAGES = (OWN ? NW : 1) * NS * STAGE;
     // what a lane reads of a weight row at a time: the 8 features of a product, of both halves of the wave where they are 4 bytes
     typedef typename std::conditional<WB_ == 16, h8_t, u2v_t>::type raw_t;
@@ -81,17 +84,17 @@ struct Shape {
     static constexpr int TJ = OWN ? TM : 1;  // 32-row groups of every wave that the write stage turns at a time
     static constexpr int T_STRIDE = NTR * 4 + 16, T_BYTES = WM * TJ * 32 * T_STRIDE;
     // LDS: the stages, then (block-quantised) all scales of the tile's rows, [8 blocks][row]; the write stage over both
-    static constexpr uint32_t scale_bytes(uint32_t k_dim) { return QUANT ? (k_dim + 255) / 256 * (NTR * 16) : 0u; }
+    static constexpr uint32_t scale_bytes(uint32_t k_dim) { return QUANT ? NTR % 64 == 0 ? (k_dim + 255) / 256 * (NTR * 16) : ((k_dim + 255) / 256 * (NTR * 16) + 1023) & ~1023u : 0u; }
     static constexpr uint32_t lds_bytes(uint32_t k_dim) {
         const uint32_t s = ALL_STAGES + scale_bytes(k_dim);
         return s > (uint32_t)(KG * T_BYTES) ? s : (uint32_t)(KG * T_BYTES);
     }
-    static_assert(X_BYTES % (1024 * LOADERS) == 0 && (W_REQ % LOADERS == 0 || LOADERS % W_REQ == 0), "whole requests per wave");
+    static_assert(X_BYTES % 1024 == 0 && W_BYTES % 1024 == 0, "whole requests");
     static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63 && NTR >= 64, "LDS of a compute unit; the request counter");
 };
 
 // input rows x weight rows (the first two: block-quantised, stages of each wave's own and more stages)
-enum TileShape { TILE_64x64_OWN, TILE_64x64_DEEP, TILE_64x64, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };
+enum TileShape { TILE_64x64_OWN, TILE_64x64_DEEP, TILE_64x64, TILE_64x96, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };
 
 template <int N>
 __device__ __forceinline__ void wait_requests() {
@@ -159,7 +162,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     int xv[S::XR], wv[S::WR];
 #pragma unroll
     for (int i = 0; i < S::XR; ++i) {
-        const uint32_t row = (loader * S::XR + i) * 8 + (lane >> 3);
+        const uint32_t row = (S::X_EVEN ? loader * S::XR + i : (loader * S::XR + i) % S::X_REQ) * 8 + (lane >> 3);
         xv[i] = (int)(row * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16);
     }
     uint32_t w_block[S::WR];  // canonical: which of the stage's two 32-feature blocks
@@ -178,7 +181,13 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                 const uint32_t row = u * 32 + (lane >> 1);
                 wv[i] = (int)(weight_row(row) * 32 + ((lane & 1) ^ ((row >> 3) & 1)) * 16);
             } else {
-                wv[i] = (int)(weight_row(u * 64 + lane) * 16);
+                if constexpr (S::NTR % 64 == 0) {
+                    wv[i] = (int)(weight_row(u * 64 + lane) * 16);
+                } else {  // a block of the tile's rows is not whole KiB: the lanes of a request go over both
+                    const uint32_t at = q * 64 + lane;
+                    wv[i] = (int)(weight_row(at % S::NTR) * 16 + at / S::NTR * (N_tile * 16));
+                    w_block[i] = 0;
+                }
             }
         } else {
             if constexpr (S::WB == 16) {
@@ -234,7 +243,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                 fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
             }
         } else {
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, base + (loader * S::XR + r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, S::X_EVEN ? base + (loader * S::XR + r - S::WR) * 1024 : base + (loader * S::XR + r - S::WR) % S::X_REQ * 1024, xv[r - S::WR], (int)x_soff);
         }
         if (r == S::REQ - 1) {  // the step's last one
             ++asked, x_soff += STRIDE * 128, w_soff += STRIDE * w_per_step;
@@ -313,9 +322,13 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     if constexpr (S::QUANT) {  // all scales first: 16 bytes (8 blocks) of 64 rows per request
         const __half *sp = pick3(tile_mat, a.scales[0], a.scales[1], a.scales[2]);
         const fa_lds_dma::rsrc_words s_rs = fa_lds_dma::make_rsrc_words(sp, N_tile * (K / 32) * 2);
-        for (uint32_t q = wave; q < (K + 255) / 256 * (S::NTR / 64); q += S::NW)
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base - own + S::ALL_STAGES + q * 1024, (int)(weight_row(q % (S::NTR / 64) * 64 + lane) * (K / 32) * 2),
-                                                    (int)(q / (S::NTR / 64) * 16));
+        const uint32_t requests = S::NTR % 64 == 0 ? (K + 255) / 256 * (S::NTR / 64) : S::scale_bytes(K) / 1024;
+        for (uint32_t q = wave; q < requests; q += S::NW) {
+            constexpr uint32_t PER = S::NTR % 64 == 0 ? S::NTR / 64 : 1;  // requests per 16 bytes of all rows, where that is whole ones
+            const uint32_t at = S::NTR % 64 == 0 ? q % PER * 64 + lane : q * 64 + lane, unit = S::NTR % 64 == 0 ? 0u : at / S::NTR;
+            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base - own + S::ALL_STAGES + q * 1024, (int)(weight_row(at % S::NTR) * (K / 32) * 2 + unit * 16),
+                                                    (int)(S::NTR % 64 == 0 ? q / PER * 16 : 0u));
+        }
     }
 #pragma unroll
     for (int s = 0; s < S::NS; ++s)
@@ -461,6 +474,7 @@ fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDe
             case TILE_64x64_OWN:
             case TILE_64x64_DEEP:
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 1, 1, 4>, 2>(ctx, scope, a);
+            case TILE_64x96: return launch_shape<Shape<WB, CANON, 2, 3, 1, 1, 1, 4>, 2>(ctx, scope, a);
             case TILE_128x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 2, 1, 3>, 2>(ctx, scope, a);
             case TILE_128x128: return launch_shape<Shape<WB, CANON, 2, 4, 1, 2, 1, 4>, 2>(ctx, scope, a);
             case TILE_256x128: return launch_shape<Shape<WB, CANON, 4, 2, 1, 2, 2, 3>, 2>(ctx, scope, a);
@@ -471,6 +485,11 @@ fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDe
             case TILE_64x64_OWN: return launch_shape<Shape<WB, CANON, 1, 1, 4, 2, 2, 3, false, true>, 1>(ctx, scope, a);
             case TILE_64x64_DEEP: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 8>, 1>(ctx, scope, a);
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 4>, 2>(ctx, scope, a);
+            case TILE_64x96:
+                if constexpr (WB == 4) {  // (3072 x 3072, 340 rows, canonical and row-major: 16.8 -> 14.8 us, 18.4 -> 15.3; Q8_0 has room for two stages, 16.4 -> 16.9)
+                    if (a.k_dim >= 1024) return launch_shape<Shape<WB, CANON, 1, 1, 4, 2, 3, 3, false, true>, 1>(ctx, scope, a);
+                }
+                return launch_shape<Shape<WB, CANON, 1, 3, 2, 2, 1, 4>, 2>(ctx, scope, a);
             case TILE_128x64: return launch_shape<Shape<WB, CANON, 1, 2, 4, 4, 1, 4>, 2>(ctx, scope, a);
             case TILE_128x128: return launch_shape<Shape<WB, CANON, 1, 4, 2, 4, 1, 4>, 2>(ctx, scope, a);
             case TILE_256x128: return launch_shape<Shape<WB, CANON, 2, 4, 1, 4, 1, 3>, 2>(ctx, scope, a);
