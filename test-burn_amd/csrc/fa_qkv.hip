@@ -401,7 +401,10 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
 // Llama-3.2-3B block with 2 / 4 / 8 / 11 rows: 113 / 113 / 115 / 117 us against 120 / 128 / 137 / 155 with the kernel for up to 16
 // rows). Up to 32 rows whose weight rows fit one round of workgroups always (a default chunk is one launch). Beyond, up to as many as
 // it is measured to beat the tile kernels with where the weight rows suit it - later where those need the normalisation's launch in
-// front (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against 5.1),
+// front (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone, F16: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against
+// 5.1; block-quantised as long as a pass over 16 weight rows has a workgroup of its own, two to a compute unit, 256 rows Q8_0 4.9
+// against 6.0, Q4_0 4.8 against 6.2, 350 rows Q8_0 row-major 6.8 against 5.9; of 256 features only one to a compute unit, 438 rows of
+// 256 x 576 take 1.17 times as long as the tiles),
 // earlier for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer) - unless the GEMM is a tenth ahead by
 // estimate: many weight rows are many passes of the input rows here, or rounds of workgroups. A launch takes the weight stream, and
 // for each pass that a compute unit has one after the other the input rows of that pass, fetched and multiplied and, with a gamma,
@@ -413,7 +416,8 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const uint32_t min_m = ctx->qkv_rows32_min_m ? ctx->qkv_rows32_min_m : PANEL_MIN_M_DEFAULT;
-    const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : 192u) : l.k_dim <= 2048 ? 128u : l.weight_bits == 16 ? 64u : 48u;
+    const bool f16 = l.weight_bits == 16;
+    const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : f16 ? 192u : 512u) : l.k_dim <= 2048 ? 128u : f16 ? 64u : 48u;
     if (min_m > 32 || l.m < min_m || l.m > max_m || l.k_dim > 3072 || l.k_dim % 32 != 0) return false;
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
@@ -421,9 +425,9 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     const PanelPlan p = panel_plan(ctx, l, false, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
     if (l.m <= 32 && p.rounds == 1) return true;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
+    if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
     // passes of a compute unit (with two workgroups on it they share its way to L2)
     const float passes = p.pk > 2 ? (float)(p.rounds * ceil_div_u32(p.n_pass, p.grid_y)) : std::max(1.0f, (float)(p.grid_x * p.n_pass) / (float)n_cus);
-    const bool f16 = l.weight_bits == 16;
     const float k = (float)l.k_dim, mb = k * (float)(l.n_dim + 2 * l.n_kv) * (f16 ? 2.0f : l.weight_bits == 8 ? 1.0625f : 0.5625f) * 1e-6f;
     const float per_pass = (float)p.nc * k / 1024.0f * (f16 ? (l.gamma ? 1.23f : 0.78f) : l.gamma ? 1.47f : 0.94f);
     return fa_gemm_estimate_us(ctx, l) >= 0.9f * (2.5f + (f16 ? 0.09f : 0.115f) * mb + passes * per_pass);

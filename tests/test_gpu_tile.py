@@ -163,6 +163,35 @@ def _quantised(f, rng, K, N, m, weights):
 
 
 @pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,N,m,panel", [
+    (896, 896, 193, True), (896, 896, 288, True),   # up to a pass for each compute unit
+    (896, 896, 289, False),
+    (1024, 512, 512, True), (1024, 512, 513, False),  # the most input rows
+    (1056, 256, 193, False),                          # longer rows
+])
+def test_route_of_a_product_of_many_rows(K, N, m, panel, weights):
+    """Block-quantised weights without a norm: the panel kernel while the passes fit one round of workgroups."""
+    announce("route of a product", K, N, m, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + N + m)
+    x, full, s, dev_w, arg = _quantised(f, rng, K, N, m, weights)
+    res = rng.uniform(-1, 1, (m, N)).astype(np.float16)
+    dx, ds, dres, dout = f.array(x), f.array(s), f.array(res), f.zeros((m, N))
+    f.profile_reset()
+    f.profile_enable(True)
+    try:
+        f.matmul(dx.arg(), arg, dout.arg(), m, N, K, c=dres.arg(), transpose_b=False, beta=0.75, b_scales=ds.arg())
+        f.synchronize()
+        assert f.profile_query("matmul_rows32_kernel")[0] == int(panel) and f.profile_query("matmul_gemm_kernel")[0] == int(not panel)
+    finally:
+        f.profile_enable(False)
+    want = orc.matmul_gemv(x, full, None, res, 0, 32, 1.0, 0.75).astype(np.float64)
+    assert np.all(np.abs(dout.download() - want) <= 2 * np.maximum(np.abs(want), 2.0 ** -10) * 2.0 ** -10 + 1e-4)
+    for b in (dx, ds, dres, dout, dev_w):
+        b.free()
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
 @pytest.mark.parametrize("K,m", [
     (4096, 70), (4160, 70),    # the last row whose scales fit every tile's part of LDS, and the first past it: 64 x 64 tiles
     (8192, 70), (8256, 70),    # ... of eight small stages up to here
