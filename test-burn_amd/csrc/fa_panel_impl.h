@@ -95,13 +95,13 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         pair_begin = row_begin >> 1, pair_end = row_end >> 1;
     }
     // Weight row of slot (tile t, row n of the tile) across the three matrices laid end to end; a slot past the workgroup's
-    // last row gives the workgroup's first row with valid = false. NeoX pairs: tile 0 holds rows of first halves of heads, tile
-    // 1 their mates half a head on.
+    // last row gives the workgroup's first row with valid = false. NeoX pairs: tile 0 (of one tile: its first 8 rows) holds rows of
+    // first halves of heads, tile 1 (the other 8) their mates half a head on.
     auto slot_row = [&](uint32_t t, uint32_t n_, bool &valid) __attribute__((always_inline)) -> uint32_t {
         if (ROPE && neox) {
-            const uint32_t p = pair_begin + n_, pv = p < pair_end ? p : pair_begin;
+            const uint32_t p = pair_begin + (NT == 2 ? n_ : n_ & 7u), pv = p < pair_end ? p : pair_begin;
             valid = p < pair_end;
-            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + (t << half_shift);
+            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + ((NT == 2 ? t : n_ >> 3) << half_shift);
         }
         const uint32_t gr = row_begin + 16u * t + n_;
         valid = gr < row_end;
@@ -400,9 +400,9 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int t = 0; t < NT; ++t) {
                 if constexpr (ROPE) {
                     const uint32_t D = 2u << half_shift, half = 1u << half_shift;
-                    // the mate: the same slot of the other tile (NeoX), or the neighbouring slot = the neighbouring lane
-                    const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], 1, 64);
-                    const _Float16 ym = neox ? y2[NT == 2 ? t ^ 1 : 0] : y_adj;
+                    // the mate: the same slot of the other tile, or 8 slots away in the one (NeoX), or the neighbouring slot
+                    const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], NT == 1 && neox ? 8 : 1, 64);
+                    const _Float16 ym = NT == 2 && neox ? y2[NT == 2 ? t ^ 1 : 0] : y_adj;
                     if (!s_ok[t] || w_col >= cols) continue;
                     const uint32_t hd = s_row[t] & (D - 1u), head = s_row[t] >> (half_shift + 1);
                     const bool first = neox ? hd < half : (hd & 1u) == 0;

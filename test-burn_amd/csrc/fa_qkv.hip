@@ -377,21 +377,28 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 struct PanelPlan {
     uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y, rounds;
 };
-static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope, bool neox_rope) {
+static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope) {
     PanelPlan p;
     const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
     p.pk = ceil_div_u32(l.k_dim, 512), p.nc = l.m <= 16 || p.pk > 4 ? 1u : 2u, p.n_pass = ceil_div_u32(l.m, 16 * p.nc);
     // Weight rows per workgroup: what a pass costs is mostly its input rows, whatever the weight rows, so as few passes as
-    // possible one after the other; of equal choices the fewest weight rows.
+    // possible on a compute unit - one after the other or, in two workgroups, side by side (Qwen2.5-0.5B, 64 rows: o_proj as 448
+    // workgroups of 4 weight rows 5.2 us, as 112 of 16 3.9); of equal choices the fewest weight rows. A second tile of weight rows
+    // costs a fifth of a pass, four fifths where the rows of F16 and Q8_0 weights are K apart and nothing is normalised (180 rows,
+    // 896 x 896: 4.9 us as 336 workgroups of 16, 5.1 as 168 of 32), and a pass with its norm a fifth more beside another.
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    uint32_t best = 0xffffffffu;
+    uint64_t best = ~0ull;
     const uint32_t least = ceil_div_u32(total_rows, n_cus) < 32 ? (ceil_div_u32(total_rows, n_cus) + 1) & ~1u : 32u;
     for (uint32_t rpw : {least, 16u, 32u}) {
-        const uint32_t gx = ceil_div_u32(total_rows, rpw), nt = neox_rope || rpw > 16 ? 2u : 1u;
-        const uint32_t slots = n_cus * (fa_panel::two_per_cu(nt, p.nc, p.pk, rope) ? 2u : 1u);
+        const uint32_t gx = ceil_div_u32(total_rows, rpw), nt = rpw > 16 ? 2u : 1u;
+        const bool two = fa_panel::two_per_cu(nt, p.nc, p.pk, rope);
+        const uint32_t slots = two ? 2 * n_cus : n_cus;
         uint32_t gy = slots / gx;
         gy = gy < 1 ? 1u : gy > p.n_pass ? p.n_pass : gy;
-        const uint32_t cost = ceil_div_u32(gx * gy, slots) * ceil_div_u32(p.n_pass, gy) * (4 + nt);
+        const uint32_t load = two ? std::max(gx * gy, n_cus) : ceil_div_u32(gx * gy, n_cus) * n_cus;
+        const uint32_t tiles = nt == 1 ? 50u : !l.canonical && l.weight_bits != 4 && !l.gamma ? 90u : 60u;
+        const uint32_t beside = two && gx * gy > n_cus && l.gamma ? 12u : 10u;
+        const uint64_t cost = (uint64_t)load * ceil_div_u32(p.n_pass, gy) * tiles * beside;
         if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy, p.rounds = ceil_div_u32(gx * gy, slots);
     }
     return p;
@@ -422,7 +429,7 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
     if (l.m < FA_GEMM_MIN_M_DEFAULT) return true;
-    const PanelPlan p = panel_plan(ctx, l, false, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
+    const PanelPlan p = panel_plan(ctx, l, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
     if (l.m <= 32 && p.rounds == 1) return true;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
@@ -458,7 +465,7 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
         d.table_rows = r.table_rows, d.normal = r.rope_normal ? 1u : 0u, d.apply = r.apply_rope ? 1u : 0u;
         a.block_shift = (d.block_size & (d.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(d.block_size) : 32u;
     }
-    const PanelPlan p = panel_plan(ctx, l, rope != nullptr, rope && !rope->rope_normal);
+    const PanelPlan p = panel_plan(ctx, l, rope != nullptr);
     a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass;
     a.scale_pairs = l.k_dim / 32 % 2 == 0 ? 1u : 0u;
     for (int i = 0; i < 3; ++i)

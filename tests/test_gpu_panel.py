@@ -100,3 +100,56 @@ def test_rows_absent_from_a_pass(K, N, NK, m, weights):
     """A wave's rows of a pass are asked for and normalised only where they are there, and there is a form for a single row per wave:
     one row group less than a pass holds and one row more, in a first, a second and a last pass, rows of two, four and six pieces."""
     test_chunk_in_one_launch(K, N, NK, m, 1, weights)
+
+
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m", [
+    (96, 6, 1, 64, 3),        # a pair of rows per workgroup
+    (1024, 14, 2, 64, 20),    # three
+    (96, 14, 2, 64, 100),     # eight, several passes
+    (2048, 16, 2, 128, 8),    # five
+    (2080, 16, 2, 128, 33),   # eight: passes spread over workgroups
+    (96, 28, 2, 128, 17),     # the most that one tile holds
+    (96, 30, 2, 128, 9),      # past it: two tiles
+])
+def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
+    """Up to 16 weight rows per workgroup, both halves of its NeoX pairs lie in one tile: the fused write stage equals the two ops to
+    the bit, in both pairings."""
+    announce("neox pairs in one tile", K, H, Hkv, D, m, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + H + m)
+    N, NK = H * D, Hkv * D
+    x, g, ws, bs = _data(rng, K, N, NK, m)
+    scales, dev_s = None, []
+    if weights == "f16":
+        dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+        arg = [w.arg() for w in dev_w]
+    else:
+        quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
+        dev_s = [f.array(s) for _, s in quant]
+        scales = [s.arg() for s in dev_s]
+        dev_w = [f.array(orc.to_canonical(q) if weights == "q8" else orc.pack_q4_0(orc.to_canonical(q))) for q, _ in quant]
+        arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev_w, (N, NK, NK))]
+    dx, dg, db = f.array(x), f.array(g), [f.array(b) for b in bs]
+    outs = [f.zeros((m, n)) for n in (N, NK, NK)]
+    cos, sin = fa.rope_tables(5e5, D, m + 3)
+    dcos, dsin = f.array(cos), f.array(sin)
+    rot = [[f.zeros((H, m, D)), f.zeros((Hkv, m + 3, D)), f.zeros((Hkv, m + 3, D))] for _ in range(2)]
+    kw = dict(gamma=dg.arg(), biases=[b.arg() for b in db], layout=1, scales=scales)
+    f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, **kw)
+    for mode in (fa.ROPE_NEOX, fa.ROPE_NORMAL):
+        p = fa.KvPrepFusedParams.make(H, Hkv, D, m, 2, m + 3, mode)
+        f.kv_prep_fused(*[o.arg() for o in outs], *[t.arg() for t in rot[0]], dcos.arg(), dsin.arg(), p)
+        f.profile_reset()
+        f.profile_enable(True)
+        try:
+            f.fused_qkv_kv_prep(dx.arg(), *arg, K, rot[1][0].arg(), dcos.arg(), dsin.arg(), p, k_cache=rot[1][1].arg(), v_cache=rot[1][2].arg(), **kw)
+            f.synchronize()
+            assert f.profile_query("fused_qkv_rows32_rope_kernel")[0] == 1
+        finally:
+            f.profile_enable(False)
+        for one, two in zip(rot[0], rot[1]):
+            got, want = two.download(), one.download()
+            assert np.any(want) and np.array_equal(got.view(np.uint16), want.view(np.uint16)), mode
+    for b in [dx, dg, dcos, dsin] + db + outs + dev_w + dev_s + rot[0] + rot[1]:
+        b.free()
