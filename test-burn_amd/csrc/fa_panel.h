@@ -10,7 +10,8 @@
 // r % 8), normalised in the registers they arrive in (no exchange between waves), written to LDS and read back as operands:
 //   * a workgroup (8 waves) owns up to 32 weight rows - two 16-row tiles - and walks over its passes of 32 input rows (16 where
 //     rows are longer than 2048 features). All its weights are requested once, straight into the operand layout, behind the
-//     first pass's input rows; a pass's rows are requested while the one before is multiplied;
+//     first pass's input rows (some of the longest rows' in two parts: SPLIT); a pass's rows are requested while the one before is
+//     multiplied;
 //   * wave w multiplies the feature blocks 16 j + 2 w and 16 j + 2 w + 1 of every 512 features (adjacent: the two requests touch
 //     the same lines);
 //   * the eight waves' partial tiles meet in LDS and are added in wave order; then alpha, bias, beta * residual and one

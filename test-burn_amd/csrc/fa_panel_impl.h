@@ -65,11 +65,21 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     typedef typename W::raw_t raw_t;
     constexpr int XROW = row_bytes<PK>(), NR = FEW ? 1 : 2 * NC, NB = 2 * PK;
     static_assert(!FEW || NC == 1, "one group of input rows");
+    constexpr bool WIDE = WB != 16 && !SUMS, TURN = TURNS<WB, PK, SUMS>;
+    constexpr int GB = !WIDE && !TURN ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
+    typedef typename std::conditional<WIDE || TURN, u4v_t, raw_t>::type req_t;
+    // A wave that asks for more than the memory takes stands still until it has (a workgroup of 32 rows of 3072 features asks for
+    // 3 us), and normalises no rows meanwhile. SPLIT: it asks for the first NA requests of a tile, and for the others when the rows are
+    // in LDS. (3072 x 3072 without a norm, F16, 2 to 16 rows: 5.8 -> 5.2 us; Q8_0 2 to 8 rows 5.5 -> 5.1, row-major 7.2 -> 6.2, 24 and 32
+    // rows 7.1 -> 6.2; FusedQkv of 5120 x 3072 Q8_0, 16 rows 9.3 -> 8.7. Two tiles of F16, and one with its rotation, lose 1 to 14 % by
+    // it, shorter rows and Q4_0 have too few requests.)
+    constexpr bool SPLIT = PK > 4 && (WB == 8 ? !ROPE || NT == 2 : WB == 16 && !ROPE && NT == 1);
+    constexpr int NA = !SPLIT ? NQ : NT == 1 ? (NQ < 8 ? NQ : 8) : SUMS ? 6 : 4;
     // The order of the first requests is input rows, the norm's weights, scales, weights. Loads complete in the order in which they
     // are issued; left to itself the compiler puts the weights ahead of the rows in most of the kernels, and what is done with
     // the rows then waits for the whole weight stream. (m 12 .. 32, K 2048 .. 3072: o_proj 4 to 14 % less. With the longest rows and a
     // norm of two rows per wave the norm's chain is longer than the weights' stream, and the compiler's mixture is 1 to 3 % better.)
-    constexpr bool ORDERED = FEW || !ROPE || PK <= 4;
+    constexpr bool ORDERED = FEW || !ROPE || PK <= 4 || SPLIT;
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
@@ -182,9 +192,6 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     // rows, 5120 x 3072 10.1 -> 9.2 us, row-major 12.6 -> 9.3; 3072 x 3072 6.4 -> 5.7, 7.9 -> 5.8; 2560 x 2048 7.7 -> 7.4. (Rows of
     // up to 1024 features are a request or two either way, row-major 1 to 5 % slower; F16 and the other block-quantised forms lose
     // 3 to 15 % by it, Q8_0 per-block sums 7 to 40 % for want of registers.)
-    constexpr bool WIDE = WB != 16 && !SUMS, TURN = TURNS<WB, PK, SUMS>;
-    constexpr int GB = !WIDE && !TURN ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
-    typedef typename std::conditional<WIDE || TURN, u4v_t, raw_t>::type req_t;
     auto kb_of = [&](int i) __attribute__((always_inline)) -> uint32_t {
         return GB == 1 ? 16u * (uint32_t)(i >> 1) + 2u * (uint32_t)wave + (uint32_t)(i & 1) : GB == 2 ? 16u * (uint32_t)i + 2u * (uint32_t)wave : 32u * (uint32_t)i + 4u * (uint32_t)wave;
     };
@@ -201,24 +208,47 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         }
     };
     req_t wv[NT][NQ];
+    auto request_weights = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        bool valid;
-        int mat;
-        const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
-        const uint32_t N = pick3(mat, rows0, rows1, rows1);
-        // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
-        const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
-        const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
-        const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
+        for (int t = 0; t < NT; ++t) {
+            bool valid;
+            int mat;
+            const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
+            const uint32_t N = pick3(mat, rows0, rows1, rows1);
+            const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
+            const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
+            const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
 #pragma unroll
-        for (int i = 0; i < NQ; ++i) {
-            const uint32_t kb = kb_of(i) + get_blk;
-            const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
-            // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
-            // block-quantised weights are finite, and their scale is zero there.)
-            if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
-            wv[t][i] = fa_norm::load_global_once<req_t>(p);
+            for (int i = from; i < to; ++i) {
+                const uint32_t kb = kb_of(i) + get_blk;
+                const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
+                if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
+                wv[t][i] = fa_norm::load_global_once<req_t>(p);
+            }
+        }
+    };
+    if constexpr (SPLIT) {
+        request_weights(0, NA);
+    } else {  // (the same in place: the compiler makes 1 to 5 % slower kernels of the call)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            bool valid;
+            int mat;
+            const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
+            const uint32_t N = pick3(mat, rows0, rows1, rows1);
+            // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
+            const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
+            const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
+            const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                const uint32_t kb = kb_of(i) + get_blk;
+                const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
+                // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
+                // block-quantised weights are finite, and their scale is zero there.)
+                if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
+                wv[t][i] = fa_norm::load_global_once<req_t>(p);
+            }
         }
     }
     if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
@@ -317,6 +347,13 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int t = 0; t < NT; ++t)
                 s_res[t] = fa_norm::load_global<_Float16>(
                     residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * pick3(s_mat[t], rows0, rows1, rows1) + s_row[t] : x_in);
+        }
+        if constexpr (SPLIT) {
+            if (pass == blockIdx.y) {
+                __builtin_amdgcn_sched_barrier(0);
+                request_weights(NA, NQ);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         if (next < n_pass) request_rows(next, false);
 #pragma unroll
