@@ -73,7 +73,8 @@ struct RowsDev {
 
 constexpr int KT = 32;  // keys per tile
 
-template <int D, int NW, bool BF16, bool PAGED>
+// POOL: 0 a contiguous cache, 1 paged, 2 paged with pools of 4 GiB or more (no 32-bit offsets)
+template <int D, int NW, bool BF16, int POOL>
 __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(RowsDev a_by_value) {
     static_assert(std::is_trivially_copyable<RowsDev>::value, "read as raw bytes from the argument block, where it is the first member");
     const RowsDev a = *(const RowsDev *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -82,6 +83,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
                  "s"(a.out_stride_h), "s"(a.out_stride_m), "s"(a.block_table), "s"(a.group_size), "s"(a.rcp_group), "s"(a.q_len),
                  "s"(a.kv_len), "s"(a.query_offset), "s"(a.causal), "s"(a.block_size), "s"(a.block_shift), "s"(a.n_kv_heads));
     asm volatile("" ::"s"(a.pool_bytes32), "s"(a.n_blocks), "s"(a.splits), "s"(a.part_acc), "s"(a.part_ml), "s"(a.scale_log2e));
+    constexpr bool PAGED = POOL != 0;
     constexpr int DSTEPS = D / 16, DBLKS = D / 32, ROWB = D * 2;
     constexpr int RB_BYTES = 16 * ROWB;                 // 16 rows of K in LDS (rows16 layout), or of V
     constexpr int HALF = 2 * RB_BYTES, TILE = 2 * HALF;  // K or V of a tile; both
@@ -123,51 +125,54 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
         vrs = make_rsrc_words(a.v + (size_t)kvh * a.v_stride_h, kv_end * (uint32_t)ROWB);
     }
     const uint32_t page_bytes = a.n_kv_heads * a.block_size * (uint32_t)ROWB;  // of one page, all heads
-    typedef const int32_t __attribute__((address_space(4))) *const_i32p;
-    const const_i32p bt = (const_i32p)a.block_table;
     const uint32_t bs_shift = a.block_shift;
-    struct Pages {
-        int32_t p[2];
-    };
-    auto pages_of = [&](uint32_t tile) __attribute__((always_inline)) -> Pages {  // of its two 16-row groups
-        Pages r = {{0, 0}};
+    // Paged: where the 16-row groups of the wave's next 32 tiles lie, group l % 2 of tile l / 2 in lane l: page, offset in a pool of less
+    // than 4 GiB, and the end of the rows that are wanted of the group. (Worked out for each request, from a page id that came
+    // through the scalar cache, that took a tile from 0.7 to 1.0 us: 500 rows after 1000, H14 / Hkv2 / D64 10.4 -> 8.7 us,
+    // 500 after 1000, H16 / Hkv2 / D128 17.2 -> 13.1.)
+    int32_t page_ids = 0, page_off = 0, page_end = 0;
+    auto fetch_pages = [&](uint32_t first_tile) __attribute__((always_inline)) {
         if (PAGED) {
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const uint32_t key = tile * KT + 16 * g;
-                r.p[g] = key < kv_end ? bt[bs_shift < 32 ? key >> bs_shift : key / a.block_size] : 0;
-            }
+            const uint32_t key = (first_tile + NW * ((uint32_t)lane >> 1)) * KT + 16 * ((uint32_t)lane & 1u), end = min(kv_end, n_tiles * KT);
+            const uint32_t entry = bs_shift < 32 ? key >> bs_shift : key / a.block_size, rip = key - entry * a.block_size;
+            page_ids = key < end ? a.block_table[entry] : 0;
+            page_off = (int)((uint32_t)page_ids * page_bytes + (kvh * a.block_size + rip) * (uint32_t)ROWB);
+            page_end = page_off + (int)((key < end ? min(16u, end - key) : 0u) * (uint32_t)ROWB);
         }
-        return r;
     };
     const int k_src = rows16_lane_src(lane, ROWB);
     const int v_src = ((lane / (16 * COLS)) * 4 + ((lane & 15) >> 2)) * ROWB + ((lane >> 4) % COLS) * 64 + (lane & 3) * 16;
     // K or V of a tile into this wave's part of the LDS. (A tile past the last is requested from an empty range: nothing is read, zeros
     // arrive, and the counts that the waits go by stay the same.)
-    auto request = [&](bool is_k, uint32_t tile, const Pages &pg) __attribute__((always_inline)) {
+    auto request = [&](bool is_k, uint32_t tile, uint32_t nth /* of the fetched ones */) __attribute__((always_inline)) {
         const uint32_t dst = lds_addr + (uint32_t)wave * TILE + (is_k ? 0 : HALF);
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const uint32_t key = tile * KT + 16 * g;
-            rsrc_words rs = is_k ? krs : vrs;
-            int so = 0;
-            if (!PAGED) {
-                so = (int)(key * (uint32_t)ROWB);
-                if (tile >= n_tiles) rs.z = 0;
-            } else {
-                const uint32_t rip = bs_shift < 32 ? key & (a.block_size - 1) : key % a.block_size;
-                if (a.pool_bytes32 != 0 && key + 16 <= kv_end) {  // all 16 rows exist
-                    so = (int)((uint32_t)pg.p[g] * page_bytes + (kvh * a.block_size + rip) * (uint32_t)ROWB);
-                } else {  // a descriptor that ends with the last visible row
-                    const uint32_t valid = key < kv_end ? min(16u, kv_end - key) : 0u;
-                    const size_t base = (((size_t)pg.p[g] * a.n_kv_heads + kvh) * a.block_size + rip) * (size_t)ROWB;
-                    rs = make_rsrc_words(reinterpret_cast<const unsigned char *>(is_k ? a.k : a.v) + base, valid * ROWB);
-                    rs.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.x), rs.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.y);
-                }
-            }
-            so = __builtin_amdgcn_readfirstlane(so), rs.z = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.z);
+        auto rows16 = [&](int g, const rsrc_words &rs, int so) __attribute__((always_inline)) {
             if (is_k) buffer_to_lds_b128<COLS, 64, 1024>(rs, dst + g * RB_BYTES, k_src, so);
             else buffer_to_lds_b128<COLS, 1024, 1024>(rs, dst + g * RB_BYTES, v_src, so);
+        };
+        if constexpr (!PAGED) {
+            rsrc_words rs = is_k ? krs : vrs;
+            if (tile >= n_tiles) rs.z = 0;
+            rs.z = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.z);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) rows16(g, rs, __builtin_amdgcn_readfirstlane((int)((tile * KT + 16 * g) * (uint32_t)ROWB)));
+        } else {
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {  // (a descriptor that ends with the group's last wanted row)
+                const int off = __builtin_amdgcn_readlane(page_off, (int)(2 * nth + g)), end = __builtin_amdgcn_readlane(page_end, (int)(2 * nth + g));
+                rsrc_words rs = is_k ? krs : vrs;
+                if constexpr (POOL == 1) {
+                    rs.z = (uint32_t)end;
+                    rows16(g, rs, off);
+                } else {
+                    const size_t page = (size_t)__builtin_amdgcn_readlane(page_ids, (int)(2 * nth + g));
+                    const uint32_t key = tile * KT + 16 * g, rip = bs_shift < 32 ? key & (a.block_size - 1) : key % a.block_size;
+                    rs = make_rsrc_words(reinterpret_cast<const unsigned char *>(is_k ? a.k : a.v) + ((page * a.n_kv_heads + kvh) * a.block_size + rip) * (size_t)ROWB, (uint32_t)(end - off));
+                    rs.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.x), rs.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.y);
+                    rs.z = (uint32_t)__builtin_amdgcn_readfirstlane((int)rs.z);
+                    rows16(g, rs, 0);
+                }
+            }
         }
     };
     constexpr int REQ = 2 * COLS;  // loads of K, or of V, of a tile
@@ -177,6 +182,8 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
         asm volatile("" ::: "memory");
     };
 
+    uint32_t tile = t_lo + (uint32_t)wave;
+    fetch_pages(tile);
     // Query rows: 2 COLS loads of 1 KiB, one per wave as far as they go, in the layout of a K tile behind the stages
     {
         const size_t q_bytes = ((size_t)(G - 1) * a.q_stride_h + (size_t)(a.q_len - 1) * a.q_stride_m + D) * 2;
@@ -189,10 +196,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
             buffer_to_lds_b128<1, 0, 0>(qrs, lds_addr + STAGES + r * 1024, (int)(at + (uint32_t)rows16_lane_src(lane, 0)), (int)(col * 64));
         }
     }
-    uint32_t tile = t_lo + (uint32_t)wave;
-    Pages pg = pages_of(tile);
-    request(true, tile, pg), request(false, tile, pg);
-    pg = pages_of(tile + NW);
+    request(true, tile, 0), request(false, tile, 0);
     wait_but(std::integral_constant<int, 2 * REQ>{});  // this wave's part of the query rows (requested first) is there
     __syncthreads();
     h8_t qreg[DSTEPS];
@@ -215,7 +219,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
     const int v_at = hi * RG_BYTES + ((lane & 15) >> 2) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
 
     const unsigned char *k_lds = lds + wave * TILE, *v_lds = k_lds + HALF + v_at;
-    for (; tile < n_tiles; tile += NW) {
+    for (uint32_t nth = 0; tile < n_tiles; tile += NW) {
         wait_but(std::integral_constant<int, REQ>{});  // K is there
         f16_t s = {};
         h8_t kk[DSTEPS];
@@ -224,7 +228,9 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
 #pragma unroll
         for (int i = 0; i < DSTEPS; ++i) s = mfma<BF16>(kk[i], qreg[i], s);
         lds_reads_done();
-        request(true, tile + NW, pg);
+        nth = (nth + 1) & 31u;
+        if (PAGED && nth == 0) fetch_pages(tile + NW);
+        request(true, tile + NW, nth);
         // accumulator i is key 32 tile + 8 (i / 4) + 4 hi + i % 4
         const uint32_t key0 = tile * KT;
         if (key0 + KT - 1 > min_limit || key0 + KT > kv_end) {
@@ -275,8 +281,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
                 oacc[b] = mfma<BF16>(va.h, pb[ks], oacc[b]);
             }
         lds_reads_done();
-        request(false, tile + NW, pg);
-        pg = pages_of(tile + 2 * NW);
+        request(false, tile + NW, nth);
     }
     wait_but(std::integral_constant<int, 0>{});  // (what was requested past the last tile delivered nothing, but must be over)
     __syncthreads();
@@ -329,15 +334,16 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
     }
 }
 
+template <int D, int NW, bool BF16>
+void launch_rows(FaLaunchScope &scope, const RowsDev &a, uint32_t grid, bool paged) {
+    if (!paged) scope.launch(flash_rows_kernel<D, NW, BF16, 0>, dim3(grid), dim3(NW * 64), 0, a);
+    else if (a.pool_bytes32) scope.launch(flash_rows_kernel<D, NW, BF16, 1>, dim3(grid), dim3(NW * 64), 0, a);
+    else scope.launch(flash_rows_kernel<D, NW, BF16, 2>, dim3(grid), dim3(NW * 64), 0, a);
+}
 template <int D, int NW>
 void launch_rows(FaLaunchScope &scope, const RowsDev &a, uint32_t grid, bool bf16, bool paged) {
-    if (bf16) {
-        if (paged) scope.launch(flash_rows_kernel<D, NW, true, true>, dim3(grid), dim3(NW * 64), 0, a);
-        else scope.launch(flash_rows_kernel<D, NW, true, false>, dim3(grid), dim3(NW * 64), 0, a);
-    } else {
-        if (paged) scope.launch(flash_rows_kernel<D, NW, false, true>, dim3(grid), dim3(NW * 64), 0, a);
-        else scope.launch(flash_rows_kernel<D, NW, false, false>, dim3(grid), dim3(NW * 64), 0, a);
-    }
+    if (bf16) launch_rows<D, NW, true>(scope, a, grid, paged);
+    else launch_rows<D, NW, false>(scope, a, grid, paged);
 }
 
 }  // namespace

@@ -135,3 +135,40 @@ def test_rows_masks_and_layouts(M, N, offset, causal, D):
     want = orc.sdpa_prefill(q, k, v, H, Hkv, D, M, N, offset, cap, causal=causal, out_layout="head_major", n_threads=8)
     assert max_abs(outs[1], want) <= TOL
     dk.free(), dv.free()
+
+
+@pytest.mark.parametrize("D,M,prefix", [(64, 40, 2300), (128, 33, 1111), (64, 2, 40)])
+def test_rows_paged_large_pool(D, M, prefix):
+    """Pools of 4 GiB, whose rows have no 32-bit byte offsets, with pages all over them: the bits of the small pools' launch."""
+    announce("prefill rows, large pool", D, M, prefix)
+    f = ctx()
+    rng = np.random.default_rng(D + M)
+    H, Hkv, bs, N = 6, 2, 16, prefix + M
+    nb = (N + bs - 1) // bs
+    k, v, q0 = (f.array(h16(rng.normal(size=(N, h * D)))) for h in (Hkv, Hkv, H))
+    q, q_rot = f.array(h16(rng.normal(size=(H, M, D)))), f.zeros((H, N, D))
+    cos, sin = (f.array(t) for t in fa.rope_tables(1e4, D, N))
+    lens, got = f.array(np.array([N], np.uint32)), []
+    for n_pages in (nb + 3, 2 ** 32 // (Hkv * bs * D * 2)):
+        table = rng.permutation(n_pages)[:nb].astype(np.int32)
+        if n_pages - 1 not in table:
+            table[-1] = n_pages - 1
+        kp, vp, bt = f.empty((n_pages, Hkv, bs, D)), f.empty((n_pages, Hkv, bs, D)), f.array(table)
+        cache = fa.paged_kv(kp, vp, bt, lens, n_pages, Hkv, bs, D, 1, nb)
+        p = fa.KvPrepFusedParams.make(H, Hkv, D, N, 0, nb * bs, fa.ROPE_NEOX)
+        f.kv_prep_fused_paged(q0.arg(), k.arg(), v.arg(), q_rot.arg(), cache, 0, cos.arg(), sin.arg(), p)
+        do = f.zeros((M, H * D))
+        n = _launches(f, lambda: f.flash_prefill_paged(q.arg(), cache, 0, do.arg(), True, prefix, H, N, M))
+        assert n[0] == 1 and n[2] == 0, n
+        got.append(do.download().view(np.uint16))
+        for b in (kp, vp, bt, do):
+            b.free()
+    assert np.any(got[0]) and np.array_equal(got[0], got[1])
+    for b in (k, v, q0, q, q_rot, cos, sin, lens):
+        b.free()
+
+
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,bs", [(28, 2, 64, 300, 4500, 16), (32, 2, 64, 260, 4100, 48)])
+def test_rows_paged_more_than_32_tiles_per_wave(H, Hkv, D, M, prefix, bs):
+    """A wave fetches where its tiles lie a second time (4 waves)."""
+    test_rows_paged(H, Hkv, D, M, prefix, False, bs)
