@@ -453,8 +453,12 @@ __device__ __forceinline__ void phase_barrier() {
 //           the 32 lanes of a transpose-read pass (4 rows x 64 B) are 256 consecutive bytes.
 // Wave w of a group moves rows 16w..16w+15 of every tile of its group (16 rows never straddle a page). Rows past
 // the visible keys come out of the buffer descriptor's bound check as zeros.
-template <int D, bool BF16, bool PAGED>
+// POOL: 0 a contiguous cache, 1 paged, 2 paged with pools of 4 GiB or more or pages of a size that is not a power of two. (One kernel
+// for both had jumps around the second's code in every request: 4000 rows, H14 / Hkv2 / D64 47.6 -> 42.6 us, H24 / Hkv8 / D128 98.8 -> 92.0,
+// which is what a contiguous cache takes.)
+template <int D, bool BF16, int POOL>
 __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_by_value) {
+    constexpr bool PAGED = POOL != 0;
     // The launch's arguments as a local copy read from its argument block in ONE trip through the scalar cache (an empty
     // statement that takes the fields as scalar inputs makes the compiler fetch them here). As a by-value struct the
     // fields were fetched where the program first needs them: thirteen dependent trips, one wait each, between the entry
@@ -562,7 +566,9 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     // page id of this wave's 16 rows of group-local tile i (wave-uniform: a scalar load)
     auto page_of = [&](int i) -> int32_t {
         const uint32_t key = (uint32_t)(t0 + 2 * i) * BN + 16 * wave;
-        return (PAGED && key < kv_end) ? bt[bs_shift < 32 ? key >> bs_shift : key / a.block_size] : 0;
+        if (!PAGED) return 0;
+        const uint32_t last = min(key, kv_end - 1);  // (no branch: the last page again past the end)
+        return bt[POOL == 1 || bs_shift < 32 ? last >> bs_shift : last / a.block_size];
     };
     // this wave's 16 rows of group-local tile i of one tensor into LDS buffer `buf`
     auto dma = [&](bool is_k, int i, int buf, int32_t page) {
@@ -570,12 +576,12 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         rsrc_words rs = is_k ? krs : vrs;
         int so = (int)(key * (uint32_t)ROWB);
         if (PAGED) {
-            const uint32_t rip = bs_shift < 32 ? key & (a.block_size - 1) : key % a.block_size;
-            if (a.pool_bytes32 != 0 && key + 16 <= kv_end) {
-                // all 16 rows exist: the pool's descriptor and a 32-bit offset to the rows
+            const uint32_t rip = POOL == 1 || bs_shift < 32 ? key & (a.block_size - 1) : key % a.block_size;
+            const uint32_t valid = key < kv_end ? min(16u, kv_end - key) : 0u;  // (a descriptor that ends with the last visible row: past it zeros)
+            if (POOL == 1 || a.pool_bytes32 != 0) {  // the pool's descriptor and a 32-bit offset to the rows
                 so = (int)((uint32_t)page * page_bytes + (kvh * a.block_size + rip) * (uint32_t)ROWB);
-            } else {  // a descriptor that ends with the last visible row (rows past it come out as zeros)
-                const uint32_t valid = key < kv_end ? min(16u, kv_end - key) : 0u;
+                rs.z = (uint32_t)so + valid * (uint32_t)ROWB;
+            } else {
                 const size_t base = (((size_t)page * a.n_kv_heads + kvh) * a.block_size + rip) * (size_t)ROWB;
                 const unsigned char *pool = reinterpret_cast<const unsigned char *>(is_k ? a.k : a.v);
                 rs = make_rsrc_words(pool + base, valid * ROWB);
@@ -1050,6 +1056,11 @@ __global__ void __launch_bounds__(256) flash_prefill_merge_kernel(PrefillMerge a
     *reinterpret_cast<h4_t *>(a.out + (size_t)head * a.out_stride_h + (size_t)q_row * a.out_stride_m + c4 * 4) = h;
 }
 
+template <int D, bool BF16>
+auto dma_kernel(int pool) {
+    return pool == 0 ? flash_prefill_dma_kernel<D, BF16, 0> : pool == 1 ? flash_prefill_dma_kernel<D, BF16, 1> : flash_prefill_dma_kernel<D, BF16, 2>;
+}
+
 }  // namespace
 
 fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
@@ -1168,14 +1179,9 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     {
         FaLaunchScope scope(ctx, lds_direct ? "flash_prefill_dma_kernel" : "flash_prefill_mfma_kernel", true);
         if (lds_direct) {
-            auto kern = flash_prefill_dma_kernel<128, false, false>;
-            if (L.head_dim == 128) {
-                kern = L.bf16 ? (L.paged ? flash_prefill_dma_kernel<128, true, true> : flash_prefill_dma_kernel<128, true, false>)
-                              : (L.paged ? flash_prefill_dma_kernel<128, false, true> : flash_prefill_dma_kernel<128, false, false>);
-            } else {
-                kern = L.bf16 ? (L.paged ? flash_prefill_dma_kernel<64, true, true> : flash_prefill_dma_kernel<64, true, false>)
-                              : (L.paged ? flash_prefill_dma_kernel<64, false, true> : flash_prefill_dma_kernel<64, false, false>);
-            }
+            const int pool = !L.paged ? 0 : a.pool_bytes32 != 0 && a.block_shift < 32 ? 1 : 2;
+            auto kern = L.head_dim == 128 ? (L.bf16 ? dma_kernel<128, true>(pool) : dma_kernel<128, false>(pool))
+                                          : (L.bf16 ? dma_kernel<64, true>(pool) : dma_kernel<64, false>(pool));
             scope.launch(kern, grid, dim3(512), 0, a);
         } else if (L.head_dim == 128 && L.bf16)
             scope.launch(flash_prefill_mfma_kernel<128, true>, grid, dim3(512), 0, a);

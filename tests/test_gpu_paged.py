@@ -585,3 +585,47 @@ def test_paged_prefill_chunk_after_prefix(H, Hkv, D, bs, prefix, M):
     pg.free()
     for b in (dq, dout):
         b.free()
+
+
+@pytest.mark.parametrize("D,M,prefix", [(64, 200, 700), (128, 129, 448)])
+def test_tiled_prefill_bits_whatever_the_pages(D, M, prefix):
+    """The tiled kernel for pools with 32-bit offsets and pages of a power of two, and the one for other pages and for pools of 4 GiB:
+    the bits of the contiguous cache."""
+    announce("tiled prefill, pools", D, M, prefix)
+    f = ctx()
+    rng = np.random.default_rng(D + M)
+    H, Hkv, N = 6, 2, prefix + M
+    rows = [f.array(h16(rng.normal(size=(N, h * D)))) for h in (H, Hkv, Hkv)]
+    q, q_rot = f.array(h16(rng.normal(size=(H, M, D)))), f.zeros((H, N, D))
+    cos, sin = (f.array(t) for t in fa.rope_tables(1e4, D, N))
+    lens, do = f.array(np.array([N], np.uint32)), f.zeros((M, H * D))
+    ins = [r.arg() for r in rows]
+    try:
+        f.set_prefill_variant(2)
+        f.set_prefill_split_k(1)
+        kc, vc = f.empty((Hkv, N, D)), f.empty((Hkv, N, D))
+        p = fa.KvPrepFusedParams.make(H, Hkv, D, N, 0, N, fa.ROPE_NEOX)
+        f.kv_prep_fused(*ins, q_rot.arg(), kc.arg(), vc.arg(), cos.arg(), sin.arg(), p)
+        f.flash_attention(q.arg(), kc.arg(), vc.arg(), do.arg(), True, prefix, H, D, N, M)
+        want = do.download().view(np.uint16).copy()
+        assert np.any(want)
+        for bs, n_pages in ((16, 0), (64, 0), (48, 0), (16, 2 ** 32 // (Hkv * 16 * D * 2))):
+            nb = (N + bs - 1) // bs
+            n_pages = n_pages or nb + 3
+            table = rng.permutation(n_pages)[:nb].astype(np.int32)
+            if n_pages - 1 not in table:
+                table[-1] = n_pages - 1
+            kp, vp, bt = f.empty((n_pages, Hkv, bs, D)), f.empty((n_pages, Hkv, bs, D)), f.array(table)
+            cache = fa.paged_kv(kp, vp, bt, lens, n_pages, Hkv, bs, D, 1, nb)
+            p = fa.KvPrepFusedParams.make(H, Hkv, D, N, 0, nb * bs, fa.ROPE_NEOX)
+            f.kv_prep_fused_paged(*ins, q_rot.arg(), cache, 0, cos.arg(), sin.arg(), p)
+            do.upload(np.zeros((M, H * D), np.float16))
+            f.flash_prefill_paged(q.arg(), cache, 0, do.arg(), True, prefix, H, N, M)
+            assert np.array_equal(do.download().view(np.uint16), want), (bs, n_pages)
+            for b in (kp, vp, bt):
+                b.free()
+    finally:
+        f.set_prefill_variant(0)
+        f.set_prefill_split_k()
+    for b in rows + [q, q_rot, cos, sin, lens, do, kc, vc]:
+        b.free()
