@@ -77,6 +77,34 @@ def test_tiles(K, H, Hkv, D, m, layout, weights):
         b.free()
 
 
+@pytest.mark.parametrize("K,N,m", [(256, 200, 130), (1024, 520, 577), (192, 2056, 520)])  # 64 x 64 tiles, with steps of each wave's own, 64 x 96
+@pytest.mark.parametrize("weights", ["f16", "q8"])
+def test_residual_asked_for_ahead_of_the_sums(K, N, m, weights):
+    """Every tile reads its own places of the residual, whatever is done with the ones past the last row: in place of it, the output is the same bits."""
+    announce("residual ahead", K, N, m, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + N + m)
+    x, w = rng.uniform(-1, 1, (m, K)).astype(np.float16), (rng.uniform(-1, 1, (N, K)) / 16).astype(np.float16)
+    res = rng.uniform(-1, 1, (m, N)).astype(np.float16)
+    q, s = orc.quantize_q8_0(w)
+    dx, dres, dout = f.array(x), f.array(res), f.zeros((m, N))
+    dw, ds = f.array(q if weights == "q8" else w), f.array(s)
+    kw = dict(transpose_b=True, beta=0.75, b_scales=ds.arg() if weights == "q8" else None)
+    try:
+        f.set_gemm_min_m(12)
+        f.matmul(dx.arg(), dw.arg(), dout.arg(), m, N, K, c=dres.arg(), **kw)
+        got = dout.download()
+        f.matmul(dx.arg(), dw.arg(), dres.arg(), m, N, K, c=dres.arg(), **kw)
+        assert np.array_equal(bits(dres.download()), bits(got))
+    finally:
+        f.set_gemm_min_m()
+    for b in (dx, dres, dout, dw, ds):
+        b.free()
+    full = orc.dequantize_blocks(q, s) if weights == "q8" else w
+    want = orc.matmul_gemv(x, full, None, res, 0, 32, 1.0, 0.75).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2 * np.maximum(np.abs(want), 2.0 ** -10) * 2.0 ** -10 + 1e-4)  # (as test_tiles)
+
+
 @pytest.mark.parametrize("weights", ["q8", "q4"])
 @pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
     (960, 2, 1, 64, 65, 1),       # the last length whose steps the waves of a tile share
