@@ -949,7 +949,7 @@ def bench_prefill_chunk(f, args, m=32, prefix=8160):
         "data": "synthetic",
         "config": {"workload": "llama3.2-3b prefill chunk of %d rows after a %d-token prefix, one layer per step: causal attention "
                                "split over the keys, merge %s, contiguous cache, %d layers' caches in rotation, graph replays"
-                               % (m, prefix, "inside the launch" if "flash_chunk_kernel" in us else "as a second launch", L)},
+                               % (m, prefix, "as a second launch" if "flash_prefill_merge_kernel" in us else "inside the launch", L)},
         "roofline": {"bound": "hbm", "achieved": nbytes / per_step / 1e9, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": nbytes / per_step / 1e9 / HBM_PEAK_GBPS, "traffic": None,
                      "kernel": " + ".join(us) + " (one step)",
