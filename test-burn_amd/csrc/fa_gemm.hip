@@ -520,6 +520,11 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
             // stages on their way (both measured in fa_tile.h; LDS beside the scales: up to 4096 and 8192 features).
             if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && tiles <= n_cus && l.k_dim <= 8192)
                 shape = l.k_dim >= 1024 && l.k_dim <= 4096 ? fa_tile::TILE_64x64_OWN : fa_tile::TILE_64x64_DEEP;
+            if (c.shape == fa_tile::TILE_64x64 && l.weight_bits != 16 && variant == 0) {  // (there too; where it fills no second round)
+                uint32_t narrow = 0;
+                for (int i = 0; i < 3; ++i) narrow += ceil_div_u32(rows[i], 32);
+                if ((uint64_t)narrow * ceil_div_u32(l.m, 64) <= n_cus) shape = fa_tile::TILE_64x32;
+            }
         }
     }
     return best;

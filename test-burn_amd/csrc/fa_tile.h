@@ -28,6 +28,10 @@
 //     FusedQkv 300 rows, 2560 x 2048 14.9 -> 13.9, 14.8 -> 13.3. Below 1024 features what it adds - the first steps of four waves
 //     arrive together, four partial tiles meet in the write stage - outweighs that (896: Q8_0 6.4 -> 6.8), above 4096 the scales
 //     leave room for two stages (5120: 17.8 -> 20.0). Steps of 32 features and eight waves: 5 to 10 % slower (half lines per request).
+//     With a workgroup for half of the compute units or fewer, the tiles are of 32 weight rows, each wave with a quarter of every
+//     step: half the weights to convert and half the products in the chain. (Against 64 x 64: o_proj 500 rows, 896 features x 896 Q8_0
+//     6.2 -> 5.6 us, Q4_0 6.3 -> 5.6; 190 rows, 2048 x 2048 9.1 -> 8.2, 8.7 -> 8.3; FusedQkv 130 rows, 2560 x 2048 12.2 -> 11.1, 12.2 ->
+//     11.3. 32 input rows x 64 instead: the last 11.7 and 11.9, o_proj of 2048 features up to 6 % slower than 64 x 64 with Q4_0.)
 //   * a 32 x 32 x 16 matrix instruction rounds its running sum twice, so a chain's error grows with the root of its length: over 3072
 //     features 5.9 x 2^-24 of the sums' size. F16 tiles of up to 128 x 128, which took the place of parts of a few hundred features
 //     added in a second launch (2.2 x 2^-24), add their accumulators to a second set every FOLD steps, between the products, for
@@ -81,7 +85,7 @@ struct Shape {
     // what a lane reads of a weight row at a time: the 8 features of a product, of both halves of the wave where they are 4 bytes
     typedef typename std::conditional<WB_ == 16, h8_t, u2v_t>::type raw_t;
     static constexpr int READS = KN * (TM + TN);
-    static constexpr int TJ = OWN ? TM : 1;  // 32-row groups of every wave that the write stage turns at a time
+    static constexpr int TJ = OWN || NTR < 64 ? TM : 1;  // 32-row groups of every wave that the write stage turns at a time
     static constexpr int T_STRIDE = NTR * 4 + 16, T_BYTES = WM * TJ * 32 * T_STRIDE;
     // LDS: the stages, then (block-quantised) all scales of the tile's rows, [8 blocks][row]; the write stage over both
     static constexpr uint32_t scale_bytes(uint32_t k_dim) { return QUANT ? NTR % 64 == 0 ? (k_dim + 255) / 256 * (NTR * 16) : ((k_dim + 255) / 256 * (NTR * 16) + 1023) & ~1023u : 0u; }
@@ -90,11 +94,11 @@ struct Shape {
         return s > (uint32_t)(KG * T_BYTES) ? s : (uint32_t)(KG * T_BYTES);
     }
     static_assert(X_BYTES % 1024 == 0 && W_BYTES % 1024 == 0, "whole requests");
-    static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63 && NTR >= 64, "LDS of a compute unit; the request counter");
+    static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63, "LDS of a compute unit; the request counter");
 };
 
-// input rows x weight rows (the first two: block-quantised, stages of each wave's own and more stages)
-enum TileShape { TILE_64x64_OWN, TILE_64x64_DEEP, TILE_64x64, TILE_64x96, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };
+// input rows x weight rows (the first three: block-quantised; with stages of each wave's own, with more stages)
+enum TileShape { TILE_64x32, TILE_64x64_OWN, TILE_64x64_DEEP, TILE_64x64, TILE_64x96, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x160 };
 
 template <int N>
 __device__ __forceinline__ void wait_requests() {
@@ -171,7 +175,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         const uint32_t q = (loader * S::WR + i) % S::W_REQ;
         w_block[i] = 0;
         if constexpr (S::CANON) {
-            constexpr uint32_t PER_BLOCK = S::W_REQ / 2;
+            constexpr uint32_t PER_BLOCK = S::W_REQ > 1 ? S::W_REQ / 2 : 1;
             const uint32_t u = q % PER_BLOCK;
             w_block[i] = q / PER_BLOCK;
             if constexpr (S::WB == 16) {
@@ -494,6 +498,7 @@ fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDe
     if constexpr (WB == 16) {
         switch (shape) {
             case TILE_64x64_OWN:
+            case TILE_64x32:
             case TILE_64x64_DEEP:
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 2, 2, 1, 1, 1, 4>, 2>(ctx, scope, a);
             case TILE_64x96: return launch_shape<Shape<WB, CANON, 2, 3, 1, 1, 1, 4>, 2>(ctx, scope, a);
@@ -506,6 +511,7 @@ fa_status launch_tile(fa_ctx *ctx, FaLaunchScope &scope, TileShape shape, GemmDe
         switch (shape) {
             case TILE_64x64_OWN: return launch_shape<Shape<WB, CANON, 1, 1, 4, 2, 2, 3, false, true>, 1>(ctx, scope, a);
             case TILE_64x64_DEEP: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 8>, 1>(ctx, scope, a);
+            case TILE_64x32: return launch_shape<Shape<WB, CANON, 1, 1, 4, 2, 1, 8>, 1>(ctx, scope, a);
             case TILE_64x64: return launch_shape<Shape<WB, CANON, 1, 2, 2, 2, 1, 4>, 2>(ctx, scope, a);
             case TILE_64x96:
                 if constexpr (WB == 4) {  // (3072 x 3072, 340 rows, canonical and row-major: 16.8 -> 14.8 us, 18.4 -> 15.3; Q8_0 has room for two stages, 16.4 -> 16.9)

@@ -126,6 +126,35 @@ def test_tiles_with_steps_of_each_waves_own(K, H, Hkv, D, m, layout, weights):
         ctx().set_gemm_variant()
 
 
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
+    (64, 3, 1, 64, 12, 1),        # one step, fewer than stages
+    (448, 2, 1, 64, 65, 0),       # seven: the unrolled loop is cut off; scales of one unit and three quarters
+    (576, 1, 1, 128, 64, 1),      # nine steps
+    (896, 14, 2, 64, 448, 1),     # 252 tiles
+    (896, 14, 2, 64, 449, 0),     # 288: tiles of 64 x 64 again
+    (1088, 1, 1, 128, 130, 1),
+    (2112, 2, 2, 64, 33, 0),
+    (8256, 1, 1, 64, 70, 1),      # past the features that the 64 x 64 forms with more stages have room for
+])
+def test_tiles_of_32_weight_rows(K, H, Hkv, D, m, layout, weights):
+    test_tiles(K, H, Hkv, D, m, layout, weights)
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
+    (192, 1, 1, 128, 65, 0), (896, 2, 1, 64, 513, 0), (1024, 2, 1, 64, 65, 1), (1088, 1, 1, 128, 64, 0), (1216, 5, 1, 64, 12, 0),
+    (4096, 1, 1, 64, 70, 0), (4160, 1, 1, 64, 20, 1)])
+def test_tiles_of_64_weight_rows_by_name(K, H, Hkv, D, m, layout, weights):
+    """The 64 x 64 forms at sizes that the narrower tiles take of themselves."""
+    f = ctx()
+    f.set_gemm_variant(3)
+    try:
+        test_tiles(K, H, Hkv, D, m, layout, weights)
+    finally:
+        f.set_gemm_variant()
+
+
 @pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
 @pytest.mark.parametrize("K,N,NK,m,panel,finish", [
     (2048, 8192, 1024, 16, True, False),    # one round of workgroups: the panel up to 32 rows
