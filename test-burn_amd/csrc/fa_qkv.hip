@@ -409,9 +409,10 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
 // rows). Up to 32 rows whose weight rows fit one round of workgroups always (a default chunk is one launch). Beyond, up to as many as
 // it is measured to beat the tile kernels with where the weight rows suit it - later where those need the normalisation's launch in
 // front (Qwen2.5-0.5B: 384 rows, both 31.8 us per layer; its o_proj alone, F16: 128 rows 4.2 against 5.0 us, 256 rows 5.3 against
-// 5.1; block-quantised as long as a pass over 16 weight rows has a workgroup of its own, two to a compute unit, 256 rows Q8_0 4.9
-// against 6.0, Q4_0 4.8 against 6.2, 350 rows Q8_0 row-major 6.8 against 5.9; of 256 features only one to a compute unit, 438 rows of
-// 256 x 576 take 1.17 times as long as the tiles),
+// 5.1; block-quantised as long as each pass has a workgroup of its own, two to a compute unit, 239 rows of 896 x 192 Q4_0 3.8 against
+// 5.2, 314 rows of 512 x 128 Q8_0 3.7 against 4.4, 228 rows of 640 x 960 Q4_0 4.5 against 4.8, 265 rows of 896 x 704 Q8_0 row-major
+// both 5.2, 30 launches 0.85 in the mean and 1.13 at worst; of 256 features only one to a compute unit, 438 rows of 256 x 576 take
+// 1.17 times as long as the tiles),
 // earlier for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer) - unless the GEMM is a tenth ahead by
 // estimate: many weight rows are many passes of the input rows here, or rounds of workgroups. A launch takes the weight stream, and
 // for each pass that a compute unit has one after the other the input rows of that pass, fetched and multiplied and, with a gamma,
