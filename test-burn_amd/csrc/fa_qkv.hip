@@ -434,6 +434,16 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     if (l.m <= 32 && p.rounds == 1) return true;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
+    // Block-quantised with a norm: where 32 input rows x 32 weight rows are more than a piece per compute unit, a second pass costs 3 us
+    // and more, which the estimate below does not see of few features: 195 rows, 512 x 2112 Q4_0 12.0 us, 8.4 with the norm's launch and
+    // the tiles; 391 rows, 640 x 1344 Q8_0 12.1, 9.2; 124 rows, 1280 x 2112 Q8_0 14.4, 9.3; just below the line 192 rows, 512 x 1344 6.2,
+    // 7.2. Of 768 to 1024 features the line is at the third pass (375 rows, 768 x 1664 13.8, 9.6; with two, 287 rows, 896 x 960 9.7, 8.4).
+    if (!f16 && l.gamma && l.m > 32 && p.nc == 2 && l.k_dim % 64 == 0 && l.n_dim % 8 == 0 && l.n_kv % 8 == 0) {
+        const uint64_t pieces = (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 32) * p.n_pass;
+        bool scales_fit = true;  // (what the tiles ask of a launch)
+        for (int i = 0; i < 3; ++i) scales_fit = scales_fit && reinterpret_cast<uintptr_t>(l.scales[i]) % 4 == 0;
+        if (scales_fit && pieces > (l.k_dim >= 768 && l.k_dim <= 1024 ? 2 : 1) * n_cus) return false;
+    }
     // passes of a compute unit (with two workgroups on it they share its way to L2)
     const float passes = p.pk > 2 ? (float)(p.rounds * ceil_div_u32(p.n_pass, p.grid_y)) : std::max(1.0f, (float)(p.grid_x * p.n_pass) / (float)n_cus);
     const float k = (float)l.k_dim, mb = k * (float)(l.n_dim + 2 * l.n_kv) * (f16 ? 2.0f : l.weight_bits == 8 ? 1.0625f : 0.5625f) * 1e-6f;

@@ -220,6 +220,16 @@ def _quantised(f, rng, K, N, m, weights):
 
 
 @pytest.mark.parametrize("weights", ["q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,panel", [
+    (640, 896, 192, 192, True), (640, 896, 192, 193, False),     # 240, 280 pieces of 32 x 32 rows
+    (960, 1856, 64, 256, True), (960, 1856, 64, 257, False),     # 496, 558
+    (1280, 1984, 64, 124, False),                                # 264
+])
+def test_route_of_a_quantised_chunk_with_a_norm(K, N, NK, m, panel, weights):
+    test_route_of_a_chunk(K, N, NK, m, panel, None, weights)
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
 @pytest.mark.parametrize("K,N,m,panel", [
     (896, 896, 193, True), (896, 896, 288, True),   # up to a pass for each compute unit
     (896, 896, 289, False),
