@@ -26,9 +26,6 @@ struct GemmDev {
     // [split][m][n_total]; gemm_finish_kernel adds them up in split order and applies the write stage
     uint32_t k_splits, steps_per_split, n_total;
     float *partial;
-    // the weights of all matrices as one range of bytes, and where in it each begins (for tiles that hold rows of two matrices)
-    const void *w_low;
-    uint32_t w_span, w_at[3];
     RopeDev rope;
 };
 

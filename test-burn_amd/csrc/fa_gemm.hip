@@ -586,15 +586,7 @@ float fa_gemm_estimate_us(const fa_ctx *ctx, const FusedQkvLaunch &l) {
 static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, uint32_t n_cus, fa_tile::TileShape &shape) {
     const uint64_t max_rows = std::max(a.rows[0], a.rows[1]);
     if (!tiles_fit(l) || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
-    // tiles over the rows of all matrices need them within the reach of one descriptor
-    uintptr_t low = (uintptr_t)l.w[0], high = low;
-    for (int i = 0; i < 3; ++i)
-        if (a.rows[i]) low = std::min(low, (uintptr_t)l.w[i]), high = std::max(high, (uintptr_t)l.w[i] + (size_t)a.rows[i] * l.k_dim * 2);
-    const bool joined = l.weight_bits == 16 && high - low < 0xfffffff0ull && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
-    if (joined) {
-        a.w_low = (const void *)low, a.w_span = (uint32_t)(high - low);
-        for (int i = 0; i < 3; ++i) a.w_at[i] = a.rows[i] ? (uint32_t)((uintptr_t)l.w[i] - low) : 0u;
-    }
+    const bool joined = l.weight_bits == 16 && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
     const float cost = best_tile(l, a.rows, n_cus, joined, ctx->gemm_variant, shape);
     if (cost == 0.0f) return false;
     if (ctx->gemm_variant != 0) return true;

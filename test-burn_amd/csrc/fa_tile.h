@@ -13,7 +13,9 @@
 //   * large launches read less per product with larger tiles but leave CUs idle where the tiles do not fill a round of
 //     workgroups: six shapes, the choice by the rounds they need (choose_tile, fa_gemm.hip). 256 x 160 (F16) fills a round where
 //     256 x 128 leaves a fifth of the chip to a second one - 8.4 to 10.5 million outputs, such as 2048 rows x 5120, and again at
-//     twice that - and may hold rows of two matrices (JOINED). 64 x 96 does so for a quarter to a half more outputs than 64 x 64 have
+//     twice that - and may hold rows of two matrices (JOINED), which lie anywhere: each request has the descriptor of its matrix (one
+//     over all three matrices asked them to be within 4 GiB, and weights further apart took the 128 x 128 tiles: 2048 rows, 5120 x 3072
+//     75 us where they now take 60 to 62 wherever they lie). 64 x 96 does so for a quarter to a half more outputs than 64 x 64 have
 //     room for. (128 x 96: no faster than 128 x 128 with a third more workgroups, 22.0 us for 700 rows of 3072 x 3072.)
 //   * block-quantised weights stay as they are up to the registers, where a wave turns its operands to f16 right in front of the
 //     product (f16(weight * scale), as the reference's tile loader: see fa_gemm.hip). That is 14 vector instructions per 8
@@ -209,21 +211,21 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     const fa_lds_dma::rsrc_words x_rs = fa_lds_dma::make_rsrc_words(reinterpret_cast<const unsigned char *>(a.x) + (size_t)m0 * K * 2, (a.m - m0) * K * 2);
     const uint32_t w_block_bytes = N_tile * 4 * S::WB;  // canonical: one 32-feature block of the matrix
     uint32_t w_step[S::WR];                             // JOINED: bytes between the steps of a request's matrix
-    fa_lds_dma::rsrc_words w_rs;
+    fa_lds_dma::rsrc_words w_rs, w_joined[S::WR];       // (JOINED: of each request's matrix, as a wave's requests may be of two)
+    uint32_t w_bytes[S::WR];
     if constexpr (S::JOINED) {
-        // one descriptor over all matrices, which lie within 4 GiB (the host has seen to that)
-        w_rs = fa_lds_dma::make_rsrc_words(a.w_low, a.w_span);
 #pragma unroll
         for (int i = 0; i < S::WR; ++i) {
             const uint32_t q = wave * S::WR + i, u = S::CANON ? q % (S::W_REQ / 2) : q;
             const uint32_t row = S::CANON ? u * 16 + (lane >> 2) : u * 8 + (lane >> 3);  // of the tile
             uint32_t r = min(n0 + (S::CANON ? u * 16 : u * 8), rows0 + 2 * rows1 - (S::CANON ? 16 : 8));  // (rows past the end: the last ones again)
             const int mat = matrix_of(r);
-            const uint32_t at = pick3(mat, a.w_at[0], a.w_at[1], a.w_at[2]), wr = paired(r + (S::CANON ? lane >> 2 : lane >> 3)), rows = mat ? rows1 : rows0;
+            const uint32_t wr = paired(r + (S::CANON ? lane >> 2 : lane >> 3)), rows = mat ? rows1 : rows0;
+            w_bytes[i] = rows * K * 2, w_joined[i] = fa_lds_dma::make_rsrc_words(pick3(mat, a.w[0], a.w[1], a.w[2]), w_bytes[i]);
             if constexpr (S::CANON)
-                wv[i] = (int)(at + w_block[i] * rows * 64 + wr * 64 + ((lane & 3) ^ ((row >> 2) & 3)) * 16), w_step[i] = rows * 128;
+                wv[i] = (int)(w_block[i] * rows * 64 + wr * 64 + ((lane & 3) ^ ((row >> 2) & 3)) * 16), w_step[i] = rows * 128;
             else
-                wv[i] = (int)(at + wr * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16), w_step[i] = 128;
+                wv[i] = (int)(wr * K * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16), w_step[i] = 128;
         }
     } else {
         w_rs = fa_lds_dma::make_rsrc_words(pick3(tile_mat, a.w[0], a.w[1], a.w[2]), N_tile * (K / 8 * S::WB));
@@ -240,7 +242,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         if (r < S::WR) {
             const uint32_t q = (loader * S::WR + r) % S::W_REQ;
             if constexpr (S::JOINED) {
-                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], 0);
+                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_joined[r], base + S::X_BYTES + q * 1024, wv[r], 0);
                 wv[r] += w_step[r];
             } else {
                 const uint32_t soff = S::CANON ? w_soff + (w_block[r] ? w_block_bytes : 0u) : w_soff;
@@ -252,7 +254,13 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         if (r == S::REQ - 1) {  // the step's last one
             ++asked, x_soff += STRIDE * 128, w_soff += STRIDE * w_per_step;
             const bool in = asked < n_steps;
-            x_now.z = in ? x_rs.z : 0u, w_now.z = in ? w_rs.z : 0u;
+            x_now.z = in ? x_rs.z : 0u;
+            if constexpr (S::JOINED) {
+#pragma unroll
+                for (int i = 0; i < S::WR; ++i) w_joined[i].z = in ? w_bytes[i] : 0u;
+            } else {
+                w_now.z = in ? w_rs.z : 0u;
+            }
         }
     };
 

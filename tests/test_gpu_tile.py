@@ -155,6 +155,40 @@ def test_tiles_of_64_weight_rows_by_name(K, H, Hkv, D, m, layout, weights):
         f.set_gemm_variant()
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("order", ["qkv", "kvq", "vqk"])
+def test_weights_anywhere_in_memory(order, layout):
+    """F16 tiles that hold rows of two matrices: the kernel, and so the bits, of a launch do not depend on where the matrices lie. The
+    bar is two f16 units of the result and six roots of 2 n roundings (test_f16_sums_are_added_in_parts) of a chain of 64 products."""
+    announce("weights anywhere", order, layout)
+    f = ctx()
+    K, N, NK, m = 1024, 3072, 1024, 2040
+    rng = np.random.default_rng(K + m + layout)
+    x = rng.normal(size=(m, K)).astype(np.float16)
+    ws = [(rng.normal(size=(n, K)) * K ** -0.5).astype(np.float16) for n in (N, NK, NK)]
+    flat = [orc.to_canonical(w) if layout else w.reshape(-1) for w in ws]
+    far = (1 << 32) + (1 << 20)
+    pool = f.empty((2 * far + N * K * 2,), np.uint8)
+    dx, outs = f.array(x), [f.zeros((m, n)) for n in (N, NK, NK)]
+    got = []
+    for apart in (False, True):
+        at, end = [0, 0, 0], 0
+        for i in ("qkv".index(c) for c in order):
+            at[i], end = end, end + (far if apart else flat[i].nbytes)
+        args = []
+        for w, o in zip(flat, at):
+            fa.check(f.lib.fa_upload(f.h, pool.ptr, o, w.ctypes.data, w.nbytes))
+            args.append(pool.arg(w.shape, offset=o, dtype=fa.DTYPE_F16))
+        f.fused_qkv(dx.arg(), *args, *[o.arg() for o in outs], K, N, NK, m, layout=layout)
+        got.append([o.download() for o in outs])
+    for near, apart, w in zip(*got, ws):
+        assert np.array_equal(bits(near), bits(apart))
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        assert np.all(np.abs(near - want) <= 2.0 ** -9 * np.abs(want) + 6 * 0.42 * 8 * 2.0 ** -24 * np.sqrt(np.mean(want ** 2)) + 2.0 ** -23)
+    for b in [pool, dx] + outs:
+        b.free()
+
+
 @pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
 @pytest.mark.parametrize("K,N,NK,m,panel,finish", [
     (2048, 8192, 1024, 16, True, False),    # one round of workgroups: the panel up to 32 rows
