@@ -485,9 +485,12 @@ __global__ void __launch_bounds__(256) gemm_finish_kernel(GemmDev a) {
 // features), times the rounds of workgroups that the launch has. The larger tiles read less per product, the smaller ones leave
 // fewer CUs idle: 64 x 96 is for 257 to 384 tiles of 64 x 64, which are one round of it (576 rows, 3072 x 2048 F16: 18.4 us as two
 // rounds or as 128 x 64, 16.0 as 64 x 96; 500 rows 3072 x 3072, with a residual, 19.5 -> 15.9, Q8_0 17.6 -> 16.4, Q4_0 17.0 -> 15.4). Three rounds
-// and more of 64 x 96, and of any small F16 tiles, take longer than their number says (1530 rows, 2048 x 3072 F16: 30.4 us in three
-// rounds of 64 x 96, 26.3 in one of 256 x 128; 1300 rows, 3072 x 3072 37.7 in four of 64 x 64, 33.7). Over 730 launches of 130 to 2200
-// rows the choice is on average within 0.1 % (F16), 0.5 % (block-quantised) of the best shape, 1.5 to 2 % without 64 x 96. `joined`: tiles may hold rows of two matrices. `variant`: a shape asked for by name (fa_set_gemm_variant).
+// and more of 64 x 96, and of any small F16 tiles, take longer than their number says (2079 rows, 2048 x 2048 F16: 30.8 us in three
+// rounds of 64 x 96, 27.5 in two of 128 x 128). It moves no F16 launch from the tiles that add their sums up in parts (fa_tile.h) to the
+// larger ones, which do not: 1300 rows, 3072 x 3072 take 33.7 us in one round of 256 x 128 and 37.7 in four of 64 x 64, but with errors
+// of 5.9 x 2^-24 of the sums' size in place of 2.2. Over 730 launches of 130 to 2200 rows the choice is on average within 0.1 % (F16), 0.5 %
+// (block-quantised) of the best shape, 1.5 to 2 % without 64 x 96. `joined`: tiles may hold rows of two matrices. `variant`: a shape
+// asked for by name (fa_set_gemm_variant).
 static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint32_t n_cus, bool joined, uint32_t variant, fa_tile::TileShape &shape) {
     struct Choice {
         fa_tile::TileShape shape;
@@ -500,7 +503,7 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
                                      {fa_tile::TILE_128x128, 128, 128, 2.6f, 2.7f},
                                      {fa_tile::TILE_256x128, 256, 128, 4.65f, 4.3f},
                                      {fa_tile::TILE_256x160, 256, 160, 6.3f, 0.0f}};
-    float best = 0.0f;
+    float best = 0.0f, in_parts = 0.0f;  // (in_parts: the least by rounds alone of 64 x 64, 128 x 64 and 128 x 128, which come first)
     for (const Choice &c : choices) {
         if (c.shape == fa_tile::TILE_256x160 && !joined) continue;
         // (a block-quantised tile's scales lie in LDS over the whole of k_dim)
@@ -513,6 +516,8 @@ static float best_tile(const FusedQkvLaunch &l, const uint32_t (&rows)[3], uint3
         const uint64_t tiles = (uint64_t)n_tiles * ceil_div_u32(l.m, c.m);
         const uint64_t rounds = (tiles + n_cus - 1) / n_cus;
         float cost = (float)rounds * (l.weight_bits == 16 ? c.f16 : c.quantised);
+        if (l.weight_bits == 16 && c.m * c.n > 128 * 128 && in_parts != 0.0f && cost >= in_parts) continue;
+        if (c.m * c.n <= 128 * 128 && c.shape != fa_tile::TILE_64x96) in_parts = in_parts == 0.0f ? cost : std::min(in_parts, cost);
         if (rounds >= 3 && (c.shape == fa_tile::TILE_64x96 || (l.weight_bits == 16 && c.m * c.n < 128 * 128))) cost *= 1.2f;
         if (best == 0.0f || cost < best) {
             best = cost, shape = c.shape;

@@ -341,17 +341,17 @@ def test_scales_at_any_half(K, m, weights):
         b.free()
 
 
-@pytest.mark.parametrize("K,m,variant", [(3072, 300, 0), (3072, 300, 1), (3072, 300, 2), (2048, 1500, 0), (3104, 300, 0)])
-def test_f16_sums_are_added_in_parts(K, m, variant):
+@pytest.mark.parametrize("K,m,variant,N", [(3072, 300, 0, 256), (3072, 300, 1, 256), (3072, 300, 2, 256), (2048, 1500, 0, 256), (3104, 300, 0, 256),
+                                           (2048, 1300, 0, 3072), (1536, 1600, 0, 2560)])
+def test_f16_sums_are_added_in_parts(K, m, variant, N):
     """The f32 sums of F16 weights behind the output's rounding: out = sums - f16(exact), so that what is left shows them to 2^-24.
     A chain of n matrix products of 16 features rounds 2 n times by 0.42 x 2^-24 rms of a partial sum that is half the final one in
     the mean square: 0.42 sqrt(n) x 2^-24 of the sums' size, 1.7 for parts of 256 features; adding N / 256 parts up rounds by
     0.42 sqrt(N / 512), 1.0 over 3072. Together 2.0, the bar 1.5 times that; one chain over 2048 features would be 4.7, over 3072
     5.8."""
-    announce("F16 sums", K, m, variant)
+    announce("F16 sums", K, m, variant, N)
     f = ctx()
     rng = np.random.default_rng(K + m)
-    N = 256
     x = rng.normal(size=(m, K)).astype(np.float16)
     w = (rng.normal(size=(N, K)) * K ** -0.5).astype(np.float16)
     exact = x.astype(np.float64) @ w.astype(np.float64).T
