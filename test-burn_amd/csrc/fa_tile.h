@@ -39,8 +39,14 @@
 //     added in a second launch (2.2 x 2^-24), add their accumulators to a second set every FOLD steps, between the products, for
 //     0.5 to 1 % of the time: 2.1 to 2.2 x 2^-24 (1.9 over 896 features, 3.3 in one chain). The larger tiles have no registers for
 //     that, and the launches that they took over had one chain as well. Block-quantised weights are rounded to f16 with their scale,
-//     2^-12 of each operand, beside which a chain's error does not count (1000 x 2^-24 of the sums' size with either); a second set
-//     would cost them 3 to 5 %.
+//     2^-12 of each operand, beside which a chain's error is small (1000 x 2^-24 of the sums' size with either). Their waves have
+//     SETS of accumulators that a wave's products go to in turn, so that a sum is KG * SETS chains and no launch is less exact than
+//     where it was before it came to these tiles (the 128 x 64 tiles' four chains for 64 x 96, the panel kernel's eight for a chunk
+//     with a norm). Q8_0, one set and two, x 2^-24: 340 rows, 3072 x 3072 3.5 -> 2.4; 200 rows, 2048 x 2048 2.0 -> 1.6; FusedQkv
+//     100 rows, 2112 x 1280 1.7 -> 1.4, 416 rows, 3072 x 896 1.7 -> 1.4 (on the panel kernel 1.5, 1.45). Q4_0's products are of
+//     fewer bits: two sets where KG is 2 (1.1 to 1.8). It costs 0.4 % of the launches with Q8_0 weights in the mean over 40 of them, up to
+//     0.5 us where eight accumulators more are cleared and added up (577 rows, 1600 x 1536 9.1 -> 9.6), 0.2 % with Q4_0; adding a
+//     second set up every few steps instead costs 5 to 9 %.
 // F16 sums run over the features in order, whatever the tile: the shapes up to 128 x 128, and the register-staged kernel, agree to
 // the bit.
 #pragma once
@@ -76,6 +82,8 @@ struct Shape {
     static constexpr bool OWN = OWN_;
     static_assert(!OWN || (QUANT && WM == 1 && WN == 1 && KG == 4), "16 bytes of a row's scales are those of a step of each wave");
     static constexpr int FOLD = WB_ == 16 && WM_ * TM_ * WN_ * TN_ <= 16 ? 4 : 0;  // steps, 0: one chain
+    // Sets of accumulators that a wave's products go to in turn (block-quantised; 256 x 128 has no registers for a second one)
+    static constexpr int SETS = QUANT && WM_ * TM_ * WN_ * TN_ <= 16 && (WB_ == 8 || KG_ == 2) ? 2 : 1;
     static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = OWN ? 4 : 4 / KG, LOADERS = OWN ? 1 : NW;  // KN: products of 16 features per wave and stage
     static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
     static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
@@ -211,7 +219,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     const fa_lds_dma::rsrc_words x_rs = fa_lds_dma::make_rsrc_words(reinterpret_cast<const unsigned char *>(a.x) + (size_t)m0 * K * 2, (a.m - m0) * K * 2);
     const uint32_t w_block_bytes = N_tile * 4 * S::WB;  // canonical: one 32-feature block of the matrix
     uint32_t w_step[S::WR];                             // JOINED: bytes between the steps of a request's matrix
-    fa_lds_dma::rsrc_words w_rs, w_joined[S::WR];       // (JOINED: of each request's matrix, as a wave's requests may be of two)
+    fa_lds_dma::rsrc_words w_rs = {}, w_joined[S::WR];     // (JOINED: of each request's matrix, as a wave's requests may be of two)
     uint32_t w_bytes[S::WR];
     if constexpr (S::JOINED) {
 #pragma unroll
@@ -323,13 +331,15 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         }
     };
 
-    f16v_t acc[S::TN][S::TM], sums[S::TN][S::TM];  // (FOLD: of the last steps, and of all before)
+    f16v_t acc[S::SETS][S::TN][S::TM], sums[S::TN][S::TM];  // (FOLD: of the last steps, and of all before)
 #pragma unroll
     for (int i = 0; i < S::TN; ++i)
 #pragma unroll
-        for (int j = 0; j < S::TM; ++j)
+        for (int j = 0; j < S::TM; ++j) {
+            sums[i][j] = f16v_t{};
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = sums[i][j][r] = 0.0f;
+            for (int t = 0; t < S::SETS; ++t) acc[t][i][j] = f16v_t{};
+        }
 
     // The residual, asked for ahead of everything else where the tile leaves registers for it: at the end of the one chain that a
     // launch of a round of such tiles is, it would be a trip to memory more (3072 x 3072, 320 rows: F16 12.8 -> 12.3 us, Q8_0 12.2 ->
@@ -372,7 +382,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     // the operands of step ks in registers - their stage is free for step ks + NS - and step ks + 1 has landed for everybody.
     // The requests go out between the products: the memory unit takes a KiB in about 20 cycles, and a wave that issues all of its
     // requests in one go leaves its matrix core idle for as long.
-    auto step = [&](uint32_t cur, uint32_t next, int ks4, bool fold, const Operands &now, Operands &then) __attribute__((always_inline)) {
+    auto step = [&](uint32_t cur, uint32_t next, int ks4, int set, bool fold, const Operands &now, Operands &then) __attribute__((always_inline)) {
         wait_requests<S::REQ *(S::NS - 2)>();
         if constexpr (S::OWN) __builtin_amdgcn_s_waitcnt(0xC07F);  // (lgkmcnt(0): the operands have left the stage that is asked for again)
         else meet();
@@ -385,9 +395,10 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 #pragma unroll
             for (int e = p * S::READS / NM; e < (p + 1) * S::READS / NM; ++e) fetch(then, next, e);
             if (j == 0) fa[i] = w_operand(now, i, q, ks4);
-            f16v_t chain = acc[i][j];
+            f16v_t &sum = acc[(set + q) % S::SETS][i][j];
+            f16v_t chain = sum;
             if (fold && q == 0) sums[i][j] += chain, chain = f16v_t{};
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], now.x[j][q], chain, 0, 0, 0);
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], now.x[j][q], chain, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0x6);  // (vector and scalar arithmetic may move: addresses, the conversion of weights)
 #pragma unroll
             for (int r = p * S::REQ / NM; r < (p + 1) * S::REQ / NM; ++r) request(r, cur);
@@ -396,6 +407,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     };
     // (unrolled over the stages, so that their places are constants; operands of even and odd steps in registers of their own)
     constexpr int UNROLL = (S::QUANT && !S::OWN) || S::FOLD ? S::NS * 4 / (S::NS % 4 == 0 ? 4 : S::NS % 2 == 0 ? 2 : 1) : S::NS % 2 == 0 ? S::NS : 2 * S::NS;
+    static_assert(UNROLL * S::KN % S::SETS == 0, "the sets come round with the unrolled loop");
     for (uint32_t left = n_steps;;) {
         bool done = false;
         if (S::OWN && left == 0) break;  // (a wave without a step)
@@ -403,8 +415,8 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         for (int u = 0; u < UNROLL; ++u) {
             const uint32_t cur = u % S::NS * S::STAGE, next = (u + 1) % S::NS * S::STAGE;
             const bool fold = S::FOLD != 0 && u % 4 == 3;
-            if (u % 2 == 0) step(cur, next, u % 4, fold, o0, o1);
-            else step(cur, next, u % 4, fold, o1, o0);
+            if (u % 2 == 0) step(cur, next, u % 4, u * S::KN % S::SETS, fold, o0, o1);
+            else step(cur, next, u % 4, u * S::KN % S::SETS, fold, o1, o0);
             if (--left == 0) {
                 done = true;
                 break;
@@ -417,8 +429,14 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 #pragma unroll
         for (int i = 0; i < S::TN; ++i)
 #pragma unroll
-            for (int j = 0; j < S::TM; ++j) acc[i][j] = sums[i][j] + acc[i][j];
+            for (int j = 0; j < S::TM; ++j) acc[0][i][j] = sums[i][j] + acc[0][i][j];
     }
+#pragma unroll
+    for (int t = 1; t < S::SETS; ++t)
+#pragma unroll
+        for (int i = 0; i < S::TN; ++i)
+#pragma unroll
+            for (int j = 0; j < S::TM; ++j) acc[0][i][j] += acc[t][i][j];
 
     // Write stage: accumulators -> LDS as f32 [input row][weight row], 32 input rows of every wave at a time, then
     // alpha * sum + bias + beta * residual, one rounding to f16, 16-byte stores (or the rotation and the stores of KvPrepFused).
@@ -432,7 +450,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             for (int i = 0; i < S::TN; ++i)
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    const f4v_t q = {acc[i][j][g * 4 + 0], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+                    const f4v_t q = {acc[0][i][j][g * 4 + 0], acc[0][i][j][g * 4 + 1], acc[0][i][j][g * 4 + 2], acc[0][i][j][g * 4 + 3]};
                     *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + ((wm * S::TJ + j - j0) * 32 + r32) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + g * 8 + h * 4) * 4) = q;
                 }
         __syncthreads();

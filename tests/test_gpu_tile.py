@@ -366,3 +366,32 @@ def test_f16_sums_are_added_in_parts(K, m, variant, N):
     assert np.sqrt(np.mean(err ** 2) / np.mean(exact ** 2)) * 2 ** 24 <= 3.0, np.sqrt(np.mean(err ** 2) / np.mean(exact ** 2)) * 2 ** 24
     for b in (dx, dw, dres, dout):
         b.free()
+
+
+@pytest.mark.parametrize("K,m,N,chains", [
+    (3072, 340, 3072, 4),  # 64 x 96 tiles
+    (896, 200, 4864, 4),
+    (4096, 288, 4096, 4),
+    (2048, 200, 2048, 8),  # 64 x 64 with steps of each wave's own
+    (1088, 400, 3072, 4),
+])
+def test_quantised_sums_are_several_chains(K, m, N, chains):
+    """The f32 sums of Q8_0 weights whose scales are powers of two (their products with the weights are exact), as in
+    test_f16_sums_are_added_in_parts: chains of n products of 16 features round by 0.42 sqrt(n) x 2^-24 of the sums' size, the output
+    (f16 of a remainder of 2^-11 of them at most, uniform) by 0.7. With half as many chains the first is 1.41 times that."""
+    announce("quantised sums", K, m, N, chains)
+    f = ctx()
+    rng = np.random.default_rng(K + m)
+    x = rng.normal(size=(m, K)).astype(np.float16)
+    q = np.clip(np.round(rng.normal(size=(N, K)) * 36), -127, 127).astype(np.int8)
+    s = (2.0 ** rng.integers(-11, -9, size=(N, K // 32))).astype(np.float16)
+    full = q.astype(np.float64) * np.repeat(s.astype(np.float64), 32, axis=1)
+    exact = x.astype(np.float64) @ full.T
+    rounded = exact.astype(np.float16)
+    dx, dw, ds, dres, dout = f.array(x), f.array(q.reshape(-1)), f.array(s), f.array(-rounded), f.zeros((m, N))
+    f.matmul(dx.arg(), dw.arg(), dout.arg(), m, N, K, c=dres.arg(), transpose_b=True, beta=1.0, b_scales=ds.arg())
+    err = dout.download().astype(np.float64) - (exact - rounded.astype(np.float64))
+    rel = np.sqrt(np.mean(err ** 2) / np.mean(exact ** 2)) * 2 ** 24
+    assert rel <= np.sqrt(0.49 + 0.42 ** 2 * K / 16 / chains), rel
+    for b in (dx, dw, ds, dres, dout):
+        b.free()
