@@ -91,14 +91,24 @@ def test_attention_block_stage_by_stage_and_end_to_end(m, prefix, q8):
         b.free()
 
 
+@pytest.mark.parametrize("attention", ["flash_rows_kernel", "flash_chunk_kernel"])
 @pytest.mark.parametrize("mode,paired_prefix", [(fa.ROPE_NORMAL, 2100), (fa.ROPE_NEOX, 2049)])
-def test_prefill_chunk_block_as_graph_replays(mode, paired_prefix):
+def test_prefill_chunk_block_as_graph_replays(mode, paired_prefix, attention):
     """The attention block of the reference's default prefill mode (a chunk of 32 rows after a prefix,
-    src/model/executor.rs:232-250) on the kernels that shape takes - FusedQkv + KvPrepFused as ONE launch, the short-chunk
-    attention kernel, the one-launch o_proj - captured as a HIP graph and replayed: every replay against the oracle's chain on
-    the same inputs (the chunk's cache rows are rewritten with the same values by every replay)."""
-    announce("prefill chunk block, graph replays", mode, paired_prefix)
+    src/model/executor.rs:232-250) on the kernels that shape takes - FusedQkv + KvPrepFused as ONE launch, the attention kernel that
+    gives 32 rows to a workgroup (and, asked for by name, the short-chunk one), the one-launch o_proj - captured as a HIP graph and
+    replayed: every replay against the oracle's chain on the same inputs (the chunk's cache rows are rewritten with the same values by
+    every replay)."""
+    announce("prefill chunk block, graph replays", mode, paired_prefix, attention)
     f = ctx()
+    f.set_prefill_variant(3 if attention == "flash_chunk_kernel" else 0)
+    try:
+        _chunk_block_as_graph_replays(f, mode, paired_prefix, attention)
+    finally:
+        f.set_prefill_variant(0)
+
+
+def _chunk_block_as_graph_replays(f, mode, paired_prefix, attention):
     m, prefix = 32, paired_prefix
     H, Hkv, D, cap = 16, 4, 128, prefix + 64
     dm, kvd = H * D, Hkv * D
@@ -129,10 +139,11 @@ def test_prefill_chunk_block_as_graph_replays(mode, paired_prefix):
     try:
         enqueue()
         f.synchronize()
-        counts = {k: f.profile_query(k)[0] for k in ("fused_qkv_rows32_rope_kernel", "flash_chunk_kernel", "matmul_rows32_kernel")}
+        counts = {k: f.profile_query(k)[0] for k in ("fused_qkv_rows32_rope_kernel", "flash_rows_kernel", "flash_chunk_kernel", "matmul_rows32_kernel")}
     finally:
         f.profile_enable(False)
-    assert counts == {"fused_qkv_rows32_rope_kernel": 1, "flash_chunk_kernel": 1, "matmul_rows32_kernel": 1}, counts
+    assert counts == {"fused_qkv_rows32_rope_kernel": 1, "flash_rows_kernel": int(attention == "flash_rows_kernel"),
+                      "flash_chunk_kernel": int(attention == "flash_chunk_kernel"), "matmul_rows32_kernel": 1}, counts
     # the oracle's chain: projections, rotation + append, causal attention of every row, o_proj with residual
     wq, wk, wv = orc.fused_qkv(hidden, *ws, gamma=gamma)
     kw, vw = kc.copy(), vc.copy()

@@ -21,11 +21,10 @@ def _launches(f, call):
     try:
         call()
         f.synchronize()
-        n = {k: f.profile_query(k)[0] for k in ("flash_rows_kernel", "flash_chunk_kernel_rows", "flash_prefill_merge_kernel", "flash_")}
+        n = {k: f.profile_query(k)[0] for k in ("flash_rows_kernel", "flash_prefill_merge_kernel", "flash_")}
     finally:
         f.profile_enable(False)
-    rows = n["flash_rows_kernel"] + n["flash_chunk_kernel_rows"]  # (the second: at most 64 query rows)
-    return rows, n["flash_prefill_merge_kernel"], n["flash_"] - rows - n["flash_prefill_merge_kernel"]
+    return n["flash_rows_kernel"], n["flash_prefill_merge_kernel"], n["flash_"] - n["flash_rows_kernel"] - n["flash_prefill_merge_kernel"]
 
 
 CASES = [
