@@ -436,13 +436,14 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
     // Block-quantised with a norm: where 32 input rows x 32 weight rows are more than a piece per compute unit, a second pass costs 3 us
     // and more, which the estimate below does not see of few features: 195 rows, 512 x 2112 Q4_0 12.0 us, 8.4 with the norm's launch and
-    // the tiles; 391 rows, 640 x 1344 Q8_0 12.1, 9.2; 124 rows, 1280 x 2112 Q8_0 14.4, 9.3; just below the line 192 rows, 512 x 1344 6.2,
-    // 7.2. Of 768 to 1024 features the line is at the third pass (375 rows, 768 x 1664 13.8, 9.6; with two, 287 rows, 896 x 960 9.7, 8.4).
+    // the tiles; 391 rows, 640 x 1344 Q8_0 12.1, 9.2; 124 rows, 1280 x 2112 Q8_0 14.4, 9.3; 375 rows, 768 x 1664 13.8, 9.6; 248 rows,
+    // 896 x 1664 Q4_0 9.65, 8.5; just below the line 192 rows, 512 x 1344 6.2, 7.2. (100 launches of 768 to 1024 features between one
+    // piece and two: 0.71 to 0.975 of the panel kernel's time, 0.87 in the mean; 180 of 256 to 2048 features below the line: 1.09 to 1.32.)
     if (!f16 && l.gamma && l.m > 32 && p.nc == 2 && l.k_dim % 64 == 0 && l.n_dim % 8 == 0 && l.n_kv % 8 == 0) {
         const uint64_t pieces = (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 32) * p.n_pass;
         bool scales_fit = true;  // (what the tiles ask of a launch)
         for (int i = 0; i < 3; ++i) scales_fit = scales_fit && reinterpret_cast<uintptr_t>(l.scales[i]) % 4 == 0;
-        if (scales_fit && pieces > (l.k_dim >= 768 && l.k_dim <= 1024 ? 2 : 1) * n_cus) return false;
+        if (scales_fit && pieces > n_cus) return false;
     }
     // passes of a compute unit (with two workgroups on it they share its way to L2)
     const float passes = p.pk > 2 ? (float)(p.rounds * ceil_div_u32(p.n_pass, p.grid_y)) : std::max(1.0f, (float)(p.grid_x * p.n_pass) / (float)n_cus);

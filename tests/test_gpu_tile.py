@@ -194,9 +194,9 @@ def test_weights_anywhere_in_memory(order, layout):
     (2048, 8192, 1024, 16, True, False),    # one round of workgroups: the panel up to 32 rows
     (2048, 8192, 1024, 48, False, False),   # many weight rows: its passes cost more than the norm's launch and the tiles
     (2048, 2048, 256, 64, True, False),
-    (1024, 4096, 1024, 40, True, False),    # no side a tenth ahead
+    (1024, 4096, 1024, 40, "f16", False),   # no side a tenth ahead (block-quantised: more than one pass per compute unit)
     (1024, 4096, 1024, 100, False, False),
-    (896, 896, 128, 400, True, False),
+    (896, 896, 128, 400, "f16", False),
     (896, 896, 128, 417, False, False),
     (3072, 40, 24, 48, True, False),        # a few weight rows
     (4096, 512, 128, 16, False, None),      # about the line between whole and divided
@@ -210,6 +210,7 @@ def test_route_of_a_chunk(K, N, NK, m, panel, finish, weights):
     (The longest rows without the norm: its f16 roundings differ from the oracle's in isolated elements, 60 in a million, more of
     them in a row of 8192 than the bar allows for, whatever kernel multiplies them.)"""
     announce("route of a chunk", K, N, NK, m, weights)
+    panel = panel is True or panel == weights
     f = ctx()
     rng = np.random.default_rng(K + N + m)
     x, g, ws, bs = _data(rng, K, N, NK, m)
@@ -256,7 +257,8 @@ def _quantised(f, rng, K, N, m, weights):
 @pytest.mark.parametrize("weights", ["q8", "q4"])
 @pytest.mark.parametrize("K,N,NK,m,panel", [
     (640, 896, 192, 192, True), (640, 896, 192, 193, False),     # 240, 280 pieces of 32 x 32 rows
-    (960, 1856, 64, 256, True), (960, 1856, 64, 257, False),     # 496, 558
+    (896, 960, 32, 256, True), (896, 960, 32, 257, False),       # 256, 288
+    (960, 1856, 64, 256, False), (960, 1856, 64, 128, True),     # 496, 248
     (1280, 1984, 64, 124, False),                                # 264
 ])
 def test_route_of_a_quantised_chunk_with_a_norm(K, N, NK, m, panel, weights):
