@@ -734,15 +734,18 @@ ChunkShape chunk_shape(const fa_ctx *ctx, const PrefillLaunch &L, bool force) {
 
 }  // namespace
 
-// By the 64-key rounds of a workgroup, the partitions and the MB of partial sums; 4 to 15 % from 440 launches of 2 to 64 rows after
-// 2000 to 36000 (with at most 4 column blocks two waves share one).
+// By the 64-key rounds of a workgroup and its column blocks (with at most 4 of them two waves share one), the partitions, and the MB of
+// partial sums, which cost a quarter within an XCD; 4 to 6 % (rms) from 700 launches of 2 to 64 rows after 2000 to 100000, keys in memory.
 float fa_prefill_chunk_estimate_us(const fa_ctx *ctx, const PrefillLaunch &L) {
     const ChunkShape c = chunk_shape(ctx, L, false);
     if (c.groups == 0) return 0.0f;
-    const float rounds = (float)ceil_div_u32(c.part_len, 64), S = (float)c.S, mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * S * 4e-6f;
-    const bool few = c.pairs <= 4;
-    if (L.head_dim == 128) return few ? 4.95f + 1.154f * rounds + 0.082f * S + 0.70f * mb : 3.95f + 1.517f * rounds + 0.116f * S + 0.586f * mb;
-    return few ? 5.82f + 0.721f * rounds + 0.035f * S + 0.896f * mb : 7.46f + 1.486f * rounds + 0.010f * S + 0.821f * mb;
+    const float rounds = (float)ceil_div_u32(c.part_len, 64), blocks = (float)c.pairs, S = (float)c.S, mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * S * 4e-6f;
+    const bool few = c.pairs <= 4, local = ctx->xcd_round_robin && c.groups % 8 == 0;
+    if (L.head_dim == 128)
+        return few ? 7.33f + rounds * (1.054f + 0.093f * blocks) + 0.0282f * S + (local ? 0.292f : 0.991f) * mb
+                   : 10.34f + rounds * (1.022f + 0.1604f * blocks) + 0.0277f * S + (local ? 0.149f : 0.713f) * mb;
+    return few ? 5.94f + rounds * (0.701f + 0.0366f * blocks) + 0.0324f * S + (local ? 0.2355f : 0.8885f) * mb
+               : 9.31f + rounds * (0.728f + 0.0908f * blocks) + (local ? 0.014f : 0.76f) * mb;
 }
 
 // Whether the chunk kernel takes this launch (set *taken); when it does, enqueues it.

@@ -1084,15 +1084,18 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     if (L.head_dim != 128 && L.head_dim != 64)
         return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "Prefill only supports head_dim=64 or 128, got %u", L.head_dim);
     // Unless a kernel or a split count has been asked for by name: the kernel that takes 32 rows to a workgroup (fa_rows.hip), for a
-    // chunk of at most 64 rows after a long prefix the memory-bound one (fa_chunk.hip), or the tiled one, by estimate. (What the first
-    // is given it takes ahead of the others by a twentieth or more. Over 2650 shapes of 2 to 8000 rows after 0 to 36000, 4 to 32 heads,
-    // each timed with all three, it was slower than the other choice by more than 3 % for nine, by 14 % at most, and 1.6 times as fast
-    // in the mean. Beyond the keys below nothing is fitted, and the short-chunk kernel reads a KV head's keys once.)
+    // chunk of at most 64 rows after a long prefix the memory-bound one (fa_chunk.hip), or the tiled one, by estimate. (The estimates are
+    // of keys that come from memory, as a layer's do in a model: of long ones that do, the first kernel takes longer (us, rows and the
+    // other: 278 rows after 7179, H24 / Hkv8 / D128 55.3, 48.6; 34 after 47550, H16 / Hkv2 / D128 47.3, 36.7; 18 after 44996, H4 / Hkv4 /
+    // D128 38.7, 24.1), of keys that lie in the last-level cache from the call before the least of all. On 4000
+    // launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, half of them with keys in memory) the
+    // choice takes 1.002 to 1.014 times as long as the best of the three, in the mean, and 0.69 to 0.76 of what the other two would: 48
+    // are slower for it by more than 3 %, by 17 % at most (profiles/prefill_choice.txt).)
     const bool automatic = ctx->prefill_variant == 0 && ctx->prefill_split_k == 0;
     const RowsPlan rows = automatic ? fa_prefill_rows_plan(ctx, L) : RowsPlan();
     if ((automatic || ctx->prefill_variant == 3) && !ctx->prefill_chunk_off) {
         const float chunk_us = rows.waves ? fa_prefill_chunk_estimate_us(ctx, L) : 0.0f;
-        if (chunk_us > 0.0f && rows.us < 0.95f * chunk_us && L.kv_len <= (L.head_dim == 128 ? 20000u : 65536u)) return fa_launch_prefill_rows(ctx, L, rows);
+        if (chunk_us > 0.0f && rows.us < 0.95f * chunk_us) return fa_launch_prefill_rows(ctx, L, rows);
         if (!rows.waves || chunk_us > 0.0f) {
             bool taken = false;
             FA_TRY(fa_launch_prefill_chunk(ctx, L, ctx->prefill_variant == 3, &taken));
@@ -1143,25 +1146,27 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     if (splits > key_tiles) splits = key_tiles;
     if (splits < 1) splits = 1;
     if (rows.waves) {
-        // What the tiled kernel takes: the longest item, in pairs of key tiles, or the items and the pairs of one CU's share; with splits
-        // also the partial states. 6 to 7 % from 1570 launches.
+        // What the tiled kernel takes: the longest item, in pairs of key tiles, or the items and the pairs of one CU's share; with splits or
+        // packed heads the partial states; and the MB of keys and values. 6 to 10 % (rms) from 2650 launches, keys in memory.
         const bool wide = L.head_dim == 128;
         auto pairs_of = [&](uint32_t last_row) -> float {
             const uint64_t end = L.causal ? (uint64_t)last_row + L.query_offset + 1 : L.kv_len;
             return (float)ceil_div_u32(ceil_div_u32(ceil_div_u32((uint32_t)(end < L.kv_len ? end : L.kv_len), BN), splits), 2);
         };
         const float longest = pairs_of(L.q_len - 1), first = pairs_of(L.q_len < BM ? L.q_len - 1 : BM - 1), share = (float)base_wgs / (float)n_cus;
+        const float kv_mb = (float)L.n_kv_heads * (float)L.kv_len * (float)L.head_dim * 4e-6f, mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * (float)splits * 4e-6f;
         float us;
-        if (splits > 1) {
-            const float mb = (float)L.n_heads * (float)L.q_len * (float)L.head_dim * (float)splits * 4e-6f;
-            us = wide ? 7.49f + 1.657f * longest + 0.709f * mb : 6.80f + 1.12f * longest + 0.84f * mb;
+        if (a.pack_heads) {
+            us = wide ? 6.17f + 1.56f * longest + 0.825f * mb + 0.144f * (float)splits + 0.0444f * kv_mb
+                      : 5.34f + 1.24f * longest + 1.03f * mb + 0.116f * (float)splits + 0.0108f * kv_mb;
+        } else if (splits > 1) {
+            us = wide ? 7.81f + 1.72f * longest + 0.604f * mb + 0.0781f * kv_mb : 7.40f + 1.07f * longest + 0.805f * mb + 0.0615f * kv_mb;
         } else {
-            const float one = wide ? -1.44f + 1.537f * longest : -0.73f + 1.149f * longest;
-            const float cu = wide ? share * (4.2f + 0.993f * (first + longest)) : share * (2.02f + 0.668f * (first + longest));
-            us = (wide ? 7.30f : 5.94f) + (one > cu ? one : cu);
+            const float one = (wide ? 1.416f : 1.108f) * longest;
+            const float cu = wide ? share * (3.52f + 1.041f * (first + longest)) : share * (2.66f + 0.66f * (first + longest));
+            us = (wide ? 6.41f : 5.43f) + (one > cu ? one : cu) + (wide ? 0.147f : 0.0775f) * kv_mb;
         }
-        // (packed heads: up to 64 rows, for which the other kernel was ahead wherever it was timed, up to 50000 keys)
-        if (a.pack_heads ? L.kv_len <= 49152u : rows.us < 0.95f * us) return fa_launch_prefill_rows(ctx, L, rows);
+        if (rows.us < us) return fa_launch_prefill_rows(ctx, L, rows);
     }
     a.splits = splits, a.part_acc = nullptr, a.part_ml = nullptr;
     if (splits > 1) {

@@ -348,11 +348,15 @@ void launch_rows(FaLaunchScope &scope, const RowsDev &a, uint32_t grid, bool bf1
 
 }  // namespace
 
-// How the kernel would be launched, and what that takes by estimate: fitted to 3000 shapes (2 to 8000 rows after 0 to 36000, 4 to 32
-// heads, each timed with every choice and with the tiled and the short-chunk kernel), within 7 to 12 % of them.
+// How the kernel would be launched, and what that takes by estimate: fitted to 2664 shapes (2 to 8000 rows after 0 to 100000, 14
+// combinations of heads, each timed with every choice, with the tiled and with the short-chunk kernel, over as many layers' caches as
+// put the keys in memory and not in a cache), within 5 to 7 % (rms) of the times that are near the best.
 //   one launch: the time of the workgroup with the most keys, or of the compute unit with the most work: its n-th workgroup is
 //   the launch's 256 n-th, later ones have fewer keys; and the tiles of all units together (their L2, their clock);
-//   keys split: the longest workgroup, and the merge launch by the splits and the MB of partial states.
+//   keys split: the longest workgroup, and the merge launch by the splits and the MB of partial states;
+//   both: the MB of keys and values (of a layer; from 9 MB on the layers of a model no longer fit the last-level cache, and a unit's only
+//   workgroup waits for memory in each round of its waves), and, split, what of them an XCD draws (a block's splits lie on one: with
+//   few blocks the other XCDs have none).
 // 8 waves, one workgroup to a CU at D 128 and two at D 64, are faster up to 256 workgroups, 4 waves (two and four) beyond.
 // H24 / Hkv8 / D128, us with 8 and 4 waves: 256 rows after 2000 15.6, 15.5; 500 rows 11.2, 8.3; 500 after 1000 20.6, 17.8.
 // H14 / Hkv2 / D64: 500 after 1000 7.5, 8.5; 1000 rows 7.7, 7.3; 2048 rows 17.9, 16.2.
@@ -379,15 +383,22 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float all = (float)wgs * (float)(longest + tiles(0)) / (float)(2 * n_cus);
     auto larger = [](float x, float y) { return x > y ? x : y; };
     const float r8 = (float)ceil_div_u32(longest, 8), r4 = (float)ceil_div_u32(longest, 4);
-    const float us8 = wide ? 1.36f + larger(1.41f * r8, 3.3f * n + 0.115f * chain + 0.047f * all) : 2.68f + larger(0.63f * r8, 0.98f * n + 0.028f * chain + 0.068f * all);
-    const float us4 = wide ? 3.04f + larger(0.62f * r4, 0.94f * n + 0.152f * chain + 0.012f * all) : 2.79f + larger(0.43f * r4, 0.88f * n + 0.016f * chain + 0.074f * all);
+    const float head_mb = (float)longest * (float)(KT * L.head_dim) * 4e-6f, kv_mb = head_mb * (float)L.n_kv_heads;
+    const bool waited = wgs <= n_cus && kv_mb > 9.0f;
+    const float us8 = wide ? 2.65f + larger(1.24f * r8, 2.53f * n + 0.137f * chain + 0.0265f * all) + (waited ? 0.386f : 0.03f) * kv_mb
+                           : 3.08f + larger(0.629f * r8, 0.857f * n + 0.0707f * chain + 0.02f * all) + (waited ? 0.206f : 0.055f) * kv_mb;
+    const float us4 = wide ? 4.19f + larger(0.61f * r4, 0.487f * n + 0.122f * chain + 0.0515f * all) + (waited ? 0.536f : 0.065f) * kv_mb
+                           : 3.25f + larger(0.453f * r4, 0.271f * n + 0.0556f * chain + 0.0408f * all) + (waited ? 0.232f : 0.074f) * kv_mb;
     plan.waves = us4 < us8 ? 4 : 8, plan.us = us4 < us8 ? us4 : us8, plan.splits = 1;
     // Keys split: all workgroups resident at once, one to a CU. (The merge launch reads the splits of a row 4, 8, 16 or 32 at a time.)
     float best = plan.us / 1.05f;
     const uint32_t most = n_cus / (ceil_div_u32(wgs, 8) * 8);
+    const uint32_t twos = L.n_kv_heads & (0u - L.n_kv_heads), xcd_heads = L.n_kv_heads / (twos < 8 ? twos : 8), xcd_blocks = ceil_div_u32(wgs, 8);
+    const float xcd_mb = head_mb * (float)(xcd_heads < xcd_blocks ? xcd_heads : xcd_blocks);
     for (uint32_t s = 2; s <= most && s * 4 <= longest && s <= 32; s = s == 16 ? 32 : s + 1) {
         const float r = (float)ceil_div_u32(ceil_div_u32(longest, s), 8), mb = (float)wgs * (float)(32 * L.head_dim) * (float)s * 4e-6f;
-        const float us = wide ? 4.2f + 1.41f * r + 0.148f * (float)s + 0.82f * mb : 4.06f + 0.67f * r + 0.131f * (float)s + 0.77f * mb;
+        const float us = wide ? 5.77f + 1.464f * r + 0.0768f * (float)s + 0.549f * mb + 0.0547f * kv_mb + 0.35f * xcd_mb
+                              : 5.28f + 0.644f * r + 0.0752f * (float)s + 0.4585f * mb + 0.0584f * kv_mb + 0.41f * xcd_mb;
         if (us < best) best = us, plan.us = us, plan.splits = s, plan.waves = 8;
     }
     return plan;
