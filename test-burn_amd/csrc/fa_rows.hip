@@ -18,7 +18,8 @@
 // It reads a block's keys once per 32 rows, 131 KB/us and CU along the rows (fa_lds_dma.h), which is why long keys under many rows
 // stay with the tiled kernel (once per 128 rows): fa_prefill_rows_plan. us before and now (tiled or short-chunk kernel before):
 //   H14 / Hkv2 / D64:   32 rows after 500 10.7 -> 4.6; 500 after 1000 14.9 -> 7.5; 2048 rows 22.7 -> 16.2; 32 after 8160 21.0 -> 9.3
-//   H24 / Hkv8 / D128:  32 after 500 12.6 -> 6.9; 128 after 1000 16.8 -> 9.5; 500 rows 12.6 -> 8.3; 32 after 8160 17.6 -> 13.0
+//   H24 / Hkv8 / D128:  32 after 500 12.6 -> 6.9; 128 after 1000 16.8 -> 9.5; 500 rows 12.6 -> 8.3; 32 after 8160 17.6 -> 13.0 (those from the
+//                       last-level cache; from memory 18.3, the short-chunk kernel 16.9)
 //   H16 / Hkv2 / D128:  500 after 1000 23.8 -> 12.2; 32 after 8160 32.6 -> 12.6
 // (The splits combined by the last workgroup of a block to finish, in the launch: 12.8 to 16.3 us for the last of these, against
 // 12.6 with the merge launch - one compute unit reads all of the block's states there.)
