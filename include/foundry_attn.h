@@ -551,7 +551,8 @@ fa_status fa_matmul(fa_ctx *ctx, const fa_tensor_arg *a, const fa_tensor_arg *b,
  * Environment: FOUNDRY_ATTN_GEMM_MIN_M (read at fa_ctx_create). */
 fa_status fa_set_gemm_min_m(fa_ctx *ctx, uint32_t min_m);
 
-/* Which GEMM kernel fa_fused_qkv / fa_matmul use (F16 results are bit-equal): 1 = operand tiles of 128 x 128 staged
+/* Which GEMM kernel fa_fused_qkv / fa_matmul use (F16 results are bit-equal, except where 0 takes tiles of 256 x 128 or
+ * 256 x 160, which add a sum up in one chain and not every 256 features): 1 = operand tiles of 128 x 128 staged
  * through registers (any shape, every weight policy); 2 = tiles of 128 x 128 loaded from memory straight into LDS; 3 =
  * the same with tiles of 64 x 64; 0 (default) = the tile by the number of output tiles that the launch has. 2 and 3 need
  * k_dim a multiple of 64, weight rows that are multiples of 8, 16-byte aligned outputs and operands below 2 GiB, and fall
