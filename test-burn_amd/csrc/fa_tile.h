@@ -44,9 +44,10 @@
 //     where it was before it came to these tiles (the 128 x 64 tiles' four chains for 64 x 96, the panel kernel's eight for a chunk
 //     with a norm). Q8_0, one set and two, x 2^-24: 340 rows, 3072 x 3072 3.5 -> 2.4; 200 rows, 2048 x 2048 2.0 -> 1.6; FusedQkv
 //     100 rows, 2112 x 1280 1.7 -> 1.4, 416 rows, 3072 x 896 1.7 -> 1.4 (on the panel kernel 1.5, 1.45). Q4_0's products are of
-//     fewer bits: two sets where KG is 2 (1.1 to 1.8). It costs 0.4 % of the launches with Q8_0 weights in the mean over 40 of them, up to
-//     0.5 us where eight accumulators more are cleared and added up (577 rows, 1600 x 1536 9.1 -> 9.6), 0.2 % with Q4_0; adding a
-//     second set up every few steps instead costs 5 to 9 %.
+//     fewer bits: two sets where KG is 2 (1.1 to 1.8). It costs 1 % of the launches with Q8_0 weights in the mean over 74 of them, up to
+//     0.5 us where 64 accumulators more are cleared and added up (577 rows, 1600 x 1536 9.1 -> 9.6), 0.2 % with Q4_0; adding a
+//     second set up every few steps instead costs 5 to 9 %. The larger tiles took no launch from a kernel of more chains, and 128 x 64
+//     and 128 x 128 tiles would be 1 to 2 % slower with two sets.
 // F16 sums run over the features in order, whatever the tile: the shapes up to 128 x 128, and the register-staged kernel, agree to
 // the bit.
 #pragma once
@@ -82,8 +83,8 @@ struct Shape {
     static constexpr bool OWN = OWN_;
     static_assert(!OWN || (QUANT && WM == 1 && WN == 1 && KG == 4), "16 bytes of a row's scales are those of a step of each wave");
     static constexpr int FOLD = WB_ == 16 && WM_ * TM_ * WN_ * TN_ <= 16 ? 4 : 0;  // steps, 0: one chain
-    // Sets of accumulators that a wave's products go to in turn (block-quantised; 256 x 128 has no registers for a second one)
-    static constexpr int SETS = QUANT && WM_ * TM_ * WN_ * TN_ <= 16 && (WB_ == 8 || KG_ == 2) ? 2 : 1;
+    // Sets of accumulators that a wave's products go to in turn (block-quantised tiles of up to 64 x 96)
+    static constexpr int SETS = QUANT && WM_ * TM_ * WN_ * TN_ <= 6 && (WB_ == 8 || KG_ == 2) ? 2 : 1;
     static constexpr int NW = WM * WN * KG, NT = NW * 64, KN = OWN ? 4 : 4 / KG, LOADERS = OWN ? 1 : NW;  // KN: products of 16 features per wave and stage
     static constexpr int MT = WM * TM * 32, NTR = WN * TN * 32;         // input rows and weight rows of the tile
     static constexpr int X_BYTES = MT * 128, W_BYTES = NTR * 8 * WB, STAGE = X_BYTES + W_BYTES;
