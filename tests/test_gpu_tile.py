@@ -22,6 +22,7 @@ pytestmark = pytest.mark.gpu
     (128, 16, 2, 64, 1030, 1),    # 128 x 64 tiles
     (576, 14, 2, 64, 2047, 0),    # 128 x 128 tiles
     (128, 40, 8, 64, 1000, 1),    # 256 x 128 tiles
+    (320, 40, 8, 64, 1000, 0),
     (192, 32, 4, 64, 520, 1),     # 64 x 96 tiles, both ops; the last one a third full, K and V of two thirds of one
     (192, 32, 4, 64, 520, 0),
     (1088, 16, 2, 128, 577, 1),   # and Q4_0 with steps of each wave's own, seventeen of them
