@@ -78,6 +78,14 @@ __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff,
     } \
 }
 FA_LDS_DMA_DEFINE(buffer_to_lds_b128, "")
+// One such load to lds_addr + ahead, a number that is known when the kernel is built: for loops with more places in LDS than there
+// are scalar registers to keep their addresses in.
+__device__ __forceinline__ void buffer_to_lds_b128_ahead(rsrc_words rs, uint32_t lds_addr, uint32_t ahead, int voff, int soff) {
+    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff), "i"(ahead)
+                 : "memory", "scc");
+}
 FA_LDS_DMA_DEFINE(buffer_to_lds_b128_nt, " nt")
 #undef FA_LDS_DMA_DEFINE
 

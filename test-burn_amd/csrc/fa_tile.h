@@ -246,19 +246,21 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     uint32_t asked = 0, x_soff = S::OWN ? wave * 128 : 0, w_soff = S::OWN ? wave * w_per_step : 0;
     fa_lds_dma::rsrc_words x_now = x_rs, w_now = w_rs;
     if (S::OWN && n_steps == 0) x_now.z = 0u, w_now.z = 0u;
+    const uint32_t x_lds = lds_base + loader * S::XR * 1024, w_lds = lds_base + S::X_BYTES + loader * S::WR * 1024;  // (JOINED)
     auto request = [&](int r, uint32_t stage) __attribute__((always_inline)) {
         const uint32_t base = lds_base + stage;
         if (r < S::WR) {
             const uint32_t q = (loader * S::WR + r) % S::W_REQ;
             if constexpr (S::JOINED) {
-                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_joined[r], base + S::X_BYTES + q * 1024, wv[r], 0);
+                fa_lds_dma::buffer_to_lds_b128_ahead(w_joined[r], w_lds, stage + r * 1024, wv[r], 0);
                 wv[r] += w_step[r];
             } else {
                 const uint32_t soff = S::CANON ? w_soff + (w_block[r] ? w_block_bytes : 0u) : w_soff;
                 fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
             }
         } else {
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, S::X_EVEN ? base + (loader * S::XR + r - S::WR) * 1024 : base + (loader * S::XR + r - S::WR) % S::X_REQ * 1024, xv[r - S::WR], (int)x_soff);
+            if constexpr (S::JOINED) fa_lds_dma::buffer_to_lds_b128_ahead(x_now, x_lds, stage + (r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
+            else fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, S::X_EVEN ? base + (loader * S::XR + r - S::WR) * 1024 : base + (loader * S::XR + r - S::WR) % S::X_REQ * 1024, xv[r - S::WR], (int)x_soff);
         }
         if (r == S::REQ - 1) {  // the step's last one
             ++asked, x_soff += STRIDE * 128, w_soff += STRIDE * w_per_step;
