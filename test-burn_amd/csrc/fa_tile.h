@@ -105,6 +105,7 @@ struct Shape {
         return s > (uint32_t)(KG * T_BYTES) ? s : (uint32_t)(KG * T_BYTES);
     }
     static_assert(X_BYTES % 1024 == 0 && W_BYTES % 1024 == 0, "whole requests");
+    static_assert(!JOINED || (X_EVEN && W_REQ % LOADERS == 0), "a wave's requests fill one run of LDS");
     static_assert(lds_bytes(0) <= 160 * 1024 && REQ * (NS - 1) <= 63, "LDS of a compute unit; the request counter");
 };
 
