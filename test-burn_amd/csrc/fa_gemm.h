@@ -2,6 +2,7 @@
 // conversion of block-quantised weights, and how the tile kernels are launched.
 #pragma once
 #include "fa_internal.h"
+#include "fa_norm.h"
 #include "fa_qkv_rope.h"
 #include "fa_quant.h"
 
@@ -27,7 +28,36 @@ struct GemmDev {
     uint32_t k_splits, steps_per_split, n_total;
     float *partial;
     RopeDev rope;
+    uint32_t page_shift;  // log2 of rope.block_size, 32 = not a power of two
 };
+
+// Rotation of the piece hd .. hd + 7 of a head: the first table column that it takes, the columns (adjacent pairs (hd + 2i, hd + 2i + 1):
+// 4 of them, from hd / 2; pairs (hd, hd + D / 2): 8, from hd mod D / 2), and the piece rotated with them.
+__device__ __forceinline__ uint32_t rope_column(const RopeDev &r, uint32_t hd) { return r.normal ? hd >> 1 : hd & ((r.head_dim >> 1) - 1u); }
+__device__ __forceinline__ void rope_columns(const RopeDev &r, uint32_t table_row, uint32_t column, h8_t &c, h8_t &s) {
+    typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
+    const size_t at = (size_t)table_row * (r.head_dim >> 1) + column;
+    if (r.normal) {
+        const h4v_t c4 = fa_norm::load_global<h4v_t>(r.cos_t + at), s4 = fa_norm::load_global<h4v_t>(r.sin_t + at);
+        c = __builtin_shufflevector(c4, c4, 0, 1, 2, 3, 0, 1, 2, 3), s = __builtin_shufflevector(s4, s4, 0, 1, 2, 3, 0, 1, 2, 3);
+    } else {
+        c = fa_norm::load_global<h8_t>(r.cos_t + at), s = fa_norm::load_global<h8_t>(r.sin_t + at);
+    }
+}
+__device__ __forceinline__ h8_t rope_piece(const RopeDev &r, h8_t y, h8_t mate, h8_t c, h8_t s, bool first) {
+    h8_t o;
+    if (r.normal) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[2 * i] = (_Float16)rope_one((float)y[2 * i], (float)y[2 * i + 1], (float)c[i], (float)s[i], true);
+            o[2 * i + 1] = (_Float16)rope_one((float)y[2 * i + 1], (float)y[2 * i], (float)c[i], (float)s[i], false);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)rope_one((float)y[e], (float)mate[e], (float)c[e], (float)s[e], first);
+    }
+    return o;
+}
 
 // Write stage of one piece: y = the projections of token gm, columns gn .. gn + 7 of matrix mat (0 Q, 1 K, 2 V),
 // already rounded to f16 as FusedQkv stores them; mate = the piece half a head away (NeoX pairing; unused otherwise).
@@ -52,25 +82,9 @@ __device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint
     }
     if (mat != 2 && r.apply) {
         const uint32_t tp = pos < r.table_rows ? pos : r.table_rows - 1;  // stay inside the tables
-        if (r.normal) {  // pairs (hd + 2i, hd + 2i + 1), table columns hd / 2 + i
-            typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
-            const h4v_t c4 = *reinterpret_cast<const h4v_t *>(r.cos_t + (size_t)tp * half + (hd >> 1));
-            const h4v_t s4 = *reinterpret_cast<const h4v_t *>(r.sin_t + (size_t)tp * half + (hd >> 1));
-            h8_t o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                o[2 * i] = (_Float16)rope_one((float)y[2 * i], (float)y[2 * i + 1], (float)c4[i], (float)s4[i], true);
-                o[2 * i + 1] = (_Float16)rope_one((float)y[2 * i + 1], (float)y[2 * i], (float)c4[i], (float)s4[i], false);
-            }
-            y = o;
-        } else {  // pairs (hd, hd + D / 2), table column hd mod D / 2
-            const bool first = hd < half;
-            const uint32_t pc = first ? hd : hd - half;
-            const h8_t c8 = *reinterpret_cast<const h8_t *>(r.cos_t + (size_t)tp * half + pc);
-            const h8_t s8 = *reinterpret_cast<const h8_t *>(r.sin_t + (size_t)tp * half + pc);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = (_Float16)rope_one((float)y[e], (float)mate[e], (float)c8[e], (float)s8[e], first);
-        }
+        h8_t c, s;
+        rope_columns(r, tp, rope_column(r, hd), c, s);
+        y = rope_piece(r, y, mate, c, s, hd < half);
     }
     *reinterpret_cast<h8_t *>(dst) = y;
 }

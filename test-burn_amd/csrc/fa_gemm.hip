@@ -624,6 +624,7 @@ static fa_status launch_gemm(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRope
         a.rope.on = 1, a.rope.head_dim = r.head_dim, a.rope.n_kv_heads = r.n_kv_heads, a.rope.position_offset = r.position_offset;
         a.rope.max_seq_len = r.max_seq_len, a.rope.block_size = r.block_size ? r.block_size : 1, a.rope.capacity = r.capacity;
         a.rope.table_rows = r.table_rows, a.rope.normal = r.rope_normal ? 1u : 0u, a.rope.apply = r.apply_rope ? 1u : 0u;
+        a.page_shift = (a.rope.block_size & (a.rope.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(a.rope.block_size) : 32u;
     }
     const bool q8 = l.scales[0] != nullptr;
     a.rows[0] = l.n_dim, a.rows[1] = l.n_kv, a.rows[2] = l.n_kv;

@@ -53,7 +53,9 @@
 #pragma once
 #include "fa_gemm.h"
 #include "fa_lds_dma.h"
+#include "fa_norm.h"
 #include <atomic>
+#include <numeric>
 #include <type_traits>
 
 namespace fa_tile {
@@ -345,23 +347,90 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             for (int t = 0; t < S::SETS; ++t) acc[t][i][j] = f16v_t{};
         }
 
+    // The write stage turns pieces of 8 outputs: piece i of a thread is number tid + i NT of the turn's, row after row, so that a thread
+    // comes back to the same NCOL columns and what depends on them - matrix, head, bias, place of the first output - is worked out once.
+    // What the pieces take from memory is asked for BATCH pieces at a time, from addresses that are valid whatever the piece. (One after
+    // the other, with the columns worked out and up to three trips to memory in a row per piece, us: 2048 rows, FusedQkv + KvPrepFused
+    // of 2560 x 2048 F16, paged 45.2 -> 40.1, with the norm; 5120 x 3072 83.2 -> 81.0; o_proj 3072 x 3072 39.2 -> 37.2; 1000 rows, 2048 x
+    // 2048 Q8_0 16.2 -> 15.4; 500 rows, 1152 x 896 Q8_0, paged 11.5 -> 11.1, o_proj of it 6.63 -> 6.76, which has nothing to ask for.)
+    constexpr bool EARLY = S::MT * S::NTR <= 64 * 96;
+    constexpr int PIECES = S::NTR / 8, TURN_PIECES = S::WM * S::TJ * 32 * PIECES, PER_TURN = (TURN_PIECES + S::NT - 1) / S::NT, TURNS = S::TM / S::TJ;
+    constexpr int NCOL = PIECES / std::gcd(S::NT, PIECES), BATCH = EARLY ? PER_TURN * TURNS : PER_TURN > 5 ? PER_TURN / 2 : PER_TURN, BATCHES = EARLY ? 1 : PER_TURN / BATCH;
+    static_assert(TURN_PIECES % S::NT == 0 || PER_TURN == 1, "the threads share the pieces evenly, or some have none");
+    static_assert(EARLY ? PER_TURN % NCOL == 0 : PER_TURN % BATCH == 0 && BATCH % NCOL == 0, "piece i of a batch has column i % NCOL");
+    struct Beside {
+        h8_t c, s;  // columns of the RoPE tables, or c = the residual
+        uint32_t page;
+    };
+    Beside beside[BATCH];
+    struct Column {
+        int mat;
+        uint32_t gn;           // row of its matrix
+        bool in;               // there is such a column
+        h8_t bias, mate_bias;  // (mate_bias: of the half of a head that the piece is rotated with)
+    } column[NCOL];
+    // Piece i of a turn: its row in LDS, and which input row that is.
+    auto lds_row = [&](int thread, int i) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(thread + i * S::NT) / PIECES; };
+    auto input_row = [&](uint32_t t, int turn) __attribute__((always_inline)) -> uint32_t { return m0 + ((t >> 5) / S::TJ * S::TM + turn * S::TJ + (t >> 5) % S::TJ) * 32 + (t & 31); };
     // The residual, asked for ahead of everything else where the tile leaves registers for it: at the end of the one chain that a
     // launch of a round of such tiles is, it would be a trip to memory more (3072 x 3072, 320 rows: F16 12.8 -> 12.3 us, Q8_0 12.2 ->
-    // 11.7, Q4_0 12.0 -> 11.6; 896 x 896, 500 rows: 6.3 -> 6.0, 6.8 -> 6.5, 6.7 -> 6.5). Threads without a place ask for the first one.
-    constexpr bool EARLY = S::MT * S::NTR <= 64 * 96;
-    constexpr int PIECES = S::NTR / 8, PER_TURN = S::WM * S::TJ * 32 * PIECES / S::NT;  // of 8 outputs, per thread and turn of the write stage
-    static_assert(!EARLY || S::WM * S::TJ * 32 * PIECES % S::NT == 0, "the threads share the pieces evenly");
-    h8_t early[EARLY ? PER_TURN * (S::TM / S::TJ) : 1];
+    // 11.7, Q4_0 12.0 -> 11.6; 896 x 896, 500 rows: 6.3 -> 6.0, 6.8 -> 6.5, 6.7 -> 6.5). The rest is asked for behind the loop: ahead of it
+    // the addresses of all that are worked out while nothing has been asked for yet (Q8_0, 500 rows, 1152 x 896: 10.2 -> 10.3 us), and
+    // behind the first requests the first steps wait for it (10.7).
     if constexpr (EARLY) {
         if (a.residual) {
 #pragma unroll
-            for (int i = 0; i < PER_TURN * (S::TM / S::TJ); ++i) {  // (the places are those of the write stage)
-                const uint32_t q = tid + i % PER_TURN * S::NT, t = q / PIECES, r = n0 + q % PIECES * 8;
-                const uint32_t gm = m0 + ((t >> 5) / S::TJ * S::TM + i / PER_TURN * S::TJ + (t >> 5) % S::TJ) * 32 + (t & 31);
-                early[i] = *reinterpret_cast<const h8_t *>(a.residual + (gm < a.m && r < N_tile ? (size_t)gm * N_tile + r : 0));
+            for (int i = 0; i < BATCH; ++i) {
+                const uint32_t gm = input_row(lds_row(tid, i % PER_TURN), i / PER_TURN), r = n0 + (uint32_t)(tid + i % PER_TURN * S::NT) % PIECES * 8;
+                beside[i].c = fa_norm::load_global<h8_t>(a.residual + (gm < a.m && r < N_tile ? (size_t)gm * N_tile + r : 0));
             }
         }
     }
+    // The launch's arguments, read where the write stage begins and not kept from the entry on, for tiles whose loop has no scalar
+    // registers to spare. (The smaller tiles would wait for them there: 0.1 us of 6.6.)
+    static_assert(std::is_trivially_copyable<GemmDev>::value, "read as raw bytes from the argument block, where it is the first member");
+    auto arguments = []() __attribute__((always_inline)) -> const GemmDev & {
+        auto g = __builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(g));
+        return *(const GemmDev *)g;
+    };
+    // The write stage's code is there once for each of what it does, so that none of it runs through the others' branches.
+    enum { PLAIN, ADJACENT, APART };  // alpha * sum + bias + beta * residual; KvPrepFused's, pairs in a piece (or no rotation) and half a head apart
+    auto by_what = [&](const GemmDev &g, auto &&f) __attribute__((always_inline)) {
+        if (!g.rope.on) f(std::integral_constant<int, PLAIN>{});
+        else if (!pairs) f(std::integral_constant<int, ADJACENT>{});
+        else f(std::integral_constant<int, APART>{});
+    };
+    auto ask_columns = [&](auto what, const GemmDev &g, int thread) __attribute__((always_inline)) {
+        constexpr int W = decltype(what)::value;
+#pragma unroll
+        for (int i = 0; i < NCOL; ++i) {
+            Column &col = column[i];
+            const uint32_t at = n0 + (uint32_t)(thread + i * S::NT) % PIECES * 8, end = S::JOINED ? rows0 + 2 * rows1 : N_tile;
+            uint32_t r = min(at, end - 8);
+            col.in = at < end && (TURN_PIECES % S::NT == 0 || thread < TURN_PIECES);
+            col.mat = matrix_of(r), col.gn = W == APART ? paired(r) : r;
+            if (g.bias[0]) {  // (all matrices have one, or none has)
+                const __half *const bias = pick3(col.mat, g.bias[0], g.bias[1], g.bias[2]);
+                col.bias = fa_norm::load_global<h8_t>(bias + col.gn);
+                if constexpr (W == APART) col.mate_bias = fa_norm::load_global<h8_t>(bias + paired(r ^ 16));
+            }
+        }
+    };
+    auto ask = [&](auto what, const GemmDev &g, Beside &w, const Column &col, uint32_t row) __attribute__((always_inline)) {
+        constexpr int W = decltype(what)::value;
+        const uint32_t gm = min(row, g.m - 1);
+        if constexpr (W == PLAIN) {
+            if (!EARLY && g.residual) w.c = fa_norm::load_global<h8_t>(g.residual + (size_t)gm * N_tile + col.gn);
+        } else {
+            const uint32_t pos = g.rope.position_offset + gm;
+            if (W == APART || g.rope.apply) rope_columns(g.rope, min(pos, g.rope.table_rows - 1), rope_column(g.rope, col.gn & (g.rope.head_dim - 1)), w.c, w.s);
+            if (g.rope.block_table) {
+                const uint32_t cache_row = min(pos, g.rope.capacity - 1);
+                w.page = fa_norm::load_global<uint32_t>(g.rope.block_table + (g.page_shift < 32 ? cache_row >> g.page_shift : cache_row / g.rope.block_size));
+            }
+        }
+    };
     if constexpr (S::QUANT) {  // all scales first: 16 bytes (8 blocks) of 64 rows per request
         const __half *sp = pick3(tile_mat, a.scales[0], a.scales[1], a.scales[2]);
         const fa_lds_dma::rsrc_words s_rs = fa_lds_dma::make_rsrc_words(sp, N_tile * (K / 32) * 2);
@@ -451,67 +520,134 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 
     // Write stage: accumulators -> LDS as f32 [input row][weight row], 32 input rows of every wave at a time, then
     // alpha * sum + bias + beta * residual, one rounding to f16, 16-byte stores (or the rotation and the stores of KvPrepFused).
+    const GemmDev &g = EARLY ? a : arguments();
+    // What the column gives to each of its pieces: where the output of input row 0 would be, and the row from which on nothing is stored.
+    struct Target {
+        __half *first;
+        uint32_t stride, end, paged_at;  // paged_at: place in a page of row 0 (K and V in a paged cache)
+        bool paged;
+    };
+    Target target[NCOL];
+    auto find_targets = [&](auto what) __attribute__((always_inline)) {
+        constexpr int W = decltype(what)::value;
 #pragma unroll
-    for (int j0 = 0; j0 < S::TM; j0 += S::TJ) {
-        __syncthreads();  // every wave is done with the stages / the previous rows have been read out
+        for (int i = 0; i < NCOL; ++i) {
+            const Column &col = column[i];
+            Target &o = target[i];
+            o.first = pick3(col.mat, g.out[0], g.out[1], g.out[2]);
+            o.end = col.in ? g.m : 0u, o.paged = false, o.paged_at = 0;
+            if constexpr (W == PLAIN) {
+                o.stride = S::JOINED ? (col.mat ? rows1 : rows0) : N_tile;
+                o.first += col.gn;
+            } else {
+                const uint32_t D = g.rope.head_dim, head = col.gn >> hd_shift, hd = col.gn & (D - 1), room = g.rope.capacity > g.rope.position_offset ? g.rope.capacity - g.rope.position_offset : 0u;
+                o.stride = D;
+                o.paged = col.mat != 0 && g.rope.block_table;
+                o.paged_at = head * g.rope.block_size * D + hd;
+                if (col.mat != 0) o.end = min(o.end, room);  // never outside the cache
+                if (!o.paged) o.first += (col.mat == 0 ? (size_t)head * g.m : (size_t)head * g.rope.max_seq_len + g.rope.position_offset) * D + hd;
+            }
+        }
+    };
+    auto write = [&](auto what, int i, const Beside &w, int first, int turn) __attribute__((always_inline)) {  // piece first + i of the turn
+        constexpr int W = decltype(what)::value;
+        const Column &col = column[i % NCOL];
+        const Target &o = target[i % NCOL];
+        const uint32_t q = (uint32_t)(tid_w + (first + i) * S::NT), t = TURN_PIECES % S::NT == 0 ? q / PIECES : min(q / PIECES, (uint32_t)(S::WM * S::TJ * 32) - 1);
+        const uint32_t gm = input_row(t, turn), n8 = q % PIECES, at = t * S::T_STRIDE;
+        auto value = [&](uint32_t place, h8_t bias) __attribute__((always_inline)) -> h8_t {
+            f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + place);
+            f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + place + 16);
+#pragma unroll
+            for (int k = 1; k < S::KG; ++k) {
+                s0 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + place);
+                s1 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + place + 16);
+            }
+            float v[8];
+            {   // (every step rounded to f32, whatever follows: a product and a sum made into one with the rounding to f16 gives other bits)
+#pragma clang fp contract(off)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (e < 4 ? s0[e & 3] : s1[e & 3]) * g.alpha;
+                if (g.bias[0]) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] += (float)bias[e];
+                }
+            }
+            if (W == PLAIN && g.residual) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = fmaf(g.beta, (float)w.c[e], v[e]);
+            }
+            h8_t y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = (_Float16)v[e];
+            return y;
+        };
+        h8_t y = value(at + n8 * 32, col.bias);
+        __half *dst = o.first + (size_t)gm * o.stride;
+        if constexpr (W != PLAIN) {
+            if (W == APART || g.rope.apply) {
+                const h8_t turned = rope_piece(g.rope, y, W == APART ? value(at + (n8 ^ 2) * 32, col.mate_bias) : y, w.c, w.s, (col.gn & (g.rope.head_dim - 1)) < (g.rope.head_dim >> 1));
+                y = col.mat != 2 ? turned : y;
+            }
+            if (g.rope.block_table) {
+                const uint32_t pos = g.rope.position_offset + gm, in_page = g.page_shift < 32 ? pos & (g.rope.block_size - 1) : pos % g.rope.block_size;
+                __half *const there = o.first + (size_t)w.page * g.rope.n_kv_heads * g.rope.block_size * g.rope.head_dim + o.paged_at + in_page * g.rope.head_dim;
+                dst = o.paged ? there : dst;
+            }
+        }
+        if (gm < o.end) fa_norm::store_global(dst, y);
+    };
+    auto to_lds = [&](int j0) __attribute__((always_inline)) {
         // register r of lane l of a 32 x 32 tile is weight row 8 (r / 4) + 4 (l / 32) + r % 4 and input row l % 32
 #pragma unroll
         for (int j = j0; j < j0 + S::TJ; ++j)
 #pragma unroll
             for (int i = 0; i < S::TN; ++i)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f4v_t q = {acc[0][i][j][g * 4 + 0], acc[0][i][j][g * 4 + 1], acc[0][i][j][g * 4 + 2], acc[0][i][j][g * 4 + 3]};
-                    *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + ((wm * S::TJ + j - j0) * 32 + r32_w) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + g * 8 + h_w * 4) * 4) = q;
-                }
-        __syncthreads();
-        auto write = [&](uint32_t q, int i) __attribute__((always_inline)) {
-            const uint32_t t = q / PIECES, n8 = q % PIECES;
-            const uint32_t gm = m0 + ((t >> 5) / S::TJ * S::TM + j0 + (t >> 5) % S::TJ) * 32 + (t & 31);
-            uint32_t r = n0 + n8 * 8;
-            const int mat = matrix_of(r);
-            const uint32_t gn = paired(r), N = S::JOINED ? (mat ? rows1 : rows0) : N_tile;
-            if (gm >= a.m || r >= N) return;
-            const __half *bias = pick3(mat, a.bias[0], a.bias[1], a.bias[2]);
-            __half *out = pick3(mat, a.out[0], a.out[1], a.out[2]);
-            const size_t o = (size_t)gm * N + gn;
-            const h8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-            const h8_t rv = !a.residual ? z : EARLY ? early[EARLY ? i : 0] : *reinterpret_cast<const h8_t *>(a.residual + o);
-            auto value = [&](uint32_t p8, uint32_t col, bool with_residual) -> h8_t {
-                f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + t * S::T_STRIDE + p8 * 32);
-                f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + t * S::T_STRIDE + p8 * 32 + 16);
-#pragma unroll
-                for (int k = 1; k < S::KG; ++k) {
-                    s0 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + t * S::T_STRIDE + p8 * 32);
-                    s1 += *reinterpret_cast<const f4v_t *>(smem + k * S::T_BYTES + t * S::T_STRIDE + p8 * 32 + 16);
-                }
-                const h8_t bv = bias ? *reinterpret_cast<const h8_t *>(bias + col) : z;
-                h8_t y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    float s = (e < 4 ? s0[e & 3] : s1[e & 3]) * a.alpha;
-                    if (bias) s += (float)bv[e];
-                    if (with_residual) s += a.beta * (float)rv[e];
-                    y[e] = (_Float16)s;
-                }
-                return y;
-            };
-            const h8_t y = value(n8, gn, a.residual != nullptr);
-            if (a.rope.on) {
-                h8_t mate = z;
-                if (pairs && mat != 2) mate = value(n8 ^ 2, paired(r ^ 16), false);
-                rope_store_piece(a, mat, gm, gn, y, mate);
-            } else {
-                *reinterpret_cast<h8_t *>(out + o) = y;
-            }
-        };
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f4v_t *>(smem + kg * S::T_BYTES + ((wm * S::TJ + j - j0) * 32 + r32_w) * S::T_STRIDE + (wn * S::TN * 32 + i * 32 + q * 8 + h_w * 4) * 4) =
+                        f4v_t{acc[0][i][j][q * 4 + 0], acc[0][i][j][q * 4 + 1], acc[0][i][j][q * 4 + 2], acc[0][i][j][q * 4 + 3]};
+    };
+    by_what(g, [&](auto what) __attribute__((always_inline)) {
+        ask_columns(what, g, tid_w);
         if constexpr (EARLY) {
 #pragma unroll
-            for (int i = 0; i < PER_TURN; ++i) write(tid_w + i * S::NT, j0 / S::TJ * PER_TURN + i);
+            for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, i % PER_TURN), i / PER_TURN));
+            find_targets(what);
+#pragma unroll
+            for (int turn = 0; turn < TURNS; ++turn) {
+                __syncthreads();  // every wave is done with the stages / the previous rows have been read out
+                to_lds(turn * S::TJ);
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < PER_TURN; ++i) write(what, i, beside[turn * PER_TURN + i], 0, turn);
+            }
         } else {
-            for (uint32_t q = tid_w; q < (uint32_t)(S::WM * S::TJ * 32 * PIECES); q += S::NT) write(q, 0);
+            // (One copy of the code for all turns and batches, the accumulators moving up by a turn: run once it comes from memory,
+            // and the instructions of 20 pieces are more than the stores take.)
+            find_targets(what);
+#pragma unroll 1
+            for (int turn = 0; turn < TURNS; ++turn) {
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, i), turn));
+                __syncthreads();
+                to_lds(0);
+#pragma unroll
+                for (int j = 0; j + S::TJ < S::TM; ++j)
+#pragma unroll
+                    for (int i = 0; i < S::TN; ++i) acc[0][i][j] = acc[0][i][j + S::TJ];
+                __syncthreads();
+#pragma unroll 1
+                for (int n = 0;; ++n) {
+#pragma unroll
+                    for (int i = 0; i < BATCH; ++i) write(what, i, beside[i], n * BATCH, turn);
+                    if (n + 1 == BATCHES) break;
+#pragma unroll
+                    for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, (n + 1) * BATCH + i), turn));
+                }
+            }
         }
-    }
+    });
 }
 
 template <class S, int MIN_WAVES>

@@ -8,6 +8,7 @@ import pytest
 import foundry_attn as fa
 import orc
 from gpu_util import announce, bits, ctx
+from test_gpu_paged import Paged
 from test_gpu_qkv import _close, _data
 
 pytestmark = pytest.mark.gpu
@@ -398,3 +399,55 @@ def test_quantised_sums_are_several_chains(K, m, N, chains):
     assert rel <= np.sqrt(0.49 + 0.42 ** 2 * K / 16 / chains), rel
     for b in (dx, dw, ds, dres, dout):
         b.free()
+
+
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,H,Hkv,D,m,bs,layer", [
+    (64, 3, 1, 64, 77, 16, 2),      # 64 x 64 (block-quantised 64 x 32): ragged rows and columns
+    (128, 16, 2, 64, 1030, 48, 2),  # 128 x 64; pages that are not a power of two
+    (64, 14, 2, 64, 2047, 16, 3),   # 128 x 128; a layer without a rotation
+    (64, 40, 8, 64, 1000, 48, 2),   # 256 x 128: two turns of the write stage
+    (192, 32, 4, 64, 520, 16, 2),   # 64 x 96: a third of a thread's pieces in each of three columns where steps are the waves' own
+    (1024, 16, 2, 128, 524, 48, 2),
+    (64, 24, 8, 128, 2040, 48, 2),  # F16: 256 x 160, five columns per thread, rows of two matrices
+    (64, 24, 8, 128, 2048, 16, 3),
+])
+def test_write_stage_into_pages(K, H, Hkv, D, m, bs, layer, weights):
+    """KvPrepFused as a tile's write stage against the two ops, bit for bit: pages, both pairings, with and without biases, layers
+    that are not rotated (every fourth)."""
+    announce("tiles, write stage into pages", K, H, Hkv, D, m, bs, layer, weights)
+    f = ctx()
+    rng = np.random.default_rng(K + H + m)
+    N, NK, pos = H * D, Hkv * D, 37
+    x, g, ws, bias = _data(rng, K, N, NK, m)
+    if weights == "f16":
+        dev, scales = [f.array(orc.to_canonical(w)) for w in ws], None
+        arg = [w.arg() for w in dev]
+    else:
+        quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
+        flat = [orc.to_canonical(q) for q, _ in quant]
+        dev = [f.array(q if weights == "q8" else orc.pack_q4_0(q)) for q in flat]
+        arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev, (N, NK, NK))]
+        dev_s = [f.array(s) for _, s in quant]
+        scales, dev = tuple(s.arg() for s in dev_s), dev + dev_s
+    cos, sin = fa.rope_tables(1e6, D, pos + m)
+    dx, dg, db, dcos, dsin = f.array(x), f.array(g), [f.array(b) for b in bias], f.array(cos), f.array(sin)
+    outs, dqr = [f.zeros((m, n)) for n in (N, NK, NK)], [f.zeros((H, m, D)) for _ in range(2)]
+    pgs = [Paged(f, np.random.default_rng(5), [0, pos, 0], Hkv, D, bs, extra_tokens=m + 1).upload() for _ in range(2)]
+    try:
+        f.set_gemm_min_m(12)
+        for mode, biases in ((fa.ROPE_NEOX, tuple(b.arg() for b in db)), (fa.ROPE_NORMAL, None), (fa.ROPE_NORMAL, tuple(b.arg() for b in db))):
+            kw = dict(gamma=dg.arg(), biases=biases, scales=scales)
+            p = fa.KvPrepFusedParams.make(H, Hkv, D, m, pos, 0, mode, layer, 4)
+            f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, **kw)
+            f.kv_prep_fused_paged(*[o.arg() for o in outs], dqr[0].arg(), pgs[0].desc, 1, dcos.arg(), dsin.arg(), p)
+            f.fused_qkv_kv_prep(dx.arg(), *arg, K, dqr[1].arg(), dcos.arg(), dsin.arg(), p, paged=pgs[1].desc, seq_index=1, **kw)
+            assert np.array_equal(bits(dqr[0].download()), bits(dqr[1].download())), mode
+            for one, two in ((pgs[0].dk, pgs[1].dk), (pgs[0].dv, pgs[1].dv)):  # the whole pools: nothing is written beside the rows
+                assert np.array_equal(bits(one.download()), bits(two.download())), mode
+    finally:
+        f.set_gemm_min_m()
+        for pg in pgs:
+            pg.free()
+        for b in dev + db + outs + dqr + [dx, dg, dcos, dsin]:
+            b.free()
