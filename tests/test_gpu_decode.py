@@ -257,6 +257,48 @@ def test_fused_decode_step_equals_separate_ops(H, Hkv, D, mode, base, layer, ste
         f.set_decode_variant()
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(14, 2, 64), (24, 8, 128), (16, 1, 64)])
+@pytest.mark.parametrize("pos", [0, 15, 16, 63, 300])
+def test_fused_step_new_token_alone_and_not_finite(H, Hkv, D, pos):
+    """The new token of a launch of few keys (4-wave workgroups) is attended as the state it is: as the only key, as the first and
+    the last of a partition, with a score that is infinite or NaN (flash_decode.metal:393-395: -1e30), and alone with values at the
+    ends of the type. Against the append and the decode kernel, which take it from the cache: N(0, 1) values, whose weights are
+    rounded to 11 bits against another maximum, to 2e-3."""
+    announce("fused step, new token alone and not finite", H, Hkv, D, pos)
+    f = ctx()
+    rng = np.random.default_rng(H + pos)
+    cap = 320
+    kc, vc = (h16(rng.normal(size=(Hkv, cap, D))) for _ in range(2))
+    kc[:, pos:], vc[:, pos:] = np.nan, np.nan  # nothing past the position may count
+    q, k, v = (h16(rng.normal(size=(1, n * D))) for n in (H, Hkv, Hkv))
+    k[0, 3] = np.inf           # the scores of the first KV head's queries
+    if pos == 0:
+        v[0, -1], v[0, -2], v[0, -3] = 65504.0, 6e-8, -0.0
+    cos, sin = fa.rope_tables(1e6, D, cap)
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, 1, pos, cap, fa.ROPE_NEOX)
+    dq, dk, dv, dcos, dsin, dqr = f.array(q), f.array(k), f.array(v), f.array(cos), f.array(sin), f.zeros((H, 1, D))
+    outs = []
+    for fused in (True, False):
+        dkc, dvc, do = f.array(kc), f.array(vc), f.zeros((1, H * D))
+        if fused:
+            f.decode_step_fused(dq.arg(), dk.arg(), dv.arg(), None, dkc.arg(), dvc.arg(), dcos.arg(), dsin.arg(), do.arg(), p)
+        else:
+            f.kv_prep_fused(dq.arg(), dk.arg(), dv.arg(), dqr.arg(), dkc.arg(), dvc.arg(), dcos.arg(), dsin.arg(), p)
+            f.flash_attention(dqr.arg((1, H * D)), dkc.arg(), dvc.arg(), do.arg(), True, pos, H, D, pos + 1, 1)
+        outs.append([x.download() for x in (do, dkc, dvc)])
+        for b in (dkc, dvc, do):
+            b.free()
+    for one, two in zip(outs[0][1:], outs[1][1:]):
+        assert np.array_equal(bits(one), bits(two))
+    a, b = (o[0].astype(np.float64) for o in outs)
+    assert np.isfinite(a).all()
+    assert max_abs(a, b) <= TOL
+    if pos == 0:  # one key: its value
+        assert np.array_equal(a.reshape(Hkv, H // Hkv, D), np.repeat(v.astype(np.float64).reshape(Hkv, 1, D), H // Hkv, axis=1))
+    for x in (dq, dk, dv, dcos, dsin, dqr):
+        x.free()
+
+
 def test_fused_step_errors_and_overflow_guard():
     announce("fused step errors")
     f = ctx()
