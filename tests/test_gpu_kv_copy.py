@@ -225,3 +225,9 @@ def test_forked_sequence_shares_prefix_blocks_and_decodes_independently():
     assert not np.array_equal(bits(gk[5][:, 9]), bits(gk[2][:, 9]))   # the two tails diverged at the new row
     for b in (dk, dv, dbt, dl, dsrc, ddst, dq, dkn, dvn, dcos, dsin, dout):
         b.free()
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 63, 64, 65])
+def test_kv_prefix_copy_at_the_edges_of_a_workgroup(n):
+    """A workgroup of the 16-byte copy moves 4 KiB, 32 of these rows: a row less, none and one more than whole workgroups."""
+    test_kv_prefix_copy_equals_oracle(3, 70, 96, 64, np.float16, n)
