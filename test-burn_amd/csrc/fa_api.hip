@@ -1647,9 +1647,7 @@ extern "C" fa_status fa_sage_cache_build(fa_ctx *ctx, const void *k_f16, uint32_
     FA_NEED(k_f16, "k_f16");
     FA_TRY(check_sage_cache(c));
     if (kv_len > c->capacity) return fa_fail(FA_ERR_INVALID_SHAPE, "Invalid shape: kv_len %u > capacity %u", kv_len, c->capacity);
-    FA_TRY(fa_launch_sage_k_mean(ctx, k_f16, c->n_kv_heads, c->capacity, c->head_dim, kv_len, c->k_mean));
-    FA_TRY(fa_launch_sage_quantize_k(ctx, k_f16, c->k_mean, c->n_kv_heads, c->capacity, c->head_dim, 0, kv_len, c->k_q, c->k_scale));
-    return fa_launch_sage_tail_copy(ctx, k_f16, c->n_kv_heads, c->capacity, c->head_dim, kv_len, c->k_tail);
+    return fa_launch_sage_build(ctx, k_f16, c->n_kv_heads, c->capacity, c->head_dim, kv_len, c->k_q, c->k_scale, c->k_mean, c->k_tail);
 }
 
 extern "C" fa_status fa_sage_decode_step(fa_ctx *ctx, const fa_tensor_arg *q, const fa_tensor_arg *k, const fa_tensor_arg *v,

@@ -334,8 +334,8 @@ struct SageAppendLaunch {
     uint32_t position, bound, capacity, head_dim, n_heads, n_kv_heads, rope_normal, apply_rope, table_rows;
 };
 fa_status fa_launch_sage_append(fa_ctx *ctx, const SageAppendLaunch &l);
-fa_status fa_launch_sage_tail_copy(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim,
-                                   uint32_t kv_len, void *tail);
+fa_status fa_launch_sage_build(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim, uint32_t kv_len,
+                               void *k_q, void *k_scale, float *mean, void *tail);
 
 // The context's device-written status words: a kernel stores 1 into the word of the condition it met.
 constexpr uint32_t FA_DEVSTAT_MERGE_TIMEOUT = 0u;   // a merging workgroup gave up waiting for a partition's partial

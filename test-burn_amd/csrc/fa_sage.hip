@@ -60,13 +60,28 @@ sage_k_colsum_kernel(const __half *k, uint32_t capacity, uint32_t kv_len, uint32
     }
 }
 
-// Adds the parts of a head in a fixed order: a workgroup of 1024 threads owns MEAN_FIN_COLS columns of one head, so that a
-// launch has D / MEAN_FIN_COLS workgroups per head and every thread adds at most a few parts, all of its loads in flight at
-// once. Thread (column d = tid % COLS, part lane tid / COLS) takes the parts pl, pl + lanes, ...; the lanes are added through
-// LDS in a tree. Latency-bound: with one workgroup of 256 threads per head, 32 dependent batches of loads deep, SmolLM3 at 32K
-// (4 heads x 512 parts x 128 columns, 1 MB) took 8.0 us of the build's 28.1; the build is 22.7 us now.
-constexpr int MEAN_FIN_COLS = 16, MEAN_FIN_NT = 1024, MEAN_FIN_LANES = MEAN_FIN_NT / MEAN_FIN_COLS;
-constexpr int MEAN_FIN_LOADS = MEAN_MAX_PARTS / MEAN_FIN_LANES;  // parts per thread at most
+// The order in which the parts of a head are added up, whoever does it: part lane l (of MEAN_LANES) takes the parts l, l +
+// MEAN_LANES, ... one after the other, the lanes are added in a tree, l with l + 32, l + 16, ..., l + 1. `lane_tree` is the last part of
+// it: v[i] holds lane first + i * STRIDE, for which it leaves the sum in v[0].
+constexpr int MEAN_LANES = 64;
+
+template <typename T, int N>
+__device__ __forceinline__ T lane_tree(T (&v)[N]) {
+#pragma unroll
+    for (int half = N / 2; half >= 1; half >>= 1) {
+#pragma unroll
+        for (int i = 0; i < half; ++i) v[i] += v[i + half];
+    }
+    return v[0];
+}
+
+// The mean as a launch of its own: a workgroup of 1024 threads owns MEAN_FIN_COLS columns of one head, so that a launch has
+// D / MEAN_FIN_COLS workgroups per head and every thread adds at most a few parts, all of its loads in flight at once. Thread
+// (column d = tid % COLS, part lane tid / COLS); the first wave adds the lanes, 16 to a thread and the last four by lane
+// exchanges. Latency-bound: with one workgroup of 256 threads per head, 32 dependent batches of loads deep, SmolLM3 at 32K
+// (4 heads x 512 parts x 128 columns, 1 MB) took 8.0 us.
+constexpr int MEAN_FIN_COLS = 16, MEAN_FIN_NT = MEAN_FIN_COLS * MEAN_LANES;
+constexpr int MEAN_FIN_LOADS = MEAN_MAX_PARTS / MEAN_LANES;  // parts per thread at most
 
 template <int D>
 __global__ void __launch_bounds__(MEAN_FIN_NT)
@@ -78,20 +93,57 @@ sage_k_mean_finish_kernel(const float *partial, uint32_t n_parts, uint32_t kv_le
     float v[MEAN_FIN_LOADS];
 #pragma unroll
     for (int u = 0; u < MEAN_FIN_LOADS; ++u) {
-        const uint32_t p = pl + u * MEAN_FIN_LANES;
+        const uint32_t p = pl + u * MEAN_LANES;
         v[u] = p < n_parts ? hp[(size_t)p * D] : 0.0f;
     }
     float t = 0.0f;
 #pragma unroll
     for (int u = 0; u < MEAN_FIN_LOADS; ++u) t += v[u];
     sm[tid] = t;
+    __syncthreads();
+    if (tid >= 64) return;
+    constexpr int PER = 64 / MEAN_FIN_COLS;  // lanes of the tree that are threads of the wave
+    float l[MEAN_LANES / PER];
 #pragma unroll
-    for (uint32_t half = MEAN_FIN_NT / 2; half >= MEAN_FIN_COLS; half >>= 1) {
-        __syncthreads();
-        if (tid < half) sm[tid] = t = t + sm[tid + half];
-    }
+    for (int i = 0; i < MEAN_LANES / PER; ++i) l[i] = sm[tid + 64 * i];
+    t = lane_tree(l);
+#pragma unroll
+    for (int half = 64 / 2; half >= MEAN_FIN_COLS; half >>= 1) t += __shfl_down(t, half);
     if (tid < MEAN_FIN_COLS) mean[(size_t)h * D + d] = kv_len ? t / (float)kv_len : 0.0f;
 }
+
+// The same mean inside a workgroup of NT threads that needs all of it, where no lane has more than one part: D values into `mu`.
+// Thread t asks for four columns (t % CH) of the lanes g, g + G, ... (g = t / CH, G = NT / CH groups): the tree's upper levels are sums
+// of its own rows, the lower ones of the G groups' sums through LDS. Ends with a barrier.
+template <int D, int NT>
+struct LaneSums {
+    static constexpr int CH = D / 4, G = NT / CH, NL = MEAN_LANES / G;
+    static_assert(NT % CH == 0 && (G & (G - 1)) == 0 && NL >= 1 && D <= NT, "groups of whole lanes");
+    sg_f4_t v[NL];
+    __device__ __forceinline__ void ask(const float *parts, uint32_t n_parts) {
+        const uint32_t c = threadIdx.x % CH, g = threadIdx.x / CH;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const uint32_t l = g + i * G;
+            v[i] = l < n_parts ? *reinterpret_cast<const sg_f4_t *>(parts + (size_t)l * D + c * 4) : sg_f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    __device__ __forceinline__ void mean(uint32_t kv_len, float (&sums)[G][D], float (&mu)[D]) {
+        const uint32_t c = threadIdx.x % CH, g = threadIdx.x / CH;
+        const sg_f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < NL; ++i) v[i] = zero + v[i];  // as the one part of a lane is added to its empty sum
+        *reinterpret_cast<sg_f4_t *>(&sums[g][c * 4]) = lane_tree(v);
+        __syncthreads();
+        if (threadIdx.x < D) {
+            float t[G];
+#pragma unroll
+            for (int i = 0; i < G; ++i) t[i] = sums[i][threadIdx.x];
+            mu[threadIdx.x] = lane_tree(t) / (float)kv_len;
+        }
+        __syncthreads();
+    }
+};
 
 __device__ __forceinline__ int quant_i8(float x, float scale) {
     if (!(scale > 0.0f)) return 0;
@@ -100,58 +152,98 @@ __device__ __forceinline__ int quant_i8(float x, float scale) {
     return (int)r;
 }
 
-// One wave per 32-row block of one head (four blocks per workgroup): the block is read ONCE - 16 bytes per lane and
-// request, all of a lane's requests in flight together - held in registers as f32 differences from the mean, reduced to
-// the block's scale with lane exchanges, quantised and stored 8 bytes per lane and row. Lane l owns dims 8 (l % CPR) ..
-// of rows l / CPR + RPP i.
+// One wave per 32-row block of one head: the block is read ONCE - 16 bytes per lane and request, all of a lane's requests in
+// flight together - held in registers as f32 differences from the mean, reduced to the block's scale with lane exchanges,
+// quantised and stored 8 bytes per lane and row. Lane l owns dims 8 (l % CPR) .. of rows l / CPR + RPP i. (Stored past the caches
+// the build is 0.5 us shorter at 32K and the first steps that read the rows are 4.5 us longer.)
+constexpr int QUANT_NT = 256;
+
 template <int D>
-__global__ void __launch_bounds__(256)
-sage_quantize_k_kernel(const __half *k, const float *mean, uint32_t capacity, uint32_t row_begin, uint32_t row_end,
-                       uint32_t n_blocks, int8_t *k_q, __half *k_scale, uint32_t n_scale_blocks) {
-    constexpr int CPR = D / 8, RPP = 64 / CPR, NI = 32 / RPP;  // chunks per row, rows per pass of the wave, passes
-    const uint32_t h = blockIdx.y, lane = threadIdx.x & 63u;
-    const uint32_t blk = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (blk >= n_blocks) return;  // uniform over the wave
-    const uint32_t b0 = row_begin + blk * FA_SAGE_BLOCK, b1 = min(row_end, b0 + FA_SAGE_BLOCK);
-    const uint32_t ch = lane % CPR, rl = lane / CPR;
-    const __half *src = k + ((size_t)h * capacity + b0) * D + ch * 8;
+struct SageBlock {
+    static constexpr int CPR = D / 8, RPP = 64 / CPR, NI = 32 / RPP;  // chunks per row, rows per pass of the wave, passes
     sg_u4_t raw[NI];
+    __device__ __forceinline__ void ask(const __half *src, uint32_t rows) {
+        const uint32_t lane = threadIdx.x & 63u, ch = lane % CPR, rl = lane / CPR;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const uint32_t row = rl + i * RPP;
-        raw[i] = b0 + row < b1 ? __builtin_nontemporal_load(reinterpret_cast<const sg_u4_t *>(src + (size_t)row * D)) : sg_u4_t{0u, 0u, 0u, 0u};
-    }
-    const sg_f4_t m0 = *reinterpret_cast<const sg_f4_t *>(mean + (size_t)h * D + ch * 8);
-    const sg_f4_t m1 = *reinterpret_cast<const sg_f4_t *>(mean + (size_t)h * D + ch * 8 + 4);
-    const float mu[8] = {m0[0], m0[1], m0[2], m0[3], m1[0], m1[1], m1[2], m1[3]};
-    float x[NI][8];
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const bool live = b0 + rl + i * RPP < b1;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            x[i][2 * w] = live ? h_lo(raw[i][w]) - mu[2 * w] : 0.0f;
-            x[i][2 * w + 1] = live ? h_hi(raw[i][w]) - mu[2 * w + 1] : 0.0f;
-            amax = fmaxf(amax, fmaxf(fabsf(x[i][2 * w]), fabsf(x[i][2 * w + 1])));
+        for (int i = 0; i < NI; ++i) {
+            const uint32_t row = rl + i * RPP;
+            raw[i] = row < rows ? __builtin_nontemporal_load(reinterpret_cast<const sg_u4_t *>(src + (size_t)row * D + ch * 8)) : sg_u4_t{0u, 0u, 0u, 0u};
         }
     }
+    // the rows as they are, for a `dst` of any alignment that an f16 array has
+    __device__ __forceinline__ void copy(uint32_t rows, __half *dst) const {
+        typedef unsigned int any_u4_t __attribute__((ext_vector_type(4), aligned(2)));
+        const uint32_t lane = threadIdx.x & 63u, ch = lane % CPR, rl = lane / CPR;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    const __half sc16 = __float2half_rn(amax / 127.0f);
-    const SageDivisor dv = sage_divisor(__half2float(sc16));
-    if (lane == 0) k_scale[(size_t)h * n_scale_blocks + b0 / FA_SAGE_BLOCK] = sc16;
-    int8_t *dst = k_q + ((size_t)h * capacity + b0) * D + ch * 8;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const uint32_t row = rl + i * RPP;
-        if (b0 + row >= b1) continue;
-        sg_u2_t o;
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            o[w] = sage_quant4_i8(x[i][4 * w], x[i][4 * w + 1], x[i][4 * w + 2], x[i][4 * w + 3], dv);
+        for (int i = 0; i < NI; ++i) {
+            const uint32_t row = rl + i * RPP;
+            if (row < rows) *reinterpret_cast<any_u4_t *>(dst + (size_t)row * D + ch * 8) = raw[i];
         }
-        *reinterpret_cast<sg_u2_t *>(dst + (size_t)row * D) = o;
+    }
+    // `rows` of the block are there (none, and nothing is written); `mean` is the head's, in global memory or LDS
+    __device__ __forceinline__ void quantize(uint32_t rows, const float *mean, int8_t *dst, __half *scale) const {
+        const uint32_t lane = threadIdx.x & 63u, ch = lane % CPR, rl = lane / CPR;
+        const sg_f4_t m0 = *reinterpret_cast<const sg_f4_t *>(mean + ch * 8);
+        const sg_f4_t m1 = *reinterpret_cast<const sg_f4_t *>(mean + ch * 8 + 4);
+        const float mu[8] = {m0[0], m0[1], m0[2], m0[3], m1[0], m1[1], m1[2], m1[3]};
+        float x[NI][8];
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const bool live = rl + i * RPP < rows;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                x[i][2 * w] = live ? h_lo(raw[i][w]) - mu[2 * w] : 0.0f;
+                x[i][2 * w + 1] = live ? h_hi(raw[i][w]) - mu[2 * w + 1] : 0.0f;
+                amax = fmaxf(amax, fmaxf(fabsf(x[i][2 * w]), fabsf(x[i][2 * w + 1])));
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+        const __half sc16 = __float2half_rn(amax / 127.0f);
+        const SageDivisor dv = sage_divisor(__half2float(sc16));
+        if (lane == 0) *scale = sc16;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const uint32_t row = rl + i * RPP;
+            if (row >= rows) continue;
+            sg_u2_t o;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                o[w] = sage_quant4_i8(x[i][4 * w], x[i][4 * w + 1], x[i][4 * w + 2], x[i][4 * w + 3], dv);
+            }
+            *reinterpret_cast<sg_u2_t *>(dst + (size_t)row * D + ch * 8) = o;
+        }
+    }
+};
+
+// Rows [row_begin, row_end). `tail` (may be null): where the exact rows of a last block that is not whole go. MEAN: the head's mean is
+// not there yet and is added up from the n_parts (at most MEAN_LANES) rows of column sums of `partial`, by every workgroup for
+// itself; the first one of a head stores it to `mean`.
+template <int D, bool MEAN>
+__global__ void __launch_bounds__(QUANT_NT)
+sage_quantize_k_kernel(const __half *k, float *mean, uint32_t capacity, uint32_t row_begin, uint32_t row_end, int8_t *k_q, __half *k_scale,
+                       uint32_t n_scale_blocks, __half *tail, const float *partial, uint32_t n_parts) {
+    const uint32_t h = blockIdx.y, blk = row_begin / FA_SAGE_BLOCK + blockIdx.x * (QUANT_NT / 64) + (threadIdx.x >> 6);
+    const uint32_t b0 = blk * FA_SAGE_BLOCK, rows = b0 < row_end ? min(row_end - b0, FA_SAGE_BLOCK) : 0u;
+    const size_t row0 = (size_t)h * capacity + b0;
+    SageBlock<D> block;
+    if constexpr (MEAN) {
+        typedef LaneSums<D, QUANT_NT> Sums;
+        __shared__ alignas(16) float sums[Sums::G][D];
+        __shared__ alignas(16) float own[D];
+        Sums lanes;
+        lanes.ask(partial + (size_t)h * n_parts * D, n_parts);
+        block.ask(k + row0 * D, rows);
+        lanes.mean(row_end, sums, own);
+        if (blockIdx.x == 0 && threadIdx.x < D) mean[(size_t)h * D + threadIdx.x] = own[threadIdx.x];
+        if (tail && rows < FA_SAGE_BLOCK) block.copy(rows, tail + (size_t)h * FA_SAGE_BLOCK * D);
+        if (rows) block.quantize(rows, own, k_q + row0 * D, k_scale + (size_t)h * n_scale_blocks + blk);
+    } else {
+        if (rows == 0) return;  // uniform over the wave
+        block.ask(k + row0 * D, rows);
+        if (tail && rows < FA_SAGE_BLOCK) block.copy(rows, tail + (size_t)h * FA_SAGE_BLOCK * D);
+        block.quantize(rows, mean + (size_t)h * D, k_q + row0 * D, k_scale + (size_t)h * n_scale_blocks + blk);
     }
 }
 
@@ -278,22 +370,7 @@ __global__ void __launch_bounds__(256) sage_append_kernel(SageAppendDev a) {
     }
 }
 
-// rows [32 (kv_len / 32), kv_len) of k [Hkv, capacity, D] -> tail [Hkv, 32, D]
-__global__ void sage_tail_copy_kernel(const __half *k, uint32_t capacity, uint32_t head_dim, uint32_t kv_len, __half *tail) {
-    const uint32_t h = blockIdx.x, b0 = kv_len / FA_SAGE_BLOCK * FA_SAGE_BLOCK, rows = kv_len - b0;
-    for (uint32_t i = threadIdx.x; i < rows * head_dim; i += blockDim.x)
-        tail[(size_t)h * FA_SAGE_BLOCK * head_dim + i] = k[((size_t)h * capacity + b0) * head_dim + i];
-}
-
 }  // namespace
-
-fa_status fa_launch_sage_tail_copy(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim,
-                                   uint32_t kv_len, void *tail) {
-    if (kv_len % FA_SAGE_BLOCK == 0) return FA_OK;
-    FaLaunchScope scope(ctx, "sage_tail_copy_kernel", true);
-    scope.launch(sage_tail_copy_kernel, dim3(n_kv_heads), dim3(256), 0, (const __half *)k, capacity, head_dim, kv_len, (__half *)tail);
-    return scope.finish();
-}
 
 fa_status fa_launch_sage_append(fa_ctx *ctx, const SageAppendLaunch &l) {
     SageAppendDev a;
@@ -308,8 +385,9 @@ fa_status fa_launch_sage_append(fa_ctx *ctx, const SageAppendLaunch &l) {
     return scope.finish();
 }
 
-fa_status fa_launch_sage_k_mean(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim,
-                                uint32_t kv_len, float *mean_out) {
+// The column sums of rows [0, kv_len) of every head, part by part, into the workspace.
+static fa_status launch_colsum(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim, uint32_t kv_len,
+                               float *&partial, uint32_t &n_parts) {
     if (((uintptr_t)k & 15u) != 0) return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "the K tensor must be 16-byte aligned");
     // Parts: about eight workgroups per compute unit over all heads (a workgroup has all of a pass - 256 threads x
     // MEAN_UNROLL requests of 16 bytes = 32 KiB - in flight at once, and eight of them fit a compute unit), each a whole
@@ -319,43 +397,73 @@ fa_status fa_launch_sage_k_mean(fa_ctx *ctx, const void *k, uint32_t n_kv_heads,
     uint32_t want = (uint32_t)((8 * n_cus + n_kv_heads - 1) / n_kv_heads);
     if (want > MEAN_MAX_PARTS) want = MEAN_MAX_PARTS;
     if (want == 0) want = 1;
-    uint32_t rows_per_part = ceil_div_u32(ceil_div_u32(kv_len ? kv_len : 1u, want), rows_per_pass) * rows_per_pass;
-    const uint32_t n_parts = ceil_div_u32(kv_len ? kv_len : 1u, rows_per_part);
+    const uint32_t rows_per_part = ceil_div_u32(ceil_div_u32(kv_len ? kv_len : 1u, want), rows_per_pass) * rows_per_pass;
+    n_parts = ceil_div_u32(kv_len ? kv_len : 1u, rows_per_part);
     FA_TRY(fa_ensure_workspace(ctx, (size_t)n_kv_heads * n_parts * head_dim * sizeof(float)));
-    float *partial = (float *)ctx->workspace;
-    {
-        FaLaunchScope scope(ctx, "sage_k_colsum_kernel", true);
-        if (head_dim == 128)
-            scope.launch(sage_k_colsum_kernel<128>, dim3(n_parts, n_kv_heads), dim3(256), 0, (const __half *)k, capacity, kv_len,
-                         rows_per_part, n_parts, partial);
-        else
-            scope.launch(sage_k_colsum_kernel<64>, dim3(n_parts, n_kv_heads), dim3(256), 0, (const __half *)k, capacity, kv_len,
-                         rows_per_part, n_parts, partial);
-        FA_TRY(scope.finish());
-    }
-    FaLaunchScope scope(ctx, "sage_k_mean_finish_kernel", true);
-    if (head_dim == 128)
-        scope.launch(sage_k_mean_finish_kernel<128>, dim3(128 / MEAN_FIN_COLS, n_kv_heads), dim3(MEAN_FIN_NT), 0, partial, n_parts, kv_len, mean_out);
-    else
-        scope.launch(sage_k_mean_finish_kernel<64>, dim3(64 / MEAN_FIN_COLS, n_kv_heads), dim3(MEAN_FIN_NT), 0, partial, n_parts, kv_len, mean_out);
+    partial = (float *)ctx->workspace;
+    FaLaunchScope scope(ctx, "sage_k_colsum_kernel", true);
+    auto kernel = head_dim == 128 ? sage_k_colsum_kernel<128> : sage_k_colsum_kernel<64>;
+    scope.launch(kernel, dim3(n_parts, n_kv_heads), dim3(256), 0, (const __half *)k, capacity, kv_len, rows_per_part, n_parts, partial);
     return scope.finish();
+}
+
+static fa_status launch_mean_finish(fa_ctx *ctx, const float *partial, uint32_t n_parts, uint32_t n_kv_heads, uint32_t head_dim,
+                                    uint32_t kv_len, float *mean) {
+    FaLaunchScope scope(ctx, "sage_k_mean_finish_kernel", true);
+    auto kernel = head_dim == 128 ? sage_k_mean_finish_kernel<128> : sage_k_mean_finish_kernel<64>;
+    scope.launch(kernel, dim3(head_dim / MEAN_FIN_COLS, n_kv_heads), dim3(MEAN_FIN_NT), 0, partial, n_parts, kv_len, mean);
+    return scope.finish();
+}
+
+// partial: null, or the n_parts rows of column sums that the mean is still to be made of
+static fa_status launch_quantize_k(fa_ctx *ctx, const void *k, float *mean, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim,
+                                   uint32_t row_begin, uint32_t row_end, void *k_q, void *k_scale, void *tail, const float *partial,
+                                   uint32_t n_parts) {
+    const dim3 grid(ceil_div_u32(row_end - row_begin, FA_SAGE_BLOCK * (QUANT_NT / 64)), n_kv_heads);
+    FaLaunchScope scope(ctx, "sage_quantize_k_kernel", true);
+    auto kernel = head_dim == 128 ? (partial ? sage_quantize_k_kernel<128, true> : sage_quantize_k_kernel<128, false>)
+                                  : (partial ? sage_quantize_k_kernel<64, true> : sage_quantize_k_kernel<64, false>);
+    scope.launch(kernel, grid, dim3(QUANT_NT), 0, (const __half *)k, mean, capacity, row_begin, row_end, (int8_t *)k_q, (__half *)k_scale,
+                 ceil_div_u32(capacity, FA_SAGE_BLOCK), (__half *)tail, partial, n_parts);
+    return scope.finish();
+}
+
+static fa_status check_quantize_k(const void *k, const float *mean, const void *k_q) {
+    if ((((uintptr_t)k | (uintptr_t)mean) & 15u) != 0 || ((uintptr_t)k_q & 7u) != 0)
+        return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "K and the mean must be 16-byte aligned, the int8 cache 8-byte aligned");
+    return FA_OK;
+}
+
+fa_status fa_launch_sage_k_mean(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim,
+                                uint32_t kv_len, float *mean_out) {
+    float *partial;
+    uint32_t n_parts;
+    FA_TRY(launch_colsum(ctx, k, n_kv_heads, capacity, head_dim, kv_len, partial, n_parts));
+    return launch_mean_finish(ctx, partial, n_parts, n_kv_heads, head_dim, kv_len, mean_out);
 }
 
 fa_status fa_launch_sage_quantize_k(fa_ctx *ctx, const void *k, const float *mean, uint32_t n_kv_heads,
                                     uint32_t capacity, uint32_t head_dim, uint32_t row_begin, uint32_t row_end,
                                     void *k_q, void *k_scale) {
     if (row_end <= row_begin) return FA_OK;
-    if ((((uintptr_t)k | (uintptr_t)mean) & 15u) != 0 || ((uintptr_t)k_q & 7u) != 0)
-        return fa_fail(FA_ERR_OPERATION_NOT_SUPPORTED, "K and the mean must be 16-byte aligned, the int8 cache 8-byte aligned");
-    const uint32_t nblk = ceil_div_u32(row_end - row_begin, FA_SAGE_BLOCK);
-    FaLaunchScope scope(ctx, "sage_quantize_k_kernel", true);
-    if (head_dim == 128)
-        scope.launch(sage_quantize_k_kernel<128>, dim3(ceil_div_u32(nblk, 4), n_kv_heads), dim3(256), 0, (const __half *)k, mean,
-                     capacity, row_begin, row_end, nblk, (int8_t *)k_q, (__half *)k_scale, ceil_div_u32(capacity, FA_SAGE_BLOCK));
-    else
-        scope.launch(sage_quantize_k_kernel<64>, dim3(ceil_div_u32(nblk, 4), n_kv_heads), dim3(256), 0, (const __half *)k, mean,
-                     capacity, row_begin, row_end, nblk, (int8_t *)k_q, (__half *)k_scale, ceil_div_u32(capacity, FA_SAGE_BLOCK));
-    return scope.finish();
+    FA_TRY(check_quantize_k(k, mean, k_q));
+    return launch_quantize_k(ctx, k, const_cast<float *>(mean), n_kv_heads, capacity, head_dim, row_begin, row_end, k_q, k_scale, nullptr, nullptr, 0);
+}
+
+fa_status fa_launch_sage_build(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, uint32_t capacity, uint32_t head_dim, uint32_t kv_len,
+                               void *k_q, void *k_scale, float *mean, void *tail) {
+    if (kv_len == 0) return fa_launch_sage_k_mean(ctx, k, n_kv_heads, capacity, head_dim, kv_len, mean);
+    FA_TRY(check_quantize_k(k, mean, k_q));
+    float *partial;
+    uint32_t n_parts;
+    FA_TRY(launch_colsum(ctx, k, n_kv_heads, capacity, head_dim, kv_len, partial, n_parts));
+    // Up to 64 parts (8192 rows at D 128, 16384 at D 64) every workgroup of the quantiser adds them up itself, 32 KiB at most that its
+    // XCD's L2 holds: 4 heads of D 128, 300 rows 11.2 -> 7.3 us, 8000 rows 11.9 -> 11.3. Beyond them a launch of its own is
+    // ahead: 64 sums per head made by 64 workgroups of 1024 threads, which the quantiser could add up as well, took 21.6 us against
+    // 21.2 at 32768 rows, 36.8 against 29.4 for 2 heads of 100000.
+    const bool own_mean = n_parts <= MEAN_LANES;
+    if (!own_mean) FA_TRY(launch_mean_finish(ctx, partial, n_parts, n_kv_heads, head_dim, kv_len, mean));
+    return launch_quantize_k(ctx, k, mean, n_kv_heads, capacity, head_dim, 0, kv_len, k_q, k_scale, tail, own_mean ? partial : nullptr, n_parts);
 }
 
 fa_status fa_launch_sage_quantize_q(fa_ctx *ctx, const void *q, uint32_t n_heads, uint32_t head_dim, void *q_q,

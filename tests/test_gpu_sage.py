@@ -217,3 +217,34 @@ def test_sage_decode_step_errors():
     f.synchronize()
     for b in list(bufs.values()) + [q, k, v, out, cos, sin, dpos]:
         b.free()
+
+
+@pytest.mark.parametrize("Hkv,D,n,cap", [
+    (3, 128, 1, 1), (1, 128, 31, 40), (4, 128, 33, 64), (2, 64, 64, 64),                    # one part; open block of 1 .. 31 rows or none
+    (2, 128, 8191, 8300), (2, 128, 8192, 8192), (2, 128, 8193, 8200), (3, 64, 16385, 16400)])  # 64 parts and 65: the mean with the quantiser or before it
+def test_sage_cache_build_is_its_separate_operations(Hkv, D, n, cap):
+    """The mean, the int8 rows and the scales are those of fa_sage_k_mean and fa_sage_quantize_k bit for bit, the open block's rows
+    are in the tail, and nothing else is written."""
+    announce("sage build", Hkv, D, n, cap)
+    f = ctx()
+    rng = np.random.default_rng(n + D)
+    k = outlier_normal(rng, (Hkv, cap, D))
+    dk, dv = f.array(k), f.zeros((Hkv, cap, D), np.float16)
+    desc, bufs = fa.sage_cache(f, 2 * Hkv, Hkv, cap, D, dv)
+    marks = dict(k_q=np.full((Hkv, cap, D), 99, np.int8), k_scale=np.full((Hkv, (cap + 31) // 32), 7, np.float16),
+                 k_tail=np.full((Hkv, 32, D), 7, np.float16))
+    for name, m in marks.items():
+        bufs[name].upload(m)
+    dmean, dkq, dks = f.zeros((Hkv, D), np.float32), f.array(marks["k_q"]), f.array(marks["k_scale"])
+    f.sage_cache_build(dk, n, desc)
+    f.sage_k_mean(dk, Hkv, cap, D, n, dmean)
+    f.sage_quantize_k(dk, dmean, Hkv, cap, D, 0, n, dkq, dks)
+    f.synchronize()
+    assert np.array_equal(bits(bufs["k_mean"].download()), bits(dmean.download()))
+    assert np.array_equal(bufs["k_q"].download(), dkq.download())
+    assert np.array_equal(bits(bufs["k_scale"].download()), bits(dks.download()))
+    want = marks["k_tail"].copy()
+    want[:, :n % 32] = k[:, n - n % 32:n]
+    assert np.array_equal(bits(bufs["k_tail"].download()), bits(want))
+    for b in (dk, dmean, dkq, dks, *bufs.values()):
+        b.free()
