@@ -77,14 +77,6 @@ union U4H {
     _Float16 e[8];
 };
 
-// The int8 quantiser of fa_sage.hip: rint(x / scale) clamped to +-127, 0 for a zero scale.
-__device__ __forceinline__ int sage_quant_i8(float x, float scale) {
-    if (!(scale > 0.0f)) return 0;
-    float r = rintf(x / scale);
-    r = fminf(fmaxf(r, -127.0f), 127.0f);
-    return (int)r;
-}
-
 constexpr int NW = FA_DECODE_NW;  // waves per workgroup; two per SIMD in all: 8 = one workgroup per CU, 4 = two, at <= 256 VGPRs
 constexpr int NT = NW * 64;  // threads per workgroup
 constexpr int BK = 16;       // keys per block (MFMA M dimension)
@@ -127,7 +119,7 @@ __device__ __forceinline__ float xor32(float x) {
     return __uint_as_float(((threadIdx.x >> 5) & 1) ? r.x : r.y);
 }
 
-// Reductions over aligned groups of 4, 8 or 32 consecutive lanes; every lane of the group gets the result. Lane
+// Reductions over aligned groups of 2 to 64 consecutive lanes; every lane of the group gets the result. Lane
 // exchanges inside a 16-lane row are DPP moves (quad permutes, then the mirrors of a half row and of a row), the step
 // across rows is a lane swap. The order of the operands is fixed, so results are reproducible.
 template <int CTRL>
@@ -136,15 +128,14 @@ __device__ __forceinline__ float dpp_mov(float v) {
 }
 template <int G, bool MAX>
 __device__ __forceinline__ float group_reduce(float v) {
-    static_assert(G == 2 || G == 4 || G == 8 || G == 32, "group sizes in use");
+    static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0, "a power of two");
     auto op = [](float x, float y) { return MAX ? fmaxf(x, y) : x + y; };
-    v = op(v, dpp_mov<0xB1>(v));               // quad_perm [1,0,3,2]: lane ^ 1
-    if (G >= 4) v = op(v, dpp_mov<0x4E>(v));   // quad_perm [2,3,0,1]: lane ^ 2
-    if (G >= 8) v = op(v, dpp_mov<0x141>(v));  // row_half_mirror: the other quad of the 8 lanes
-    if (G >= 32) {
-        v = op(v, dpp_mov<0x140>(v));          // row_mirror: the other half of the row
-        v = op(v, xor16(v));
-    }
+    v = op(v, dpp_mov<0xB1>(v));                // quad_perm [1,0,3,2]: lane ^ 1
+    if (G >= 4) v = op(v, dpp_mov<0x4E>(v));    // quad_perm [2,3,0,1]: lane ^ 2
+    if (G >= 8) v = op(v, dpp_mov<0x141>(v));   // row_half_mirror: the other quad of the 8 lanes
+    if (G >= 16) v = op(v, dpp_mov<0x140>(v));  // row_mirror: the other half of the row
+    if (G >= 32) v = op(v, xor16(v));
+    if (G >= 64) v = op(v, xor32(v));
     return v;
 }
 
@@ -969,13 +960,11 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             FA_TR(1);
             n_raw = read_len();
             const uint32_t p0 = min(n_raw, min(a.capacity, a.kv_len_bound)) - 1;
-            {
-                // ... and the block's V rows as soon as the position says where they are (same conditions as below)
-                const uint32_t N0 = p0 + 1;
-                if (n_raw == N0 && N0 > 0 && p0 >= k0 && p0 < k0 + chunk && split < (N0 + a.chunk - 1) / a.chunk) {
-                    const uint32_t r0 = p0 & (FA_SAGE_BLOCK - 1);
-                    issue_v((p0 - r0 - k0) / BK, r0 / BK + 1, 0);
-                }
+            // (same conditions as below)
+            const bool owner = n_raw == p0 + 1 && p0 + 1 > 0 && p0 >= k0 && p0 < k0 + chunk && split < (p0 + a.chunk) / a.chunk;
+            if (owner) {  // ... and the block's V rows as soon as the position says where they are
+                const uint32_t r0 = p0 & (FA_SAGE_BLOCK - 1);
+                issue_v((p0 - r0 - k0) / BK, r0 / BK + 1, 0);
             }
             if (rope_on) {  // the table row through the scalar cache, as below
                 const uint32_t tp = min(p0, a.table_rows - 1);
@@ -1027,11 +1016,6 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
                 cu.u = *reinterpret_cast<const uint4 *>(cp + pc * 16), su.u = *reinterpret_cast<const uint4 *>(sp + pc * 16);
                 return rope8(x, mate, cu, su, false, sgm < PPR / 2, false).u;
             };
-            // the new K row (lanes 0 .. D/8 - 1 hold it; the others rotate zeros along so that the exchange is uniform)
-            {
-                const uint4 kr = rotate_piece(kv4);
-                if (lane < PPR) *reinterpret_cast<uint4 *>(st_krot + lane * 8) = kr;
-            }
             // The query: rotated, then quantised per head with the head's own scale max|q| / 127 (f32), as
             // sage_append_kernel does it - here 8 values per lane (the operand layout would make every lane divide 16
             // KSTEPS values, most of them for heads the group does not have) - and handed over as int8 rows in LDS.
@@ -1041,22 +1025,19 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
                 const uint32_t e = lane + 64 * i, row = e / PPR;
                 U4H o;
                 o.u = rotate_piece(qv[i]);
-                float amax = 0.0f;
+                float x[8], amax = 0.0f;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf((float)o.e[t]));
+                for (int t = 0; t < 8; ++t) x[t] = (float)o.e[t];
 #pragma unroll
-                for (int off = 1; off < PPR; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+                for (int t = 0; t < 8; t += 2) amax = sage_max3(amax, x[t], x[t + 1]);
+                amax = group_reduce<PPR, true>(amax);
                 const float qs = amax / 127.0f;
-                union {
-                    uint2 u;
-                    int8_t b[8];
-                } q8;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) q8.b[t] = (int8_t)sage_quant_i8((float)o.e[t], qs);
+                const SageDivisor dv = sage_divisor(qs);
+                const uint2 q8 = make_uint2(sage_quant4_i8(x[0], x[1], x[2], x[3], dv), sage_quant4_i8(x[4], x[5], x[6], x[7], dv));
                 if (row < gt) {
-                    *reinterpret_cast<uint2 *>(st_q8 + row * D + sgm * 8) = q8.u;
+                    *reinterpret_cast<uint2 *>(st_q8 + row * D + sgm * 8) = q8;
                     if (sgm == 0) sm_qscale[row] = qs;
-                    if (split == 0 && a.q_q_out) *reinterpret_cast<uint2 *>(a.q_q_out + (size_t)(head0 + row) * D + sgm * 8) = q8.u;
+                    if (split == 0 && a.q_q_out) *reinterpret_cast<uint2 *>(a.q_q_out + (size_t)(head0 + row) * D + sgm * 8) = q8;
                     if (split == 0 && sgm == 0 && a.q_scale_out) a.q_scale_out[head0 + row] = qs;
                 }
             }
@@ -1069,6 +1050,12 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
                 q_lds[j * 64 + lane] = head_ok ? *reinterpret_cast<const uint4 *>(st_q8 + n * D + (4 * j + c) * 16) : make_uint4(0, 0, 0, 0);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
             if (lane == 0) __hip_atomic_store(&sm_q_ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            // The new K row (lanes 0 .. D/8 - 1 hold it; the others rotate zeros along so that the exchange is uniform), for the
+            // workgroup that attends it and after what every workgroup waits for.
+            if (owner) {
+                const uint4 kr = rotate_piece(kv4);
+                if (lane < PPR) *reinterpret_cast<uint4 *>(st_krot + lane * 8) = kr;
+            }
             __builtin_amdgcn_s_setprio(0);
         } else {
             __syncthreads();  // wave 0 has queued its requests
@@ -1357,6 +1344,9 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             // The open block, rows b0 .. p: its earlier rows are exact in the tail, the new row is in the staging area.
             // All of them are quantised anew (a block has one scale, and the new row may raise it), stored, and attended
             // from the registers they were made in; rows past p carry no weight.
+            // One wave does it, 64 values to a lane, and up to about 16K keys it is what the launch waits for: its instructions count.
+            // (Seven per value, lane exchanges in registers, the rows' choice instead of branches, and the query likewise: a step of
+            // SmolLM3 at 300 / 8000 / 20000 / 32768 keys 10.1 -> 8.3, 11.3 -> 9.7, 11.5 -> 10.2, 13.9 -> 13.6 us.)
             const bool writer = y % a.sub_per_kv == 0;
             const uint32_t r = p & (FA_SAGE_BLOCK - 1), b0 = p - r, nsb = r / BK + 1;
             __half *tail = a.sage_tail + (size_t)kvh * FA_SAGE_BLOCK * D;
@@ -1364,27 +1354,26 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             float kx[2][KSTEPS][16];
             float amax = 0.0f;
 #pragma unroll
-            for (int sb = 0; sb < 2; ++sb)
+            for (int sb = 0; sb < 2; ++sb) {
+                const uint32_t row = sb * BK + n;
+                float peak = 0.0f;
 #pragma unroll
                 for (int j = 0; j < KSTEPS; ++j) {
-                    const uint32_t row = sb * BK + n, col = (4 * j + c) * 16;
-                    U4H t0, t1;
-                    t0.u = make_uint4(0, 0, 0, 0), t1.u = t0.u;
-                    if (row < r) {
-                        t0 = kk[sb][j], t1 = vv[2][sb * KSTEPS + j];  // requested before the first barrier
-                    } else if (row == r) {
-                        t0.u = *reinterpret_cast<const uint4 *>(st_krot + col);
-                        t1.u = *reinterpret_cast<const uint4 *>(st_krot + col + 8);
-                    }
+                    const uint32_t col = (4 * j + c) * 16;
+                    const u4_t nw[2] = {*reinterpret_cast<const u4_t *>(st_krot + col), *reinterpret_cast<const u4_t *>(st_krot + col + 8)};
+                    const u4_t old[2] = {__builtin_bit_cast(u4_t, kk[sb][j].u), __builtin_bit_cast(u4_t, vv[2][sb * KSTEPS + j].u)};  // requested before the first barrier
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float v = (float)(i < 8 ? t0.e[i] : t1.e[i - 8]) - st_mean[col + i];
-                        kx[sb][j][i] = row <= r ? v : 0.0f;
-                        amax = fmaxf(amax, fabsf(kx[sb][j][i]));
+                    for (int w = 0; w < 8; ++w) {
+                        const uint32_t word = row == r ? nw[w / 4][w % 4] : old[w / 4][w % 4];
+                        const f2_t mu = *reinterpret_cast<const f2_t *>(st_mean + col + 2 * w);
+                        float *x = kx[sb][j] + 2 * w;
+                        x[0] = sage_lo_minus(word, mu.x), x[1] = sage_hi_minus(word, mu.y);
+                        peak = sage_max3(peak, x[0], x[1]);
                     }
                 }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+                amax = fmaxf(amax, row <= r ? peak : 0.0f);  // (what the rows past the new one come to is masked below and not stored)
+            }
+            amax = group_reduce<64, true>(amax);
             FA_TR(12);
             const __half sc16 = __float2half_rn(amax / 127.0f);
             const SageDivisor dv = sage_divisor(__half2float(sc16));

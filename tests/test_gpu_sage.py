@@ -248,3 +248,57 @@ def test_sage_cache_build_is_its_separate_operations(Hkv, D, n, cap):
     assert np.array_equal(bits(bufs["k_tail"].download()), bits(want))
     for b in (dk, dmean, dkq, dks, *bufs.values()):
         b.free()
+
+
+@pytest.mark.parametrize("launches", [0, 1, 2], ids=["quantiser", "one_launch", "two_launches"])
+def test_sage_special_queries_and_rows_match_the_oracle_bit_for_bit(launches):
+    """Queries of zeros, with an infinity, with a NaN, subnormal, over the f16 range and exactly half way between two steps, and a new
+    row that brings an infinity into the open block of one head and is as far below the others as f16 goes in the other."""
+    announce("sage special queries", launches)
+    f = ctx()
+    rng = np.random.default_rng(11)
+    H, Hkv, D, P, cap = 12, 2, 128, 70, 96
+    q = h16(rng.normal(size=(H, D)))
+    q[0] = 0
+    q[1, 5] = np.float16(np.inf)
+    q[2, 9] = np.float16(np.nan)
+    q[3] = h16(rng.normal(size=D) * 1e-7)
+    q[4] = h16(rng.uniform(-65504, 65504, size=D))
+    q[5] = h16(np.clip((np.arange(D) % 255 - 127).astype(np.float32) + 0.5, -126.5, 126.5))
+    q[5, 0] = np.float16(127.0)
+    q[6], q[6, 3] = 0, np.float16(np.nan)
+    dq, dqq, dqs = f.array(q.reshape(1, H * D)), f.zeros((H, D), np.int8), f.zeros((H,), np.float32)
+    with np.errstate(all="ignore"):
+        want_qq, want_qs = orc.sage_quantize_q(q, H, D)
+    if launches == 0:
+        f.sage_quantize_q(dq, H, D, dqq, dqs)
+        f.synchronize()
+        assert np.array_equal(dqq.download(), want_qq)
+        assert np.array_equal(dqs.download().view(np.uint32), want_qs.view(np.uint32))
+        return
+    f.set_sage_step_variant(launches)
+    kc = h16(rng.normal(size=(Hkv, cap, D)))
+    kc[:, P:] = 0
+    k, v = h16(rng.normal(size=(1, Hkv * D))), h16(rng.normal(size=(1, Hkv * D)))
+    k[0, 7], k[0, D:] = np.float16(-np.inf), np.float16(6e-8)
+    dk, dv = f.array(kc), f.zeros((Hkv, cap, D), np.float16)
+    desc, bufs = fa.sage_cache(f, H, Hkv, cap, D, dv)
+    f.sage_cache_build(dk, P, desc)
+    f.synchronize()
+    mean = bufs["k_mean"].download()
+    cos, sin = fa.rope_tables(1e6, D, cap)
+    dkn, dvn, dcos, dsin, dout = f.array(k), f.array(v), f.array(cos), f.array(sin), f.zeros((H * D,), np.float16)
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, 1, P, cap, fa.ROPE_NEOX, layer_idx=3, no_rope_layer_step=4)  # nothing is rotated
+    f.sage_decode_step(dq.arg(), dkn.arg(), dvn.arg(), desc, dcos.arg(), dsin.arg(), dout.arg(), p)
+    f.synchronize()
+    f.set_sage_step_variant(1)
+    kc[:, P] = k.reshape(Hkv, D)
+    with np.errstate(all="ignore"):
+        want_kq, want_ks = orc.sage_quantize_k(kc, mean, Hkv, cap, D, P + 1)
+    assert np.array_equal(bufs["q_q"].download(), want_qq)
+    assert np.array_equal(bufs["q_scale"].download().view(np.uint32), want_qs.view(np.uint32))
+    nb = (P + 32) // 32
+    assert np.array_equal(bits(bufs["k_scale"].download()[:, :nb]), bits(want_ks[:, :nb]))
+    assert np.array_equal(bufs["k_q"].download()[:, :P + 1], want_kq[:, :P + 1])
+    for b in (dq, dqq, dqs, dk, dkn, dvn, dcos, dsin, dout, *bufs.values()):
+        b.free()

@@ -56,3 +56,37 @@ def test_shared_divisor_sequence_equals_division():
         out = subprocess.run([exe], capture_output=True, text=True)
         assert out.returncode == 0, out.stdout[-800:]
         assert "bad 0" in out.stdout
+
+
+def one_step_source():
+    """The sequence with one step per quotient, as the kernels have it: block scales as above, and every f16 value / 127 (a query's
+    scale; one binade of them, the rest is the same up to a power of two) with every f16 value of up to 13 binades below."""
+    src = SRC.replace("isfinite(q0) ? q2 : q0", "isfinite(q0) ? q1 : q0")
+    assert src != SRC
+    query = r"""
+    for (int a = 1024; a < 2048; ++a) {
+        const float d = (float)a / 127.0f;
+        for (int off = -1; off <= 1; ++off) {
+            const float r0 = step(1.0f / d, off), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+            for (int e = 0; e < 14; ++e)
+                for (int m = 1024; m < 2048; ++m) {
+                    const float x = ldexpf((float)m, -e), q0 = x * r, q1 = fmaf(fmaf(-d, q0, x), r, q0);
+                    if (x > (float)a) break;
+                    ++n;
+                    if (q1 != x / d) ++bad;
+                }
+        }
+    }
+"""
+    return src.replace('    printf("checked', query + '    printf("checked')
+
+
+def test_one_step_equals_division():
+    with tempfile.TemporaryDirectory() as tmp:
+        src, exe = os.path.join(tmp, "t.c"), os.path.join(tmp, "t")
+        with open(src, "w") as fh:
+            fh.write(one_step_source())
+        subprocess.run(["gcc", "-O2", "-ffp-contract=off", "-o", exe, src, "-lm"], check=True)
+        out = subprocess.run([exe], capture_output=True, text=True)
+        assert out.returncode == 0, out.stdout[-800:]
+        assert "bad 0" in out.stdout
