@@ -629,6 +629,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     // count is complete instead of meeting the others at a barrier: a wave reaches that point only when all of its
     // block requests have been accepted, which for the last one is most of the launch's streaming time.
     __shared__ uint32_t sm_q_ready;
+    __shared__ uint32_t sm_open;         // SAGE + FUSED: waves that have put their share of the open block into the staging area
     __shared__ float sm_qscale[MAX_GT];  // SAGE + FUSED: the per-head scales of the query quantised in this workgroup
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -912,11 +913,14 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     U4H qraw;
     qraw.u = make_uint4(0, 0, 0, 0);
     // SAGE + FUSED, wave 0's staging area (its own V region, unused until it attends the open block): the quantised rows
-    // of the group's query heads, the rotated new K row, the smoothing mean.
+    // of the group's query heads, the rotated new K row, the smoothing mean, the waves' largest values of the open block, its rows.
     int8_t *st_q8 = reinterpret_cast<int8_t *>(smem);  // [MAX_GT][D]
     __half *st_krot = reinterpret_cast<__half *>(smem + MAX_GT * D);
     float *st_mean = reinterpret_cast<float *>(st_krot + D);
-    static_assert(!(SAGE && FUSED) || MAX_GT * D + D * 2 + D * 4 <= MBX * BK * VRS, "staging fits a wave's V region");
+    float *st_peak = st_mean + D;                                  // [NW]
+    __half *st_rows = reinterpret_cast<__half *>(st_peak + NW);    // [32][D], the block's rows, and in their place
+    int8_t *st_k8 = reinterpret_cast<int8_t *>(st_rows);           // [32][D]
+    static_assert(!(SAGE && FUSED) || MAX_GT * D + D * 2 + D * 4 + NW * 4 + (int)FA_SAGE_BLOCK * D * 2 <= MBX * BK * VRS, "staging fits a wave's V region");
     uint4 sage_vnew = make_uint4(0, 0, 0, 0);
     if constexpr (SAGE && FUSED) {
         if (wave == 0) {
@@ -936,24 +940,20 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             if (lane < D / 8) kv4 = *reinterpret_cast<const uint4 *>(a.k_in + (size_t)b * a.kvin_stride_b + (size_t)kvh * D + lane * 8);
             if (lane < D / 4) mv4 = *reinterpret_cast<const uint4 *>(a.sage_mean + (size_t)kvh * D + lane * 4);
             sage_vnew = *reinterpret_cast<const uint4 *>(a.v_in + (size_t)b * a.kvin_stride_b + (size_t)kvh * D + (lane % VLPR) * 8);
-            // The exact rows of the open 32-row block, all 32 of them whatever the position turns out to be (the rows at
-            // and past it are not used): the workgroup that owns the new token quantises the block anew, which is the
-            // longest thing any wave of the launch does, and a request made after the barrier would queue behind the
-            // other waves' blocks. Lane (n, c) takes the two halves of segment 4j + c of rows n and 16 + n; they are
-            // parked in block registers that this wave does not otherwise use until then.
-            static_assert(2 * KSTEPS <= VLB && MBX >= 3, "the open block's rows are parked in kk[0..1] and vv[2]");
+            // The exact rows of the open 32-row block, all 32 of them whatever the position turns out to be (the rows at and
+            // past it are not used): the workgroup that owns the new token quantises the block anew, and a request made after
+            // the barrier would queue behind the other waves' blocks. They are parked in block registers that this wave does not
+            // otherwise use until then.
+            static_assert((int)FA_SAGE_BLOCK * D / 512 == 4 * KSTEPS && 2 * KSTEPS <= VLB && MBX >= 3, "parked in kk[0..1] and vv[2]");
             {
-                const __half *tail_rows = a.sage_tail + (size_t)kvh * FA_SAGE_BLOCK * D;
+                const __half *tail_rows = a.sage_tail + (size_t)kvh * FA_SAGE_BLOCK * D + lane * 8;
 #pragma unroll
-                for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-                    for (int j = 0; j < KSTEPS; ++j) {
-                        const __half *src = tail_rows + (size_t)(sb * BK + n) * D + (4 * j + c) * 16;
-                        kk[sb][j].u = *reinterpret_cast<const uint4 *>(src);
-                        vv[2][sb * KSTEPS + j].u = *reinterpret_cast<const uint4 *>(src + 8);
-                    }
+                for (int i = 0; i < 2 * KSTEPS; ++i) {
+                    kk[i / KSTEPS][i % KSTEPS].u = *reinterpret_cast<const uint4 *>(tail_rows + i * 512);
+                    vv[2][i].u = *reinterpret_cast<const uint4 *>(tail_rows + (2 * KSTEPS + i) * 512);
+                }
             }
-            if (lane == 0) sm_q_ready = 0;
+            if (lane == 0) sm_q_ready = 0, sm_open = 0;
             __builtin_amdgcn_sched_barrier(0);
             __syncthreads();  // releases the streaming waves
             __builtin_amdgcn_sched_barrier(0);
@@ -1055,6 +1055,13 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             if (owner) {
                 const uint4 kr = rotate_piece(kv4);
                 if (lane < PPR) *reinterpret_cast<uint4 *>(st_krot + lane * 8) = kr;
+#pragma unroll
+                for (int i = 0; i < 2 * KSTEPS; ++i) {
+                    *reinterpret_cast<uint4 *>(st_rows + lane * 8 + i * 512) = kk[i / KSTEPS][i % KSTEPS].u;
+                    *reinterpret_cast<uint4 *>(st_rows + lane * 8 + (2 * KSTEPS + i) * 512) = vv[2][i].u;
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                if (lane == 0) __hip_atomic_store(&sm_q_ready, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
             __builtin_amdgcn_s_setprio(0);
         } else {
@@ -1213,6 +1220,56 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     if (SAGE && FUSED && head_ok) qsc = sm_qscale[n] * a.scale_log2e;
     FA_TR(3);
 
+    __half open_scale = __float2half(0.0f);
+    if constexpr (SAGE && FUSED) {
+        if (owns_new) {  // uniform over the workgroup
+            // The open block's rows up to p, quantised anew (a block has one scale, and the new row may raise it), by all waves
+            // while their own blocks are on their way; wave 0 attends and stores it (below). With all of it in wave 0, 64 values to a lane,
+            // the launch waited for that up to about 16K keys: SmolLM3, a step at 2000 / 8000 / 12000 / 32768 keys 8.6 -> 8.4,
+            // 9.8 -> 9.5, 10.1 -> 9.8, 13.6 -> 13.6 us. (Each wave asking for its share of the rows itself holds up the first requests
+            // of all workgroups: 1 % less below 12000 keys, 1 to 2 % more at 20000.)
+            const uint32_t r = p & (FA_SAGE_BLOCK - 1);
+            // Thread t has piece t % TPR (8 dims) of row t / TPR (+ NT i / TPR) of the block.
+            constexpr int TPR = D / 8, TI = ((int)FA_SAGE_BLOCK * TPR + NT - 1) / NT;
+            constexpr bool WHOLE = (int)FA_SAGE_BLOCK * TPR % NT == 0;  // (else the last threads repeat the last piece)
+            float x[TI][8], peak = 0.0f;
+            while (__hip_atomic_load(&sm_q_ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < 2u) __builtin_amdgcn_s_sleep(1);  // the new row is there
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+                const uint32_t item = WHOLE ? tid + NT * i : min((uint32_t)(tid + NT * i), FA_SAGE_BLOCK * TPR - 1), row = item / TPR, col = item % TPR * 8;
+                const U4H nw = {*reinterpret_cast<const uint4 *>(st_krot + col)};
+                const f4_t m0 = *reinterpret_cast<const f4_t *>(st_mean + col), m1 = *reinterpret_cast<const f4_t *>(st_mean + col + 4);
+                const uint4 old = *reinterpret_cast<const uint4 *>(st_rows + item * 8);
+                const u4_t raw = __builtin_bit_cast(u4_t, row == r ? nw.u : old);
+                float pk = 0.0f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    x[i][2 * w] = sage_lo_minus(raw[w], w < 2 ? m0[2 * w] : m1[2 * w - 4]);
+                    x[i][2 * w + 1] = sage_hi_minus(raw[w], w < 2 ? m0[2 * w + 1] : m1[2 * w - 3]);
+                    pk = sage_max3(pk, x[i][2 * w], x[i][2 * w + 1]);
+                }
+                peak = fmaxf(peak, row <= r ? pk : 0.0f);  // (what the rows past the new one come to is masked below and not stored)
+            }
+            peak = group_reduce<64, true>(peak);
+            if (lane == 0) st_peak[wave] = peak;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < NW; ++w) peak = fmaxf(peak, st_peak[w]);
+            FA_TR(12);
+            open_scale = __float2half_rn(peak / 127.0f);
+            const SageDivisor dv = sage_divisor(__half2float(open_scale));
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+                const uint32_t item = WHOLE ? tid + NT * i : min((uint32_t)(tid + NT * i), FA_SAGE_BLOCK * TPR - 1), row = item / TPR, col = item % TPR * 8;
+                *reinterpret_cast<uint2 *>(st_k8 + row * D + col) =
+                    make_uint2(sage_quant4_i8(x[i][0], x[i][1], x[i][2], x[i][3], dv), sage_quant4_i8(x[i][4], x[i][5], x[i][6], x[i][7], dv));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0) __hip_atomic_fetch_add(&sm_open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    }
+
     f4_t oacc[DBLK];
 #pragma unroll
     for (int blk = 0; blk < DBLK; ++blk) oacc[blk] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
@@ -1341,51 +1398,18 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
 
     if constexpr (SAGE && FUSED) {
         if (owns_new && wave == 0) {
-            // The open block, rows b0 .. p: its earlier rows are exact in the tail, the new row is in the staging area.
-            // All of them are quantised anew (a block has one scale, and the new row may raise it), stored, and attended
-            // from the registers they were made in; rows past p carry no weight.
-            // One wave does it, 64 values to a lane, and up to about 16K keys it is what the launch waits for: its instructions count.
-            // (Seven per value, lane exchanges in registers, the rows' choice instead of branches, and the query likewise: a step of
-            // SmolLM3 at 300 / 8000 / 20000 / 32768 keys 10.1 -> 8.3, 11.3 -> 9.7, 11.5 -> 10.2, 13.9 -> 13.6 us.)
+            // The open block, rows b0 .. p, quantised above: attended from the staging area, then stored; rows past p carry no weight.
             const bool writer = y % a.sub_per_kv == 0;
             const uint32_t r = p & (FA_SAGE_BLOCK - 1), b0 = p - r, nsb = r / BK + 1;
             __half *tail = a.sage_tail + (size_t)kvh * FA_SAGE_BLOCK * D;
-            // (the V rows of the block were requested when the position was read; the new row is patched in below)
-            float kx[2][KSTEPS][16];
-            float amax = 0.0f;
-#pragma unroll
-            for (int sb = 0; sb < 2; ++sb) {
-                const uint32_t row = sb * BK + n;
-                float peak = 0.0f;
-#pragma unroll
-                for (int j = 0; j < KSTEPS; ++j) {
-                    const uint32_t col = (4 * j + c) * 16;
-                    const u4_t nw[2] = {*reinterpret_cast<const u4_t *>(st_krot + col), *reinterpret_cast<const u4_t *>(st_krot + col + 8)};
-                    const u4_t old[2] = {__builtin_bit_cast(u4_t, kk[sb][j].u), __builtin_bit_cast(u4_t, vv[2][sb * KSTEPS + j].u)};  // requested before the first barrier
-#pragma unroll
-                    for (int w = 0; w < 8; ++w) {
-                        const uint32_t word = row == r ? nw[w / 4][w % 4] : old[w / 4][w % 4];
-                        const f2_t mu = *reinterpret_cast<const f2_t *>(st_mean + col + 2 * w);
-                        float *x = kx[sb][j] + 2 * w;
-                        x[0] = sage_lo_minus(word, mu.x), x[1] = sage_hi_minus(word, mu.y);
-                        peak = sage_max3(peak, x[0], x[1]);
-                    }
-                }
-                amax = fmaxf(amax, row <= r ? peak : 0.0f);  // (what the rows past the new one come to is masked below and not stored)
-            }
-            amax = group_reduce<64, true>(amax);
-            FA_TR(12);
-            const __half sc16 = __float2half_rn(amax / 127.0f);
-            const SageDivisor dv = sage_divisor(__half2float(sc16));
             int8_t *kq = const_cast<int8_t *>(reinterpret_cast<const int8_t *>(kbase)) + (size_t)b0 * D;
+            // (the V rows of the block were requested when the position was read; the new row is patched in below)
+            while (__hip_atomic_load(&sm_open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < (uint32_t)NW) __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 #pragma unroll
             for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-                for (int j = 0; j < KSTEPS; ++j) {
-                    const float *kv = kx[sb][j];
-                    kk[sb][j].u = make_uint4(sage_quant4_i8(kv[0], kv[1], kv[2], kv[3], dv), sage_quant4_i8(kv[4], kv[5], kv[6], kv[7], dv),
-                                             sage_quant4_i8(kv[8], kv[9], kv[10], kv[11], dv), sage_quant4_i8(kv[12], kv[13], kv[14], kv[15], dv));
-                }
+                for (int j = 0; j < KSTEPS; ++j) kk[sb][j].u = *reinterpret_cast<const uint4 *>(st_k8 + (sb * BK + n) * D + (4 * j + c) * 16);
             // the new V row into its place among the block's rows (load i holds rows i VRPL .. of a 16-row block)
             {
                 const uint32_t rr = r % BK, sbn = r / BK;
@@ -1397,7 +1421,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             }
             // (the V blocks go through this wave's LDS region, which is the staging area: take the rotated row out first)
             const uint4 krot16 = *reinterpret_cast<const uint4 *>(st_krot + (lane % (D / 8)) * 8);
-            ksr[0] = ksr[1] = (_Float16)sc16;
+            ksr[0] = ksr[1] = (_Float16)open_scale;
             FA_TR(13);
             consume(b0, nsb, p + 1, 0, 0);
             FA_TR(14);
@@ -1409,7 +1433,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
                     for (int j = 0; j < KSTEPS; ++j)
                         if ((uint32_t)(sb * BK + n) <= r)
                             *reinterpret_cast<uint4 *>(kq + (size_t)(sb * BK + n) * D + (4 * j + c) * 16) = kk[sb][j].u;
-                if (lane == 0) const_cast<__half *>(a.k_scale)[(size_t)kvh * a.ks_stride + b0 / FA_SAGE_BLOCK] = sc16;
+                if (lane == 0) const_cast<__half *>(a.k_scale)[(size_t)kvh * a.ks_stride + b0 / FA_SAGE_BLOCK] = open_scale;
                 if (lane < D / 8) *reinterpret_cast<uint4 *>(tail + (size_t)r * D + lane * 8) = krot16;
                 if (lane < VLPR) *reinterpret_cast<uint4 *>(const_cast<__half *>(vbase) + (size_t)p * D + lane * 8) = sage_vnew;
             }

@@ -37,7 +37,8 @@ __device__ __forceinline__ uint32_t sage_quant_byte(float x, const SageDivisor &
 }
 
 // Four values -> four int8 in a word (value i in byte i). Six instructions per value with its share of the packing; with a
-// second step, a rounding, two for the clamp and a conversion they were nearly ten.
+// second step, a rounding, two for the clamp and a conversion they were nearly ten. (A decode step of SmolLM3 at 300 / 8000 / 20000 /
+// 32768 keys, the query and the difference from the mean likewise: 10.1 -> 8.4, 11.3 -> 9.8, 11.5 -> 10.2, 13.9 -> 13.6 us.)
 __device__ __forceinline__ uint32_t sage_quant4_i8(float x0, float x1, float x2, float x3, const SageDivisor &v) {
     const uint32_t lo = __builtin_amdgcn_perm(sage_quant_byte(x1, v), sage_quant_byte(x0, v), 0x0c0c0400u);
     const uint32_t hi = __builtin_amdgcn_perm(sage_quant_byte(x3, v), sage_quant_byte(x2, v), 0x0c0c0400u);
