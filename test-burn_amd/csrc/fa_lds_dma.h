@@ -20,7 +20,9 @@ __device__ __forceinline__ rsrc_words make_rsrc_words(const void *base, uint32_t
 // buffer_to_lds_b128 is for tiles that other workgroups read again (they should stay in L2); buffer_to_lds_b128_nt
 // marks rows that are read once per launch as non-temporal, so that a launch's stream does not push the kernel's
 // own code out of L2 (a workgroup then starts with instruction fetches from memory). (When the steps differ, the
-// source-offset update sits between the m0 write and the load that needs it.)
+// source-offset update sits between the m0 write and the load that needs it.) A vector memory instruction must come five wait
+// states after a vector instruction (v_readlane of a page's place, of a spilled scalar) that wrote a scalar it reads. The compiler keeps
+// them for its own instructions and does not look into these, which had as few as two; the move to m0 and the s_nop 3 are five.
 #define FA_LDS_DMA_DEFINE(NAME, POLICY) \
 template <int N, int SRC_STEP, int DST_STEP> \
 __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff, int soff) { \
@@ -28,7 +30,7 @@ __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff,
     if constexpr (SRC_STEP == DST_STEP) { \
         static_assert((N - 1) * SRC_STEP < 4096, "12-bit immediate"); \
         if constexpr (N == 4) \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\t" \
                          "buffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" "\n\t" \
                          "buffer_load_dwordx4 %1, %2, %3 offen offset:%4" POLICY " lds" "\n\t" \
                          "buffer_load_dwordx4 %1, %2, %3 offen offset:%5" POLICY " lds" "\n\t" \
@@ -37,21 +39,21 @@ __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff,
                          : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff), "n"(SRC_STEP), "n"(2 * SRC_STEP), "n"(3 * SRC_STEP) \
                          : "memory"); \
         else if constexpr (N == 2) \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t" \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\t" \
                          "buffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" "\n\t" \
                          "buffer_load_dwordx4 %1, %2, %3 offen offset:%4" POLICY " lds" \
                          : \
                          : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff), "n"(SRC_STEP) \
                          : "memory"); \
         else \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" \
                          : \
                          : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff) \
                          : "memory"); \
     } else { \
         int so = soff; \
         if constexpr (N == 4) \
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\t" \
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 3\n\t" \
                          "buffer_load_dwordx4 %2, %3, %0 offen" POLICY " lds" "\n\t" \
                          "s_add_i32 m0, %1, %5\n\ts_add_i32 %0, %0, %4\n\t" \
                          "buffer_load_dwordx4 %2, %3, %0 offen" POLICY " lds" "\n\t" \
@@ -63,7 +65,7 @@ __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff,
                          : "s"(lds_addr), "v"(voff), "s"(rs), "n"(SRC_STEP), "n"(DST_STEP), "n"(2 * DST_STEP), "n"(3 * DST_STEP) \
                          : "memory", "scc"); \
         else if constexpr (N == 2) \
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\t" \
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 3\n\t" \
                          "buffer_load_dwordx4 %2, %3, %0 offen" POLICY " lds" "\n\t" \
                          "s_add_i32 m0, %1, %5\n\ts_add_i32 %0, %0, %4\n\t" \
                          "buffer_load_dwordx4 %2, %3, %0 offen" POLICY " lds" \
@@ -71,7 +73,7 @@ __device__ __forceinline__ void NAME(rsrc_words rs, uint32_t lds_addr, int voff,
                          : "s"(lds_addr), "v"(voff), "s"(rs), "n"(SRC_STEP), "n"(DST_STEP) \
                          : "memory", "scc"); \
         else \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen" POLICY " lds" \
                          : \
                          : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff) \
                          : "memory"); \
@@ -81,7 +83,7 @@ FA_LDS_DMA_DEFINE(buffer_to_lds_b128, "")
 // One such load to lds_addr + ahead, a number that is known when the kernel is built: for loops with more places in LDS than there
 // are scalar registers to keep their addresses in.
 __device__ __forceinline__ void buffer_to_lds_b128_ahead(rsrc_words rs, uint32_t lds_addr, uint32_t ahead, int voff, int soff) {
-    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff), "i"(ahead)
                  : "memory", "scc");
