@@ -38,6 +38,14 @@ class TensorArg(C.Structure):
                 ("dims", C.c_size_t * 4), ("strides", C.c_size_t * 4)]
 
 
+def tensor_args(args):
+    """A C array of the arguments: their bytes one after the other, where they are all of the type itself (56 of them, the caches of 28
+    layers, 1.2 us; given to the array's constructor, which sets element after element, 12.8)."""
+    if {*map(type, args)} == {TensorArg}:
+        return (TensorArg * len(args)).from_buffer_copy(b"".join(args))
+    return (TensorArg * max(len(args), 1))(*args)
+
+
 class KvPrepFusedParams(C.Structure):
     _fields_ = [(n, C.c_uint32) for n in (
         "d_model", "kv_dim", "head_dim", "n_heads", "n_kv_heads", "group_size", "seq_len", "position_offset",
@@ -480,7 +488,7 @@ class Foundry:
     def kv_prefix_copy_batch(self, srcs, dsts, prefix_len):
         n = len(srcs)
         assert n == len(dsts)
-        sa, da = (TensorArg * max(n, 1))(*srcs), (TensorArg * max(n, 1))(*dsts)
+        sa, da = tensor_args(srcs), tensor_args(dsts)
         check(self.lib.fa_kv_prefix_copy_batch(self.h, sa, da, n, prefix_len))
 
     def sage_k_mean(self, k, n_kv_heads, capacity, head_dim, kv_len, mean_out):

@@ -103,3 +103,27 @@ def test_header_is_plain_c99_and_links_from_c(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "InvalidShape" in out.stdout
+
+
+def test_tensor_args_are_the_arguments():
+    """The array that a batched call takes holds the arguments' bytes in order, in both of the ways that it is made."""
+    class Derived(fa.TensorArg):
+        pass
+
+    def arg(cls, i):
+        t = cls()
+        t.buffer, t.offset, t.dtype, t.rank = 4096 * (i + 1), 16 * i, i, 3
+        t.dims[:], t.strides[:] = [i + 1, i + 2, i + 3, 0], [i + 4, i + 5, 1, 0]
+        return t
+
+    for cls in (fa.TensorArg, Derived):
+        for n in (1, 2, 57):
+            args = [arg(cls, i) for i in range(n)]
+            array = fa.tensor_args(args)
+            assert array._type_ is fa.TensorArg and len(array) == n
+            assert bytes(array) == b"".join(bytes(a) for a in args)
+    assert len(fa.tensor_args([])) == 1
+    with pytest.raises(TypeError):
+        fa.tensor_args([arg(fa.TensorArg, 0), bytes(88)])
+    with pytest.raises(TypeError):
+        fa.tensor_args([bytes(88)])
