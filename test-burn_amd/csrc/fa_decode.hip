@@ -1,6 +1,7 @@
 // Host-side launch logic of the flash-decode kernels (partition sizing, scratch, kernel selection).
 #include "fa_decode_impl.h"
 
+#include <algorithm>
 #include <mutex>
 
 // Decode partials of the entry point that allocates nothing (fa_decode_step_fused_noalloc): every GPU the library runs
@@ -97,6 +98,9 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         return c;
     };
     uint32_t waves = ctx->decode_waves;  // 0 = by the rule above
+    const uint32_t n4 = (uint32_t)gt * L.head_dim / 4;  // records (float4 columns of all heads) per partition
+    const bool one = L.batch == 1 && ctx->decode_waves == 0;
+    const bool one_pass = n4 <= 128, int8 = L.sage_fused || L.q_scale;  // (one_pass: two lanes of four waves' for each record)
     bool short_context = false;
     if (waves == 0) {
         const uint32_t c8 = chunk ? chunk : auto_chunk(8, n_cus);
@@ -107,17 +111,38 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         if (waves == 8 && !chunk) {
             const uint32_t s_max = groups >= n_cus ? 1u : (uint32_t)(n_cus / groups);
             short_context = ceil_div_u32(bound, s_max) <= 4u * BK;
+            // One sequence: up to 128 keys to a unit's share (one round of a workgroup's three streaming waves) where the four waves
+            // fold and merge their heads in one pass; where they do not, up to 96 partitions of 64. us, eight waves or 64 keys -> this:
+            //   H24 / Hkv8 / D128: 2100 keys 7.60 -> 6.51, 3000 7.78 -> 6.92, 4000 8.09 -> 7.75; H32 / Hkv32 / D128: 600 7.83 -> 6.64
+            //   H16 / Hkv4 / D128: 5000 9.35 -> 8.66, 8000 10.27 -> 9.85 (int8 10.1 -> 10.3: not for its four groups)
+            //   H14 / Hkv2 / D64: 5000 7.39 -> 6.66, 8000 7.72 -> 7.08, 16000 9.08 -> 8.42
+            //   H16 / Hkv2 / D128, two passes: 7000 11.00 -> 10.22 with eight waves; 6000 10.35, 10.39 (H8 / Hkv1 9.55, 9.99)
+            if (one && one_pass && (!int8 || s_max > 64)) short_context = ceil_div_u32(bound, s_max) <= 8u * BK;
+            else if (one && !one_pass) short_context = short_context && bound <= 96u * 4u * BK;
             if (short_context) waves = 4;
         }
     }
-    if (chunk == 0) chunk = waves == 4 ? auto_chunk(4, short_context ? n_cus : 2 * n_cus) : auto_chunk(8, n_cus);
+    if (chunk == 0) {
+        chunk = waves == 4 ? auto_chunk(4, short_context ? n_cus : 2 * n_cus) : auto_chunk(8, n_cus);
+        if (one) {
+            // One sequence of few head groups has units for more partitions than are worth their records. Up to 64 partitions are merged
+            // in registers, more of them through LDS: they stay at 64 as long as that leaves four waves 128 keys, eight waves 256, and
+            // eight waves that fold in two passes have 192 at least. us, by the units -> by this rule:
+            //   H16 / Hkv2 / D128: 8000 keys 11.36 -> 10.31, 12000 11.75 -> 10.87, 16000 12.78 -> 11.30, 24000 13.13 -> 12.70
+            //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07, 20000 9.40 -> 8.99, 30000 9.68 -> 9.50 (int8 10.3 -> 10.5 from 20000 on: not there)
+            const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK;
+            uint32_t least = 0;
+            if (waves == 4) least = short_context ? std::min(8u * BK, by64) : 0u;
+            else if (!int8 || !one_pass || by64 <= 16u * BK) least = std::max(one_pass ? 0u : 12u * BK, std::min(16u * BK, by64));
+            chunk = std::max(chunk, least);
+        }
+    }
     chunk = (chunk + BK - 1) / BK * BK;
     // the int8 step in one launch: the open 32-row block must lie inside one partition
     if (L.sage_fused) chunk = (chunk + FA_SAGE_BLOCK - 1) / FA_SAGE_BLOCK * FA_SAGE_BLOCK;
     uint32_t S = ceil_div_u32(bound, chunk);
     // The polled merge needs every workgroup of the launch resident at once (the merging workgroup of a head group
     // occupies its compute unit while it waits) and its partials in the context's pattern-filled buffer.
-    const uint32_t n4 = (uint32_t)gt * L.head_dim / 4;  // records (float4 columns of all heads) per partition
     const uint64_t slots = waves == 4 ? 2 * n_cus : n_cus;
     // a workgroup reads ceil(n4 / partitions) columns of every partition (fewer than n4 + partitions records for
     // any partition count up to S), at most POLL_IPT records per thread
@@ -191,9 +216,12 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         // workgroups: the grid is padded to 8 head groups, group g's workgroups land on XCD g, and the workgroups of
         // the groups that do not exist leave at once. Such a launch is all latency (its partitions were sized for that
         // above), and the exchange through one XCD's L2 is most of a microsecond shorter than through device-coherent
-        // accesses (6.15 -> 5.4 us per launch at 1K context).
+        // accesses (6.15 -> 5.4 us per launch at 1K context). A workgroup to a compute unit: with up to two, the XCDs of the groups
+        // are what the launch waits for (H14 / Hkv2 / D64, 2100 keys, 33 partitions 6.74 padded, 6.19 not, 4000 keys 7.50, 6.68; H16 / Hkv4 /
+        // D128, 4000 8.86, 8.12), except with three groups and more of int8 rows (4000 keys 10.6, 10.8) or many records (H32 / Hkv4 /
+        // D128, 2100 keys 9.61, 9.96).
         if (!a.xcd_local && ctx->xcd_round_robin && L.batch == 1 && groups < 8 && waves == 4) {  // (only the 4-wave kernels know of the padding)
-            const uint64_t per_xcd = (uint64_t)2u * (n_cus / 8u);
+            const uint64_t per_xcd = (ny > 2 && (int8 || !one_pass) ? 2u : 1u) * (n_cus / 8u);
             const size_t need_pad = (size_t)8 * S * n4 * 32;
             if (S <= per_xcd && (uint64_t)8 * S <= slots && need_pad <= ctx->poll_ws_bytes) ny_grid = 8, a.xcd_local = 1u, a.ny_real = ny;
         }
