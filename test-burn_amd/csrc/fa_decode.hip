@@ -102,7 +102,16 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     const bool one = L.batch == 1 && ctx->decode_waves == 0;
     const bool one_pass = n4 <= 128, int8 = L.sage_fused || L.q_scale;  // (one_pass: two lanes of four waves' for each record)
     bool short_context = false;
-    if (waves == 0) {
+    // As few keys as four waves have in one round of requests: one partition, which writes the output itself. (The longest sequence 80 / 120
+    // keys, partitions of 64 or 128 -> one: H24 / Hkv8 / D128 5.87, 5.93 -> 4.94, 5.00 us; H16 / Hkv2 / D128 6.21, 6.30 -> 5.11, 5.24;
+    // H14 / Hkv2 / D64 5.06, 4.99 -> 4.03, 4.09; 8 paged sequences of 16-140, H16 / Hkv2 / D128 7.54 -> 6.33. 180 keys in two rounds: 5.97 ->
+    // 5.91, 7.13 -> 6.20, 5.06 -> 4.79, but H16 / Hkv4 5.76 -> 6.18.) Not where units go without (60 sequences of 90-100, Hkv4: 6.35, 6.81),
+    // and a contiguous cache whose length the device has is asked for up to the bound: with more than two head groups the rows
+    // past the length cost as much below 64 keys (a block of H24 / Hkv8: 17.6 -> 18.2) as the merge does above (18.7 -> 18.3).
+    const bool whole = waves == 0 && !chunk && 2 * groups <= n_cus && (L.paged || !L.d_len || ny <= 2) && bound <= (int8 ? 8u : 3u * MBX) * BK;
+    if (whole) {
+        waves = 4, chunk = ceil_div_u32(bound, (uint32_t)BK) * BK;
+    } else if (waves == 0) {
         const uint32_t c8 = chunk ? chunk : auto_chunk(8, n_cus);
         waves = groups * ceil_div_u32(bound, (c8 + BK - 1) / BK * BK) > n_cus ? 4u : 8u;
         // A context so short that even four waves get at most one block each (at most 64 keys per compute unit's
@@ -119,6 +128,9 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             //   H16 / Hkv2 / D128, two passes: 7000 11.00 -> 10.22 with eight waves; 6000 10.35, 10.39 (H8 / Hkv1 9.55, 9.99)
             if (one && one_pass && (!int8 || s_max > 64)) short_context = ceil_div_u32(bound, s_max) <= 8u * BK;
             else if (one && !one_pass) short_context = short_context && bound <= 96u * 4u * BK;
+            // A batch: eight waves where four fold in two passes. (H16 / Hkv2 / D128: 2 sequences of 125-1000 tokens 8.85 -> 8.25 us, of
+            // 500-4000 10.04 -> 9.27, 5 of 37-300 8.55 -> 7.87, 32 of 12-100 6.84 -> 6.29)
+            else if (L.batch >= 2 && !one_pass) short_context = false;
             if (short_context) waves = 4;
         }
     }

@@ -300,8 +300,8 @@ def test_fused_step_new_token_alone_and_not_finite(H, Hkv, D, pos):
 
 
 @pytest.mark.parametrize("H,Hkv,D,lengths", [
-    (24, 8, 128, (2048, 2049, 4096, 4097)), (16, 4, 128, (2048, 2049, 4097, 8192, 8193)), (16, 2, 128, (2049, 4097, 6144, 6145, 12289, 16385, 32769)),
-    (14, 2, 64, (2049, 4097, 8193, 16384, 16385, 32769)), (8, 1, 128, (2049, 6145, 16385)), (32, 4, 128, (2049, 4097, 6145)), (32, 32, 128, (513, 1024, 1025))])
+    (24, 8, 128, (1, 65, 144, 145, 2048, 2049, 4096, 4097)), (16, 4, 128, (2048, 2049, 4097, 8192, 8193)), (16, 2, 128, (2049, 4097, 6144, 6145, 12289, 16385, 32769)),
+    (14, 2, 64, (63, 65, 129, 144, 145, 2049, 4097, 8193, 16384, 16385, 32769)), (8, 1, 128, (2049, 6145, 16385)), (32, 4, 128, (2049, 4097, 6145)), (32, 32, 128, (513, 1024, 1025))])
 def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
     """How one sequence is divided - waves, keys of a partition, where the partitions of a group lie - changes with its length: either
     side of each line, the fused step against f64 attention and, with f16 and with int8 keys, against the two-launch merge."""
@@ -311,7 +311,7 @@ def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
     cap = max(lengths)
     kc, vc = (h16(rng.normal(size=(Hkv, cap, D))) for _ in range(2))
     dk, dv = f.array(kc), f.array(vc)
-    cos, sin = fa.rope_tables(1e6, D, 1)
+    cos, sin = fa.rope_tables(1e6, D, cap)
     dcos, dsin = f.array(cos), f.array(sin)
     for n in lengths:
         q = h16(rng.normal(size=(1, H * D)))
@@ -319,7 +319,7 @@ def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
         w = np.exp(s - s.max(axis=-1, keepdims=True))
         want = np.matmul(w / w.sum(axis=-1, keepdims=True), vc[:, :n].astype(np.float64)).reshape(H, D)
         dq, dkn, dvn = f.array(q), f.array(kc[:, n - 1].reshape(1, -1)), f.array(vc[:, n - 1].reshape(1, -1))
-        # (nothing is rotated: layer 3 of a model that leaves out every 4th; the tables' one row is enough for a device-side position)
+        # (nothing is rotated: layer 3 of a model that leaves out every 4th)
         p = fa.KvPrepFusedParams.make(H, Hkv, D, 1, n - 1, cap, fa.ROPE_NEOX, layer_idx=3, no_rope_layer_step=4)
         dpos, outs = f.array(np.array([n - 1], np.uint32)), []
         desc, bufs = fa.sage_cache(f, H, Hkv, cap, D, dv)
@@ -327,7 +327,10 @@ def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
         for merge in (2, 1):
             f.set_decode_variant(merge=merge)
             do, do8 = f.zeros((1, H * D)), f.zeros((1, H * D))
-            f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p, dpos, n)
+            if merge == 2:  # a length that the host has, and one that the device has
+                f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p)
+            else:
+                f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p, dpos, n)
             f.sage_decode_step(dq.arg(), dkn.arg(), dvn.arg(), desc, dcos.arg(), dsin.arg(), do8.arg(), p, d_position=dpos, kv_len_bound=n)
             f.synchronize()
             outs.append([x.download().reshape(H, D) for x in (do, do8)])
