@@ -106,36 +106,54 @@ __device__ __forceinline__ void store_out4(__half *op, const float (&o)[4], bool
 }
 
 
-// Value of lane (l ^ 16) / (l ^ 32): one VALU lane-swap each on gfx950.
-__device__ __forceinline__ float xor16(float x) {
-    const unsigned v = __float_as_uint(x);
-    u2_t r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    // the swap exchanges the odd 16-lane rows of the first operand with the even rows of the second
-    return __uint_as_float(((threadIdx.x >> 4) & 1) ? r.x : r.y);
+// Lane exchanges, as few instructions as they go. A launch of a few microseconds runs through the code after its loop once, and each wave
+// waits for every line of it to be fetched: 1.4 KB less of it (selects between the two results of a swap, and moves ahead of DPP
+// operations, both for nothing) took a step over 1024 keys from 8.06 to 7.50 us at 2 K/V heads of 128 and from 5.62 to 5.32 at 2 of 64,
+// one over 8192 at 8 of 128 from 9.87 to 9.53, 16 int8 steps over 32768 from 237.5 to 233.3. `both`: op of a lane's value and that of lane l ^ 16 / l ^ 32, one VALU swap of lane groups whose two results are the
+// operands in either order (op commutes). Inside a row of 16 lanes the exchange is part of the operation (DPP: every lane has its
+// source, so the bound control is free to be what lets the compiler fold the move).
+struct OpMax {
+    __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); }
+};
+struct OpAdd {
+    __device__ __forceinline__ float operator()(float x, float y) const { return x + y; }
+};
+template <class Op>
+__device__ __forceinline__ float both16(float x) {
+    const u2_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return Op()(__uint_as_float(r.x), __uint_as_float(r.y));
 }
-__device__ __forceinline__ float xor32(float x) {
-    const unsigned v = __float_as_uint(x);
-    u2_t r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return __uint_as_float(((threadIdx.x >> 5) & 1) ? r.x : r.y);
+template <class Op>
+__device__ __forceinline__ float both32(float x) {
+    const u2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return Op()(__uint_as_float(r.x), __uint_as_float(r.y));
 }
-
-// Reductions over aligned groups of 2 to 64 consecutive lanes; every lane of the group gets the result. Lane
-// exchanges inside a 16-lane row are DPP moves (quad permutes, then the mirrors of a half row and of a row), the step
-// across rows is a lane swap. The order of the operands is fixed, so results are reproducible.
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
+// One step of a reduction over aligned groups of consecutive lanes, which doubles the group: step 1 pairs, step 6 the wave.
+template <int STEP, class Op>
+__device__ __forceinline__ float group_step(float v) {
+    if constexpr (STEP == 1) return Op()(v, dpp_mov<0xB1>(v));   // quad_perm [1,0,3,2]: lane ^ 1
+    if constexpr (STEP == 2) return Op()(v, dpp_mov<0x4E>(v));   // quad_perm [2,3,0,1]: lane ^ 2
+    if constexpr (STEP == 3) return Op()(v, dpp_mov<0x141>(v));  // row_half_mirror: the other quad of the 8 lanes
+    if constexpr (STEP == 4) return Op()(v, dpp_mov<0x140>(v));  // row_mirror: the other half of the row
+    if constexpr (STEP == 5) return both16<Op>(v);
+    if constexpr (STEP == 6) return both32<Op>(v);
+}
+// Reductions over groups of 2 to 64 lanes; every lane of the group gets the result. The order of the operands is fixed, so results are
+// reproducible.
 template <int G, bool MAX>
 __device__ __forceinline__ float group_reduce(float v) {
     static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0, "a power of two");
-    auto op = [](float x, float y) { return MAX ? fmaxf(x, y) : x + y; };
-    v = op(v, dpp_mov<0xB1>(v));                // quad_perm [1,0,3,2]: lane ^ 1
-    if (G >= 4) v = op(v, dpp_mov<0x4E>(v));    // quad_perm [2,3,0,1]: lane ^ 2
-    if (G >= 8) v = op(v, dpp_mov<0x141>(v));   // row_half_mirror: the other quad of the 8 lanes
-    if (G >= 16) v = op(v, dpp_mov<0x140>(v));  // row_mirror: the other half of the row
-    if (G >= 32) v = op(v, xor16(v));
-    if (G >= 64) v = op(v, xor32(v));
+    typedef typename std::conditional<MAX, OpMax, OpAdd>::type Op;
+    v = group_step<1, Op>(v);
+    if constexpr (G >= 4) v = group_step<2, Op>(v);
+    if constexpr (G >= 8) v = group_step<3, Op>(v);
+    if constexpr (G >= 16) v = group_step<4, Op>(v);
+    if constexpr (G >= 32) v = group_step<5, Op>(v);
+    if constexpr (G >= 64) v = group_step<6, Op>(v);
     return v;
 }
 
@@ -447,23 +465,24 @@ __device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint
         }
         // the group's maximum, then the weighted sums; `sh` steps of lane exchanges each
         float mstar = m_r;
-        if (sh >= 1) mstar = fmaxf(mstar, dpp_mov<0xB1>(mstar));
-        if (sh >= 2) mstar = fmaxf(mstar, dpp_mov<0x4E>(mstar));
-        if (sh >= 3) mstar = fmaxf(mstar, dpp_mov<0x141>(mstar));
-        if (sh >= 4) mstar = fmaxf(mstar, dpp_mov<0x140>(mstar));
-        if (sh >= 5) mstar = fmaxf(mstar, xor16(mstar));
-        if (sh >= 6) mstar = fmaxf(mstar, xor32(mstar));
+        if (sh >= 1) mstar = group_step<1, OpMax>(mstar);
+        if (sh >= 2) mstar = group_step<2, OpMax>(mstar);
+        if (sh >= 3) mstar = group_step<3, OpMax>(mstar);
+        if (sh >= 4) mstar = group_step<4, OpMax>(mstar);
+        if (sh >= 5) mstar = group_step<5, OpMax>(mstar);
+        if (sh >= 6) mstar = group_step<6, OpMax>(mstar);
         const float w = fast_exp2(m_r - mstar);
         float v[5] = {l_r * w, acc[0] * w, acc[1] * w, acc[2] * w, acc[3] * w};
+        auto add = [&](auto step) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < 5; ++e) {
-            if (sh >= 1) v[e] += dpp_mov<0xB1>(v[e]);
-            if (sh >= 2) v[e] += dpp_mov<0x4E>(v[e]);
-            if (sh >= 3) v[e] += dpp_mov<0x141>(v[e]);
-            if (sh >= 4) v[e] += dpp_mov<0x140>(v[e]);
-            if (sh >= 5) v[e] += xor16(v[e]);
-            if (sh >= 6) v[e] += xor32(v[e]);
-        }
+            for (int e = 0; e < 5; ++e) v[e] = group_step<decltype(step)::value, OpAdd>(v[e]);
+        };
+        if (sh >= 1) add(std::integral_constant<int, 1>{});
+        if (sh >= 2) add(std::integral_constant<int, 2>{});
+        if (sh >= 3) add(std::integral_constant<int, 3>{});
+        if (sh >= 4) add(std::integral_constant<int, 4>{});
+        if (sh >= 5) add(std::integral_constant<int, 5>{});
+        if (sh >= 6) add(std::integral_constant<int, 6>{});
         if (col < n4 && p == 0) {
             const uint32_t h = col / CG, c4 = col - h * CG;
             const float L = v[0];
@@ -1326,8 +1345,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
             }
             mt = fmaxf(mt, s[i]);
         }
-        mt = fmaxf(mt, xor16(mt));
-        mt = fmaxf(mt, xor32(mt));
+        mt = both32<OpMax>(both16<OpMax>(mt));
 #ifdef FA_DECODE_TRACE
         if (tstamp[4] == 0) FA_TR(4);  // the first round's K blocks have arrived and S is there
 #endif
@@ -1465,8 +1483,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
                           : __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[0][j].h, q_op(j).h, sf, 0, 0, 0);
             float sc = sf[0] * qsc;  // in lanes c == 0
             sc = c == 0 ? (isfinite(sc) ? sc : -1e30f) : -INFINITY;
-            sc = fmaxf(sc, xor16(sc));
-            sc = fmaxf(sc, xor32(sc));
+            sc = both32<OpMax>(both16<OpMax>(sc));
             m_run = fmaxf(m_run, sc);
             const float weight = fast_exp2(sc - m_run);  // (0 below -1e30)
             l_run = c == 0 ? weight : 0.0f;
@@ -1496,8 +1513,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
 
     FA_TR(6);
     // the head's sum over the four 16-lane rows (the running max is already common to them)
-    l_run += xor16(l_run);
-    l_run += xor32(l_run);
+    l_run = both32<OpAdd>(both16<OpAdd>(l_run));
 
     // Fold of the NW waves through LDS: sm_acc[wave][head][D] (+ 8 floats per wave, see below), sm_ml[wave][head][2].
     // With up to OWN_GT heads the states have a region of their own, so a wave writes its state as soon as it is done (the
