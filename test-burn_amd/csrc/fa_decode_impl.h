@@ -87,6 +87,11 @@ constexpr int OWN_GT = 8;    // up to this many, the waves' states at the end of
 using DecodeDev = ::FaDecodeDev;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// Where a launch mostly goes, so that what it runs through lies in a row (a macro: an inline function loses the hint). The way from the
+// loop through the fold and the merge in one XCD's L2 without a jump over the other forms: 1 to 2 % of a step (1024 keys, 2 K/V heads of
+// 128: 7.49 to 7.41 us; 2000 keys, 8 of 128: 6.23 to 6.11; 16 int8 steps over 8000 keys: 183.3 to 179.6), the other forms within +-1 %.
+#define FA_LIKELY(x) __builtin_expect(!!(x), 1)
+#define FA_UNLIKELY(x) __builtin_expect(!!(x), 0)
 
 // Element i of a 16-byte data chunk as f32 / an f32 rounded (to nearest even) to the storage type.
 __device__ __forceinline__ float elem_f32(const U4H &x, int i, bool bf16) {
@@ -109,9 +114,10 @@ __device__ __forceinline__ void store_out4(__half *op, const float (&o)[4], bool
 // Lane exchanges, as few instructions as they go. A launch of a few microseconds runs through the code after its loop once, and each wave
 // waits for every line of it to be fetched: 1.4 KB less of it (selects between the two results of a swap, and moves ahead of DPP
 // operations, both for nothing) took a step over 1024 keys from 8.06 to 7.50 us at 2 K/V heads of 128 and from 5.62 to 5.32 at 2 of 64,
-// one over 8192 at 8 of 128 from 9.87 to 9.53, 16 int8 steps over 32768 from 237.5 to 233.3. `both`: op of a lane's value and that of lane l ^ 16 / l ^ 32, one VALU swap of lane groups whose two results are the
-// operands in either order (op commutes). Inside a row of 16 lanes the exchange is part of the operation (DPP: every lane has its
-// source, so the bound control is free to be what lets the compiler fold the move).
+// one over 8192 at 8 of 128 from 9.87 to 9.53, 16 int8 steps over 32768 from 237.5 to 233.3.
+// `both`: op of a lane's value and that of lane l ^ 16 / l ^ 32, one VALU swap of lane groups whose two results are the operands in
+// either order (op commutes). Inside a row of 16 lanes the exchange is part of the operation (DPP: every lane has its source, so the
+// bound control is free to be what lets the compiler fold the move).
 struct OpMax {
     __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); }
 };
@@ -449,12 +455,12 @@ __device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint
                          ml.x != POLL_SENTINEL && ml.y != POLL_SENTINEL);
             }
             if (!__any(pend)) break;
-            if (wall_clock64() - t_begin > a.poll_ticks) {
+            if (FA_UNLIKELY(wall_clock64() - t_begin > a.poll_ticks)) {
                 ok = false;
                 break;
             }
         }
-        if (!ok) break;  // uniform over the wave
+        if (FA_UNLIKELY(!ok)) break;  // uniform over the wave
         float m_r = valid ? __uint_as_float(ml.x) : -1e30f, l_r = valid ? __uint_as_float(ml.y) : 0.0f;
         f4_t acc = valid ? __builtin_bit_cast(f4_t, x) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
         if (valid) {  // consumed: back to the pattern for the next launch
@@ -1194,7 +1200,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     // A position at or past the launch bound / the capacity: the token is neither appended nor attended. The host
     // finds the bit at its next synchronize.
     if (FUSED && (BAL ? place.dropped : n_raw > N) && tid == 0 && blockIdx.x == 0 && y == 0 && a.status) a.status[FA_DEVSTAT_APPEND_DROPPED] = 1u;
-    if (split >= nsplits || pad_wg) {  // uniform over the workgroup
+    if (FA_UNLIKELY(split >= nsplits || pad_wg)) {  // uniform over the workgroup
         FA_TR_FLUSH();
         return;
     }
@@ -1520,7 +1526,7 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
     // waves finish spread over the streaming time) and only the last wave's write is left before the barrier; with
     // more heads the region would not fit beside the V tiles and reuses them once every wave is done with them.
     const bool own_region = gt <= OWN_GT;
-    if (!own_region) __syncthreads();  // every wave is done with its V region
+    if (FA_UNLIKELY(!own_region)) __syncthreads();  // every wave is done with its V region
     float *sm_acc = own_region ? reinterpret_cast<float *>(rope_lds + 2 * D) : reinterpret_cast<float *>(smem);
     const uint32_t wstr = gt * D + 8;  // a wave pair is 2 wstr apart: 64 bytes off a multiple of the bank span
     float *sm_ml = sm_acc + (size_t)NW * wstr;
@@ -1565,19 +1571,19 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) A[i] = group_reduce<LPC, false>(a0[i] * e0 + a1[i] * e1);
         if (!valid || wsel != 0) continue;
-        if (nsplits == 1) {
+        if (FA_UNLIKELY(nsplits == 1)) {
             const float inv = (isfinite(L) && fabsf(L) > 1e-6f) ? (1.0f / L) : 1.0f;
             __half *op = tl.out + (size_t)b * tl.out_stride_b + (size_t)(head0 + h) * tl.out_stride_h + c4 * 4;
             const float ov[4] = {A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv};
             store_out4(op, ov, BF16);
-        } else if (polled) {
+        } else if (FA_LIKELY(polled)) {
             // record of (this partition, column idx); a word that equals the arrival pattern would never be seen as arrived
             const u4_t r0 = {__float_as_uint(not_sentinel(A[0])), __float_as_uint(not_sentinel(A[1])),
                              __float_as_uint(not_sentinel(A[2])), __float_as_uint(not_sentinel(A[3]))};
             const u2_t r1 = {__float_as_uint(not_sentinel(ms)), __float_as_uint(not_sentinel(L))};
             const __amdgpu_buffer_rsrc_t rs = make_rsrc(tl.part_acc + gpart * (gt * CG) * 8);
             const uint32_t ro = (split * (gt * CG) + (uint32_t)idx) * 32u;
-            if (xcd_local) {
+            if (FA_LIKELY(xcd_local)) {
                 __builtin_amdgcn_raw_buffer_store_b128(r0, rs, (int)ro, 0, 0);
                 __builtin_amdgcn_raw_buffer_store_b64(r1, rs, (int)ro + 16, 0, 0);
             } else {
@@ -1599,16 +1605,16 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         }
     }
     FA_TR(9);
-    if (nsplits == 1 || !in_kernel) {
+    if (FA_UNLIKELY(nsplits == 1 || !in_kernel)) {
         FA_TR_FLUSH();
         return;
     }
-    if (polled) {
+    if (FA_LIKELY(polled)) {
         bool ok;
-        if (nsplits <= 64) {
-            ok = xcd_local ? coop_merge_in_registers<D, true>(tl, b, y, split, nsplits, gpart, tid)
-                             : coop_merge_in_registers<D, false>(tl, b, y, split, nsplits, gpart, tid);
-            if (!ok && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
+        if (FA_LIKELY(nsplits <= 64)) {
+            ok = FA_LIKELY(xcd_local) ? coop_merge_in_registers<D, true>(tl, b, y, split, nsplits, gpart, tid)
+                                      : coop_merge_in_registers<D, false>(tl, b, y, split, nsplits, gpart, tid);
+            if (FA_UNLIKELY(!ok) && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
             FA_TR(10);
             FA_TR_FLUSH();
             return;
