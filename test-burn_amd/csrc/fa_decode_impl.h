@@ -296,7 +296,7 @@ __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, 
 }
 
 // Cooperative polled merge (one launch, no ticket). Every partition's workgroup writes its partial state as records
-//   rec[group][partition][column] = {acc.x, acc.y, acc.z, acc.w, m, l, -, -}    column = head * D/4 + float4 column
+//   sums[group][column][partition] = {acc.x, acc.y, acc.z, acc.w}, then stats[..][..] = {m, l}    column = head * D/4 + float4 column
 // and then merges a share of the columns itself: workgroup c of the group's `nsplits` owns columns c, c + nsplits, ...
 // and reads those columns' records of ALL partitions. What bounds a merge is how fast one compute unit can request
 // the partials (one unit pulling a head group's 50 KB needs about 2 us), so the reads are spread over all of them.
@@ -306,10 +306,14 @@ __device__ __forceinline__ void merge_and_store(const DecodeDev &a, uint32_t b, 
 // nothing is stored and false is returned - and writes the pattern back over what it has consumed (each record is
 // read by exactly one thread of the launch). No workgroup waits for one that has not been started yet unless the
 // launch exceeds the resident capacity, which the host rules out.
+// The merging wave's loads are the scarce thing (several hundred waves poll at once in one L2), so the records of a column lie side by
+// side, sums and (m, l) apart: 64 partitions are 12 cache lines. As 32-byte records with the columns side by side a load met 64 lines,
+// 4 or 8 KB apart and so in one channel of the L2, twice; the stores, one pass of scattered pieces now, cost less than that. 3000 and
+// 16000 keys, 2 K/V heads of 128 with 8 query heads each: 8.61 -> 7.82 and 11.20 -> 10.45 us a step; 8000 at 4 with 4: 9.66 -> 8.88.
 constexpr uint32_t POLL_SENTINEL = 0xffffffffu;
 constexpr int POLL_IPT = 4;  // records per thread, at most
-__device__ __forceinline__ float not_sentinel(float v) {  // the pattern is a NaN: a partial stores the canonical one instead
-    return __float_as_uint(v) == POLL_SENTINEL ? __uint_as_float(0x7fc00000u) : v;
+__device__ __forceinline__ uint32_t not_sentinel(float v) {  // the pattern is a NaN, the largest word: a partial stores the next one, a NaN too
+    return min(__float_as_uint(v), POLL_SENTINEL - 1u);
 }
 // LOCAL: every workgroup of the head group runs on the same XCD. Records are then written with plain stores (they go
 // through to that XCD's L2) and read with device-scope loads (which pass the compute unit's own cache and hit the L2):
@@ -322,6 +326,7 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
     const uint32_t gt = a.gt, n4 = gt * CG;
     const uint32_t my_cols = n4 > c ? (n4 - c + nsplits - 1) / nsplits : 0u;
     const uint32_t items = my_cols * nsplits;  // <= NT * POLL_IPT (host)
+    const uint32_t ml_base = nsplits * n4 * 16u;
     const size_t g = (size_t)b * gridDim.y + y;
     const float *rec = a.part_acc + g * S * n4 * 8;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(rec);
@@ -331,17 +336,17 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
     bool timed_out = false;
     u4_t x[POLL_IPT];
     u2_t ml[POLL_IPT];
-    uint32_t off[POLL_IPT];  // byte offset of the record
+    uint32_t rec_of[POLL_IPT];
     uint32_t pend = 0;
 #pragma unroll
     for (int j = 0; j < POLL_IPT; ++j) {
         const uint32_t t = tid + j * NT;
         if (t < items) {
             const uint32_t i = t / nsplits, p = t - i * nsplits;
-            off[j] = ((p * n4) + c + i * nsplits) * 32u;
+            rec_of[j] = (c + i * nsplits) * nsplits + p;
             pend |= 1u << j;
         } else {
-            off[j] = 0;
+            rec_of[j] = 0;
         }
     }
     const uint32_t mine = pend;
@@ -349,8 +354,8 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 #pragma unroll
         for (int j = 0; j < POLL_IPT; ++j) {
             if (pend >> j & 1u) {
-                x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[j], 0, LD_POLICY);
-                ml[j] = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off[j] + 16, 0, LD_POLICY);
+                x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(rec_of[j] * 16u), 0, LD_POLICY);
+                ml[j] = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)(ml_base + rec_of[j] * 8u), 0, LD_POLICY);
             }
         }
 #pragma unroll
@@ -384,8 +389,8 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 #pragma unroll
         for (int j = 0; j < POLL_IPT; ++j) {
             if (mine >> j & 1u) {
-                __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)off[j], 0, ST_POLICY);
-                __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)off[j] + 16, 0, ST_POLICY);
+                __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)(rec_of[j] * 16u), 0, ST_POLICY);
+                __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)(ml_base + rec_of[j] * 8u), 0, ST_POLICY);
             }
         }
     }
@@ -427,78 +432,75 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 }
 
 // The same merge for up to 64 partitions, without LDS and without a barrier: a column's records are read by a group
-// of P2 consecutive lanes (P2 = the power of two that holds the partitions), one partition per lane, and the group
+// of G consecutive lanes (G = the power of two that holds the partitions), one partition per lane, and the group
 // folds them with lane exchanges. A wave depends on no other wave.
-template <int D, bool LOCAL>
-__device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t c,
-                                                        uint32_t nsplits, size_t first, int tid) {  // first: the group's first partition
+// What a wave runs through here and in the fold before it is a chain of some hundred instructions, several cycles each since a SIMD has
+// one or two waves: the code is written once for each G, without a branch for each step of the exchange, and the addresses of the other
+// forms of a launch are not on its way. With the steps behind branches and one fold for all forms, a step over 300 / 1024 keys at 2 K/V
+// heads of 128 took 6.90 / 7.42 us instead of 6.30 / 6.87, over 1024 at 2 of 64 5.32 instead of 4.98.
+template <int D, bool LOCAL, bool BF16, int G>
+__device__ __forceinline__ bool coop_merge_of_group(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t c, uint32_t nsplits,
+                                                    __amdgpu_buffer_rsrc_t rs, int tid) {  // rs: the group's records
     constexpr int LD_POLICY = LOCAL ? 0x10 /* sc1 */ : CACHE_COHERENT, ST_POLICY = LOCAL ? 0 : CACHE_COHERENT;
     constexpr int CG = D / 4;
     const uint32_t gt = a.gt, n4 = gt * CG;
-    const uint32_t sh = 32u - (uint32_t)__builtin_clz(nsplits - 1u);  // 2 <= nsplits <= 64: 1 .. 6
-    const uint32_t p = (uint32_t)tid & ((1u << sh) - 1u), gi = (uint32_t)tid >> sh, gpw = (uint32_t)NT >> sh;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.part_acc + first * n4 * 8);
+    const uint32_t p = (uint32_t)tid % G, gi = (uint32_t)tid / G;
+    const uint32_t ml_base = nsplits * n4 * 16u;
     const unsigned long long t_begin = wall_clock64();
-    bool ok = true;
-    for (uint32_t base = 0; c + base * nsplits < n4; base += gpw) {  // uniform over the workgroup
-        const uint32_t col = c + (base + gi) * nsplits;
+    for (uint32_t base = 0; c + base * nsplits < n4; base += NT / G) {  // uniform over the workgroup
+        const uint32_t col = c + __umul24(base + gi, nsplits);
         const bool valid = col < n4 && p < nsplits;
-        const uint32_t off = (p * n4 + col) * 32u;
-        u4_t x = {0u, 0u, 0u, 0u};
-        u2_t ml = {0u, 0u};
+        const uint32_t rec = __umul24(col, nsplits) + p, off = rec * 16u, off_ml = ml_base + rec * 8u;
+        u4_t x = {0u, 0u, 0u, 0u};  // (what a lane without a record keeps)
+        u2_t ml = {__float_as_uint(-1e30f), 0u};
         bool pend = valid;
         for (;;) {
             if (pend) {
                 x = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, LD_POLICY);
-                ml = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off + 16, 0, LD_POLICY);
+                ml = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off_ml, 0, LD_POLICY);
                 pend = !(x.x != POLL_SENTINEL && x.y != POLL_SENTINEL && x.z != POLL_SENTINEL && x.w != POLL_SENTINEL &&
                          ml.x != POLL_SENTINEL && ml.y != POLL_SENTINEL);
             }
             if (!__any(pend)) break;
-            if (FA_UNLIKELY(wall_clock64() - t_begin > a.poll_ticks)) {
-                ok = false;
-                break;
-            }
+            if (FA_UNLIKELY(wall_clock64() - t_begin > a.poll_ticks)) return false;  // uniform over the wave
         }
-        if (FA_UNLIKELY(!ok)) break;  // uniform over the wave
-        float m_r = valid ? __uint_as_float(ml.x) : -1e30f, l_r = valid ? __uint_as_float(ml.y) : 0.0f;
-        f4_t acc = valid ? __builtin_bit_cast(f4_t, x) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        const float m_r = __uint_as_float(ml.x), l_r = __uint_as_float(ml.y);
+        const f4_t acc = __builtin_bit_cast(f4_t, x);
         if (valid) {  // consumed: back to the pattern for the next launch
             const u4_t sent4 = {POLL_SENTINEL, POLL_SENTINEL, POLL_SENTINEL, POLL_SENTINEL};
             const u2_t sent2 = {POLL_SENTINEL, POLL_SENTINEL};
             __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)off, 0, ST_POLICY);
-            __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)off + 16, 0, ST_POLICY);
+            __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)off_ml, 0, ST_POLICY);
         }
-        // the group's maximum, then the weighted sums; `sh` steps of lane exchanges each
-        float mstar = m_r;
-        if (sh >= 1) mstar = group_step<1, OpMax>(mstar);
-        if (sh >= 2) mstar = group_step<2, OpMax>(mstar);
-        if (sh >= 3) mstar = group_step<3, OpMax>(mstar);
-        if (sh >= 4) mstar = group_step<4, OpMax>(mstar);
-        if (sh >= 5) mstar = group_step<5, OpMax>(mstar);
-        if (sh >= 6) mstar = group_step<6, OpMax>(mstar);
+        // the group's maximum, then the weighted sums
+        const float mstar = group_reduce<G, true>(m_r);
         const float w = fast_exp2(m_r - mstar);
         float v[5] = {l_r * w, acc[0] * w, acc[1] * w, acc[2] * w, acc[3] * w};
-        auto add = [&](auto step) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < 5; ++e) v[e] = group_step<decltype(step)::value, OpAdd>(v[e]);
-        };
-        if (sh >= 1) add(std::integral_constant<int, 1>{});
-        if (sh >= 2) add(std::integral_constant<int, 2>{});
-        if (sh >= 3) add(std::integral_constant<int, 3>{});
-        if (sh >= 4) add(std::integral_constant<int, 4>{});
-        if (sh >= 5) add(std::integral_constant<int, 5>{});
-        if (sh >= 6) add(std::integral_constant<int, 6>{});
+        for (int e = 0; e < 5; ++e) v[e] = group_reduce<G, false>(v[e]);
         if (col < n4 && p == 0) {
             const uint32_t h = col / CG, c4 = col - h * CG;
             const float L = v[0];
             const float inv = (isfinite(L) && fabsf(L) > 1e-6f) ? (1.0f / L) : 1.0f;
             __half *op = a.out + (size_t)b * a.out_stride_b + (size_t)(y * gt + h) * a.out_stride_h + c4 * 4;
             const float ov[4] = {v[1] * inv, v[2] * inv, v[3] * inv, v[4] * inv};
-            store_out4(op, ov, a.bf16 != 0);
+            store_out4(op, ov, BF16);
         }
     }
-    return ok;
+    return true;
+}
+
+template <int D, bool LOCAL, bool BF16>
+__device__ __forceinline__ bool coop_merge_in_registers(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t c, uint32_t nsplits,
+                                                        __amdgpu_buffer_rsrc_t rs, int tid) {
+    switch (32u - (uint32_t)__builtin_clz(nsplits - 1u)) {  // 2 <= nsplits <= 64
+        case 1: return coop_merge_of_group<D, LOCAL, BF16, 2>(a, b, y, c, nsplits, rs, tid);
+        case 2: return coop_merge_of_group<D, LOCAL, BF16, 4>(a, b, y, c, nsplits, rs, tid);
+        case 3: return coop_merge_of_group<D, LOCAL, BF16, 8>(a, b, y, c, nsplits, rs, tid);
+        case 4: return coop_merge_of_group<D, LOCAL, BF16, 16>(a, b, y, c, nsplits, rs, tid);
+        case 5: return coop_merge_of_group<D, LOCAL, BF16, 32>(a, b, y, c, nsplits, rs, tid);
+        default: return coop_merge_of_group<D, LOCAL, BF16, 64>(a, b, y, c, nsplits, rs, tid);
+    }
 }
 
 // Sums over the wave and running sums along its lanes of a non-negative integer (DPP moves within the rows of 16 lanes, then the
@@ -1542,82 +1544,68 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
 
     const bool in_kernel = tl.merge_in_kernel != 0, polled = tl.merge_in_kernel == 2;
     // the first partition of this (sequence, head group) in the exchange buffers
-    const size_t gpart = BAL ? (size_t)y * S + place.first : ((size_t)b * GY + y) * S;
-    const size_t gbase = gpart * gt;  // and its first row
+    // (a number of records that are there: 32 bits hold it)
+    const uint32_t gpart = BAL ? y * S + place.first : (b * GY + y) * S;
     bool xcd_local = tl.xcd_local != 0;
     if (BAL) {  // all of the sequence's partitions among the slots of this XCD?
         const uint32_t per_xcd = a.bal_slots >> 16, xcd_first = ((blockIdx.x + gridDim.x * blockIdx.y) & 7u) * per_xcd;
         xcd_local = gpart >= xcd_first && gpart + nsplits <= xcd_first + per_xcd;  // (never for per_xcd = 0)
     }
-    const uint32_t prow = split * gt;
     constexpr int CG = D / 4;
     // LPC = NW / 2 consecutive lanes share a column (head h, float4 column c4): lane j merges the states of waves 2j and
     // 2j + 1, the group merges its lanes' results, and its first lane owns the column's state. One pass for up to 4 heads.
+    // (Once for each form of a launch, so that the addresses of one are not computed on the way of another.)
     constexpr int LPC = NW / 2;
-    const int wsel = tid % LPC;
-    for (int base = 0; base < (int)gt * CG * LPC; base += NT) {  // uniform over the workgroup
-        const int idx = (base + tid) / LPC;
-        const bool valid = idx < (int)gt * CG;
-        const int h = valid ? idx / CG : 0, c4 = valid ? idx % CG : 0;
-        const f2_t ml0 = *reinterpret_cast<const f2_t *>(sm_ml + ((2 * wsel) * gt + h) * 2);
-        const f2_t ml1 = *reinterpret_cast<const f2_t *>(sm_ml + ((2 * wsel + 1) * gt + h) * 2);
-        const f4_t a0 = *reinterpret_cast<const f4_t *>(sm_acc + (size_t)(2 * wsel) * wstr + h * D + c4 * 4);
-        const f4_t a1 = *reinterpret_cast<const f4_t *>(sm_acc + (size_t)(2 * wsel + 1) * wstr + h * D + c4 * 4);
-        const float m_w = fmaxf(ml0.x, ml1.x);
-        const float ms = group_reduce<LPC, true>(m_w);
-        const float e0 = fast_exp2(ml0.x - ms), e1 = fast_exp2(ml1.x - ms);
-        const float L = group_reduce<LPC, false>(ml0.y * e0 + ml1.y * e1);
-        f4_t A;
+    auto fold = [&](auto &&put) __attribute__((always_inline)) {
+        const uint32_t wsel = tid % LPC;
+        for (int base = 0; base < (int)gt * CG * LPC; base += NT) {  // uniform over the workgroup
+            const int idx = (base + tid) / LPC;
+            const bool valid = idx < (int)gt * CG;
+            const uint32_t h = valid ? idx / CG : 0, c4 = valid ? idx % CG : 0;
+            const uint32_t st = __umul24(2 * wsel, gt) + h;  // (fewer than 2^24 floats)
+            const f2_t ml0 = *reinterpret_cast<const f2_t *>(sm_ml + st * 2);
+            const f2_t ml1 = *reinterpret_cast<const f2_t *>(sm_ml + (st + gt) * 2);
+            const float *s0 = sm_acc + __umul24(2 * wsel, wstr) + h * D + c4 * 4;
+            const f4_t a0 = *reinterpret_cast<const f4_t *>(s0);
+            const f4_t a1 = *reinterpret_cast<const f4_t *>(s0 + wstr);
+            const float m_w = fmaxf(ml0.x, ml1.x);
+            const float ms = group_reduce<LPC, true>(m_w);
+            const float e0 = fast_exp2(ml0.x - ms), e1 = fast_exp2(ml1.x - ms);
+            const float L = group_reduce<LPC, false>(ml0.y * e0 + ml1.y * e1);
+            f4_t A;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) A[i] = group_reduce<LPC, false>(a0[i] * e0 + a1[i] * e1);
-        if (!valid || wsel != 0) continue;
-        if (FA_UNLIKELY(nsplits == 1)) {
-            const float inv = (isfinite(L) && fabsf(L) > 1e-6f) ? (1.0f / L) : 1.0f;
-            __half *op = tl.out + (size_t)b * tl.out_stride_b + (size_t)(head0 + h) * tl.out_stride_h + c4 * 4;
-            const float ov[4] = {A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv};
-            store_out4(op, ov, BF16);
-        } else if (FA_LIKELY(polled)) {
-            // record of (this partition, column idx); a word that equals the arrival pattern would never be seen as arrived
-            const u4_t r0 = {__float_as_uint(not_sentinel(A[0])), __float_as_uint(not_sentinel(A[1])),
-                             __float_as_uint(not_sentinel(A[2])), __float_as_uint(not_sentinel(A[3]))};
-            const u2_t r1 = {__float_as_uint(not_sentinel(ms)), __float_as_uint(not_sentinel(L))};
-            const __amdgpu_buffer_rsrc_t rs = make_rsrc(tl.part_acc + gpart * (gt * CG) * 8);
-            const uint32_t ro = (split * (gt * CG) + (uint32_t)idx) * 32u;
-            if (FA_LIKELY(xcd_local)) {
-                __builtin_amdgcn_raw_buffer_store_b128(r0, rs, (int)ro, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b64(r1, rs, (int)ro + 16, 0, 0);
-            } else {
-                __builtin_amdgcn_raw_buffer_store_b128(r0, rs, (int)ro, 0, CACHE_COHERENT);
-                __builtin_amdgcn_raw_buffer_store_b64(r1, rs, (int)ro + 16, 0, CACHE_COHERENT);
-            }
-        } else if (in_kernel) {
-            float *pa = tl.part_acc + gbase * D, *pm = tl.part_ml + gbase * 2;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, A), make_rsrc(pa),
-                                                   (int)(((prow + h) * D + c4 * 4) * 4u), 0, CACHE_COHERENT);
-            if (c4 == 0) {
-                f2_t mlv = {ms, L};
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, mlv), make_rsrc(pm),
-                                                      (int)((prow + h) * 2 * 4u), 0, CACHE_COHERENT);
+            for (int i = 0; i < 4; ++i) A[i] = group_reduce<LPC, false>(a0[i] * e0 + a1[i] * e1);
+            if (valid && wsel == 0) put((uint32_t)idx, h, c4, A, ms, L);
+        }
+    };
+    if (FA_LIKELY(polled && nsplits > 1)) {
+        // record of (this partition, column idx); a word that equals the arrival pattern would never be seen as arrived
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(tl.part_acc + (uint64_t)gpart * (gt * CG * 8u));
+        const uint32_t ml_base = nsplits * (gt * CG) * 16u;
+        auto record = [&](auto policy) __attribute__((always_inline)) {
+            fold([&](uint32_t idx, uint32_t, uint32_t, f4_t A, float ms, float L) __attribute__((always_inline)) {
+                const u4_t r0 = {not_sentinel(A[0]), not_sentinel(A[1]), not_sentinel(A[2]), not_sentinel(A[3])};
+                const u2_t r1 = {not_sentinel(ms), not_sentinel(L)};
+                const uint32_t rec = __umul24(idx, nsplits) + split;
+                __builtin_amdgcn_raw_buffer_store_b128(r0, rs, (int)(rec * 16u), 0, decltype(policy)::value);
+                __builtin_amdgcn_raw_buffer_store_b64(r1, rs, (int)(ml_base + rec * 8u), 0, decltype(policy)::value);
+            });
+        };
+        bool ok;
+        if (FA_LIKELY(xcd_local)) {
+            record(std::integral_constant<int, 0>{});
+            FA_TR(9);
+            if (FA_LIKELY(nsplits <= 64)) {
+                ok = coop_merge_in_registers<D, true, BF16>(tl, b, y, split, nsplits, rs, tid);
+                goto merged;
             }
         } else {
-            *reinterpret_cast<f4_t *>(tl.part_acc + (gbase + prow + h) * D + c4 * 4) = A;
-            if (c4 == 0) tl.part_ml[(gbase + prow + h) * 2] = ms, tl.part_ml[(gbase + prow + h) * 2 + 1] = L;
-        }
-    }
-    FA_TR(9);
-    if (FA_UNLIKELY(nsplits == 1 || !in_kernel)) {
-        FA_TR_FLUSH();
-        return;
-    }
-    if (FA_LIKELY(polled)) {
-        bool ok;
-        if (FA_LIKELY(nsplits <= 64)) {
-            ok = FA_LIKELY(xcd_local) ? coop_merge_in_registers<D, true>(tl, b, y, split, nsplits, gpart, tid)
-                                      : coop_merge_in_registers<D, false>(tl, b, y, split, nsplits, gpart, tid);
-            if (FA_UNLIKELY(!ok) && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
-            FA_TR(10);
-            FA_TR_FLUSH();
-            return;
+            record(std::integral_constant<int, CACHE_COHERENT>{});
+            FA_TR(9);
+            if (nsplits <= 64) {
+                ok = coop_merge_in_registers<D, false, BF16>(tl, b, y, split, nsplits, rs, tid);
+                goto merged;
+            }
         }
         __syncthreads();  // the fold above read the LDS region that the merge reuses
         if (xcd_local) {
@@ -1625,9 +1613,44 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         } else {
             ok = coop_merge_and_store<D, false>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));
         }
-        if (!ok && tid == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
+    merged:
+        if (FA_UNLIKELY(!ok) && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
+        FA_TR(10);
+        FA_TR_FLUSH();
         return;
     }
+    if (nsplits == 1) {
+        fold([&](uint32_t, uint32_t h, uint32_t c4, f4_t A, float, float L) __attribute__((always_inline)) {
+            const float inv = (isfinite(L) && fabsf(L) > 1e-6f) ? (1.0f / L) : 1.0f;
+            __half *op = tl.out + (size_t)b * tl.out_stride_b + (size_t)(head0 + h) * tl.out_stride_h + c4 * 4;
+            const float ov[4] = {A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv};
+            store_out4(op, ov, BF16);
+        });
+        FA_TR(9);
+        FA_TR_FLUSH();
+        return;
+    }
+    const size_t gbase = (size_t)gpart * gt;  // the first row of the group
+    const uint32_t prow = split * gt;
+    if (!in_kernel) {
+        fold([&](uint32_t, uint32_t h, uint32_t c4, f4_t A, float ms, float L) __attribute__((always_inline)) {
+            *reinterpret_cast<f4_t *>(tl.part_acc + (gbase + prow + h) * D + c4 * 4) = A;
+            if (c4 == 0) tl.part_ml[(gbase + prow + h) * 2] = ms, tl.part_ml[(gbase + prow + h) * 2 + 1] = L;
+        });
+        FA_TR(9);
+        FA_TR_FLUSH();
+        return;
+    }
+    fold([&](uint32_t, uint32_t h, uint32_t c4, f4_t A, float ms, float L) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, A), make_rsrc(tl.part_acc + gbase * D),
+                                               (int)(((prow + h) * D + c4 * 4) * 4u), 0, CACHE_COHERENT);
+        if (c4 == 0) {
+            f2_t mlv = {ms, L};
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2_t, mlv), make_rsrc(tl.part_ml + gbase * 2),
+                                                  (int)((prow + h) * 2 * 4u), 0, CACHE_COHERENT);
+        }
+    });
+    FA_TR(9);
 
     // The last workgroup of this (sequence, head group) to arrive merges all partitions. The partials were
     // stored write-through; wait until those stores have completed (vmcnt(0)), then take a ticket. No

@@ -445,6 +445,39 @@ def test_polled_merge_equals_merge_kernel_over_many_launches():
             b.free()
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(16, 2, 128), (14, 2, 64), (32, 4, 128), (12, 12, 64)])
+def test_polled_merge_of_every_number_of_partitions(H, Hkv, D):
+    """The polled merge has a form for each power of two that holds the partitions (up to 64, in registers), one above, and finds a
+    record by column, partition and their number: either side of each power, the partitions' workgroups on one XCD and spread over
+    them, against f64 attention and, to one f16 unit in the last place, against the two-launch merge; then once more with the numbers in
+    descending order, in the record buffer that the other layouts have left."""
+    announce("polled merge, partitions", H, Hkv, D)
+    f = ctx()
+    rng = np.random.default_rng(5 * H + D)
+    counts, kps = (1, 2, 3, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65), 64
+    cap = kps * max(counts)
+    q, k, v = (h16(rng.normal(size=s)) for s in ((H, D), (Hkv, cap, D), (Hkv, cap, D)))
+    dq, dk, dv = f.array(q), f.array(k), f.array(v)
+    outs = {m: f.zeros((1, H * D)) for m in (1, 2)}
+    try:
+        for parts in counts + counts[::-1]:
+            n = kps * (parts - 1) + 1 + parts % kps
+            for merge, do in outs.items():
+                f.set_decode_variant(kps, merge)
+                f.flash_attention(dq.arg((1, H * D)), dk.arg(), dv.arg(), do.arg(), True, n - 1, H, D, n, 1)
+            f.synchronize()
+            a, b = (outs[m].download().astype(np.float64).reshape(H, D) for m in (1, 2))
+            s = np.einsum("kgd,knd->kgn", q.reshape(Hkv, H // Hkv, D).astype(np.float64), k[:, :n].astype(np.float64)) / np.sqrt(D)
+            w = np.exp(s - s.max(axis=-1, keepdims=True))
+            want = np.matmul(w / w.sum(axis=-1, keepdims=True), v[:, :n].astype(np.float64)).reshape(H, D)
+            assert max_abs(b, want) <= TOL, parts
+            assert np.all(np.abs(a - b) <= np.maximum(np.abs(a), 2.0 ** -14) * 2.0 ** -10), parts
+    finally:
+        f.set_decode_variant()
+    for x in (dq, dk, dv, *outs.values()):
+        x.free()
+
+
 def test_polled_merge_gives_up_cleanly():
     """Failure handling of the polled merge, forced from the host: with a wait bound of zero a merging workgroup gives
     up at its first look unless every record is already there. Every kernel still ends normally. The give-up is
