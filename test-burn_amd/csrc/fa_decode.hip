@@ -121,13 +121,15 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             const uint32_t s_max = groups >= n_cus ? 1u : (uint32_t)(n_cus / groups);
             short_context = ceil_div_u32(bound, s_max) <= 4u * BK;
             // One sequence: up to 128 keys to a unit's share (one round of a workgroup's three streaming waves) where the four waves
-            // fold and merge their heads in one pass; where they do not, up to 96 partitions of 64. us, eight waves or 64 keys -> this:
+            // fold and merge their heads in one pass, up to 64 where they do not, and only as far as 64 partitions of 128 keys go, the
+            // most that are merged in registers. us, eight waves or 64 keys -> this (the last two lines: more partitions, or eight waves):
             //   H24 / Hkv8 / D128: 2100 keys 7.60 -> 6.51, 3000 7.78 -> 6.92, 4000 8.09 -> 7.75; H32 / Hkv32 / D128: 600 7.83 -> 6.64
             //   H16 / Hkv4 / D128: 5000 9.35 -> 8.66, 8000 10.27 -> 9.85 (int8 10.1 -> 10.3: not for its four groups)
-            //   H14 / Hkv2 / D64: 5000 7.39 -> 6.66, 8000 7.72 -> 7.08, 16000 9.08 -> 8.42
-            //   H16 / Hkv2 / D128, two passes: 7000 11.00 -> 10.22 with eight waves; 6000 10.35, 10.39 (H8 / Hkv1 9.55, 9.99)
-            if (one && one_pass && (!int8 || s_max > 64)) short_context = ceil_div_u32(bound, s_max) <= 8u * BK;
-            else if (one && !one_pass) short_context = short_context && bound <= 96u * 4u * BK;
+            //   H14 / Hkv2 / D64: 5000 7.39 -> 6.66, 8000 7.72 -> 7.08; four waves beyond: 8300 6.90, 7.45, 10000 7.27, 7.60 (int8 8.8, 9.9)
+            //   H16 / Hkv2 / D128, two passes: 6200 9.17 -> 8.65, 7000 9.28 -> 8.73, 8100 9.33 -> 8.61 (int8 6200
+            //   11.7 -> 11.9: not there)
+            if (one && one_pass && (!int8 || s_max > 64)) short_context = ceil_div_u32(bound, std::min(s_max, 64u)) <= 8u * BK;
+            else if (one && !one_pass) short_context = short_context && bound <= (int8 ? 96u * 4u * BK : 64u * 8u * BK);
             // A batch: eight waves where four fold in two passes. (H16 / Hkv2 / D128: 2 sequences of 125-1000 tokens 8.85 -> 8.25 us, of
             // 500-4000 10.04 -> 9.27, 5 of 37-300 8.55 -> 7.87, 32 of 12-100 6.84 -> 6.29)
             else if (L.batch >= 2 && !one_pass) short_context = false;
@@ -138,14 +140,18 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         chunk = waves == 4 ? auto_chunk(4, short_context ? n_cus : 2 * n_cus) : auto_chunk(8, n_cus);
         if (one) {
             // One sequence of few head groups has units for more partitions than are worth their records. Up to 64 partitions are merged
-            // in registers, more of them through LDS: they stay at 64 as long as that leaves four waves 128 keys, eight waves 256, and
-            // eight waves that fold in two passes have 192 at least. us, by the units -> by this rule:
-            //   H16 / Hkv2 / D128: 8000 keys 11.36 -> 10.31, 12000 11.75 -> 10.87, 16000 12.78 -> 11.30, 24000 13.13 -> 12.70
-            //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07, 20000 9.40 -> 8.99, 30000 9.68 -> 9.50 (int8 10.3 -> 10.5 from 20000 on: not there)
+            // in registers, more of them through LDS: they stay at 64 as long as that leaves four waves 128 keys, eight waves 320 (of int8
+            // keys 512), beyond which eight waves have 256 and int8 keys that fold in one pass as many as the units; eight waves that
+            // fold in two passes have 192 at least. us, by the units -> by this rule (the second number of a pair: 256 keys):
+            //   H16 / Hkv2 / D128: 8000 keys 11.36 -> 10.31, 12000 11.75 -> 10.87, 16000 12.78 -> 11.30; 17000 11.46 -> 10.82, 20000
+            //   11.82 -> 11.59, but 25000 12.42 -> 13.03; int8 20000 12.9 -> 11.8, 32768 14.1 -> 13.8
+            //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07; 17000 8.70 -> 7.67, 20000 8.69 -> 8.01, 25000 8.95 -> 8.89, but 30000 9.17 -> 9.38; int8
+            //   20000 10.2 -> 9.1, 32768 10.7 -> 10.0
             const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK;
             uint32_t least = 0;
             if (waves == 4) least = short_context ? std::min(8u * BK, by64) : 0u;
-            else if (!int8 || !one_pass || by64 <= 16u * BK) least = std::max(one_pass ? 0u : 12u * BK, std::min(16u * BK, by64));
+            else if (by64 <= (int8 ? 32u : 20u) * BK) least = std::max(one_pass ? 0u : 12u * BK, by64);
+            else if (!int8 || !one_pass) least = 16u * BK;
             chunk = std::max(chunk, least);
         }
     }
