@@ -147,9 +147,12 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             //   11.82 -> 11.59, but 25000 12.42 -> 13.03; int8 20000 12.9 -> 11.8, 32768 14.1 -> 13.8
             //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07; 17000 8.70 -> 7.67, 20000 8.69 -> 8.01, 25000 8.95 -> 8.89, but 30000 9.17 -> 9.38; int8
             //   20000 10.2 -> 9.1, 32768 10.7 -> 10.0
-            const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK;
+            // Four waves stay at 32 as long as that leaves no more than two blocks to each of the three that stream, 96 keys: half a wave
+            // merges a column then instead of a whole one. us, 64 keys -> this: H32 / Hkv4 / D128: 2500 8.22 -> 7.33, 3000 8.41 -> 6.99; H16 /
+            // Hkv2 / D128: 3000 7.82 -> 7.40 (int8 2500 11.4 -> 10.3); H12 / Hkv6 / D64: 3000 5.60 -> 5.07; 96 keys in 42 partitions: 4000 7.77 -> 8.14.
+            const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK, by32 = ceil_div_u32(ceil_div_u32(bound, 32u), (uint32_t)BK) * BK;
             uint32_t least = 0;
-            if (waves == 4) least = short_context ? std::min(8u * BK, by64) : 0u;
+            if (waves == 4) least = !short_context ? 0u : by32 <= 6u * BK ? by32 : std::min(8u * BK, by64);
             else if (by64 <= (int8 ? 32u : 20u) * BK) least = std::max(one_pass ? 0u : 12u * BK, by64);
             else if (!int8 || !one_pass) least = 16u * BK;
             chunk = std::max(chunk, least);

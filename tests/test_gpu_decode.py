@@ -300,8 +300,8 @@ def test_fused_step_new_token_alone_and_not_finite(H, Hkv, D, pos):
 
 
 @pytest.mark.parametrize("H,Hkv,D,lengths", [
-    (24, 8, 128, (1, 65, 144, 145, 2048, 2049, 4096, 4097)), (16, 4, 128, (2048, 2049, 4097, 8192, 8193)), (16, 2, 128, (2049, 4097, 6144, 6145, 8192, 8193, 12289, 16385, 20480, 20481, 32768, 32769)),
-    (14, 2, 64, (63, 65, 129, 144, 145, 2049, 4097, 8192, 8193, 16384, 16385, 20480, 20481, 32768, 32769)), (8, 1, 128, (2049, 6145, 8192, 8193, 16385)), (32, 4, 128, (2049, 4097, 6145)), (32, 32, 128, (513, 1024, 1025))])
+    (24, 8, 128, (1, 65, 144, 145, 2048, 2049, 4096, 4097)), (16, 4, 128, (2048, 2049, 4097, 8192, 8193)), (16, 2, 128, (2049, 3072, 3073, 4097, 6144, 6145, 8192, 8193, 12289, 16385, 20480, 20481, 32768, 32769)),
+    (14, 2, 64, (63, 65, 129, 144, 145, 2049, 3072, 3073, 4097, 8192, 8193, 16384, 16385, 20480, 20481, 32768, 32769)), (8, 1, 128, (2049, 6145, 8192, 8193, 16385)), (32, 4, 128, (2049, 3072, 3073, 4097, 6145)), (32, 32, 128, (513, 1024, 1025))])
 def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
     """How one sequence is divided - waves, keys of a partition, where the partitions of a group lie - changes with its length: either
     side of each line, the fused step against f64 attention and, with f16 and with int8 keys, against the two-launch merge."""
