@@ -525,8 +525,8 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     const GemmDev &g = EARLY ? a : arguments();
     // What the column gives to each of its pieces: where the output of input row 0 would be, and the row from which on nothing is stored.
     struct Target {
-        __half *first;
-        uint32_t stride, end, paged_at;  // paged_at: place in a page of row 0 (K and V in a paged cache)
+        __half *first;  // (of a paged cache: of row 0 of page 0, 64 bits, as everything in a pool: one page of all heads may be 8 GiB)
+        uint32_t stride, end;
         bool paged;
     };
     Target target[NCOL];
@@ -537,7 +537,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             const Column &col = column[i];
             Target &o = target[i];
             o.first = pick3(col.mat, g.out[0], g.out[1], g.out[2]);
-            o.end = col.in ? g.m : 0u, o.paged = false, o.paged_at = 0;
+            o.end = col.in ? g.m : 0u, o.paged = false;
             if constexpr (W == PLAIN) {
                 o.stride = S::JOINED ? (col.mat ? rows1 : rows0) : N_tile;
                 o.first += col.gn;
@@ -545,9 +545,8 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                 const uint32_t D = g.rope.head_dim, head = col.gn >> hd_shift, hd = col.gn & (D - 1), room = g.rope.capacity > g.rope.position_offset ? g.rope.capacity - g.rope.position_offset : 0u;
                 o.stride = D;
                 o.paged = col.mat != 0 && g.rope.block_table;
-                o.paged_at = head * g.rope.block_size * D + hd;
                 if (col.mat != 0) o.end = min(o.end, room);  // never outside the cache
-                if (!o.paged) o.first += (col.mat == 0 ? (size_t)head * g.m : (size_t)head * g.rope.max_seq_len + g.rope.position_offset) * D + hd;
+                o.first += (col.mat == 0 ? (size_t)head * g.m : o.paged ? (size_t)head * g.rope.block_size : (size_t)head * g.rope.max_seq_len + g.rope.position_offset) * D + hd;
             }
         }
     };
@@ -593,7 +592,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             }
             if (g.rope.block_table) {
                 const uint32_t pos = g.rope.position_offset + gm, in_page = g.page_shift < 32 ? pos & (g.rope.block_size - 1) : pos % g.rope.block_size;
-                __half *const there = o.first + (size_t)w.page * g.rope.n_kv_heads * g.rope.block_size * g.rope.head_dim + o.paged_at + in_page * g.rope.head_dim;
+                __half *const there = o.first + ((size_t)w.page * g.rope.n_kv_heads * g.rope.block_size + in_page) * g.rope.head_dim;
                 dst = o.paged ? there : dst;
             }
         }

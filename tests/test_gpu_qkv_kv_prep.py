@@ -151,6 +151,41 @@ def test_fused_op_into_a_paged_cache(H, Hkv, D, K, m, pos, bs, mode):
         b.free()
 
 
+@pytest.mark.parametrize("bs", [1 << 22, (1 << 22) + 16])
+def test_fused_op_into_pages_of_which_one_holds_8_gib(bs):
+    """A pool of one very large page per sequence: the last head's rows lie 2^32 elements and more behind the first one's. The rows of
+    every head are where the paged layout has them ([page][head][row][dim]), against the two ops into a pool of small pages."""
+    announce("fused qkv + kv prep, one page of 8 GiB", bs)
+    f = ctx()
+    H, Hkv, D, K, m, pos = 9, 9, 128, 256, 40, 5
+    rng = np.random.default_rng(bs % 1000)
+    x, g, ws, _ = _data(rng, K, H * D, Hkv * D, m)
+    cos, sin = fa.rope_tables(1e6, D, pos + m)
+    dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+    dx, dg, dcos, dsin = f.array(x), f.array(g), f.array(cos), f.array(sin)
+    dq, dk, dv = (f.zeros((m, n)) for n in (H * D, Hkv * D, Hkv * D))
+    dqr = f.zeros((H, m, D))
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, m, pos, 0, fa.ROPE_NEOX)
+    pg = Paged(f, np.random.default_rng(5), [pos], Hkv, D, 16, extra_tokens=m + 1).upload()
+    pools = [fa.DevBuf(f, (Hkv, bs, D), np.float16) for _ in range(2)]
+    table, lens = f.zeros((1, 1), np.int32), f.array(np.array([pos], np.uint32))
+    assert (Hkv - 1) * bs * D >= 1 << 32
+    big = fa.paged_kv(pools[0], pools[1], table, lens, 1, Hkv, bs, D, 1, 1)
+    f.fused_qkv(dx.arg(), *[w.arg() for w in dev_w], dq.arg(), dk.arg(), dv.arg(), K, H * D, Hkv * D, m, gamma=dg.arg())
+    f.kv_prep_fused_paged(dq.arg(), dk.arg(), dv.arg(), dqr.arg(), pg.desc, 0, dcos.arg(), dsin.arg(), p)
+    f.fused_qkv_kv_prep(dx.arg(), *[w.arg() for w in dev_w], K, dqr.arg(), dcos.arg(), dsin.arg(), p, paged=big, seq_index=0, gamma=dg.arg())
+    f.synchronize()
+    for small, pool in ((pg.dk, pools[0]), (pg.dv, pools[1])):
+        want = orc.paged_gather(small.download(), pg.bt[0], Hkv, 16, D, pos + m)[:, pos:]
+        got = np.empty((m, D), np.float16)
+        for head in range(Hkv):
+            fa.check(f.lib.fa_download(f.h, got.ctypes.data, pool.ptr, ((head * bs) + pos) * D * 2, got.nbytes))
+            assert np.array_equal(bits(got), bits(want[head])), head
+    pg.free()
+    for b in dev_w + [dx, dg, dcos, dsin, dq, dk, dv, dqr, table, lens] + pools:
+        b.free()
+
+
 def test_fused_op_of_a_short_chunk_is_one_launch():
     """A chunk of 12 to 32 rows (the reference's default prefill chunk, src/model/executor.rs:232-250) against 2048 or 3072
     features: RMSNorm, projections, RoPE and the cache append leave ONE kernel (the profiler's launch counts)."""
