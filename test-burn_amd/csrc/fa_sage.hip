@@ -454,11 +454,17 @@ fa_status fa_launch_sage_build(fa_ctx *ctx, const void *k, uint32_t n_kv_heads, 
     float *partial;
     uint32_t n_parts;
     FA_TRY(launch_colsum(ctx, k, n_kv_heads, capacity, head_dim, kv_len, partial, n_parts));
-    // Up to 64 parts (8192 rows at D 128, 16384 at D 64) every workgroup of the quantiser adds them up itself, 32 KiB at most that its
-    // XCD's L2 holds: 4 heads of D 128, 300 rows 11.2 -> 7.3 us, 8000 rows 11.9 -> 11.3. Beyond them a launch of its own is
-    // ahead: 64 sums per head made by 64 workgroups of 1024 threads, which the quantiser could add up as well, took 21.6 us against
-    // 21.2 at 32768 rows, 36.8 against 29.4 for 2 heads of 100000.
-    const bool own_mean = n_parts <= MEAN_LANES;
+    // Where a lane has one part at most (up to 64 of them: their number grows with the rows, by one per 128 at D 128 and 256 at D 64, and
+    // falls with the heads) every workgroup of the quantiser adds them up itself: a launch less for sums that are read once per 128 rows
+    // from its XCD's L2. 4 heads of D 128, 300 rows 8.1 -> 6.3 us, 4000 9.6 -> 8.4, 8000 10.4 -> 10.1. What they all read again has to
+    // stay small beside that launch, 24 MB at D 128 and 48 at D 64 (16 heads of D 128, 4000 rows, 8 MB 13.5 -> 12.2, 8000, 33 MB 19.1 ->
+    // 19.5; 32 heads, 4000, 17 MB 19.2 -> 18.6, 8000, 65 MB 31.9 -> 33.4, 16000, 129 MB 58.8 -> 61.9; D 64, 16 heads, 16000, 32 MB 20.2 ->
+    // 19.3, 32 heads, 65 MB 32.9 -> 33.1), or what each of them does: up to 32 parts, half of its own rows (64 heads of D 128, 8000 rows
+    // 58.8 -> 59.4, 16000 109.7 -> 107.9, 32000 222.7 -> 217.2). Beyond 64 parts a launch of its own is ahead: 64 sums per head made by 64
+    // workgroups of 1024 threads, which the quantiser could add up as well, took 21.6 us against 21.2 at 32768 rows of 4 heads, 36.8 against
+    // 29.4 for 2 heads of 100000.
+    const uint64_t again = (uint64_t)n_kv_heads * ceil_div_u32(kv_len, FA_SAGE_BLOCK * (QUANT_NT / 64)) * n_parts * head_dim * sizeof(float);
+    const bool own_mean = n_parts <= MEAN_LANES / 2 || (n_parts <= MEAN_LANES && again <= (head_dim == 128 ? 24u : 48u) << 20);
     if (!own_mean) FA_TRY(launch_mean_finish(ctx, partial, n_parts, n_kv_heads, head_dim, kv_len, mean));
     return launch_quantize_k(ctx, k, mean, n_kv_heads, capacity, head_dim, 0, kv_len, k_q, k_scale, tail, own_mean ? partial : nullptr, n_parts);
 }

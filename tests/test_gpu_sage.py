@@ -221,7 +221,8 @@ def test_sage_decode_step_errors():
 
 @pytest.mark.parametrize("Hkv,D,n,cap", [
     (3, 128, 1, 1), (1, 128, 31, 40), (4, 128, 33, 64), (2, 64, 64, 64),                    # one part; open block of 1 .. 31 rows or none
-    (2, 128, 8191, 8300), (2, 128, 8192, 8192), (2, 128, 8193, 8200), (3, 64, 16385, 16400)])  # 64 parts and 65: the mean with the quantiser or before it
+    (2, 128, 8191, 8300), (2, 128, 8192, 8192), (2, 128, 8193, 8200), (3, 64, 16385, 16400),  # 64 parts and 65: the mean with the quantiser or before it
+    (16, 128, 7040, 7040), (16, 128, 7041, 7056), (32, 64, 14080, 14080), (32, 64, 14081, 14096)])  # fewer, but more of them than the quantiser reads again
 def test_sage_cache_build_is_its_separate_operations(Hkv, D, n, cap):
     """The mean, the int8 rows and the scales are those of fa_sage_k_mean and fa_sage_quantize_k bit for bit, the open block's rows
     are in the tail, and nothing else is written."""
@@ -236,7 +237,15 @@ def test_sage_cache_build_is_its_separate_operations(Hkv, D, n, cap):
     for name, m in marks.items():
         bufs[name].upload(m)
     dmean, dkq, dks = f.zeros((Hkv, D), np.float32), f.array(marks["k_q"]), f.array(marks["k_scale"])
+    f.profile_reset()
+    f.profile_enable(True)
     f.sage_cache_build(dk, n, desc)
+    f.synchronize()
+    f.profile_enable(False)
+    rows_per_part = 128 if D == 128 else 256
+    if n <= 64 * rows_per_part and Hkv <= 32:  # (then the parts are of one pass each)
+        again = Hkv * -(-n // 128) * -(-n // rows_per_part) * D * 4
+        assert f.profile_query("sage_k_mean_finish_kernel")[0] == int(again > (24 if D == 128 else 48) << 20)
     f.sage_k_mean(dk, Hkv, cap, D, n, dmean)
     f.sage_quantize_k(dk, dmean, Hkv, cap, D, 0, n, dkq, dks)
     f.synchronize()
