@@ -827,7 +827,8 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         for (int mb = 0; mb < MBX; ++mb) {
             if ((uint32_t)mb >= m) break;
             const uint32_t row0 = k0 + (blk + mb) * BK;
-            if (SAGE) ksr[mb] = reinterpret_cast<const _Float16 *>(a.k_scale)[(size_t)kvh * a.ks_stride + row0 / FA_SAGE_BLOCK];
+            // (a partition may end past the capacity: its rows there read as zero, and its scales are the last one)
+            if (SAGE) ksr[mb] = reinterpret_cast<const _Float16 *>(a.k_scale)[(size_t)kvh * a.ks_stride + min(row0 / FA_SAGE_BLOCK, a.ks_stride - 1u)];
             if (!PAGED) {
 #pragma unroll
                 for (int j = 0; j < KSTEPS; ++j)
