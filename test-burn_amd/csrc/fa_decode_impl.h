@@ -472,10 +472,15 @@ __device__ __forceinline__ bool coop_merge_of_group(const DecodeDev &a, uint32_t
             __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)off, 0, ST_POLICY);
             __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)off_ml, 0, ST_POLICY);
         }
-        // the group's maximum, then the weighted sums
+        // the group's maximum, then the weighted sums (the products rounded on their own: made one with the first step's sum, a lane would
+        // round its neighbour's product and not its own, and two lanes of a pair would have different sums)
         const float mstar = group_reduce<G, true>(m_r);
         const float w = fast_exp2(m_r - mstar);
-        float v[5] = {l_r * w, acc[0] * w, acc[1] * w, acc[2] * w, acc[3] * w};
+        float v[5];
+        {
+#pragma clang fp contract(off)
+            v[0] = l_r * w, v[1] = acc[0] * w, v[2] = acc[1] * w, v[3] = acc[2] * w, v[4] = acc[3] * w;
+        }
 #pragma unroll
         for (int e = 0; e < 5; ++e) v[e] = group_reduce<G, false>(v[e]);
         if (col < n4 && p == 0) {

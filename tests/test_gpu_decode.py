@@ -478,6 +478,34 @@ def test_polled_merge_of_every_number_of_partitions(H, Hkv, D):
         x.free()
 
 
+@pytest.mark.parametrize("H,Hkv,D,parts", [(16, 2, 128, 4), (16, 2, 128, 64), (32, 8, 128, 8), (14, 2, 64, 16)])
+def test_polled_merge_adds_a_pair_of_partitions_in_either_order(H, Hkv, D, parts):
+    """The merge in registers adds partitions p and p ^ 1, then those sums and their neighbours', and so on: with the keys of every
+    partition p and p ^ x exchanged it adds the same numbers in the other order, which is the same sum, bit for bit."""
+    announce("polled merge, partitions exchanged", H, Hkv, D, parts)
+    f = ctx()
+    rng = np.random.default_rng(parts + D)
+    kps, n = 64, 64 * parts
+    k, v = (h16(rng.normal(size=(Hkv, parts, kps, D))) for _ in range(2))
+    order = np.arange(parts)
+    caches = [[f.array(x[:, order ^ e].reshape(Hkv, n, D)) for x in (k, v)] for e in (0, 1, 2, parts - 1)]
+    dq, outs = f.zeros((1, H * D)), [f.zeros((1, H * D)) for _ in caches]
+    try:
+        f.set_decode_variant(kps, 2)
+        for trial in range(60):
+            dq.upload(h16(rng.normal(size=(1, H * D))))
+            for (dk, dv), do in zip(caches, outs):
+                f.flash_attention(dq.arg(), dk.arg(), dv.arg(), do.arg(), True, n - 1, H, D, n, 1)
+            f.synchronize()
+            got = [bits(do.download()) for do in outs]
+            for other in got[1:]:
+                assert np.array_equal(got[0], other), trial
+    finally:
+        f.set_decode_variant()
+    for b in [dq, *outs, *(x for c in caches for x in c)]:
+        b.free()
+
+
 def test_polled_merge_gives_up_cleanly():
     """Failure handling of the polled merge, forced from the host: with a wait bound of zero a merging workgroup gives
     up at its first look unless every record is already there. Every kernel still ends normally. The give-up is
