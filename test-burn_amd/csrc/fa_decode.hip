@@ -232,7 +232,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
     }
     if (polled) {
         a.merge_in_kernel = 2u;
-        a.xcd_local = !bal_slots && ctx->xcd_round_robin && groups % 8 == 0 ? 1u : 0u;
+        a.xcd_local = !bal_slots && ctx->xcd_round_robin && groups % 8 == 0 && S <= 64 ? 1u : 0u;  // (up to 64: merged in registers)
         // Fewer than 8 head groups (Qwen2.5-0.5B has 2 KV heads) and few enough partitions for an XCD to hold a group's
         // workgroups: the grid is padded to 8 head groups, group g's workgroups land on XCD g, and the workgroups of
         // the groups that do not exist leave at once. Such a launch is all latency (its partitions were sized for that
@@ -242,7 +242,7 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         // D128, 4000 8.86, 8.12), except with three groups and more of int8 rows (4000 keys 10.6, 10.8) or many records (H32 / Hkv4 /
         // D128, 2100 keys 9.61, 9.96).
         if (!a.xcd_local && ctx->xcd_round_robin && L.batch == 1 && groups < 8 && waves == 4) {  // (only the 4-wave kernels know of the padding)
-            const uint64_t per_xcd = (ny > 2 && (int8 || !one_pass) ? 2u : 1u) * (n_cus / 8u);
+            const uint64_t per_xcd = std::min<uint64_t>(64u, (ny > 2 && (int8 || !one_pass) ? 2u : 1u) * (n_cus / 8u));
             const size_t need_pad = (size_t)8 * S * n4 * 32;
             if (S <= per_xcd && (uint64_t)8 * S <= slots && need_pad <= ctx->poll_ws_bytes) ny_grid = 8, a.xcd_local = 1u, a.ny_real = ny;
         }

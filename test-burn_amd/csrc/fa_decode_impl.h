@@ -315,13 +315,9 @@ constexpr int POLL_IPT = 4;  // records per thread, at most
 __device__ __forceinline__ uint32_t not_sentinel(float v) {  // the pattern is a NaN, the largest word: a partial stores the next one, a NaN too
     return min(__float_as_uint(v), POLL_SENTINEL - 1u);
 }
-// LOCAL: every workgroup of the head group runs on the same XCD. Records are then written with plain stores (they go
-// through to that XCD's L2) and read with device-scope loads (which pass the compute unit's own cache and hit the L2):
-// a quarter of a microsecond from store to load instead of a trip to memory and back.
-template <int D, bool LOCAL>
+template <int D>
 __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_t b, uint32_t y, uint32_t c,
                                                      uint32_t nsplits, uint32_t S, int tid, float *sm) {
-    constexpr int LD_POLICY = LOCAL ? 0x10 /* sc1 */ : CACHE_COHERENT, ST_POLICY = LOCAL ? 0 : CACHE_COHERENT;
     constexpr int CG = D / 4;
     const uint32_t gt = a.gt, n4 = gt * CG;
     const uint32_t my_cols = n4 > c ? (n4 - c + nsplits - 1) / nsplits : 0u;
@@ -354,8 +350,8 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 #pragma unroll
         for (int j = 0; j < POLL_IPT; ++j) {
             if (pend >> j & 1u) {
-                x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(rec_of[j] * 16u), 0, LD_POLICY);
-                ml[j] = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)(ml_base + rec_of[j] * 8u), 0, LD_POLICY);
+                x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(rec_of[j] * 16u), 0, CACHE_COHERENT);
+                ml[j] = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)(ml_base + rec_of[j] * 8u), 0, CACHE_COHERENT);
             }
         }
 #pragma unroll
@@ -389,8 +385,8 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 #pragma unroll
         for (int j = 0; j < POLL_IPT; ++j) {
             if (mine >> j & 1u) {
-                __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)(rec_of[j] * 16u), 0, ST_POLICY);
-                __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)(ml_base + rec_of[j] * 8u), 0, ST_POLICY);
+                __builtin_amdgcn_raw_buffer_store_b128(sent4, rs, (int)(rec_of[j] * 16u), 0, CACHE_COHERENT);
+                __builtin_amdgcn_raw_buffer_store_b64(sent2, rs, (int)(ml_base + rec_of[j] * 8u), 0, CACHE_COHERENT);
             }
         }
     }
@@ -434,6 +430,9 @@ __device__ __forceinline__ bool coop_merge_and_store(const DecodeDev &a, uint32_
 // The same merge for up to 64 partitions, without LDS and without a barrier: a column's records are read by a group
 // of G consecutive lanes (G = the power of two that holds the partitions), one partition per lane, and the group
 // folds them with lane exchanges. A wave depends on no other wave.
+// LOCAL: every workgroup of the head group runs on the same XCD (which has room for no more than 64 of them). Records are then
+// written with plain stores (they go through to that XCD's L2) and read with device-scope loads (which pass the compute unit's own
+// cache and hit the L2): a quarter of a microsecond from store to load instead of a trip to memory and back.
 // What a wave runs through here and in the fold before it is a chain of some hundred instructions, several cycles each since a SIMD has
 // one or two waves: the code is written once for each G, without a branch for each step of the exchange, and the addresses of the other
 // forms of a launch are not on its way. With the steps behind branches and one fold for all forms, a step over 300 / 1024 keys at 2 K/V
@@ -1601,25 +1600,17 @@ __global__ void __launch_bounds__(NT, NW == 8 ? 1 : 2) flash_decode_mfma_kernel(
         if (FA_LIKELY(xcd_local)) {
             record(std::integral_constant<int, 0>{});
             FA_TR(9);
-            if (FA_LIKELY(nsplits <= 64)) {
-                ok = coop_merge_in_registers<D, true, BF16>(tl, b, y, split, nsplits, rs, tid);
-                goto merged;
-            }
+            ok = coop_merge_in_registers<D, true, BF16>(tl, b, y, split, nsplits, rs, tid);
         } else {
             record(std::integral_constant<int, CACHE_COHERENT>{});
             FA_TR(9);
             if (nsplits <= 64) {
                 ok = coop_merge_in_registers<D, false, BF16>(tl, b, y, split, nsplits, rs, tid);
-                goto merged;
+            } else {
+                __syncthreads();  // the fold above read the LDS region that the merge reuses
+                ok = coop_merge_and_store<D>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));
             }
         }
-        __syncthreads();  // the fold above read the LDS region that the merge reuses
-        if (xcd_local) {
-            ok = coop_merge_and_store<D, true>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));
-        } else {
-            ok = coop_merge_and_store<D, false>(tl, b, y, split, nsplits, S, tid, reinterpret_cast<float *>(smem));
-        }
-    merged:
         if (FA_UNLIKELY(!ok) && lane == 0 && tl.status) tl.status[FA_DEVSTAT_MERGE_TIMEOUT] = 1u;
         FA_TR(10);
         FA_TR_FLUSH();
