@@ -148,11 +148,15 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07; 17000 8.70 -> 7.67, 20000 8.69 -> 8.01, 25000 8.95 -> 8.89, but 30000 9.17 -> 9.38; int8
             //   20000 10.2 -> 9.1, 32768 10.7 -> 10.0
             // Four waves stay at 32 as long as that leaves no more than two blocks to each of the three that stream, 96 keys: half a wave
-            // merges a column then instead of a whole one. us, 64 keys -> this: H32 / Hkv4 / D128: 2500 8.22 -> 7.33, 3000 8.41 -> 6.99; H16 /
-            // Hkv2 / D128: 3000 7.82 -> 7.40 (int8 2500 11.4 -> 10.3); H12 / Hkv6 / D64: 3000 5.60 -> 5.07; 96 keys in 42 partitions: 4000 7.77 -> 8.14.
+            // merges a column then instead of a whole one. us, 64 keys -> this: H32 / Hkv4 / D128: 2560 8.20 -> 6.63, 3000 8.39 -> 7.03; H16 /
+            // Hkv4 / D128: 2560 6.97 -> 6.26, 3000 6.93 -> 6.71; H16 / Hkv2 / D128: 2560 7.61 -> 7.03, 3000 7.95 -> 7.36 (int8 10.4 -> 8.7); H12 /
+            // Hkv6 / D64: 3000 5.70 -> 5.04; H9 / Hkv3 / D64 0.98 to 1.03 times; 96 keys in 42 partitions: 4000 7.77 -> 8.14. Not for one or two
+            // head groups of f16 that fold in one pass: 32 partitions put each of them on one XCD (below), which their rows come into no faster than
+            // that, and more of them spread over all: H14 / Hkv2 / D64: 2560 5.47 -> 5.72, 3072 5.47 -> 5.77; H4 / Hkv1 / D64: 2560
+            // 5.14 -> 5.75; H4 / Hkv2 / D128: 3072 6.10 -> 6.85. (int8 rows are half as many bytes: H14 / Hkv2 / D64 7.5 -> 6.9.)
             const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK, by32 = ceil_div_u32(ceil_div_u32(bound, 32u), (uint32_t)BK) * BK;
             uint32_t least = 0;
-            if (waves == 4) least = !short_context ? 0u : by32 <= 6u * BK ? by32 : std::min(8u * BK, by64);
+            if (waves == 4) least = !short_context ? 0u : by32 <= 6u * BK && (ny > 2 || !one_pass || int8) ? by32 : std::min(8u * BK, by64);
             else if (by64 <= (int8 ? 32u : 20u) * BK) least = std::max(one_pass ? 0u : 12u * BK, by64);
             else if (!int8 || !one_pass) least = 16u * BK;
             chunk = std::max(chunk, least);
