@@ -244,9 +244,11 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
         // accesses (6.15 -> 5.4 us per launch at 1K context). A workgroup to a compute unit: with up to two, the XCDs of the groups
         // are what the launch waits for (H14 / Hkv2 / D64, 2100 keys, 33 partitions 6.74 padded, 6.19 not, 4000 keys 7.50, 6.68; H16 / Hkv4 /
         // D128, 4000 8.86, 8.12), except with three groups and more of int8 rows (4000 keys 10.6, 10.8) or many records (H32 / Hkv4 /
-        // D128, 2100 keys 9.61, 9.96).
+        // D128, 2100 keys 9.61, 9.96), and with int8 rows and many records whatever the groups (H16 / Hkv2 / D128 int8, 3200 / 3600 / 4000
+        // keys 10.04, 10.42 / 9.53, 9.82 / 9.80, 10.03; H16 / Hkv1 / D64 9.12, 9.40 / 8.59, 8.92 / 8.80, 8.92; of one and two
+        // groups with few records 0.96 to 1.02 times).
         if (!a.xcd_local && ctx->xcd_round_robin && L.batch == 1 && groups < 8 && waves == 4) {  // (only the 4-wave kernels know of the padding)
-            const uint64_t per_xcd = std::min<uint64_t>(64u, (ny > 2 && (int8 || !one_pass) ? 2u : 1u) * (n_cus / 8u));
+            const uint64_t per_xcd = std::min<uint64_t>(64u, ((int8 ? ny > 2 || !one_pass : ny > 2 && !one_pass) ? 2u : 1u) * (n_cus / 8u));
             const size_t need_pad = (size_t)8 * S * n4 * 32;
             if (S <= per_xcd && (uint64_t)8 * S <= slots && need_pad <= ctx->poll_ws_bytes) ny_grid = 8, a.xcd_local = 1u, a.ny_real = ny;
         }
