@@ -261,11 +261,11 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                 wv[r] += w_step[r];
             } else {
                 const uint32_t soff = S::CANON ? w_soff + (w_block[r] ? w_block_bytes : 0u) : w_soff;
-                fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
+                fa_lds_dma::buffer_to_lds_b128_scalar<1, 0, 0>(w_now, base + S::X_BYTES + q * 1024, wv[r], __builtin_amdgcn_readfirstlane((int)soff));
             }
         } else {
             if constexpr (S::JOINED) fa_lds_dma::buffer_to_lds_b128_ahead(x_now, x_lds, stage + (r - S::WR) * 1024, xv[r - S::WR], (int)x_soff);
-            else fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(x_now, S::X_EVEN ? base + (loader * S::XR + r - S::WR) * 1024 : base + (loader * S::XR + r - S::WR) % S::X_REQ * 1024, xv[r - S::WR], (int)x_soff);
+            else fa_lds_dma::buffer_to_lds_b128_scalar<1, 0, 0>(x_now, S::X_EVEN ? base + (loader * S::XR + r - S::WR) * 1024 : base + (loader * S::XR + r - S::WR) % S::X_REQ * 1024, xv[r - S::WR], (int)x_soff);
         }
         if (r == S::REQ - 1) {  // the step's last one
             ++asked, x_soff += STRIDE * 128, w_soff += STRIDE * w_per_step;
@@ -440,7 +440,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         for (uint32_t q = wave; q < requests; q += S::NW) {
             constexpr uint32_t PER = S::NTR % 64 == 0 ? S::NTR / 64 : 1;  // requests per 16 bytes of all rows, where that is whole ones
             const uint32_t at = S::NTR % 64 == 0 ? q % PER * 64 + lane : q * 64 + lane, unit = S::NTR % 64 == 0 ? 0u : at / S::NTR;
-            fa_lds_dma::buffer_to_lds_b128<1, 0, 0>(s_rs, lds_base - own + S::ALL_STAGES + q * 1024, (int)(weight_row(at % S::NTR) * (K / 32) * 2 + unit * 16),
+            fa_lds_dma::buffer_to_lds_b128_scalar<1, 0, 0>(s_rs, lds_base - own + S::ALL_STAGES + q * 1024, (int)(weight_row(at % S::NTR) * (K / 32) * 2 + unit * 16),
                                                     (int)(S::NTR % 64 == 0 ? q / PER * 16 : 0u));
         }
     }
