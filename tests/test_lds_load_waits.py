@@ -14,8 +14,8 @@ STATES = 5
 
 def scalars(operand):
     """Numbers of the scalar registers that an operand names."""
-    if operand == "vcc":
-        return {106, 107}
+    if operand.startswith("vcc"):
+        return {"vcc": {106, 107}, "vcc_lo": {106}, "vcc_hi": {107}}[operand]
     m = re.fullmatch(r"s\[(\d+):(\d+)\]|s(\d+)", operand)
     if not m:
         return set()
