@@ -128,7 +128,13 @@ __device__ __forceinline__ void meet() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-template <class S, int MIN_WAVES>
+// What the write stage does: alpha * sum + bias + beta * residual; KvPrepFused's, pairs in a piece (or no rotation) and half a head apart.
+// ANY: a kernel has all three and the launch says which. A tile with stages of its own has a kernel for each: 33 KB of code, of which a
+// launch runs through the loop and one part far from it, became 19 to 23 KB that it runs through in a row (Q4_0, FusedQkv + KvPrepFused of
+// 400 rows x 2560 x 2048 19.1 -> 18.5 us, o_proj of 400 rows x 3072 x 3072 15.8 -> 15.4, 700 rows x 2048 x 2048 13.3 -> 13.0; the other tiles
+// within 1 %).
+enum Form { PLAIN, ADJACENT, APART, ANY };
+template <class S, int MIN_WAVES, Form FORM>
 __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -161,7 +167,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 
     // Matrix and weight row of tile row t. With the NeoX rotation as the write stage, 32 tile rows are 16 rows of a head and the 16
     // that they are rotated with, half a head further on, so that a tile of any width holds both of a pair.
-    const bool pairs = a.rope.on && a.rope.apply && !a.rope.normal;
+    const bool pairs = FORM == ANY ? a.rope.on && a.rope.apply && !a.rope.normal : FORM == APART;
     const uint32_t hd_shift = a.rope.head_dim == 128 ? 7u : 6u;
     auto paired = [&](uint32_t r) -> uint32_t {
         if (!pairs) return r;
@@ -397,9 +403,9 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         return *(const GemmDev *)g;
     };
     // The write stage's code is there once for each of what it does, so that none of it runs through the others' branches.
-    enum { PLAIN, ADJACENT, APART };  // alpha * sum + bias + beta * residual; KvPrepFused's, pairs in a piece (or no rotation) and half a head apart
     auto by_what = [&](const GemmDev &g, auto &&f) __attribute__((always_inline)) {
-        if (!g.rope.on) f(std::integral_constant<int, PLAIN>{});
+        if constexpr (FORM != ANY) f(std::integral_constant<int, FORM>{});
+        else if (!g.rope.on) f(std::integral_constant<int, PLAIN>{});
         else if (!pairs) f(std::integral_constant<int, ADJACENT>{});
         else f(std::integral_constant<int, APART>{});
     };
@@ -656,20 +662,31 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     });
 }
 
-template <class S, int MIN_WAVES>
-fa_status launch_shape(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
+template <class S, int MIN_WAVES, Form FORM>
+fa_status launch_form(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
     static std::atomic<bool> lds_allowed_on[64];  // per device (contexts of several threads may get here together: the calls are idempotent)
     std::atomic<bool> &lds_allowed = lds_allowed_on[ctx->device & 63];
     if (!lds_allowed.load(std::memory_order_acquire)) {
-        FA_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<S, MIN_WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        FA_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<S, MIN_WAVES, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         lds_allowed.store(true, std::memory_order_release);
     }
     a.n_tiles = 0, a.m_tiles = ceil_div_u32(a.m, S::MT);
     for (int i = 0; i < 3; ++i) a.tiles[i] = ceil_div_u32(a.rows[i], S::NTR), a.n_tiles += a.tiles[i];
     if (S::JOINED) a.n_tiles = ceil_div_u32(a.rows[0] + 2 * a.rows[1], S::NTR);
     const uint32_t grid = ceil_div_u32(a.n_tiles * a.m_tiles, 8) * 8;
-    scope.launch((tile_gemm_kernel<S, MIN_WAVES>), dim3(grid), dim3(S::NT), S::lds_bytes(a.k_dim), a);
+    scope.launch((tile_gemm_kernel<S, MIN_WAVES, FORM>), dim3(grid), dim3(S::NT), S::lds_bytes(a.k_dim), a);
     return FA_OK;
+}
+
+template <class S, int MIN_WAVES>
+fa_status launch_shape(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
+    if constexpr (S::OWN) {
+        if (!a.rope.on) return launch_form<S, MIN_WAVES, PLAIN>(ctx, scope, a);
+        if (a.rope.apply && !a.rope.normal) return launch_form<S, MIN_WAVES, APART>(ctx, scope, a);
+        return launch_form<S, MIN_WAVES, ADJACENT>(ctx, scope, a);
+    } else {
+        return launch_form<S, MIN_WAVES, ANY>(ctx, scope, a);
+    }
 }
 
 template <int WB, bool CANON>
