@@ -122,12 +122,12 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             short_context = ceil_div_u32(bound, s_max) <= 4u * BK;
             // One sequence: up to 128 keys to a unit's share (one round of a workgroup's three streaming waves) where the four waves
             // fold and merge their heads in one pass, up to 64 where they do not, and only as far as 64 partitions of 128 keys go, the
-            // most that are merged in registers. us, eight waves or 64 keys -> this (the last two lines: more partitions, or eight waves):
-            //   H24 / Hkv8 / D128: 2100 keys 7.60 -> 6.51, 3000 7.78 -> 6.92, 4000 8.09 -> 7.75; H32 / Hkv32 / D128: 600 7.83 -> 6.64
-            //   H16 / Hkv4 / D128: 5000 9.35 -> 8.66, 8000 10.27 -> 9.85 (int8 10.1 -> 10.3: not for its four groups)
-            //   H14 / Hkv2 / D64: 5000 7.39 -> 6.66, 8000 7.72 -> 7.08; four waves beyond: 8300 6.90, 7.45, 10000 7.27, 7.60 (int8 8.8, 9.9)
-            //   H16 / Hkv2 / D128, two passes: 6200 9.17 -> 8.65, 7000 9.28 -> 8.73, 8100 9.33 -> 8.61 (int8 6200
-            //   11.7 -> 11.9: not there)
+            // most that are merged in registers. us, the better of eight waves and 64 keys -> this:
+            //   H24 / Hkv8 / D128: 2100 keys 6.41 -> 5.78, 3000 6.83 -> 6.24, 4000 7.07 -> 7.03; H32 / Hkv32 / D128: 600 6.36 -> 5.67
+            //   H16 / Hkv4 / D128: 5000 8.64 -> 7.47, 8000 9.32 -> 8.73 (int8 9.1 -> 9.9: not for its four groups)
+            //   H14 / Hkv2 / D64: 5000 6.89 -> 5.91, 8000 7.04 -> 6.48; eight and four waves beyond: 8300 7.12, 7.35, 10000 7.26, 7.46 (int8 7.4, 7.5)
+            //   H16 / Hkv2 / D128, two passes: 6200 9.25 -> 8.65, 7000 9.35 -> 8.59, 8100 9.26 -> 8.49 (int8 6200
+            //   10.2 -> 10.9: not there)
             if (one && one_pass && (!int8 || s_max > 64)) short_context = ceil_div_u32(bound, std::min(s_max, 64u)) <= 8u * BK;
             else if (one && !one_pass) short_context = short_context && bound <= (int8 ? 96u * 4u * BK : 64u * 8u * BK);
             // A batch: eight waves where four fold in two passes. (H16 / Hkv2 / D128: 2 sequences of 125-1000 tokens 8.85 -> 8.25 us, of
@@ -142,11 +142,12 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             // One sequence of few head groups has units for more partitions than are worth their records. Up to 64 partitions are merged
             // in registers, more of them through LDS: they stay at 64 as long as that leaves four waves 128 keys, eight waves 320 (of int8
             // keys 512), beyond which eight waves have 256 and int8 keys that fold in one pass as many as the units; eight waves that
-            // fold in two passes have 192 at least. us, by the units -> by this rule (the second number of a pair: 256 keys):
-            //   H16 / Hkv2 / D128: 8000 keys 11.36 -> 10.31, 12000 11.75 -> 10.87, 16000 12.78 -> 11.30; 17000 11.46 -> 10.82, 20000
-            //   11.82 -> 11.59, but 25000 12.42 -> 13.03; int8 20000 12.9 -> 11.8, 32768 14.1 -> 13.8
-            //   H14 / Hkv2 / D64: 12000 8.71 -> 8.07; 17000 8.70 -> 7.67, 20000 8.69 -> 8.01, 25000 8.95 -> 8.89, but 30000 9.17 -> 9.38; int8
-            //   20000 10.2 -> 9.1, 32768 10.7 -> 10.0
+            // fold in two passes have 192 at least. us, by the units -> by this rule:
+            //   H16 / Hkv2 / D128: 9000 keys 10.74 -> 9.18, 12000 11.11 -> 9.50, 16000 11.96 -> 10.23, 17000 11.56 -> 10.63, 20000 11.68 -> 11.39; 256
+            //   keys: 25000 12.28 -> 12.16, 30000 12.89 -> 12.78 (64 partitions of 400 at 25000: 0.6 more); int8 20000 12.1 -> 10.7, 24000 12.5 ->
+            //   11.5, from there to 32768 by what the units' number is rounded to: 26000 12.0 -> 12.4, 28000 12.7 -> 12.4, 30000 12.3 -> 12.7
+            //   H14 / Hkv2 / D64: 9000 8.07 -> 7.13, 12000 8.12 -> 7.55, 17000 8.52 -> 7.53, 20000 8.69 -> 7.80; 256 keys: 25000 9.06 -> 8.80, 30000 9.05 ->
+            //   8.99; int8 20000 8.9 -> 7.7, 32768 9.0 -> 8.9
             // Four waves stay at 32 as long as that leaves no more than two blocks to each of the three that stream, 96 keys: half a wave
             // merges a column then instead of a whole one. us, 64 keys -> this: H32 / Hkv4 / D128: 2560 8.20 -> 6.63, 3000 8.39 -> 7.03; H16 /
             // Hkv4 / D128: 2560 6.97 -> 6.26, 3000 6.93 -> 6.71; H16 / Hkv2 / D128: 2560 7.61 -> 7.03, 3000 7.95 -> 7.36 (int8 10.4 -> 8.7); H12 /
@@ -155,8 +156,21 @@ fa_status fa_launch_decode(fa_ctx *ctx, const DecodeLaunch &L) {
             // that, and more of them spread over all: H14 / Hkv2 / D64: 2560 5.47 -> 5.72, 3072 5.47 -> 5.77; H4 / Hkv1 / D64: 2560
             // 5.14 -> 5.75; H4 / Hkv2 / D128: 3072 6.10 -> 6.85. (int8 rows are half as many bytes: H14 / Hkv2 / D64 7.5 -> 6.9.)
             const uint32_t by64 = ceil_div_u32(ceil_div_u32(bound, 64u), (uint32_t)BK) * BK, by32 = ceil_div_u32(ceil_div_u32(bound, 32u), (uint32_t)BK) * BK;
+            // Where the device has the length, or a second launch merges (a step that allocates nothing), the bound is mostly above it, and up to half
+            // of it the units that 64 partitions leave idle are missed where a key is 512 bytes and the fold takes two passes: 192 keys from
+            // 273 (257) on. us, by the units with records as they were (a partition's columns side by side), by 64 partitions, this; lengths of a
+            // sixteenth, a quarter, half and all of the bound:
+            //   H16 / Hkv2 / D128, bound 18432: 9.06 10.07 10.56 12.06, 9.64 10.21 10.42 10.76, 8.56 9.33 9.32 11.14
+            //     20480: 9.28 10.19 10.60 12.22, 9.94 10.58 10.81 11.18, 8.84 9.53 9.69 11.65; allocating nothing 9.85 10.19 10.83 12.26, 11.17
+            //     11.42 11.65 12.34, 9.71 9.99 10.70 12.15;  17408, 272 keys: 9.01 9.87 10.23 11.75, 9.31 9.90 10.12 10.51 (192 keys 11.22)
+            //   H8 / Hkv1 / D128, bound 20480: 8.97 9.60 10.70 11.40, 9.60 10.16 10.31 10.60, 8.29 8.93 9.15 10.68
+            // Elsewhere 64 partitions are ahead at every length, or lose less at short ones than they gain (H16 / Hkv2 / D128, bound 16384: by the
+            // units as they were 9.50 10.26 10.78 12.30, 8.79 9.28 9.67 10.04; 8192, allocating nothing: 7.95 8.32 8.88 10.25, 8.29 8.53 8.75 9.48; of one head
+            // group, H8 / Hkv1 / D128, 16384: 8.11 8.68 9.62 11.28, 8.44 8.89 9.07 9.50).
+            const bool beyond = !int8 && !one_pass && L.head_dim > 64 && (L.d_len || L.static_scratch);
             uint32_t least = 0;
             if (waves == 4) least = !short_context ? 0u : by32 <= 6u * BK && (ny > 2 || !one_pass || int8) ? by32 : std::min(8u * BK, by64);
+            else if (beyond && by64 > (L.static_scratch ? 16u : 17u) * BK && by64 <= 20u * BK) least = 12u * BK;
             else if (by64 <= (int8 ? 32u : 20u) * BK) least = std::max(one_pass ? 0u : 12u * BK, by64);
             else if (!int8 || !one_pass) least = 16u * BK;
             chunk = std::max(chunk, least);

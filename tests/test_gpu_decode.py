@@ -344,6 +344,50 @@ def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
         b.free()
 
 
+@pytest.mark.parametrize("H,Hkv,D,bounds", [
+    (16, 2, 128, (8192, 8193, 16384, 16385, 17408, 17409, 20480, 20481)), (8, 1, 128, (17408, 17409)), (16, 1, 64, (17409, 20480)), (14, 2, 64, (8192, 17409))])
+def test_one_sequence_of_less_than_its_bound(H, Hkv, D, bounds):
+    """A step whose length the device has is divided by its bound: recorded once and replayed at growing lengths below it, and the form
+    that allocates nothing, which merges in a second launch, against f64 attention either side of the lines that hold for them."""
+    announce("one sequence, less than its bound", H, Hkv, D, bounds)
+    f = ctx()
+    rng = np.random.default_rng(3 * H + D)
+    cap = max(bounds)
+    kc, vc = (h16(rng.normal(size=(Hkv, cap, D))) for _ in range(2))
+    cos, sin = fa.rope_tables(1e6, D, cap)
+    dk, dv, dcos, dsin, dpos = f.array(kc), f.array(vc), f.array(cos), f.array(sin), f.array(np.zeros(1, np.uint32))
+    q = h16(rng.normal(size=(1, H * D)))
+    dq, dkn, dvn, outs = f.array(q), f.zeros((1, Hkv * D)), f.zeros((1, Hkv * D)), [f.zeros((1, H * D)) for _ in range(2)]
+    # (nothing is rotated: layer 3 of a model that leaves out every 4th)
+    p = fa.KvPrepFusedParams.make(H, Hkv, D, 1, 0, cap, fa.ROPE_NEOX, layer_idx=3, no_rope_layer_step=4)
+    for bound in bounds:
+        def steps():
+            for noalloc, do in enumerate(outs):
+                f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p, dpos, bound,
+                                    noalloc=bool(noalloc))
+        lengths = (1, 193, bound // 4 + 1, bound // 2, bound)
+        dkn.upload(kc[:, 0].reshape(1, -1)), dvn.upload(vc[:, 0].reshape(1, -1))
+        steps()
+        f.synchronize()
+        f.start_capture()
+        steps()
+        graph = f.end_capture()
+        for n in lengths:
+            dpos.upload(np.array([n - 1], np.uint32))
+            dkn.upload(kc[:, n - 1].reshape(1, -1)), dvn.upload(vc[:, n - 1].reshape(1, -1))
+            graph.launch()
+            f.synchronize()
+            s = np.einsum("kgd,knd->kgn", q.reshape(Hkv, H // Hkv, D).astype(np.float64), kc[:, :n].astype(np.float64)) / np.sqrt(D)
+            w = np.exp(s - s.max(axis=-1, keepdims=True))
+            want = np.matmul(w / w.sum(axis=-1, keepdims=True), vc[:, :n].astype(np.float64)).reshape(H, D)
+            for do in outs:
+                assert max_abs(do.download().reshape(H, D), want) <= TOL, (bound, n)
+        graph.destroy()
+        dpos.upload(np.zeros(1, np.uint32))
+    for b in (dk, dv, dcos, dsin, dpos, dq, dkn, dvn, *outs):
+        b.free()
+
+
 def test_fused_step_errors_and_overflow_guard():
     announce("fused step errors")
     f = ctx()
