@@ -395,7 +395,9 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         }
     }
     // The launch's arguments, read where the write stage begins and not kept from the entry on, for tiles whose loop has no scalar
-    // registers to spare. (The smaller tiles would wait for them there: 0.1 us of 6.6.)
+    // registers to spare. (The smaller tiles would wait for them there: 0.1 us of 6.6.) For speed only: kept in lanes of a vector register,
+    // as a few of the smaller tiles' are, they are read back as they were written. Built that way the largest tiles pass the same tests,
+    // and no lane of any kernel is found to be read before or after its time (tests/test_spilled_scalars.py looks at the built code).
     static_assert(std::is_trivially_copyable<GemmDev>::value, "read as raw bytes from the argument block, where it is the first member");
     auto arguments = []() __attribute__((always_inline)) -> const GemmDev & {
         auto g = __builtin_amdgcn_kernarg_segment_ptr();
