@@ -124,3 +124,33 @@ def test_prefill_bf16_vs_oracle(D, H, Hkv, M, prefix):
     assert max_abs(got, want) <= TOL_BF16
     for b in (dq, dk, dv, do):
         b.free()
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(16, 2, 128), (14, 2, 64), (32, 4, 128)])
+def test_polled_merge_of_every_number_of_partitions_bf16(H, Hkv, D):
+    """The merge inside the launch has a form of its own for bf16 outputs, for each power of two that holds the partitions and one above:
+    either side of each power, against f64 attention and, to one bf16 unit in the last place, against the two-launch merge."""
+    announce("polled merge, partitions, bf16", H, Hkv, D)
+    f = ctx()
+    rng = np.random.default_rng(7 * H + D)
+    counts, kps = (2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65), 64
+    cap = kps * max(counts)
+    q, k, v = (orc.bf16_pack(rng.normal(size=s)) for s in ((H, D), (Hkv, cap, D), (Hkv, cap, D)))
+    dq, dk, dv = up(f, q), up(f, k), up(f, v)
+    outs = {m: f.zeros((1, H * D)) for m in (1, 2)}
+    try:
+        for parts in counts:
+            n = kps * (parts - 1) + 1 + parts % kps
+            for merge, do in outs.items():
+                f.set_decode_variant(kps, merge)
+                f.flash_attention(dq.arg((1, H * D), dtype=BF), dk.arg(dtype=BF), dv.arg(dtype=BF), do.arg(dtype=BF), True, n - 1, H, D, n, 1)
+            f.synchronize()
+            a, b = (orc.bf16_unpack(outs[m].download()).astype(np.float64).reshape(H, D) for m in (1, 2))
+            want = rm.gqa_decode_f64(orc.bf16_unpack(q), orc.bf16_unpack(k), orc.bf16_unpack(v), H, Hkv, D, n)
+            assert max_abs(b, want) <= TOL_BF16, parts
+            # adjacent bf16 values are 2^-7 of themselves apart at most
+            assert np.all(np.abs(a - b) <= np.maximum(np.abs(a), 2.0 ** -14) * 2.0 ** -7), parts
+    finally:
+        f.set_decode_variant()
+    for x in (dq, dk, dv, *outs.values()):
+        x.free()

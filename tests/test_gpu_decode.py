@@ -324,18 +324,20 @@ def test_one_sequence_where_its_partitions_change(H, Hkv, D, lengths):
         dpos, outs = f.array(np.array([n - 1], np.uint32)), []
         desc, bufs = fa.sage_cache(f, H, Hkv, cap, D, dv)
         f.sage_cache_build(dk, n - 1, desc)
-        for merge in (2, 1):
-            f.set_decode_variant(merge=merge)
-            do, do8 = f.zeros((1, H * D)), f.zeros((1, H * D))
-            if merge == 2:  # a length that the host has, and one that the device has
-                f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p)
-            else:
-                f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p, dpos, n)
-            f.sage_decode_step(dq.arg(), dkn.arg(), dvn.arg(), desc, dcos.arg(), dsin.arg(), do8.arg(), p, d_position=dpos, kv_len_bound=n)
-            f.synchronize()
-            outs.append([x.download().reshape(H, D) for x in (do, do8)])
-            do.free(), do8.free()
-        f.set_decode_variant()
+        try:
+            for merge in (2, 1):
+                f.set_decode_variant(merge=merge)
+                do, do8 = f.zeros((1, H * D)), f.zeros((1, H * D))
+                if merge == 2:  # a length that the host has, and one that the device has
+                    f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p)
+                else:
+                    f.decode_step_fused(dq.arg(), dkn.arg(), dvn.arg(), None, dk.arg(), dv.arg(), dcos.arg(), dsin.arg(), do.arg(), p, dpos, n)
+                f.sage_decode_step(dq.arg(), dkn.arg(), dvn.arg(), desc, dcos.arg(), dsin.arg(), do8.arg(), p, d_position=dpos, kv_len_bound=n)
+                f.synchronize()
+                outs.append([x.download().reshape(H, D) for x in (do, do8)])
+                do.free(), do8.free()
+        finally:
+            f.set_decode_variant()
         assert max_abs(outs[0][0], want) <= TOL, n
         assert max_abs(outs[0][0], outs[1][0]) <= TOL and max_abs(outs[0][1], outs[1][1]) <= TOL, n
         for b in (dq, dkn, dvn, dpos, *(b for k, b in bufs.items() if k != "v")):
