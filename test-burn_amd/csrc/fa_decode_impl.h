@@ -111,13 +111,15 @@ __device__ __forceinline__ void store_out4(__half *op, const float (&o)[4], bool
 }
 
 
-// Lane exchanges, as few instructions as they go. A launch of a few microseconds runs through the code after its loop once, and each wave
-// waits for every line of it to be fetched: 1.4 KB less of it (selects between the two results of a swap, and moves ahead of DPP
-// operations, both for nothing) took a step over 1024 keys from 8.06 to 7.50 us at 2 K/V heads of 128 and from 5.62 to 5.32 at 2 of 64,
-// one over 8192 at 8 of 128 from 9.87 to 9.53, 16 int8 steps over 32768 from 237.5 to 233.3.
+// Lane exchanges. A launch of a few microseconds runs through the code after its loop once, and each wave waits for every line of it to
+// be fetched: 1.4 KB less of it (selects between the two results of a swap; `old` values and bounds of DPP moves that have none) took a
+// step over 1024 keys from 8.06 to 7.50 us at 2 K/V heads of 128 and from 5.62 to 5.32 at 2 of 64, one over 8192 at 8 of 128 from 9.87 to 9.53, 16
+// int8 steps over 32768 from 237.5 to 233.3.
 // `both`: op of a lane's value and that of lane l ^ 16 / l ^ 32, one VALU swap of lane groups whose two results are the operands in
-// either order (op commutes). Inside a row of 16 lanes the exchange is part of the operation (DPP: every lane has its source, so the
-// bound control is free to be what lets the compiler fold the move).
+// either order (op commutes). Inside a row of 16 lanes the exchange is a DPP move, every lane of which has its source (so the bound control
+// is free). In a step of a sum the compiler makes it part of the addition, one instruction. In a step of a maximum it does not: it makes the
+// moved value canonical first (fmaxf, of what might be a signalling NaN for all it knows), so that such a step is a move, two maxima and
+// the wait between them, and three maxima behind a swap.
 struct OpMax {
     __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); }
 };
