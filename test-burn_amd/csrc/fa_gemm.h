@@ -31,32 +31,51 @@ struct GemmDev {
     uint32_t page_shift;  // log2 of rope.block_size, 32 = not a power of two
 };
 
-// Rotation of the piece hd .. hd + 7 of a head: the first table column that it takes, the columns (adjacent pairs (hd + 2i, hd + 2i + 1):
-// 4 of them, from hd / 2; pairs (hd, hd + D / 2): 8, from hd mod D / 2), and the piece rotated with them.
-__device__ __forceinline__ uint32_t rope_column(const RopeDev &r, uint32_t hd) { return r.normal ? hd >> 1 : hd & ((r.head_dim >> 1) - 1u); }
-__device__ __forceinline__ void rope_columns(const RopeDev &r, uint32_t table_row, uint32_t column, h8_t &c, h8_t &s) {
-    typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
-    const size_t at = (size_t)table_row * (r.head_dim >> 1) + column;
-    if (r.normal) {
-        const h4v_t c4 = fa_norm::load_global<h4v_t>(r.cos_t + at), s4 = fa_norm::load_global<h4v_t>(r.sin_t + at);
-        c = __builtin_shufflevector(c4, c4, 0, 1, 2, 3, 0, 1, 2, 3), s = __builtin_shufflevector(s4, s4, 0, 1, 2, 3, 0, 1, 2, 3);
-    } else {
-        c = fa_norm::load_global<h8_t>(r.cos_t + at), s = fa_norm::load_global<h8_t>(r.sin_t + at);
-    }
+typedef _Float16 h4v_t __attribute__((ext_vector_type(4)));
+
+// x * c - mate * s (`first`), or x * c + mate * s, of f16 values: the products are exact in f32, so one rounded sum of an exact product and
+// another is what rope_one gives, in two instructions that take the f16 halves as they lie in the registers.
+template <int X, int M, int C>
+__device__ __forceinline__ float rope_mix(uint32_t x, uint32_t mate, uint32_t c, uint32_t s, bool first) {
+    const float neg_zero = -0.0f;  // (a sum with -0 keeps the sign of a zero product)
+    float t;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[%4,%5,0] op_sel_hi:[1,1,0]" : "=v"(t) : "v"(mate), "v"(s), "v"(neg_zero), "n"(M), "n"(C));
+    if (first) asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[%4,%5,0] op_sel_hi:[1,1,0]" : "=v"(t) : "v"(x), "v"(c), "v"(t), "n"(X), "n"(C));
+    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[%4,%5,0] op_sel_hi:[1,1,0]" : "=v"(t) : "v"(x), "v"(c), "v"(t), "n"(X), "n"(C));
+    return t;
 }
-__device__ __forceinline__ h8_t rope_piece(const RopeDev &r, h8_t y, h8_t mate, h8_t c, h8_t s, bool first) {
+typedef uint32_t rope_u4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t rope_u2_t __attribute__((ext_vector_type(2)));
+// Rotation of a piece of 8 dims whose pairs are (2i, 2i + 1): 4 table columns
+__device__ __forceinline__ h8_t rope_adjacent(h8_t y, h4v_t c4, h4v_t s4) {
+    const rope_u4_t y2 = __builtin_bit_cast(rope_u4_t, y);
+    const rope_u2_t c = __builtin_bit_cast(rope_u2_t, c4), s = __builtin_bit_cast(rope_u2_t, s4);
     h8_t o;
-    if (r.normal) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[2 * i] = (_Float16)rope_one((float)y[2 * i], (float)y[2 * i + 1], (float)c[i], (float)s[i], true);
-            o[2 * i + 1] = (_Float16)rope_one((float)y[2 * i + 1], (float)y[2 * i], (float)c[i], (float)s[i], false);
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (_Float16)rope_one((float)y[e], (float)mate[e], (float)c[e], (float)s[e], first);
+    for (int i = 0; i < 2; ++i) {
+        o[4 * i] = (_Float16)rope_mix<0, 1, 0>(y2[2 * i], y2[2 * i], c[i], s[i], true), o[4 * i + 1] = (_Float16)rope_mix<1, 0, 0>(y2[2 * i], y2[2 * i], c[i], s[i], false);
+        o[4 * i + 2] = (_Float16)rope_mix<0, 1, 1>(y2[2 * i + 1], y2[2 * i + 1], c[i], s[i], true), o[4 * i + 3] = (_Float16)rope_mix<1, 0, 1>(y2[2 * i + 1], y2[2 * i + 1], c[i], s[i], false);
     }
     return o;
+}
+// ... whose pairs are half a head apart, `mate` the piece there: 8 columns; `first`: the piece is of the first half
+__device__ __forceinline__ h8_t rope_apart(h8_t y, h8_t mate, h8_t c8, h8_t s8, bool first) {
+    const rope_u4_t x = __builtin_bit_cast(rope_u4_t, y), m = __builtin_bit_cast(rope_u4_t, mate), c = __builtin_bit_cast(rope_u4_t, c8);
+    rope_u4_t s = __builtin_bit_cast(rope_u4_t, s8);
+    h8_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t sgn = first ? s[i] ^ 0x80008000u : s[i];
+        o[2 * i] = (_Float16)rope_mix<0, 0, 0>(x[i], m[i], c[i], sgn, false), o[2 * i + 1] = (_Float16)rope_mix<1, 1, 1>(x[i], m[i], c[i], sgn, false);
+    }
+    return o;
+}
+// Rotation of the piece hd .. hd + 7 of a head from the tables' row
+__device__ __forceinline__ h8_t rope_piece(const RopeDev &r, uint32_t table_row, uint32_t hd, h8_t y, h8_t mate) {
+    const uint32_t half = r.head_dim >> 1, column = r.normal ? hd >> 1 : hd & (half - 1u);
+    const size_t at = (size_t)table_row * half + column;
+    if (r.normal) return rope_adjacent(y, fa_norm::load_global<h4v_t>(r.cos_t + at), fa_norm::load_global<h4v_t>(r.sin_t + at));
+    return rope_apart(y, mate, fa_norm::load_global<h8_t>(r.cos_t + at), fa_norm::load_global<h8_t>(r.sin_t + at), hd < half);
 }
 
 // Write stage of one piece: y = the projections of token gm, columns gn .. gn + 7 of matrix mat (0 Q, 1 K, 2 V),
@@ -64,7 +83,7 @@ __device__ __forceinline__ h8_t rope_piece(const RopeDev &r, h8_t y, h8_t mate, 
 // Q goes to q_rot[h][gm][hd], K (rotated) and V (as is) to cache row position_offset + gm of KV head h.
 __device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint32_t gm, uint32_t gn, h8_t y, const h8_t mate) {
     const RopeDev &r = a.rope;
-    const uint32_t D = r.head_dim, half = D >> 1, h = gn / D, hd = gn - h * D;
+    const uint32_t D = r.head_dim, h = gn / D, hd = gn - h * D;
     const uint32_t pos = r.position_offset + gm;
     __half *dst;
     if (mat == 0) {
@@ -82,9 +101,7 @@ __device__ __forceinline__ void rope_store_piece(const GemmDev &a, int mat, uint
     }
     if (mat != 2 && r.apply) {
         const uint32_t tp = pos < r.table_rows ? pos : r.table_rows - 1;  // stay inside the tables
-        h8_t c, s;
-        rope_columns(r, tp, rope_column(r, hd), c, s);
-        y = rope_piece(r, y, mate, c, s, hd < half);
+        y = rope_piece(r, tp, hd, y, mate);
     }
     *reinterpret_cast<h8_t *>(dst) = y;
 }

@@ -131,8 +131,9 @@ __device__ __forceinline__ void meet() {
 // What the write stage does: alpha * sum + bias + beta * residual; KvPrepFused's, pairs in a piece (or no rotation) and half a head apart.
 // ANY: a kernel has all three and the launch says which. A tile with stages of its own has a kernel for each: 33 KB of code, of which a
 // launch runs through the loop and one part far from it, became 19 to 23 KB that it runs through in a row (Q4_0, FusedQkv + KvPrepFused of
-// 400 rows x 2560 x 2048 19.1 -> 18.5 us, o_proj of 400 rows x 3072 x 3072 15.8 -> 15.4, 700 rows x 2048 x 2048 13.3 -> 13.0; the other tiles
-// within 1 %).
+// 400 rows x 2560 x 2048 19.1 -> 18.5 us, o_proj of 400 rows x 3072 x 3072 15.8 -> 15.4, 700 rows x 2048 x 2048 13.3 -> 13.0), and so have the
+// block-quantised tiles of eight stages, whose loops have no scalar registers left (o_proj of 128 rows x 3072 x 3072 Q8_0 11.4 -> 10.8, Q4_0 11.0 -> 10.8)
+// and 256 x 160 (0.5 %; the other tiles within 1 %).
 enum Form { PLAIN, ADJACENT, APART, ANY };
 template <class S, int MIN_WAVES, Form FORM>
 __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) {
@@ -366,20 +367,24 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     constexpr int NCOL = PIECES / std::gcd(S::NT, PIECES), BATCH = EARLY ? PER_TURN * TURNS : PER_TURN > 5 ? PER_TURN / 2 : PER_TURN, BATCHES = EARLY ? 1 : PER_TURN / BATCH;
     static_assert(TURN_PIECES % S::NT == 0 || PER_TURN == 1, "the threads share the pieces evenly, or some have none");
     static_assert(EARLY ? PER_TURN % NCOL == 0 : PER_TURN % BATCH == 0 && BATCH % NCOL == 0, "piece i of a batch has column i % NCOL");
-    struct Beside {
-        h8_t c, s;  // columns of the RoPE tables, or c = the residual
-        uint32_t page;
-    };
-    Beside beside[BATCH];
+    // Piece i of a column is STEP rows of LDS below the one before, and ROW_STEP input rows.
+    constexpr int STEP = NCOL * S::NT / PIECES, ROW_STEP = S::TJ == S::TM ? STEP : STEP * S::TM;
+    static_assert(S::TJ == S::TM || (S::TJ == 1 && STEP % 32 == 0) || PER_TURN <= NCOL, "the rows of a column are evenly apart");
+    h8_t early[EARLY ? BATCH : 1];  // the residual
     struct Column {
         int mat;
         uint32_t gn;           // row of its matrix
+        uint32_t at, mate_at;  // its first piece in LDS (mate_at: the one that it is rotated with)
+        uint32_t row;          // ... and the input row of that one
         bool in;               // there is such a column
         h8_t bias, mate_bias;  // (mate_bias: of the half of a head that the piece is rotated with)
     } column[NCOL];
     // Piece i of a turn: its row in LDS, and which input row that is.
-    auto lds_row = [&](int thread, int i) __attribute__((always_inline)) -> uint32_t { return (uint32_t)(thread + i * S::NT) / PIECES; };
-    auto input_row = [&](uint32_t t, int turn) __attribute__((always_inline)) -> uint32_t { return m0 + ((t >> 5) / S::TJ * S::TM + turn * S::TJ + (t >> 5) % S::TJ) * 32 + (t & 31); };
+    auto lds_row = [&](int thread, int i) __attribute__((always_inline)) -> uint32_t {
+        const uint32_t t = (uint32_t)(thread + i * S::NT) / PIECES;
+        return TURN_PIECES % S::NT == 0 ? t : min(t, (uint32_t)(S::WM * S::TJ * 32) - 1);
+    };
+    auto input_row = [&](uint32_t t) __attribute__((always_inline)) -> uint32_t { return m0 + ((t >> 5) / S::TJ * S::TM + (t >> 5) % S::TJ) * 32 + (t & 31); };
     // The residual, asked for ahead of everything else where the tile leaves registers for it: at the end of the one chain that a
     // launch of a round of such tiles is, it would be a trip to memory more (3072 x 3072, 320 rows: F16 12.8 -> 12.3 us, Q8_0 12.2 ->
     // 11.7, Q4_0 12.0 -> 11.6; 896 x 896, 500 rows: 6.3 -> 6.0, 6.8 -> 6.5, 6.7 -> 6.5). The rest is asked for behind the loop: ahead of it
@@ -389,8 +394,8 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
         if (a.residual) {
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) {
-                const uint32_t gm = input_row(lds_row(tid, i % PER_TURN), i / PER_TURN), r = n0 + (uint32_t)(tid + i % PER_TURN * S::NT) % PIECES * 8;
-                beside[i].c = fa_norm::load_global<h8_t>(a.residual + (gm < a.m && r < N_tile ? (size_t)gm * N_tile + r : 0));
+                const uint32_t gm = input_row(lds_row(tid, i % PER_TURN)) + i / PER_TURN * (S::TJ * 32), r = n0 + (uint32_t)(tid + i % PER_TURN * S::NT) % PIECES * 8;
+                early[i] = fa_norm::load_global<h8_t>(a.residual + (gm < a.m && r < N_tile ? (size_t)gm * N_tile + r : 0));
             }
         }
     }
@@ -416,28 +421,16 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
 #pragma unroll
         for (int i = 0; i < NCOL; ++i) {
             Column &col = column[i];
-            const uint32_t at = n0 + (uint32_t)(thread + i * S::NT) % PIECES * 8, end = S::JOINED ? rows0 + 2 * rows1 : N_tile;
+            const uint32_t n8 = (uint32_t)(thread + i * S::NT) % PIECES, t = lds_row(thread, i);
+            const uint32_t at = n0 + n8 * 8, end = S::JOINED ? rows0 + 2 * rows1 : N_tile;
             uint32_t r = min(at, end - 8);
             col.in = at < end && (TURN_PIECES % S::NT == 0 || thread < TURN_PIECES);
             col.mat = matrix_of(r), col.gn = W == APART ? paired(r) : r;
+            col.row = input_row(t), col.at = t * S::T_STRIDE + n8 * 32, col.mate_at = t * S::T_STRIDE + (n8 ^ 2) * 32;
             if (g.bias[0]) {  // (all matrices have one, or none has)
                 const __half *const bias = pick3(col.mat, g.bias[0], g.bias[1], g.bias[2]);
                 col.bias = fa_norm::load_global<h8_t>(bias + col.gn);
                 if constexpr (W == APART) col.mate_bias = fa_norm::load_global<h8_t>(bias + paired(r ^ 16));
-            }
-        }
-    };
-    auto ask = [&](auto what, const GemmDev &g, Beside &w, const Column &col, uint32_t row) __attribute__((always_inline)) {
-        constexpr int W = decltype(what)::value;
-        const uint32_t gm = min(row, g.m - 1);
-        if constexpr (W == PLAIN) {
-            if (!EARLY && g.residual) w.c = fa_norm::load_global<h8_t>(g.residual + (size_t)gm * N_tile + col.gn);
-        } else {
-            const uint32_t pos = g.rope.position_offset + gm;
-            if (W == APART || g.rope.apply) rope_columns(g.rope, min(pos, g.rope.table_rows - 1), rope_column(g.rope, col.gn & (g.rope.head_dim - 1)), w.c, w.s);
-            if (g.rope.block_table) {
-                const uint32_t cache_row = min(pos, g.rope.capacity - 1);
-                w.page = fa_norm::load_global<uint32_t>(g.rope.block_table + (g.page_shift < 32 ? cache_row >> g.page_shift : cache_row / g.rope.block_size));
             }
         }
     };
@@ -540,9 +533,29 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     struct Target {
         __half *first;  // (of a paged cache: of row 0 of page 0, 64 bits, as everything in a pool: one page of all heads may be 8 GiB)
         uint32_t stride, end;
-        bool paged;
+        bool paged, turn;
+        const __half *cos_t, *sin_t;  // the tables at its first column
     };
     Target target[NCOL];
+    // What a piece takes from memory. (Nothing is done with it where it is asked for, and there is no branch around it - a table that is
+    // not wanted is read at its first row, or the input in its place -: what waits for one piece's, ahead of the next piece's request, is
+    // a trip to memory per piece. With the columns of both pairings behind a branch, and copied out of it, the write stage of FusedQkv +
+    // KvPrepFused, 2048 rows of 5120 x 3072, took 16 us where that of the projections alone takes 6; with the rotation's products and sums
+    // from the f16 halves (rope_mix) and the rows of a column a constant apart it takes 8. With the norm, before -> now: F16 2048 rows of 5120 x
+    // 3072 76.0 -> 69.1 us, 1200 rows 50.0 -> 47.8, Q4_0 2048 rows 94.2 -> 87.7, Q8_0 1000 rows 49.2 -> 46.0, 500 rows 31.1 -> 29.6, 500 rows of
+    // 1152 x 896 10.8 -> 10.7; o_proj of 1500 rows x 2048 x 2048 Q8_0 19.3 -> 18.5, F16 17.3 -> 17.2.)
+    struct Side {
+        h8_t c, s;     // columns of the RoPE tables, half a head apart; c = the residual
+        h4v_t c4, s4;  // ... of pairs in a piece
+        uint32_t page;
+    };
+    // (the kernel's arguments as far as every piece needs them)
+    const uint32_t m_all = g.m, pos0 = g.rope.position_offset, last_entry = g.rope.table_rows - 1, last_row = g.rope.capacity - 1;
+    const uint32_t half_dim = g.rope.on && g.rope.apply ? g.rope.head_dim >> 1 : 0u, page_size = g.rope.block_size, page_shift = g.page_shift;
+    const float alpha = g.alpha, beta = g.beta;
+    const int32_t *const table = g.rope.block_table;
+    const __half *const residual = g.residual;
+    const bool has_bias = g.bias[0] != nullptr;
     auto find_targets = [&](auto what) __attribute__((always_inline)) {
         constexpr int W = decltype(what)::value;
 #pragma unroll
@@ -550,25 +563,44 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             const Column &col = column[i];
             Target &o = target[i];
             o.first = pick3(col.mat, g.out[0], g.out[1], g.out[2]);
-            o.end = col.in ? g.m : 0u, o.paged = false;
+            o.end = col.in ? m_all : 0u, o.paged = false, o.turn = false;
             if constexpr (W == PLAIN) {
                 o.stride = S::JOINED ? (col.mat ? rows1 : rows0) : N_tile;
                 o.first += col.gn;
             } else {
-                const uint32_t D = g.rope.head_dim, head = col.gn >> hd_shift, hd = col.gn & (D - 1), room = g.rope.capacity > g.rope.position_offset ? g.rope.capacity - g.rope.position_offset : 0u;
+                const uint32_t D = g.rope.head_dim, head = col.gn >> hd_shift, hd = col.gn & (D - 1), room = g.rope.capacity > pos0 ? g.rope.capacity - pos0 : 0u;
+                const uint32_t first_column = W == APART ? hd & ((D >> 1) - 1) : hd >> 1;
                 o.stride = D;
-                o.paged = col.mat != 0 && g.rope.block_table;
+                o.paged = col.mat != 0 && table, o.turn = col.mat != 2 && (W == APART || half_dim != 0);
                 if (col.mat != 0) o.end = min(o.end, room);  // never outside the cache
-                o.first += (col.mat == 0 ? (size_t)head * g.m : o.paged ? (size_t)head * g.rope.block_size : (size_t)head * g.rope.max_seq_len + g.rope.position_offset) * D + hd;
+                o.first += (col.mat == 0 ? (size_t)head * m_all : o.paged ? (size_t)head * page_size : (size_t)head * g.rope.max_seq_len + pos0) * D + hd;
+                o.cos_t = half_dim ? g.rope.cos_t + first_column : reinterpret_cast<const __half *>(g.x);
+                o.sin_t = half_dim ? g.rope.sin_t + first_column : reinterpret_cast<const __half *>(g.x);
             }
         }
     };
-    auto write = [&](auto what, int i, const Beside &w, int first, int turn) __attribute__((always_inline)) {  // piece first + i of the turn
+    auto ask = [&](auto what, Side &w, int i, uint32_t row) __attribute__((always_inline)) {  // (of column i)
         constexpr int W = decltype(what)::value;
-        const Column &col = column[i % NCOL];
-        const Target &o = target[i % NCOL];
-        const uint32_t q = (uint32_t)(tid_w + (first + i) * S::NT), t = TURN_PIECES % S::NT == 0 ? q / PIECES : min(q / PIECES, (uint32_t)(S::WM * S::TJ * 32) - 1);
-        const uint32_t gm = input_row(t, turn), n8 = q % PIECES, at = t * S::T_STRIDE;
+        const uint32_t gm = min(row, m_all - 1);
+        const Target &o = target[i];
+        if constexpr (W == PLAIN) {
+            if (!EARLY && residual) w.c = fa_norm::load_global<h8_t>(residual + (size_t)gm * N_tile + column[i].gn);
+        } else {
+            const uint32_t pos = pos0 + gm;
+            const size_t at = (size_t)min(pos, last_entry) * half_dim;
+            if constexpr (W == APART) w.c = fa_norm::load_global<h8_t>(o.cos_t + at), w.s = fa_norm::load_global<h8_t>(o.sin_t + at);
+            else w.c4 = fa_norm::load_global<h4v_t>(o.cos_t + at), w.s4 = fa_norm::load_global<h4v_t>(o.sin_t + at);
+            if (table) {
+                const uint32_t cache_row = min(pos, last_row);
+                w.page = fa_norm::load_global<uint32_t>(table + (page_shift < 32 ? cache_row >> page_shift : cache_row / page_size));
+            }
+        }
+    };
+    auto write = [&](auto what, int i, const Side &w, uint32_t down, uint32_t row) __attribute__((always_inline)) {  // column i, `down` bytes of LDS below its first piece
+        constexpr int W = decltype(what)::value;
+        const Column &col = column[i];
+        const Target &o = target[i];
+        const uint32_t gm = row;
         auto value = [&](uint32_t place, h8_t bias) __attribute__((always_inline)) -> h8_t {
             f4v_t s0 = *reinterpret_cast<const f4v_t *>(smem + place);
             f4v_t s1 = *reinterpret_cast<const f4v_t *>(smem + place + 16);
@@ -581,31 +613,31 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
             {   // (every step rounded to f32, whatever follows: a product and a sum made into one with the rounding to f16 gives other bits)
 #pragma clang fp contract(off)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = (e < 4 ? s0[e & 3] : s1[e & 3]) * g.alpha;
-                if (g.bias[0]) {
+                for (int e = 0; e < 8; ++e) v[e] = (e < 4 ? s0[e & 3] : s1[e & 3]) * alpha;
+                if (has_bias) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] += (float)bias[e];
                 }
             }
-            if (W == PLAIN && g.residual) {
+            if (W == PLAIN && residual) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = fmaf(g.beta, (float)w.c[e], v[e]);
+                for (int e = 0; e < 8; ++e) v[e] = fmaf(beta, (float)w.c[e], v[e]);
             }
             h8_t y;
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[e] = (_Float16)v[e];
             return y;
         };
-        h8_t y = value(at + n8 * 32, col.bias);
+        h8_t y = value(col.at + down, col.bias);
         __half *dst = o.first + (size_t)gm * o.stride;
         if constexpr (W != PLAIN) {
-            if (W == APART || g.rope.apply) {
-                const h8_t turned = rope_piece(g.rope, y, W == APART ? value(at + (n8 ^ 2) * 32, col.mate_bias) : y, w.c, w.s, (col.gn & (g.rope.head_dim - 1)) < (g.rope.head_dim >> 1));
-                y = col.mat != 2 ? turned : y;
-            }
-            if (g.rope.block_table) {
-                const uint32_t pos = g.rope.position_offset + gm, in_page = g.page_shift < 32 ? pos & (g.rope.block_size - 1) : pos % g.rope.block_size;
-                __half *const there = o.first + ((size_t)w.page * g.rope.n_kv_heads * g.rope.block_size + in_page) * g.rope.head_dim;
+            h8_t turned;
+            if constexpr (W == APART) turned = rope_apart(y, value(col.mate_at + down, col.mate_bias), w.c, w.s, (col.gn & (g.rope.head_dim - 1)) < half_dim);
+            else turned = rope_adjacent(y, w.c4, w.s4);
+            y = o.turn ? turned : y;
+            if (table) {
+                const uint32_t pos = pos0 + gm, in_page = page_shift < 32 ? pos & (page_size - 1) : pos % page_size;
+                __half *const there = o.first + ((size_t)w.page * g.rope.n_kv_heads * page_size + in_page) * g.rope.head_dim;
                 dst = o.paged ? there : dst;
             }
         }
@@ -624,26 +656,41 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     };
     by_what(g, [&](auto what) __attribute__((always_inline)) {
         ask_columns(what, g, tid_w);
+        find_targets(what);
         if constexpr (EARLY) {
+            Side side[BATCH];
 #pragma unroll
-            for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, i % PER_TURN), i / PER_TURN));
-            find_targets(what);
+            for (int i = 0; i < BATCH; ++i) {
+                if (decltype(what)::value == PLAIN) side[i].c = early[i];
+                ask(what, side[i], i % NCOL, column[i % NCOL].row + i % PER_TURN / NCOL * ROW_STEP + i / PER_TURN * (S::TJ * 32));
+            }
 #pragma unroll
             for (int turn = 0; turn < TURNS; ++turn) {
                 __syncthreads();  // every wave is done with the stages / the previous rows have been read out
                 to_lds(turn * S::TJ);
                 __syncthreads();
 #pragma unroll
-                for (int i = 0; i < PER_TURN; ++i) write(what, i, beside[turn * PER_TURN + i], 0, turn);
+                for (int i = 0; i < PER_TURN; ++i)
+                    write(what, i % NCOL, side[turn * PER_TURN + i], i / NCOL * (STEP * S::T_STRIDE), column[i % NCOL].row + i / NCOL * ROW_STEP + turn * (S::TJ * 32));
             }
         } else {
             // (One copy of the code for all turns and batches, the accumulators moving up by a turn: run once it comes from memory,
-            // and the instructions of 20 pieces are more than the stores take.)
-            find_targets(what);
+            // and the instructions of 20 pieces are more than the stores take. What a batch takes from memory is asked for ahead of
+            // the one before it.)
+            constexpr int PER_COLUMN = BATCH / NCOL;  // pieces of a column in a batch
+            Side now[BATCH], next[BATCH];
+            auto ask_batch = [&](Side(&side)[BATCH], uint32_t rows) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i) ask(what, side[i], i % NCOL, column[i % NCOL].row + i / NCOL * ROW_STEP + rows);
+            };
+            if (BATCHES > 1) ask_batch(now, 0);
 #pragma unroll 1
             for (int turn = 0; turn < TURNS; ++turn) {
-#pragma unroll
-                for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, i), turn));
+                auto after = [&](int n) __attribute__((always_inline)) -> uint32_t {  // rows of the batch behind batch n (past the last: nobody takes them)
+                    return n + 1 < BATCHES ? (n + 1) * (PER_COLUMN * ROW_STEP) + turn * (S::TJ * 32) : (turn + 1) * (S::TJ * 32);
+                };
+                if (BATCHES > 1) ask_batch(next, after(0));
+                else ask_batch(now, turn * (S::TJ * 32));
                 __syncthreads();
                 to_lds(0);
 #pragma unroll
@@ -652,12 +699,16 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
                     for (int i = 0; i < S::TN; ++i) acc[0][i][j] = acc[0][i][j + S::TJ];
                 __syncthreads();
 #pragma unroll 1
-                for (int n = 0;; ++n) {
+                for (int n = 0; n < BATCHES; ++n) {
+                    const uint32_t rows = n * (PER_COLUMN * ROW_STEP) + turn * (S::TJ * 32);
+                    if (n > 0) ask_batch(next, after(n));
 #pragma unroll
-                    for (int i = 0; i < BATCH; ++i) write(what, i, beside[i], n * BATCH, turn);
-                    if (n + 1 == BATCHES) break;
+                    for (int i = 0; i < BATCH; ++i)
+                        write(what, i % NCOL, now[i], (uint32_t)(n * PER_COLUMN + i / NCOL) * (STEP * S::T_STRIDE), column[i % NCOL].row + i / NCOL * ROW_STEP + rows);
+                    if (BATCHES > 1) {
 #pragma unroll
-                    for (int i = 0; i < BATCH; ++i) ask(what, g, beside[i], column[i % NCOL], input_row(lds_row(tid_w, (n + 1) * BATCH + i), turn));
+                        for (int i = 0; i < BATCH; ++i) now[i] = next[i];
+                    }
                 }
             }
         }
@@ -682,7 +733,7 @@ fa_status launch_form(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
 
 template <class S, int MIN_WAVES>
 fa_status launch_shape(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
-    if constexpr (S::OWN) {
+    if constexpr (S::OWN || (S::QUANT && S::NS == 8) || S::JOINED) {
         if (!a.rope.on) return launch_form<S, MIN_WAVES, PLAIN>(ctx, scope, a);
         if (a.rope.apply && !a.rope.normal) return launch_form<S, MIN_WAVES, APART>(ctx, scope, a);
         return launch_form<S, MIN_WAVES, ADJACENT>(ctx, scope, a);

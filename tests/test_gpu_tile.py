@@ -451,3 +451,36 @@ def test_write_stage_into_pages(K, H, Hkv, D, m, bs, layer, weights):
             pg.free()
         for b in dev + db + outs + dqr + [dx, dg, dcos, dsin]:
             b.free()
+
+
+@pytest.mark.parametrize("mode", [fa.ROPE_NORMAL, fa.ROPE_NEOX])
+@pytest.mark.parametrize("H,Hkv,D,m", [(3, 1, 64, 77), (24, 8, 128, 2040)])  # a tile whose pieces are all asked for ahead, and 256 x 160
+def test_rotation_of_the_smallest_and_largest_values(H, Hkv, D, m, mode):
+    """KvPrepFused as a tile's write stage against the two ops where the projections are zeros of both signs, denormals, the largest
+    values and infinities, and so are the tables: the same bits, a NaN wherever there is one."""
+    announce("tiles, rotation of extreme values", H, Hkv, D, m, mode)
+    f = ctx()
+    rng = np.random.default_rng(H + m)
+    K, N, NK = 64, H * D, Hkv * D
+    values = np.array([0.0, -0.0, 6e-8, -6e-8, 1e-5, -1e-5, 0.333, -1.7, 300.0, 65504.0, -65504.0], np.float16)
+    x = np.zeros((m, K), np.float16)  # one feature per row: the projections are that value times a weight
+    x[np.arange(m), rng.integers(0, K, m)] = rng.choice(np.array([1.0, -1.0, 2.0, 0.25], np.float16), m)
+    ws = [rng.choice(values, (n, K)) for n in (N, NK, NK)]
+    cos, sin = (rng.choice(np.array([0.0, -0.0, 1.0, -1.0, 6e-8, 0.7, -1e-5], np.float16), (m + 3, D // 2)) for _ in range(2))
+    dev, dx, dcos, dsin = [f.array(orc.to_canonical(w)) for w in ws], f.array(x), f.array(cos), f.array(sin)
+    outs, dqr = [f.zeros((m, n)) for n in (N, NK, NK)], [f.zeros((H, m, D)) for _ in range(2)]
+    kc, vc = ([f.zeros((Hkv, m + 3, D)) for _ in range(2)] for _ in range(2))
+    try:
+        f.set_gemm_min_m(12)
+        p = fa.KvPrepFusedParams.make(H, Hkv, D, m, 3, m + 3, mode)
+        f.fused_qkv(dx.arg(), *[w.arg() for w in dev], *[o.arg() for o in outs], K, N, NK, m)
+        f.kv_prep_fused(*[o.arg() for o in outs], dqr[0].arg(), kc[0].arg(), vc[0].arg(), dcos.arg(), dsin.arg(), p)
+        f.fused_qkv_kv_prep(dx.arg(), *[w.arg() for w in dev], K, dqr[1].arg(), dcos.arg(), dsin.arg(), p, k_cache=kc[1].arg(), v_cache=vc[1].arg())
+        for one, two in (dqr, kc, vc):
+            one, two = one.download(), two.download()
+            assert np.array_equal(np.isnan(one), np.isnan(two))
+            assert np.array_equal(bits(one)[~np.isnan(one)], bits(two)[~np.isnan(two)])
+    finally:
+        f.set_gemm_min_m()
+        for b in dev + outs + dqr + kc + vc + [dx, dcos, dsin]:
+            b.free()
