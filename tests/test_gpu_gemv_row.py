@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("K,N,NK", [
     (32, 8, 8),          # one block, one group per matrix
     (160, 40, 24),       # a workgroup's groups across the three matrices
+    (672, 24, 8),        # six waves (block-quantised three): the sums of those that a workgroup has not
+    (896, 16, 8),        # seven (four)
     (1056, 1544, 8),     # F16: one block past what eight waves of one unit hold; two groups per workgroup
     (2080, 4104, 16),    # the quantised forms: the same; three groups per workgroup, the last one partly filled
     (4096, 520, 520),    # F16: the longest row; the quantised forms: two units
