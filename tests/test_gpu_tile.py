@@ -107,6 +107,28 @@ def test_residual_asked_for_ahead_of_the_sums(K, N, m, weights):
     assert np.all(np.abs(got - want) <= 2 * np.maximum(np.abs(want), 2.0 ** -10) * 2.0 ** -10 + 1e-4)  # (as test_tiles)
 
 
+@pytest.mark.parametrize("row_tiles", [1, 8, 9, 11, 33])  # weight tiles of all input tiles in a row, and in fours, the last ones of one to four
+@pytest.mark.parametrize("col_tiles", [1, 2, 3, 4, 5, 6, 7])
+def test_every_output_tile_once(row_tiles, col_tiles):
+    """64 x 64 tiles (64 features: a launch of one step) of whole numbers, whose sums f16 holds: exact, in every tile of the launch."""
+    announce("every tile", row_tiles, col_tiles)
+    f = ctx()
+    K, m, N = 64, 64 * row_tiles - 3, 64 * col_tiles - 8
+    rng = np.random.default_rng(row_tiles * 8 + col_tiles)
+    x, w = rng.integers(-3, 4, (m, K)).astype(np.float16), rng.integers(-3, 4, (N, K)).astype(np.float16)
+    dx, dw, dout = f.array(x), f.array(w), f.array(np.full((m, N), np.nan, np.float16))
+    try:
+        f.set_gemm_min_m(12)
+        f.set_gemm_variant(3)
+        f.matmul(dx.arg(), dw.arg(), dout.arg(), m, N, K, transpose_b=True)
+    finally:
+        f.set_gemm_variant()
+        f.set_gemm_min_m()
+    assert np.array_equal(dout.download(), (x.astype(np.float32) @ w.astype(np.float32).T).astype(np.float16))
+    for b in (dx, dw, dout):
+        b.free()
+
+
 @pytest.mark.parametrize("weights", ["q8", "q4"])
 @pytest.mark.parametrize("K,H,Hkv,D,m,layout", [
     (960, 2, 1, 64, 65, 1),       # the last length whose steps the waves of a tile share
