@@ -22,7 +22,7 @@ struct GemmDev {
     const __half *x;        // [m, k_dim] (already normalised when the op has a gamma)
     const __half *residual; // nullable, [m, rows[0]]
     uint32_t k_dim, m, m_tiles, n_tiles, canonical, vec_store;
-    uint32_t panel_inv;     // (2^32 - 1) / (input tiles x weight tiles that are gone through together)
+    uint32_t panel_inv;     // fa_inverse(input tiles x weight tiles that are gone through together)
     float alpha, beta;
     // the feature steps are divided over k_splits workgroups per output tile, which store f32 partial tiles
     // [split][m][n_total]; gemm_finish_kernel adds them up in split order and applies the write stage

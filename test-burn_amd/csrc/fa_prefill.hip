@@ -67,6 +67,7 @@ struct PrefillDev {
     uint32_t part_rows;          // rows per (head, query tile, split) in the partial buffers: BM, or 32 pack_nb when heads are packed
     float *part_acc, *part_ml;   // [head][query tile][split][part_rows][D] unnormalised sums, [..][part_rows][2] (max, sum)
     float scale_log2e;
+    uint32_t inv_head_splits, inv_splits, inv_group, inv_blocks;  // fa_inverse of n_heads * splits, splits, group_size and pack_blocks
     uint32_t out_aligned16;         // output base and strides are multiples of 16 bytes: rows leave as whole 16-byte pieces
     unsigned long long *clock_out;  // nullable: per workgroup {shader-clock ticks, 100 MHz wall ticks} from start to end
 };
@@ -471,7 +472,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
                  "s"(a.kv_len), "s"(a.query_offset), "s"(a.causal), "s"(a.block_size), "s"(a.block_shift), "s"(a.n_kv_heads));
     asm volatile("" ::"s"(a.splits), "s"(a.n_qt), "s"(a.n_items), "s"(a.n_workgroups), "s"(a.pool_bytes32), "s"(a.pack_heads),
                  "s"(a.pack_nb), "s"(a.pack_blocks), "s"(a.part_rows), "s"(a.part_acc), "s"(a.part_ml), "s"(a.scale_log2e),
-                 "s"(a.out_aligned16), "s"(a.clock_out));
+                 "s"(a.out_aligned16), "s"(a.clock_out), "s"(a.inv_head_splits), "s"(a.inv_splits), "s"(a.inv_group), "s"(a.inv_blocks));
     constexpr int DSTEPS = D / 16, DBLKS = D / 32, ROWB = D * 2, CHK = D / 8;
     constexpr int K_TILE = BN * ROWB, V_TILE = BN * ROWB, GRP_LDS = 2 * K_TILE + 2 * V_TILE;
     constexpr int RB_BYTES = CHK * 256;  // one 16-row block of a K tile
@@ -506,34 +507,41 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     struct WaveRows {
         uint32_t head, row0, ok;
     };
-    auto wave_rows = [&](uint32_t item, uint32_t w) __attribute__((always_inline)) -> WaveRows {
-        WaveRows r;
+    struct Place {
+        uint32_t q_tile, head, split, kvh, pair0;  // (packed heads: the first of the KV group and of the item's pairs)
+    };
+    // (Quotients by products, and once for an item: eight divisions stood between a workgroup's entry and its first request. 500 rows after
+    // 500, H24 / Hkv8 / D128 14.07 -> 13.97 us; 256 rows 6.35 -> 6.29; 200 after 4000, H14 / Hkv2 / D64 12.4 -> 12.3.)
+    auto place_of = [&](uint32_t item) __attribute__((always_inline)) -> Place {
+        Place p;
         if (a.pack_heads) {
             // pair p of the KV group = (head p % G, rows 32 (p / G) ..); this item holds pairs 4 (item's index) .. + 3
-            const uint32_t hb = item / S, kv = hb / a.pack_blocks, pr = (hb - kv * a.pack_blocks) * 4 + w;
-            const uint32_t rb = pr / a.group_size, h_in = pr - rb * a.group_size;
-            r.ok = rb < a.pack_nb ? 1u : 0u;
-            r.head = kv * a.group_size + (r.ok ? h_in : 0u), r.row0 = r.ok ? rb * 32 : 0u;
+            const uint32_t hb = fa_quotient(item, S, a.inv_splits);
+            p.q_tile = 0, p.split = item - hb * S, p.kvh = fa_quotient(hb, a.pack_blocks, a.inv_blocks);
+            p.head = p.kvh * a.group_size, p.pair0 = (hb - p.kvh * a.pack_blocks) * 4;
         } else {
-            const uint32_t qi = item / (a.n_heads * S);
-            r.head = (item - qi * (a.n_heads * S)) / S, r.row0 = (n_qt - 1 - qi) * BM + 32 * w, r.ok = 1u;
+            const uint32_t qi = fa_quotient(item, a.n_heads * S, a.inv_head_splits), rest = item - qi * (a.n_heads * S);
+            p.q_tile = n_qt - 1 - qi, p.head = fa_quotient(rest, S, a.inv_splits), p.split = rest - p.head * S;
+            p.kvh = fa_quotient(p.head, a.group_size, a.inv_group), p.pair0 = 0;
+        }
+        return p;
+    };
+    auto wave_rows = [&](const Place &p, uint32_t w) __attribute__((always_inline)) -> WaveRows {
+        WaveRows r;
+        if (a.pack_heads) {
+            const uint32_t pr = p.pair0 + w, rb = fa_quotient(pr, a.group_size, a.inv_group), h_in = pr - rb * a.group_size;
+            r.ok = rb < a.pack_nb ? 1u : 0u;
+            r.head = p.head + (r.ok ? h_in : 0u), r.row0 = r.ok ? rb * 32 : 0u;
+        } else {
+            r.head = p.head, r.row0 = p.q_tile * BM + 32 * w, r.ok = 1u;
         }
         return r;
     };
-    auto enter_item = [&](uint32_t item) {
-        if (a.pack_heads) {
-            const uint32_t hb = item / S;
-            q_tile = 0, split = item - hb * S, kvh = hb / a.pack_blocks;
-            head = kvh * a.group_size;
-        } else {
-            const uint32_t qi = item / (a.n_heads * S), rest = item - qi * (a.n_heads * S);
-            q_tile = n_qt - 1 - qi, head = rest / S, split = rest - head * S;
-            kvh = head / a.group_size;
-        }
+    auto enter_item = [&](const Place &p) {
         // (uniform values that come out of a branch and end up in the scalar operands of the DMA instructions)
-        kvh = (uint32_t)__builtin_amdgcn_readfirstlane((int)kvh), head = (uint32_t)__builtin_amdgcn_readfirstlane((int)head);
-        split = (uint32_t)__builtin_amdgcn_readfirstlane((int)split), q_tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)q_tile);
-        w_row0 = wave_rows(item, (uint32_t)wave).row0;
+        kvh = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.kvh), head = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.head);
+        split = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.split), q_tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.q_tile);
+        w_row0 = wave_rows(p, (uint32_t)wave).row0;
         q0 = q_tile * BM;
         kv_end = a.kv_len;
         if (a.causal) {
@@ -541,7 +549,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             kv_end = (uint32_t)min((uint64_t)a.kv_len, last);
         }
         const int all_tiles = (int)((kv_end + BN - 1) / BN);
-        const int per_split = (all_tiles + (int)S - 1) / (int)S;
+        const int per_split = (int)fa_quotient((uint32_t)all_tiles + S - 1, S, a.inv_splits);
         const int t_lo = min(all_tiles, (int)split * per_split);
         const int n_tiles = min(all_tiles, t_lo + per_split);
         t0 = t_lo + grp;                                  // group g attends tiles t0, t0 + 2, ...
@@ -601,12 +609,12 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
     // picks its operand pieces out of them. (Loading the pieces straight from memory, 16 bytes from each of 64 places
     // per instruction, cost every workgroup 2.6 us.)
     const size_t q_bytes = ((size_t)(a.q_len - 1) * a.q_stride_m + D) * 2;
-    auto q_dma = [&](uint32_t item) {
+    auto q_dma = [&](const Place &p) {
         int ql = lane;
         asm volatile("" : "+v"(ql));  // the lane's source offset is worked out here, not kept in a register across the loop
         const int q_lane_src = rows16_lane_src(ql, (int)(a.q_stride_m * 2));
         // the 16 rows this wave moves are half of the 32 rows of wave (wave8 / 2) of either group
-        const WaveRows wr = wave_rows(item, (uint32_t)wave8 >> 1);
+        const WaveRows wr = wave_rows(p, (uint32_t)wave8 >> 1);
         const uint32_t row0 = wr.row0 + 16 * ((uint32_t)wave8 & 1);
         const rsrc_words qrs = make_rsrc_words(a.q + (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)wr.head) * a.q_stride_h, (uint32_t)q_bytes * (uint32_t)__builtin_amdgcn_readfirstlane((int)wr.ok));
         buffer_to_lds_b128<K_DMA, 64, 1024>(qrs, q_lds_addr + wave8 * RB_BYTES, q_lane_src, (int)(row0 * (uint32_t)(a.q_stride_m * 2)));
@@ -734,7 +742,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         int lo = lane;
         asm volatile("" : "+v"(lo));
         const int n = lo & 31, hi = lo >> 5, lane = lo;
-        const WaveRows owr = wave_rows(o_item, (uint32_t)wave);  // this wave's rows of the item
+        const WaveRows owr = wave_rows(place_of(o_item), (uint32_t)wave);  // this wave's rows of the item
         if (!owr.ok) return;  // (a packed item with fewer heads than waves)
         const uint32_t o_head = owr.head, o_row0 = owr.row0;
         const uint32_t o_split = a.pack_heads ? o_item % S : (o_item % (a.n_heads * S)) % S;
@@ -860,8 +868,11 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             dma(false, 0, 0, p0);
         }
     };
-    enter_item(item);
-    q_dma(item);
+    {
+        const Place p = place_of(item);
+        enter_item(p);
+        q_dma(p);
+    }
     first_tiles();
     while (true) {
         const uint32_t next_item = item_of(round + 1);
@@ -955,7 +966,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
             phase_barrier();
             // every wave has taken its query rows out of LDS (each passed a barrier since): the next item's may come
             const bool stage_now = j == 0 && has_next;
-            if (stage_now) q_dma(next_item);
+            if (stage_now) q_dma(place_of(next_item));
             if (j == 0 && ntg > 0) k_prefetch(1);
             if (j < ntg) mfma_phase(j);  // ---- MFMA phase
             // the rows requested in the last VALU phase have landed (the query rows just requested may take longer)
@@ -980,8 +991,9 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         const uint32_t o_item = item;
         if (has_next) {
             item = next_item, ++round;
-            enter_item(item);
-            if (!q_staged) q_dma(item);
+            const Place p = place_of(item);
+            enter_item(p);
+            if (!q_staged) q_dma(p);
             first_tiles();
         }
         if (grp == 0) write_item(o_item, std::integral_constant<int, 0>());
@@ -1169,6 +1181,7 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
         if (rows.us < us) return fa_launch_prefill_rows(ctx, L, rows);
     }
     a.splits = splits, a.part_acc = nullptr, a.part_ml = nullptr;
+    a.inv_splits = fa_inverse(splits), a.inv_head_splits = fa_inverse(L.n_heads * splits), a.inv_group = fa_inverse(L.group_size), a.inv_blocks = fa_inverse(a.pack_blocks);
     if (splits > 1) {
         const size_t rows = (size_t)L.n_heads * ceil_div_u32(L.q_len, BM) * splits * a.part_rows;
         const size_t acc_bytes = rows * L.head_dim * sizeof(float);

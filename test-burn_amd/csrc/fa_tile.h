@@ -162,9 +162,7 @@ __global__ void __launch_bounds__(S::NT, MIN_WAVES) tile_gemm_kernel(GemmDev a) 
     uint32_t nt, mt;
     {
         const uint32_t G = a.m_tiles > 8 ? 4u : 1u;  // (of many input rows, the tiles at work together in an XCD are 8 x 4, not 16 x 2)
-        uint32_t panel = __umulhi(v, a.panel_inv), rem = v - panel * G * a.m_tiles;  // v / (G * m_tiles), or one less
-        if (rem >= G * a.m_tiles) rem -= G * a.m_tiles, ++panel;
-        const uint32_t w = min(G, a.n_tiles - panel * G);
+        const uint32_t panel = fa_quotient(v, G * a.m_tiles, a.panel_inv), rem = v - panel * G * a.m_tiles, w = min(G, a.n_tiles - panel * G);
         mt = w == 3 ? __umulhi(rem, 0x55555556u) : rem >> (w >> 1), nt = panel * G + rem - mt * w;
     }
     int tile_mat = 0;
@@ -736,7 +734,7 @@ fa_status launch_form(fa_ctx *ctx, FaLaunchScope &scope, GemmDev &a) {
     a.n_tiles = 0, a.m_tiles = ceil_div_u32(a.m, S::MT);
     for (int i = 0; i < 3; ++i) a.tiles[i] = ceil_div_u32(a.rows[i], S::NTR), a.n_tiles += a.tiles[i];
     if (S::JOINED) a.n_tiles = ceil_div_u32(a.rows[0] + 2 * a.rows[1], S::NTR);
-    a.panel_inv = 0xffffffffu / (a.m_tiles > 8 ? 4 * a.m_tiles : a.m_tiles);
+    a.panel_inv = fa_inverse(a.m_tiles > 8 ? 4 * a.m_tiles : a.m_tiles);
     const uint32_t grid = ceil_div_u32(a.n_tiles * a.m_tiles, 8) * 8;
     scope.launch((tile_gemm_kernel<S, MIN_WAVES, FORM>), dim3(grid), dim3(S::NT), S::lds_bytes(a.k_dim), a);
     return FA_OK;
