@@ -279,6 +279,7 @@ fa_status fa_launch_prefill_merge(fa_ctx *ctx, const PrefillMerge &g, uint32_t h
 struct RowsPlan {
     uint32_t waves = 0, splits = 1;  // waves 0: the kernel cannot take the launch
     float us = 0.0f;                 // estimate
+    uint32_t turn = 0;               // rounds of a window attended in turned orders (fa_rows.hip), 0: one order
 };
 RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &a);
 fa_status fa_launch_prefill_rows(fa_ctx *ctx, const PrefillLaunch &a, const RowsPlan &plan);

@@ -1099,7 +1099,8 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     // chunk of at most 64 rows after a long prefix the memory-bound one (fa_chunk.hip), or the tiled one, by estimate. (The estimates are
     // of keys that come from memory, as a layer's do in a model: of long ones that do, the first kernel takes longer (us, rows and the
     // other: 278 rows after 7179, H24 / Hkv8 / D128 55.3, 48.6; 34 after 47550, H16 / Hkv2 / D128 47.3, 36.7; 18 after 44996, H4 / Hkv4 /
-    // D128 38.7, 24.1), of keys that lie in the last-level cache from the call before the least of all. On 4000
+    // D128 38.7, 24.1; the first of them 47 in turned orders, rows_turn), of keys that lie in the last-level cache from the call before the
+    // least of all: where the first and the second are level, the first is a fifth ahead from a cache, 32 after 8160 17.1, 17.2 and 13.0, 16.1. On 4000
     // launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, half of them with keys in memory) the
     // choice takes 1.002 to 1.014 times as long as the best of the three, in the mean, and 0.69 to 0.76 of what the other two would: 48
     // are slower for it by more than 3 %, by 17 % at most (profiles/prefill_choice.txt).)
@@ -1107,7 +1108,7 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     const RowsPlan rows = automatic ? fa_prefill_rows_plan(ctx, L) : RowsPlan();
     if ((automatic || ctx->prefill_variant == 3) && !ctx->prefill_chunk_off) {
         const float chunk_us = rows.waves ? fa_prefill_chunk_estimate_us(ctx, L) : 0.0f;
-        if (chunk_us > 0.0f && rows.us < 0.95f * chunk_us) return fa_launch_prefill_rows(ctx, L, rows);
+        if (chunk_us > 0.0f && rows.us < (rows.turn ? 1.02f : 0.95f) * chunk_us) return fa_launch_prefill_rows(ctx, L, rows);
         if (!rows.waves || chunk_us > 0.0f) {
             bool taken = false;
             FA_TRY(fa_launch_prefill_chunk(ctx, L, ctx->prefill_variant == 3, &taken));
@@ -1178,7 +1179,10 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
             const float cu = wide ? share * (3.52f + 1.041f * (first + longest)) : share * (2.66f + 0.66f * (first + longest));
             us = (wide ? 6.41f : 5.43f) + (one > cu ? one : cu) + (wide ? 0.147f : 0.0775f) * kv_mb;
         }
-        if (rows.us < us) return fa_launch_prefill_rows(ctx, L, rows);
+        // (For launches in turned orders this estimate is up to a tenth too long, or they take longer than theirs where many rounds of one
+        // workgroup's follow: of 420 of 4 to 2500 rows the choice is within 0.9 % of the best in the mean with 0.92 of it, 1.5 % with the whole.)
+        const float ahead = !rows.turn ? 1.0f : rows.splits == 1 && L.kv_len > 6144 ? 0.82f : 0.92f;
+        if (rows.us < ahead * us) return fa_launch_prefill_rows(ctx, L, rows);
     }
     a.splits = splits, a.part_acc = nullptr, a.part_ml = nullptr;
     a.inv_splits = fa_inverse(splits), a.inv_head_splits = fa_inverse(L.n_heads * splits), a.inv_group = fa_inverse(L.group_size), a.inv_blocks = fa_inverse(a.pack_blocks);

@@ -15,11 +15,13 @@
 //     operand of this one's has been read, V likewise: one tile's room per wave, and the other waves of the SIMD fill the gaps
 //     (at D 64 two stages per wave, which leave room for half as many waves, are 5 to 20 % slower);
 //   * the waves' sums meet once, in LDS, and a thread folds its (row, 4 dims) of all of them and writes the row out.
+//   * the blocks that read the same keys through one L2 begin at different ones of them, so that what the first to come asks of memory
+//     is there for the others, and they do not all ask one channel of the L2 at a time (rows_turn).
 // It reads a block's keys once per 32 rows, 131 KB/us and CU along the rows (fa_lds_dma.h), which is why long keys under many rows
 // stay with the tiled kernel (once per 128 rows): fa_prefill_rows_plan. us before and now (tiled or short-chunk kernel before):
 //   H14 / Hkv2 / D64:   32 rows after 500 10.7 -> 4.6; 500 after 1000 14.9 -> 7.5; 2048 rows 22.7 -> 16.2; 32 after 8160 21.0 -> 9.3
 //   H24 / Hkv8 / D128:  32 after 500 12.6 -> 6.9; 128 after 1000 16.8 -> 9.5; 500 rows 12.6 -> 8.3; 32 after 8160 17.6 -> 13.0 (those from the
-//                       last-level cache; from memory 18.3, the short-chunk kernel 16.9)
+//                       last-level cache; from memory 17.1, the short-chunk kernel 17.2)
 //   H16 / Hkv2 / D128:  500 after 1000 23.8 -> 12.2; 32 after 8160 32.6 -> 12.6
 // (The splits combined by the last workgroup of a block to finish, in the launch: 12.8 to 16.3 us for the last of these, against
 // 12.6 with the merge launch - one compute unit reads all of the block's states there.)
@@ -68,6 +70,8 @@ struct RowsDev {
     uint32_t pool_bytes32;  // paged: size of each pool when below 4 GiB (whole pages then go by a 32-bit offset), else 0
     uint32_t n_blocks;      // blocks per KV head
     uint32_t inv_splits, inv_kv_heads;  // fa_inverse
+    uint32_t turn;          // TURN: rounds that the workgroups of a KV head attend in turned orders, a power of two up to 32
+    uint32_t pair_step;     // log2 of how many blocks apart two of a KV head on one XCD are
     uint32_t splits;        // > 1: a block's keys are divided over as many workgroups, whose states a merge launch combines
     float *part_acc, *part_ml;  // [KV head][block][split][32][D] unnormalised sums, [..][32][2] (max, sum)
     float scale_log2e;
@@ -76,7 +80,8 @@ struct RowsDev {
 constexpr int KT = 32;  // keys per tile
 
 // POOL: 0 a contiguous cache, 1 paged, 2 paged with pools of 4 GiB or more (no 32-bit offsets)
-template <int D, int NW, bool BF16, int POOL>
+// TURN: the workgroups that read the same keys through one L2 begin at different ones (rows_turn)
+template <int D, int NW, bool BF16, int POOL, bool TURN>
 __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(RowsDev a_by_value) {
     static_assert(std::is_trivially_copyable<RowsDev>::value, "read as raw bytes from the argument block, where it is the first member");
     const RowsDev a = *(const RowsDev *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -84,7 +89,8 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
     asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.out), "s"(a.q_stride_h), "s"(a.q_stride_m), "s"(a.k_stride_h), "s"(a.v_stride_h),
                  "s"(a.out_stride_h), "s"(a.out_stride_m), "s"(a.block_table), "s"(a.group_size), "s"(a.rcp_group), "s"(a.q_len),
                  "s"(a.kv_len), "s"(a.query_offset), "s"(a.causal), "s"(a.block_size), "s"(a.block_shift), "s"(a.n_kv_heads));
-    asm volatile("" ::"s"(a.pool_bytes32), "s"(a.n_blocks), "s"(a.splits), "s"(a.part_acc), "s"(a.part_ml), "s"(a.scale_log2e), "s"(a.inv_splits), "s"(a.inv_kv_heads));
+    asm volatile("" ::"s"(a.pool_bytes32), "s"(a.n_blocks), "s"(a.splits), "s"(a.part_acc), "s"(a.part_ml), "s"(a.scale_log2e), "s"(a.inv_splits), "s"(a.inv_kv_heads),
+                 "s"(TURN ? a.turn : 0), "s"(TURN ? a.pair_step : 0));
     constexpr bool PAGED = POOL != 0;
     constexpr int DSTEPS = D / 16, DBLKS = D / 32, ROWB = D * 2;
     constexpr int RB_BYTES = 16 * ROWB;                 // 16 rows of K in LDS (rows16 layout), or of V
@@ -184,8 +190,37 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
         asm volatile("" ::: "memory");
     };
 
-    uint32_t tile = t_lo + (uint32_t)wave;
+    const uint32_t first_tile = t_lo + (uint32_t)wave;
+    uint32_t tile = first_tile, nth = 0;  // (tile nth of those that pages have been looked up for)
     fetch_pages(tile);
+    // TURN: the wave's tiles are first_tile + NW r, r < rounds, in windows of a.turn rounds from `base` on, each attended from a round
+    // of its own on and around (a last window that is shorter than that round is far: from its last)
+    uint32_t rounds = 0, turned = 0, base = 0, len = 0, left = 0, next = 0;
+    if constexpr (TURN) {
+        rounds = first_tile < n_tiles ? (n_tiles - first_tile + NW - 1) / NW : 0;
+        turned = ((from_last >> a.pair_step) * 5) & (a.turn - 1);  // (neighbours far apart)
+        len = left = min(a.turn, rounds), nth = next = len ? min(turned, len - 1) : 0;
+        tile = first_tile + NW * nth;
+    }
+    auto find_next = [&]() __attribute__((always_inline)) {  // (while a tile is waited for)
+        if constexpr (TURN) {
+            if (--left == 0) {
+                base += len, len = left = min(a.turn, rounds - base);
+                next = base + (len ? min(turned, len - 1) : 0);
+            } else if (++next == base + len) {
+                next = base;
+            }
+        }
+    };
+    auto next_tile = [&]() __attribute__((always_inline)) {
+        if constexpr (!TURN) {
+            tile += NW, nth = (nth + 1) & 31u;
+            if (PAGED && nth == 0) fetch_pages(tile);
+        } else {
+            if (PAGED && left == len && (base & 31u) == 0) fetch_pages(first_tile + NW * base);
+            tile = len ? first_tile + NW * next : n_tiles, nth = next & 31u;
+        }
+    };
     // Query rows: 2 COLS loads of 1 KiB, one per wave as far as they go, in the layout of a K tile behind the stages
     {
         const size_t q_bytes = ((size_t)(G - 1) * a.q_stride_h + (size_t)(a.q_len - 1) * a.q_stride_m + D) * 2;
@@ -198,7 +233,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
             buffer_to_lds_b128<1, 0, 0>(qrs, lds_addr + STAGES + r * 1024, (int)(at + (uint32_t)rows16_lane_src(lane, 0)), (int)(col * 64));
         }
     }
-    request(true, tile, 0), request(false, tile, 0);
+    request(true, tile, nth), request(false, tile, nth);
     wait_but(std::integral_constant<int, 2 * REQ>{});  // this wave's part of the query rows (requested first) is there
     __syncthreads();
     h8_t qreg[DSTEPS];
@@ -221,7 +256,8 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
     const int v_at = hi * RG_BYTES + ((lane & 15) >> 2) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
 
     const unsigned char *k_lds = lds + wave * TILE, *v_lds = k_lds + HALF + v_at;
-    for (uint32_t nth = 0; tile < n_tiles; tile += NW) {
+    while (tile < n_tiles) {
+        find_next();
         wait_but(std::integral_constant<int, REQ>{});  // K is there
         f16_t s = {};
         h8_t kk[DSTEPS];
@@ -230,11 +266,10 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
 #pragma unroll
         for (int i = 0; i < DSTEPS; ++i) s = mfma<BF16>(kk[i], qreg[i], s);
         lds_reads_done();
-        nth = (nth + 1) & 31u;
-        if (PAGED && nth == 0) fetch_pages(tile + NW);
-        request(true, tile + NW, nth);
-        // accumulator i is key 32 tile + 8 (i / 4) + 4 hi + i % 4
         const uint32_t key0 = tile * KT;
+        next_tile();
+        request(true, tile, nth);
+        // accumulator i is key 32 tile + 8 (i / 4) + 4 hi + i % 4
         if (key0 + KT - 1 > min_limit || key0 + KT > kv_end) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -283,7 +318,7 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
                 oacc[b] = mfma<BF16>(va.h, pb[ks], oacc[b]);
             }
         lds_reads_done();
-        request(false, tile + NW, nth);
+        request(false, tile, nth);
     }
     wait_but(std::integral_constant<int, 0>{});  // (what was requested past the last tile delivered nothing, but must be over)
     __syncthreads();
@@ -336,19 +371,47 @@ __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(Ro
     }
 }
 
-template <int D, int NW, bool BF16>
+template <int D, int NW, bool BF16, bool TURN>
 void launch_rows(FaLaunchScope &scope, const RowsDev &a, uint32_t grid, bool paged) {
-    if (!paged) scope.launch(flash_rows_kernel<D, NW, BF16, 0>, dim3(grid), dim3(NW * 64), 0, a);
-    else if (a.pool_bytes32) scope.launch(flash_rows_kernel<D, NW, BF16, 1>, dim3(grid), dim3(NW * 64), 0, a);
-    else scope.launch(flash_rows_kernel<D, NW, BF16, 2>, dim3(grid), dim3(NW * 64), 0, a);
+    if (!paged) scope.launch(flash_rows_kernel<D, NW, BF16, 0, TURN>, dim3(grid), dim3(NW * 64), 0, a);
+    else if (a.pool_bytes32) scope.launch(flash_rows_kernel<D, NW, BF16, 1, TURN>, dim3(grid), dim3(NW * 64), 0, a);
+    else scope.launch(flash_rows_kernel<D, NW, BF16, 2, TURN>, dim3(grid), dim3(NW * 64), 0, a);
 }
 template <int D, int NW>
 void launch_rows(FaLaunchScope &scope, const RowsDev &a, uint32_t grid, bool bf16, bool paged) {
-    if (bf16) launch_rows<D, NW, true>(scope, a, grid, paged);
-    else launch_rows<D, NW, false>(scope, a, grid, paged);
+    if (bf16) a.turn ? launch_rows<D, NW, true, true>(scope, a, grid, paged) : launch_rows<D, NW, true, false>(scope, a, grid, paged);
+    else a.turn ? launch_rows<D, NW, false, true>(scope, a, grid, paged) : launch_rows<D, NW, false, false>(scope, a, grid, paged);
 }
 
 }  // namespace
+
+// log2 of how many blocks apart two blocks of a KV head are that run on the same XCD (which has every eighth pair)
+static uint32_t mates_apart(uint32_t n_kv_heads) {
+    uint32_t step = 0;
+    while (((n_kv_heads << step) & 7u) != 0) ++step;
+    return step;
+}
+
+// Which launches attend their keys in turned orders, in windows of how many rounds (0: all blocks in one order).
+// Blocks of a KV head that share an XCD read the same keys. In one order they ask for the same lines at the same time, so that memory is
+// asked for one block's worth of tiles and its latency stands in every round; each from another round on, the first requests of all are
+// the whole window, and later rounds find it in the L2. A window's tiles of all streams of an XCD (its KV heads, times the splits) take
+// 3.1 MB of its 4: at 4.2 MB and beyond keys are read again (H16 / Hkv2 / D128, 30 rows after 33878, 16 splits: 29.0 us in one order, 31.7
+// with windows of 4 MB, 38.9 of 8). Where keys lie in a cache anyway and a unit has one workgroup or few, the longer start and the scalar
+// work of a round are 0.1 to 0.3 us of 5 to 10: launches of more than 4 MB, or of several workgroups per unit with many rounds. D 64 in windows
+// of two rounds loses up to 5 % there (44 rows after 5314, H14 / Hkv2: 8.8, 9.1). us in one order -> turned, keys from memory:
+//   H24 / Hkv8 / D128:  500 after 1000 20.5 -> 17.7; 187 after 1130 14.8 -> 12.5; 32 after 8160 18.3 -> 17.0; 68 after 13543 35.0 -> 30.6
+//   H32 / Hkv8 / D128:  194 after 2151 21.1 -> 16.9; H8 / Hkv8: 1928 after 1015 34.4 -> 27.8; H16 / Hkv2: 131 after 11517 34.5 -> 29.6
+//   D 64:  H32 / Hkv8, 1447 after 591 31.7 -> 27.7; H14 / Hkv2, 992 after 10818 64.8 -> 59.1
+static uint32_t rows_turn(const PrefillLaunch &L, uint32_t wgs, uint32_t n_blocks, uint32_t longest, float kv_mb, uint32_t waves, uint32_t splits) {
+    const uint32_t rounds = ceil_div_u32(ceil_div_u32(longest, splits), waves);
+    if (!(kv_mb > 4.0f || (wgs > 600 && rounds >= 8)) || (n_blocks - 1) >> mates_apart(L.n_kv_heads) == 0) return 0;
+    const uint32_t twos = L.n_kv_heads & (0u - L.n_kv_heads), streams = L.n_kv_heads / (twos < 8 ? twos : 8) * splits;
+    const uint32_t round_kb = waves * KT * L.head_dim * 4 / 1024;
+    uint32_t turn = 1;
+    while (turn < 32 && turn * 2 <= rounds && (uint64_t)turn * 2 * streams * round_kb <= 3100) turn *= 2;
+    return turn >= (L.head_dim == 128 ? 2u : 4u) ? turn : 0u;
+}
 
 // How the kernel would be launched, and what that takes by estimate: fitted to 2664 shapes (2 to 8000 rows after 0 to 100000, 14
 // combinations of heads, each timed with every choice, with the tiled and with the short-chunk kernel, over as many layers' caches as
@@ -387,11 +450,17 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float r8 = (float)ceil_div_u32(longest, 8), r4 = (float)ceil_div_u32(longest, 4);
     const float head_mb = (float)longest * (float)(KT * L.head_dim) * 4e-6f, kv_mb = head_mb * (float)L.n_kv_heads;
     const bool waited = wgs <= n_cus && kv_mb > 9.0f;
-    const float us8 = wide ? 2.65f + larger(1.24f * r8, 2.53f * n + 0.137f * chain + 0.0265f * all) + (waited ? 0.386f : 0.03f) * kv_mb
-                           : 3.08f + larger(0.629f * r8, 0.857f * n + 0.0707f * chain + 0.02f * all) + (waited ? 0.206f : 0.055f) * kv_mb;
-    const float us4 = wide ? 4.19f + larger(0.61f * r4, 0.487f * n + 0.122f * chain + 0.0515f * all) + (waited ? 0.536f : 0.065f) * kv_mb
-                           : 3.25f + larger(0.453f * r4, 0.271f * n + 0.0556f * chain + 0.0408f * all) + (waited ? 0.232f : 0.074f) * kv_mb;
-    plan.waves = us4 < us8 ? 4 : 8, plan.us = us4 < us8 ? us4 : us8, plan.splits = 1;
+    const uint32_t turn8 = rows_turn(L, wgs, n_blocks, longest, kv_mb, 8, 1), turn4 = rows_turn(L, wgs, n_blocks, longest, kv_mb, 4, 1);
+    // (turned: 390 launches, 4 to 5 % rms)
+    const float us8 = turn8 ? (wide ? 2.69f + larger(1.086f * r8, 3.11f * n + 0.122f * chain + 0.0135f * all) + (wgs <= n_cus ? 0.188f : 0.133f) * kv_mb
+                                    : 3.48f + larger(0.583f * r8, 0.970f * n + 0.042f * chain + 0.0334f * all) + 0.359f * kv_mb)
+                      : wide ? 2.65f + larger(1.24f * r8, 2.53f * n + 0.137f * chain + 0.0265f * all) + (waited ? 0.386f : 0.03f) * kv_mb
+                             : 3.08f + larger(0.629f * r8, 0.857f * n + 0.0707f * chain + 0.02f * all) + (waited ? 0.206f : 0.055f) * kv_mb;
+    const float us4 = turn4 ? (wide ? 4.93f + larger(0.638f * r4, 0.987f * n + 0.0872f * chain + 0.0565f * all) + (wgs <= n_cus ? 0.103f : 0.08f) * kv_mb
+                                    : 3.17f + larger(0.434f * r4, 0.397f * n + 0.0519f * chain + 0.0243f * all) + 0.355f * kv_mb)
+                      : wide ? 4.19f + larger(0.61f * r4, 0.487f * n + 0.122f * chain + 0.0515f * all) + (waited ? 0.536f : 0.065f) * kv_mb
+                             : 3.25f + larger(0.453f * r4, 0.271f * n + 0.0556f * chain + 0.0408f * all) + (waited ? 0.232f : 0.074f) * kv_mb;
+    plan.waves = us4 < us8 ? 4 : 8, plan.us = us4 < us8 ? us4 : us8, plan.turn = us4 < us8 ? turn4 : turn8, plan.splits = 1;
     // Keys split: all workgroups resident at once, one to a CU. (The merge launch reads the splits of a row 4, 8, 16 or 32 at a time.)
     float best = plan.us / 1.05f;
     const uint32_t most = n_cus / (ceil_div_u32(wgs, 8) * 8);
@@ -399,9 +468,12 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float xcd_mb = head_mb * (float)(xcd_heads < xcd_blocks ? xcd_heads : xcd_blocks);
     for (uint32_t s = 2; s <= most && s * 4 <= longest && s <= 32; s = s == 16 ? 32 : s + 1) {
         const float r = (float)ceil_div_u32(ceil_div_u32(longest, s), 8), mb = (float)wgs * (float)(32 * L.head_dim) * (float)s * 4e-6f;
-        const float us = wide ? 5.77f + 1.464f * r + 0.0768f * (float)s + 0.549f * mb + 0.0547f * kv_mb + 0.35f * xcd_mb
-                              : 5.28f + 0.644f * r + 0.0752f * (float)s + 0.4585f * mb + 0.0584f * kv_mb + 0.41f * xcd_mb;
-        if (us < best) best = us, plan.us = us, plan.splits = s, plan.waves = 8;
+        const uint32_t turn = rows_turn(L, wgs, n_blocks, longest, kv_mb, 8, s);
+        const float us = turn ? (wide ? 6.99f + 1.183f * r + 0.0149f * (float)s + 0.3715f * mb + 0.0674f * kv_mb + 0.507f * xcd_mb
+                                      : 6.28f + 0.674f * r + 0.0385f * (float)s + 0.4104f * mb + 0.0761f * kv_mb + 0.337f * xcd_mb)
+                         : wide ? 5.77f + 1.464f * r + 0.0768f * (float)s + 0.549f * mb + 0.0547f * kv_mb + 0.35f * xcd_mb
+                                : 5.28f + 0.644f * r + 0.0752f * (float)s + 0.4585f * mb + 0.0584f * kv_mb + 0.41f * xcd_mb;
+        if (us < best) best = us, plan.us = us, plan.splits = s, plan.waves = 8, plan.turn = turn;
     }
     return plan;
 }
@@ -423,6 +495,7 @@ fa_status fa_launch_prefill_rows(fa_ctx *ctx, const PrefillLaunch &L, const Rows
     a.scale_log2e = L.scale * 1.4426950408889634f;
     a.splits = plan.splits, a.inv_splits = fa_inverse(a.splits), a.inv_kv_heads = fa_inverse(a.n_kv_heads);
     a.part_acc = a.part_ml = nullptr;
+    a.turn = plan.turn, a.pair_step = mates_apart(L.n_kv_heads);
     const uint32_t pairs = L.n_kv_heads * a.n_blocks, grid = ceil_div_u32(pairs, 8) * 8 * a.splits;
     if (a.splits > 1) {  // (at most one workgroup per CU: 4.2 MB)
         const size_t rows = (size_t)pairs * a.splits * 32, acc_bytes = rows * L.head_dim * sizeof(float);

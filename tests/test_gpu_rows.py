@@ -173,6 +173,32 @@ def test_rows_paged_more_than_32_tiles_per_wave(H, Hkv, D, M, prefix, bs):
     test_rows_paged(H, Hkv, D, M, prefix, False, bs)
 
 
+TURNED = [
+    # More than 4 MB of keys: blocks that share an XCD attend windows of rounds, each from a round of its own on
+    # H, Hkv, D, rows, prefix, splits expected
+    (24, 8, 128, 300, 950, False),   # windows of 4 or 8 rounds, the last one shorter; every block another number of keys
+    (24, 8, 128, 300, 1020, False),
+    (8, 8, 128, 66, 3001, True),     # 3 blocks, keys split: a window of 2 rounds, splits of unequal lengths
+    (6, 2, 128, 200, 4100, True),    # two blocks of a KV head to an XCD, and three
+    (16, 8, 128, 700, 400, False),   # several workgroups to a unit
+    (16, 8, 64, 200, 2350, False),   # D 64
+    (20, 5, 128, 120, 2000, False),  # KV heads that are not a divisor of 8: every eighth block of one is on the same XCD
+]
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f16", "bf16"])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", TURNED)
+def test_rows_turned_contiguous(H, Hkv, D, M, prefix, split, bf16):
+    test_rows_contiguous(H, Hkv, D, M, prefix, split, bf16)
+
+
+@pytest.mark.parametrize("bs", [16, 48])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", TURNED + [(32, 2, 64, 620, 3700, False)])
+def test_rows_turned_paged(H, Hkv, D, M, prefix, split, bs):
+    """The last: several windows, and more than 32 tiles to a wave, whose pages are looked up a second time at a window's start."""
+    test_rows_paged(H, Hkv, D, M, prefix, split, bs)
+
+
 @pytest.mark.parametrize("H,Hkv,D,M,prefix", [(24, 8, 128, 278, 7179), (16, 2, 128, 34, 47550), (32, 8, 128, 51, 19165), (4, 4, 128, 18, 44996)])
 def test_long_keys_from_memory_stay_with_the_other_kernels(H, Hkv, D, M, prefix):
     """Shapes that take 1.15 to 1.6 times as long on this kernel where their keys come from memory: the choice is another one, with its
