@@ -8,16 +8,17 @@
 // the matrix instruction's operand (16 rows x 64 bytes, one row per lane of a 16-lane group) moves 37 KB/us into a compute unit
 // from L2, a request along a row 108 to 130 KB/us. So rows are fetched along themselves, whole rows per wave (row r by wave
 // r % 8), normalised in the registers they arrive in (no exchange between waves), written to LDS and read back as operands:
-//   * a workgroup (8 waves) owns up to 32 weight rows - two 16-row tiles - and walks over its passes of 32 input rows (16 where
-//     rows are longer than 2048 features). All its weights are requested once, straight into the operand layout, behind the
-//     first pass's input rows (some of the longest rows' in two parts: SPLIT); a pass's rows are requested while the one before is
-//     multiplied;
+//   * a workgroup (8 waves) owns up to 32 weight rows - two 16-row tiles - and walks over its passes of 32 input rows. All its weights
+//     are requested once, straight into the operand layout, behind the first pass's input rows; a pass's rows are requested while the
+//     one before is multiplied;
+//   * rows of more than 2048 features: 16 input rows to a workgroup and no second pass, but up to five tiles, a few of whose requests are
+//     on their way at a time (RING, and panel_plan for what both gave);
 //   * wave w multiplies the feature blocks 16 j + 2 w and 16 j + 2 w + 1 of every 512 features (adjacent: the two requests touch
 //     the same lines);
 //   * the eight waves' partial tiles meet in LDS and are added in wave order; then alpha, bias, beta * residual and one
 //     rounding, or the KvPrepFused work on the rounded values (a workgroup then takes whole rotation pairs);
 //   * few weight rows and many input rows: the passes are spread over workgroups (grid y), each keeping its 32 weight rows;
-//   * NeoX pairs of a workgroup of up to 16 weight rows lie in one tile, 8 rows from each half (two tiles of which half the rows did
+//   * NeoX pairs of a workgroup of up to 16 weight rows, and of the last of an odd number of tiles, lie in one tile, 8 rows from each half (two tiles of which half the rows did
 //     not exist: 1152 x 896, 8 rows, F16 4.4 -> 3.8 us, Q8_0 4.9 -> 4.0, Q4_0 5.0 -> 4.1; 2560 x 2048 6.4 -> 5.4, 7.0 -> 5.4, 6.7 -> 5.2).
 // Block-quantised weights become f16(weight * scale) as in the GEMM (src/metals/mma/tile_loader.metal:100-120); below 12 input
 // rows (SUMS) they follow the weight stream: a matrix instruction covers one 32-feature block, its f32 sums times the scale.
@@ -39,7 +40,7 @@ struct PanelDev {
     __half *out[3];
     uint32_t rows0, rows1, total_rows;  // of W_q, of W_k and W_v each, of all
     const __half *x, *gamma, *residual;
-    uint32_t k_dim, m, rows_per_wg, canonical, n_pass;
+    uint32_t k_dim, m, rows_per_wg, canonical, n_pass, inv_pass /* fa_inverse */;
     float eps, inv_k, alpha, beta;
     RopeDev r;
     uint32_t scale_pairs;  // a row holds an even number of scales, 4-byte aligned
@@ -57,20 +58,20 @@ template <int PK>
 constexpr int LDS_SHARE = (PK <= 2 ? 80 * 1024 : 160 * 1024) - 6 * 1024;  // two workgroups per compute unit, or one; less the scales
 // Two workgroups per compute unit: rows of up to 1024 features, except where the registers do not allow it.
 constexpr bool two_per_cu(uint32_t nt, uint32_t nc, uint32_t pk, bool rope) { return pk <= 2 && !(rope && nt == 2 && nc == 2); }
-// The waves' sums get LDS of their own where it is there (a barrier less per pass), else they go over the rows.
-template <int NT, int NC, int PK>
-constexpr bool REDUCE_APART = NC * 16 * row_bytes<PK>() + reduce_bytes<NT, NC>() + (G_IN_LDS<PK> ? PK * 1024 : 0) <= LDS_SHARE<PK>;
-template <int NT, int NC, int PK>
-constexpr int lds_rows_bytes() {
-    const int rows = NC * 16 * row_bytes<PK>(), red = reduce_bytes<NT, NC>();
-    return REDUCE_APART<NT, NC, PK> ? rows + red : rows > red ? rows : red;
-}
 // Block-quantised weights: their scales as f16 [block][slot], with 8 bytes between blocks: a wave writes the blocks of two or three
 // rows side by side, all of them to one bank without (o_proj of 1536 features x 4096 rows, 40 input rows: Q8_0 7.06 -> 6.64 us).
 template <int NT>
 constexpr int scale_stride() { return NT * 16 + 4; }
 template <int NT, int PK>
 constexpr int scale_bytes() { return scale_stride<NT>() * PK * 16 * 2; }
+// The waves' sums get LDS of their own where it is there (a barrier less per pass), else they go over the rows.
+template <int NT, int NC, int PK>
+constexpr bool REDUCE_APART = NC * 16 * row_bytes<PK>() + reduce_bytes<NT, NC>() + (G_IN_LDS<PK> ? PK * 1024 : 0) + (NT > 3 ? scale_bytes<NT, PK>() : 0) <= LDS_SHARE<PK>;
+template <int NT, int NC, int PK>
+constexpr int lds_rows_bytes() {
+    const int rows = NC * 16 * row_bytes<PK>(), red = reduce_bytes<NT, NC>();
+    return REDUCE_APART<NT, NC, PK> ? rows + red : rows > red ? rows : red;
+}
 // Q4_0 with per-block sums, more than 1024 features: weights are fetched along memory and turned into operand order in LDS.
 template <int WB, int PK, bool SUMS>
 constexpr bool TURNS = WB == 4 && SUMS && PK > 2;

@@ -69,33 +69,42 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     constexpr int GB = !WIDE && !TURN ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
     typedef typename std::conditional<WIDE || TURN, u4v_t, raw_t>::type req_t;
     // A wave that asks for more than the memory takes stands still until it has (a workgroup of 32 rows of 3072 features asks for
-    // 3 us), and normalises no rows meanwhile. SPLIT: it asks for the first NA requests of a tile, and for the others when the rows are
-    // in LDS. (3072 x 3072 without a norm, F16, 2 to 16 rows: 5.8 -> 5.2 us; Q8_0 2 to 8 rows 5.5 -> 5.1, row-major 7.2 -> 6.2, 24 and 32
-    // rows 7.1 -> 6.2; FusedQkv of 5120 x 3072 Q8_0, 16 rows 9.3 -> 8.7. Two tiles of F16, and one with its rotation, lose 1 to 14 % by
-    // it, shorter rows and Q4_0 have too few requests.)
-    constexpr bool SPLIT = PK > 4 && (WB == 8 ? !ROPE || NT == 2 : WB == 16 && !ROPE && NT == 1);
-    constexpr int NA = !SPLIT ? NQ : NT == 1 ? (NQ < 8 ? NQ : 8) : SUMS ? 6 : 4;
+    // 3 us), and normalises no rows meanwhile. RING, of the longest rows, whose workgroups have one pass each: it asks for the first NF
+    // requests of a tile, and for another whenever one has been multiplied - REST: for all others when the rows are in LDS (F16, 9 rows
+    // of 3072 features: 4.9 us, one by one 5.1). All tiles' first requests come before any second one. FusedQkv of 5120 x 3072, all asked
+    // for at once tile after tile -> this, us: F16 2 rows 9.7 -> 8.4, 16 rows 10.8 -> 9.7; Q8_0 9.1 -> 7.7, 11 rows 10.6 -> 9.2; Q4_0,
+    // whose requests are few and all made at once, 8.7 -> 8.2.
+    constexpr bool RING = PK > 4, REST = RING && WB == 16 && NT == 1;
+    constexpr int NF = !RING || WB == 4 ? NQ : WB == 16 ? (NT <= 2 ? 8 : NT == 3 ? 6 : 4) : NT == 1 ? (NQ < 8 ? NQ : 8) : NT == 2 ? 4 : NT == 3 ? 3 : 2;
+    constexpr int NA = REST ? NQ : NF;  // places in registers
     // The order of the first requests is input rows, the norm's weights, scales, weights. Loads complete in the order in which they
     // are issued; left to itself the compiler puts the weights ahead of the rows in most of the kernels, and what is done with
     // the rows then waits for the whole weight stream. (m 12 .. 32, K 2048 .. 3072: o_proj 4 to 14 % less. With the longest rows and a
     // norm of two rows per wave the norm's chain is longer than the weights' stream, and the compiler's mixture is 1 to 3 % better.)
-    constexpr bool ORDERED = FEW || !ROPE || PK <= 4 || SPLIT;
+    constexpr bool ORDERED = FEW || !ROPE || PK <= 4 || WB == 8 || NT > 2;
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
+    const uint32_t inv_pass = RING ? a.inv_pass : 0;
     const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
     const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
     const uint32_t normal = a.r.normal, head_dim = a.r.head_dim, scale_pairs = a.scale_pairs;
     // (the launch's arguments in two trips through the scalar cache: what the first requests need, and the rest behind them)
     asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(rows0), "s"(rows1), "s"(total_rows), "s"(x_in), "s"(gamma), "s"(K), "s"(m_rows),
-                 "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass));
+                 "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass), "s"(inv_pass));
     if constexpr (WB != 16) asm volatile("" ::"s"(sp0), "s"(sp1), "s"(sp2), "s"(scale_pairs));
     if constexpr (ROPE) asm volatile("" ::"s"(normal), "s"(head_dim));
     const bool canonical = canonical_u != 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, c = lane >> 4;
     const uint32_t nkb = K / 32, n_pieces = K / 8;
-    const uint32_t row_begin = blockIdx.x * rows_per_wg;
+    // RING: the workgroups of the passes of the same weight rows one after the other on one XCD
+    uint32_t along = blockIdx.x, first_pass = blockIdx.y;
+    if constexpr (RING) {
+        const uint32_t eighth = blockIdx.x >> 3, group = fa_quotient(eighth, n_pass, inv_pass);
+        along = group * 8 + (blockIdx.x & 7), first_pass = eighth - group * n_pass;
+    }
+    const uint32_t row_begin = along * rows_per_wg;
     const uint32_t row_end = min(total_rows, row_begin + rows_per_wg);
     if (row_begin >= row_end) return;
     // ROPE (rows_per_wg is even, the matrices hold whole heads): the pairing and the head size
@@ -105,13 +114,14 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
         pair_begin = row_begin >> 1, pair_end = row_end >> 1;
     }
     // Weight row of slot (tile t, row n of the tile) across the three matrices laid end to end; a slot past the workgroup's
-    // last row gives the workgroup's first row with valid = false. NeoX pairs: tile 0 (of one tile: its first 8 rows) holds rows of
-    // first halves of heads, tile 1 (the other 8) their mates half a head on.
+    // last row gives the workgroup's first row with valid = false. NeoX pairs: tiles 0 and 2 (of an odd number the last tile's first 8
+    // rows) hold rows of first halves of heads, tiles 1 and 3 (the other 8) their mates half a head on.
     auto slot_row = [&](uint32_t t, uint32_t n_, bool &valid) __attribute__((always_inline)) -> uint32_t {
         if (ROPE && neox) {
-            const uint32_t p = pair_begin + (NT == 2 ? n_ : n_ & 7u), pv = p < pair_end ? p : pair_begin;
+            const bool both = NT % 2 == 1 && t == NT - 1;
+            const uint32_t p = pair_begin + 16u * (t >> 1) + (both ? n_ & 7u : n_), pv = p < pair_end ? p : pair_begin;
             valid = p < pair_end;
-            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + ((NT == 2 ? t : n_ >> 3) << half_shift);
+            return ((pv >> half_shift) << (half_shift + 1)) + (pv & ((1u << half_shift) - 1u)) + ((both ? n_ >> 3 : t & 1u) << half_shift);
         }
         const uint32_t gr = row_begin + 16u * t + n_;
         valid = gr < row_end;
@@ -135,7 +145,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int j = 0; j < PK; ++j) xr[i][j] = *reinterpret_cast<const h8_t *>(row + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
         }
     };
-    uint32_t pass = blockIdx.y;
+    uint32_t pass = first_pass;
     request_rows(pass, true);
     if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
     h8_t gv[PK];
@@ -207,49 +217,37 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int b = 0; b < 4; ++b) w[b] = *reinterpret_cast<const uint32_t *>(turn + b * 256 + n * 16 + c * 4);
         }
     };
-    req_t wv[NT][NQ];
-    auto request_weights = [&](int from, int to) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            bool valid;
-            int mat;
-            const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
-            const uint32_t N = pick3(mat, rows0, rows1, rows1);
-            const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
-            const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
-            const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
-#pragma unroll
-            for (int i = from; i < to; ++i) {
-                const uint32_t kb = kb_of(i) + get_blk;
-                const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
-                if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
-                wv[t][i] = fa_norm::load_global_once<req_t>(p);
-            }
-        }
+    req_t wv[NT][NA];
+    const unsigned char *w_at[NT];  // block 0 of the lane's row in each tile, and how far apart blocks are
+    uint32_t w_step[NT];
+    auto request_weights = [&](int t, int i) __attribute__((always_inline)) {
+        const uint32_t kb = kb_of(i) + get_blk;
+        const unsigned char *p = w_at[t] + (size_t)min(kb, nkb - 1u) * w_step[t];
+        // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
+        // block-quantised weights are finite, and their scale is zero there.)
+        if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
+        wv[t][i % NA] = NT > 2 ? fa_norm::load_global<req_t>(p) : fa_norm::load_global_once<req_t>(p);
     };
-    if constexpr (SPLIT) {
-        request_weights(0, NA);
-    } else {  // (the same in place: the compiler makes 1 to 5 % slower kernels of the call)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            bool valid;
-            int mat;
-            const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
-            const uint32_t N = pick3(mat, rows0, rows1, rows1);
-            // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
-            const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
-            const unsigned char *p0 = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
-            const uint32_t kb_stride = (canonical ? N * 32 : 32) * WB / 8;
+    for (int t = 0; t < NT; ++t) {
+        bool valid;
+        int mat;
+        const uint32_t lrow = locate(slot_row((uint32_t)t, get_row, valid), mat);
+        const uint32_t N = pick3(mat, rows0, rows1, rows1);
+        // canonical (blocked by 32 features): (k % 32) + 32 * (row + (k / 32) * N); row-major: row * K + k
+        const uint32_t in_block = GB == 1 ? (uint32_t)c * WB : GB == 2 ? ((uint32_t)c & 1u) * 16u : 0u;  // bytes
+        w_at[t] = pick3(mat, w0, w1, w2) + (canonical ? (size_t)lrow * 32 : (size_t)lrow * K) * WB / 8 + in_block;
+        w_step[t] = (canonical ? N * 32 : 32) * WB / 8;
+        if constexpr (!RING) {
 #pragma unroll
-            for (int i = 0; i < NQ; ++i) {
-                const uint32_t kb = kb_of(i) + get_blk;
-                const unsigned char *p = p0 + (size_t)min(kb, nkb - 1u) * kb_stride;
-                // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
-                // block-quantised weights are finite, and their scale is zero there.)
-                if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
-                wv[t][i] = fa_norm::load_global_once<req_t>(p);
-            }
+            for (int i = 0; i < NF; ++i) request_weights(t, i);
         }
+    }
+    if constexpr (RING) {
+#pragma unroll
+        for (int i = 0; i < NF; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) request_weights(t, i);
     }
     if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
     if (G_IN_LDS<PK> && ORDERED && gamma) {
@@ -284,7 +282,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     float *red = reinterpret_cast<float *>(smem + (APART ? NC * 16 * XROW : 0));  // [NW][NT][NC][16][17]; not APART: over the rows once they have been read
 
     while (true) {
-        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = pass + gridDim.y;
+        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = RING ? n_pass : pass + gridDim.y;
         if (gamma) {  // x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16; a wave holds whole rows
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
@@ -308,7 +306,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int h = 0; h < NC; ++h) d[t][h] = d2[t][h] = f4v_t{0.0f, 0.0f, 0.0f, 0.0f};
         _Float16 s_res[NT], rc[NT], rs[NT];
         uint32_t r_pos = 0, r_blk = 0;
-        if (!APART && pass != blockIdx.y) __syncthreads();  // the sums have been read
+        if (!APART && pass != first_pass) __syncthreads();  // the sums have been read
 #pragma unroll
         for (int i = 0; i < NR; ++i)
 #pragma unroll
@@ -318,7 +316,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 *reinterpret_cast<h8_t *>(smem + (wave + 8 * i) * XROW + (j * 64 + lane) * 16) = v;
             }
         if constexpr (WB != 16) {
-            if (pass == blockIdx.y) {
+            if (pass == first_pass) {
 #pragma unroll
                 for (int i = 0; i < SC_LOADS; ++i) {
                     uint32_t slot, kb2;
@@ -348,19 +346,18 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 s_res[t] = fa_norm::load_global<_Float16>(
                     residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * pick3(s_mat[t], rows0, rows1, rows1) + s_row[t] : x_in);
         }
-        if constexpr (SPLIT) {
-            if (pass == blockIdx.y) {
-                __builtin_amdgcn_sched_barrier(0);
-                request_weights(NA, NQ);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        if constexpr (REST) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = NF; i < NQ; ++i) request_weights(0, i);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (next < n_pass) request_rows(next, false);
+        if (!RING && next < n_pass) request_rows(next, false);
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
-            if (TURN && pass == blockIdx.y) {
+            if (TURN && pass == first_pass) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) operand_order(wv[t][i]);
+                for (int t = 0; t < NT; ++t) operand_order(wv[t][i % NA]);
             }
             const uint32_t kb = kb_of(i) + (TURN ? 0u : lane_blk);
             const unsigned char *xp = smem + n * XROW + kb * 64 + (GB == 1 || TURN ? c * 16 : GB == 2 ? (c & 1) * 32 : 0);
@@ -369,7 +366,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             _Float16 sc[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                raw[t] = wv[t][i];
+                raw[t] = wv[t][i % NA];
                 // (opaque: made f16 here in every pass, not ahead of the passes, where it would wait for the weights)
                 if constexpr (WB != 16) asm volatile("" : "+v"(raw[t]));
                 if constexpr (WIDE) sc[t] = scp[t * 16];
@@ -402,6 +399,14 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                             sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[h], sum, 0, 0, 0);
                         }
                     }
+                }
+            }
+            if constexpr (RING && !REST) {
+                if (i + NA < NQ) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) request_weights(t, i + NA);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
@@ -437,9 +442,9 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
             for (int t = 0; t < NT; ++t) {
                 if constexpr (ROPE) {
                     const uint32_t D = 2u << half_shift, half = 1u << half_shift;
-                    // the mate: the same slot of the other tile, or 8 slots away in the one (NeoX), or the neighbouring slot
-                    const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], NT == 1 && neox ? 8 : 1, 64);
-                    const _Float16 ym = NT == 2 && neox ? y2[NT == 2 ? t ^ 1 : 0] : y_adj;
+                    // the mate: the same slot of the other tile, or 8 slots away in a tile of both halves (NeoX), or the neighbouring slot
+                    const _Float16 y_adj = (_Float16)__shfl_xor((float)y2[t], NT % 2 == 1 && t == NT - 1 && neox ? 8 : 1, 64);
+                    const _Float16 ym = (t ^ 1) < NT && neox ? y2[(t ^ 1) < NT ? t ^ 1 : 0] : y_adj;
                     if (!s_ok[t] || w_col >= cols) continue;
                     const uint32_t hd = s_row[t] & (D - 1u), head = s_row[t] >> (half_shift + 1);
                     const bool first = neox ? hd < half : (hd & 1u) == 0;
@@ -464,7 +469,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 }
             }
         }
-        if (next >= n_pass) break;
+        if (RING || next >= n_pass) break;
         pass = next;
     }
 }
@@ -493,6 +498,12 @@ fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32
     if (a.m <= 8 && (!Q || sums)) return nt == 1 ? launch_pk<WB, 1, 1, Q, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, Q, true>(scope, rope, pk, grid, a);
     if constexpr (Q) {
         if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true, false>(scope, rope, pk, grid, a);
+    }
+    if (nt > 2) {  // (rows of more than 2048 features)
+        if (nt == 3) return rope ? launch_one<WB, 3, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 6, false, false, false>(scope, grid, a);
+        if (nt == 4) return rope ? launch_one<WB, 4, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 4, 1, 6, false, false, false>(scope, grid, a);
+        if constexpr (!Q) return rope ? launch_one<WB, 5, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 5, 1, 6, false, false, false>(scope, grid, a);
+        return fa_fail(FA_ERR_INVALID_OPERATION, "panel kernel: %u tiles of block-quantised weight rows", nt);
     }
     if (nt == 1) return nc == 1 ? launch_pk<WB, 1, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 1, 2, false, false>(scope, rope, pk, grid, a);
     return nc == 1 ? launch_pk<WB, 2, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 2, false, false>(scope, rope, pk, grid, a);

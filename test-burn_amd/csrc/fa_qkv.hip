@@ -401,6 +401,20 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
         const uint64_t cost = (uint64_t)load * ceil_div_u32(p.n_pass, gy) * tiles * beside;
         if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy, p.rounds = ceil_div_u32(gx * gy, slots);
     }
+    // Rows of more than 2048 features: a workgroup per pass, with as many weight rows as put all of them in one round of workgroups. (One
+    // workgroup for both passes, 20 weight rows: the second pass's rows are asked for, normalised and multiplied behind the first's. FusedQkv of
+    // 5120 x 3072, 32 rows, F16 14.5 -> 11.5 us, Q8_0 14.3 -> 10.7, Q4_0 13.7 -> 10.6; 64 rows F16 19.3 -> 15.5; o_proj of 3072 x 3072,
+    // 32 rows F16 8.1 -> 7.4, 48 rows 10.0 -> 7.7, Q8_0 10.0 -> 7.5.) The workgroups of the same weight rows are next to each other on an
+    // XCD, so that memory is read once.
+    if (p.pk > 4) {
+        if (p.n_pass > 1) {
+            const uint32_t beside = n_cus / (8 * p.n_pass) * 8, rows = (ceil_div_u32(total_rows, beside ? beside : 8) + 1) & ~1u;
+            p.rows_per_wg = rows < 80 ? rows : 80;  // (five tiles: registers)
+            p.nt = ceil_div_u32(p.rows_per_wg, 16), p.grid_x = ceil_div_u32(total_rows, p.rows_per_wg);
+            p.rounds = ceil_div_u32(ceil_div_u32(p.grid_x, 8) * 8 * p.n_pass, n_cus);
+        }
+        p.grid_y = p.n_pass;
+    }
     return p;
 }
 
@@ -412,27 +426,33 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
 // 5.1; block-quantised as long as each pass has a workgroup of its own, two to a compute unit, 239 rows of 896 x 192 Q4_0 3.8 against
 // 5.2, 314 rows of 512 x 128 Q8_0 3.7 against 4.4, 228 rows of 640 x 960 Q4_0 4.5 against 4.8, 265 rows of 896 x 704 Q8_0 row-major
 // both 5.2, 30 launches 0.85 in the mean and 1.13 at worst; of 256 features only one to a compute unit, 438 rows of 256 x 576 take
-// 1.17 times as long as the tiles),
-// earlier for block-quantised weights of 3072 features (64 rows: 48.2 against 44.8 us per layer) - unless the GEMM is a tenth ahead by
+// 1.17 times as long as the tiles) - unless the GEMM is a tenth ahead by
 // estimate: many weight rows are many passes of the input rows here, or rounds of workgroups. A launch takes the weight stream, and
 // for each pass that a compute unit has one after the other the input rows of that pass, fetched and multiplied and, with a gamma,
 // normalised (fitted to launches of 12 to 416 rows over 512 to 3072 features and 512 to 10240 weight rows; of 1380 with both sides
 // measured, none that leaves is more than 2 % slower for it). us, here and as a GEMM: 2048 x 10240 32 rows 16.6, 12.4, 100 rows 44.5,
-// 17.6; 2048 x 2560 64 rows 8.2, 11.0, 100 rows 12.8, 11.1; 1024 x 6144 100 rows 13.2, 8.8; 3072 x 5120 32 rows 13.5, 13.5, 64 rows
-// 20.1, 14.7. An explicit GEMM threshold (fa_set_gemm_min_m) wins.
+// 17.6; 2048 x 2560 64 rows 8.2, 11.0, 100 rows 12.8, 11.1; 1024 x 6144 100 rows 13.2, 8.8. An explicit GEMM threshold (fa_set_gemm_min_m) wins.
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const uint32_t min_m = ctx->qkv_rows32_min_m ? ctx->qkv_rows32_min_m : PANEL_MIN_M_DEFAULT;
     const bool f16 = l.weight_bits == 16;
-    const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : f16 ? 192u : 512u) : l.k_dim <= 2048 ? 128u : f16 ? 64u : 48u;
+    const uint32_t max_m = l.k_dim <= 1024 ? (l.gamma ? 416u : f16 ? 192u : 512u) : l.k_dim <= 2048 ? 128u : 64u;
     if (min_m > 32 || l.m < min_m || l.m > max_m || l.k_dim > 3072 || l.k_dim % 32 != 0) return false;
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
     if (l.m < FA_GEMM_MIN_M_DEFAULT) return true;
     const PanelPlan p = panel_plan(ctx, l, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
-    if (l.m <= 32 && p.rounds == 1) return true;
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
+    if (l.m <= 32 && p.rounds == 1 && l.n_dim + 2 * l.n_kv <= 32 * n_cus) return true;
+    // More than 2048 features: a workgroup has one pass, with the weight rows that put all passes in one round (up to 80). Never behind
+    // the GEMM with F16 weights then, and always where they need a second round; block-quantised weights, which are made f16 for each
+    // pass, up to 48 of them, 64 of more than 2560 features. us, here and as a GEMM, 3072 features: 5120 rows F16 57 rows 13.3, 16.1; 10240 x
+    // 2560 F16 19 rows 14.7, 16.7; 4288 rows Q8_0 37 rows 11.2, 13.3; 2240 rows Q8_0 52 rows 9.6, 12.4; beyond the line 5184 x 2560 36
+    // rows Q4_0 13.2, 11.4 and Q8_0 12.9, 12.2; 5120 x 2304 57 rows Q4_0 13.5, 11.0; second round 5312 rows F16 58 rows 26.0, 19.7.
+    // (240 launches of 2112 to 3072 features x 1024 to 10600 rows.)
+    if (p.pk > 4)
+        return p.rounds == 1 && (f16 || ((l.m <= 48 || l.gamma || l.k_dim > 2304) && p.rows_per_wg <= (l.k_dim > 2560 ? 64u : 48u)));
     if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
     // Block-quantised with a norm: where 32 input rows x 32 weight rows are more than a piece per compute unit, a second pass costs 3 us
     // and more, which the estimate below does not see of few features: 195 rows, 512 x 2112 Q4_0 12.0 us, 8.4 with the norm's launch and
@@ -478,13 +498,13 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
         a.block_shift = (d.block_size & (d.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(d.block_size) : 32u;
     }
     const PanelPlan p = panel_plan(ctx, l, rope != nullptr);
-    a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass;
+    a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass, a.inv_pass = fa_inverse(p.n_pass);
     a.scale_pairs = l.k_dim / 32 % 2 == 0 ? 1u : 0u;
     for (int i = 0; i < 3; ++i)
         if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) a.scale_pairs = 0;
     FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
     const bool sums = l.m < FA_GEMM_MIN_M_DEFAULT;  // (of interest to block-quantised weights only: the arithmetic, see fa_panel.h)
-    const dim3 grid(p.grid_x, p.grid_y);
+    const dim3 grid = p.pk > 4 ? dim3(ceil_div_u32(p.grid_x, 8) * 8 * p.n_pass) : dim3(p.grid_x, p.grid_y);
     if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
     else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
     else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));

@@ -75,6 +75,22 @@ def test_chunk_in_one_launch(K, N, NK, m, layout, weights):
         b.free()
 
 
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,layout", [
+    (2112, 4112, 520, 17, 0),   # 42 weight rows to a workgroup: three tiles, the last of 10 rows; the second pass of one row
+    (3072, 4104, 512, 32, 1),   # the same, passes of 16 rows
+    (3072, 4496, 1800, 18, 1),  # four tiles
+    (2592, 3080, 520, 33, 0),   # three passes, an odd number of feature blocks
+    (3072, 2056, 520, 64, 1),   # four passes, workgroups of the last group of eight without rows
+])
+def test_long_rows_a_workgroup_for_each_pass(K, N, NK, m, layout, weights):
+    test_chunk_in_one_launch(K, N, NK, m, layout, weights)
+
+
+def test_long_rows_in_five_tiles():
+    test_chunk_in_one_launch(2592, 3840, 640, 64, 1, "f16")  # 80 weight rows to a workgroup, block-quantised as a GEMM
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
 @pytest.mark.parametrize("K,m", [(32, 2), (96, 11), (96, 12), (896, 33), (1056, 5), (2016, 20), (2080, 5), (2080, 17)])
@@ -111,10 +127,13 @@ def test_rows_absent_from_a_pass(K, N, NK, m, weights):
     (2080, 16, 2, 128, 33),   # eight: passes spread over workgroups
     (96, 28, 2, 128, 17),     # the most that one tile holds
     (96, 30, 2, 128, 9),      # past it: two tiles
+    (3072, 24, 8, 128, 32),   # 20 pairs: 16 in two tiles, 4 in a third
+    (2816, 24, 12, 128, 19),  # 24: the third is full
+    (3072, 24, 8, 128, 40),   # 32 in four tiles
 ])
 def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
-    """Up to 16 weight rows per workgroup, both halves of its NeoX pairs lie in one tile: the fused write stage equals the two ops to
-    the bit, in both pairings."""
+    """Up to 16 weight rows per workgroup, and in the last of an odd number of tiles, both halves of NeoX pairs lie in one tile: the fused
+    write stage equals the two ops to the bit, in both pairings."""
     announce("neox pairs in one tile", K, H, Hkv, D, m, weights)
     f = ctx()
     rng = np.random.default_rng(K + H + m)
