@@ -40,7 +40,8 @@ struct PanelDev {
     __half *out[3];
     uint32_t rows0, rows1, total_rows;  // of W_q, of W_k and W_v each, of all
     const __half *x, *gamma, *residual;
-    uint32_t k_dim, m, rows_per_wg, canonical, n_pass, inv_pass /* fa_inverse */;
+    uint32_t k_dim, m, rows_per_wg, canonical, n_pass;
+    uint32_t beside, inv_beside;  // workgroups of the same weight rows on one XCD, side by side, and fa_inverse of it; 0: along grid y
     float eps, inv_k, alpha, beta;
     RopeDev r;
     uint32_t scale_pairs;  // a row holds an even number of scales, 4-byte aligned

@@ -85,24 +85,25 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
-    const uint32_t inv_pass = RING ? a.inv_pass : 0;
+    constexpr bool BESIDE = NC == 1 && !FEW;  // (the branch in the others took 3 to 5 % of a short launch)
+    const uint32_t beside = BESIDE || RING ? a.beside : 0, inv_beside = BESIDE || RING ? a.inv_beside : 0;
     const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
     const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
     const uint32_t normal = a.r.normal, head_dim = a.r.head_dim, scale_pairs = a.scale_pairs;
     // (the launch's arguments in two trips through the scalar cache: what the first requests need, and the rest behind them)
     asm volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(rows0), "s"(rows1), "s"(total_rows), "s"(x_in), "s"(gamma), "s"(K), "s"(m_rows),
-                 "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass), "s"(inv_pass));
+                 "s"(rows_per_wg), "s"(canonical_u), "s"(n_pass));
+    if constexpr (BESIDE || RING) asm volatile("" ::"s"(beside), "s"(inv_beside));
     if constexpr (WB != 16) asm volatile("" ::"s"(sp0), "s"(sp1), "s"(sp2), "s"(scale_pairs));
     if constexpr (ROPE) asm volatile("" ::"s"(normal), "s"(head_dim));
     const bool canonical = canonical_u != 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, c = lane >> 4;
     const uint32_t nkb = K / 32, n_pieces = K / 8;
-    // RING: the workgroups of the passes of the same weight rows one after the other on one XCD
-    uint32_t along = blockIdx.x, first_pass = blockIdx.y;
-    if constexpr (RING) {
-        const uint32_t eighth = blockIdx.x >> 3, group = fa_quotient(eighth, n_pass, inv_pass);
-        along = group * 8 + (blockIdx.x & 7), first_pass = eighth - group * n_pass;
+    uint32_t along = blockIdx.x, first_pass = blockIdx.y, pass_step = gridDim.y;
+    if (RING || (BESIDE && beside)) {
+        const uint32_t eighth = blockIdx.x >> 3, group = fa_quotient(eighth, beside, inv_beside);
+        along = group * 8 + (blockIdx.x & 7), first_pass = eighth - group * beside, pass_step = beside;
     }
     const uint32_t row_begin = along * rows_per_wg;
     const uint32_t row_end = min(total_rows, row_begin + rows_per_wg);
@@ -282,7 +283,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     float *red = reinterpret_cast<float *>(smem + (APART ? NC * 16 * XROW : 0));  // [NW][NT][NC][16][17]; not APART: over the rows once they have been read
 
     while (true) {
-        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = RING ? n_pass : pass + gridDim.y;
+        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = RING ? n_pass : pass + pass_step;
         if (gamma) {  // x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16; a wave holds whole rows
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
@@ -499,6 +500,7 @@ fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32
     if constexpr (Q) {
         if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true, false>(scope, rope, pk, grid, a);
     }
+    if (nt == 3 && pk <= 4) return rope ? launch_one<WB, 3, 1, 4, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 4, false, false, false>(scope, grid, a);
     if (nt > 2) {  // (rows of more than 2048 features)
         if (nt == 3) return rope ? launch_one<WB, 3, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 6, false, false, false>(scope, grid, a);
         if (nt == 4) return rope ? launch_one<WB, 4, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 4, 1, 6, false, false, false>(scope, grid, a);

@@ -87,6 +87,18 @@ def test_long_rows_a_workgroup_for_each_pass(K, N, NK, m, layout, weights):
     test_chunk_in_one_launch(K, N, NK, m, layout, weights)
 
 
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,layout", [
+    (2048, 2056, 256, 40, 1),  # 34 weight rows to a workgroup: two rows in a third tile; three passes, the last of 8 rows
+    (2048, 2304, 384, 64, 0),  # three full tiles, four passes
+    (1056, 3000, 544, 17, 1),  # two tiles, a pass of one row
+    (640, 1504, 272, 33, 0),   # two tiles of short rows
+    (896, 1024, 128, 41, 1),   # one tile
+])
+def test_shorter_rows_a_workgroup_for_each_pass(K, N, NK, m, layout, weights):
+    test_chunk_in_one_launch(K, N, NK, m, layout, weights)
+
+
 def test_long_rows_in_five_tiles():
     test_chunk_in_one_launch(2592, 3840, 640, 64, 1, "f16")  # 80 weight rows to a workgroup, block-quantised as a GEMM
 
@@ -130,6 +142,8 @@ def test_rows_absent_from_a_pass(K, N, NK, m, weights):
     (3072, 24, 8, 128, 32),   # 20 pairs: 16 in two tiles, 4 in a third
     (2816, 24, 12, 128, 19),  # 24: the third is full
     (3072, 24, 8, 128, 40),   # 32 in four tiles
+    (2048, 16, 4, 128, 40),   # 20 of shorter rows
+    (1024, 14, 2, 64, 60),    # 9 in two tiles, four passes
 ])
 def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
     """Up to 16 weight rows per workgroup, and in the last of an odd number of tiles, both halves of NeoX pairs lie in one tile: the fused
