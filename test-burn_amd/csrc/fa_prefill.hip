@@ -1099,7 +1099,7 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     // chunk of at most 64 rows after a long prefix the memory-bound one (fa_chunk.hip), or the tiled one, by estimate. (The estimates are
     // of keys that come from memory, as a layer's do in a model: of long ones that do, the first kernel takes longer (us, rows and the
     // other: 278 rows after 7179, H24 / Hkv8 / D128 55.3, 48.6; 34 after 47550, H16 / Hkv2 / D128 47.3, 36.7; 18 after 44996, H4 / Hkv4 /
-    // D128 38.7, 24.1; the first of them 47 in turned orders, rows_turn), of keys that lie in the last-level cache from the call before the
+    // D128 38.7, 24.1; the first of them 47 in turned orders, RowsTurn), of keys that lie in the last-level cache from the call before the
     // least of all: where the first and the second are level, the first is a fifth ahead from a cache, 32 after 8160 17.1, 17.2 and 13.0, 16.1. On 4000
     // launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, half of them with keys in memory) the
     // choice takes 1.002 to 1.014 times as long as the best of the three, in the mean, and 0.69 to 0.76 of what the other two would: 48

@@ -16,7 +16,7 @@
 //     (at D 64 two stages per wave, which leave room for half as many waves, are 5 to 20 % slower);
 //   * the waves' sums meet once, in LDS, and a thread folds its (row, 4 dims) of all of them and writes the row out.
 //   * the blocks that read the same keys through one L2 begin at different ones of them, so that what the first to come asks of memory
-//     is there for the others, and they do not all ask one channel of the L2 at a time (rows_turn).
+//     is there for the others, and they do not all ask one channel of the L2 at a time (RowsTurn).
 // It reads a block's keys once per 32 rows, 131 KB/us and CU along the rows (fa_lds_dma.h), which is why long keys under many rows
 // stay with the tiled kernel (once per 128 rows): fa_prefill_rows_plan. us before and now (tiled or short-chunk kernel before):
 //   H14 / Hkv2 / D64:   32 rows after 500 10.7 -> 4.6; 500 after 1000 14.9 -> 7.5; 2048 rows 22.7 -> 16.2; 32 after 8160 21.0 -> 9.3
@@ -80,7 +80,7 @@ struct RowsDev {
 constexpr int KT = 32;  // keys per tile
 
 // POOL: 0 a contiguous cache, 1 paged, 2 paged with pools of 4 GiB or more (no 32-bit offsets)
-// TURN: the workgroups that read the same keys through one L2 begin at different ones (rows_turn)
+// TURN: the workgroups that read the same keys through one L2 begin at different ones (RowsTurn)
 template <int D, int NW, bool BF16, int POOL, bool TURN>
 __global__ void __launch_bounds__(NW * 64, D == 64 ? 4 : 2) flash_rows_kernel(RowsDev a_by_value) {
     static_assert(std::is_trivially_copyable<RowsDev>::value, "read as raw bytes from the argument block, where it is the first member");
@@ -403,15 +403,24 @@ static uint32_t mates_apart(uint32_t n_kv_heads) {
 //   H24 / Hkv8 / D128:  500 after 1000 20.5 -> 17.7; 187 after 1130 14.8 -> 12.5; 32 after 8160 18.3 -> 17.0; 68 after 13543 35.0 -> 30.6
 //   H32 / Hkv8 / D128:  194 after 2151 21.1 -> 16.9; H8 / Hkv8: 1928 after 1015 34.4 -> 27.8; H16 / Hkv2: 131 after 11517 34.5 -> 29.6
 //   D 64:  H32 / Hkv8, 1447 after 591 31.7 -> 27.7; H14 / Hkv2, 992 after 10818 64.8 -> 59.1
-static uint32_t rows_turn(const PrefillLaunch &L, uint32_t wgs, uint32_t n_blocks, uint32_t longest, float kv_mb, uint32_t waves, uint32_t splits) {
-    const uint32_t rounds = ceil_div_u32(ceil_div_u32(longest, splits), waves);
-    if (!(kv_mb > 4.0f || (wgs > 600 && rounds >= 8)) || (n_blocks - 1) >> mates_apart(L.n_kv_heads) == 0) return 0;
-    const uint32_t twos = L.n_kv_heads & (0u - L.n_kv_heads), streams = L.n_kv_heads / (twos < 8 ? twos : 8) * splits;
-    const uint32_t round_kb = waves * KT * L.head_dim * 4 / 1024;
-    uint32_t turn = 1;
-    while (turn < 32 && turn * 2 <= rounds && (uint64_t)turn * 2 * streams * round_kb <= 3100) turn *= 2;
-    return turn >= (L.head_dim == 128 ? 2u : 4u) ? turn : 0u;
-}
+struct RowsTurn {
+    uint32_t longest = 0, wgs = 0, xcd_heads_kb = 0;  // 0: in one order
+    bool large = false, wide = false;
+    RowsTurn(const PrefillLaunch &L, uint32_t wgs_, uint32_t n_blocks, uint32_t longest_, float kv_mb) : longest(longest_), wgs(wgs_), large(kv_mb > 4.0f), wide(L.head_dim == 128) {
+        if (!(large || wgs > 600) || (n_blocks - 1) >> mates_apart(L.n_kv_heads) == 0) return;
+        const uint32_t twos = L.n_kv_heads & (0u - L.n_kv_heads);
+        xcd_heads_kb = L.n_kv_heads / (twos < 8 ? twos : 8) * (KT * L.head_dim * 4 / 1024);  // of a tile for each wave of a stream
+    }
+    uint32_t operator()(uint32_t waves, uint32_t splits) const {
+        if (!xcd_heads_kb) return 0;
+        const uint32_t rounds = ceil_div_u32(ceil_div_u32(longest, splits), waves), held = 3100 / (xcd_heads_kb * waves * splits);
+        if (!large && rounds < 8) return 0;
+        uint32_t most = rounds < held ? rounds : held;
+        most = most < 32 ? most : 32;
+        const uint32_t turn = most ? 1u << (31 - __builtin_clz(most)) : 0u;
+        return turn >= (wide ? 2u : 4u) ? turn : 0u;
+    }
+};
 
 // How the kernel would be launched, and what that takes by estimate: fitted to 2664 shapes (2 to 8000 rows after 0 to 100000, 14
 // combinations of heads, each timed with every choice, with the tiled and with the short-chunk kernel, over as many layers' caches as
@@ -450,7 +459,8 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float r8 = (float)ceil_div_u32(longest, 8), r4 = (float)ceil_div_u32(longest, 4);
     const float head_mb = (float)longest * (float)(KT * L.head_dim) * 4e-6f, kv_mb = head_mb * (float)L.n_kv_heads;
     const bool waited = wgs <= n_cus && kv_mb > 9.0f;
-    const uint32_t turn8 = rows_turn(L, wgs, n_blocks, longest, kv_mb, 8, 1), turn4 = rows_turn(L, wgs, n_blocks, longest, kv_mb, 4, 1);
+    const RowsTurn turned(L, wgs, n_blocks, longest, kv_mb);
+    const uint32_t turn8 = turned(8, 1), turn4 = turned(4, 1);
     // (turned: 390 launches, 4 to 5 % rms)
     const float us8 = turn8 ? (wide ? 2.69f + larger(1.086f * r8, 3.11f * n + 0.122f * chain + 0.0135f * all) + (wgs <= n_cus ? 0.188f : 0.133f) * kv_mb
                                     : 3.48f + larger(0.583f * r8, 0.970f * n + 0.042f * chain + 0.0334f * all) + 0.359f * kv_mb)
@@ -468,7 +478,7 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float xcd_mb = head_mb * (float)(xcd_heads < xcd_blocks ? xcd_heads : xcd_blocks);
     for (uint32_t s = 2; s <= most && s * 4 <= longest && s <= 32; s = s == 16 ? 32 : s + 1) {
         const float r = (float)ceil_div_u32(ceil_div_u32(longest, s), 8), mb = (float)wgs * (float)(32 * L.head_dim) * (float)s * 4e-6f;
-        const uint32_t turn = rows_turn(L, wgs, n_blocks, longest, kv_mb, 8, s);
+        const uint32_t turn = turned(8, s);
         const float us = turn ? (wide ? 6.99f + 1.183f * r + 0.0149f * (float)s + 0.3715f * mb + 0.0674f * kv_mb + 0.507f * xcd_mb
                                       : 6.28f + 0.674f * r + 0.0385f * (float)s + 0.4104f * mb + 0.0761f * kv_mb + 0.337f * xcd_mb)
                          : wide ? 5.77f + 1.464f * r + 0.0768f * (float)s + 0.549f * mb + 0.0547f * kv_mb + 0.35f * xcd_mb
