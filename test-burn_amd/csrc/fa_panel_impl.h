@@ -52,10 +52,10 @@ struct Weights<4> {
 // What a lane reads in the place of an F16 weight block past the row's last.
 static __device__ const h8_t zero_weights = {0, 0, 0, 0, 0, 0, 0, 0};
 
-// FEW: at most 8 input rows, one per wave: the other half of the 16 columns is not loaded, normalised or stored. (8 rows, two per
+// FEW: at most 8 input rows, in the launch or (EIGHTS) to a workgroup, those of the same weight rows side by side, one per wave: the other half of the 16 columns is not loaded, normalised or stored. (8 rows, two per
 // wave -> one: QKV with its norm, 5120 x 3072 F16 10.1 -> 9.3 us, Q8_0 10.1 -> 9.0, Q4_0 10.0 -> 8.3; 1152 x 896 F16 4.8 -> 4.4;
 // 3072 x 3072 without a norm 6.5 -> 5.8, 6.0 -> 5.5, 6.4 -> 5.1.)
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW>
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS>
 __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     static_assert(std::is_trivially_copyable<PanelDev>::value, "read as raw bytes from the argument block, where it is the first member");
@@ -65,6 +65,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     typedef typename W::raw_t raw_t;
     constexpr int XROW = row_bytes<PK>(), NR = FEW ? 1 : 2 * NC, NB = 2 * PK;
     static_assert(!FEW || NC == 1, "one group of input rows");
+    constexpr uint32_t PASS = FEW ? 8 : NC * 16;  // input rows of a pass
     constexpr bool WIDE = WB != 16 && !SUMS, TURN = TURNS<WB, PK, SUMS>;
     constexpr int GB = !WIDE && !TURN ? 1 : WB == 8 ? 2 : 4, NQ = NB / GB;  // blocks per request, requests per tile
     typedef typename std::conditional<WIDE || TURN, u4v_t, raw_t>::type req_t;
@@ -85,7 +86,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
-    constexpr bool BESIDE = NC == 1 && !FEW;  // (the branch in the others took 3 to 5 % of a short launch)
+    constexpr bool BESIDE = NC == 1 && (!FEW || EIGHTS);  // (the branch in the others takes 3 to 5 % of a short launch)
     const uint32_t beside = BESIDE || RING ? a.beside : 0, inv_beside = BESIDE || RING ? a.inv_beside : 0;
     const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
     const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
@@ -140,8 +141,8 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     auto request_rows = [&](uint32_t pass, bool first) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-            if (i > (first ? 1 : 0) && pass * (NC * 16u) + 8u * i >= m_rows) break;  // (uniform: no such rows in the pass; the first one is not waited for)
-            const __half *row = x_in + (size_t)min(pass * (NC * 16u) + (uint32_t)wave + 8u * i, m_rows - 1u) * K;
+            if (i > (first ? 1 : 0) && pass * PASS + 8u * i >= m_rows) break;  // (uniform: no such rows in the pass; the first one is not waited for)
+            const __half *row = x_in + (size_t)min(pass * PASS + (uint32_t)wave + 8u * i, m_rows - 1u) * K;
 #pragma unroll
             for (int j = 0; j < PK; ++j) xr[i][j] = *reinterpret_cast<const h8_t *>(row + min((uint32_t)(j * 64 + lane), n_pieces - 1u) * 8u);
         }
@@ -283,7 +284,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     float *red = reinterpret_cast<float *>(smem + (APART ? NC * 16 * XROW : 0));  // [NW][NT][NC][16][17]; not APART: over the rows once they have been read
 
     while (true) {
-        const uint32_t m0 = pass * (NC * 16u), cols = min(NC * 16u, m_rows - m0), next = RING ? n_pass : pass + pass_step;
+        const uint32_t m0 = pass * PASS, cols = min(PASS, m_rows - m0), next = RING ? n_pass : pass + pass_step;
         if (gamma) {  // x * rsqrt(mean(x^2) + eps) * gamma in f32, rounded to f16; a wave holds whole rows
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
@@ -475,16 +476,16 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     }
 }
 
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW>
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS = false>
 fa_status launch_one(FaLaunchScope &scope, dim3 grid, const PanelDev &a) {
     constexpr int lds = lds_bytes<WB, NT, NC, PK, SUMS>();
     static std::atomic<uint64_t> allowed{0};  // devices this kernel's LDS size has been asked for on (the calls are idempotent)
     const uint64_t bit = 1ull << (scope.ctx->device & 63);
     if (!(allowed.load(std::memory_order_acquire) & bit)) {
-        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         allowed.fetch_or(bit, std::memory_order_release);
     }
-    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW>, grid, dim3(NTHREADS), lds, a);
+    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS>, grid, dim3(NTHREADS), lds, a);
     return FA_OK;
 }
 template <int WB, int NT, int NC, bool SUMS, bool FEW>
@@ -493,10 +494,21 @@ fa_status launch_pk(FaLaunchScope &scope, bool rope, uint32_t pk, dim3 grid, con
     if (NC == 2 || pk <= 4) return rope ? launch_one<WB, NT, NC, 4, true, SUMS, FEW>(scope, grid, a) : launch_one<WB, NT, NC, 4, false, SUMS, FEW>(scope, grid, a);
     return rope ? launch_one<WB, NT, 1, 6, true, SUMS, FEW>(scope, grid, a) : launch_one<WB, NT, 1, 6, false, SUMS, FEW>(scope, grid, a);  // (16 rows per pass: registers)
 }
+template <int WB, int NT, bool SUMS>
+fa_status launch_eights(FaLaunchScope &scope, bool rope, uint32_t pk, dim3 grid, const PanelDev &a) {  // (rows of up to 2048 features)
+    if (pk <= 2) return rope ? launch_one<WB, NT, 1, 2, true, SUMS, true, true>(scope, grid, a) : launch_one<WB, NT, 1, 2, false, SUMS, true, true>(scope, grid, a);
+    return rope ? launch_one<WB, NT, 1, 4, true, SUMS, true, true>(scope, grid, a) : launch_one<WB, NT, 1, 4, false, SUMS, true, true>(scope, grid, a);
+}
 template <int WB>
-fa_status launch(FaLaunchScope &scope, bool rope, bool sums, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a) {
+fa_status launch(FaLaunchScope &scope, bool rope, bool sums, bool eights, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a) {
     constexpr bool Q = WB != 16;  // (block-quantised weights have per-block sums wherever there are as few rows)
     if (a.m <= 8 && (!Q || sums)) return nt == 1 ? launch_pk<WB, 1, 1, Q, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, Q, true>(scope, rope, pk, grid, a);
+    if (eights) {
+        if constexpr (Q) {
+            if (sums) return nt == 1 ? launch_eights<WB, 1, true>(scope, rope, pk, grid, a) : launch_eights<WB, 2, true>(scope, rope, pk, grid, a);
+        }
+        return nt == 1 ? launch_eights<WB, 1, false>(scope, rope, pk, grid, a) : launch_eights<WB, 2, false>(scope, rope, pk, grid, a);
+    }
     if constexpr (Q) {
         if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true, false>(scope, rope, pk, grid, a);
     }

@@ -376,6 +376,7 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 // of input rows per pass, weight rows per workgroup, workgroups along the passes.
 struct PanelPlan {
     uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y, rounds;
+    bool eights = false;  // passes of 8 input rows
     uint32_t beside;  // grid_y where the workgroups of the same weight rows lie side by side on an XCD, else 0
 };
 static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope) {
@@ -407,18 +408,18 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
     // 5120 x 3072, 32 rows, F16 14.5 -> 11.5 us, Q8_0 14.3 -> 10.7, Q4_0 13.7 -> 10.6; 64 rows F16 19.3 -> 15.5; o_proj of 3072 x 3072,
     // 32 rows F16 8.1 -> 7.4, 48 rows 10.0 -> 7.7, Q8_0 10.0 -> 7.5.) The workgroups of the same weight rows are next to each other on an
     // XCD, so that memory is read once.
-    // Shorter rows of 17 to 64 input rows likewise, 16 to a workgroup instead of 32, while up to two tiles of weight rows (three of more than
+    // Shorter rows of 17 to 64 input rows (96 with a gamma, of up to 1024 features) likewise, 16 to a workgroup instead of 32, while up to two tiles of weight rows (three of more than
     // 1024 features) reach: half of the norm, which every workgroup works out for itself, for twice the weight rows. With a gamma always -
     // 32 rows of 1152 x 896 F16 5.4 -> 4.4 us, Q8_0 5.6 -> 4.5, of 2560 x 2048 8.3 -> 7.5, 8.1 -> 7.3, 48 rows 9.3 -> 7.8, 9.1 -> 7.1, 64 rows
-    // 9.6 -> 8.7, 9.2 -> 8.2; but for the rotation of Q8_0 in two tiles of two pieces, 5.25 -> 5.46 -, without one where one tile reaches or the
+    // 9.6 -> 8.7, 9.2 -> 8.2, 80 rows of 1152 x 896 F16 5.4 -> 5.0; but for the rotation of Q8_0 in two tiles of two pieces, 5.25 -> 5.46 -, without one where one tile reaches or the
     // other way has more than one round of passes: 32 rows of 896 x 896 F16 4.1 -> 3.4, of 2048 x 2048 5.9 -> 5.0, Q8_0 5.5 -> 4.5, 45 rows of 2240
     // x 2048 Q4_0 6.3 -> 5.3; beyond the lines 27 rows of 2688 x 2048 Q4_0 5.2 -> 5.4, 39 of 2048 x 2048 4.6 -> 5.4.
     const uint32_t passes = ceil_div_u32(l.m, 16);
     const bool wide = p.pk > 4;
-    if (passes > 1 && (wide || passes <= 4)) {
+    if (passes > 1 && (wide || passes <= (l.gamma && p.pk <= 2 ? 6u : 4u))) {
         const uint32_t groups = n_cus / (8 * passes) * 8, rows = (ceil_div_u32(total_rows, groups ? groups : 8) + 1) & ~1u;
         const uint32_t most = wide ? 80u /* five tiles: registers */ : p.pk > 2 ? 48u : 32u;
-        const bool ahead = l.gamma ? !(rope && l.weight_bits == 8 && p.pk <= 2 && rows > 16 && passes == 4)
+        const bool ahead = l.gamma ? !(rope && l.weight_bits == 8 && p.pk <= 2 && rows > 16 && passes >= 4)
                                    : rows <= 16 || (passes == 3 ? total_rows > 8 * n_cus && rows <= 40 : rows > 32);
         if (wide || (rows <= most && ahead)) {
             p.nc = 1, p.n_pass = passes, p.rows_per_wg = rows < most ? rows : most, p.nt = ceil_div_u32(p.rows_per_wg, 16);
@@ -426,7 +427,19 @@ static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rop
             p.rounds = ceil_div_u32(ceil_div_u32(p.grid_x, 8) * 8 * passes, n_cus);
         }
     }
-    p.beside = wide || (p.nc == 1 && p.grid_y == passes && passes > 1) ? p.n_pass : 0;
+    // 9 to 24 rows of up to 2048 features: 8 to a workgroup where that takes no more tiles of weight rows - with a gamma, or 9 to 16 rows
+    // (F16: of up to 1024 features). us, 16 rows to a workgroup -> 8: 1152 x 896 with a gamma 16 rows F16 4.3 -> 3.9, Q8_0 4.4 -> 4.1, 24 rows
+    // 4.3 -> 3.7, Q4_0 4.5 -> 3.8; 2560 x 2048 24 rows F16 7.4 -> 7.0, Q8_0 7.2 -> 6.3, Q4_0 7.0 -> 6.0; without one 2048 x 2048 16 rows Q4_0 4.4 ->
+    // 4.0, 896 x 896 F16 3.4 -> 3.25. With a tile more 16 rows of 2560 x 2048 F16 6.3 -> 6.6, without a gamma 24 rows of 2048 x 2048 4.9 -> 5.9.
+    const uint32_t eights = ceil_div_u32(l.m, 8);
+    if (!wide && p.nc == 1 && (eights == 2 || (eights == 3 && l.gamma)) && (l.gamma || p.pk <= 2 || l.weight_bits != 16)) {
+        const uint32_t groups = n_cus / (8 * eights) * 8, rows = (ceil_div_u32(total_rows, groups ? groups : 8) + 1) & ~1u;
+        if (rows <= 16 * p.nt) {
+            p.eights = true, p.n_pass = p.grid_y = eights, p.rows_per_wg = rows, p.grid_x = ceil_div_u32(total_rows, rows), p.rounds = 1;
+            p.nt = ceil_div_u32(rows, 16);
+        }
+    }
+    p.beside = wide || (p.nc == 1 && p.n_pass > 1 && p.grid_y == p.n_pass) ? p.n_pass : 0;
     return p;
 }
 
@@ -517,9 +530,9 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
     FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
     const bool sums = l.m < FA_GEMM_MIN_M_DEFAULT;  // (of interest to block-quantised weights only: the arithmetic, see fa_panel.h)
     const dim3 grid = p.beside ? dim3(ceil_div_u32(p.grid_x, 8) * 8 * p.beside) : dim3(p.grid_x, p.grid_y);
-    if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
-    else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
-    else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.nt, p.nc, p.pk, grid, a));
+    if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
+    else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
+    else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
     return scope.finish();
 }
 

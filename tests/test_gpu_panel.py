@@ -99,6 +99,19 @@ def test_shorter_rows_a_workgroup_for_each_pass(K, N, NK, m, layout, weights):
     test_chunk_in_one_launch(K, N, NK, m, layout, weights)
 
 
+@pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
+@pytest.mark.parametrize("K,N,NK,m,layout", [
+    (96, 776, 40, 9, 1),       # 8 input rows to a workgroup: a second pass of one row; the weight stream's arithmetic of block-quantised weights
+    (896, 896, 128, 16, 0),    # two full passes
+    (2048, 1800, 120, 11, 1),  # longer rows, 16 weight rows to a workgroup
+    (2048, 2048, 264, 17, 0),  # three passes of two tiles with the norm, two of 16 rows without
+    (1056, 1000, 136, 23, 1),  # three, the last of 7 rows
+    (640, 1200, 40, 90, 1),    # six passes of 16
+])
+def test_passes_of_8_rows(K, N, NK, m, layout, weights):
+    test_chunk_in_one_launch(K, N, NK, m, layout, weights)
+
+
 def test_long_rows_in_five_tiles():
     test_chunk_in_one_launch(2592, 3840, 640, 64, 1, "f16")  # 80 weight rows to a workgroup, block-quantised as a GEMM
 
@@ -144,6 +157,8 @@ def test_rows_absent_from_a_pass(K, N, NK, m, weights):
     (3072, 24, 8, 128, 40),   # 32 in four tiles
     (2048, 16, 4, 128, 40),   # 20 of shorter rows
     (1024, 14, 2, 64, 60),    # 9 in two tiles, four passes
+    (896, 14, 2, 64, 13),     # 5, passes of 8 rows
+    (2048, 16, 2, 128, 24),   # 16 in two tiles, passes of 8 rows
 ])
 def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
     """Up to 16 weight rows per workgroup, and in the last of an odd number of tiles, both halves of NeoX pairs lie in one tile: the fused
