@@ -28,6 +28,7 @@
 
 #include "fa_internal.h"
 #include "fa_norm.h"
+#include "fa_panel_plan.h"
 #include "fa_qkv_rope.h"
 
 namespace fa_panel {
@@ -57,8 +58,6 @@ template <int PK>
 constexpr bool G_IN_LDS = PK > 4;  // the longest rows: the norm's weights in LDS instead of registers
 template <int PK>
 constexpr int LDS_SHARE = (PK <= 2 ? 80 * 1024 : 160 * 1024) - 6 * 1024;  // two workgroups per compute unit, or one; less the scales
-// Two workgroups per compute unit: rows of up to 1024 features, except where the registers do not allow it.
-constexpr bool two_per_cu(uint32_t nt, uint32_t nc, uint32_t pk, bool rope) { return pk <= 2 && !(rope && nt == 2 && nc == 2); }
 // Block-quantised weights: their scales as f16 [block][slot], with 8 bytes between blocks: a wave writes the blocks of two or three
 // rows side by side, all of them to one bank without (o_proj of 1536 features x 4096 rows, 40 input rows: Q8_0 7.06 -> 6.64 us).
 template <int NT>

@@ -372,75 +372,9 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 
 }  // namespace
 
-// How a FusedQkv / MatMul launch runs on the panel kernel (fa_panel.h): 16-row tiles of weight rows per workgroup, 16-row groups
-// of input rows per pass, weight rows per workgroup, workgroups along the passes.
-struct PanelPlan {
-    uint32_t nt, nc, pk, rows_per_wg, n_pass, grid_x, grid_y, rounds;
-    bool eights = false;  // passes of 8 input rows
-    uint32_t beside;  // grid_y where the workgroups of the same weight rows lie side by side on an XCD, else 0
-};
-static PanelPlan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope) {
-    PanelPlan p;
-    const uint32_t total_rows = l.n_dim + 2 * l.n_kv;
-    p.pk = ceil_div_u32(l.k_dim, 512), p.nc = l.m <= 16 || p.pk > 4 ? 1u : 2u, p.n_pass = ceil_div_u32(l.m, 16 * p.nc);
-    // Weight rows per workgroup: what a pass costs is mostly its input rows, whatever the weight rows, so as few passes as
-    // possible on a compute unit - one after the other or, in two workgroups, side by side (Qwen2.5-0.5B, 64 rows: o_proj as 448
-    // workgroups of 4 weight rows 5.2 us, as 112 of 16 3.9); of equal choices the fewest weight rows. A second tile of weight rows
-    // costs a fifth of a pass, four fifths where the rows of F16 and Q8_0 weights are K apart and nothing is normalised (180 rows,
-    // 896 x 896: 4.9 us as 336 workgroups of 16, 5.1 as 168 of 32), and a pass with its norm a fifth more beside another.
+static fa_panel::Plan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope) {
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    uint64_t best = ~0ull;
-    const uint32_t least = ceil_div_u32(total_rows, n_cus) < 32 ? (ceil_div_u32(total_rows, n_cus) + 1) & ~1u : 32u;
-    for (uint32_t rpw : {least, 16u, 32u}) {
-        const uint32_t gx = ceil_div_u32(total_rows, rpw), nt = rpw > 16 ? 2u : 1u;
-        const bool two = fa_panel::two_per_cu(nt, p.nc, p.pk, rope);
-        const uint32_t slots = two ? 2 * n_cus : n_cus;
-        uint32_t gy = slots / gx;
-        gy = gy < 1 ? 1u : gy > p.n_pass ? p.n_pass : gy;
-        const uint32_t load = two ? std::max(gx * gy, n_cus) : ceil_div_u32(gx * gy, n_cus) * n_cus;
-        const uint32_t tiles = nt == 1 ? 50u : !l.canonical && l.weight_bits != 4 && !l.gamma ? 90u : 60u;
-        const uint32_t beside = two && gx * gy > n_cus && l.gamma ? 12u : 10u;
-        const uint64_t cost = (uint64_t)load * ceil_div_u32(p.n_pass, gy) * tiles * beside;
-        if (cost < best) best = cost, p.nt = nt, p.rows_per_wg = rpw, p.grid_x = gx, p.grid_y = gy, p.rounds = ceil_div_u32(gx * gy, slots);
-    }
-    // Rows of more than 2048 features: a workgroup per pass, with as many weight rows as put all of them in one round of workgroups. (One
-    // workgroup for both passes, 20 weight rows: the second pass's rows are asked for, normalised and multiplied behind the first's. FusedQkv of
-    // 5120 x 3072, 32 rows, F16 14.5 -> 11.5 us, Q8_0 14.3 -> 10.7, Q4_0 13.7 -> 10.6; 64 rows F16 19.3 -> 15.5; o_proj of 3072 x 3072,
-    // 32 rows F16 8.1 -> 7.4, 48 rows 10.0 -> 7.7, Q8_0 10.0 -> 7.5.) The workgroups of the same weight rows are next to each other on an
-    // XCD, so that memory is read once.
-    // Shorter rows of 17 to 64 input rows (96 with a gamma, of up to 1024 features) likewise, 16 to a workgroup instead of 32, while up to two tiles of weight rows (three of more than
-    // 1024 features) reach: half of the norm, which every workgroup works out for itself, for twice the weight rows. With a gamma always -
-    // 32 rows of 1152 x 896 F16 5.4 -> 4.4 us, Q8_0 5.6 -> 4.5, of 2560 x 2048 8.3 -> 7.5, 8.1 -> 7.3, 48 rows 9.3 -> 7.8, 9.1 -> 7.1, 64 rows
-    // 9.6 -> 8.7, 9.2 -> 8.2, 80 rows of 1152 x 896 F16 5.4 -> 5.0; but for the rotation of Q8_0 in two tiles of two pieces, 5.25 -> 5.46 -, without one where one tile reaches or the
-    // other way has more than one round of passes: 32 rows of 896 x 896 F16 4.1 -> 3.4, of 2048 x 2048 5.9 -> 5.0, Q8_0 5.5 -> 4.5, 45 rows of 2240
-    // x 2048 Q4_0 6.3 -> 5.3; beyond the lines 27 rows of 2688 x 2048 Q4_0 5.2 -> 5.4, 39 of 2048 x 2048 4.6 -> 5.4.
-    const uint32_t passes = ceil_div_u32(l.m, 16);
-    const bool wide = p.pk > 4;
-    if (passes > 1 && (wide || passes <= (l.gamma && p.pk <= 2 ? 6u : 4u))) {
-        const uint32_t groups = n_cus / (8 * passes) * 8, rows = (ceil_div_u32(total_rows, groups ? groups : 8) + 1) & ~1u;
-        const uint32_t most = wide ? 80u /* five tiles: registers */ : p.pk > 2 ? 48u : 32u;
-        const bool ahead = l.gamma ? !(rope && l.weight_bits == 8 && p.pk <= 2 && rows > 16 && passes >= 4)
-                                   : rows <= 16 || (passes == 3 ? total_rows > 8 * n_cus && rows <= 40 : rows > 32);
-        if (wide || (rows <= most && ahead)) {
-            p.nc = 1, p.n_pass = passes, p.rows_per_wg = rows < most ? rows : most, p.nt = ceil_div_u32(p.rows_per_wg, 16);
-            p.grid_x = ceil_div_u32(total_rows, p.rows_per_wg), p.grid_y = passes;
-            p.rounds = ceil_div_u32(ceil_div_u32(p.grid_x, 8) * 8 * passes, n_cus);
-        }
-    }
-    // 9 to 24 rows of up to 2048 features: 8 to a workgroup where that takes no more tiles of weight rows - with a gamma, or 9 to 16 rows
-    // (F16: of up to 1024 features). us, 16 rows to a workgroup -> 8: 1152 x 896 with a gamma 16 rows F16 4.3 -> 3.9, Q8_0 4.4 -> 4.1, 24 rows
-    // 4.3 -> 3.7, Q4_0 4.5 -> 3.8; 2560 x 2048 24 rows F16 7.4 -> 7.0, Q8_0 7.2 -> 6.3, Q4_0 7.0 -> 6.0; without one 2048 x 2048 16 rows Q4_0 4.4 ->
-    // 4.0, 896 x 896 F16 3.4 -> 3.25. With a tile more 16 rows of 2560 x 2048 F16 6.3 -> 6.6, without a gamma 24 rows of 2048 x 2048 4.9 -> 5.9.
-    const uint32_t eights = ceil_div_u32(l.m, 8);
-    if (!wide && p.nc == 1 && (eights == 2 || (eights == 3 && l.gamma)) && (l.gamma || p.pk <= 2 || l.weight_bits != 16)) {
-        const uint32_t groups = n_cus / (8 * eights) * 8, rows = (ceil_div_u32(total_rows, groups ? groups : 8) + 1) & ~1u;
-        if (rows <= 16 * p.nt) {
-            p.eights = true, p.n_pass = p.grid_y = eights, p.rows_per_wg = rows, p.grid_x = ceil_div_u32(total_rows, rows), p.rounds = 1;
-            p.nt = ceil_div_u32(rows, 16);
-        }
-    }
-    p.beside = wide || (p.nc == 1 && p.n_pass > 1 && p.grid_y == p.n_pass) ? p.n_pass : 0;
-    return p;
+    return fa_panel::panel_plan({l.n_dim + 2 * l.n_kv, l.k_dim, l.m, (uint32_t)l.weight_bits, l.canonical, l.gamma != nullptr, rope}, n_cus);
 }
 
 // Whether a FusedQkv / MatMul launch goes to the panel kernel: rows of up to 3072 features, from two input rows (four layers of the
@@ -467,7 +401,7 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
     if (l.m < FA_GEMM_MIN_M_DEFAULT) return true;
-    const PanelPlan p = panel_plan(ctx, l, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
+    const fa_panel::Plan p = panel_plan(ctx, l, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
     if (l.m <= 32 && p.rounds == 1 && l.n_dim + 2 * l.n_kv <= 32 * n_cus) return true;
     // More than 2048 features: a workgroup has one pass, with the weight rows that put all passes in one round (up to 80). Never behind
@@ -522,7 +456,7 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
         d.table_rows = r.table_rows, d.normal = r.rope_normal ? 1u : 0u, d.apply = r.apply_rope ? 1u : 0u;
         a.block_shift = (d.block_size & (d.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(d.block_size) : 32u;
     }
-    const PanelPlan p = panel_plan(ctx, l, rope != nullptr);
+    const fa_panel::Plan p = panel_plan(ctx, l, rope != nullptr);
     a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass, a.beside = p.beside, a.inv_beside = p.beside ? fa_inverse(p.beside) : 0;
     a.scale_pairs = l.k_dim / 32 % 2 == 0 ? 1u : 0u;
     for (int i = 0; i < 3; ++i)
@@ -530,6 +464,8 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
     FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
     const bool sums = l.m < FA_GEMM_MIN_M_DEFAULT;  // (of interest to block-quantised weights only: the arithmetic, see fa_panel.h)
     const dim3 grid = p.beside ? dim3(ceil_div_u32(p.grid_x, 8) * 8 * p.beside) : dim3(p.grid_x, p.grid_y);
+    if (!fa_panel::has_kernel({a.total_rows, l.k_dim, l.m, (uint32_t)l.weight_bits, l.canonical, l.gamma != nullptr, rope != nullptr}, p))
+        return fa_fail(FA_ERR_INVALID_OPERATION, "panel kernel: no form of %u tiles x %u groups for rows of %u features", p.nt, p.nc, l.k_dim);
     if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
     else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
     else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
@@ -561,6 +497,7 @@ fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_
     // gamma, this kernel against the GEMM (norm kernel, split-K GEMM, finish kernel): m = 4: 10.4 / 16.7 us, m = 10:
     // 13.8 / 16.9, m = 12 (from where only one workgroup's input rows fit a CU's LDS): 18.8 / 17.0, m = 16: 19.7 / 17.5,
     // m = 24 (two passes): 35.1 / 18.2.
+    static_assert(fa_panel::BLOCK_SUMS_BELOW == FA_GEMM_MIN_M_DEFAULT, "the panel kernel follows the weight stream's arithmetic below the GEMM's");
     constexpr uint32_t GEMM_MIN_M_DEFAULT = FA_GEMM_MIN_M_DEFAULT;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const bool gemm_ok = l.k_dim % (q8 ? 32 : 8) == 0 && aligned16(l.x) && aligned16(l.w[0]) && aligned16(l.w[1]) &&
