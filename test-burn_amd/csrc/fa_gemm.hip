@@ -573,7 +573,7 @@ static float divided_us(const FusedQkvLaunch &l, const Division &d, uint32_t n_c
 
 // What the tile kernels ask of the features, the weight rows and the scales: whole steps of 64 features, whole 16-byte stores, pairs of
 // scales.
-static bool tiles_fit(const FusedQkvLaunch &l) {
+bool fa_gemm_tiles_fit(const FusedQkvLaunch &l) {
     for (int i = 0; i < 3; ++i)
         if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) return false;
     return l.k_dim % 64 == 0 && l.n_dim % 8 == 0 && l.n_kv % 8 == 0 && (l.weight_bits == 16 || l.k_dim <= 16384);
@@ -583,14 +583,14 @@ float fa_gemm_estimate_us(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u, rows[3] = {l.n_dim, l.n_kv, l.n_kv};
     const float divided = divided_us(l, divide(l, n_cus, false), n_cus);
     fa_tile::TileShape shape;
-    return tiles_fit(l) ? std::min(divided, tile_us(l, best_tile(l, rows, n_cus, false, 0, shape))) : divided;
+    return fa_gemm_tiles_fit(l) ? std::min(divided, tile_us(l, best_tile(l, rows, n_cus, false, 0, shape))) : divided;
 }
 
 // Whether the tile kernels (fa_tile.h) take a launch, and with which tile: whole steps of 64 features, whole 16-byte stores, operands
 // below 2 GiB (32-bit offsets).
 static bool choose_tile(const fa_ctx *ctx, const FusedQkvLaunch &l, GemmDev &a, uint32_t n_cus, fa_tile::TileShape &shape) {
     const uint64_t max_rows = std::max(a.rows[0], a.rows[1]);
-    if (!tiles_fit(l) || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
+    if (!fa_gemm_tiles_fit(l) || !a.vec_store || (uint64_t)l.m * l.k_dim * 2 >= 0x7fffffffull || max_rows * l.k_dim * 2 >= 0x7fffffffull) return false;
     const bool joined = l.weight_bits == 16 && a.rows[0] % 32 == 0 && a.rows[1] % 32 == 0;
     const float cost = best_tile(l, a.rows, n_cus, joined, ctx->gemm_variant, shape);
     if (cost == 0.0f) return false;

@@ -321,6 +321,7 @@ struct FusedQkvLaunch {
 fa_status fa_launch_fused_qkv(fa_ctx *ctx, const FusedQkvLaunch &l, bool weight_stream_only = false);
 fa_status fa_launch_fused_qkv_gemm(fa_ctx *ctx, const FusedQkvLaunch &l);  // fa_gemm.hip: many input rows
 float fa_gemm_estimate_us(const fa_ctx *ctx, const FusedQkvLaunch &l);     // ... and what that would take, norm included
+bool fa_gemm_tiles_fit(const FusedQkvLaunch &l);  // whether its tile kernels can take the launch
 fa_status fa_launch_gemv_row(fa_ctx *ctx, const FusedQkvLaunch &l, bool *taken);  // fa_gemv.hip: one input row
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l);       // fa_qkv.hip: a chunk that the one-launch kernel for short chunks (fa_panel.h) takes
 

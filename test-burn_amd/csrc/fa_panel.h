@@ -81,8 +81,8 @@ constexpr int turn_at() { return (lds_rows_bytes<NT, NC, PK>() + (G_IN_LDS<PK> ?
 template <int WB, int NT, int NC, int PK, bool SUMS>
 constexpr int lds_bytes() { return turn_at<WB, NT, NC, PK>() + (TURNS<WB, PK, SUMS> ? NW * 1024 : 0); }
 
-// launchers per weight width (one translation unit each): eights = passes of 8 input rows, nt = 16-row tiles of weight rows, nc = 16-row groups of input rows per pass, pk = 512-feature pieces
+// launchers per weight width (one translation unit each)
 template <int WB>
-fa_status launch(FaLaunchScope &scope, bool rope, bool sums, bool eights, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a);
+fa_status launch(FaLaunchScope &scope, bool rope, bool sums, const Plan &plan, const PanelDev &a);
 
 }  // namespace fa_panel

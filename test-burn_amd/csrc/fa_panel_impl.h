@@ -55,7 +55,7 @@ static __device__ const h8_t zero_weights = {0, 0, 0, 0, 0, 0, 0, 0};
 // FEW: at most 8 input rows, in the launch or (EIGHTS) to a workgroup, those of the same weight rows side by side, one per wave: the other half of the 16 columns is not loaded, normalised or stored. (8 rows, two per
 // wave -> one: QKV with its norm, 5120 x 3072 F16 10.1 -> 9.3 us, Q8_0 10.1 -> 9.0, Q4_0 10.0 -> 8.3; 1152 x 896 F16 4.8 -> 4.4;
 // 3072 x 3072 without a norm 6.5 -> 5.8, 6.0 -> 5.5, 6.4 -> 5.1.)
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS>
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS, bool WALK>
 __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     static_assert(std::is_trivially_copyable<PanelDev>::value, "read as raw bytes from the argument block, where it is the first member");
@@ -75,18 +75,23 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     // of 3072 features: 4.9 us, one by one 5.1). All tiles' first requests come before any second one. FusedQkv of 5120 x 3072, all asked
     // for at once tile after tile -> this, us: F16 2 rows 9.7 -> 8.4, 16 rows 10.8 -> 9.7; Q8_0 9.1 -> 7.7, 11 rows 10.6 -> 9.2; Q4_0,
     // whose requests are few and all made at once, 8.7 -> 8.2.
-    constexpr bool RING = PK > 4, REST = RING && WB == 16 && NT == 1;
-    constexpr int NF = !RING || WB == 4 ? NQ : WB == 16 ? (NT <= 2 ? 8 : NT == 3 ? 6 : 4) : NT == 1 ? (NQ < 8 ? NQ : 8) : NT == 2 ? 4 : NT == 3 ? 3 : 2;
+    // WALK, of the longest rows: workgroups that go on to further passes keep all their weights. SPLIT: some of them, too, ask for a
+    // tile's other requests when the first pass's rows are in LDS (o_proj of 3072 x 3072 Q8_0 24 and 32 rows 7.1 -> 6.2 us).
+    static_assert(!WALK || PK > 4, "shorter rows have one kernel for both");
+    constexpr bool RING = PK > 4 && !WALK, SPLIT = WALK && (WB == 8 ? !ROPE || NT == 2 : WB == 16 && !ROPE && NT == 1);
+    constexpr bool REST = (RING && WB == 16 && NT == 1) || SPLIT;
+    constexpr int NF = SPLIT ? (NT == 1 ? (NQ < 8 ? NQ : 8) : 4)
+                       : !RING || WB == 4 ? NQ : WB == 16 ? (NT <= 2 ? 8 : NT == 3 ? 6 : 4) : NT == 1 ? (NQ < 8 ? NQ : 8) : NT == 2 ? 4 : NT == 3 ? 3 : 2;
     constexpr int NA = REST ? NQ : NF;  // places in registers
     // The order of the first requests is input rows, the norm's weights, scales, weights. Loads complete in the order in which they
     // are issued; left to itself the compiler puts the weights ahead of the rows in most of the kernels, and what is done with
     // the rows then waits for the whole weight stream. (m 12 .. 32, K 2048 .. 3072: o_proj 4 to 14 % less. With the longest rows and a
     // norm of two rows per wave the norm's chain is longer than the weights' stream, and the compiler's mixture is 1 to 3 % better.)
-    constexpr bool ORDERED = FEW || !ROPE || PK <= 4 || WB == 8 || NT > 2;
+    constexpr bool ORDERED = FEW || !ROPE || PK <= 4 || (WALK ? SPLIT : WB == 8 || NT > 2);
     const unsigned char *const w0 = a.w[0], *const w1 = a.w[1], *const w2 = a.w[2];
     const uint32_t rows0 = a.rows0, rows1 = a.rows1, total_rows = a.total_rows;
     const __half *const x_in = a.x, *const gamma = a.gamma;
-    constexpr bool BESIDE = NC == 1 && (!FEW || EIGHTS);  // (the branch in the others takes 3 to 5 % of a short launch)
+    constexpr bool BESIDE = NC == 1 && (!FEW || EIGHTS) && !WALK;  // (the branch in the others takes 3 to 5 % of a short launch)
     const uint32_t beside = BESIDE || RING ? a.beside : 0, inv_beside = BESIDE || RING ? a.inv_beside : 0;
     const uint32_t K = a.k_dim, m_rows = a.m, rows_per_wg = a.rows_per_wg, canonical_u = a.canonical, n_pass = a.n_pass;
     const __half *const sp0 = a.scales[0], *const sp1 = a.scales[1], *const sp2 = a.scales[2];
@@ -349,10 +354,14 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                     residual ? residual + (size_t)(m0 + min(w_col, cols - 1u)) * pick3(s_mat[t], rows0, rows1, rows1) + s_row[t] : x_in);
         }
         if constexpr (REST) {
-            __builtin_amdgcn_sched_barrier(0);
+            if (RING || pass == first_pass) {
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = NF; i < NQ; ++i) request_weights(0, i);
-            __builtin_amdgcn_sched_barrier(0);
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int i = NF; i < NQ; ++i) request_weights(t, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         if (!RING && next < n_pass) request_rows(next, false);
 #pragma unroll
@@ -476,16 +485,16 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     }
 }
 
-template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS = false>
+template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS = false, bool WALK = false>
 fa_status launch_one(FaLaunchScope &scope, dim3 grid, const PanelDev &a) {
     constexpr int lds = lds_bytes<WB, NT, NC, PK, SUMS>();
     static std::atomic<uint64_t> allowed{0};  // devices this kernel's LDS size has been asked for on (the calls are idempotent)
     const uint64_t bit = 1ull << (scope.ctx->device & 63);
     if (!(allowed.load(std::memory_order_acquire) & bit)) {
-        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        FA_HIP(hipFuncSetAttribute((const void *)panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS, WALK>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         allowed.fetch_or(bit, std::memory_order_release);
     }
-    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS>, grid, dim3(NTHREADS), lds, a);
+    scope.launch(panel_kernel<WB, NT, NC, PK, ROPE, SUMS, FEW, EIGHTS, WALK>, grid, dim3(NTHREADS), lds, a);
     return FA_OK;
 }
 template <int WB, int NT, int NC, bool SUMS, bool FEW>
@@ -499,11 +508,19 @@ fa_status launch_eights(FaLaunchScope &scope, bool rope, uint32_t pk, dim3 grid,
     if (pk <= 2) return rope ? launch_one<WB, NT, 1, 2, true, SUMS, true, true>(scope, grid, a) : launch_one<WB, NT, 1, 2, false, SUMS, true, true>(scope, grid, a);
     return rope ? launch_one<WB, NT, 1, 4, true, SUMS, true, true>(scope, grid, a) : launch_one<WB, NT, 1, 4, false, SUMS, true, true>(scope, grid, a);
 }
+template <int WB, int NT>
+fa_status launch_walk(FaLaunchScope &scope, bool rope, dim3 grid, const PanelDev &a) {  // (rows of more than 2048 features)
+    return rope ? launch_one<WB, NT, 1, 6, true, false, false, false, true>(scope, grid, a) : launch_one<WB, NT, 1, 6, false, false, false, false, true>(scope, grid, a);
+}
 template <int WB>
-fa_status launch(FaLaunchScope &scope, bool rope, bool sums, bool eights, uint32_t nt, uint32_t nc, uint32_t pk, dim3 grid, const PanelDev &a) {
+fa_status launch(FaLaunchScope &scope, bool rope, bool sums, const Plan &plan, const PanelDev &a) {
     constexpr bool Q = WB != 16;  // (block-quantised weights have per-block sums wherever there are as few rows)
+    const uint32_t nt = plan.nt, nc = plan.nc, pk = plan.pk;
+    if (!has_kernel(Shape{a.total_rows, a.k_dim, a.m, (uint32_t)WB, a.canonical != 0, a.gamma != nullptr, rope}, plan))
+        return fa_fail(FA_ERR_INVALID_OPERATION, "panel kernel: no form %d of %u tiles x %u groups for rows of %u features", (int)plan.form, nt, nc, a.k_dim);
+    const dim3 grid = plan.form == WALK ? dim3(plan.grid_x, plan.grid_y) : dim3(plan.workgroups());
     if (a.m <= 8 && (!Q || sums)) return nt == 1 ? launch_pk<WB, 1, 1, Q, true>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, Q, true>(scope, rope, pk, grid, a);
-    if (eights) {
+    if (plan.form == EIGHTS) {
         if constexpr (Q) {
             if (sums) return nt == 1 ? launch_eights<WB, 1, true>(scope, rope, pk, grid, a) : launch_eights<WB, 2, true>(scope, rope, pk, grid, a);
         }
@@ -512,12 +529,12 @@ fa_status launch(FaLaunchScope &scope, bool rope, bool sums, bool eights, uint32
     if constexpr (Q) {
         if (sums) return nt == 1 ? launch_pk<WB, 1, 1, true, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 1, true, false>(scope, rope, pk, grid, a);
     }
+    if (plan.form == WALK && pk > 4) return nt == 1 ? launch_walk<WB, 1>(scope, rope, grid, a) : launch_walk<WB, 2>(scope, rope, grid, a);
     if (nt == 3 && pk <= 4) return rope ? launch_one<WB, 3, 1, 4, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 4, false, false, false>(scope, grid, a);
-    if (nt > 2) {  // (rows of more than 2048 features)
-        if (nt == 3) return rope ? launch_one<WB, 3, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 6, false, false, false>(scope, grid, a);
-        if (nt == 4) return rope ? launch_one<WB, 4, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 4, 1, 6, false, false, false>(scope, grid, a);
-        if constexpr (!Q) return rope ? launch_one<WB, 5, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 5, 1, 6, false, false, false>(scope, grid, a);
-        return fa_fail(FA_ERR_INVALID_OPERATION, "panel kernel: %u tiles of block-quantised weight rows", nt);
+    if (nt == 3) return rope ? launch_one<WB, 3, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 3, 1, 6, false, false, false>(scope, grid, a);
+    if (nt == 4) return rope ? launch_one<WB, 4, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 4, 1, 6, false, false, false>(scope, grid, a);
+    if constexpr (!Q) {
+        if (nt == 5) return rope ? launch_one<WB, 5, 1, 6, true, false, false>(scope, grid, a) : launch_one<WB, 5, 1, 6, false, false, false>(scope, grid, a);
     }
     if (nt == 1) return nc == 1 ? launch_pk<WB, 1, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 1, 2, false, false>(scope, rope, pk, grid, a);
     return nc == 1 ? launch_pk<WB, 2, 1, false, false>(scope, rope, pk, grid, a) : launch_pk<WB, 2, 2, false, false>(scope, rope, pk, grid, a);

@@ -1,4 +1,4 @@
 // Panel kernels for 8-bit weights.
 #include "fa_panel_impl.h"
 
-template fa_status fa_panel::launch<8>(FaLaunchScope &, bool, bool, bool, uint32_t, uint32_t, uint32_t, dim3, const PanelDev &);
+template fa_status fa_panel::launch<8>(FaLaunchScope &, bool, bool, const Plan &, const PanelDev &);

@@ -372,9 +372,8 @@ __global__ void __launch_bounds__(QKV_NT, 2) fused_qkv_kernel(QkvDev a_by_value)
 
 }  // namespace
 
-static fa_panel::Plan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, bool rope) {
-    const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    return fa_panel::panel_plan({l.n_dim + 2 * l.n_kv, l.k_dim, l.m, (uint32_t)l.weight_bits, l.canonical, l.gamma != nullptr, rope}, n_cus);
+static fa_panel::Shape panel_shape(const FusedQkvLaunch &l, bool rope) {
+    return {l.n_dim + 2 * l.n_kv, l.k_dim, l.m, (uint32_t)l.weight_bits, l.canonical, l.gamma != nullptr, rope};
 }
 
 // Whether a FusedQkv / MatMul launch goes to the panel kernel: rows of up to 3072 features, from two input rows (four layers of the
@@ -388,9 +387,10 @@ static fa_panel::Plan panel_plan(const fa_ctx *ctx, const FusedQkvLaunch &l, boo
 // 1.17 times as long as the tiles) - unless the GEMM is a tenth ahead by
 // estimate: many weight rows are many passes of the input rows here, or rounds of workgroups. A launch takes the weight stream, and
 // for each pass that a compute unit has one after the other the input rows of that pass, fetched and multiplied and, with a gamma,
-// normalised (fitted to launches of 12 to 416 rows over 512 to 3072 features and 512 to 10240 weight rows; of 1380 with both sides
-// measured, none that leaves is more than 2 % slower for it). us, here and as a GEMM: 2048 x 10240 32 rows 16.6, 12.4, 100 rows 44.5,
-// 17.6; 2048 x 2560 64 rows 8.2, 11.0, 100 rows 12.8, 11.1; 1024 x 6144 100 rows 13.2, 8.8. An explicit GEMM threshold (fa_set_gemm_min_m) wins.
+// normalised (fitted to walks over passes, of launches of 12 to 416 rows over 512 to 3072 features and 512 to 10240 weight rows; a
+// workgroup for each pass, where there is one, takes less than the estimate says, so that what stays would stay). us, here and as a GEMM:
+// 2048 x 10240 32 rows 16.6, 12.4, 100 rows 44.5, 17.6; 2048 x 2560 64 rows 8.2, 11.0, 100 rows 12.8, 11.1; 1024 x 6144 100 rows 13.2, 8.8. An
+// explicit GEMM threshold (fa_set_gemm_min_m) wins.
 bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     constexpr uint32_t PANEL_MIN_M_DEFAULT = 2;
     auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
@@ -401,29 +401,30 @@ bool fa_qkv_rows32_takes(const fa_ctx *ctx, const FusedQkvLaunch &l) {
     if (ctx->gemm_min_m && (l.weight_bits != 16 || l.m >= ctx->gemm_min_m)) return false;
     if (!aligned16(l.x) || !aligned16(l.w[0]) || !aligned16(l.w[1]) || !aligned16(l.w[2]) || !aligned16(l.gamma)) return false;
     if (l.m < FA_GEMM_MIN_M_DEFAULT) return true;
-    const fa_panel::Plan p = panel_plan(ctx, l, false);  // (the write stage must not decide: a fused op takes the route of its two ops)
     const uint32_t n_cus = ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u;
-    if (l.m <= 32 && p.rounds == 1 && l.n_dim + 2 * l.n_kv <= 32 * n_cus) return true;
-    // More than 2048 features: a workgroup has one pass, with the weight rows that put all passes in one round (up to 80). Never behind
-    // the GEMM with F16 weights then, and always where they need a second round; block-quantised weights, which are made f16 for each
-    // pass, up to 48 of them, 64 of more than 2560 features. us, here and as a GEMM, 3072 features: 5120 rows F16 57 rows 13.3, 16.1; 10240 x
-    // 2560 F16 19 rows 14.7, 16.7; 4288 rows Q8_0 37 rows 11.2, 13.3; 2240 rows Q8_0 52 rows 9.6, 12.4; beyond the line 5184 x 2560 36
-    // rows Q4_0 13.2, 11.4 and Q8_0 12.9, 12.2; 5120 x 2304 57 rows Q4_0 13.5, 11.0; second round 5312 rows F16 58 rows 26.0, 19.7.
-    // (240 launches of 2112 to 3072 features x 1024 to 10600 rows.)
-    if (p.pk > 4)
-        return p.rounds == 1 && (f16 || ((l.m <= 48 || l.gamma || l.k_dim > 2304) && p.rows_per_wg <= (l.k_dim > 2560 ? 64u : 48u)));
+    // (the write stage must not decide: a fused op takes the route of its two ops)
+    const fa_panel::Shape shape = panel_shape(l, false);
+    const bool tiles_fit = fa_gemm_tiles_fit(l);  // (where they don't, the GEMM is a divided one of three launches: 1.5 to 4 times as long)
+    if (l.k_dim > 2048 && l.m > 16) {
+        // A workgroup for each pass: 0.69 to 0.97 of the tiles' time, but for F16 row-major weights in five tiles (1.09 to 1.36, 16 launches) and
+        // block-quantised ones, which are made f16 for each pass, in four tiles: up to 2560 features Q4_0 1.09, Q8_0 1.06 and with a gamma 0.95;
+        // longer Q4_0 1.04 and with a gamma 0.97, Q8_0 0.93 and 0.90 (75 launches in all).
+        const fa_panel::Plan b = fa_panel::panel_plan(shape, n_cus);
+        const bool q8 = l.weight_bits == 8;
+        if (b.form == fa_panel::BESIDE)
+            return !tiles_fit || (f16 ? l.canonical || b.nt < 5 : b.nt < 4 || (l.k_dim <= 2560 ? q8 && l.gamma != nullptr : q8 || l.gamma != nullptr));
+        if (!f16 && tiles_fit && b.grid_y < b.n_pass) return false;  // (walking over passes: 1.2 to 3 times the tiles' time, 200 launches)
+    }
+    const fa_panel::Plan p = fa_panel::walk_plan(shape, n_cus);
+    if (l.m <= 32 && p.rounds == 1) return true;
+    if (l.k_dim > 2048 && tiles_fit && p.rounds > 1) return false;  // (1.06 to 3.2 times the tiles' time, 50 launches)
     if (!l.gamma && l.m > 192 && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 16) * p.n_pass > (l.k_dim >= 512 ? 2 : 1) * n_cus) return false;
     // Block-quantised with a norm: where 32 input rows x 32 weight rows are more than a piece per compute unit, a second pass costs 3 us
     // and more, which the estimate below does not see of few features: 195 rows, 512 x 2112 Q4_0 12.0 us, 8.4 with the norm's launch and
     // the tiles; 391 rows, 640 x 1344 Q8_0 12.1, 9.2; 124 rows, 1280 x 2112 Q8_0 14.4, 9.3; 375 rows, 768 x 1664 13.8, 9.6; 248 rows,
     // 896 x 1664 Q4_0 9.65, 8.5; just below the line 192 rows, 512 x 1344 6.2, 7.2. (100 launches of 768 to 1024 features between one
     // piece and two: 0.71 to 0.975 of the panel kernel's time, 0.87 in the mean; 180 of 256 to 2048 features below the line: 1.09 to 1.32.)
-    if (!f16 && l.gamma && l.m > 32 && p.nc == 2 && l.k_dim % 64 == 0 && l.n_dim % 8 == 0 && l.n_kv % 8 == 0) {
-        const uint64_t pieces = (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 32) * p.n_pass;
-        bool scales_fit = true;  // (what the tiles ask of a launch)
-        for (int i = 0; i < 3; ++i) scales_fit = scales_fit && reinterpret_cast<uintptr_t>(l.scales[i]) % 4 == 0;
-        if (scales_fit && pieces > n_cus) return false;
-    }
+    if (!f16 && l.gamma && l.m > 32 && p.nc == 2 && tiles_fit && (uint64_t)ceil_div_u32(l.n_dim + 2 * l.n_kv, 32) * p.n_pass > n_cus) return false;
     // passes of a compute unit (with two workgroups on it they share its way to L2)
     const float passes = p.pk > 2 ? (float)(p.rounds * ceil_div_u32(p.n_pass, p.grid_y)) : std::max(1.0f, (float)(p.grid_x * p.n_pass) / (float)n_cus);
     const float k = (float)l.k_dim, mb = k * (float)(l.n_dim + 2 * l.n_kv) * (f16 ? 2.0f : l.weight_bits == 8 ? 1.0625f : 0.5625f) * 1e-6f;
@@ -456,19 +457,16 @@ static fa_status launch_panel(fa_ctx *ctx, const FusedQkvLaunch &l, const QkvRop
         d.table_rows = r.table_rows, d.normal = r.rope_normal ? 1u : 0u, d.apply = r.apply_rope ? 1u : 0u;
         a.block_shift = (d.block_size & (d.block_size - 1)) == 0 ? (uint32_t)__builtin_ctz(d.block_size) : 32u;
     }
-    const fa_panel::Plan p = panel_plan(ctx, l, rope != nullptr);
-    a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass, a.beside = p.beside, a.inv_beside = p.beside ? fa_inverse(p.beside) : 0;
+    const fa_panel::Plan p = fa_panel::panel_plan(panel_shape(l, rope != nullptr), ctx->n_cus > 0 ? (uint32_t)ctx->n_cus : 256u);
+    a.rows_per_wg = p.rows_per_wg, a.n_pass = p.n_pass, a.beside = p.beside(), a.inv_beside = a.beside ? fa_inverse(a.beside) : 0;
     a.scale_pairs = l.k_dim / 32 % 2 == 0 ? 1u : 0u;
     for (int i = 0; i < 3; ++i)
         if (reinterpret_cast<uintptr_t>(l.scales[i]) % 4 != 0) a.scale_pairs = 0;
     FaLaunchScope scope(ctx, rope ? "fused_qkv_rows32_rope_kernel" : l.n_kv ? "fused_qkv_rows32_kernel" : "matmul_rows32_kernel", true);
     const bool sums = l.m < FA_GEMM_MIN_M_DEFAULT;  // (of interest to block-quantised weights only: the arithmetic, see fa_panel.h)
-    const dim3 grid = p.beside ? dim3(ceil_div_u32(p.grid_x, 8) * 8 * p.beside) : dim3(p.grid_x, p.grid_y);
-    if (!fa_panel::has_kernel({a.total_rows, l.k_dim, l.m, (uint32_t)l.weight_bits, l.canonical, l.gamma != nullptr, rope != nullptr}, p))
-        return fa_fail(FA_ERR_INVALID_OPERATION, "panel kernel: no form of %u tiles x %u groups for rows of %u features", p.nt, p.nc, l.k_dim);
-    if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
-    else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
-    else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p.eights, p.nt, p.nc, p.pk, grid, a));
+    if (l.weight_bits == 16) FA_TRY(fa_panel::launch<16>(scope, rope != nullptr, sums, p, a));
+    else if (l.weight_bits == 8) FA_TRY(fa_panel::launch<8>(scope, rope != nullptr, sums, p, a));
+    else FA_TRY(fa_panel::launch<4>(scope, rope != nullptr, sums, p, a));
     return scope.finish();
 }
 

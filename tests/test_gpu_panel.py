@@ -116,6 +116,21 @@ def test_long_rows_in_five_tiles():
     test_chunk_in_one_launch(2592, 3840, 640, 64, 1, "f16")  # 80 weight rows to a workgroup, block-quantised as a GEMM
 
 
+@pytest.mark.parametrize("K,N,NK,m,layout,weights", [
+    (2592, 4104, 520, 40, 0, "f16"),  # three passes by one workgroup with two tiles (the product without a norm: 18 weight rows)
+    (2592, 3000, 24, 40, 0, "f16"),   # the product in one tile
+    (2592, 4104, 520, 40, 0, "q8"),
+    (2592, 4104, 520, 33, 1, "q8"),   # the last pass of one row
+    (2592, 4104, 520, 33, 1, "q4"),
+    (2592, 1160, 64, 35, 0, "q8"),    # one tile, a workgroup for each pass
+    (2592, 264, 72, 20, 1, "q4"),
+])
+def test_long_rows_walked_over(K, N, NK, m, layout, weights):
+    """Rows of more than 2048 features whose workgroups keep all their weights and go on to further passes (which of them do:
+    test_panel_plan.py)."""
+    test_chunk_in_one_launch(K, N, NK, m, layout, weights)
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("weights", ["f16", "q8", "q4"])
 @pytest.mark.parametrize("K,m", [(32, 2), (96, 11), (96, 12), (896, 33), (1056, 5), (2016, 20), (2080, 5), (2080, 17)])
@@ -160,30 +175,31 @@ def test_rows_absent_from_a_pass(K, N, NK, m, weights):
     (896, 14, 2, 64, 13),     # 5, passes of 8 rows
     (2048, 16, 2, 128, 24),   # 16 in two tiles, passes of 8 rows
 ])
-def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
+def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights, layout=1, norm=True):
     """Up to 16 weight rows per workgroup, and in the last of an odd number of tiles, both halves of NeoX pairs lie in one tile: the fused
     write stage equals the two ops to the bit, in both pairings."""
-    announce("neox pairs in one tile", K, H, Hkv, D, m, weights)
+    announce("neox pairs in one tile", K, H, Hkv, D, m, weights, layout, norm)
     f = ctx()
     rng = np.random.default_rng(K + H + m)
     N, NK = H * D, Hkv * D
     x, g, ws, bs = _data(rng, K, N, NK, m)
     scales, dev_s = None, []
     if weights == "f16":
-        dev_w = [f.array(orc.to_canonical(w)) for w in ws]
+        dev_w = [f.array(orc.to_canonical(w) if layout else w.reshape(-1)) for w in ws]
         arg = [w.arg() for w in dev_w]
     else:
         quant = [orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w) for w in ws]
         dev_s = [f.array(s) for _, s in quant]
         scales = [s.arg() for s in dev_s]
-        dev_w = [f.array(orc.to_canonical(q) if weights == "q8" else orc.pack_q4_0(orc.to_canonical(q))) for q, _ in quant]
+        flat = [orc.to_canonical(q) if layout else q.reshape(-1) for q, _ in quant]
+        dev_w = [f.array(q if weights == "q8" else orc.pack_q4_0(q)) for q in flat]
         arg = [w.arg() if weights == "q8" else w.arg((n, K), dtype=fa.DTYPE_Q4_0) for w, n in zip(dev_w, (N, NK, NK))]
     dx, dg, db = f.array(x), f.array(g), [f.array(b) for b in bs]
     outs = [f.zeros((m, n)) for n in (N, NK, NK)]
     cos, sin = fa.rope_tables(5e5, D, m + 3)
     dcos, dsin = f.array(cos), f.array(sin)
     rot = [[f.zeros((H, m, D)), f.zeros((Hkv, m + 3, D)), f.zeros((Hkv, m + 3, D))] for _ in range(2)]
-    kw = dict(gamma=dg.arg(), biases=[b.arg() for b in db], layout=1, scales=scales)
+    kw = dict(gamma=dg.arg() if norm else None, biases=[b.arg() for b in db], layout=layout, scales=scales)
     f.fused_qkv(dx.arg(), *arg, *[o.arg() for o in outs], K, N, NK, m, **kw)
     for mode in (fa.ROPE_NEOX, fa.ROPE_NORMAL):
         p = fa.KvPrepFusedParams.make(H, Hkv, D, m, 2, m + 3, mode)
@@ -201,3 +217,15 @@ def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights):
             assert np.any(want) and np.array_equal(got.view(np.uint16), want.view(np.uint16)), mode
     for b in [dx, dg, dcos, dsin] + db + outs + dev_w + dev_s + rot[0] + rot[1]:
         b.free()
+
+
+@pytest.mark.parametrize("K,H,Hkv,D,m,weights,layout,norm", [
+    (2592, 40, 1, 128, 33, "f16", 0, True),  # two tiles, three passes by one workgroup
+    (2592, 24, 3, 128, 40, "f16", 0, False),  # one tile
+    (2592, 40, 1, 128, 33, "q8", 1, True),
+    (2592, 19, 1, 64, 35, "q8", 1, True),    # one tile, a workgroup for each pass
+    (2592, 40, 1, 128, 33, "q4", 0, True),
+    (2592, 19, 1, 64, 35, "q4", 1, True),
+])
+def test_rotation_of_long_rows_walked_over(K, H, Hkv, D, m, weights, layout, norm):
+    test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights, layout, norm)
