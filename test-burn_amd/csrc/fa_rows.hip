@@ -513,7 +513,7 @@ fa_status fa_launch_prefill_rows(fa_ctx *ctx, const PrefillLaunch &L, const Rows
         a.part_acc = (float *)ctx->workspace, a.part_ml = (float *)((char *)ctx->workspace + acc_bytes);
     }
     {
-        FaLaunchScope scope(ctx, "flash_rows_kernel", true);
+        FaLaunchScope scope(ctx, a.turn ? "flash_rows_kernel_turned" : "flash_rows_kernel", true);
         if (L.head_dim == 128) {
             if (plan.waves == 8) launch_rows<128, 8>(scope, a, grid, L.bf16, L.paged);
             else launch_rows<128, 4>(scope, a, grid, L.bf16, L.paged);

@@ -199,6 +199,48 @@ def test_rows_turned_paged(H, Hkv, D, M, prefix, split, bs):
     test_rows_paged(H, Hkv, D, M, prefix, split, bs)
 
 
+IN_TURNED_ORDERS = [
+    # H, Hkv, D, rows, prefix, splits expected
+    (24, 8, 128, 300, 950, False),   # one workgroup to a unit, four waves: windows of 8 rounds and a last one of fewer
+    (24, 8, 128, 300, 1020, False),  # eight waves, windows of 4
+    (20, 5, 128, 120, 2000, False),  # KV heads that are not a divisor of 8
+    (8, 8, 128, 66, 3001, True),     # split: windows of 2
+    (16, 8, 128, 700, 1500, False),  # several workgroups to a unit
+    (32, 8, 64, 300, 5000, False),   # D 64, windows of 32 rounds, more than 32 tiles to a wave: pages are looked up a second time
+]
+
+
+def _turned():
+    """Launches in turned orders since the profile was last reset."""
+    return ctx().profile_query("flash_rows_kernel_turned")[0]
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f16", "bf16"])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", IN_TURNED_ORDERS)
+def test_turned_orders_contiguous(H, Hkv, D, M, prefix, split, bf16):
+    test_rows_contiguous(H, Hkv, D, M, prefix, split, bf16)
+    assert _turned() == 1
+
+
+@pytest.mark.parametrize("bs", [16, 48])
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", IN_TURNED_ORDERS)
+def test_turned_orders_paged(H, Hkv, D, M, prefix, split, bs):
+    test_rows_paged(H, Hkv, D, M, prefix, split, bs)
+    assert _turned() == 1
+
+
+def test_turned_orders_large_pool():
+    test_rows_paged_large_pool(128, 100, 9000)
+    assert _turned() == 1
+
+
+@pytest.mark.parametrize("M,N,offset,causal", [(200, 9300, 0, False), (200, 9300, 9400, True)])
+def test_turned_orders_masks(M, N, offset, causal):
+    """Without the causal mask; query positions past the keys' end."""
+    test_rows_masks_and_layouts(M, N, offset, causal, 128)
+    assert _turned() == 1
+
+
 @pytest.mark.parametrize("H,Hkv,D,M,prefix", [(24, 8, 128, 278, 7179), (16, 2, 128, 34, 47550), (32, 8, 128, 51, 19165), (4, 4, 128, 18, 44996)])
 def test_long_keys_from_memory_stay_with_the_other_kernels(H, Hkv, D, M, prefix):
     """Shapes that take 1.15 to 1.6 times as long on this kernel where their keys come from memory: the choice is another one, with its
