@@ -1100,10 +1100,10 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     // of keys that come from memory, as a layer's do in a model: of long ones that do, the first kernel takes longer (us, rows and the
     // other: 278 rows after 7179, H24 / Hkv8 / D128 55.3, 48.6; 34 after 47550, H16 / Hkv2 / D128 47.3, 36.7; 18 after 44996, H4 / Hkv4 /
     // D128 38.7, 24.1; the first of them 47 in turned orders, RowsTurn), of keys that lie in the last-level cache from the call before the
-    // least of all: where the first and the second are level, the first is a fifth ahead from a cache, 32 after 8160 17.1, 17.2 and 13.0, 16.1. On 4000
-    // launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, half of them with keys in memory) the
-    // choice takes 1.002 to 1.014 times as long as the best of the three, in the mean, and 0.69 to 0.76 of what the other two would: 48
-    // are slower for it by more than 3 %, by 17 % at most (profiles/prefill_choice.txt).)
+    // least of all. On 2200 launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, a third of them with
+    // keys in the cache, a quarter paged) the choice takes 1.004 to 1.011 times as long as the best of the three, in the mean, and 0.75 to 0.84
+    // of what the other two would: 32 are slower for it by more than 3 %, by 29 % at most (profiles/prefill_choice.txt). Where the first is
+    // 0.95 to 1.02 of the second's estimate it takes 0.93 of its time in turned orders (RowsTurn; 1.02 to 1.1: 1.04) and 0.99 in one.)
     const bool automatic = ctx->prefill_variant == 0 && ctx->prefill_split_k == 0;
     const RowsPlan rows = automatic ? fa_prefill_rows_plan(ctx, L) : RowsPlan();
     if ((automatic || ctx->prefill_variant == 3) && !ctx->prefill_chunk_off) {
@@ -1179,8 +1179,9 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
             const float cu = wide ? share * (3.52f + 1.041f * (first + longest)) : share * (2.66f + 0.66f * (first + longest));
             us = (wide ? 6.41f : 5.43f) + (one > cu ? one : cu) + (wide ? 0.147f : 0.0775f) * kv_mb;
         }
-        // (For launches in turned orders this estimate is up to a tenth too long, or they take longer than theirs where many rounds of one
-        // workgroup's follow: of 420 of 4 to 2500 rows the choice is within 0.9 % of the best in the mean with 0.92 of it, 1.5 % with the whole.)
+        // (Launches in turned orders take longer against this than by the estimates. Theirs / this kernel's time by the ratio of the estimates, of
+        // 260 launches: unsplit over up to 6144 keys 0.79 at 0.7-0.82, 0.95 at 0.82-0.92, 1.03 at 0.92-1; over more 0.98, 1.03, 1.12; split
+        // 0.80, 0.90, 1.01. In one order 0.76, 0.90, 1.00, and 1.06 at 1-1.1.)
         const float ahead = !rows.turn ? 1.0f : rows.splits == 1 && L.kv_len > 6144 ? 0.82f : 0.92f;
         if (rows.us < ahead * us) return fa_launch_prefill_rows(ctx, L, rows);
     }

@@ -397,24 +397,28 @@ static uint32_t mates_apart(uint32_t n_kv_heads) {
 // asked for one block's worth of tiles and its latency stands in every round; each from another round on, the first requests of all are
 // the whole window, and later rounds find it in the L2. A window's tiles of all streams of an XCD (its KV heads, times the splits) take
 // 3.1 MB of its 4: at 4.2 MB and beyond keys are read again (H16 / Hkv2 / D128, 30 rows after 33878, 16 splits: 29.0 us in one order, 31.7
-// with windows of 4 MB, 38.9 of 8). Where keys lie in a cache anyway and a unit has one workgroup or few, the longer start and the scalar
-// work of a round are 0.1 to 0.3 us of 5 to 10: launches of more than 4 MB, or of several workgroups per unit with many rounds. D 64 in windows
-// of two rounds loses up to 5 % there (44 rows after 5314, H14 / Hkv2: 8.8, 9.1). us in one order -> turned, keys from memory:
+// with windows of 4 MB, 38.9 of 8). The longer start and the scalar work of a round are 0.1 to 0.3 us: turned from 4 MB of keys on where a unit
+// has one workgroup, 8 where it has several, and, split, from 9 (D 64: 16). Turned / one order in the mean of 1400 launches of 2 to 8000 rows
+// after 0 to 100000, keys from memory (800 with keys in the last-level cache in brackets):
+//   one workgroup   4-8 MB 0.99 (0.96)    8-16 0.86 (0.99)    from 16 0.82 (0.83)
+//   several         up to 8 1.00 (1.00)   8-16 0.96 (1.00)    from 16 0.97 (0.99)
+//   split, D 128    up to 9 1.04 (1.02)   9-16 0.96 (1.04)    from 16 0.94 (1.00)
+//          D 64     up to 8 1.06 (1.04)   8-16 1.02 (1.05)    from 16 0.94 (1.00)
+// us in one order -> turned, keys from memory:
 //   H24 / Hkv8 / D128:  500 after 1000 20.5 -> 17.7; 187 after 1130 14.8 -> 12.5; 32 after 8160 18.3 -> 17.0; 68 after 13543 35.0 -> 30.6
 //   H32 / Hkv8 / D128:  194 after 2151 21.1 -> 16.9; H8 / Hkv8: 1928 after 1015 34.4 -> 27.8; H16 / Hkv2: 131 after 11517 34.5 -> 29.6
 //   D 64:  H32 / Hkv8, 1447 after 591 31.7 -> 27.7; H14 / Hkv2, 992 after 10818 64.8 -> 59.1
 struct RowsTurn {
-    uint32_t longest = 0, wgs = 0, xcd_heads_kb = 0;  // 0: in one order
-    bool large = false, wide = false;
-    RowsTurn(const PrefillLaunch &L, uint32_t wgs_, uint32_t n_blocks, uint32_t longest_, float kv_mb) : longest(longest_), wgs(wgs_), large(kv_mb > 4.0f), wide(L.head_dim == 128) {
-        if (!(large || wgs > 600) || (n_blocks - 1) >> mates_apart(L.n_kv_heads) == 0) return;
+    uint32_t longest = 0, xcd_heads_kb = 0;  // 0: in one order
+    bool wide = false;
+    RowsTurn(const PrefillLaunch &L, uint32_t wgs, uint32_t n_blocks, uint32_t longest_, float kv_mb, uint32_t n_cus) : longest(longest_), wide(L.head_dim == 128) {
+        if (kv_mb <= (wgs <= n_cus ? 4.0f : 8.0f) || (n_blocks - 1) >> mates_apart(L.n_kv_heads) == 0) return;
         const uint32_t twos = L.n_kv_heads & (0u - L.n_kv_heads);
         xcd_heads_kb = L.n_kv_heads / (twos < 8 ? twos : 8) * (KT * L.head_dim * 4 / 1024);  // of a tile for each wave of a stream
     }
     uint32_t operator()(uint32_t waves, uint32_t splits) const {
         if (!xcd_heads_kb) return 0;
         const uint32_t rounds = ceil_div_u32(ceil_div_u32(longest, splits), waves), held = 3100 / (xcd_heads_kb * waves * splits);
-        if (!large && rounds < 8) return 0;
         uint32_t most = rounds < held ? rounds : held;
         most = most < 32 ? most : 32;
         const uint32_t turn = most ? 1u << (31 - __builtin_clz(most)) : 0u;
@@ -459,7 +463,7 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
     const float r8 = (float)ceil_div_u32(longest, 8), r4 = (float)ceil_div_u32(longest, 4);
     const float head_mb = (float)longest * (float)(KT * L.head_dim) * 4e-6f, kv_mb = head_mb * (float)L.n_kv_heads;
     const bool waited = wgs <= n_cus && kv_mb > 9.0f;
-    const RowsTurn turned(L, wgs, n_blocks, longest, kv_mb);
+    const RowsTurn turned(L, wgs, n_blocks, longest, kv_mb, n_cus);
     const uint32_t turn8 = turned(8, 1), turn4 = turned(4, 1);
     // (turned: 390 launches, 4 to 5 % rms)
     const float us8 = turn8 ? (wide ? 2.69f + larger(1.086f * r8, 3.11f * n + 0.122f * chain + 0.0135f * all) + (wgs <= n_cus ? 0.188f : 0.133f) * kv_mb
@@ -485,6 +489,7 @@ RowsPlan fa_prefill_rows_plan(const fa_ctx *ctx, const PrefillLaunch &L) {
                                 : 5.28f + 0.644f * r + 0.0752f * (float)s + 0.4585f * mb + 0.0584f * kv_mb + 0.41f * xcd_mb;
         if (us < best) best = us, plan.us = us, plan.splits = s, plan.waves = 8, plan.turn = turn;
     }
+    if (plan.splits > 1 && kv_mb <= (wide ? 9.0f : 16.0f)) plan.turn = 0;  // (see RowsTurn; which division is best the estimates above still tell)
     return plan;
 }
 

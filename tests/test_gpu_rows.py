@@ -222,6 +222,17 @@ def test_turned_orders_contiguous(H, Hkv, D, M, prefix, split, bf16):
     assert _turned() == 1
 
 
+@pytest.mark.parametrize("H,Hkv,D,M,prefix,split", [
+    (6, 2, 128, 200, 4100, True),    # 4.4 MB of keys, split
+    (14, 2, 64, 54, 15370, True),    # 7.9
+    (16, 8, 128, 700, 400, False),   # 4.5, several workgroups to a unit
+])
+def test_one_order_of_fewer_keys(H, Hkv, D, M, prefix, split):
+    """Between 4 MB and where turned orders are ahead of one for launches that are split or have several workgroups to a unit."""
+    test_rows_contiguous(H, Hkv, D, M, prefix, split, False)
+    assert _turned() == 0
+
+
 @pytest.mark.parametrize("bs", [16, 48])
 @pytest.mark.parametrize("H,Hkv,D,M,prefix,split", IN_TURNED_ORDERS)
 def test_turned_orders_paged(H, Hkv, D, M, prefix, split, bs):
