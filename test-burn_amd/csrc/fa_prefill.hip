@@ -742,10 +742,10 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         int lo = lane;
         asm volatile("" : "+v"(lo));
         const int n = lo & 31, hi = lo >> 5, lane = lo;
-        const WaveRows owr = wave_rows(place_of(o_item), (uint32_t)wave);  // this wave's rows of the item
+        const Place o_place = place_of(o_item);
+        const WaveRows owr = wave_rows(o_place, (uint32_t)wave);  // this wave's rows of the item
         if (!owr.ok) return;  // (a packed item with fewer heads than waves)
         const uint32_t o_head = owr.head, o_row0 = owr.row0;
-        const uint32_t o_split = a.pack_heads ? o_item % S : (o_item % (a.n_heads * S)) % S;
         const float o_m = m_run;  // untouched since the exchange, like l_run: this lane's half of the row's keys
         typedef unsigned int u2v __attribute__((ext_vector_type(2)));
         const u2v lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
@@ -753,7 +753,7 @@ __global__ void __launch_bounds__(512, 1) flash_prefill_dma_kernel(PrefillDev a_
         const uint32_t q_row = o_row0 + n;
         if (S > 1) {  // flash_prefill.metal:592-617
             if (q_row < a.q_len) {
-                const size_t prow = (size_t)((o_head * n_qt + q_row / BM) * S + o_split) * a.part_rows + q_row % BM;
+                const size_t prow = (size_t)((o_head * n_qt + q_row / BM) * S + o_place.split) * a.part_rows + q_row % BM;
                 float *pa = a.part_acc + prow * D;
 #pragma unroll
                 for (int b = g * HB; b < (g + 1) * HB; ++b)
