@@ -219,6 +219,12 @@ def test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights, layout=1, norm=True):
         b.free()
 
 
+@pytest.mark.parametrize("K,H,Hkv,D,m", [(3072, 24, 8, 128, 64), (2592, 36, 1, 128, 57)])
+def test_neox_pairs_in_five_tiles(K, H, Hkv, D, m):
+    """40 pairs to a workgroup, 32 in two pairs of tiles and 8 in a fifth; 38 of them, and a last pass of 9 rows."""
+    test_neox_pairs_in_one_tile(K, H, Hkv, D, m, "f16")
+
+
 @pytest.mark.parametrize("K,H,Hkv,D,m,weights,layout,norm", [
     (2592, 40, 1, 128, 33, "f16", 0, True),  # two tiles, three passes by one workgroup
     (2592, 24, 3, 128, 40, "f16", 0, False),  # one tile

@@ -112,6 +112,7 @@ def test_fused_op_equals_the_two_ops(H, Hkv, D, K, m, pos, cap, mode, norm, bias
     (14, 2, 64, 896, 7, 9, 32, fa.ROPE_NEOX),         # a few rows (the weight-stream form)
     (16, 2, 128, 2048, 30, 40, 16, fa.ROPE_NEOX),     # a chunk of the one-launch weight stream: rows across three blocks
     (24, 8, 128, 3072, 32, 37, 16, fa.ROPE_NORMAL),
+    (24, 8, 128, 3072, 57, 37, 16, fa.ROPE_NEOX),     # five tiles of weight rows to a workgroup
 ])
 def test_fused_op_into_a_paged_cache(H, Hkv, D, K, m, pos, bs, mode):
     announce("fused qkv + kv prep, paged", H, Hkv, D, K, m, pos, bs, mode)

@@ -54,7 +54,7 @@ int main() {
         expect(896, 896, 32, bits, 1, 0, 0, BESIDE, 1), expect(1152, 896, 16, bits, 1, 1, 0, EIGHTS, 1), expect(2560, 2048, 24, bits, 1, 1, 1, EIGHTS, 2);
         expect(2560, 2048, 24, bits, 0, 1, 1, bits == 4 ? EIGHTS : WALK, bits == 4 ? 2 : 1);
     }
-    expect(5120, 2592, 64, 16, 1, 1, 0, BESIDE, 5), expect(5120, 3072, 64, 16, 1, 1, 1, BESIDE, 5);
+    expect(5120, 2592, 64, 16, 1, 1, 0, BESIDE, 5), expect(5120, 3072, 64, 16, 1, 1, 1, BESIDE, 5), expect(4864, 2592, 57, 16, 1, 1, 1, BESIDE, 5), expect(5120, 3072, 57, 16, 1, 1, 1, BESIDE, 5);
     for (uint32_t n_cus = 8; n_cus <= 320; n_cus += n_cus < 64 ? 4 : 8)
         for (uint32_t bits : {4u, 8u, 16u})
             for (int flags = 0; flags < 8; ++flags)
