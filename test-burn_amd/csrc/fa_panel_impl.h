@@ -227,13 +227,19 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
     req_t wv[NT][NA];
     const unsigned char *w_at[NT];  // block 0 of the lane's row in each tile, and how far apart blocks are
     uint32_t w_step[NT];
+    // Weights are kept in the caches by kernels whose workgroups share them on an XCD, but for F16 rows of more than 1024 features in up to
+    // two tiles, and block-quantised ones of more than 2048: the same kernels have launches that share nothing, which take 1.05 times as long
+    // (o_proj of 3072 x 3072 F16, 5 rows 5.40 -> 5.67 us, of 2048 x 2048 16 rows 4.40 -> 4.61). 0.96 to 0.99 of the nontemporal loads' time in the mean
+    // (250 launches of 9 to 64 rows): FusedQkv + KvPrepFused of 1152 x 896, 32 rows F16 4.33 -> 4.09, of 2560 x 2048, 24 rows Q8_0 6.14 -> 6.07, o_proj
+    // of 2048 x 2048, 16 rows Q8_0 3.99 -> 3.80.
+    constexpr bool SHARED = NT > 2 || (BESIDE && PK <= (WB == 16 ? 2 : 4));
     auto request_weights = [&](int t, int i) __attribute__((always_inline)) {
         const uint32_t kb = kb_of(i) + get_blk;
         const unsigned char *p = w_at[t] + (size_t)min(kb, nkb - 1u) * w_step[t];
         // (F16: zeros past the last block. The input is zero there, but an infinite weight read again would make NaN of it;
         // block-quantised weights are finite, and their scale is zero there.)
         if (WB == 16 && kb >= nkb) p = reinterpret_cast<const unsigned char *>(&zero_weights);
-        wv[t][i % NA] = NT > 2 ? fa_norm::load_global<req_t>(p) : fa_norm::load_global_once<req_t>(p);
+        wv[t][i % NA] = SHARED ? fa_norm::load_global<req_t>(p) : fa_norm::load_global_once<req_t>(p);
     };
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
