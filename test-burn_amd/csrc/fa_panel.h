@@ -8,18 +8,22 @@
 // the matrix instruction's operand (16 rows x 64 bytes, one row per lane of a 16-lane group) moves 37 KB/us into a compute unit
 // from L2, a request along a row 108 to 130 KB/us. So rows are fetched along themselves, whole rows per wave (row r by wave
 // r % 8), normalised in the registers they arrive in (no exchange between waves), written to LDS and read back as operands:
-//   * a workgroup (8 waves) owns up to 32 weight rows - two 16-row tiles - and walks over its passes of 32 input rows. All its weights
-//     are requested once, straight into the operand layout, behind the first pass's input rows; a pass's rows are requested while the
-//     one before is multiplied;
-//   * rows of more than 2048 features: 16 input rows to a workgroup and no second pass, but up to five tiles, a few of whose requests are
-//     on their way at a time (RING, and panel_plan for what both gave);
+//   * a workgroup (8 waves) owns one or more 16-row tiles of weight rows. Its passes of input rows are divided in one of three forms, chosen
+//     in fa_panel_plan.h:
+//       - WALK: up to two tiles and passes of 32 input rows (16 of more than 2048 features), which it goes through one after the other. All its
+//         weights are requested once, straight into the operand layout, behind the first pass's input rows; a pass's rows are requested
+//         while the one before is multiplied. Few weight rows and many input rows: the passes are spread over workgroups (grid y);
+//       - BESIDE: one pass of 16 input rows and up to five tiles (two of up to 1024 features, three of up to 2048); the workgroups of the same
+//         weight rows lie next to each other on an XCD. Of more than 2048 features a few requests of every tile are on their way at a
+//         time (RING);
+//       - EIGHTS: the same with passes of 8 rows and up to two tiles;
 //   * wave w multiplies the feature blocks 16 j + 2 w and 16 j + 2 w + 1 of every 512 features (adjacent: the two requests touch
 //     the same lines);
 //   * the eight waves' partial tiles meet in LDS and are added in wave order; then alpha, bias, beta * residual and one
 //     rounding, or the KvPrepFused work on the rounded values (a workgroup then takes whole rotation pairs);
-//   * few weight rows and many input rows: the passes are spread over workgroups (grid y), each keeping its 32 weight rows;
-//   * NeoX pairs of a workgroup of up to 16 weight rows, and of the last of an odd number of tiles, lie in one tile, 8 rows from each half (two tiles of which half the rows did
-//     not exist: 1152 x 896, 8 rows, F16 4.4 -> 3.8 us, Q8_0 4.9 -> 4.0, Q4_0 5.0 -> 4.1; 2560 x 2048 6.4 -> 5.4, 7.0 -> 5.4, 6.7 -> 5.2).
+//   * NeoX pairs of a workgroup of up to 16 weight rows, and of the last of an odd number of tiles, lie in one tile, 8 rows from each half
+//     (two tiles of which half the rows did not exist: 1152 x 896, 8 rows, F16 4.4 -> 3.8 us, Q8_0 4.9 -> 4.0, Q4_0 5.0 -> 4.1; 2560 x 2048
+//     6.4 -> 5.4, 7.0 -> 5.4, 6.7 -> 5.2).
 // Block-quantised weights become f16(weight * scale) as in the GEMM (src/metals/mma/tile_loader.metal:100-120); below 12 input
 // rows (SUMS) they follow the weight stream: a matrix instruction covers one 32-feature block, its f32 sums times the scale.
 #pragma once
