@@ -52,9 +52,9 @@ struct Weights<4> {
 // What a lane reads in the place of an F16 weight block past the row's last.
 static __device__ const h8_t zero_weights = {0, 0, 0, 0, 0, 0, 0, 0};
 
-// FEW: at most 8 input rows, in the launch or (EIGHTS) to a workgroup, those of the same weight rows side by side, one per wave: the other half of the 16 columns is not loaded, normalised or stored. (8 rows, two per
-// wave -> one: QKV with its norm, 5120 x 3072 F16 10.1 -> 9.3 us, Q8_0 10.1 -> 9.0, Q4_0 10.0 -> 8.3; 1152 x 896 F16 4.8 -> 4.4;
-// 3072 x 3072 without a norm 6.5 -> 5.8, 6.0 -> 5.5, 6.4 -> 5.1.)
+// FEW: at most 8 input rows to a workgroup, one per wave - the launch has no more, or (EIGHTS) they are one of its passes: the other half of
+// the 16 columns is not loaded, normalised or stored. (8 rows, two per wave -> one: QKV with its norm, 5120 x 3072 F16 10.1 -> 9.3 us, Q8_0
+// 10.1 -> 9.0, Q4_0 10.0 -> 8.3; 1152 x 896 F16 4.8 -> 4.4; 3072 x 3072 without a norm 6.5 -> 5.8, 6.0 -> 5.5, 6.4 -> 5.1.)
 template <int WB, int NT, int NC, int PK, bool ROPE, bool SUMS, bool FEW, bool EIGHTS, bool WALK>
 __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 2)) panel_kernel(PanelDev a_by_value) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -311,8 +311,10 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                 for (int j = 0; j < PK; ++j) xr[i][j] = fa_norm::scale8(xr[i][j], inv_rms, G_IN_LDS<PK> ? g_lds[j * 64 + lane] : gv[j]);
             }
         }
-        constexpr int CHAINS = WB == 16 && PK > 4 ? 2 : 1;
-        f4v_t d[NT][NC], d2[NT][NC];  // (the longest rows: two chains, 2.0 x 2^-24 of the sums' size as their error, 2.4 with one)
+        // The longest rows: two chains of sums. Their error in units of 2^-24 of the sums' size, 12 to 64 rows of 2112 to 3072 features: F16 2.0, 2.4
+        // with one; Q8_0 1.8 to 2.1 (one 2.1 to 2.4, the GEMM's tiles 2.0 to 2.3), Q4_0 1.8 to 2.1 (2.2 to 2.4, 3.0) for 0 to 1 % of the time.
+        constexpr int CHAINS = PK > 4 && (WB == 16 || (RING && !SUMS)) ? 2 : 1;
+        f4v_t d[NT][NC], d2[NT][NC];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -412,7 +414,7 @@ __global__ void __launch_bounds__(NTHREADS, (two_per_cu(NT, NC, PK, ROPE) ? 4 : 
                         const h8_t w = WB == 16 ? W::f16(W::part(raw[t], 0), (_Float16)1.0f) : W::f16(W::part(raw[t], st), sc[t]);
 #pragma unroll
                         for (int h = 0; h < NC; ++h) {
-                            f4v_t &sum = i % CHAINS ? d2[t][h] : d[t][h];
+                            f4v_t &sum = (GB == 1 ? i : st) % CHAINS ? d2[t][h] : d[t][h];
                             sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[h], sum, 0, 0, 0);
                         }
                     }

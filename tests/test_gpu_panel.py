@@ -235,3 +235,36 @@ def test_neox_pairs_in_five_tiles(K, H, Hkv, D, m):
 ])
 def test_rotation_of_long_rows_walked_over(K, H, Hkv, D, m, weights, layout, norm):
     test_neox_pairs_in_one_tile(K, H, Hkv, D, m, weights, layout, norm)
+
+
+@pytest.mark.parametrize("weights", ["q8", "q4"])
+def test_sums_of_long_rows_are_as_exact_as_the_tiles(weights):
+    """The f32 sums behind the rounding to f16, from 2^10 (sum - its f16 value), against 64 bits: the error of 56 rows of 3072 features is no
+    larger than that of the GEMM's tiles, which take more rows than that."""
+    K, N, m, S = 3072, 2048, 56, 2.0 ** 10
+    announce("panel, error of the sums", weights)
+    f = ctx()
+    rng = np.random.default_rng(5)
+    x = rng.normal(size=(m, K)).astype(np.float16)
+    w = (rng.normal(size=(N, K)) * K ** -0.5).astype(np.float16)
+    q, s = orc.quantize_q8_0(w) if weights == "q8" else orc.quantize_q4_0(w)
+    exact = x.astype(np.float64) @ orc.dequantize_blocks(q, s).astype(np.float64).T
+    c = exact.astype(np.float16)
+    dw = f.array(q.reshape(-1) if weights == "q8" else orc.pack_q4_0(q.reshape(-1)))
+    arg = dw.arg() if weights == "q8" else dw.arg((N, K), dtype=fa.DTYPE_Q4_0)
+    dx, ds, dc, do, error = f.array(x), f.array(s), f.array(c), f.zeros((m, N)), []
+    for min_m, name in ((0, "matmul_rows32_kernel"), (1, "matmul_gemm_kernel")):
+        f.set_gemm_min_m(min_m)
+        f.profile_reset()
+        f.profile_enable(True)
+        try:
+            f.matmul(dx.arg(), arg, do.arg(), m, N, K, c=dc.arg(), transpose_b=True, alpha=S, beta=-S, b_scales=ds.arg())
+            f.synchronize()
+            assert f.profile_query(name)[0] == 1
+        finally:
+            f.profile_enable(False)
+            f.set_gemm_min_m()
+        error.append(np.sqrt(np.mean((do.download() / S - (exact - c)) ** 2) / np.mean(exact ** 2)) * 2.0 ** 24)
+    assert 0 < error[0] <= error[1] < 4, error
+    for b in (dx, dw, ds, dc, do):
+        b.free()
