@@ -1101,8 +1101,8 @@ fa_status fa_launch_prefill(fa_ctx *ctx, const PrefillLaunch &L) {
     // other: 278 rows after 7179, H24 / Hkv8 / D128 55.3, 48.6; 34 after 47550, H16 / Hkv2 / D128 47.3, 36.7; 18 after 44996, H4 / Hkv4 /
     // D128 38.7, 24.1; the first of them 47 in turned orders, RowsTurn), of keys that lie in the last-level cache from the call before the
     // least of all. On 2200 launches beside the fitted ones (2 to 8000 rows after 0 to 100000, 11 combinations of heads, a third of them with
-    // keys in the cache, a quarter paged) the choice takes 1.004 to 1.011 times as long as the best of the three, in the mean, and 0.75 to 0.84
-    // of what the other two would: 32 are slower for it by more than 3 %, by 29 % at most (profiles/prefill_choice.txt). Where the first is
+    // keys in the cache, a quarter paged) the choice takes 1.004 to 1.010 times as long as the best of the three, in the mean, and 0.75 to 0.83
+    // of what the other two would: 20 are slower for it by more than 3 %, by 16 % at most (profiles/prefill_choice.txt). Where the first is
     // 0.95 to 1.02 of the second's estimate it takes 0.93 of its time in turned orders (RowsTurn; 1.02 to 1.1: 1.04) and 0.99 in one.)
     const bool automatic = ctx->prefill_variant == 0 && ctx->prefill_split_k == 0;
     const RowsPlan rows = automatic ? fa_prefill_rows_plan(ctx, L) : RowsPlan();
